@@ -21,7 +21,8 @@
 // before they meet the values).
 //
 // This is the kernel of the true 32-bit path and the fallback for sizes that the
-// matrix-core kernels refuse.
+// matrix-core kernels refuse.  Float32 heads of 32, 64, 128 or 256 channels in pages of a multiple of 16 keys take
+// `attn_rows_f32_kernel` below, which walks the same keys on the float32 matrix instruction.
 #include "common.h"
 
 #include <math.h>
@@ -148,6 +149,232 @@ __global__ __launch_bounds__(64) void attn_generic_kernel(const TX* __restrict__
     }
 }
 
+// ------------------------------------------------------------------ float32 rows on the matrix cores
+// Attention of float32 queries to float32 pages: a workgroup of four wavefronts owns 16 rows of one kv head, `tp`
+// consecutive tokens of `hp` heads each.  Keys go in blocks of 16 that start at multiples of 16, block b to wavefront
+// b % 4, each of which keeps a running softmax of its own for every row; the four meet in LDS in their order.  Blocks and
+// shares are counted from key 0, and a block that a row sees nothing of leaves its sums as they are, so a row's result
+// does not depend on the rows beside it.
+//
+// S[key][row] = K Q^T comes out of v_mfma_f32_16x16x4_f32 with keys 4 g + e (g = lane / 16) of row lane % 16 in a lane,
+// which is how the next product, out[channel][row] += V^T P, wants its column operand: the e-th instruction takes keys
+// 4 g + e, and a value row of the cache (the slots of a page side by side a channel) is read four keys a lane.
+//
+// What bounds it: trips to memory (a block's keys and values are asked for together, 16 KB a wavefront for 128 channels).
+// 333 tokens, 16 heads over 4 kv heads of 128: 279 us with a wavefront a (token, head), which fetches every key for every
+// row, 28 us with this.
+typedef __attribute__((ext_vector_type(4))) float f32x4;
+
+template <int DB>
+__global__ __launch_bounds__(256) void attn_rows_f32_kernel(const float* __restrict__ q, float* __restrict__ out,
+                                                            const float* __restrict__ kcache,
+                                                            const float* __restrict__ vcache,
+                                                            const int* __restrict__ positions,
+                                                            const int* __restrict__ token_entry,
+                                                            const int* __restrict__ block_table,
+                                                            const float* __restrict__ gate, int64_t gate_stride,
+                                                            const float* __restrict__ sink, AttnArgs a, int tokens, int tp,
+                                                            int hp) {
+    constexpr int D = 16 * DB;
+    __shared__ f32x4 acc_s[4][DB][PULSE_WAVE];
+    __shared__ float m_s[4][16], l_s[4][16];
+
+    const int group = a.nq / a.nkv;
+    const int t0 = blockIdx.x * tp;
+    const int kvh = blockIdx.y, h0 = kvh * group + blockIdx.z * hp;
+    const int lane = threadIdx.x % PULSE_WAVE;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / PULSE_WAVE);
+    const int r = lane % 16, kg = lane / 16;
+    const int t_end = min(t0 + tp, tokens);
+
+    // this lane's row (a row past the end is row 0 of the tile, sees nothing and is not written)
+    const bool live = r / hp < tp && t0 + r / hp < t_end && blockIdx.z * hp + r % hp < group;
+    const int t = live ? t0 + r / hp : t0;
+    const int h = live ? h0 + r % hp : h0;
+    const int pos = live ? positions[t] : -1;
+    int lo = a.chunk > 0 ? pos - pos % a.chunk : (a.window > 0 && pos - a.window + 1 > 0) ? pos - a.window + 1 : 0;
+    lo = live ? lo : 0;
+    const int n_first = live ? min(a.keep_first, lo) : 0;
+    const float* qrow = q + static_cast<int64_t>(t) * a.q_stride + static_cast<int64_t>(h) * D;
+    f32x4 qf[DB], acc[DB];
+#pragma unroll
+    for (int c = 0; c < DB; ++c) {
+        qf[c] = *reinterpret_cast<const f32x4*>(qrow + 16 * c + 4 * kg) * a.scale;
+        acc[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    float m = -INFINITY, l = 0.f;    // l: of this lane's keys
+
+    auto block = [&](int b, const int* bt, bool in_entry) __attribute__((always_inline)) {
+        const int key0 = 16 * b, pi = key0 / a.page_size;
+        const int page = pi < a.bt_width ? bt[pi] : -1;
+        if (page < 0 || page >= a.num_pages) return;
+        const int slot = key0 % a.page_size;
+        const int64_t pg = (static_cast<int64_t>(page) * a.nkv + kvh) * D * a.page_size;
+        const float* krow = kcache + pg + static_cast<int64_t>(slot + r) * D + 4 * kg;
+        const float* vrow = vcache + pg + static_cast<int64_t>(r) * a.page_size + slot + 4 * kg;
+        f32x4 kf[DB], vf[DB];
+#pragma unroll
+        for (int c = 0; c < DB; ++c) kf[c] = *reinterpret_cast<const f32x4*>(krow + 16 * c);
+#pragma unroll
+        for (int c = 0; c < DB; ++c) vf[c] = *reinterpret_cast<const f32x4*>(vrow + static_cast<int64_t>(16 * c) * a.page_size);
+        f32x4 s = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int c = 0; c < DB; ++c)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) s = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[c][e], qf[c][e], s, 0, 0, 0);
+        bool seen[4], all = true;
+        float top = -INFINITY;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int j = key0 + 4 * kg + e;
+            seen[e] = in_entry && j <= pos && (j >= lo || j < n_first);
+            all = all && seen[e];
+            if (a.cap > 0.f) s[e] = a.cap * tanhf(s[e] / a.cap);
+            s[e] = seen[e] ? s[e] : -INFINITY;
+            top = fmaxf(top, s[e]);
+        }
+        top = fmaxf(top, __shfl_xor(top, 16, PULSE_WAVE));
+        top = fmaxf(top, __shfl_xor(top, 32, PULSE_WAVE));
+        const float m_new = fmaxf(m, top);
+        const float alpha = m_new == -INFINITY ? 1.f : expf(m - m_new);
+        f32x4 p;
+        float sum = 0.f;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            p[e] = s[e] == -INFINITY ? 0.f : expf(s[e] - m_new);
+            sum += p[e];
+        }
+        l = l * alpha + sum;
+        m = m_new;
+#pragma unroll
+        for (int c = 0; c < DB; ++c) acc[c] *= alpha;
+        // A weight of 0 keeps an unseen key out of a row only while the key's value is finite.  Where rows differ in
+        // what they see of the block (or its slots were never written), values that are not go row by row instead.
+        const bool partly = __ballot(!all) != 0;
+        bool odd = false;
+        if (partly) {
+#pragma unroll
+            for (int c = 0; c < DB; ++c)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) odd = odd || !(fabsf(vf[c][e]) < INFINITY);
+        }
+        if (partly && __ballot(odd) != 0) {
+            for (int row = 0; row < 16; ++row) {
+                // what row `row` sees of this lane's four keys (lane 16 g + row holds it for keys 4 g + e)
+                bool sees[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) sees[e] = (__ballot(seen[e]) >> (16 * kg + row)) & 1ull;
+#pragma unroll
+                for (int c = 0; c < DB; ++c) {
+                    f32x4 one = acc[c];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        one = __builtin_amdgcn_mfma_f32_16x16x4f32(sees[e] ? vf[c][e] : 0.f, p[e], one, 0, 0, 0);
+                    if (r == row) acc[c] = one;
+                }
+            }
+        } else {
+#pragma unroll
+            for (int c = 0; c < DB; ++c)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) acc[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[c][e], p[e], acc[c], 0, 0, 0);
+        }
+    };
+
+    for (int ta = t0; ta < t_end;) {      // a tile may hold tokens of several entries: one after the other
+        const int entry = token_entry[ta];
+        int hi = -1, low = 0x7fffffff, kept = 0, tb = ta;
+        for (; tb < t_end && token_entry[tb] == entry; ++tb) {
+            const int p = positions[tb];
+            const int l0 = a.chunk > 0 ? p - p % a.chunk : (a.window > 0 && p - a.window + 1 > 0) ? p - a.window + 1 : 0;
+            hi = max(hi, p);
+            low = min(low, l0);
+            kept = max(kept, min(a.keep_first, l0));
+        }
+        const int* bt = block_table + static_cast<int64_t>(entry) * a.bt_width;
+        const bool in_entry = t >= ta && t < tb;
+        const int first = (kept + 15) / 16, from = max(low / 16, first), to = hi / 16;
+        for (int b = wave; b < first && b <= to; b += 4) block(b, bt, in_entry);
+        for (int b = from + ((wave - from) & 3); b <= to; b += 4) block(b, bt, in_entry);
+        ta = tb;
+    }
+
+    l += __shfl_xor(l, 16, PULSE_WAVE);
+    l += __shfl_xor(l, 32, PULSE_WAVE);
+    if (kg == 0) {
+        m_s[wave][r] = m;
+        l_s[wave][r] = l;
+    }
+#pragma unroll
+    for (int c = 0; c < DB; ++c) acc_s[wave][c][lane] = acc[c];
+    __syncthreads();
+    if (!live) return;
+    float top = m_s[0][r];
+#pragma unroll
+    for (int w = 1; w < 4; ++w) top = fmaxf(top, m_s[w][r]);
+    float factor[4], den = 0.f;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+        factor[w] = m_s[w][r] == -INFINITY ? 0.f : expf(m_s[w][r] - top);
+        den += l_s[w][r] * factor[w];
+    }
+    float rescale = 1.f;
+    if (sink) {      // one more term of the denominator, exp(sink[h]), with no key and no value
+        const float sk = sink[h];
+        if (top == -INFINITY) { den = 1.f; }
+        else if (sk > top) { rescale = expf(top - sk); den = den * rescale + 1.f; }
+        else den += expf(sk - top);
+    }
+    float inv = den > 0.f ? 1.0f / den : 0.f;
+    const float* grow = gate ? gate + static_cast<int64_t>(t) * gate_stride : nullptr;
+    if (grow && !a.gate_per_channel) inv *= 1.0f / (1.0f + expf(-grow[h]));
+    float* orow = out + static_cast<int64_t>(t) * a.o_stride + static_cast<int64_t>(h) * D;
+#pragma unroll
+    for (int c = 0; c < DB; ++c) {
+        if (c % 4 != wave) continue;
+        f32x4 v = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int w = 0; w < 4; ++w)
+            if (factor[w] != 0.f) v += acc_s[w][c][lane] * factor[w];
+        v *= rescale * inv;
+        const int ch = 16 * c + 4 * kg;
+        if (grow && a.gate_per_channel) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (ch + e < a.gate_width) v[e] *= 1.0f / (1.0f + expf(-grow[static_cast<int64_t>(h) * a.gate_width + ch + e]));
+        }
+        *reinterpret_cast<f32x4*>(orow + ch) = v;
+    }
+}
+
+// Whether the kernel above takes a call (everything float32, own values): what its 16-byte accesses ask for.
+bool rows_f32_takes(const AttnArgs& a, const void* q, const void* out, const void* kcache, const void* vcache) {
+    auto aligned = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
+    return (a.d == 32 || a.d == 64 || a.d == 128 || a.d == 256) && a.page_size % 16 == 0 && !a.all_values && a.nkv < 65536 &&
+           a.q_stride % 4 == 0 && a.o_stride % 4 == 0 && aligned(q) && aligned(out) && aligned(kcache) && aligned(vcache);
+}
+
+int launch_rows_f32(const void* q, void* out, const void* kcache, const void* vcache, const int* positions,
+                    const int* token_entry, const int* block_table, const void* gate, int64_t gate_stride, const float* sink,
+                    const AttnArgs& a, int tokens, hipStream_t stream) {
+    const int group = a.nq / a.nkv;
+    const int hp = group < 16 ? group : 16;
+    // Few tokens (decoding) get a tile each: their keys are those of one request or another, and more tiles fill the chip.
+    const int tp = tokens <= 64 ? 1 : 16 / hp;
+    const dim3 grid((tokens + tp - 1) / tp, a.nkv, (group + hp - 1) / hp);
+#define PULSE_ROWS_LAUNCH(DB)                                                                                            \
+    hipLaunchKernelGGL((attn_rows_f32_kernel<DB>), grid, dim3(256), 0, stream, static_cast<const float*>(q),             \
+                       static_cast<float*>(out), static_cast<const float*>(kcache), static_cast<const float*>(vcache),  \
+                       positions, token_entry, block_table, static_cast<const float*>(gate), gate_stride, sink, a, tokens, \
+                       tp, hp)
+    if (a.d == 32) PULSE_ROWS_LAUNCH(2);
+    else if (a.d == 64) PULSE_ROWS_LAUNCH(4);
+    else if (a.d == 128) PULSE_ROWS_LAUNCH(8);
+    else PULSE_ROWS_LAUNCH(16);
+#undef PULSE_ROWS_LAUNCH
+    return 0;
+}
+
 template <typename TX, typename TC, typename TO>
 int launch_generic(int acc, const void* q, void* out, const void* kcache, const void* vcache, const int* positions,
                    const int* token_entry, const int* block_table, const void* gate, int64_t gate_stride,
@@ -198,6 +425,11 @@ extern "C" int pulse_attn_generic_ex(const void* q, int64_t q_stride, void* out,
     a.page_size = page_size; a.num_pages = num_pages; a.bt_width = bt_width; a.scale = scale; a.window = window; a.chunk = chunk;
     a.cap = softcap; a.gate_per_channel = gate_width > 0 ? 1 : 0; a.gate_width = gate_width;
     a.keep_first = window > 0 ? keep_first : 0; a.all_values = all_values ? 1 : 0;
+    if (x_dtype == PULSE_F32 && c_dtype == PULSE_F32 && rows_f32_takes(a, q, out, kcache, vcache)) {
+        launch_rows_f32(q, out, kcache, vcache, positions, token_entry, block_table, gate, gate_stride, sink, a, tokens, stream);
+        PULSE_LAUNCH_CHECK("attn_generic");
+        return 0;
+    }
     const size_t lds = static_cast<size_t>(d) * sizeof(float) + PULSE_WAVE * sizeof(float) + PULSE_WAVE * sizeof(long long);
     const int acc = (width + PULSE_WAVE - 1) / PULSE_WAVE;
     PULSE_DISPATCH_DTYPE(x_dtype, TX, PULSE_DISPATCH_DTYPE(c_dtype, TC,

@@ -53,6 +53,16 @@ __device__ __forceinline__ pulse_i32x4 stream_load16(const void* p) {
     return __builtin_nontemporal_load(static_cast<const pulse_i32x4*>(p));
 }
 
+// 16 bytes a lane from memory straight into LDS: lane i's piece lands at lds_base + 16 i (a wavefront-wide address), from a
+// pointer a lane, or from `offset` bytes behind a base in scalar registers.  The compiler knows nothing of these copies, so
+// the waits for them are written out where they are used.
+__device__ __forceinline__ void load_to_lds(const void* p, uint32_t lds_base) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(lds_base), "v"(p) : "memory", "m0");
+}
+__device__ __forceinline__ void load_to_lds(const void* base, uint32_t offset, uint32_t lds_base) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(lds_base), "v"(offset), "s"(base) : "memory", "m0");
+}
+
 template <typename T> __device__ __forceinline__ float to_f32(T v);
 template <> __device__ __forceinline__ float to_f32<float>(float v) { return v; }
 template <> __device__ __forceinline__ float to_f32<bf16_t>(bf16_t v) { return bf16_to_f32(v); }

@@ -1,77 +1,313 @@
-// C[M, N] = A[M, K] * W[N, K]^T with float32 multiply-adds in a fixed order.
+// C[M, N] = A[M, K] * W[N, K]^T in float32, every output added up in an order of its own that M has no part in.
 //
-// This is the matrix product of the true 32-bit path: no matrix-core
-// instruction and no reduced-precision mode is involved, every product and sum
-// is an IEEE float32 fma.  Each output element is accumulated over k = 0..K-1 in
-// ascending order whatever M is, so a row's result does not depend on what else
-// is in the batch.  Inputs may be stored as bfloat16 (they are widened exactly).
-// (reference: cublasSgemm, src/ops/kernels/cuda/matmul_kernel.cu:70-88)
+// This is the matrix product of the true 32-bit path.  Products and sums are float32 throughout: the matrix
+// instruction is v_mfma_f32_16x16x4_f32, which multiplies and accumulates in float32 (no reduced-precision mode).
+// Inputs may be stored as bfloat16 (they are widened exactly).  (reference: cublasSgemm,
+// src/ops/kernels/cuda/matmul_kernel.cu:70-88)
+//
+// The order: K is cut into blocks of 16 and the blocks into four shares, one a wavefront of the workgroup that owns the
+// output; a share is added up block after block, and the four shares in their order.  The cut depends on K alone and
+// every shape of tile walks a share in the same way, so a row's result does not depend on what else is in the batch.
+//
+// What bounds it: the matrix cores (256 float32 operations a clock and compute unit) from about 100 rows on, the weights'
+// way from memory below.  Wavefronts that share K instead of the tile fetch nothing twice in a workgroup and walk without
+// a barrier; the next blocks are asked for before these are multiplied.  Measured, weight rows x K at a number of rows,
+// against scalar multiply-adds on a 64 x 64 tile in LDS (16 k a barrier), in us: 2,048 x 8,192 at 333 rows 830 -> 105
+// (106 TFLOP/s), 16,384 x 2,048 at 333 rows 699 -> 202 (110), 2,048 x 8,192 at 1,024 rows 271 (127), 32,000 x 2,048 at one
+// row 276 -> 55 (4.7 TB/s).  The error against 64 bits halves (K of 2,048: 8e-7 -> 4e-7): four shorter sums.
 #include "common.h"
 
 namespace {
 
-constexpr int BM = 64;
-constexpr int BN = 64;
-constexpr int BK = 16;
-constexpr int TM = 4;
-constexpr int TN = 4;
+typedef __attribute__((ext_vector_type(4))) float f32x4;
 
-template <typename TA, typename TW, typename TC>
-__global__ __launch_bounds__(256) void gemm_f32_kernel(const TA* __restrict__ A, const TW* __restrict__ W,
-                                                       TC* __restrict__ C, int M, int N, int K,
-                                                       int64_t lda, int64_t ldw, int64_t ldc) {
-    __shared__ float As[BK][BM + 4];
-    __shared__ float Ws[BK][BN + 4];
-    const int tid = threadIdx.x;
-    const int tx = tid % 16;  // column group
-    const int ty = tid / 16;  // row group
-    const int m0 = blockIdx.y * BM;
-    const int n0 = blockIdx.x * BN;
+constexpr int SHARES = 4;   // wavefronts a workgroup, each with a share of K
+constexpr int KB = 16;      // k a block: four a lane group of the matrix instruction
 
-    float acc[TM][TN];
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j) acc[i][j] = 0.f;
+struct GemmArgs {
+    const void* A;
+    const void* W;
+    void* C;
+    int c_bf16;
+    int c_wide;     // float32 results can be stored four at a time
+    int M, N, K;
+    int64_t lda, ldw, ldc;
+    int tiles_m, tiles_n;
+};
 
-    // each thread stages 4 elements of A and 4 of W per k-step: row = tid / 4, k = (tid % 4) * 4 + e
-    const int lrow = tid / 4;
-    const int lk = (tid % 4) * 4;
-
-    for (int k0 = 0; k0 < K; k0 += BK) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const int k = k0 + lk + e;
-            const int m = m0 + lrow;
-            const int n = n0 + lrow;
-            As[lk + e][lrow] = (m < M && k < K) ? to_f32<TA>(A[static_cast<int64_t>(m) * lda + k]) : 0.f;
-            Ws[lk + e][lrow] = (n < N && k < K) ? to_f32<TW>(W[static_cast<int64_t>(n) * ldw + k]) : 0.f;
+// Values k .. k + 3 of a row.  VEC: the row can be read in pieces of four, and K is a multiple of 4; a piece past the end is
+// then the row's last piece, read for nobody, so that no lane branches round a load.
+template <typename T, bool VEC>
+__device__ __forceinline__ f32x4 load4(const T* row, int k, int K) {
+    f32x4 v;
+    if constexpr (VEC) {
+        const int at = min(k, K - 4);
+        if constexpr (sizeof(T) == 4) {
+            v = *reinterpret_cast<const f32x4*>(row + at);
+        } else {
+            const uint2 raw = *reinterpret_cast<const uint2*>(row + at);
+            v[0] = __uint_as_float(raw.x << 16);
+            v[1] = __uint_as_float(raw.x & 0xffff0000u);
+            v[2] = __uint_as_float(raw.y << 16);
+            v[3] = __uint_as_float(raw.y & 0xffff0000u);
         }
+    } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = k + e < K ? to_f32<T>(row[k + e]) : 0.f;
+    }
+    return v;
+}
+
+// Four results of row m, for weight rows n .. n + 3 (a lane of the matrix instruction's result holds weight rows
+// 4 * (l / 16) + e for row l % 16 of A).
+__device__ __forceinline__ void store_tile(const GemmArgs& a, int m, int n, f32x4 v) {
+    if (m >= a.M) return;
+    const int64_t at = static_cast<int64_t>(m) * a.ldc + n;
+    if (a.c_bf16) {
+        bf16_t* c = static_cast<bf16_t*>(a.C) + at;
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            if (n + e < a.N) c[e] = f32_to_bf16(v[e]);
+    } else if (a.c_wide) {
+        if (n < a.N) *reinterpret_cast<f32x4*>(static_cast<float*>(a.C) + at) = v;
+    } else {
+        float* c = static_cast<float*>(a.C) + at;
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            if (n + e < a.N) c[e] = v[e];
+    }
+}
+
+// A workgroup's tile is 16 * BN weight rows (the row operand) by 16 * BM rows of A (the column operand); U blocks of k
+// are a stage.
+template <typename TA, typename TW, bool VEC, int BM, int BN, int U>
+__global__ __launch_bounds__(SHARES* PULSE_WAVE) void gemm_f32_kernel(GemmArgs a) {
+    constexpr int TILES = BM * BN;
+    constexpr int PASS = TILES % 8 == 0 ? 8 : TILES % 6 == 0 ? 6 : TILES % 9 == 0 ? 9 : TILES;     // tiles of the matrix instruction a pass of the meeting in LDS
+    __shared__ f32x4 meet[SHARES][PASS][PULSE_WAVE];
+
+    // (the workgroups of a die, every eighth, take neighbouring tiles: those of one span of weight rows)
+    const int total = a.tiles_m * a.tiles_n;
+    const int per_die = (total + 7) / 8;
+    const int tile = (blockIdx.x % 8) * per_die + blockIdx.x / 8;
+    if (static_cast<int>(blockIdx.x / 8) >= per_die || tile >= total) return;
+    const int m0 = tile % a.tiles_m * (16 * BM), n0 = tile / a.tiles_m * (16 * BN);
+
+    const int lane = threadIdx.x % PULSE_WAVE;
+    const int share = threadIdx.x / PULSE_WAVE;
+    const int r = lane % 16, kg = lane / 16;
+    const int blocks = (a.K + KB - 1) / KB;
+    const int b_end = static_cast<int>(static_cast<int64_t>(blocks) * (share + 1) / SHARES);
+    int b = static_cast<int>(static_cast<int64_t>(blocks) * share / SHARES);
+
+    // (rows past the end are the last row again: their results are not written)
+    const TA* arow[BM];
+    const TW* wrow[BN];
+#pragma unroll
+    for (int i = 0; i < BM; ++i)
+        arow[i] = static_cast<const TA*>(a.A) + static_cast<int64_t>(min(m0 + 16 * i + r, a.M - 1)) * a.lda;
+#pragma unroll
+    for (int j = 0; j < BN; ++j)
+        wrow[j] = static_cast<const TW*>(a.W) + static_cast<int64_t>(min(n0 + 16 * j + r, a.N - 1)) * a.ldw;
+
+    f32x4 acc[BN][BM];
+#pragma unroll
+    for (int j = 0; j < BN; ++j)
+#pragma unroll
+        for (int i = 0; i < BM; ++i) acc[j][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+    f32x4 av[2][U][BM], wv[2][U][BN];
+    auto fetch = [&](int set, int block) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int k = (block + u) * KB + 4 * kg;
+#pragma unroll
+            for (int j = 0; j < BN; ++j) wv[set][u][j] = load4<TW, VEC>(wrow[j], k, a.K);
+#pragma unroll
+            for (int i = 0; i < BM; ++i) av[set][u][i] = load4<TA, VEC>(arow[i], k, a.K);
+        }
+        __builtin_amdgcn_sched_barrier(0);   // (the loads stay ahead of the products that they hide behind)
+    };
+    auto multiply = [&](int set) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int j = 0; j < BN; ++j)
+#pragma unroll
+                    for (int i = 0; i < BM; ++i)
+                        acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[set][u][j][e], av[set][u][i][e], acc[j][i], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    // What lies behind the share's end is zeros on both sides, which leaves the sums as they are.
+    const int k_end = min(a.K, b_end * KB);
+    auto clear_behind = [&](int set, int block) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int k = (block + u) * KB + 4 * kg;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const bool in = k + e < k_end;
+#pragma unroll
+                for (int j = 0; j < BN; ++j) wv[set][u][j][e] = in ? wv[set][u][j][e] : 0.f;
+#pragma unroll
+                for (int i = 0; i < BM; ++i) av[set][u][i][e] = in ? av[set][u][i][e] : 0.f;
+            }
+        }
+    };
+    const int b_full = min(b_end, a.K / KB);    // blocks that lie inside K as a whole
+    fetch(0, b);
+    for (; b + 2 * U <= b_full; b += 2 * U) {
+        fetch(1, b + U);
+        multiply(0);
+        fetch(0, b + 2 * U);
+        multiply(1);
+    }
+    for (; b < b_end; b += 2 * U) {             // (at most twice)
+        fetch(1, b + U);
+        clear_behind(0, b);
+        multiply(0);
+        clear_behind(1, b + U);
+        multiply(1);
+        if (b + 2 * U < b_end) fetch(0, b + 2 * U);
+    }
+
+    // The shares meet in LDS, a few tiles at a time; wavefront t % 4 adds up the four results of tile t.
+#pragma unroll
+    for (int t0 = 0; t0 < TILES; t0 += PASS) {
+        if (t0 > 0) __syncthreads();
+#pragma unroll
+        for (int t = 0; t < PASS; ++t) meet[share][t][lane] = acc[(t0 + t) / BM][(t0 + t) % BM];
         __syncthreads();
 #pragma unroll
-        for (int kk = 0; kk < BK; ++kk) {
-            float a[TM], b[TN];
+        for (int t = 0; t < PASS; ++t) {
+            if (t % SHARES != share) continue;
+            f32x4 v = meet[0][t][lane];
 #pragma unroll
-            for (int i = 0; i < TM; ++i) a[i] = As[kk][ty * TM + i];
-#pragma unroll
-            for (int j = 0; j < TN; ++j) b[j] = Ws[kk][tx * TN + j];
-#pragma unroll
-            for (int i = 0; i < TM; ++i)
-#pragma unroll
-                for (int j = 0; j < TN; ++j) acc[i][j] = fmaf(a[i], b[j], acc[i][j]);
+            for (int s = 1; s < SHARES; ++s) v += meet[s][t][lane];
+            store_tile(a, m0 + 16 * ((t0 + t) % BM) + r, n0 + 16 * ((t0 + t) / BM) + 4 * kg, v);
         }
+    }
+}
+
+// The same walk for many rows of float32 operands, the operands through LDS: read straight into registers, the sixteen
+// lanes that an instruction serves together touch sixteen rows, and the compute unit's cache looks up a line for 16
+// bytes of each.  A wavefront copies its own share's blocks (16 rows x 64 bytes an instruction, four lanes a row) into
+// S stages of its own, so the walk has no barrier here either.
+template <int BM, int BN, int S>
+__global__ __launch_bounds__(SHARES* PULSE_WAVE) void gemm_f32_staged_kernel(GemmArgs a) {
+    constexpr int TILES = BM * BN;
+    constexpr int STAGE = (BM + BN) * 1024;
+    constexpr int PASS = TILES % 8 == 0 ? 8 : TILES % 6 == 0 ? 6 : TILES % 9 == 0 ? 9 : TILES;
+    constexpr int MEET = SHARES * PASS * PULSE_WAVE * 16;
+    __shared__ __attribute__((aligned(1024))) char lds[SHARES * S * STAGE > MEET ? SHARES * S * STAGE : MEET];
+
+    const int total = a.tiles_m * a.tiles_n;
+    const int per_die = (total + 7) / 8;
+    const int tile = (blockIdx.x % 8) * per_die + blockIdx.x / 8;
+    if (static_cast<int>(blockIdx.x / 8) >= per_die || tile >= total) return;
+    const int m0 = tile % a.tiles_m * (16 * BM), n0 = tile / a.tiles_m * (16 * BN);
+
+    const int lane = threadIdx.x % PULSE_WAVE;
+    const int share = __builtin_amdgcn_readfirstlane(threadIdx.x / PULSE_WAVE);
+    const int r = lane % 16, kg = lane / 16;
+    const int blocks = (a.K + KB - 1) / KB;
+    const int b_end = static_cast<int>(static_cast<int64_t>(blocks) * (share + 1) / SHARES);
+    const int b0 = static_cast<int>(static_cast<int64_t>(blocks) * share / SHARES);
+
+    // Copies: lane i brings the piece that belongs at place i % 4 of row i / 4; piece c of row q sits at place
+    // c ^ (q / 4 % 4), so that the eight lanes which LDS serves together read eight different places.
+    const int crow = lane / 4, cpiece = (lane % 4) ^ (crow / 4 % 4);
+    const float* from[BN + BM];
+#pragma unroll
+    for (int j = 0; j < BN; ++j)
+        from[j] = static_cast<const float*>(a.W) + static_cast<int64_t>(min(n0 + 16 * j + crow, a.N - 1)) * a.ldw;
+#pragma unroll
+    for (int i = 0; i < BM; ++i)
+        from[BN + i] = static_cast<const float*>(a.A) + static_cast<int64_t>(min(m0 + 16 * i + crow, a.M - 1)) * a.lda;
+    char* mine = lds + share * S * STAGE;
+    const uint32_t mine_at = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(
+        (void __attribute__((address_space(3)))*)(mine)));
+    auto copy = [&](int block, int stage) __attribute__((always_inline)) {
+        const int at = min(block * KB + 4 * cpiece, a.K - 4);    // (past the end: the row's last piece, for nobody)
+#pragma unroll
+        for (int t = 0; t < BN + BM; ++t) load_to_lds(from[t] + at, mine_at + stage * STAGE + t * 1024);
+    };
+
+    f32x4 acc[BN][BM];
+#pragma unroll
+    for (int j = 0; j < BN; ++j)
+#pragma unroll
+        for (int i = 0; i < BM; ++i) acc[j][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+    const int read_at = r * 64 + (kg ^ (r / 4 % 4)) * 16;
+    const int k_end = min(a.K, b_end * KB);
+    auto multiply = [&](int stage, int block, bool whole) __attribute__((always_inline)) {
+        f32x4 v[BN + BM];
+#pragma unroll
+        for (int t = 0; t < BN + BM; ++t) v[t] = *reinterpret_cast<const f32x4*>(mine + stage * STAGE + t * 1024 + read_at);
+        if (!whole) {    // what lies behind the share's end is zeros on both sides
+#pragma unroll
+            for (int t = 0; t < BN + BM; ++t)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[t][e] = block * KB + 4 * kg + e < k_end ? v[t][e] : 0.f;
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int j = 0; j < BN; ++j)
+#pragma unroll
+                for (int i = 0; i < BM; ++i)
+                    acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[j][e], v[BN + i][e], acc[j][i], 0, 0, 0);
+    };
+    // Block b lies in stage (b - b0) % S; S - 1 blocks are on their way while one is multiplied.
+#pragma unroll
+    for (int s = 0; s < S - 1; ++s) copy(b0 + s, s);
+    const int b_full = min(b_end, a.K / KB);
+    int stage = 0;
+    for (int b = b0; b < b_end; ++b) {
+        const int next = stage == 0 ? S - 1 : stage - 1;
+        copy(b + S - 1, next);
+        asm volatile("s_waitcnt vmcnt(%0)" : : "n"((S - 1) * (BN + BM)) : "memory");
+        multiply(stage, b, b < b_full);
+        stage = stage == S - 1 ? 0 : stage + 1;
+    }
+    asm volatile("s_waitcnt vmcnt(0)" : : : "memory");   // the last copies, which nobody reads, must not land in what follows
+    __syncthreads();
+
+    f32x4* meet = reinterpret_cast<f32x4*>(lds);          // [SHARES][PASS][64]
+#pragma unroll
+    for (int t0 = 0; t0 < TILES; t0 += PASS) {
+        if (t0 > 0) __syncthreads();
+#pragma unroll
+        for (int t = 0; t < PASS; ++t) meet[(share * PASS + t) * PULSE_WAVE + lane] = acc[(t0 + t) / BM][(t0 + t) % BM];
         __syncthreads();
-    }
 #pragma unroll
-    for (int i = 0; i < TM; ++i) {
-        const int m = m0 + ty * TM + i;
-        if (m >= M) continue;
+        for (int t = 0; t < PASS; ++t) {
+            if (t % SHARES != share) continue;
+            f32x4 v = meet[t * PULSE_WAVE + lane];
 #pragma unroll
-        for (int j = 0; j < TN; ++j) {
-            const int n = n0 + tx * TN + j;
-            if (n < N) C[static_cast<int64_t>(m) * ldc + n] = from_f32<TC>(acc[i][j]);
+            for (int s = 1; s < SHARES; ++s) v += meet[(s * PASS + t) * PULSE_WAVE + lane];
+            store_tile(a, m0 + 16 * ((t0 + t) % BM) + r, n0 + 16 * ((t0 + t) / BM) + 4 * kg, v);
         }
     }
+}
+
+template <int BM, int BN, int S>
+void launch_staged(GemmArgs a, hipStream_t stream) {
+    a.tiles_m = (a.M + 16 * BM - 1) / (16 * BM);
+    a.tiles_n = (a.N + 16 * BN - 1) / (16 * BN);
+    const unsigned grid = static_cast<unsigned>((static_cast<int64_t>(a.tiles_m) * a.tiles_n + 7) / 8 * 8);
+    hipLaunchKernelGGL((gemm_f32_staged_kernel<BM, BN, S>), dim3(grid), dim3(SHARES * PULSE_WAVE), 0, stream, a);
+}
+
+template <typename TA, typename TW, bool VEC, int BM, int BN, int U>
+void launch(GemmArgs a, hipStream_t stream) {
+    a.tiles_m = (a.M + 16 * BM - 1) / (16 * BM);
+    a.tiles_n = (a.N + 16 * BN - 1) / (16 * BN);
+    const unsigned grid = static_cast<unsigned>((static_cast<int64_t>(a.tiles_m) * a.tiles_n + 7) / 8 * 8);
+    hipLaunchKernelGGL((gemm_f32_kernel<TA, TW, VEC, BM, BN, U>), dim3(grid), dim3(SHARES * PULSE_WAVE), 0, stream, a);
 }
 
 }  // namespace
@@ -83,12 +319,43 @@ extern "C" int pulse_gemm_f32(const void* A, int a_dtype, const void* W, int w_d
     PULSE_REQUIRE(pulse_dtype_ok(a_dtype) && pulse_dtype_ok(w_dtype) && pulse_dtype_ok(c_dtype), "gemm_f32: bad dtype tag");
     PULSE_REQUIRE(A && W && C, "gemm_f32: null pointer");
     if (M == 0) return 0;
-    const unsigned gx = (N + BN - 1) / BN, gy = (M + BM - 1) / BM;
-    PULSE_REQUIRE(gy < 65536, "gemm_f32: M=%d is too large for one launch", M);
-    PULSE_DISPATCH_DTYPE(a_dtype, TA, PULSE_DISPATCH_DTYPE(w_dtype, TW, PULSE_DISPATCH_DTYPE(c_dtype, TC,
-        hipLaunchKernelGGL((gemm_f32_kernel<TA, TW, TC>), dim3(gx, gy), dim3(256), 0, stream,
-                           static_cast<const TA*>(A), static_cast<const TW*>(W), static_cast<TC*>(C), M, N, K,
-                           lda, ldw, ldc))));
+    PULSE_REQUIRE((M + 63) / 64 < 65536, "gemm_f32: M=%d is too large for one launch", M);
+    PULSE_REQUIRE(static_cast<int64_t>((M + 15) / 16) * ((N + 15) / 16) < (1ll << 30), "gemm_f32: %d x %d outputs are too many",
+                  M, N);
+    const bool wide = c_dtype == PULSE_F32 && ldc % 4 == 0 && N % 4 == 0 && reinterpret_cast<uintptr_t>(C) % 16 == 0;
+    GemmArgs a{A, W, C, c_dtype == PULSE_BF16 ? 1 : 0, wide ? 1 : 0, M, N, K, lda, ldw, ldc, 0, 0};
+    const int a_size = a_dtype == PULSE_BF16 ? 2 : 4, w_size = w_dtype == PULSE_BF16 ? 2 : 4;
+    const bool vec = K % 4 == 0 && lda % 4 == 0 && ldw % 4 == 0 && reinterpret_cast<uintptr_t>(A) % (4 * a_size) == 0 &&
+                     reinterpret_cast<uintptr_t>(W) % (4 * w_size) == 0;
+    // Up to 16 rows a product is the weights' way from memory: tiles of one block of weight rows with four blocks of k a
+    // stage, four blocks of weight rows where there are enough of them for every compute unit (16,384 x 2,048 at 12 rows
+    // 38 -> 30 us; 2,048 x 8,192 29 -> 74).
+    if (M <= 16 || !vec || a_size != 4 || w_size != 4) {
+        PULSE_DISPATCH_DTYPE(a_dtype, TA, PULSE_DISPATCH_DTYPE(w_dtype, TW,
+            if (!vec) launch<TA, TW, false, 2, 2, 1>(a, stream);
+            else if (M > 16) launch<TA, TW, true, 2, 2, 2>(a, stream);
+            else if (N >= 64 * pulse_compute_units()) launch<TA, TW, true, 1, 4, 2>(a, stream);
+            else launch<TA, TW, true, 1, 1, 4>(a, stream)));
+    } else {
+        // The tile whose fullest compute unit ends first: workgroups on it x (pairs of blocks in a tile + 2, what a
+        // workgroup costs beside its products).  Measured at 333 rows: 2,048 weight rows of 8,192 133 / 144 / 105 / 134 us
+        // with tiles of 2 x 2, 2 x 4, 3 x 4, 4 x 4 blocks, the rule's 18 / 20 / 14 / 18; 16,384 of 2,048 248 / 225 / 202 /
+        // 220 us, 132 / 110 / 98 / 108.
+        static constexpr int shapes[][2] = {{4, 4}, {3, 4}, {2, 4}, {2, 2}};
+        const int64_t units = pulse_compute_units();
+        int best = 0;
+        int64_t least = 0;
+        for (int i = 0; i < 4; ++i) {
+            const int64_t tiles = static_cast<int64_t>((M + 16 * shapes[i][0] - 1) / (16 * shapes[i][0])) *
+                                  ((N + 16 * shapes[i][1] - 1) / (16 * shapes[i][1]));
+            const int64_t cost = (tiles + units - 1) / units * (shapes[i][0] * shapes[i][1] + 2);
+            if (i == 0 || cost < least) { best = i; least = cost; }
+        }
+        if (best == 0) launch_staged<4, 4, 3>(a, stream);
+        else if (best == 1) launch_staged<3, 4, 3>(a, stream);
+        else if (best == 2) launch_staged<2, 4, 3>(a, stream);
+        else launch_staged<2, 2, 3>(a, stream);
+    }
     PULSE_LAUNCH_CHECK("gemm_f32");
     return 0;
 }

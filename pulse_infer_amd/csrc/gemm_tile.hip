@@ -64,12 +64,6 @@ struct TileArgs {
 // (eight in a row, or sixteen) then lie in different 16-byte places of what LDS serves at once.
 __device__ __forceinline__ int swz(int row) { return (row & 7) ^ ((row >> 3) & 1); }
 
-// 16 bytes a lane from memory straight into LDS: lane i's piece, `offset` bytes behind `base`, lands at lds_base + 16 i
-// (a wavefront-wide address).  The compiler knows nothing of these copies, so the waits for them are written out below.
-__device__ __forceinline__ void load_to_lds(const void* base, uint32_t offset, uint32_t lds_base) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(lds_base), "v"(offset), "s"(base) : "memory", "m0");
-}
-
 template <int MODE>
 __global__ __launch_bounds__(NW* PULSE_WAVE) void gemm_tile_kernel(TileArgs a) {
     __shared__ __attribute__((aligned(1024))) char lds[2 * STAGE_BYTES];

@@ -1002,11 +1002,6 @@ struct WideShape {
     static_assert(KT == NW, "a wavefront copies one key tile and one value tile of every block");
 };
 
-// 16 bytes a lane from memory straight into LDS: lane i's piece lands at lds_base + 16 i (a wavefront-wide address).
-__device__ __forceinline__ void load_to_lds(const void* from, uint32_t lds_base) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(lds_base), "v"(from) : "memory", "m0");
-}
-
 #if PULSE_WIDE_CT > 2 || PULSE_HEAD_DIM > 128   // (the accumulators take most of the registers, the stages most of LDS)
 #define PULSE_WIDE_WAVES_PER_EU __attribute__((amdgpu_waves_per_eu(1, 1)))
 #else

@@ -247,7 +247,7 @@ def gather_rows(src: torch.Tensor, rows: torch.Tensor, out: torch.Tensor) -> Non
 
 
 def gemm_f32(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor) -> None:
-    """out[M, N] = a[M, K] @ w[N, K]^T with float32 fused multiply-adds in a fixed order."""
+    """out[M, N] = a[M, K] @ w[N, K]^T in float32, every output added up in an order that the number of rows has no part in."""
     _gpu("gemm_f32", a, w, out)
     _need(a.dim() == 2 and w.dim() == 2 and out.dim() == 2, "gemm_f32: matrices are needed")
     m, k = a.shape

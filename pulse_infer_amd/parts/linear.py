@@ -10,8 +10,8 @@ Three products stand behind it:
   package's product in output tiles of 256 x 256, which can apply SwiGLU on the way
   out or leave float32 results of shares of the inner dimension (``OWN_MANY_ROWS``
   says which products go there);
-* the float32 run, and any weight kept in 32-bit: this package's own
-  fused-multiply-add kernel, with no reduced-precision mode anywhere.
+* the float32 run, and any weight kept in 32-bit: this package's own kernel on the
+  float32 matrix instruction, with no reduced-precision mode anywhere.
 """
 from __future__ import annotations
 
@@ -102,7 +102,7 @@ class Linear:
             if not self.rows_aligned(x, w):
                 # The vendor library is handed only operands whose rows keep 16-byte alignment (inner sizes that are
                 # multiples of 8, which every shape of a real model is); anything else goes through this package's
-                # fused-multiply-add product, which takes any shape and guards every access.
+                # float32 product, which takes any shape and guards every access.
                 kernels.gemm_f32(x, w, out)
                 return out
             global library_calls
