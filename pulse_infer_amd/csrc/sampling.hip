@@ -14,7 +14,7 @@
 // With top-k (or top-p alone on a peaked row) the row is read three times: the maximum, a histogram of the values
 // that locates the k-th largest, and the collection of what lies at or above its bin; the rest happens on that
 // short list in LDS.  Rows that do not fit (many equal values, a flat row under top-p alone) take passes over the
-// whole vocabulary for every bit of a threshold, with the same result.
+// whole vocabulary for their threshold, with the same result.
 // Differences, both of measure zero or none in distribution: the kept sets are
 // found as thresholds (tokens equal to the threshold are all kept), and the
 // cumulative walk runs in vocabulary order rather than sorted order.  The
@@ -44,29 +44,48 @@ struct RowView {
     const uint32_t* banned;  // bit per token, or null
     float penalty;
     int vocab;
-    // (without a branch on what was loaded: the loads of several entries can then be in flight together)
+    __device__ __forceinline__ bool masked() const { return seen != nullptr || banned != nullptr; }
+    // The value of entry i; MASKED is masked(), asked once before a loop: a branch on either pointer beside every load would
+    // have each load waited for before the next is issued.  (A row that has one of the masks reads it in both's place.)
+    template <bool MASKED>
     __device__ __forceinline__ float at(int i) const {
         const float x = logits[i];
-        const bool out = banned ? ((banned[i >> 5] >> (i & 31)) & 1u) != 0u : false;
-        const bool was = seen ? ((seen[i >> 5] >> (i & 31)) & 1u) != 0u : false;
+        if constexpr (!MASKED) return x != x ? -INFINITY : x;
+        const uint32_t bit = 1u << (i & 31);
+        const uint32_t b = (banned ? banned : seen)[i >> 5], s = (seen ? seen : banned)[i >> 5];
+        const bool out = banned != nullptr && (b & bit) != 0u, was = seen != nullptr && (s & bit) != 0u;
         return (out || x != x) ? -INFINITY : (was ? x - penalty : x);
     }
 };
 
-// f(i, value) for i = first, first + step, .. below end, in that order; the values of eight entries are asked for
-// before the first is used (a workgroup alone on its row otherwise waits out a trip to memory for every entry).
+template <bool V>
+struct Is { static constexpr bool value = V; };
+
+// f(Is<row.masked()>)
+template <typename F>
+__device__ __forceinline__ void by_mask(const RowView& row, F f) {
+    if (row.masked()) f(Is<true>());
+    else f(Is<false>());
+}
+
+// f(i, value) for i = first, first + step, .. below end, in that order; the values of AHEAD entries are asked for
+// before the first is used (a workgroup alone on its row otherwise waits out a trip to memory for every entry).  32 rows of
+// 151,936 with all options among them: 565 us with the masks' branches beside every load, 503 without.
 template <typename F>
 __device__ __forceinline__ void sweep(const RowView& row, int first, int end, int step, F f) {
-    constexpr int AHEAD = 8;
-    int i = first;
-    for (; i + (AHEAD - 1) * step < end; i += AHEAD * step) {
-        float x[AHEAD];
+    by_mask(row, [&](auto masked) __attribute__((always_inline)) {
+        constexpr bool MASKED = decltype(masked)::value;
+        constexpr int AHEAD = MASKED ? 8 : 16;
+        int i = first;
+        for (; i + (AHEAD - 1) * step < end; i += AHEAD * step) {
+            float x[AHEAD];
 #pragma unroll
-        for (int u = 0; u < AHEAD; ++u) x[u] = row.at(i + u * step);
+            for (int u = 0; u < AHEAD; ++u) x[u] = row.at<MASKED>(i + u * step);
 #pragma unroll
-        for (int u = 0; u < AHEAD; ++u) f(i + u * step, x[u]);
-    }
-    for (; i < end; i += step) f(i, row.at(i));
+            for (int u = 0; u < AHEAD; ++u) f(i + u * step, x[u]);
+        }
+        for (; i < end; i += step) f(i, row.at<MASKED>(i));
+    });
 }
 
 __device__ float block_sum_f(float v, float* scratch) { return block_sum(v, scratch); }
@@ -229,14 +248,135 @@ __device__ bool finish_on_list(const int* list_i, float* list_x, int n, bool by_
     return true;
 }
 
+// What the kernels in front of sample_kernel leave of a row that the chunks could not choose for: the histogram's counts and
+// masses, then the mass of each of sample_kernel's wavefronts (as it would sum it) and the smallest number of each.
+constexpr int REST_MASS = 2 * HIST_BINS, REST_LOWEST = REST_MASS + SAMPLE_WAVES;
+constexpr int REST_WORDS = REST_LOWEST + SAMPLE_WAVES;
+
+__device__ __forceinline__ void add_in_group(float* p, float v) {
+    __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
+constexpr int CANDIDATES = 15;   // thresholds whose masses are summed side by side in a pass
+
+// The largest threshold t with M(t) >= want (see sample_kernel), from the histogram of a row under top-p alone; false where
+// the bracket does not hold it (or too many tokens share the bins), and then nothing is said.  Called by a whole workgroup.
+__device__ bool nucleus_edge(const RowView& row, float want, float best, float inv_t, float scale, const int* hist,
+                             const float* hist_w, float* sf, int* si, int* list_i, float* list_x, uint32_t* cand,
+                             unsigned long long* nearest, uint32_t& thr) {
+    const int lane = threadIdx.x % PULSE_WAVE, wave = threadIdx.x / PULSE_WAVE;
+    // the first bin at which the masses from the top reach `want`: thread t sums bins 2 t and 2 t + 1
+    constexpr int PER = HIST_BINS / SAMPLE_THREADS;
+    static_assert(PER == 2, "two bins a thread");
+    const float w0 = hist_w[2 * threadIdx.x], w1 = hist_w[2 * threadIdx.x + 1];
+    float pre = w0 + w1;
+#pragma unroll
+    for (int off = 1; off < PULSE_WAVE; off <<= 1) {
+        const float up = __shfl_up(pre, off, PULSE_WAVE);
+        if (lane >= off) pre += up;
+    }
+    __syncthreads();
+    if (lane == PULSE_WAVE - 1) sf[wave] = pre;
+    if (threadIdx.x == 0) { si[0] = HIST_BINS; si[1] = 0; *nearest = ~0ull; }
+    if (threadIdx.x < CANDIDATES) cand[threadIdx.x] = 0u;
+    __syncthreads();
+    float before = 0.f;
+    for (int w = 0; w < wave; ++w) before += sf[w];
+    const float through1 = before + pre, through0 = through1 - w1;     // masses through this thread's bins
+    if (through0 >= want) atomicMin(&si[0], 2 * static_cast<int>(threadIdx.x));
+    else if (through1 >= want) atomicMin(&si[0], 2 * static_cast<int>(threadIdx.x) + 1);
+    __syncthreads();
+    const int at = si[0];
+    if (at >= HIST_BINS) return false;
+    const int b0 = max(0, at - 1), b1 = min(HIST_BINS - 1, at + 1);
+    int count = 0;
+    for (int b = b0; b <= b1; ++b) count += hist[b];
+    if (count > LIST_CAP) return false;
+    float mine = 0.f;
+    for (int b = threadIdx.x; b < b0; b += SAMPLE_THREADS) mine += hist_w[b];
+    const float base = block_sum_f(mine, sf);       // the mass above the three bins
+    // their tokens, in any order: keys and weights
+    sweep(row, threadIdx.x, row.vocab, SAMPLE_THREADS, [&](int, float x) {
+        if (x == -INFINITY) return;
+        const int b = min(HIST_BINS - 1, static_cast<int>((best - x) * scale));
+        if (b < b0 || b > b1) return;
+        const int e = atomicAdd(&si[1], 1);
+        if (e < LIST_CAP) {
+            list_i[e] = static_cast<int>(order_key(x));
+            list_x[e] = expf((x - best) * inv_t);
+        }
+    });
+    __syncthreads();
+    const int n = si[1];
+    if (n > LIST_CAP || n == 0) return false;
+    // every token's place among them and the mass through it; of those that reach `want`, the one placed first
+    int place[LIST_CAP / SAMPLE_THREADS];
+    uint32_t keys[LIST_CAP / SAMPLE_THREADS];
+#pragma unroll
+    for (int u = 0; u < LIST_CAP / SAMPLE_THREADS; ++u) {
+        const int e = threadIdx.x + u * SAMPLE_THREADS;
+        place[u] = -1;
+        keys[u] = 0u;
+        if (e >= n) continue;
+        const uint32_t key = static_cast<uint32_t>(list_i[e]);
+        float through = base;
+        int higher = 0;
+        for (int j = 0; j < n; ++j) {
+            const uint32_t other = static_cast<uint32_t>(list_i[j]);
+            through += other >= key ? list_x[j] : 0.f;
+            higher += other > key ? 1 : 0;
+        }
+        place[u] = higher;
+        keys[u] = key;
+        if (through >= want) atomicMin(nearest, static_cast<unsigned long long>(higher));
+    }
+    __syncthreads();
+    if (*nearest == ~0ull) return false;
+    const int first = static_cast<int>(*nearest) - CANDIDATES / 2;
+#pragma unroll
+    for (int u = 0; u < LIST_CAP / SAMPLE_THREADS; ++u)
+        if (place[u] >= first && place[u] >= 0 && place[u] < first + CANDIDATES) cand[place[u] - first] = keys[u];
+    __syncthreads();
+    // M at the candidates (equal tokens share a place, and the places behind it stay empty: 0)
+    uint32_t t[CANDIDATES], least = 0xffffffffu;
+    float above[CANDIDATES];
+#pragma unroll
+    for (int j = 0; j < CANDIDATES; ++j) {
+        t[j] = cand[j];
+        above[j] = 0.f;
+        if (t[j] != 0u && t[j] < least) least = t[j];
+    }
+    sweep(row, threadIdx.x, row.vocab, SAMPLE_THREADS, [&](int, float x) {
+        if (x == -INFINITY) return;
+        const uint32_t key = order_key(x);
+        if (key < least) return;
+        const float w = expf((x - best) * inv_t);
+#pragma unroll
+        for (int j = 0; j < CANDIDATES; ++j)
+            if (key >= t[j]) above[j] += w;
+    });
+    bool below = false, found = false;      // a larger candidate's mass falls short; the first that does not is known
+#pragma unroll
+    for (int j = 0; j < CANDIDATES; ++j) {
+        const float m = block_sum_f(above[j], sf);
+        if (t[j] == 0u || found) continue;
+        if (m < want) below = true;
+        else if (below) { found = true; thr = t[j]; }
+        else return false;                  // (the same for every thread)
+    }
+    return found;
+}
+
 __global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
     const float* __restrict__ logits, int vocab, int64_t row_stride, const float* __restrict__ temperature,
     const int* __restrict__ top_k, const float* __restrict__ top_p, const float* __restrict__ uniform,
     const float* __restrict__ penalty, const int* __restrict__ seen_row, const uint32_t* __restrict__ seen_masks,
-    const uint32_t* __restrict__ banned, int mask_words, int* __restrict__ out, const int* __restrict__ done) {
+    const uint32_t* __restrict__ banned, int mask_words, int* __restrict__ out, const int* __restrict__ done,
+    const float* __restrict__ part_max, const int* __restrict__ part_idx, int chunks, const int* __restrict__ rest) {
     __shared__ float sf[SAMPLE_WAVES];
     __shared__ int si[SAMPLE_WAVES];
     __shared__ int hist[HIST_BINS];
+    __shared__ float hist_w[HIST_BINS];     // top-p alone: the bins' masses (in the order of arrival: good for a bracket)
     if (done && done[blockIdx.x]) return;   // the kernels that work in chunks have chosen this row's token already
     __shared__ int wave_bins[SAMPLE_WAVES];
     __shared__ int region_i[SAMPLE_WAVES][WAVE_CAP];
@@ -246,6 +386,8 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
     __shared__ float list_x[LIST_CAP];
     __shared__ float part_sum[SAMPLE_WAVES];
     __shared__ int list_done;
+    __shared__ uint32_t cand[CANDIDATES];
+    __shared__ unsigned long long nearest;
 
     const int r = blockIdx.x;
     const int lane = threadIdx.x % PULSE_WAVE, wave = threadIdx.x / PULSE_WAVE;
@@ -257,13 +399,21 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
     row.seen = (seen_masks && seen_row && seen_row[r] >= 0 && row.penalty > 0.f)
                    ? seen_masks + static_cast<int64_t>(seen_row[r]) * mask_words : nullptr;
 
-    // largest logit, lowest index among equals; the smallest number too (the histogram's range)
+    // largest logit, lowest index among equals (from the chunks' where the kernels before left them); the smallest number
+    // too (the histogram's range), here or with the mass below
     float best = -INFINITY, lowest = INFINITY;
     int best_i = 0x7fffffff;
-    sweep(row, threadIdx.x, vocab, SAMPLE_THREADS, [&](int i, float x) {
-        if (x > best) { best = x; best_i = i; }
-        if (x != -INFINITY) lowest = fminf(lowest, x);
-    });
+    if (part_max) {
+        for (int c = threadIdx.x; c < chunks; c += SAMPLE_THREADS) {
+            const float v = part_max[static_cast<int64_t>(r) * chunks + c];
+            const int i = part_idx[static_cast<int64_t>(r) * chunks + c];
+            if (v > best || (v == best && i < best_i)) { best = v; best_i = i; }
+        }
+    } else {
+        sweep(row, threadIdx.x, vocab, SAMPLE_THREADS, [&](int i, float x) {
+            if (x > best) { best = x; best_i = i; }
+        });
+    }
     block_argmax(best, best_i, sf, si);
     if (best_i == 0x7fffffff) {  // everything banned or NaN
         if (threadIdx.x == 0) out[r] = -1;
@@ -289,14 +439,23 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
     constexpr int LIST_TRY = 1024;
     const bool by_k = k > 0 && k < vocab;
     const int k_list = by_k ? k : min(vocab - 1, LIST_TRY);
+    float whole = 0.f;   // without top-k: the mass of the whole vocabulary, which top_p refers to
+    float bin_scale = 0.f;
     if (by_k || (use_p && k_list > 0)) {
-        float whole = 0.f;   // without top-k: the mass of the whole vocabulary, which top_p refers to
-        if (!by_k) {
+        if (rest) {      // (the kernels before have been over the row for both, and for the histogram)
+            rest += static_cast<int64_t>(r) * REST_WORDS;
+            for (int w = 0; w < SAMPLE_WAVES; ++w) whole += __int_as_float(rest[REST_MASS + w]);
+            lowest = __int_as_float(rest[REST_LOWEST + threadIdx.x % SAMPLE_WAVES]);
+        } else if (!by_k) {
             float mass = 0.f;
             sweep(row, threadIdx.x, vocab, SAMPLE_THREADS, [&](int, float x) {
-                if (x != -INFINITY) mass += expf((x - best) * inv_t);
+                if (x != -INFINITY) { mass += expf((x - best) * inv_t); lowest = fminf(lowest, x); }
             });
             whole = block_sum_f(mass, sf);
+        } else {
+            sweep(row, threadIdx.x, vocab, SAMPLE_THREADS, [&](int, float x) {
+                if (x != -INFINITY) lowest = fminf(lowest, x);
+            });
         }
         lowest = -block_max_f(-lowest, sf);
         const float scale = static_cast<float>(HIST_BINS) / (best - lowest);
@@ -304,12 +463,22 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
         auto bin_of = [&](float x) { return min(HIST_BINS - 1, static_cast<int>((best - x) * scale)); };  // 0: the largest values
         int edge = -1, listed = 0;
         if (ranged) {
-            for (int b = threadIdx.x; b < HIST_BINS; b += SAMPLE_THREADS) hist[b] = 0;
+            for (int b = threadIdx.x; b < HIST_BINS; b += SAMPLE_THREADS) {
+                hist[b] = rest ? rest[b] : 0;
+                hist_w[b] = rest ? __int_as_float(rest[HIST_BINS + b]) : 0.f;
+            }
             __syncthreads();
-            sweep(row, threadIdx.x, vocab, SAMPLE_THREADS, [&](int, float x) {
-                if (x != -INFINITY) atomicAdd(&hist[bin_of(x)], 1);
-            });
-            __syncthreads();
+            if (!rest) {
+                sweep(row, threadIdx.x, vocab, SAMPLE_THREADS, [&](int, float x) {
+                    if (x != -INFINITY) {
+                        const int b = bin_of(x);
+                        atomicAdd(&hist[b], 1);
+                        if (!by_k) add_in_group(&hist_w[b], expf((x - best) * inv_t));
+                    }
+                });
+                __syncthreads();
+            }
+            if (!by_k) bin_scale = scale;
             // the bin in which the count from the top reaches k: first by wavefronts' shares of the bins, then by bins
             constexpr int SHARE = HIST_BINS / SAMPLE_WAVES;
             int mine = 0;
@@ -327,15 +496,22 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
                 edge = b;
             }
         }
-        if (edge >= 0 && listed <= LIST_CAP) {
+        bool may_hold = true;    // whether the list can hold top_p of the row (its mass is known to a thousandth at least)
+        if (!by_k && edge >= 0) {
+            float above = 0.f;
+            for (int b = threadIdx.x; b <= edge; b += SAMPLE_THREADS) above += hist_w[b];
+            may_hold = block_sum_f(above, sf) >= 0.999f * p * whole;
+        }
+        if (edge >= 0 && listed <= LIST_CAP && may_hold) {
             int count = 0;
+            by_mask(row, [&](auto masked) __attribute__((always_inline)) {
             constexpr int AHEAD = 8;   // steps of 64 entries whose values are asked for together
             for (int base = part_begin; base < part_end; base += AHEAD * PULSE_WAVE) {
                 float xs[AHEAD];
 #pragma unroll
                 for (int u = 0; u < AHEAD; ++u) {
                     const int i = base + u * PULSE_WAVE + lane;
-                    xs[u] = i < part_end ? row.at(i) : -INFINITY;
+                    xs[u] = i < part_end ? row.at<decltype(masked)::value>(i) : -INFINITY;
                 }
 #pragma unroll
                 for (int u = 0; u < AHEAD; ++u) {
@@ -348,6 +524,7 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
                     count += __builtin_popcountll(mask);
                 }
             }
+            });
             if (lane == 0) region_n[wave] = count;
             __syncthreads();
             bool fits = true;
@@ -366,8 +543,10 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
                 // the first wavefront finishes alone (lane l holds entries l, l + 64, ..); the others wait for its word
                 if (wave == 0) {
                     int token;
-                    const bool enough = finish_on_list<LIST_PER_LANE>(list_i, list_x, n, by_k, k, use_p, p, whole, best, inv_t, uniform[r],
-                                                       best_i, token);
+                    const bool enough = n <= 8 * PULSE_WAVE
+                        ? finish_on_list<8>(list_i, list_x, n, by_k, k, use_p, p, whole, best, inv_t, uniform[r], best_i, token)
+                        : finish_on_list<LIST_PER_LANE>(list_i, list_x, n, by_k, k, use_p, p, whole, best, inv_t, uniform[r],
+                                                        best_i, token);
                     if (lane == 0) {
                         if (enough) out[r] = token;   // else (only without top-k) the list is too short: the passes
                         list_done = enough ? 1 : 0;   // over the whole vocabulary
@@ -391,16 +570,29 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
         }
     }
     auto weight_of = [&](float x) { return (x != -INFINITY && order_key(x) >= keep) ? expf((x - best) * inv_t) : 0.f; };
-    auto weight = [&](int i) { return weight_of(row.at(i)); };
     if (use_p) {
-        float mass = 0.f;
-        sweep(row, threadIdx.x, vocab, SAMPLE_THREADS, [&](int, float x) { mass += weight_of(x); });
-        const float want = p * block_sum_f(mass, sf);
-        // The largest threshold whose kept mass still reaches `want`, four bits of it a pass over the row: the masses
+        // M(t), the mass at or above a threshold t as this kernel sums it (every thread its entries in their order, then the
+        // threads): no larger for a larger t, so the largest t with M(t) >= want is one value however it is looked for.
+        uint32_t thr = 0u;
+        bool found = false;
+        float want;
+        if (!by_k && bin_scale > 0.f) {
+            // Top-p alone: the histogram's masses say near which token the sum reaches `want`; the tokens of that bin and
+            // its neighbours are ranked, and M is summed, in its own order, for the fifteen round that place side by side.
+            // (A search for the threshold's bits, four a pass, takes eight such passes.  32 rows of 151,936, this kernel:
+            // 661 us with the search, 377 with this, 158 with the mass and the histogram made by the kernels in front.)
+            want = p * whole;
+            found = nucleus_edge(row, want, best, inv_t, bin_scale, hist, hist_w, sf, si, list_i, list_x, cand, &nearest, thr);
+        } else {
+            float mass = 0.f;
+            sweep(row, threadIdx.x, vocab, SAMPLE_THREADS, [&](int, float x) { mass += weight_of(x); });
+            want = p * block_sum_f(mass, sf);
+        }
+        // Else the largest threshold whose kept mass still reaches `want`, four bits of it a pass over the row: the masses
         // above the fifteen candidates of a digit are summed side by side (each in the order in which a pass for it
         // alone would sum it, so the choice is that of a search bit by bit, in an eighth of the passes).
-        uint32_t thr = 0u;
-        for (int shift = 28; shift >= 0; shift -= 4) {
+        if (!found) thr = 0u;
+        for (int shift = 28; shift >= 0 && !found; shift -= 4) {
             float above[15];
 #pragma unroll
             for (int j = 0; j < 15; ++j) above[j] = 0.f;
@@ -445,8 +637,11 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
         run = INFINITY;
     }
     if (wave != who) return;
-    int last;
-    const int e = wave_walk(part_begin, part_end, run == INFINITY ? INFINITY : target - run, weight, last);
+    int last, e;
+    by_mask(row, [&](auto masked) __attribute__((always_inline)) {
+        e = wave_walk(part_begin, part_end, run == INFINITY ? INFINITY : target - run,
+                      [&](int i) { return weight_of(row.at<decltype(masked)::value>(i)); }, last);
+    });
     if (lane == 0) out[r] = e >= 0 ? e : (last >= 0 ? last : best_i);
 }
 
@@ -653,11 +848,13 @@ __global__ __launch_bounds__(SIMPLE_THREADS) void topk_collect_kernel(
     const RowView row = simple_row(logits, r, row_stride, vocab, penalty, seen_row, seen_masks, banned, mask_words);
     const int begin = chunk * SIMPLE_CHUNK + static_cast<int>(threadIdx.x) * PER;
     float xs[PER];
+    by_mask(row, [&](auto masked) __attribute__((always_inline)) {
 #pragma unroll
-    for (int j = 0; j < PER; ++j) {
-        const int i = begin + j;
-        xs[j] = i < vocab ? row.at(i) : -INFINITY;
-    }
+        for (int j = 0; j < PER; ++j) {
+            const int i = begin + j;
+            xs[j] = i < vocab ? row.at<decltype(masked)::value>(i) : -INFINITY;
+        }
+    });
     // the k-th largest of the chunks' maxima, bit by bit (chunks <= 2 * 64: two a lane)
     if (wave == 0) {
         uint32_t keys[2];
@@ -826,12 +1023,89 @@ __global__ __launch_bounds__(PULSE_WAVE) void chunked_choose_kernel(
     }
     const RowView row = simple_row(logits, r, row_stride, vocab, penalty, seen_row, seen_masks, banned, mask_words);
     const int begin = who * SIMPLE_CHUNK, end = min(vocab, begin + SIMPLE_CHUNK);
-    int last;
-    const int e = wave_walk(begin, end, rest, [&](int i) {
-        const float x = row.at(i);
-        return x != -INFINITY ? expf((x - best) * inv_t) : 0.f;
-    }, last);
+    int last, e;
+    by_mask(row, [&](auto masked) __attribute__((always_inline)) {
+        e = wave_walk(begin, end, rest, [&](int i) {
+            const float x = row.at<decltype(masked)::value>(i);
+            return x != -INFINITY ? expf((x - best) * inv_t) : 0.f;
+        }, last);
+    });
     if (lane == 0) { out[r] = e >= 0 ? e : (last >= 0 ? last : best_i); done[r] = 1; }
+}
+
+// ---- the rows that are left, before sample_kernel ---------------------------------------------------------------
+// A workgroup a row goes over its row at the rate of one compute unit; of what sample_kernel needs to know of the whole row,
+// the mass (a wavefront of it summed by a wavefront here, entries and order as there), the smallest number and the
+// histogram are made by as many workgroups as there are wavefronts in it, and by eight: 17 and 30 us for 13 rows of 151,936,
+// where the passes inside sample_kernel took 220.
+__global__ __launch_bounds__(PULSE_WAVE) void rest_mass_kernel(
+    const float* __restrict__ logits, int vocab, int64_t row_stride, const float* __restrict__ temperature,
+    const int* __restrict__ top_k, const float* __restrict__ penalty, const int* __restrict__ seen_row,
+    const uint32_t* __restrict__ seen_masks, const uint32_t* __restrict__ banned, int mask_words,
+    const float* __restrict__ part_max, int chunks, const int* __restrict__ done, int* __restrict__ rest) {
+    const int r = blockIdx.y, wave = blockIdx.x, lane = threadIdx.x;
+    if (done[r]) return;
+    rest += static_cast<int64_t>(r) * REST_WORDS;
+    constexpr int SLICE = 2 * HIST_BINS / SAMPLE_WAVES;
+    for (int b = lane; b < SLICE; b += PULSE_WAVE) rest[wave * SLICE + b] = 0;
+    const float best = simple_row_max(part_max + static_cast<int64_t>(r) * chunks, chunks);
+    const float inv_t = 1.0f / temperature[r];
+    const int k = top_k ? top_k[r] : 0;
+    const RowView row = simple_row(logits, r, row_stride, vocab, penalty, seen_row, seen_masks, banned, mask_words);
+    float mass = 0.f, lowest = INFINITY;
+    if (k > 0 && k < vocab) {
+        sweep(row, wave * PULSE_WAVE + lane, vocab, SAMPLE_THREADS, [&](int, float x) {
+            if (x != -INFINITY) lowest = fminf(lowest, x);
+        });
+    } else {
+        sweep(row, wave * PULSE_WAVE + lane, vocab, SAMPLE_THREADS, [&](int, float x) {
+            if (x != -INFINITY) { mass += expf((x - best) * inv_t); lowest = fminf(lowest, x); }
+        });
+    }
+    mass = wave_sum(mass);
+    lowest = -wave_max(-lowest);
+    if (lane == 0) {
+        rest[REST_MASS + wave] = __float_as_int(mass);
+        rest[REST_LOWEST + wave] = __float_as_int(lowest);
+    }
+}
+
+constexpr int REST_GROUPS = 8;
+
+__global__ __launch_bounds__(SIMPLE_THREADS) void rest_histogram_kernel(
+    const float* __restrict__ logits, int vocab, int64_t row_stride, const float* __restrict__ temperature,
+    const int* __restrict__ top_k, const float* __restrict__ penalty, const int* __restrict__ seen_row,
+    const uint32_t* __restrict__ seen_masks, const uint32_t* __restrict__ banned, int mask_words,
+    const float* __restrict__ part_max, int chunks, const int* __restrict__ done, int* __restrict__ rest) {
+    __shared__ int hist[HIST_BINS];
+    __shared__ float hist_w[HIST_BINS];
+    const int r = blockIdx.y;
+    if (done[r]) return;
+    rest += static_cast<int64_t>(r) * REST_WORDS;
+    for (int b = threadIdx.x; b < HIST_BINS; b += SIMPLE_THREADS) { hist[b] = 0; hist_w[b] = 0.f; }
+    const float best = simple_row_max(part_max + static_cast<int64_t>(r) * chunks, chunks);
+    float lowest = INFINITY;
+    for (int w = 0; w < SAMPLE_WAVES; ++w) lowest = fminf(lowest, __int_as_float(rest[REST_LOWEST + w]));
+    const float inv_t = 1.0f / temperature[r];
+    const int k = top_k ? top_k[r] : 0;
+    const bool by_k = k > 0 && k < vocab;
+    const float scale = static_cast<float>(HIST_BINS) / (best - lowest);
+    __syncthreads();
+    if (!(best > lowest && scale < INFINITY)) return;    // (as sample_kernel: no histogram)
+    const RowView row = simple_row(logits, r, row_stride, vocab, penalty, seen_row, seen_masks, banned, mask_words);
+    sweep(row, blockIdx.x * SIMPLE_THREADS + threadIdx.x, vocab, REST_GROUPS * SIMPLE_THREADS, [&](int, float x) {
+        if (x != -INFINITY) {
+            const int b = min(HIST_BINS - 1, static_cast<int>((best - x) * scale));
+            atomicAdd(&hist[b], 1);
+            if (!by_k) add_in_group(&hist_w[b], expf((x - best) * inv_t));
+        }
+    });
+    __syncthreads();
+    for (int b = threadIdx.x; b < HIST_BINS; b += SIMPLE_THREADS) {
+        if (hist[b] == 0) continue;
+        atomicAdd(&rest[b], hist[b]);
+        if (!by_k) unsafeAtomicAdd(reinterpret_cast<float*>(rest) + HIST_BINS + b, hist_w[b]);
+    }
 }
 
 }  // namespace
@@ -920,7 +1194,8 @@ extern "C" int pulse_sample(const float* logits, int rows, int vocab, int64_t ro
     if (rows == 0) return 0;
     hipLaunchKernelGGL(sample_kernel, dim3(rows), dim3(SAMPLE_THREADS), 0, stream, logits, vocab, row_stride,
                        temperature, top_k, top_p, uniform, penalty, seen_row, seen_masks, banned, mask_words, out,
-                       static_cast<const int*>(nullptr));
+                       static_cast<const int*>(nullptr), static_cast<const float*>(nullptr),
+                       static_cast<const int*>(nullptr), 0, static_cast<const int*>(nullptr));
     PULSE_LAUNCH_CHECK("sample");
     return 0;
 }
@@ -933,7 +1208,8 @@ extern "C" int pulse_sample(const float* logits, int rows, int vocab, int64_t ro
 // them, which skips the rows that are done.  What a row's choice is does not depend on the
 // other rows.  Scratch, with chunks = pulse_sample_chunks(vocab): part_max, part_mass (float32), part_idx, seg_n
 // (int32) of rows * chunks entries; seg_i (int32), seg_x (float32) of rows * chunks * pulse_sample_segment()
-// entries; done (int32) of rows entries.
+// entries; done (int32) of rows entries; rest (int32) of rows * pulse_sample_rest() entries.
+extern "C" int pulse_sample_rest() { return REST_WORDS; }
 extern "C" int pulse_sample_chunks(int vocab) { return (vocab + SIMPLE_CHUNK - 1) / SIMPLE_CHUNK; }
 extern "C" int pulse_sample_segment() { return TOPK_SEGMENT; }
 
@@ -941,10 +1217,10 @@ extern "C" int pulse_sample_chunked(const float* logits, int rows, int vocab, in
                                     const int* top_k, const float* top_p, const float* uniform, const float* penalty,
                                     const int* seen_row, const uint32_t* seen_masks, const uint32_t* banned,
                                     int mask_words, float* part_max, int* part_idx, float* part_mass, int* seg_i,
-                                    float* seg_x, int* seg_n, int* done, int* out, hipStream_t stream) {
+                                    float* seg_x, int* seg_n, int* done, int* rest, int* out, hipStream_t stream) {
     PULSE_REQUIRE(rows >= 0 && vocab > 0 && row_stride >= vocab, "sample_chunked: bad sizes rows=%d V=%d", rows, vocab);
     PULSE_REQUIRE(rows < 65536, "sample_chunked: at most 65535 rows");
-    PULSE_REQUIRE(logits && out && part_max && part_idx && part_mass && seg_i && seg_x && seg_n && done,
+    PULSE_REQUIRE(logits && out && part_max && part_idx && part_mass && seg_i && seg_x && seg_n && done && rest,
                   "sample_chunked: null pointer");
     PULSE_REQUIRE(!temperature || uniform, "sample_chunked: temperature sampling needs uniform numbers");
     PULSE_REQUIRE((!seen_masks && !banned) || mask_words * 32 >= vocab, "sample_chunked: masks cover %d tokens, "
@@ -971,9 +1247,17 @@ extern "C" int pulse_sample_chunked(const float* logits, int rows, int vocab, in
                        part_idx, part_mass, seg_i, seg_x, seg_n, chunks, out, done);
     PULSE_LAUNCH_CHECK("sample_chunked (choice)");
     if (temperature && (top_k || top_p)) {   // (without them every row is done)
+        hipLaunchKernelGGL(rest_mass_kernel, dim3(SAMPLE_WAVES, rows), dim3(PULSE_WAVE), 0, stream, logits, vocab, row_stride,
+                           temperature, top_k, penalty, seen_row, seen_masks, banned, mask_words, part_max, chunks,
+                           static_cast<const int*>(done), rest);
+        PULSE_LAUNCH_CHECK("sample_chunked (masses of the rest)");
+        hipLaunchKernelGGL(rest_histogram_kernel, dim3(REST_GROUPS, rows), dim3(SIMPLE_THREADS), 0, stream, logits, vocab,
+                           row_stride, temperature, top_k, penalty, seen_row, seen_masks, banned, mask_words, part_max,
+                           chunks, static_cast<const int*>(done), rest);
+        PULSE_LAUNCH_CHECK("sample_chunked (histograms of the rest)");
         hipLaunchKernelGGL(sample_kernel, dim3(rows), dim3(SAMPLE_THREADS), 0, stream, logits, vocab, row_stride,
                            temperature, top_k, top_p, uniform, penalty, seen_row, seen_masks, banned, mask_words, out,
-                           static_cast<const int*>(done));
+                           static_cast<const int*>(done), part_max, part_idx, chunks, static_cast<const int*>(rest));
         PULSE_LAUNCH_CHECK("sample_chunked (the rest)");
     }
     return 0;

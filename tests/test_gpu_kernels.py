@@ -443,6 +443,54 @@ def test_sampling_at_a_real_vocabulary(k, mode, vocab, chunked):
     assert again.item() == got[5]
 
 
+@pytest.mark.parametrize("vocab", [3, 65, 1025, 2049, 40000])
+@pytest.mark.parametrize("ties", [False, True])
+def test_top_p_alone_on_flat_rows_at_the_edges_of_the_passes(k, vocab, ties):
+    """Rows whose top-p share is no short list: the threshold comes from the ranked tokens around it (or, where too many
+    are equal, from a search), with masks and without, in chunks and a workgroup a row."""
+    rows, temp = 12, 0.9
+    gen = torch.Generator().manual_seed(vocab)
+    logits = torch.randn(rows, vocab, generator=gen) * 1.5
+    if ties:
+        logits = (logits * 4).round() / 4
+    logits[2] = 0.5                                       # one value only
+    logits[4, : vocab // 2] = float("-inf")
+    top_p = torch.linspace(0.05, 0.999, rows)
+    uniform = torch.rand(rows, generator=gen)
+    words = (vocab + 31) // 32
+    seen = torch.randint(-2 ** 31, 2 ** 31 - 1, (rows, words), generator=gen).to(torch.int32)
+    banned = torch.zeros(words, dtype=torch.int32)
+    banned[0] = 2                                         # token 1
+    seen_row = torch.tensor([i if i % 3 else -1 for i in range(rows)], dtype=torch.int32)
+    penalty = torch.where(seen_row >= 0, 0.75, 0.0)
+    dev = lambda t: t.to(DEV)
+    kw = dict(temperature=dev(torch.full((rows,), temp)), top_p=dev(top_p), uniform=dev(uniform), penalty=dev(penalty),
+              seen_row=dev(seen_row), seen_masks=dev(seen), banned=dev(banned))
+    chunked, whole = (torch.full((rows,), -9, dtype=torch.int32, device=DEV) for _ in range(2))
+    k.sample_chunked(dev(logits), chunked, _chunked_scratch(k, rows, vocab), **kw)
+    k.sample(dev(logits), whole, **kw)
+    bit = lambda mask, i: (int(mask[i >> 5]) >> (i & 31)) & 1
+    for r, (t, other) in enumerate(zip(chunked.tolist(), whole.tolist())):
+        x = logits[r].to(F64).clone()
+        if seen_row[r] >= 0:
+            x -= 0.75 * torch.tensor([bit(seen[r], i) for i in range(vocab)], dtype=F64)
+        x[1] = float("-inf")
+        w = torch.exp((x - x.max()) / temp)
+        order = torch.argsort(w, descending=True, stable=True)
+        through = torch.cumsum(w[order], 0)
+        # float32 sums of up to 40,000 terms in some order: 2e-5 of the mass; the edge may lie that far either way
+        slack = 2e-5 * float(w.sum())
+        ok = False
+        for want in (float(top_p[r]) * float(w.sum()) - slack, float(top_p[r]) * float(w.sum()) + slack):
+            edge = x[order[min(int((through < want).sum()), vocab - 1)]]
+            kept = torch.where(x >= edge, w, torch.zeros_like(w))
+            cum = torch.cumsum(kept, 0)
+            target = float(uniform[r]) * float(cum[-1])
+            ok = ok or all(float(kept[v]) > 0 and float(cum[v] - kept[v]) - slack <= target <= float(cum[v]) + slack
+                           for v in (t, other))
+        assert ok, (r, t, other)
+
+
 def _chunked_scratch(k, rows, vocab):
     scratch = k.sample_chunked_scratch(rows, vocab, DEV)
     for t in scratch.values():                             # nothing that was not written is used
