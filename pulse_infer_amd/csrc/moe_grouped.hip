@@ -7,6 +7,8 @@
 // (index >= experts) are in no tile.  Which place a pair gets among its expert's depends on the order in which the
 // threads arrive; no result depends on it, since every row of a product is computed by itself.
 //
+// pulse_moe_gate_up_grouped and pulse_moe_down_grouped run on the loop of tile_loop.h (moe_tile_kernel) where the inner
+// dimension is a multiple of 64.  Else:
 // pulse_moe_gate_up_grouped: a workgroup of four wavefronts per (tile, 64 inner columns); a wavefront owns 16 gate
 // rows and the 16 up rows beside them and walks the hidden size in steps of 32 with v_mfma_f32_16x16x32_bf16, the
 // weight rows as the row operand, up to RB blocks of 16 gathered token rows as the column operand;
@@ -17,6 +19,7 @@
 // The launches are sized by the step's shape alone (the most tiles it can have); workgroups behind the number of
 // tiles leave at once.
 #include "common.h"
+#include "tile_loop.h"
 
 #include <math.h>
 
@@ -320,6 +323,178 @@ __global__ void moe_combine_kernel(const TX* __restrict__ x, const float* __rest
     out[at] = acc;
 }
 
+// ------------------------------------------------------------------ many rows an expert
+// Tiles of 32, 64 or 128 gathered rows against WR weight rows (for gate and up: slabs of 16 gate rows and the 16 up rows
+// beside them, so that a lane holds both of an inner column), on the loop of tile_loop.h.
+//
+// What bounds it: the matrix cores for tiles of 128 rows, the weights' way from memory for an expert of few rows.  Neighbouring
+// workgroups of a die take the tiles of a panel, which share weight rows and gathered rows in that die's L2.
+struct GroupArgs {
+    const bf16_t* x;             // gate and up: [tokens, K], row pair / top; down: act [pairs, K], row pair
+    const bf16_t* w[2];          // stacked [experts, N, K]; down: the first
+    void* out;                   // act [pairs, N] bfloat16, or y [pairs, N] float32
+    const int* order;
+    const int* tile_expert;
+    const int* tile_row0;
+    const int* tile_rows;
+    const int* num_tiles;
+    const float* in_weight;
+    int K, N, top, tiles_n;
+    int act_kind;
+    float limit;
+};
+
+constexpr int GROUP_PANEL = 4;   // tiles of rows a panel of the tile order
+
+template <bool DOWN, int WR, int XR, int WN, int WM, int S>
+__global__ __launch_bounds__(256) void moe_tile_kernel(GroupArgs a) {
+    using Loop = TileLoop<WR, XR, WN, WM, S>;
+    constexpr int COLS = DOWN ? WR : WR / 2;       // output columns of a tile
+    __shared__ __attribute__((aligned(1024))) char lds[Loop::LDS];
+    __shared__ int pair_s[XR];
+    __shared__ float weight_s[XR];
+
+    const int tiles_m = *a.num_tiles, total = tiles_m * a.tiles_n;
+    const int per_die = (total + 7) / 8;
+    const int t = (blockIdx.x % 8) * per_die + blockIdx.x / 8;
+    if (static_cast<int>(blockIdx.x / 8) >= per_die || t >= total) return;
+    const int panel = t / (GROUP_PANEL * a.tiles_n);
+    const int panel_m = min(GROUP_PANEL, tiles_m - panel * GROUP_PANEL);
+    const int in_panel = t - panel * GROUP_PANEL * a.tiles_n;
+    const int tile = panel * GROUP_PANEL + in_panel % panel_m;
+    const int n0 = in_panel / panel_m * COLS;
+    const int e = a.tile_expert[tile], row0 = a.tile_row0[tile], rows = a.tile_rows[tile];
+
+    const int tid = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(tid / PULSE_WAVE);
+    const int lane = tid % PULSE_WAVE;
+    for (int i = tid; i < XR; i += 256) {
+        const int p = i < rows ? a.order[row0 + i] : -1;
+        pair_s[i] = p;
+        weight_s[i] = p >= 0 && a.in_weight ? a.in_weight[p] : 1.f;
+    }
+    __syncthreads();
+
+    // (rows past the end are the tile's first row, weight rows past the end the last one: their results are not written)
+    const bf16_t* from[Loop::PER];
+#pragma unroll
+    for (int j = 0; j < Loop::PER; ++j) {
+        const int row = (wave * Loop::PER + j) * 8 + lane / 8;
+        const int c = (lane % 8) ^ Loop::swz(row < WR ? row : row - WR);
+        if (row < WR) {
+            const int n = DOWN ? n0 + row : n0 + row / 32 * 16 + row % 16;
+            const bf16_t* w = DOWN ? a.w[0] : (row & 16) ? a.w[1] : a.w[0];
+            from[j] = w + (static_cast<int64_t>(e) * a.N + min(n, a.N - 1)) * a.K + c * 8;
+        } else {
+            const int p = max(pair_s[row - WR], 0);
+            const int from_row = DOWN ? (pair_s[row - WR] < 0 ? pair_s[0] : p) : (pair_s[row - WR] < 0 ? pair_s[0] : p) / a.top;
+            from[j] = a.x + static_cast<int64_t>(from_row) * a.K + c * 8;
+        }
+    }
+    Loop loop;
+    loop.run(from, lds, wave, lane, a.K);
+
+    // Results leave through LDS, a wavefront's 32 rows at a time, in whole 16-byte pieces of rows.
+    constexpr int TN = Loop::TN, TM = Loop::TM;
+    constexpr int WAVE_LDS = Loop::LDS / 4;
+    char* mine = lds + wave * WAVE_LDS;
+    const int wave_n = wave % WN, wave_m = wave / WN, h = lane / 32;
+    const int n_wave = n0 + wave_n * TN * (DOWN ? 32 : 16);
+#pragma unroll
+    for (int g = 0; g < TM; ++g) {
+        const int m_base = (wave_m * TM + g) * 32;
+        if (m_base >= rows) break;
+        if constexpr (!DOWN) {
+            constexpr int W_COLS = TN * 16, PITCH = W_COLS * 2 + 16;
+            static_assert(32 * PITCH <= WAVE_LDS, "a wavefront's piece of LDS holds 32 rows of its part of the tile");
+            const float wgt = weight_s[m_base + lane % 32];
+#pragma unroll
+            for (int f = 0; f < TN; ++f)
+#pragma unroll
+                for (int q = 0; q < 2; ++q) {
+                    tile_bf16x4 v;
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        // an expert that is fed weight * x: both products are linear, so the factor goes onto their results
+                        float gate = loop.acc[f][g][q * 4 + i] * wgt, up = loop.acc[f][g][8 + q * 4 + i] * wgt;
+                        if (a.act_kind == 1) {   // clamped: min(g, limit) * sigmoid(1.702 g) * (clamp(u) + 1)
+                            gate = fminf(gate, a.limit);
+                            up = fminf(fmaxf(up, -a.limit), a.limit);
+                            v[i] = (__bf16)(gate / (1.0f + expf(-1.702f * gate)) * (up + 1.0f));
+                        } else {
+                            v[i] = (__bf16)(gate / (1.0f + expf(-gate)) * up);
+                        }
+                    }
+                    *reinterpret_cast<tile_bf16x4*>(mine + (lane % 32) * PITCH + (f * 16 + q * 8 + h * 4) * 2) = v;
+                }
+            tile_wave_sync();
+            constexpr int PCS = W_COLS / 8, ROWS = PULSE_WAVE / PCS;
+#pragma unroll
+            for (int it = 0; it < 32 / ROWS; ++it) {
+                const int row = it * ROWS + lane / PCS, pc = lane % PCS;
+                const uint4 v = *reinterpret_cast<const uint4*>(mine + row * PITCH + pc * 16);
+                const int p = pair_s[m_base + row], n = n_wave + pc * 8;
+                if (p >= 0 && n < a.N)
+                    *reinterpret_cast<uint4*>(static_cast<bf16_t*>(a.out) + static_cast<int64_t>(p) * a.N + n) = v;
+            }
+            tile_wave_sync();
+        } else {
+            constexpr int FP = TN < 2 ? TN : 2;        // 32-row pieces of W a pass
+            constexpr int W_COLS = FP * 32, PITCH = W_COLS * 4 + 16;
+            static_assert(32 * PITCH <= WAVE_LDS && TN % FP == 0, "a wavefront's piece of LDS holds 32 rows of a pass");
+#pragma unroll
+            for (int f0 = 0; f0 < TN; f0 += FP) {
+#pragma unroll
+                for (int f = 0; f < FP; ++f)
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        float4 v;
+                        v.x = loop.acc[f0 + f][g][q * 4];
+                        v.y = loop.acc[f0 + f][g][q * 4 + 1];
+                        v.z = loop.acc[f0 + f][g][q * 4 + 2];
+                        v.w = loop.acc[f0 + f][g][q * 4 + 3];
+                        *reinterpret_cast<float4*>(mine + (lane % 32) * PITCH + (f * 32 + q * 8 + h * 4) * 4) = v;
+                    }
+                tile_wave_sync();
+                constexpr int PCS = W_COLS / 4, ROWS = PULSE_WAVE / PCS;
+#pragma unroll
+                for (int it = 0; it < 32 / ROWS; ++it) {
+                    const int row = it * ROWS + lane / PCS, pc = lane % PCS;
+                    const float4 v = *reinterpret_cast<const float4*>(mine + row * PITCH + pc * 16);
+                    const int p = pair_s[m_base + row], n = n_wave + f0 * 32 + pc * 4;
+                    if (p >= 0 && n < a.N)
+                        *reinterpret_cast<float4*>(static_cast<float*>(a.out) + static_cast<int64_t>(p) * a.N + n) = v;
+                }
+                tile_wave_sync();
+            }
+        }
+    }
+}
+
+template <bool DOWN, int WR, int XR, int WN, int WM, int S>
+void launch_tiles(GroupArgs a, int max_tiles, hipStream_t stream) {
+    constexpr int COLS = DOWN ? WR : WR / 2;
+    a.tiles_n = (a.N + COLS - 1) / COLS;
+    const int64_t grid = (static_cast<int64_t>(max_tiles) * a.tiles_n + 7) / 8 * 8;
+    hipLaunchKernelGGL((moe_tile_kernel<DOWN, WR, XR, WN, WM, S>), dim3(static_cast<unsigned>(grid)), dim3(256), 0, stream, a);
+}
+
+// Which shape a list's tiles take: lists of 32 rows (decoding) and of 64 are bound by the weights' way from memory, lists of
+// 128 by the matrix cores.  Measured, 16 experts of 1,536 x 4,096, 4 chosen a token, gate and up / down in us, at 8, 64, 211,
+// 400, 600, 1,024, 2,048 tokens:
+//   32 rows (weights 128, 3 stages)    79 / 28    85 / 31   109 / 43   165 / 65
+//   64 rows (weights 128, 3 stages)    79 / 28    84 / 32    89 / 39   105 / 40   150 / 60   219 / 106   359 / 195
+//   128 rows (weights 256, 3 stages)   92 / 31    97 / 34   103 / 37   105 / 39   157 / 62   146 / 99    277 / 169
+//   tiles of 256 x 256, 2 stages                                                  264 / 96   273 / 159   283 / 178
+//   as before: 32 rows, K shared out   78 / 33   110 / 57   219 / 132
+//   as before: 128 rows, X in LDS     150 / 81   150 / 81   184 / 104                        370 / 318   522 / 511
+template <bool DOWN>
+void launch_tiles_for(const GroupArgs& a, int max_tiles, int rows, hipStream_t stream) {
+    if (rows <= 32) launch_tiles<DOWN, 128, 32, 4, 1, 3>(a, max_tiles, stream);
+    else if (rows <= 64) launch_tiles<DOWN, 128, 64, 4, 1, 3>(a, max_tiles, stream);
+    else launch_tiles<DOWN, 256, 128, 2, 2, 3>(a, max_tiles, stream);
+}
+
 }  // namespace
 
 extern "C" int pulse_moe_group(const int* idx, int pairs, int experts, int tile_rows_max, int max_tiles, int* rank,
@@ -348,10 +523,17 @@ extern "C" int pulse_moe_gate_up_grouped(const void* x, const void* wg, const vo
     PULSE_REQUIRE(hidden > 0 && ff > 0 && top > 0 && max_tiles > 0, "moe_gate_up_grouped: bad sizes");
     PULSE_REQUIRE(hidden % 8 == 0 && aligned16(x) && aligned16(wg) && aligned16(wu),
                   "moe_gate_up_grouped: rows must be multiples of 8 values and 16-byte aligned");
-    PULSE_REQUIRE(tile_rows_max == 32 || tile_rows_max == 128, "moe_gate_up_grouped: tiles of 32 or 128 rows");
+    PULSE_REQUIRE(tile_rows_max == 32 || tile_rows_max == 64 || tile_rows_max == 128, "moe_gate_up_grouped: tiles of 32, 64 or 128 rows");
     PULSE_REQUIRE(x && wg && wu && order && tile_expert && tile_row0 && tile_rows && num_tiles && act,
                   "moe_gate_up_grouped: null pointer");
     PULSE_REQUIRE((ff + 15) / 16 < 65536, "moe_gate_up_grouped: an inner width of %d is too large", ff);
+    if (hidden % 64 == 0 && ff % 8 == 0 && aligned16(act)) {   // (the loop walks K in whole steps of 64; rows leave in 16-byte pieces)
+        launch_tiles_for<false>({static_cast<const bf16_t*>(x), {static_cast<const bf16_t*>(wg), static_cast<const bf16_t*>(wu)},
+                                 act, order, tile_expert, tile_row0, tile_rows, num_tiles, in_weight, hidden, ff, top, 0,
+                                 act_kind, limit}, max_tiles, tile_rows_max, stream);
+        PULSE_LAUNCH_CHECK("moe_gate_up_grouped");
+        return 0;
+    }
     const dim3 grid(max_tiles, (ff + 63) / 64);
     if (tile_rows_max == 32)
         hipLaunchKernelGGL(moe_gate_up_grouped_kernel<2>, dim3(max_tiles, (ff + 15) / 16), dim3(256), 0, stream, static_cast<const bf16_t*>(x),
@@ -371,10 +553,17 @@ extern "C" int pulse_moe_down_grouped(const void* act, const void* wd, const int
     PULSE_REQUIRE(hidden > 0 && ff > 0 && max_tiles > 0, "moe_down_grouped: bad sizes");
     PULSE_REQUIRE(ff % 8 == 0 && aligned16(act) && aligned16(wd),
                   "moe_down_grouped: rows must be multiples of 8 values and 16-byte aligned");
-    PULSE_REQUIRE(tile_rows_max == 32 || tile_rows_max == 128, "moe_down_grouped: tiles of 32 or 128 rows");
+    PULSE_REQUIRE(tile_rows_max == 32 || tile_rows_max == 64 || tile_rows_max == 128, "moe_down_grouped: tiles of 32, 64 or 128 rows");
     PULSE_REQUIRE(act && wd && order && tile_expert && tile_row0 && tile_rows && num_tiles && y,
                   "moe_down_grouped: null pointer");
     PULSE_REQUIRE((hidden + 15) / 16 < 65536, "moe_down_grouped: a width of %d is too large", hidden);
+    if (ff % 64 == 0 && hidden % 4 == 0 && aligned16(y)) {
+        launch_tiles_for<true>({static_cast<const bf16_t*>(act), {static_cast<const bf16_t*>(wd), nullptr}, y, order, tile_expert,
+                                tile_row0, tile_rows, num_tiles, nullptr, ff, hidden, 1, 0, 0, 0.f}, max_tiles, tile_rows_max,
+                               stream);
+        PULSE_LAUNCH_CHECK("moe_down_grouped");
+        return 0;
+    }
     const dim3 grid(max_tiles, (hidden + 63) / 64);
     if (tile_rows_max == 32)
         hipLaunchKernelGGL(moe_down_grouped_kernel<2>, dim3(max_tiles, (hidden + 15) / 16), dim3(256), 0, stream, static_cast<const bf16_t*>(act),

@@ -1,0 +1,110 @@
+// The loop of a matrix product on an output tile of WR weight rows x XR rows of X, bfloat16 operands, float32 sums: four
+// wavefronts, WN along the weight rows and WM along the rows of X, on v_mfma_f32_32x32x16_bf16.
+//
+// K goes in steps of 64 through S stages of LDS (the tile's rows of W, then of X, 128 bytes a row), filled straight from
+// memory; S - 1 steps are on their way while one is multiplied, and there is one barrier a step: behind it, this step's
+// stage is whole and the stage of the step before is free for the copies that go out between this step's products.  Many
+// stages are for what bounds a product of few rows, the weights' way from memory: a compute unit must have some tens of
+// kilobytes on their way all the time (6 TB/s x 2 us over 256 units: 48 KB).
+//
+// The tile of the matrix instruction is D[n][m] = W . X^T: lane l holds column m = l % 32 and rows n = 8 (i / 4) +
+// 4 (l / 32) + i % 4, i = 0 .. 15, of a 32 x 32 piece.
+#pragma once
+#include "common.h"
+
+typedef __attribute__((ext_vector_type(8))) __bf16 tile_bf16x8;
+typedef __attribute__((ext_vector_type(4))) __bf16 tile_bf16x4;
+typedef __attribute__((ext_vector_type(16))) float tile_f32x16;
+
+template <int WR, int XR, int WN, int WM, int S>
+struct TileLoop {
+    static constexpr int BK = 64;
+    static constexpr int ROW_BYTES = BK * 2;
+    static constexpr int STAGE = (WR + XR) * ROW_BYTES;
+    static constexpr int NW = WN * WM;
+    static constexpr int TN = WR / 32 / WN, TM = XR / 32 / WM;       // 32-row pieces a wavefront
+    static constexpr int CHUNKS = (WR + XR) / 8;                     // 1 KB (8 rows) each
+    static constexpr int PER = CHUNKS / NW;                          // a wavefront copies
+    static constexpr int LDS = S * STAGE;
+    static_assert(CHUNKS % NW == 0 && TN >= 1 && TM >= 1 && S >= 2, "whole chunks and pieces a wavefront");
+
+    // Piece c (16 bytes) of row r of a stage sits at place c ^ swz(r): the rows that neighbouring lanes read together then
+    // lie in different places of what LDS serves at once.
+    static __device__ __forceinline__ int swz(int row) { return (row & 7) ^ ((row >> 3) & 1); }
+
+    tile_f32x16 acc[TN][TM];
+
+    // from[j]: where this lane's 16 bytes of the wavefront's j-th chunk start in memory at k = 0; chunk j of wavefront w is
+    // chunk w * PER + j of the stage, lane i brings piece (i % 8) ^ swz(row) of its row i / 8.
+    __device__ __forceinline__ void run(const bf16_t* const (&from)[PER], char* lds, int wave, int lane, int K) {
+        const int wave_n = wave % WN, wave_m = wave / WN;
+        const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(
+            (void __attribute__((address_space(3)))*)(lds)));
+        const int steps = K / BK;
+        auto copy = [&](int step, int stage, int j) __attribute__((always_inline)) {
+            load_to_lds(from[j] + min(step, steps - 1) * BK, lds0 + stage * STAGE + (wave * PER + j) * 1024);
+        };
+        const int h = lane / 32, e = h ^ swz(lane % 32);
+        int w_at[4], x_at[4];
+#pragma unroll
+        for (int kk = 0; kk < 4; ++kk) {
+            const int place = (e ^ (kk << 1)) * 16;
+            w_at[kk] = (wave_n * TN * 32 + lane % 32) * ROW_BYTES + place;
+            x_at[kk] = (WR + wave_m * TM * 32 + lane % 32) * ROW_BYTES + place;
+        }
+#pragma unroll
+        for (int f = 0; f < TN; ++f)
+#pragma unroll
+            for (int g = 0; g < TM; ++g)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) acc[f][g][i] = 0.f;
+
+#pragma unroll
+        for (int s = 0; s < S - 1; ++s)
+#pragma unroll
+            for (int j = 0; j < PER; ++j) copy(s, s, j);
+        int stage = 0;
+        for (int s = 0; s < steps; ++s) {
+            // this wavefront's copies of this step have landed, and behind the barrier everyone's have
+            asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" : : "n"((S - 2) * PER) : "memory");
+            const char* base = lds + stage * STAGE;
+            const int into = stage == 0 ? S - 1 : stage - 1;
+            tile_bf16x8 wf[2][TN], xf[2][TM];
+            auto read = [&](int kk, int buf) __attribute__((always_inline)) {
+#pragma unroll
+                for (int g = 0; g < TM; ++g) xf[buf][g] = *reinterpret_cast<const tile_bf16x8*>(base + x_at[kk] + g * 32 * ROW_BYTES);
+#pragma unroll
+                for (int f = 0; f < TN; ++f) wf[buf][f] = *reinterpret_cast<const tile_bf16x8*>(base + w_at[kk] + f * 32 * ROW_BYTES);
+            };
+            read(0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int kk = 0; kk < 4; ++kk) {
+                if (kk < 3) read(kk + 1, (kk + 1) & 1);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int p = 0; p < TN * TM; ++p) {
+                    acc[p / TM][p % TM] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[kk & 1][p / TM], xf[kk & 1][p % TM],
+                                                                                  acc[p / TM][p % TM], 0, 0, 0);
+                    __builtin_amdgcn_sched_barrier(0);
+                    // the copies, spread evenly over the step's products
+                    constexpr int ALL = 4 * TN * TM;
+                    const int q = kk * TN * TM + p;
+#pragma unroll
+                    for (int j = q * PER / ALL; j < (q + 1) * PER / ALL; ++j) copy(s + S - 1, into, j);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+            stage = stage == S - 1 ? 0 : stage + 1;
+        }
+        // the last copies, which nobody reads, must not land in what follows
+        asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" : : : "memory");
+    }
+};
+
+// A wavefront's own order of what it writes to and reads from LDS.
+__device__ __forceinline__ void tile_wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}

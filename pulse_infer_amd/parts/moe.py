@@ -160,10 +160,9 @@ class RoutedExperts(Part):
         routed = ws.buffer("moe.out", tokens, self.hidden, torch.float32)
         later = None
         if kernels.moe_grouped_takes(x, self.w_gate, self.w_down):
-            # bfloat16: the pairs grouped by expert on the device, every expert's rows on the matrix cores; tiles of
-            # 128 rows once an expert gets about that many
+            # bfloat16: the pairs grouped by expert on the device, every expert's rows on the matrix cores
             pairs = tokens * self.top
-            rows = kernels.MOE_TILE_ROWS[1] if pairs >= 64 * self.experts else kernels.MOE_TILE_ROWS[0]
+            rows = kernels.moe_tile_rows(pairs, self.experts)
             y = ws.buffer("moe.y", pairs, self.hidden, torch.float32)
             ints = ws.buffer("moe.ints", 2 * pairs + 3 * kernels.moe_max_tiles(pairs, self.experts, rows) + 1, 1, torch.int32)
             if defer and not self.identity and self.shared_gate is None:

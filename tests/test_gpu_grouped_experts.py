@@ -1,0 +1,54 @@
+"""Experts' products grouped by expert where their tiles end."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+F64 = torch.float64
+
+
+def rnd(*shape, seed):
+    return torch.randn(shape, generator=torch.Generator().manual_seed(seed))
+
+
+# rows an expert gets: none, one, a tile of 32, 64 and 128 rows and one more and one less; widths of one step of the loop, of
+# several, with a remainder of the tile's columns, and inner widths that are no multiple of 64 (the other kernels)
+@pytest.mark.parametrize("hidden,ff", [(64, 64), (320, 192), (192, 136), (200, 64)])
+@pytest.mark.parametrize("rows", [32, 64, 128])
+@pytest.mark.parametrize("form", ["silu", "clamped_on_input"])
+def test_grouped_experts_at_the_edges_of_their_tiles(hidden, ff, rows, form):
+    from pulse_infer_amd.ops import kernels
+
+    counts = [0, 1, rows - 1, rows, rows + 1, 2 * rows + 5, 0, 17]
+    experts, pairs = len(counts), sum(counts)
+    chosen = torch.cat([torch.full((c,), e) for e, c in enumerate(counts)])
+    chosen = chosen[torch.randperm(pairs, generator=torch.Generator().manual_seed(1))]
+    top = 1
+    x = rnd(pairs, hidden, seed=2).to(torch.bfloat16)
+    wg, wu = ((rnd(experts, ff, hidden, seed=3 + i) * hidden ** -0.5).to(torch.bfloat16) for i in range(2))
+    wd = (rnd(experts, hidden, ff, seed=5) * ff ** -0.5).to(torch.bfloat16)
+    weight = torch.rand(pairs, 1, generator=torch.Generator().manual_seed(6)) + 0.5
+    idx = chosen.to(torch.int32).view(pairs, 1)
+    act = torch.full((pairs, ff), float("nan"), dtype=torch.bfloat16, device=DEV)
+    y = torch.full((pairs, hidden), float("nan"), device=DEV)
+    out = torch.full((pairs, hidden), float("nan"), device=DEV)
+    ints = torch.full((2 * pairs + 3 * kernels.moe_max_tiles(pairs, experts, rows) + 1,), -5, dtype=torch.int32, device=DEV)
+    limit = 0.8
+    kw = dict(weight_on_input=True, activation="clamped_swish", limit=limit) if form != "silu" else {}
+    kernels.moe_grouped(x.to(DEV), wg.to(DEV), wu.to(DEV), wd.to(DEV), idx.to(DEV), weight.to(DEV), act, y, out, ints, rows, **kw)
+    xd, e = x.to(F64), chosen
+    g = torch.einsum("th,tfh->tf", xd, wg.to(F64)[e])
+    u = torch.einsum("th,tfh->tf", xd, wu.to(F64)[e])
+    if form == "silu":
+        want_act = g * torch.sigmoid(g) * u
+    else:
+        g, u = (g * weight).clamp(max=limit), (u * weight).clamp(-limit, limit)
+        want_act = g * torch.sigmoid(1.702 * g) * (u + 1.0)
+    got_act = act.cpu().to(F64)
+    # float32 sums of `hidden` products of about 1 / sqrt(hidden) each, through an activation of slope 2 at most, rounded once
+    assert ((got_act - want_act).abs() <= 2.0 ** -8 * want_act.abs() + 1e-5 * (1.0 + want_act.abs().max())).all()
+    want = torch.einsum("tf,thf->th", got_act, wd.to(F64)[e])          # (of the rounded activations)
+    size = torch.einsum("tf,thf->th", got_act.abs(), wd.to(F64)[e].abs())
+    if form == "silu":
+        want, size = want * weight, size * weight
+    assert ((out.cpu().to(F64) - want).abs() <= (ff + 4) * 2.0 ** -24 * size).all()
