@@ -46,34 +46,64 @@ __global__ __launch_bounds__(GROUP_THREADS) void moe_group_kernel(const int* __r
                                                                   int* __restrict__ tile_rows,
                                                                   int* __restrict__ num_tiles) {
     __shared__ int count[MAX_EXPERTS];
-    __shared__ int first[MAX_EXPERTS];
+    __shared__ int first[MAX_EXPERTS];       // an expert's first place
+    __shared__ int first_tile[MAX_EXPERTS + 1];
     const int tid = threadIdx.x;
     for (int e = tid; e < experts; e += GROUP_THREADS) count[e] = 0;
     __syncthreads();
-    for (int a = tid; a < pairs; a += GROUP_THREADS) {
-        const int e = idx[a];
-        if (e >= 0 && e < experts) rank[a] = atomicAdd(&count[e], 1);
+    // (the choices of eight rounds are asked for together: a round by itself waits out a trip to memory)
+    constexpr int AHEAD = 8;
+    for (int a0 = tid; a0 < pairs; a0 += AHEAD * GROUP_THREADS) {
+        int es[AHEAD];
+#pragma unroll
+        for (int u = 0; u < AHEAD; ++u) es[u] = a0 + u * GROUP_THREADS < pairs ? idx[a0 + u * GROUP_THREADS] : -1;
+#pragma unroll
+        for (int u = 0; u < AHEAD; ++u)
+            if (es[u] >= 0 && es[u] < experts) rank[a0 + u * GROUP_THREADS] = atomicAdd(&count[es[u]], 1);
     }
     __syncthreads();
-    if (tid == 0) {
+    if (tid < PULSE_WAVE) {       // places and tiles before an expert: sums over the experts, 64 at a time
         int at = 0, tiles = 0;
-        for (int e = 0; e < experts; ++e) {
-            first[e] = at;
-            const int c = count[e];
-            for (int m = 0; m < c && tiles < max_tiles; m += tile_rows_max) {
-                tile_expert[tiles] = e;
-                tile_row0[tiles] = at + m;
-                tile_rows[tiles] = min(tile_rows_max, c - m);
-                ++tiles;
+        for (int e0 = 0; e0 < experts; e0 += PULSE_WAVE) {
+            const int e = e0 + tid;
+            const int c = e < experts ? count[e] : 0, n = (c + tile_rows_max - 1) / tile_rows_max;
+            int pre_c = c, pre_n = n;
+#pragma unroll
+            for (int off = 1; off < PULSE_WAVE; off <<= 1) {
+                const int uc = __shfl_up(pre_c, off, PULSE_WAVE), un = __shfl_up(pre_n, off, PULSE_WAVE);
+                if (tid >= off) { pre_c += uc; pre_n += un; }
             }
-            at += c;
+            if (e < experts) {
+                first[e] = at + pre_c - c;
+                first_tile[e] = tiles + pre_n - n;
+            }
+            at += __shfl(pre_c, PULSE_WAVE - 1, PULSE_WAVE);
+            tiles += __shfl(pre_n, PULSE_WAVE - 1, PULSE_WAVE);
         }
-        *num_tiles = tiles;
+        if (tid == 0) *num_tiles = min(tiles, max_tiles);
     }
     __syncthreads();
-    for (int a = tid; a < pairs; a += GROUP_THREADS) {
-        const int e = idx[a];
-        if (e >= 0 && e < experts) order[first[e] + rank[a]] = a;
+    for (int e = tid / 16; e < experts; e += GROUP_THREADS / 16) {      // sixteen threads an expert write its tiles
+        const int c = count[e];
+        for (int m = tid % 16; m * tile_rows_max < c; m += 16) {
+            const int t = first_tile[e] + m;
+            if (t >= max_tiles) break;
+            tile_expert[t] = e;
+            tile_row0[t] = first[e] + m * tile_rows_max;
+            tile_rows[t] = min(tile_rows_max, c - m * tile_rows_max);
+        }
+    }
+    for (int a0 = tid; a0 < pairs; a0 += AHEAD * GROUP_THREADS) {
+        int es[AHEAD], at[AHEAD];
+#pragma unroll
+        for (int u = 0; u < AHEAD; ++u) {
+            const int a = a0 + u * GROUP_THREADS;
+            es[u] = a < pairs ? idx[a] : -1;
+            at[u] = es[u] >= 0 && es[u] < experts ? rank[a] : -1;
+        }
+#pragma unroll
+        for (int u = 0; u < AHEAD; ++u)
+            if (at[u] >= 0) order[first[es[u]] + at[u]] = a0 + u * GROUP_THREADS;
     }
 }
 
