@@ -59,6 +59,9 @@ __device__ __forceinline__ pulse_i32x4 stream_load16(const void* p) {
 __device__ __forceinline__ void load_to_lds(const void* p, uint32_t lds_base) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(lds_base), "v"(p) : "memory", "m0");
 }
+__device__ __forceinline__ void stream_to_lds(const void* p, uint32_t lds_base) {   // (nontemporal, see stream_load16)
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off nt" : : "s"(lds_base), "v"(p) : "memory", "m0");
+}
 __device__ __forceinline__ void load_to_lds(const void* base, uint32_t offset, uint32_t lds_base) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(lds_base), "v"(offset), "s"(base) : "memory", "m0");
 }

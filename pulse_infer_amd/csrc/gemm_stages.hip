@@ -1,0 +1,226 @@
+// C[M, N] = X[M, K] W[N, K]^T for some tens to some hundreds of rows (short prompts, portions beside decoded tokens):
+// bfloat16 operands, float32 sums on the matrix cores, on the loop of tile_loop.h.
+// (reference: cuBLAS for every product, src/ops/kernels/cuda/matmul_kernel.cu:132-154)
+//
+// What bounds it: the bytes that the fullest compute unit copies into LDS.  A unit takes in 40 to 65 bytes a nanosecond
+// whatever the tile's shape, less where they are weights that come from memory, so the shape and the shares of K are
+// chosen for the least of them (`plan_for`).  Measured with weights from memory, us, against the vendor library's product
+// (gate and up: with its pass for SwiGLU behind it) and this package's shared-out product for up to 192 rows:
+//                                   97 rows              192                  357                 509
+//   gate + up, 24,576 x 4,096       45 (library 56)      55 (66)              97 (84)             105 (96)
+//   qkv, 6,144 x 4,096              20 (26)              27 (36)              29 (40)             30 (36)
+//   o, 4,096 x 4,096, shares        12 (25; 16 shared)   14 (39; 21 shared)   23 (29)             22 (28)
+//   down, 4,096 x 12,288, shares    24 (45; 33 shared)   31 (92; 45 shared)   47 (67)             53 (83)
+// Weights are read past the caches (nontemporal): 5 % where they are the time.
+#include "common.h"
+#include "tile_loop.h"
+
+namespace {
+
+enum { OUT_BF16 = 0, OUT_SWIGLU = 1, OUT_F32 = 2 };
+
+struct StageArgs {
+    const bf16_t* X;
+    int64_t ldx;
+    const bf16_t* W;
+    int64_t ldw;
+    void* C;
+    int64_t ldc;
+    int M, N, K;          // K: of one share
+    int tiles_m, tiles_n;
+    int splits;           // shares of K, each with a float32 result of its own
+    int64_t part_stride;  // elements between the shares' results
+};
+
+constexpr int PANEL = 8;  // tiles of rows a panel of the tile order
+
+template <int MODE, int WR, int XR, int WN, int WM, int S>
+__global__ __launch_bounds__(256) void gemm_stages_kernel(StageArgs a) {
+    using Loop = TileLoop<WR, XR, WN, WM, S, true>;
+    __shared__ __attribute__((aligned(1024))) char lds[Loop::LDS];
+
+    // The workgroups of a die (every eighth) take neighbouring tiles, in panels of eight tiles of rows, which share
+    // their operands in that die's L2; a share of K is a whole set of tiles.
+    const int tiles = a.tiles_m * a.tiles_n, total = tiles * a.splits;
+    const int per_die = (total + 7) / 8;
+    const int t_all = (blockIdx.x % 8) * per_die + blockIdx.x / 8;
+    if (static_cast<int>(blockIdx.x / 8) >= per_die || t_all >= total) return;
+    const int split = t_all / tiles, t = t_all - split * tiles;
+    const int panel = t / (PANEL * a.tiles_n);
+    const int panel_m = min(PANEL, a.tiles_m - panel * PANEL);
+    const int in_panel = t - panel * PANEL * a.tiles_n;
+    const int m0 = (panel * PANEL + in_panel % panel_m) * XR, n0 = in_panel / panel_m * WR;
+
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / PULSE_WAVE);
+    const int lane = threadIdx.x % PULSE_WAVE;
+    const int64_t k0 = static_cast<int64_t>(split) * a.K;
+    const bf16_t* from[Loop::PER];       // (rows past an operand's end are its last row: their results are not written)
+#pragma unroll
+    for (int j = 0; j < Loop::PER; ++j) {
+        const int row = Loop::row_of(j, wave, lane);
+        from[j] = (j < Loop::PER_W ? a.W + static_cast<int64_t>(min(n0 + row, a.N - 1)) * a.ldw
+                                   : a.X + static_cast<int64_t>(min(m0 + row, a.M - 1)) * a.ldx) +
+                  k0 + Loop::piece_of(row, lane) * 8;
+    }
+    Loop loop;
+    loop.run(from, lds, wave, lane, a.K);
+
+    // Results leave through LDS, a wavefront's 32 rows at a time, in whole 16-byte pieces of rows.
+    constexpr int TN = Loop::TN, TM = Loop::TM;
+    constexpr int FP = TN % 4 == 0 ? (MODE == OUT_F32 ? 2 : 4) : TN % 2 == 0 ? 2 : 1;     // 32-row pieces of W a pass
+    constexpr int SIZE = MODE == OUT_F32 ? 4 : 2;
+    constexpr int COLS = MODE == OUT_SWIGLU ? FP * 16 : FP * 32, PITCH = COLS * SIZE + 16;
+    constexpr int PCS = COLS * SIZE / 16, ROWS = PULSE_WAVE / PCS;
+    constexpr int WAVE_LDS = Loop::LDS / 4;
+    static_assert(32 * PITCH <= WAVE_LDS && TN % FP == 0, "a wavefront's piece of LDS holds 32 rows of a pass");
+    char* mine = lds + wave * WAVE_LDS;
+    const int wave_n = wave % WN, wave_m = wave / WN, h = lane / 32;
+    const int n_wave = (n0 + wave_n * TN * 32) / (MODE == OUT_SWIGLU ? 2 : 1);
+    const int n_end = MODE == OUT_SWIGLU ? a.N / 2 : a.N;
+    char* out = static_cast<char*>(a.C) + (MODE == OUT_F32 ? split * a.part_stride * 4 : 0);
+#pragma unroll
+    for (int g = 0; g < TM; ++g) {
+        const int m_base = m0 + (wave_m * TM + g) * 32;
+        if (m_base >= a.M) break;
+#pragma unroll
+        for (int f0 = 0; f0 < TN; f0 += FP) {
+#pragma unroll
+            for (int f = 0; f < FP; ++f) {
+                const tile_f32x16& acc = loop.acc[f0 + f][g];
+                char* at = mine + (lane % 32) * PITCH;
+                if constexpr (MODE == OUT_F32) {
+#pragma unroll
+                    for (int q = 0; q < 4; ++q)
+                        *reinterpret_cast<float4*>(at + (f * 32 + q * 8 + h * 4) * 4) =
+                            float4{acc[q * 4], acc[q * 4 + 1], acc[q * 4 + 2], acc[q * 4 + 3]};
+                } else if constexpr (MODE == OUT_BF16) {
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        tile_bf16x4 v;
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) v[i] = (__bf16)acc[q * 4 + i];
+                        *reinterpret_cast<tile_bf16x4*>(at + (f * 32 + q * 8 + h * 4) * 2) = v;
+                    }
+                } else {     // weight rows alternate in slabs of 16: the gate rows of 16 outputs, their up rows behind
+#pragma unroll
+                    for (int q = 0; q < 2; ++q) {
+                        tile_bf16x4 v;
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            const float gate = acc[q * 4 + i], up = acc[8 + q * 4 + i];
+                            v[i] = (__bf16)(gate * __builtin_amdgcn_rcpf(1.0f + __expf(-gate)) * up);
+                        }
+                        *reinterpret_cast<tile_bf16x4*>(at + (f * 16 + q * 8 + h * 4) * 2) = v;
+                    }
+                }
+            }
+            tile_wave_sync();
+#pragma unroll
+            for (int it = 0; it < 32 / ROWS; ++it) {
+                const int row = it * ROWS + lane / PCS, pc = lane % PCS;
+                const uint4 v = *reinterpret_cast<const uint4*>(mine + row * PITCH + pc * 16);
+                const int m = m_base + row, n = n_wave + f0 * (MODE == OUT_SWIGLU ? 16 : 32) + pc * (16 / SIZE);
+                if (m < a.M && n < n_end)
+                    *reinterpret_cast<uint4*>(out + (static_cast<int64_t>(m) * a.ldc + n) * SIZE) = v;
+            }
+            tile_wave_sync();
+        }
+    }
+}
+
+template <int MODE, int WR, int XR, int WN, int WM, int S>
+void launch(StageArgs a, hipStream_t stream) {
+    a.tiles_m = (a.M + XR - 1) / XR;
+    a.tiles_n = (a.N + WR - 1) / WR;
+    const int64_t grid = (static_cast<int64_t>(a.tiles_m) * a.tiles_n * a.splits + 7) / 8 * 8;
+    hipLaunchKernelGGL((gemm_stages_kernel<MODE, WR, XR, WN, WM, S>), dim3(static_cast<unsigned>(grid)), dim3(256), 0, stream, a);
+}
+
+// weight rows and rows of X a tile (the kernels below, in this order)
+constexpr int SHAPES[][2] = {{32, 128}, {64, 64}, {64, 128}, {96, 128}, {128, 64}, {128, 128}, {192, 128}, {256, 128}};
+constexpr int NUM_SHAPES = sizeof(SHAPES) / sizeof(SHAPES[0]);
+
+template <int MODE>
+void launch_shape(int shape, const StageArgs& a, hipStream_t s) {
+    switch (shape) {
+        case 0: return launch<MODE, 32, 128, 1, 4, 4>(a, s);
+        case 1: return launch<MODE, 64, 64, 2, 2, 6>(a, s);
+        case 2: return launch<MODE, 64, 128, 2, 2, 6>(a, s);
+        case 3: return launch<MODE, 96, 128, 1, 4, 5>(a, s);
+        case 4: return launch<MODE, 128, 64, 4, 1, 3>(a, s);
+        case 5: return launch<MODE, 128, 128, 2, 2, 4>(a, s);
+        case 6: return launch<MODE, 192, 128, 2, 2, 3>(a, s);
+        default: return launch<MODE, 256, 128, 2, 2, 3>(a, s);
+    }
+}
+
+struct Plan { int shape, splits; };
+
+// The shape (and, for float32 results in shares, their number: `shares` 0 leaves it open) whose fullest compute unit copies
+// least: workgroups on it x rows a stage x steps of K, in units of 128 bytes (3.2 ns on the whole), and for every share its
+// results' way to memory and back to whoever adds them up (8 bytes a value at 4 TB/s).
+Plan plan_for(int M, int N, int K, int shares) {
+    const int64_t units = pulse_compute_units();
+    Plan best{0, 1};
+    double least = 0.0;
+    bool any = false;
+    for (int splits = shares > 0 ? shares : 1; splits <= (shares > 0 ? shares : 16); ++splits) {
+        if (K % (64 * splits)) continue;
+        for (int i = 0; i < NUM_SHAPES; ++i) {
+            const int64_t tiles = static_cast<int64_t>((M + SHAPES[i][1] - 1) / SHAPES[i][1]) *
+                                  ((N + SHAPES[i][0] - 1) / SHAPES[i][0]) * splits;
+            const double cost = static_cast<double>((tiles + units - 1) / units) * (SHAPES[i][0] + SHAPES[i][1]) *
+                                    (K / splits / 64) + (shares == 1 ? 0.0 : splits * (8.0 / 4000.0 / 3.2) * M * N);
+            if (!any || cost < least) { best = {i, splits}; least = cost; any = true; }
+        }
+    }
+    return best;
+}
+
+bool aligned16(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
+
+}  // namespace
+
+// Whether the product takes these sizes: an inner dimension whose shares are multiples of 64, weight rows in multiples of
+// 8 (of 32 with SwiGLU inside, of 4 for float32 results), shares only with float32 results.
+extern "C" int pulse_gemm_stages_takes(int M, int N, int K, int mode, int splits) {
+    if (M <= 0 || N <= 0 || K <= 0 || splits < 1 || mode < OUT_BF16 || mode > OUT_F32) return 0;
+    if (splits > 1 && mode != OUT_F32) return 0;
+    if (K % (64 * splits)) return 0;
+    const int n_step = mode == OUT_SWIGLU ? 32 : (mode == OUT_BF16 ? 8 : 4);
+    if (N % n_step) return 0;
+    return static_cast<int64_t>((M + 63) / 64) * ((N + 31) / 32) * splits <= (1 << 28);
+}
+
+// How many shares of K float32 results are best made in (0: a shape that the product does not take).
+extern "C" int pulse_gemm_stages_shares(int M, int N, int K) {
+    if (!pulse_gemm_stages_takes(M, N, K, OUT_F32, 1)) return 0;
+    return plan_for(M, N, K, 0).splits;
+}
+
+// mode 0: C [M, N] bfloat16.  mode 1: the rows of W alternate in slabs of 16 gate rows and their 16 up rows;
+// C [M, N / 2] bfloat16 = silu(gate) * up.  mode 2: float32, one result [M, N] for every share of K, `part_stride`
+// elements apart (the shares are added up by whoever reads them, in order).
+extern "C" int pulse_gemm_stages(const void* X, int64_t ldx, const void* W, int64_t ldw, void* C, int64_t ldc, int M, int N,
+                                 int K, int mode, int splits, int64_t part_stride, hipStream_t stream) {
+    PULSE_REQUIRE(pulse_gemm_stages_takes(M, N, K, mode, splits),
+                  "gemm_stages: %d rows x %d weight rows x inner dimension %d, mode %d, %d shares: the inner dimension must "
+                  "be a multiple of 64 a share, the weight rows a multiple of 8 (32 with SwiGLU, 4 for float32 results), "
+                  "shares need float32 results", M, N, K, mode, splits);
+    PULSE_REQUIRE(X && W && C && aligned16(X) && aligned16(W) && aligned16(C), "gemm_stages: operands must be aligned to 16 bytes");
+    PULSE_REQUIRE(ldx >= K && ldw >= K && ldx % 8 == 0 && ldw % 8 == 0, "gemm_stages: rows of X and W must be K long at "
+                  "least and start at multiples of 16 bytes (strides %lld, %lld)", (long long)ldx, (long long)ldw);
+    const int out_cols = mode == OUT_SWIGLU ? N / 2 : N;
+    PULSE_REQUIRE(ldc >= out_cols && ldc % (mode == OUT_F32 ? 4 : 8) == 0, "gemm_stages: rows of the result must be %d long "
+                  "at least and start at multiples of 16 bytes (stride %lld)", out_cols, (long long)ldc);
+    PULSE_REQUIRE(splits == 1 || (part_stride >= static_cast<int64_t>(M - 1) * ldc + N && part_stride % 4 == 0),
+                  "gemm_stages: the shares' results overlap (stride %lld)", (long long)part_stride);
+    StageArgs a{static_cast<const bf16_t*>(X), ldx, static_cast<const bf16_t*>(W), ldw, C, ldc, M, N, K / splits, 0, 0, splits,
+                splits > 1 ? part_stride : 0};
+    const int shape = plan_for(M, N, K, splits).shape;
+    if (mode == OUT_BF16) launch_shape<OUT_BF16>(shape, a, stream);
+    else if (mode == OUT_SWIGLU) launch_shape<OUT_SWIGLU>(shape, a, stream);
+    else launch_shape<OUT_F32>(shape, a, stream);
+    PULSE_LAUNCH_CHECK("gemm_stages");
+    return 0;
+}

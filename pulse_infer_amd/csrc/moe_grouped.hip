@@ -409,16 +409,14 @@ __global__ __launch_bounds__(256) void moe_tile_kernel(GroupArgs a) {
     const bf16_t* from[Loop::PER];
 #pragma unroll
     for (int j = 0; j < Loop::PER; ++j) {
-        const int row = (wave * Loop::PER + j) * 8 + lane / 8;
-        const int c = (lane % 8) ^ Loop::swz(row < WR ? row : row - WR);
-        if (row < WR) {
+        const int row = Loop::row_of(j, wave, lane), piece = Loop::piece_of(row, lane);
+        if (j < Loop::PER_W) {
             const int n = DOWN ? n0 + row : n0 + row / 32 * 16 + row % 16;
             const bf16_t* w = DOWN ? a.w[0] : (row & 16) ? a.w[1] : a.w[0];
-            from[j] = w + (static_cast<int64_t>(e) * a.N + min(n, a.N - 1)) * a.K + c * 8;
+            from[j] = w + (static_cast<int64_t>(e) * a.N + min(n, a.N - 1)) * a.K + piece * 8;
         } else {
-            const int p = max(pair_s[row - WR], 0);
-            const int from_row = DOWN ? (pair_s[row - WR] < 0 ? pair_s[0] : p) : (pair_s[row - WR] < 0 ? pair_s[0] : p) / a.top;
-            from[j] = a.x + static_cast<int64_t>(from_row) * a.K + c * 8;
+            const int p = pair_s[row] < 0 ? pair_s[0] : pair_s[row];
+            from[j] = a.x + static_cast<int64_t>(DOWN ? p : p / a.top) * a.K + piece * 8;
         }
     }
     Loop loop;

@@ -16,17 +16,17 @@ typedef __attribute__((ext_vector_type(8))) __bf16 tile_bf16x8;
 typedef __attribute__((ext_vector_type(4))) __bf16 tile_bf16x4;
 typedef __attribute__((ext_vector_type(16))) float tile_f32x16;
 
-template <int WR, int XR, int WN, int WM, int S>
+template <int WR, int XR, int WN, int WM, int S, bool NT = false>
 struct TileLoop {
     static constexpr int BK = 64;
     static constexpr int ROW_BYTES = BK * 2;
     static constexpr int STAGE = (WR + XR) * ROW_BYTES;
     static constexpr int NW = WN * WM;
     static constexpr int TN = WR / 32 / WN, TM = XR / 32 / WM;       // 32-row pieces a wavefront
-    static constexpr int CHUNKS = (WR + XR) / 8;                     // 1 KB (8 rows) each
-    static constexpr int PER = CHUNKS / NW;                          // a wavefront copies
+    static constexpr int PER_W = WR / 8 / NW, PER_X = XR / 8 / NW;   // chunks of 1 KB (8 rows) a wavefront copies
+    static constexpr int PER = PER_W + PER_X;
     static constexpr int LDS = S * STAGE;
-    static_assert(CHUNKS % NW == 0 && TN >= 1 && TM >= 1 && S >= 2, "whole chunks and pieces a wavefront");
+    static_assert(WR % (8 * NW) == 0 && XR % (8 * NW) == 0 && TN >= 1 && TM >= 1 && S >= 2, "whole chunks and pieces a wavefront");
 
     // Piece c (16 bytes) of row r of a stage sits at place c ^ swz(r): the rows that neighbouring lanes read together then
     // lie in different places of what LDS serves at once.
@@ -34,15 +34,27 @@ struct TileLoop {
 
     tile_f32x16 acc[TN][TM];
 
-    // from[j]: where this lane's 16 bytes of the wavefront's j-th chunk start in memory at k = 0; chunk j of wavefront w is
-    // chunk w * PER + j of the stage, lane i brings piece (i % 8) ^ swz(row) of its row i / 8.
+    // Row (of the tile's W for j < PER_W, else of its X) and piece that this lane brings with the wavefront's j-th chunk.
+    static __device__ __forceinline__ int row_of(int j, int wave, int lane) {
+        return (j < PER_W ? wave * PER_W + j : wave * PER_X + j - PER_W) * 8 + lane / 8;
+    }
+    static __device__ __forceinline__ int piece_of(int row, int lane) { return (lane % 8) ^ swz(row); }
+
+    // from[j]: where that piece lies in memory at k = 0.
     __device__ __forceinline__ void run(const bf16_t* const (&from)[PER], char* lds, int wave, int lane, int K) {
         const int wave_n = wave % WN, wave_m = wave / WN;
         const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(
             (void __attribute__((address_space(3)))*)(lds)));
         const int steps = K / BK;
         auto copy = [&](int step, int stage, int j) __attribute__((always_inline)) {
-            load_to_lds(from[j] + min(step, steps - 1) * BK, lds0 + stage * STAGE + (wave * PER + j) * 1024);
+            const bf16_t* at = from[j] + min(step, steps - 1) * BK;
+            if (j < PER_W) {
+                const uint32_t to = lds0 + stage * STAGE + (wave * PER_W + j) * 1024;
+                if constexpr (NT) stream_to_lds(at, to);
+                else load_to_lds(at, to);
+            } else {
+                load_to_lds(at, lds0 + stage * STAGE + WR * ROW_BYTES + (wave * PER_X + j - PER_W) * 1024);
+            }
         };
         const int h = lane / 32, e = h ^ swz(lane % 32);
         int w_at[4], x_at[4];

@@ -8,10 +8,12 @@ result tensor is asked for, and nothing falls back to another implementation.
 from __future__ import annotations
 
 import ctypes
+import functools
 from typing import Any, Optional
 
 import torch
 
+from . import library
 from .library import KernelError, call
 
 _TAG = {torch.float32: 0, torch.bfloat16: 1}
@@ -443,6 +445,43 @@ def gemm_tile(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, swiglu: bool 
               f"gemm_tile: out must be bfloat16 [{m}, {cols}]")
         mode, ldc, part_stride, splits = (1 if swiglu else 0), (out.stride(0) if m > 1 else cols), 0, 1
     call("pulse_gemm_tile", _ptr(a), _i64(a.stride(0) if m > 1 else k), _ptr(w), _i64(w.stride(0) if n > 1 else k),
+         _ptr(out), _i64(ldc), _i32(m), _i32(n), _i32(k), _i32(mode), _i32(splits), _i64(part_stride), _stream(),
+         label=f"N={n} K={k}")
+
+
+@functools.lru_cache(maxsize=4096)
+def gemm_stages_shares(m: int, n: int, k: int) -> int:
+    """Shares of K that ``gemm_stages`` makes float32 results in best (a function of the sizes alone); 0: it does not take
+    the shape."""
+    return int(library.load().pulse_gemm_stages_shares(_i32(m), _i32(n), _i32(k)))
+
+
+def gemm_stages_takes(m: int, n: int, k: int, swiglu: bool = False) -> bool:
+    """Whether ``gemm_stages`` takes a shape with bfloat16 results (as pulse_gemm_stages_takes)."""
+    return m > 0 and n > 0 and k > 0 and k % 64 == 0 and n % (32 if swiglu else 8) == 0
+
+
+def gemm_stages(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, swiglu: bool = False) -> None:
+    """a @ w^T for some tens to some hundreds of rows of bfloat16, several stages of the operands on their way through LDS.
+    ``out`` as for ``gemm_tile``: bfloat16 [M, N], with ``swiglu`` [M, N / 2], or float32 [shares, M, N]."""
+    _gpu("gemm_stages", a, w, out)
+    _need(a.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and a.dim() == 2 and w.dim() == 2
+          and a.stride(1) == 1 and w.stride(1) == 1, "gemm_stages: a and w must be bfloat16 matrices with contiguous rows")
+    m, k = a.shape
+    n = w.shape[0]
+    _need(w.shape[1] == k, f"gemm_stages: inner sizes differ ({k} and {w.shape[1]})")
+    if out.dtype == torch.float32:
+        splits = out.shape[0]
+        _need(not swiglu and out.dim() == 3 and tuple(out.shape[1:]) == (m, n) and out.is_contiguous() and n % 4 == 0
+              and k % (64 * splits) == 0, f"gemm_stages: float32 results go to contiguous [shares, {m}, {n}]")
+        mode, ldc, part_stride = 2, n, m * n if splits > 1 else 0
+    else:
+        cols = n // 2 if swiglu else n
+        _need(gemm_stages_takes(m, n, k, swiglu) and out.dtype == torch.bfloat16 and out.dim() == 2
+              and tuple(out.shape) == (m, cols) and out.stride(1) == 1,
+              f"gemm_stages: M={m} N={n} K={k} is not a shape it takes, or out is not bfloat16 [{m}, {cols}]")
+        mode, ldc, part_stride, splits = (1 if swiglu else 0), (out.stride(0) if m > 1 else cols), 0, 1
+    call("pulse_gemm_stages", _ptr(a), _i64(a.stride(0) if m > 1 else k), _ptr(w), _i64(w.stride(0) if n > 1 else k),
          _ptr(out), _i64(ldc), _i32(m), _i32(n), _i32(k), _i32(mode), _i32(splits), _i64(part_stride), _stream(),
          label=f"N={n} K={k}")
 

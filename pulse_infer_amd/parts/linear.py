@@ -1,10 +1,12 @@
 """y = x W^T for a weight stored [out, in] (reference: src/layer/linear.cpp:213).
 
-Three products stand behind it:
+Four products stand behind it:
 
 * few rows (decoding, short portions) of bfloat16: this package's weight-streaming
   matrix-core kernel, which can also add into the float32 residual or apply SwiGLU;
-* many rows of bfloat16: the vendor library's product (torch.matmul / torch.mm,
+* 65 rows to some hundreds of bfloat16: this package's product with several stages of its
+  operands on their way through LDS (``takes_stages`` says where it is the faster one);
+* more rows of bfloat16: the vendor library's product (torch.matmul / torch.mm,
   i.e. hipBLASLt/rocBLAS, float32 accumulation, bfloat16 or float32 output), as
   the reference uses cuBLAS (src/ops/kernels/cuda/matmul_kernel.cu:132-154), or this
   package's product in output tiles of 256 x 256, which can apply SwiGLU on the way
@@ -69,7 +71,10 @@ class Linear:
             if x.shape[0] > self.MID_ROWS[1]:
                 if kernels.gate_code(swiglu) != 1:
                     raise ValueError("the tiled product applies silu only")
-                kernels.gemm_tile(x, w, out, swiglu=True)
+                if self.takes_stages(x, w, swiglu=True):
+                    kernels.gemm_stages(x, w, out, swiglu=True)
+                else:
+                    kernels.gemm_tile(x, w, out, swiglu=True)
             elif x.shape[0] > kernels.SKINNY_FAST_ROWS:
                 kernels.gemm_mid(x, w, out, swiglu=swiglu, waves=self.swiglu_waves_for(x.shape[0]) or 4)
             else:
@@ -94,6 +99,10 @@ class Linear:
                     return out
                 waves = 10 if w.shape[0] >= 64 * compute_units() else 2
                 kernels.gemm_mid(x, w, out.view(1, *out.shape) if out.dtype == torch.float32 else out, waves=waves)
+                return out
+            if own and out.dtype == torch.bfloat16 and self.takes_stages(x, w) and out.stride(1) == 1 \
+                    and out.stride(0) % 8 == 0 and out.data_ptr() % 16 == 0:
+                kernels.gemm_stages(x, w, out)
                 return out
             if own and out.dtype == torch.bfloat16 and self.takes_tiles(x, w) and out.stride(1) == 1 \
                     and out.stride(0) % 8 == 0 and out.data_ptr() % 16 == 0:
@@ -137,6 +146,13 @@ class Linear:
         Otherwise the product is written to ``scratch`` and returned for the caller to add.  ``leave_stats=False``:
         no ``RowStats`` are made (their buffers are the workspace's, one set a width: a caller that still reads the
         set of the rows as they were before this update says so)."""
+        splits = self.stage_shares_for(x) if workspace is not None else 0
+        if splits:
+            rows = x.shape[0]
+            parts = workspace.buffer(f"linear.parts.{self.out_features}.{self.in_features}", splits * rows,
+                                     self.out_features, torch.float32).view(splits, rows, self.out_features)
+            kernels.gemm_stages(x, self.weight, parts)
+            return parts
         splits, waves = self.shares_and_waves_for(x) if workspace is not None else (0, 0)
         if splits:
             rows = x.shape[0]
@@ -237,6 +253,34 @@ class Linear:
         if out.dtype == torch.float32:
             return out.is_contiguous() and out.data_ptr() % 16 == 0 and w.shape[0] % 4 == 0
         return out.dtype == torch.bfloat16 and out.stride(1) == 1 and out.stride(0) % 4 == 0 and out.data_ptr() % 16 == 0
+
+    # Where the product in stages is the fastest (the figures are beside its kernel): with SwiGLU inside and for updates
+    # in shares of a wide inner dimension up to 256 rows, beyond which the library's large tiles have the better of the
+    # matrix cores; for plain products and shares of a narrower one as long as the library leaves compute units idle (6,144
+    # weight rows of 4,096 at 1,024 rows 48 us against 51; 4,096 of 4,096 at 509 rows 22 against 28, at 700 33 against
+    # 34).  Small products stay where they are.
+    STAGE_ROWS = (65, 256)
+    STAGE_ROWS_NARROW = (512, 1024)     # updates in shares; plain products of at most 32 weight rows a compute unit
+    STAGE_MIN_WEIGHT = 1 << 22
+
+    def takes_stages(self, x: torch.Tensor, w: Optional[torch.Tensor] = None, swiglu: bool = False) -> bool:
+        """Whether a bfloat16 product of this many rows (with SwiGLU inside, or as it is) runs as this package's product
+        in stages."""
+        w = self.weight if w is None else w
+        rows, (n, k) = x.shape[0], w.shape
+        most = self.STAGE_ROWS[1] if swiglu or n > 32 * compute_units() else self.STAGE_ROWS_NARROW[1]
+        return (self.library and x.dtype == torch.bfloat16 and self.STAGE_ROWS[0] <= rows <= most
+                and n * k >= self.STAGE_MIN_WEIGHT and self.operands_ok(x) and kernels.gemm_stages_takes(rows, n, k, swiglu))
+
+    def stage_shares_for(self, x: torch.Tensor) -> int:
+        """Into how many shares of the inner dimension the product in stages cuts an update that the next norm adds up; 0:
+        not this product."""
+        rows, n, k = x.shape[0], self.out_features, self.in_features
+        most = self.STAGE_ROWS[1] if k >= self.LIBRARY_SHARES_MIN_K else self.STAGE_ROWS_NARROW[0]
+        if not (self.library and x.dtype == torch.bfloat16 and self.STAGE_ROWS[0] <= rows <= most
+                and n * k >= self.STAGE_MIN_WEIGHT and self.operands_ok(x)) or n % 4 or k % 64:
+            return 0
+        return kernels.gemm_stages_shares(rows, n, k)
 
     TILE_MIN_ROWS = 256          # from here on the tiled product for many rows is a candidate
 

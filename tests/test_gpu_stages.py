@@ -1,0 +1,57 @@
+"""The product in stages (some tens to some hundreds of rows) where its tiles and its shares of K end."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+F64 = torch.float64
+
+
+def rnd(*shape, seed):
+    return torch.randn(shape, generator=torch.Generator().manual_seed(seed))
+
+
+# every tile the plan knows, with remainders of rows and weight rows, one step of K and many, one row and several panels
+@pytest.mark.parametrize("shape", [(1, 32, 64), (65, 96, 128), (97, 6144, 192), (97, 24576, 64), (128, 4096, 1024),
+                                   (130, 24608, 128), (193, 12288, 64), (256, 4128, 320), (357, 6176, 64), (1030, 2080, 128)])
+def test_product_in_stages_at_the_edges_of_its_tiles(shape):
+    from pulse_infer_amd.ops import kernels
+
+    m, n, k = shape
+    x, w = rnd(m, k, seed=1).to(torch.bfloat16), rnd(n, k, seed=2).to(torch.bfloat16)
+    xd, wd = torch.empty(m, k + 8, dtype=torch.bfloat16, device=DEV)[:, :k], w.to(DEV)
+    xd.copy_(x)                                         # (rows may lie further apart than they are long)
+    want, size = x.to(F64) @ w.to(F64).T, x.to(F64).abs() @ w.to(F64).abs().T
+    exact = (k + 2) * 2.0 ** -24 * size                 # a float32 sum of k exact products, in any order
+    out = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device=DEV)
+    kernels.gemm_stages(xd, wd, out)
+    assert ((out.cpu().to(F64) - want).abs() <= exact + 2.0 ** -8 * want.abs()).all()
+    best = kernels.gemm_stages_shares(m, n, k)
+    assert best >= 1 and k % (64 * best) == 0
+    for shares in {1, best, k // 64}:
+        parts = torch.full((shares, m, n), float("nan"), device=DEV)
+        kernels.gemm_stages(xd, wd, parts)
+        got = parts.cpu().to(F64)
+        assert ((got.sum(0) - want).abs() <= exact).all(), shares
+        part = k // shares
+        last = x[:, k - part:].to(F64) @ w[:, k - part:].to(F64).T
+        assert ((got[-1] - last).abs() <= exact).all(), shares
+    slab = torch.arange(n) // 16 % 2
+    gate, up = want[:, slab == 0] / k ** 0.5, want[:, slab == 1] / k ** 0.5
+    xs = (x.float() / k ** 0.5).to(torch.bfloat16) if (k ** 0.5).is_integer() and k in (64, 1024) else None
+    if xs is not None:                                  # (a power of two: the scaled rows are exact)
+        act = torch.full((m, n // 2), float("nan"), dtype=torch.bfloat16, device=DEV)
+        kernels.gemm_stages(xs.to(DEV), wd, act, swiglu=True)
+        wanted = gate * torch.sigmoid(gate) * up
+        # hardware exponential and reciprocal (relative 2^-21 each), one rounding to bfloat16
+        assert ((act.cpu().to(F64) - wanted).abs() <= 2.0 ** -7.9 * wanted.abs() + 1e-5).all()
+
+
+def test_product_in_stages_refuses_what_it_cannot_read():
+    from pulse_infer_amd.ops import kernels
+    from pulse_infer_amd.ops.library import KernelError
+
+    x, w = torch.zeros(70, 96, dtype=torch.bfloat16, device=DEV), torch.zeros(64, 96, dtype=torch.bfloat16, device=DEV)
+    assert not kernels.gemm_stages_takes(70, 64, 96) and kernels.gemm_stages_shares(70, 64, 96) == 0
+    with pytest.raises((KernelError, ValueError)):
+        kernels.gemm_stages(x, w, torch.empty(70, 64, dtype=torch.bfloat16, device=DEV))
