@@ -50,8 +50,8 @@ __device__ __forceinline__ bf16x8 zeros8() {
     return __builtin_bit_cast(bf16x8, u32x4{0u, 0u, 0u, 0u});
 }
 
-template <int R, int CT>
-__global__ __launch_bounds__(256, R == 1 ? 3 : 1) void attn_wide_kernel(const bf16_t* __restrict__ q, float* __restrict__ out,
+template <int R, int CT, int AHEAD, int PER_SIMD>
+__global__ __launch_bounds__(256, PER_SIMD) void attn_wide_kernel(const bf16_t* __restrict__ q, float* __restrict__ out,
                                                         const bf16_t* __restrict__ kcache,
                                                         const bf16_t* __restrict__ vcache,
                                                         const int* __restrict__ positions,
@@ -131,18 +131,28 @@ __global__ __launch_bounds__(256, R == 1 ? 3 : 1) void attn_wide_kernel(const bf
         for (int t = 0; t < 2; ++t)
             krow[t] = page[t] >= 0 ? kcache + ((static_cast<int64_t>(page[t]) * a.nkv + kvh) * a.page_size + off[t] + r) * d
                                    : nullptr;
-        for (int e0 = 0; e0 < d; e0 += 32) {
-            const int e = e0 + 8 * g;
-            const bool in = e < d;
-            bf16x8 ka[2];
+        // (the operands of AHEAD pieces of 32 channels are asked for together: a piece by itself waits out a trip to
+        // memory, and a wavefront of a step of few tokens has a block or two of keys in all.  8 requests of 1,500 tokens,
+        // a latent row of 576 channels: 28 us a piece at a time, 26 so.)
+        for (int e0 = 0; e0 < d; e0 += 32 * AHEAD) {
+            bf16x8 ka[AHEAD][2], qb[AHEAD][R];
 #pragma unroll
-            for (int t = 0; t < 2; ++t) ka[t] = (in && krow[t]) ? *reinterpret_cast<const bf16x8*>(krow[t] + e) : zeros8();
+            for (int u = 0; u < AHEAD; ++u) {
+                const int e = e0 + 32 * u + 8 * g;
+                const bool in = e < d;
 #pragma unroll
-            for (int rr = 0; rr < R; ++rr) {
-                const bf16x8 qb = in ? *reinterpret_cast<const bf16x8*>(qrow[rr] + e) : zeros8();
+                for (int t = 0; t < 2; ++t)
+                    ka[u][t] = (in && krow[t]) ? *reinterpret_cast<const bf16x8*>(krow[t] + e) : zeros8();
 #pragma unroll
-                for (int t = 0; t < 2; ++t) s[rr][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka[t], qb, s[rr][t], 0, 0, 0);
+                for (int rr = 0; rr < R; ++rr) qb[u][rr] = in ? *reinterpret_cast<const bf16x8*>(qrow[rr] + e) : zeros8();
             }
+#pragma unroll
+            for (int u = 0; u < AHEAD; ++u)
+#pragma unroll
+                for (int rr = 0; rr < R; ++rr)
+#pragma unroll
+                    for (int t = 0; t < 2; ++t)
+                        s[rr][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka[u][t], qb[u][rr], s[rr][t], 0, 0, 0);
         }
         // every row's scores of keys jbase[t] + 4 g + i become its weights, in the order the P^T operand wants them
         bf16x8 pb[R];
@@ -308,15 +318,19 @@ __global__ __launch_bounds__(256, R == 1 ? 3 : 1) void attn_wide_kernel(const bf
 __global__ void attn_wide_merge_kernel(const float* __restrict__ part, const float* __restrict__ part_ml,
                                        float* __restrict__ out, int64_t o_stride, const float* __restrict__ sink, int nq,
                                        int w, int wv, int n_splits) {
+    // (n_splits is at most 64: a lane a split, every wavefront for itself; the splits' values are then read eight at a time.
+    // A split at a time, 15 splits of 8 tokens of 32 heads took 14 us, 5.4 so.)
+    __shared__ float factor[PULSE_WAVE];
     const int tok = blockIdx.x, head = blockIdx.y;
     const int64_t at = (static_cast<int64_t>(tok) * nq + head) * n_splits;
-    float m_all = -INFINITY;
-    for (int s = 0; s < n_splits; ++s) m_all = fmaxf(m_all, part_ml[2 * (at + s)]);
-    float l_all = 0.f;
-    for (int s = 0; s < n_splits; ++s) {
-        const float m = part_ml[2 * (at + s)];
-        l_all += (m == -INFINITY) ? 0.f : part_ml[2 * (at + s) + 1] * expf(m - m_all);
-    }
+    const int lane = threadIdx.x % PULSE_WAVE;
+    const float m = lane < n_splits ? part_ml[2 * (at + lane)] : -INFINITY;
+    const float l = lane < n_splits ? part_ml[2 * (at + lane) + 1] : 0.f;
+    const float m_all = wave_max(m);
+    const float f = m == -INFINITY ? 0.f : expf(m - m_all);
+    float l_all = wave_sum(f == 0.f ? 0.f : l * f);
+    if (threadIdx.x < PULSE_WAVE) factor[lane] = f;
+    __syncthreads();
     float scale_out = 1.f;
     if (sink) {
         const float sk = sink[head];
@@ -326,11 +340,19 @@ __global__ void attn_wide_merge_kernel(const float* __restrict__ part, const flo
     }
     const float inv = l_all > 0.f ? scale_out / l_all : 0.f;
     float* orow = out + static_cast<int64_t>(tok) * o_stride + static_cast<int64_t>(head) * w;
+    constexpr int AHEAD = 8;
     for (int ch = threadIdx.x; ch < wv; ch += blockDim.x) {
+        const float* from = part + at * w + ch;
         float sum = 0.f;
-        for (int s = 0; s < n_splits; ++s) {
-            const float m = part_ml[2 * (at + s)];
-            if (m != -INFINITY) sum = fmaf(part[(at + s) * w + ch], expf(m - m_all), sum);
+        for (int s0 = 0; s0 < n_splits; s0 += AHEAD) {
+            float v[AHEAD];
+#pragma unroll
+            for (int u = 0; u < AHEAD; ++u) v[u] = from[static_cast<int64_t>(min(s0 + u, n_splits - 1)) * w];
+#pragma unroll
+            for (int u = 0; u < AHEAD; ++u) {      // (a split without keys has left nothing)
+                const float fu = s0 + u < n_splits ? factor[s0 + u] : 0.f;
+                if (fu != 0.f) sum = fmaf(v[u], fu, sum);
+            }
         }
         orow[ch] = sum * inv;
     }
@@ -373,14 +395,20 @@ extern "C" int pulse_attn_wide(const void* q, int64_t q_stride, float* out, int6
     a.n_splits = n_splits; a.part = part; a.part_ml = part_ml;
     if (row_tiles == 4) {
         const dim3 grid(n_items, (wv + 127) / 128, n_splits);
-        hipLaunchKernelGGL((attn_wide_kernel<4, 8>), grid, dim3(256), 0, stream, static_cast<const bf16_t*>(q), out,
+        hipLaunchKernelGGL((attn_wide_kernel<4, 8, 1, 1>), grid, dim3(256), 0, stream, static_cast<const bf16_t*>(q), out,
                            static_cast<const bf16_t*>(kcache), static_cast<const bf16_t*>(vcache), positions, token_entry,
                            block_table, items, sink, a);
     } else {
         const dim3 grid(n_items, (wv + 255) / 256, n_splits);
-        hipLaunchKernelGGL((attn_wide_kernel<1, MAX_TILES>), grid, dim3(256), 0, stream, static_cast<const bf16_t*>(q), out,
-                           static_cast<const bf16_t*>(kcache), static_cast<const bf16_t*>(vcache), positions, token_entry,
-                           block_table, items, sink, a);
+        // Steps of few tokens, whose keys are shared out, ask for six pieces of a key ahead and need the registers of a
+        // wavefront and a half for it; prompt portions have enough wavefronts to wait for one another (three a SIMD).
+#define PULSE_WIDE(AHEAD, PER_SIMD)                                                                                      \
+    hipLaunchKernelGGL((attn_wide_kernel<1, MAX_TILES, AHEAD, PER_SIMD>), grid, dim3(256), 0, stream,                    \
+                       static_cast<const bf16_t*>(q), out, static_cast<const bf16_t*>(kcache),                           \
+                       static_cast<const bf16_t*>(vcache), positions, token_entry, block_table, items, sink, a)
+        if (n_splits > 1) PULSE_WIDE(6, 2);
+        else PULSE_WIDE(1, 3);
+#undef PULSE_WIDE
     }
     PULSE_LAUNCH_CHECK("attn_wide");
     if (n_splits > 1 && tokens > 0) {

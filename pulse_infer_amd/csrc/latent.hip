@@ -161,52 +161,72 @@ template <> __device__ __forceinline__ hp_bf16x8 load8<float>(const float* p) {
     return out;
 }
 
-// A workgroup takes 16 TT tokens of one head; a wavefront a tile of 16 output channels at a time, whose W operands serve
-// all TT token tiles.  W rows are the matrix cores' row operand (m = output channel), the tokens' rows of x the column
-// operand, so a lane ends up with four neighbouring channels of its token: one 8-byte store.
-template <typename TX, int TT>
+// A workgroup takes 16 TT tokens of one head and 4 / KW tiles of 16 output channels; KW of its wavefronts share a tile's K out
+// in steps of 32 and meet in LDS in their order.  W rows are the matrix cores' row operand (m = output channel), the tokens'
+// rows of x the column operand, so a lane ends up with four neighbouring channels of its token.
+//
+// What bounds it for few tokens: trips to memory.  A workgroup a head walked all its tiles a piece of 32 values at a time: 8
+// tokens, 32 heads, 512 x 128 and 128 x 512 18 us each, 5.3 and 5.2 with a workgroup a few tiles and the pieces of
+// AHEAD steps asked for together.
+template <typename TX, int TT, int KW>
 __global__ __launch_bounds__(256) void heads_product_kernel(const TX* __restrict__ x, int64_t x_stride, int x_head,
                                                             const bf16_t* __restrict__ w, const bf16_t* __restrict__ gate,
                                                             int64_t gate_stride, bf16_t* __restrict__ y, int64_t y_stride,
                                                             int y_head, int tokens, int m_out, int k_in, float scale, int gate_heads) {
+    __shared__ hp_f32x4 meet[KW > 1 ? 4 : 1][TT][PULSE_WAVE];
     const int t0 = blockIdx.x * (16 * TT), h = blockIdx.y;
     const int lane = threadIdx.x % PULSE_WAVE, wave = threadIdx.x / PULSE_WAVE;
     const int r = lane % 16, g = lane / 16;
+    const int m0 = (static_cast<int>(blockIdx.z) * (4 / KW) + wave / KW) * 16, share = wave % KW;
     const TX* xrow[TT];
 #pragma unroll
     for (int u = 0; u < TT; ++u)
         xrow[u] = x + static_cast<int64_t>(min(t0 + 16 * u + r, tokens - 1)) * x_stride + static_cast<int64_t>(h) * x_head;
     const hp_bf16x8 zero = __builtin_bit_cast(hp_bf16x8, make_uint4(0u, 0u, 0u, 0u));
-    for (int m0 = wave * 16; m0 < m_out; m0 += 64) {
-        const int m = m0 + r;
-        const bf16_t* wrow = m < m_out ? w + (static_cast<int64_t>(h) * m_out + m) * k_in : nullptr;
-        hp_f32x4 acc[TT];
+    const int m = m0 + r;
+    const bf16_t* wrow = m < m_out ? w + (static_cast<int64_t>(h) * m_out + m) * k_in : nullptr;
+    hp_f32x4 acc[TT];
 #pragma unroll
-        for (int u = 0; u < TT; ++u) acc[u] = hp_f32x4{0.f, 0.f, 0.f, 0.f};
-        for (int k0 = 0; k0 < k_in; k0 += 32) {
-            const int k = k0 + 8 * g;
+    for (int u = 0; u < TT; ++u) acc[u] = hp_f32x4{0.f, 0.f, 0.f, 0.f};
+    constexpr int AHEAD = TT == 1 ? 4 : 2;
+    for (int k0 = share * 32; k0 < k_in; k0 += 32 * KW * AHEAD) {
+        hp_bf16x8 wa[AHEAD], xb[AHEAD][TT];
+#pragma unroll
+        for (int v = 0; v < AHEAD; ++v) {
+            const int k = k0 + 32 * KW * v + 8 * g;
             const bool in = k < k_in;
-            const hp_bf16x8 wa = (in && wrow) ? *reinterpret_cast<const hp_bf16x8*>(wrow + k) : zero;
+            wa[v] = (in && wrow) ? *reinterpret_cast<const hp_bf16x8*>(wrow + k) : zero;
 #pragma unroll
-            for (int u = 0; u < TT; ++u) {
-                const hp_bf16x8 xb = in ? load8<TX>(xrow[u] + k) : zero;
-                acc[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa, xb, acc[u], 0, 0, 0);
-            }
+            for (int u = 0; u < TT; ++u) xb[v][u] = in ? load8<TX>(xrow[u] + k) : zero;
         }
-        // lane: token r of every tile, channels m0 + 4 g + i
 #pragma unroll
-        for (int u = 0; u < TT; ++u) {
-            const int tok = t0 + 16 * u + r, c0 = m0 + 4 * g;
-            if (tok < tokens) {
-                bf16_t* dst = y + static_cast<int64_t>(tok) * y_stride + static_cast<int64_t>(h) * y_head + c0;
-                const bf16_t* gr = gate ? gate + static_cast<int64_t>(tok) * gate_stride + (gate_heads ? h : static_cast<int64_t>(h) * m_out + c0) : nullptr;
+        for (int v = 0; v < AHEAD; ++v)
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    if (c0 + i < m_out) {
-                        float v = acc[u][i] * scale;
-                        if (gr) v *= 1.0f / (1.0f + expf(-bf16_to_f32(gr[gate_heads ? 0 : i])));
-                        dst[i] = f32_to_bf16(v);
-                    }
+            for (int u = 0; u < TT; ++u) acc[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa[v], xb[v][u], acc[u], 0, 0, 0);
+    }
+    if constexpr (KW > 1) {
+#pragma unroll
+        for (int u = 0; u < TT; ++u) meet[wave][u][lane] = acc[u];
+        __syncthreads();
+        if (share != 0) return;
+#pragma unroll
+        for (int u = 0; u < TT; ++u)
+#pragma unroll
+            for (int i = 1; i < KW; ++i) acc[u] += meet[wave + i][u][lane];
+    }
+    // lane: token r of every tile, channels m0 + 4 g + i
+#pragma unroll
+    for (int u = 0; u < TT; ++u) {
+        const int tok = t0 + 16 * u + r, c0 = m0 + 4 * g;
+        if (tok < tokens) {
+            bf16_t* dst = y + static_cast<int64_t>(tok) * y_stride + static_cast<int64_t>(h) * y_head + c0;
+            const bf16_t* gr = gate ? gate + static_cast<int64_t>(tok) * gate_stride + (gate_heads ? h : static_cast<int64_t>(h) * m_out + c0) : nullptr;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                if (c0 + i < m_out) {
+                    float v = acc[u][i] * scale;
+                    if (gr) v *= 1.0f / (1.0f + expf(-bf16_to_f32(gr[gate_heads ? 0 : i])));
+                    dst[i] = f32_to_bf16(v);
                 }
             }
         }
@@ -415,14 +435,20 @@ extern "C" int pulse_heads_product(const void* x, int64_t x_stride, int x_head, 
     PULSE_REQUIRE(reinterpret_cast<uintptr_t>(x) % 16 == 0 && (x_stride * xb) % 16 == 0 && (static_cast<int64_t>(x_head) * xb) % 16 == 0 &&
                   reinterpret_cast<uintptr_t>(w) % 16 == 0, "heads_product: operands must be 16-byte aligned");
     if (tokens == 0) return 0;
-#define PULSE_HEADS(TT_)                                                                                                 \
+    // K shared out from 256 values on, while there are few tokens: there the walk along K is what a workgroup waits for.
+    const int kw = tokens < 256 && k_in >= 256 ? 4 : 1;
+    const unsigned tiles_m = (m_out + 15) / 16, groups = (tiles_m + 4 / kw - 1) / (4 / kw);
+    PULSE_REQUIRE(groups < 65536, "heads_product: %d output channels are too many", m_out);
+#define PULSE_HEADS(TT_, KW_)                                                                                            \
     PULSE_DISPATCH_DTYPE(x_dtype, TX,                                                                                    \
-        hipLaunchKernelGGL((heads_product_kernel<TX, TT_>), dim3((tokens + 16 * TT_ - 1) / (16 * TT_), heads), dim3(256), 0, \
+        hipLaunchKernelGGL((heads_product_kernel<TX, TT_, KW_>), dim3((tokens + 16 * TT_ - 1) / (16 * TT_), heads, groups), \
+                           dim3(256), 0,                                                                                 \
                            stream, static_cast<const TX*>(x), x_stride, x_head, static_cast<const bf16_t*>(w),           \
                            static_cast<const bf16_t*>(gate), gate_stride, static_cast<bf16_t*>(y), y_stride, y_head,     \
                            tokens, m_out, k_in, scale, gate_heads))
-    if (tokens >= 256) PULSE_HEADS(4);
-    else PULSE_HEADS(1);
+    if (tokens >= 256) PULSE_HEADS(4, 1);
+    else if (kw == 4) PULSE_HEADS(1, 4);
+    else PULSE_HEADS(1, 1);
 #undef PULSE_HEADS
     PULSE_LAUNCH_CHECK("heads_product");
     return 0;
