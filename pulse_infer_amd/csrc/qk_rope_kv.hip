@@ -221,18 +221,16 @@ __device__ __forceinline__ uint32_t pack2(float lo, float hi) {
     return static_cast<uint32_t>(f32_to_bf16(lo)) | (static_cast<uint32_t>(f32_to_bf16(hi)) << 16);
 }
 
+// One wavefront of it: the heads from number `y` * 64 / LPH on of token t.
 template <typename TW, int PAIRING, int LPH>
-__global__ __launch_bounds__(64) void qk_rope_kv_vec_kernel(bf16_t* __restrict__ qkv, const TW* __restrict__ q_w,
-                                                            const TW* __restrict__ k_w, const float* __restrict__ cos_t,
-                                                            const float* __restrict__ sin_t, bf16_t* __restrict__ kcache,
-                                                            bf16_t* __restrict__ vcache, const int* __restrict__ positions,
-                                                            const int* __restrict__ token_entry,
-                                                            const int* __restrict__ block_table, QkRopeArgs a) {
+__device__ __forceinline__ void qk_rope_rows(int t, int y, int lane, bf16_t* __restrict__ qkv, const TW* __restrict__ q_w,
+                                             const TW* __restrict__ k_w, const float* __restrict__ cos_t,
+                                             const float* __restrict__ sin_t, bf16_t* __restrict__ kcache,
+                                             const int* __restrict__ positions, const int* __restrict__ token_entry,
+                                             const int* __restrict__ block_table, const QkRopeArgs& a) {
     constexpr int HPW = PULSE_WAVE / LPH;
-    const int t = blockIdx.x;
-    const int lane = threadIdx.x;
     const int c = lane % LPH;
-    const int hh = blockIdx.y * HPW + lane / LPH;
+    const int hh = y * HPW + lane / LPH;
     const int heads = a.write_kv ? a.nq + a.nkv : a.nq;
     const int d = a.d;
     const int half_rot = a.rotary_dim / 2;
@@ -342,16 +340,13 @@ __global__ __launch_bounds__(64) void qk_rope_kv_vec_kernel(bf16_t* __restrict__
 // just as correctly, only in smaller pieces).  Written from the kernel above, a token at a time, the same bytes
 // took twice as long as everything else that kernel does.
 constexpr int VW_TOKENS = 16;
-constexpr int VW_THREADS = 256;
+constexpr int VEC_THREADS = 256;
 
-__global__ __launch_bounds__(VW_THREADS) void v_page_write_kernel(const bf16_t* __restrict__ qkv, bf16_t* __restrict__ vcache,
-                                                                  const int* __restrict__ positions,
-                                                                  const int* __restrict__ token_entry,
-                                                                  const int* __restrict__ block_table, QkRopeArgs a,
-                                                                  int tokens) {
-    const int t = blockIdx.x * VW_TOKENS + threadIdx.x % VW_TOKENS;
+__device__ __forceinline__ void v_page_rows(int tile, int g, const bf16_t* __restrict__ qkv, bf16_t* __restrict__ vcache,
+                                            const int* __restrict__ positions, const int* __restrict__ token_entry,
+                                            const int* __restrict__ block_table, const QkRopeArgs& a, int tokens) {
+    const int t = tile * VW_TOKENS + threadIdx.x % VW_TOKENS;
     const int cg = threadIdx.x / VW_TOKENS;
-    const int g = blockIdx.y;
     if (t >= tokens) return;
     const int pos = positions[t];
     const int page = block_table[static_cast<int64_t>(token_entry[t]) * a.bt_width + pos / a.page_size];
@@ -359,7 +354,7 @@ __global__ __launch_bounds__(VW_THREADS) void v_page_write_kernel(const bf16_t* 
     const int slot = pos % a.page_size;
     const bf16_t* src = qkv + static_cast<int64_t>(t) * a.row_stride + static_cast<int64_t>(a.v_head0 + g) * a.d;
     bf16_t* dst = vcache + (static_cast<int64_t>(page) * a.nkv + g) * a.d * a.page_size + slot;
-    for (int c0 = cg * 8; c0 < a.d; c0 += 8 * (VW_THREADS / VW_TOKENS)) {
+    for (int c0 = cg * 8; c0 < a.d; c0 += 8 * (VEC_THREADS / VW_TOKENS)) {
         const uint4 raw = *reinterpret_cast<const uint4*>(src + c0);
         const uint32_t words[4] = {raw.x, raw.y, raw.z, raw.w};
 #pragma unroll
@@ -368,13 +363,46 @@ __global__ __launch_bounds__(VW_THREADS) void v_page_write_kernel(const bf16_t* 
     }
 }
 
+// Both in one launch: the first `rope_groups` workgroups are four wavefronts of rows each, the others 16 tokens' values of a
+// kv head.  (Neither reads what the other writes: q's columns are the only ones written in place, and the values are never
+// among them.)  Two launches took 4.0 + 2.9 us at 97 tokens, 5.6 + 4.8 at 509, 12.3 + 5.3 at 2,048 (32 + 8 heads of 128);
+// one 4.0, 5.7, 15.6.
+template <typename TW, int PAIRING, int LPH>
+__global__ __launch_bounds__(VEC_THREADS) void qk_rope_kv_vec_kernel(bf16_t* __restrict__ qkv, const TW* __restrict__ q_w,
+                                                                     const TW* __restrict__ k_w,
+                                                                     const float* __restrict__ cos_t,
+                                                                     const float* __restrict__ sin_t,
+                                                                     bf16_t* __restrict__ kcache, bf16_t* __restrict__ vcache,
+                                                                     const int* __restrict__ positions,
+                                                                     const int* __restrict__ token_entry,
+                                                                     const int* __restrict__ block_table, QkRopeArgs a,
+                                                                     int tokens, int per_token, int rope_groups) {
+    const int b = blockIdx.x;
+    if (b < rope_groups) {
+        const int64_t row = static_cast<int64_t>(b) * (VEC_THREADS / PULSE_WAVE) + threadIdx.x / PULSE_WAVE;
+        if (row >= static_cast<int64_t>(tokens) * per_token) return;
+        qk_rope_rows<TW, PAIRING, LPH>(static_cast<int>(row / per_token), static_cast<int>(row % per_token),
+                                       threadIdx.x % PULSE_WAVE, qkv, q_w, k_w, cos_t, sin_t, kcache, positions, token_entry,
+                                       block_table, a);
+    } else {
+        v_page_rows((b - rope_groups) / a.nkv, (b - rope_groups) % a.nkv, qkv, vcache, positions, token_entry, block_table, a,
+                    tokens);
+    }
+}
+
 template <typename TW, int PAIRING>
-void launch_vec(int lph, dim3 block, hipStream_t stream, int tokens, int heads, bf16_t* qkv, const TW* q_w, const TW* k_w,
+void launch_vec(int lph, hipStream_t stream, int tokens, int heads, bf16_t* qkv, const TW* q_w, const TW* k_w,
                 const float* cos_t, const float* sin_t, bf16_t* kcache, bf16_t* vcache, const int* positions,
                 const int* token_entry, const int* block_table, const QkRopeArgs& a) {
+    const int value_groups = a.write_kv ? (tokens + VW_TOKENS - 1) / VW_TOKENS * a.nkv : 0;
 #define PULSE_VEC(L)                                                                                                    \
-    hipLaunchKernelGGL((qk_rope_kv_vec_kernel<TW, PAIRING, L>), dim3(tokens, (heads + 64 / L - 1) / (64 / L)), block, 0,  \
-                       stream, qkv, q_w, k_w, cos_t, sin_t, kcache, vcache, positions, token_entry, block_table, a)
+    do {                                                                                                                \
+        const int per_token = (heads + 64 / L - 1) / (64 / L);                                                          \
+        const int rope_groups = static_cast<int>((static_cast<int64_t>(tokens) * per_token + 3) / 4);                   \
+        hipLaunchKernelGGL((qk_rope_kv_vec_kernel<TW, PAIRING, L>), dim3(rope_groups + value_groups), dim3(VEC_THREADS), 0, \
+                           stream, qkv, q_w, k_w, cos_t, sin_t, kcache, vcache, positions, token_entry, block_table, a,  \
+                           tokens, per_token, rope_groups);                                                             \
+    } while (0)
     if (lph <= 2) PULSE_VEC(2);
     else if (lph <= 4) PULSE_VEC(4);
     else if (lph <= 8) PULSE_VEC(8);
@@ -419,6 +447,7 @@ extern "C" int pulse_qk_rope_kv(void* qkv, int x_dtype, int64_t row_stride, cons
     a.page_size = page_size; a.num_pages = num_pages; a.bt_width = bt_width; a.write_kv = write_kv;
     a.norm = q_w ? 1 : (plain_norm ? 2 : 0); a.v_head0 = v_head0; a.temp_coef = temp_coef; a.temp_every = temp_every;
     const int heads = write_kv ? nq + nkv : nq;
+    PULSE_REQUIRE(static_cast<int64_t>(tokens) * heads < (1ll << 30), "qk_rope_kv: %d tokens of %d heads are too many", tokens, heads);
     // the 16-byte path: bfloat16 activations and cache, 8-element chunks that the rotation does not cut
     const bool vec = x_dtype == PULSE_BF16 && (!write_kv || c_dtype == PULSE_BF16) && d % 8 == 0 && a.rotary_dim % 8 == 0 && row_stride % 8 == 0 &&
                      (reinterpret_cast<uintptr_t>(qkv) % 16) == 0 && (reinterpret_cast<uintptr_t>(kcache) % 16) == 0 &&
@@ -428,20 +457,14 @@ extern "C" int pulse_qk_rope_kv(void* qkv, int x_dtype, int64_t row_stride, cons
         const int lph = d / 8;
         PULSE_DISPATCH_DTYPE(w_dtype, TW,
             if (pairing == 0)
-                launch_vec<TW, 0>(lph, dim3(64), stream, tokens, heads, static_cast<bf16_t*>(qkv), static_cast<const TW*>(q_w),
+                launch_vec<TW, 0>(lph, stream, tokens, heads, static_cast<bf16_t*>(qkv), static_cast<const TW*>(q_w),
                                   static_cast<const TW*>(k_w), cos_t, sin_t, static_cast<bf16_t*>(kcache),
                                   static_cast<bf16_t*>(vcache), positions, token_entry, block_table, a);
             else
-                launch_vec<TW, 1>(lph, dim3(64), stream, tokens, heads, static_cast<bf16_t*>(qkv), static_cast<const TW*>(q_w),
+                launch_vec<TW, 1>(lph, stream, tokens, heads, static_cast<bf16_t*>(qkv), static_cast<const TW*>(q_w),
                                   static_cast<const TW*>(k_w), cos_t, sin_t, static_cast<bf16_t*>(kcache),
                                   static_cast<bf16_t*>(vcache), positions, token_entry, block_table, a));
         PULSE_LAUNCH_CHECK("qk_rope_kv");
-        if (write_kv) {
-            hipLaunchKernelGGL(v_page_write_kernel, dim3((tokens + VW_TOKENS - 1) / VW_TOKENS, nkv), dim3(VW_THREADS), 0, stream,
-                               static_cast<const bf16_t*>(qkv), static_cast<bf16_t*>(vcache), positions, token_entry,
-                               block_table, a, tokens);
-            PULSE_LAUNCH_CHECK("v_page_write");
-        }
         return 0;
     }
     const dim3 grid(tokens, heads);
