@@ -60,6 +60,8 @@ struct RowView {
 
 template <bool V>
 struct Is { static constexpr bool value = V; };
+template <int V>
+struct Int { static constexpr int value = V; };
 
 // f(Is<row.masked()>)
 template <typename F>
@@ -138,7 +140,7 @@ __device__ void block_argmax(float& v, int& idx, float* sv, int* si) {
 template <typename Weight>
 __device__ int wave_walk(int begin, int end, float rest, Weight weight, int& last) {
     const int lane = threadIdx.x % PULSE_WAVE;
-    constexpr int AHEAD = 8;   // steps of 64 entries whose weights are asked for together (a step's trip to memory
+    constexpr int AHEAD = 16;  // steps of 64 entries whose weights are asked for together (a step's trip to memory
                                // would otherwise be waited for before the next one starts)
     float run = 0.f;
     last = -1;
@@ -257,7 +259,7 @@ __device__ __forceinline__ void add_in_group(float* p, float v) {
     __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
-constexpr int CANDIDATES = 15;   // thresholds whose masses are summed side by side in a pass
+constexpr int CANDIDATES = 15;   // most thresholds whose masses are summed side by side in a pass
 
 // The largest threshold t with M(t) >= want (see sample_kernel), from the histogram of a row under top-p alone; false where
 // the bracket does not hold it (or too many tokens share the bins), and then nothing is said.  Called by a whole workgroup.
@@ -278,7 +280,6 @@ __device__ bool nucleus_edge(const RowView& row, float want, float best, float i
     __syncthreads();
     if (lane == PULSE_WAVE - 1) sf[wave] = pre;
     if (threadIdx.x == 0) { si[0] = HIST_BINS; si[1] = 0; *nearest = ~0ull; }
-    if (threadIdx.x < CANDIDATES) cand[threadIdx.x] = 0u;
     __syncthreads();
     float before = 0.f;
     for (int w = 0; w < wave; ++w) before += sf[w];
@@ -332,39 +333,48 @@ __device__ bool nucleus_edge(const RowView& row, float want, float best, float i
     }
     __syncthreads();
     if (*nearest == ~0ull) return false;
-    const int first = static_cast<int>(*nearest) - CANDIDATES / 2;
+    // M at the places round that one.  The histogram's masses are good to a few units in the last place of the whole, which is
+    // less than a token there unless the row is very flat: two places to either side first, seven where those do not hold it.
+    auto try_round = [&](auto count) __attribute__((always_inline)) {
+        constexpr int C = decltype(count)::value;
+        const int first = static_cast<int>(*nearest) - C / 2;
+        __syncthreads();
+        if (threadIdx.x < C) cand[threadIdx.x] = 0u;
+        __syncthreads();
 #pragma unroll
-    for (int u = 0; u < LIST_CAP / SAMPLE_THREADS; ++u)
-        if (place[u] >= first && place[u] >= 0 && place[u] < first + CANDIDATES) cand[place[u] - first] = keys[u];
-    __syncthreads();
-    // M at the candidates (equal tokens share a place, and the places behind it stay empty: 0)
-    uint32_t t[CANDIDATES], least = 0xffffffffu;
-    float above[CANDIDATES];
+        for (int u = 0; u < LIST_CAP / SAMPLE_THREADS; ++u)
+            if (place[u] >= first && place[u] >= 0 && place[u] < first + C) cand[place[u] - first] = keys[u];
+        __syncthreads();
+        // (equal tokens share a place, and the places behind it stay empty: 0)
+        uint32_t t[C], least = 0xffffffffu;
+        float above[C];
 #pragma unroll
-    for (int j = 0; j < CANDIDATES; ++j) {
-        t[j] = cand[j];
-        above[j] = 0.f;
-        if (t[j] != 0u && t[j] < least) least = t[j];
-    }
-    sweep(row, threadIdx.x, row.vocab, SAMPLE_THREADS, [&](int, float x) {
-        if (x == -INFINITY) return;
-        const uint32_t key = order_key(x);
-        if (key < least) return;
-        const float w = expf((x - best) * inv_t);
+        for (int j = 0; j < C; ++j) {
+            t[j] = cand[j];
+            above[j] = 0.f;
+            if (t[j] != 0u && t[j] < least) least = t[j];
+        }
+        sweep(row, threadIdx.x, row.vocab, SAMPLE_THREADS, [&](int, float x) {
+            if (x == -INFINITY) return;
+            const uint32_t key = order_key(x);
+            if (key < least) return;
+            const float w = expf((x - best) * inv_t);
 #pragma unroll
-        for (int j = 0; j < CANDIDATES; ++j)
-            if (key >= t[j]) above[j] += w;
-    });
-    bool below = false, found = false;      // a larger candidate's mass falls short; the first that does not is known
+            for (int j = 0; j < C; ++j)
+                if (key >= t[j]) above[j] += w;
+        });
+        bool below = false, found = false, open = true;      // a larger candidate's mass falls short; the first that does not is known
 #pragma unroll
-    for (int j = 0; j < CANDIDATES; ++j) {
-        const float m = block_sum_f(above[j], sf);
-        if (t[j] == 0u || found) continue;
-        if (m < want) below = true;
-        else if (below) { found = true; thr = t[j]; }
-        else return false;                  // (the same for every thread)
-    }
-    return found;
+        for (int j = 0; j < C; ++j) {
+            const float m = block_sum_f(above[j], sf);
+            if (t[j] == 0u || found || !open) continue;
+            if (m < want) below = true;
+            else if (below) { found = true; thr = t[j]; }
+            else open = false;                               // (the same for every thread)
+        }
+        return found;
+    };
+    return try_round(Int<5>()) || try_round(Int<CANDIDATES>());
 }
 
 __global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
@@ -578,7 +588,7 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
         float want;
         if (!by_k && bin_scale > 0.f) {
             // Top-p alone: the histogram's masses say near which token the sum reaches `want`; the tokens of that bin and
-            // its neighbours are ranked, and M is summed, in its own order, for the fifteen round that place side by side.
+            // its neighbours are ranked, and M is summed, in its own order, for the five (or fifteen) round that place side by side.
             // (A search for the threshold's bits, four a pass, takes eight such passes.  32 rows of 151,936, this kernel:
             // 661 us with the search, 377 with this, 158 with the mass and the histogram made by the kernels in front.)
             want = p * whole;
@@ -1036,7 +1046,7 @@ __global__ __launch_bounds__(PULSE_WAVE) void chunked_choose_kernel(
 // ---- the rows that are left, before sample_kernel ---------------------------------------------------------------
 // A workgroup a row goes over its row at the rate of one compute unit; of what sample_kernel needs to know of the whole row,
 // the mass (a wavefront of it summed by a wavefront here, entries and order as there), the smallest number and the
-// histogram are made by as many workgroups as there are wavefronts in it, and by eight: 17 and 30 us for 13 rows of 151,936,
+// histogram are made by as many workgroups as there are wavefronts in it: 17 and 30 us for 13 rows of 151,936,
 // where the passes inside sample_kernel took 220.
 __global__ __launch_bounds__(PULSE_WAVE) void rest_mass_kernel(
     const float* __restrict__ logits, int vocab, int64_t row_stride, const float* __restrict__ temperature,
@@ -1070,7 +1080,7 @@ __global__ __launch_bounds__(PULSE_WAVE) void rest_mass_kernel(
     }
 }
 
-constexpr int REST_GROUPS = 8;
+constexpr int REST_GROUPS = 16;
 
 __global__ __launch_bounds__(SIMPLE_THREADS) void rest_histogram_kernel(
     const float* __restrict__ logits, int vocab, int64_t row_stride, const float* __restrict__ temperature,
