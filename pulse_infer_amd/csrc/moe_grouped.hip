@@ -376,9 +376,9 @@ struct GroupArgs {
 
 constexpr int GROUP_PANEL = 4;   // tiles of rows a panel of the tile order
 
-template <bool DOWN, int WR, int XR, int WN, int WM, int S>
-__global__ __launch_bounds__(256) void moe_tile_kernel(GroupArgs a) {
-    using Loop = TileLoop<WR, XR, WN, WM, S>;
+template <bool DOWN, int WR, int XR, int WN, int WM, int S, bool NT>
+__global__ __launch_bounds__(WN* WM* PULSE_WAVE) void moe_tile_kernel(GroupArgs a) {
+    using Loop = TileLoop<WR, XR, WN, WM, S, NT>;
     constexpr int COLS = DOWN ? WR : WR / 2;       // output columns of a tile
     __shared__ __attribute__((aligned(1024))) char lds[Loop::LDS];
     __shared__ int pair_s[XR];
@@ -398,7 +398,7 @@ __global__ __launch_bounds__(256) void moe_tile_kernel(GroupArgs a) {
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid / PULSE_WAVE);
     const int lane = tid % PULSE_WAVE;
-    for (int i = tid; i < XR; i += 256) {
+    for (int i = tid; i < XR; i += Loop::NW * PULSE_WAVE) {
         const int p = i < rows ? a.order[row0 + i] : -1;
         pair_s[i] = p;
         weight_s[i] = p >= 0 && a.in_weight ? a.in_weight[p] : 1.f;
@@ -424,7 +424,7 @@ __global__ __launch_bounds__(256) void moe_tile_kernel(GroupArgs a) {
 
     // Results leave through LDS, a wavefront's 32 rows at a time, in whole 16-byte pieces of rows.
     constexpr int TN = Loop::TN, TM = Loop::TM;
-    constexpr int WAVE_LDS = Loop::LDS / 4;
+    constexpr int WAVE_LDS = Loop::LDS / Loop::NW;
     char* mine = lds + wave * WAVE_LDS;
     const int wave_n = wave % WN, wave_m = wave / WN, h = lane / 32;
     const int n_wave = n0 + wave_n * TN * (DOWN ? 32 : 16);
@@ -499,28 +499,35 @@ __global__ __launch_bounds__(256) void moe_tile_kernel(GroupArgs a) {
     }
 }
 
-template <bool DOWN, int WR, int XR, int WN, int WM, int S>
+template <bool DOWN, int WR, int XR, int WN, int WM, int S, bool NT>
 void launch_tiles(GroupArgs a, int max_tiles, hipStream_t stream) {
     constexpr int COLS = DOWN ? WR : WR / 2;
     a.tiles_n = (a.N + COLS - 1) / COLS;
     const int64_t grid = (static_cast<int64_t>(max_tiles) * a.tiles_n + 7) / 8 * 8;
-    hipLaunchKernelGGL((moe_tile_kernel<DOWN, WR, XR, WN, WM, S>), dim3(static_cast<unsigned>(grid)), dim3(256), 0, stream, a);
+    hipLaunchKernelGGL((moe_tile_kernel<DOWN, WR, XR, WN, WM, S, NT>), dim3(static_cast<unsigned>(grid)), dim3(WN * WM * PULSE_WAVE), 0,
+                       stream, a);
 }
 
 // Which shape a list's tiles take: lists of 32 rows (decoding) and of 64 are bound by the weights' way from memory, lists of
-// 128 by the matrix cores.  Measured, 16 experts of 1,536 x 4,096, 4 chosen a token, gate and up / down in us, at 8, 64, 211,
-// 400, 600, 1,024, 2,048 tokens:
-//   32 rows (weights 128, 3 stages)    79 / 28    85 / 31   109 / 43   165 / 65
-//   64 rows (weights 128, 3 stages)    79 / 28    84 / 32    89 / 39   105 / 40   150 / 60   219 / 106   359 / 195
-//   128 rows (weights 256, 3 stages)   92 / 31    97 / 34   103 / 37   105 / 39   157 / 62   146 / 99    277 / 169
-//   tiles of 256 x 256, 2 stages                                                  264 / 96   273 / 159   283 / 178
-//   as before: 32 rows, K shared out   78 / 33   110 / 57   219 / 132
-//   as before: 128 rows, X in LDS     150 / 81   150 / 81   184 / 104                        370 / 318   522 / 511
+// 128 by the matrix cores.  `once`: an expert's weights are read for one tile or hardly more, and go past the caches; where
+// two tiles of an expert follow each other they find each other's weights there.  Measured, 16 experts of 1,536 x 4,096, 4
+// chosen a token, gate and up alone / with down in us, at 8, 64, 130, 211, 300, 400, 500, 600, 1,024, 2,048 tokens:
+//   32 rows (weights 128, 3 stages)         79/115  84/125  109/159
+//     once                                  71/103  74/110  116/168
+//     once, weights 64 (2 wavefronts, 4)    68/101  70/110  105/161
+//   64 rows (weights 128, 3 stages)         79/115  85/126   89/131   88/142  108/178  101/168  124/199  148/238  215/335  348/561
+//     once                                  70/103  75/111   77/117   86/139  135/213  124/201  154/241  211/319  257/405  501/755
+//   128 rows (weights 256, 3 stages)                96/138  101/147  102/150  104/154  107/158  151/227  164/236  132/239  259/425
+//     once                                          90/130   94/134   95/139   95/144   97/145  154/220  163/239  143/246  271/432
+//   the kernels above, 32 rows, K shared    78/111 110/167  219/351
+//   the kernels above, 128 rows            150/231 150/231           184/288           370/688 (at 400 tokens)
 template <bool DOWN>
-void launch_tiles_for(const GroupArgs& a, int max_tiles, int rows, hipStream_t stream) {
-    if (rows <= 32) launch_tiles<DOWN, 128, 32, 4, 1, 3>(a, max_tiles, stream);
-    else if (rows <= 64) launch_tiles<DOWN, 128, 64, 4, 1, 3>(a, max_tiles, stream);
-    else launch_tiles<DOWN, 256, 128, 2, 2, 3>(a, max_tiles, stream);
+void launch_tiles_for(const GroupArgs& a, int max_tiles, int rows, bool once, hipStream_t stream) {
+    if (rows <= 32) launch_tiles<DOWN, 64, 32, 2, 1, 4, true>(a, max_tiles, stream);
+    else if (rows <= 64 && once) launch_tiles<DOWN, 128, 64, 4, 1, 3, true>(a, max_tiles, stream);
+    else if (rows <= 64) launch_tiles<DOWN, 128, 64, 4, 1, 3, false>(a, max_tiles, stream);
+    else if (once) launch_tiles<DOWN, 256, 128, 2, 2, 3, true>(a, max_tiles, stream);
+    else launch_tiles<DOWN, 256, 128, 2, 2, 3, false>(a, max_tiles, stream);
 }
 
 }  // namespace
@@ -544,7 +551,7 @@ static bool aligned16(const void* p) { return reinterpret_cast<uintptr_t>(p) % 1
 
 extern "C" int pulse_moe_gate_up_grouped(const void* x, const void* wg, const void* wu, const int* order,
                                          const int* tile_expert, const int* tile_row0, const int* tile_rows,
-                                         const int* num_tiles, int max_tiles, int tile_rows_max, void* act, int hidden,
+                                         const int* num_tiles, int max_tiles, int tile_rows_max, int once, void* act, int hidden,
                                          int ff, int top, const float* in_weight, int act_kind, float limit,
                                          hipStream_t stream) {
     PULSE_REQUIRE(act_kind == 0 || act_kind == 1, "moe_gate_up_grouped: unknown activation %d", act_kind);
@@ -558,7 +565,7 @@ extern "C" int pulse_moe_gate_up_grouped(const void* x, const void* wg, const vo
     if (hidden % 64 == 0 && ff % 8 == 0 && aligned16(act)) {   // (the loop walks K in whole steps of 64; rows leave in 16-byte pieces)
         launch_tiles_for<false>({static_cast<const bf16_t*>(x), {static_cast<const bf16_t*>(wg), static_cast<const bf16_t*>(wu)},
                                  act, order, tile_expert, tile_row0, tile_rows, num_tiles, in_weight, hidden, ff, top, 0,
-                                 act_kind, limit}, max_tiles, tile_rows_max, stream);
+                                 act_kind, limit}, max_tiles, tile_rows_max, once != 0, stream);
         PULSE_LAUNCH_CHECK("moe_gate_up_grouped");
         return 0;
     }
@@ -577,7 +584,7 @@ extern "C" int pulse_moe_gate_up_grouped(const void* x, const void* wg, const vo
 
 extern "C" int pulse_moe_down_grouped(const void* act, const void* wd, const int* order, const int* tile_expert,
                                       const int* tile_row0, const int* tile_rows, const int* num_tiles, int max_tiles,
-                                      int tile_rows_max, float* y, int hidden, int ff, hipStream_t stream) {
+                                      int tile_rows_max, int once, float* y, int hidden, int ff, hipStream_t stream) {
     PULSE_REQUIRE(hidden > 0 && ff > 0 && max_tiles > 0, "moe_down_grouped: bad sizes");
     PULSE_REQUIRE(ff % 8 == 0 && aligned16(act) && aligned16(wd),
                   "moe_down_grouped: rows must be multiples of 8 values and 16-byte aligned");
@@ -588,7 +595,7 @@ extern "C" int pulse_moe_down_grouped(const void* act, const void* wd, const int
     if (ff % 64 == 0 && hidden % 4 == 0 && aligned16(y)) {
         launch_tiles_for<true>({static_cast<const bf16_t*>(act), {static_cast<const bf16_t*>(wd), nullptr}, y, order, tile_expert,
                                 tile_row0, tile_rows, num_tiles, nullptr, ff, hidden, 1, 0, 0, 0.f}, max_tiles, tile_rows_max,
-                               stream);
+                               once != 0, stream);
         PULSE_LAUNCH_CHECK("moe_down_grouped");
         return 0;
     }

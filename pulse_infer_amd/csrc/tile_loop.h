@@ -1,5 +1,5 @@
-// The loop of a matrix product on an output tile of WR weight rows x XR rows of X, bfloat16 operands, float32 sums: four
-// wavefronts, WN along the weight rows and WM along the rows of X, on v_mfma_f32_32x32x16_bf16.
+// The loop of a matrix product on an output tile of WR weight rows x XR rows of X, bfloat16 operands, float32 sums:
+// WN wavefronts along the weight rows by WM along the rows of X, on v_mfma_f32_32x32x16_bf16.
 //
 // K goes in steps of 64 through S stages of LDS (the tile's rows of W, then of X, 128 bytes a row), filled straight from
 // memory; S - 1 steps are on their way while one is multiplied, and there is one barrier a step: behind it, this step's
