@@ -7,13 +7,19 @@
 // chosen for the least of them (`plan_for`).  Measured with weights from memory, us, against the vendor library's product
 // (gate and up: with its pass for SwiGLU behind it) and this package's shared-out product for up to 192 rows:
 //                                   97 rows              192                  357                 509
-//   gate + up, 24,576 x 4,096       45 (library 56)      55 (66)              97 (84)             105 (96)
-//   qkv, 6,144 x 4,096              20 (26)              27 (36)              29 (40)             30 (36)
-//   o, 4,096 x 4,096, shares        12 (25; 16 shared)   14 (39; 21 shared)   23 (29)             22 (28)
-//   down, 4,096 x 12,288, shares    24 (45; 33 shared)   31 (92; 45 shared)   47 (67)             53 (83)
-// Weights are read past the caches (nontemporal): 5 % where they are the time.
+//   gate + up, 24,576 x 4,096       44 (library 54)      54 (64)              71 (84)             87 (96)
+//   qkv, 6,144 x 4,096              20 (25)              26 (36)              30 (41)             33 (42)
+//   o, 4,096 x 4,096, shares        13 (25; 16 shared)   17 (37; 21 shared)   22 (29)             24 (32)
+//   down, 4,096 x 12,288, shares    25 (44; 34 shared)   33 (92; 47 shared)   42 (52 shared)      51 (59 shared)
+// From some 260 rows on tiles of 192 or 256 rows of X (their weights through three stages, X, which comes from L2, through
+// two where LDS holds no third) take the place of the library's: 357 rows of gate + up ran 96 us in tiles of 192 x 128.
+// Steps of 32 of K in twice the stages, the other way to fit such tiles, bring 64 bytes of a row at a time, which a unit
+// takes in at half the rate (192 x 256: 107 us).
+// Weights are read past the caches (nontemporal) by tiles of up to 128 rows of X: 5 % where they are the time; the larger
+// tiles, whose weights are read by several, lose 2 % by it.
 #include "common.h"
 #include "tile_loop.h"
+#include <algorithm>
 
 namespace {
 
@@ -34,9 +40,9 @@ struct StageArgs {
 
 constexpr int PANEL = 8;  // tiles of rows a panel of the tile order
 
-template <int MODE, int WR, int XR, int WN, int WM, int S>
+template <int MODE, int WR, int XR, int WN, int WM, int S, int SX, bool NT>
 __global__ __launch_bounds__(256) void gemm_stages_kernel(StageArgs a) {
-    using Loop = TileLoop<WR, XR, WN, WM, S, true>;
+    using Loop = TileLoop<WR, XR, WN, WM, S, NT, SX>;
     __shared__ __attribute__((aligned(1024))) char lds[Loop::LDS];
 
     // The workgroups of a die (every eighth) take neighbouring tiles, in panels of eight tiles of rows, which share
@@ -128,16 +134,17 @@ __global__ __launch_bounds__(256) void gemm_stages_kernel(StageArgs a) {
     }
 }
 
-template <int MODE, int WR, int XR, int WN, int WM, int S>
+template <int MODE, int WR, int XR, int WN, int WM, int S, int SX = S, bool NT = true>
 void launch(StageArgs a, hipStream_t stream) {
     a.tiles_m = (a.M + XR - 1) / XR;
     a.tiles_n = (a.N + WR - 1) / WR;
     const int64_t grid = (static_cast<int64_t>(a.tiles_m) * a.tiles_n * a.splits + 7) / 8 * 8;
-    hipLaunchKernelGGL((gemm_stages_kernel<MODE, WR, XR, WN, WM, S>), dim3(static_cast<unsigned>(grid)), dim3(256), 0, stream, a);
+    hipLaunchKernelGGL((gemm_stages_kernel<MODE, WR, XR, WN, WM, S, SX, NT>), dim3(static_cast<unsigned>(grid)), dim3(256), 0, stream, a);
 }
 
 // weight rows and rows of X a tile (the kernels below, in this order)
-constexpr int SHAPES[][2] = {{32, 128}, {64, 64}, {64, 128}, {96, 128}, {128, 64}, {128, 128}, {192, 128}, {256, 128}};
+constexpr int SHAPES[][2] = {{32, 128}, {64, 64}, {64, 128}, {96, 128}, {128, 64}, {128, 128}, {192, 128}, {256, 128},
+                               {192, 192}, {192, 256}, {256, 192}, {256, 256}};
 constexpr int NUM_SHAPES = sizeof(SHAPES) / sizeof(SHAPES[0]);
 
 template <int MODE>
@@ -150,28 +157,41 @@ void launch_shape(int shape, const StageArgs& a, hipStream_t s) {
         case 4: return launch<MODE, 128, 64, 4, 1, 3>(a, s);
         case 5: return launch<MODE, 128, 128, 2, 2, 4>(a, s);
         case 6: return launch<MODE, 192, 128, 2, 2, 3>(a, s);
-        default: return launch<MODE, 256, 128, 2, 2, 3>(a, s);
+        case 7: return launch<MODE, 256, 128, 2, 2, 3>(a, s);
+        case 8: return launch<MODE, 192, 192, 2, 2, 3, 3, false>(a, s);
+        case 9: return launch<MODE, 192, 256, 2, 2, 3, 2, false>(a, s);
+        case 10: return launch<MODE, 256, 192, 2, 2, 3, 2, false>(a, s);
+        default: return launch<MODE, 256, 256, 2, 2, 3, 2, false>(a, s);
     }
 }
 
-struct Plan { int shape, splits; };
+struct Plan { int shape, splits; double ns; };
 
-// The shape (and, for float32 results in shares, their number: `shares` 0 leaves it open) whose fullest compute unit copies
-// least: workgroups on it x rows a stage x steps of K, in units of 128 bytes (3.2 ns on the whole), and for every share its
-// results' way to memory and back to whoever adds them up (8 bytes a value at 4 TB/s).
+// The shape (and, for float32 results in shares, their number: `shares` 0 leaves it open) of the least estimated time.  A
+// row of a stage (128 bytes) takes a compute unit 3.1 ns.  Tiles of more than 128 rows of X hold weights long enough for
+// their further rounds to find them near: 2 ns a row then, or what its products take on the matrix cores (1.13 x their
+// time at the rate of a large product, 5.5 flops a picosecond a unit), and 0.75 of that for a last round that leaves half
+// the units idle.  Every share adds its results' way to memory and back to whoever adds them up (8 bytes a value at 4
+// TB/s).  Estimated / measured, 24,576 x 4,096 with SwiGLU, us: 97 rows 96 x 128 44 / 44, 128 x 128 51 / 50; 357 rows
+// 192 x 192 76 / 71, 192 x 256 89 / 82; 509 rows 192 x 256 89 / 87, 256 x 256 111 / 104, 192 x 192 123 / 120; 700 rows
+// 192 x 192 139 / 132, 192 x 256 151 / 152; 1,024 rows 192 x 256 172 / 181.
 Plan plan_for(int M, int N, int K, int shares) {
     const int64_t units = pulse_compute_units();
-    Plan best{0, 1};
-    double least = 0.0;
+    Plan best{0, 1, 0.0};
     bool any = false;
     for (int splits = shares > 0 ? shares : 1; splits <= (shares > 0 ? shares : 16); ++splits) {
         if (K % (64 * splits)) continue;
         for (int i = 0; i < NUM_SHAPES; ++i) {
-            const int64_t tiles = static_cast<int64_t>((M + SHAPES[i][1] - 1) / SHAPES[i][1]) *
-                                  ((N + SHAPES[i][0] - 1) / SHAPES[i][0]) * splits;
-            const double cost = static_cast<double>((tiles + units - 1) / units) * (SHAPES[i][0] + SHAPES[i][1]) *
-                                    (K / splits / 64) + (shares == 1 ? 0.0 : splits * (8.0 / 4000.0 / 3.2) * M * N);
-            if (!any || cost < least) { best = {i, splits}; least = cost; any = true; }
+            const int wr = SHAPES[i][0], xr = SHAPES[i][1];
+            const int64_t tiles = static_cast<int64_t>((M + xr - 1) / xr) * ((N + wr - 1) / wr) * splits;
+            const int64_t rounds = (tiles + units - 1) / units, last = tiles - (rounds - 1) * units;
+            double row = rounds * 3.1;
+            if (xr > 128) {
+                const double later = std::max(2.0, 1.13 * wr * xr * 128.0 / (wr + xr) / 5500.0);
+                row = std::max(3.1, later) + (rounds - 1) * later - (rounds > 1 && 2 * last <= units ? 0.25 * later : 0.0);
+            }
+            const double ns = row * (wr + xr) * (K / splits / 64) + (shares == 1 ? 0.0 : splits * 8.0 / 4000.0 * M * N);
+            if (!any || ns < best.ns) { best = {i, splits, ns}; any = true; }
         }
     }
     return best;
@@ -196,6 +216,12 @@ extern "C" int pulse_gemm_stages_takes(int M, int N, int K, int mode, int splits
 extern "C" int pulse_gemm_stages_shares(int M, int N, int K) {
     if (!pulse_gemm_stages_takes(M, N, K, OUT_F32, 1)) return 0;
     return plan_for(M, N, K, 0).splits;
+}
+
+// The estimated time of bfloat16 results in nanoseconds, at most 2 s (0: a shape that the product
+// does not take).
+extern "C" int pulse_gemm_stages_time(int M, int N, int K) {
+    return pulse_gemm_stages_takes(M, N, K, OUT_BF16, 1) ? static_cast<int>(std::min(plan_for(M, N, K, 1).ns, 2e9)) : 0;
 }
 
 // mode 0: C [M, N] bfloat16.  mode 1: the rows of W alternate in slabs of 16 gate rows and their 16 up rows;

@@ -1,11 +1,12 @@
 // The loop of a matrix product on an output tile of WR weight rows x XR rows of X, bfloat16 operands, float32 sums:
 // WN wavefronts along the weight rows by WM along the rows of X, on v_mfma_f32_32x32x16_bf16.
 //
-// K goes in steps of 64 through S stages of LDS (the tile's rows of W, then of X, 128 bytes a row), filled straight from
-// memory; S - 1 steps are on their way while one is multiplied, and there is one barrier a step: behind it, this step's
-// stage is whole and the stage of the step before is free for the copies that go out between this step's products.  Many
-// stages are for what bounds a product of few rows, the weights' way from memory: a compute unit must have some tens of
-// kilobytes on their way all the time (6 TB/s x 2 us over 256 units: 48 KB).
+// K goes in steps of 64 through S stages of LDS for the tile's rows of W and SX for those of X (128 bytes a row), filled
+// straight from memory; S - 1 steps are on their way while one is multiplied, and there is one barrier a step, before its
+// last products: behind it, the next step's stages are whole, and this step's, whose operands everyone then holds, are free
+// for the copies that go out between these products and the next step's.  Many stages are for what bounds a product of few
+// rows, the weights' way from memory: a compute unit must have some tens of kilobytes on their way all the time (6 TB/s x
+// 2 us over 256 units: 48 KB).  X comes from L2 and may have one stage less: it goes out first.
 //
 // The tile of the matrix instruction is D[n][m] = W . X^T: lane l holds column m = l % 32 and rows n = 8 (i / 4) +
 // 4 (l / 32) + i % 4, i = 0 .. 15, of a 32 x 32 piece.
@@ -16,17 +17,19 @@ typedef __attribute__((ext_vector_type(8))) __bf16 tile_bf16x8;
 typedef __attribute__((ext_vector_type(4))) __bf16 tile_bf16x4;
 typedef __attribute__((ext_vector_type(16))) float tile_f32x16;
 
-template <int WR, int XR, int WN, int WM, int S, bool NT = false>
+template <int WR, int XR, int WN, int WM, int S, bool NT = false, int SX = S>
 struct TileLoop {
     static constexpr int BK = 64;
     static constexpr int ROW_BYTES = BK * 2;
-    static constexpr int STAGE = (WR + XR) * ROW_BYTES;
+    static constexpr int STAGE_W = WR * ROW_BYTES, STAGE_X = XR * ROW_BYTES, X0 = S * STAGE_W;
     static constexpr int NW = WN * WM;
     static constexpr int TN = WR / 32 / WN, TM = XR / 32 / WM;       // 32-row pieces a wavefront
     static constexpr int PER_W = WR / 8 / NW, PER_X = XR / 8 / NW;   // chunks of 1 KB (8 rows) a wavefront copies
     static constexpr int PER = PER_W + PER_X;
-    static constexpr int LDS = S * STAGE;
-    static_assert(WR % (8 * NW) == 0 && XR % (8 * NW) == 0 && TN >= 1 && TM >= 1 && S >= 2, "whole chunks and pieces a wavefront");
+    static constexpr int KK = BK / 16;                               // products of the matrix instruction's depth a step
+    static constexpr int LDS = X0 + SX * STAGE_X;
+    static_assert(WR % (8 * NW) == 0 && XR % (8 * NW) == 0 && TN >= 1 && TM >= 1 && SX >= 2 && S >= SX,
+                  "whole chunks and pieces a wavefront");
 
     // Piece c (16 bytes) of row r of a stage sits at place c ^ swz(r): the rows that neighbouring lanes read together then
     // lie in different places of what LDS serves at once.
@@ -46,23 +49,24 @@ struct TileLoop {
         const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(
             (void __attribute__((address_space(3)))*)(lds)));
         const int steps = K / BK;
-        auto copy = [&](int step, int stage, int j) __attribute__((always_inline)) {
-            const bf16_t* at = from[j] + min(step, steps - 1) * BK;
-            if (j < PER_W) {
-                const uint32_t to = lds0 + stage * STAGE + (wave * PER_W + j) * 1024;
+        // The j-th copy of a batch, X first; a batch: W of one step into its slot, X of another into its.
+        auto copy = [&](int step_w, int slot_w, int step_x, int slot_x, int j) __attribute__((always_inline)) {
+            if (j < PER_X) {
+                load_to_lds(from[PER_W + j] + min(step_x, steps - 1) * BK, lds0 + X0 + slot_x * STAGE_X + (wave * PER_X + j) * 1024);
+            } else {
+                const bf16_t* at = from[j - PER_X] + min(step_w, steps - 1) * BK;
+                const uint32_t to = lds0 + slot_w * STAGE_W + (wave * PER_W + j - PER_X) * 1024;
                 if constexpr (NT) stream_to_lds(at, to);
                 else load_to_lds(at, to);
-            } else {
-                load_to_lds(at, lds0 + stage * STAGE + WR * ROW_BYTES + (wave * PER_X + j - PER_W) * 1024);
             }
         };
         const int h = lane / 32, e = h ^ swz(lane % 32);
-        int w_at[4], x_at[4];
+        int w_at[KK], x_at[KK];
 #pragma unroll
-        for (int kk = 0; kk < 4; ++kk) {
+        for (int kk = 0; kk < KK; ++kk) {
             const int place = (e ^ (kk << 1)) * 16;
             w_at[kk] = (wave_n * TN * 32 + lane % 32) * ROW_BYTES + place;
-            x_at[kk] = (WR + wave_m * TM * 32 + lane % 32) * ROW_BYTES + place;
+            x_at[kk] = X0 + (wave_m * TM * 32 + lane % 32) * ROW_BYTES + place;
         }
 #pragma unroll
         for (int f = 0; f < TN; ++f)
@@ -71,46 +75,60 @@ struct TileLoop {
 #pragma unroll
                 for (int i = 0; i < 16; ++i) acc[f][g][i] = 0.f;
 
+        // The batch of step s, W of step s + S and X of step s + SX, goes out behind that step's barrier: FIRST copies of it
+        // between the step's last products, the others between the next step's.
+        constexpr int ALL = KK * TN * TM, FIRST = TN * TM * PER / ALL;
+        constexpr int LATER = (SX - 2) * PER + (S > SX ? PER_W : 0);   // copies behind the last that the next step needs
 #pragma unroll
-        for (int s = 0; s < S - 1; ++s)
+        for (int s = -S; s < -1; ++s)
 #pragma unroll
-            for (int j = 0; j < PER; ++j) copy(s, s, j);
-        int stage = 0;
+            for (int j = s + SX >= 0 ? 0 : PER_X; j < PER; ++j) copy(s + S, s + S, s + SX, s + SX, j);
+#pragma unroll
+        for (int j = 0; j < FIRST; ++j) copy(S - 1, S - 1, SX - 1, SX - 1, j);
+        tile_bf16x8 wf[2][TN], xf[2][TM];
+        auto read = [&](int slot_w, int slot_x, int kk, int buf) __attribute__((always_inline)) {
+#pragma unroll
+            for (int g = 0; g < TM; ++g) xf[buf][g] = *reinterpret_cast<const tile_bf16x8*>(lds + slot_x * STAGE_X + x_at[kk] + g * 32 * ROW_BYTES);
+#pragma unroll
+            for (int f = 0; f < TN; ++f) wf[buf][f] = *reinterpret_cast<const tile_bf16x8*>(lds + slot_w * STAGE_W + w_at[kk] + f * 32 * ROW_BYTES);
+        };
+        asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" : : "n"(LATER + FIRST) : "memory");
+        read(0, 0, 0, 0);
+        int sw = 0, sx = 0;
         for (int s = 0; s < steps; ++s) {
-            // this wavefront's copies of this step have landed, and behind the barrier everyone's have
-            asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" : : "n"((S - 2) * PER) : "memory");
-            const char* base = lds + stage * STAGE;
-            const int into = stage == 0 ? S - 1 : stage - 1;
-            tile_bf16x8 wf[2][TN], xf[2][TM];
-            auto read = [&](int kk, int buf) __attribute__((always_inline)) {
+            const int next_w = sw == S - 1 ? 0 : sw + 1, before_w = sw == 0 ? S - 1 : sw - 1;
+            const int next_x = sx == SX - 1 ? 0 : sx + 1, before_x = sx == 0 ? SX - 1 : sx - 1;
 #pragma unroll
-                for (int g = 0; g < TM; ++g) xf[buf][g] = *reinterpret_cast<const tile_bf16x8*>(base + x_at[kk] + g * 32 * ROW_BYTES);
-#pragma unroll
-                for (int f = 0; f < TN; ++f) wf[buf][f] = *reinterpret_cast<const tile_bf16x8*>(base + w_at[kk] + f * 32 * ROW_BYTES);
-            };
-            read(0, 0);
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int kk = 0; kk < 4; ++kk) {
-                if (kk < 3) read(kk + 1, (kk + 1) & 1);
+            for (int kk = 0; kk < KK; ++kk) {
+                __builtin_amdgcn_sched_barrier(0);
+                if (kk == KK - 1) {
+                    // this wavefront's copies of the next step have landed and its operands are here; behind the barrier
+                    // that holds for everyone
+                    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"(LATER) : "memory");
+                    read(next_w, next_x, 0, (kk + 1) & 1);
+                } else {
+                    read(sw, sx, kk + 1, (kk + 1) & 1);
+                }
                 __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                 for (int p = 0; p < TN * TM; ++p) {
                     acc[p / TM][p % TM] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[kk & 1][p / TM], xf[kk & 1][p % TM],
                                                                                   acc[p / TM][p % TM], 0, 0, 0);
                     __builtin_amdgcn_sched_barrier(0);
-                    // the copies, spread evenly over the step's products
-                    constexpr int ALL = 4 * TN * TM;
-                    const int q = kk * TN * TM + p;
+                    // the copies, spread evenly over the products
+                    const int q = (kk == KK - 1 ? 0 : kk + 1) * TN * TM + p;
 #pragma unroll
-                    for (int j = q * PER / ALL; j < (q + 1) * PER / ALL; ++j) copy(s + S - 1, into, j);
+                    for (int j = q * PER / ALL; j < (q + 1) * PER / ALL; ++j) {
+                        if (kk == KK - 1) copy(s + S, sw, s + SX, sx, j);
+                        else copy(s + S - 1, before_w, s + SX - 1, before_x, j);
+                    }
                     __builtin_amdgcn_sched_barrier(0);
                 }
             }
-            stage = stage == S - 1 ? 0 : stage + 1;
+            sw = next_w, sx = next_x;
         }
         // the last copies, which nobody reads, must not land in what follows
-        asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" : : : "memory");
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" : : : "memory");
     }
 };
 

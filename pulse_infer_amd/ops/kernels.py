@@ -456,6 +456,12 @@ def gemm_stages_shares(m: int, n: int, k: int) -> int:
     return int(library.load().pulse_gemm_stages_shares(_i32(m), _i32(n), _i32(k)))
 
 
+@functools.lru_cache(maxsize=4096)
+def gemm_stages_time(m: int, n: int, k: int) -> int:
+    """What ``gemm_stages`` is estimated to take for bfloat16 results, nanoseconds (a function of the sizes alone)."""
+    return int(library.load().pulse_gemm_stages_time(_i32(m), _i32(n), _i32(k)))
+
+
 def gemm_stages_takes(m: int, n: int, k: int, swiglu: bool = False) -> bool:
     """Whether ``gemm_stages`` takes a shape with bfloat16 results (as pulse_gemm_stages_takes)."""
     return m > 0 and n > 0 and k > 0 and k % 64 == 0 and n % (32 if swiglu else 8) == 0

@@ -254,13 +254,20 @@ class Linear:
             return out.is_contiguous() and out.data_ptr() % 16 == 0 and w.shape[0] % 4 == 0
         return out.dtype == torch.bfloat16 and out.stride(1) == 1 and out.stride(0) % 4 == 0 and out.data_ptr() % 16 == 0
 
-    # Where the product in stages is the fastest (the figures are beside its kernel): with SwiGLU inside and for updates
-    # in shares of a wide inner dimension up to 256 rows, beyond which the library's large tiles have the better of the
-    # matrix cores; for plain products and shares of a narrower one as long as the library leaves compute units idle (6,144
-    # weight rows of 4,096 at 1,024 rows 48 us against 51; 4,096 of 4,096 at 509 rows 22 against 28, at 700 33 against
-    # 34).  Small products stay where they are.
-    STAGE_ROWS = (65, 256)
-    STAGE_ROWS_NARROW = (512, 1024)     # updates in shares; plain products of at most 32 weight rows a compute unit
+    # Where the product in stages is the fastest (more figures are beside its kernel).  With SwiGLU inside: up to 768 rows
+    # where a compute unit gets 192 weight rows at most (gate and up of 24,576 x 4,096 at
+    # 357, 512 and 700 rows 74, 97 and 139 us, the library's product and the pass behind it 97, 105 and 165; of 34,816 x
+    # 5,120 153, 196 and 247 against 171, 201 and 282; of 51,200 x 5,120, wider than that, 202, 312 and 384 against 212,
+    # 279 and 396); otherwise, up to 1,536 rows, where its tiles fill their rounds, which its estimate tells: at least 1.1
+    # PFLOP/s (24,576 x 4,096 at 1,024 rows 176 against 184, but at 800 173 against 154; 34,816 x 5,120 at 1,024 322
+    # against 410).  Plain products as long as the library leaves compute units idle (6,144 x 4,096 at 1,024 rows 51
+    # against 53), updates in shares up to 512 rows (4,096 x 4,096 at 512 rows 25 against 31, 4,096 x 12,288 at 357 47
+    # against 52, 2,560 x 9,728 27 against 41).  Small products stay where they are.
+    STAGE_ROWS = (65, 256)              # any of these
+    STAGE_ROWS_SWIGLU = (768, 1536)
+    STAGE_SWIGLU_RATE = 1100            # flops a nanosecond
+    STAGE_ROWS_SHARES = 512
+    STAGE_ROWS_NARROW = 1024            # plain products of at most 32 weight rows a compute unit
     STAGE_MIN_WEIGHT = 1 << 22
 
     def takes_stages(self, x: torch.Tensor, w: Optional[torch.Tensor] = None, swiglu: bool = False) -> bool:
@@ -268,16 +275,21 @@ class Linear:
         in stages."""
         w = self.weight if w is None else w
         rows, (n, k) = x.shape[0], w.shape
-        most = self.STAGE_ROWS[1] if swiglu or n > 32 * compute_units() else self.STAGE_ROWS_NARROW[1]
-        return (self.library and x.dtype == torch.bfloat16 and self.STAGE_ROWS[0] <= rows <= most
-                and n * k >= self.STAGE_MIN_WEIGHT and self.operands_ok(x) and kernels.gemm_stages_takes(rows, n, k, swiglu))
+        if not (self.library and x.dtype == torch.bfloat16 and self.STAGE_ROWS[0] <= rows <= self.STAGE_ROWS_SWIGLU[1]
+                and n * k >= self.STAGE_MIN_WEIGHT and self.operands_ok(x) and kernels.gemm_stages_takes(rows, n, k, swiglu)):
+            return False
+        if rows <= self.STAGE_ROWS[1]:
+            return True
+        if not swiglu:
+            return n <= 32 * compute_units() and rows <= self.STAGE_ROWS_NARROW
+        return ((n <= 192 * compute_units() and rows <= self.STAGE_ROWS_SWIGLU[0])
+                or kernels.gemm_stages_time(rows, n, k) * self.STAGE_SWIGLU_RATE <= 2 * rows * n * k)
 
     def stage_shares_for(self, x: torch.Tensor) -> int:
         """Into how many shares of the inner dimension the product in stages cuts an update that the next norm adds up; 0:
         not this product."""
         rows, n, k = x.shape[0], self.out_features, self.in_features
-        most = self.STAGE_ROWS[1] if k >= self.LIBRARY_SHARES_MIN_K else self.STAGE_ROWS_NARROW[0]
-        if not (self.library and x.dtype == torch.bfloat16 and self.STAGE_ROWS[0] <= rows <= most
+        if not (self.library and x.dtype == torch.bfloat16 and self.STAGE_ROWS[0] <= rows <= self.STAGE_ROWS_SHARES
                 and n * k >= self.STAGE_MIN_WEIGHT and self.operands_ok(x)) or n % 4 or k % 64:
             return 0
         return kernels.gemm_stages_shares(rows, n, k)

@@ -13,7 +13,9 @@ def rnd(*shape, seed):
 
 # every tile the plan knows, with remainders of rows and weight rows, one step of K and many, one row and several panels
 @pytest.mark.parametrize("shape", [(1, 32, 64), (65, 96, 128), (97, 6144, 192), (97, 24576, 64), (128, 4096, 1024),
-                                   (130, 24608, 128), (193, 12288, 64), (256, 4128, 320), (357, 6176, 64), (1030, 2080, 128)])
+                                   (130, 24608, 128), (193, 12288, 64), (256, 4128, 320), (357, 6176, 64), (1030, 2080, 128),
+                                   # tiles of 192 and 256 rows of X: 192 x 192, 192 x 256, 256 x 192, 256 x 256, panels of them
+                                   (357, 24544, 64), (509, 24544, 1024), (357, 24608, 64), (509, 24608, 64), (2100, 8224, 128)])
 def test_product_in_stages_at_the_edges_of_its_tiles(shape):
     from pulse_infer_amd.ops import kernels
 
