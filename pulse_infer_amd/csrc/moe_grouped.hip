@@ -227,7 +227,9 @@ __global__ __launch_bounds__(256) void moe_gate_up_grouped_kernel(const bf16_t* 
                                                                   float limit) {
     const int tile = blockIdx.x;
     if (tile >= *num_tiles) return;
-    const int e = tile_expert[tile], row0 = tile_row0[tile], rows = tile_rows[tile];
+    const int e = tile_expert[tile], row0 = tile_row0[tile] + blockIdx.z * (RB * 16);   // (z: 16 RB rows of a longer tile)
+    const int rows = min(tile_rows[tile] - static_cast<int>(blockIdx.z) * (RB * 16), RB * 16);
+    if (rows <= 0) return;
     const int lane = threadIdx.x % PULSE_WAVE, wave = threadIdx.x / PULSE_WAVE;
     const int r = lane % 16, kg = lane / 16;
     constexpr bool SHARED_K = RB == 2;
@@ -295,7 +297,9 @@ __global__ __launch_bounds__(256) void moe_down_grouped_kernel(const bf16_t* __r
                                                                int hidden, int ff) {
     const int tile = blockIdx.x;
     if (tile >= *num_tiles) return;
-    const int e = tile_expert[tile], row0 = tile_row0[tile], rows = tile_rows[tile];
+    const int e = tile_expert[tile], row0 = tile_row0[tile] + blockIdx.z * (RB * 16);   // (z: 16 RB rows of a longer tile)
+    const int rows = min(tile_rows[tile] - static_cast<int>(blockIdx.z) * (RB * 16), RB * 16);
+    if (rows <= 0) return;
     const int lane = threadIdx.x % PULSE_WAVE, wave = threadIdx.x / PULSE_WAVE;
     const int r = lane % 16, kg = lane / 16;
     constexpr bool SHARED_K = RB == 2;
@@ -354,10 +358,10 @@ __global__ void moe_combine_kernel(const TX* __restrict__ x, const float* __rest
 }
 
 // ------------------------------------------------------------------ many rows an expert
-// Tiles of 32, 64 or 128 gathered rows against WR weight rows (for gate and up: slabs of 16 gate rows and the 16 up rows
+// Tiles of 32, 64, 128 or 192 gathered rows against WR weight rows (for gate and up: slabs of 16 gate rows and the 16 up rows
 // beside them, so that a lane holds both of an inner column), on the loop of tile_loop.h.
 //
-// What bounds it: the matrix cores for tiles of 128 rows, the weights' way from memory for an expert of few rows.  Neighbouring
+// What bounds it: what a compute unit copies into LDS for tiles of 192 rows, the weights' way from memory for an expert of few rows.  Neighbouring
 // workgroups of a die take the tiles of a panel, which share weight rows and gathered rows in that die's L2.
 struct GroupArgs {
     const bf16_t* x;             // gate and up: [tokens, K], row pair / top; down: act [pairs, K], row pair
@@ -376,9 +380,9 @@ struct GroupArgs {
 
 constexpr int GROUP_PANEL = 4;   // tiles of rows a panel of the tile order
 
-template <bool DOWN, int WR, int XR, int WN, int WM, int S, bool NT>
+template <bool DOWN, int WR, int XR, int WN, int WM, int S, int SX, bool NT>
 __global__ __launch_bounds__(WN* WM* PULSE_WAVE) void moe_tile_kernel(GroupArgs a) {
-    using Loop = TileLoop<WR, XR, WN, WM, S, NT>;
+    using Loop = TileLoop<WR, XR, WN, WM, S, NT, SX>;
     constexpr int COLS = DOWN ? WR : WR / 2;       // output columns of a tile
     __shared__ __attribute__((aligned(1024))) char lds[Loop::LDS];
     __shared__ int pair_s[XR];
@@ -456,10 +460,10 @@ __global__ __launch_bounds__(WN* WM* PULSE_WAVE) void moe_tile_kernel(GroupArgs 
                     *reinterpret_cast<tile_bf16x4*>(mine + (lane % 32) * PITCH + (f * 16 + q * 8 + h * 4) * 2) = v;
                 }
             tile_wave_sync();
-            constexpr int PCS = W_COLS / 8, ROWS = PULSE_WAVE / PCS;
+            constexpr int PCS = W_COLS / 8;
 #pragma unroll
-            for (int it = 0; it < 32 / ROWS; ++it) {
-                const int row = it * ROWS + lane / PCS, pc = lane % PCS;
+            for (int it = 0; it < 32 * PCS / PULSE_WAVE; ++it) {
+                const int row = (it * PULSE_WAVE + lane) / PCS, pc = (it * PULSE_WAVE + lane) % PCS;
                 const uint4 v = *reinterpret_cast<const uint4*>(mine + row * PITCH + pc * 16);
                 const int p = pair_s[m_base + row], n = n_wave + pc * 8;
                 if (p >= 0 && n < a.N)
@@ -467,7 +471,7 @@ __global__ __launch_bounds__(WN* WM* PULSE_WAVE) void moe_tile_kernel(GroupArgs 
             }
             tile_wave_sync();
         } else {
-            constexpr int FP = TN < 2 ? TN : 2;        // 32-row pieces of W a pass
+            constexpr int FP = TN % 2 == 0 ? 2 : TN;   // 32-row pieces of W a pass
             constexpr int W_COLS = FP * 32, PITCH = W_COLS * 4 + 16;
             static_assert(32 * PITCH <= WAVE_LDS && TN % FP == 0, "a wavefront's piece of LDS holds 32 rows of a pass");
 #pragma unroll
@@ -484,10 +488,10 @@ __global__ __launch_bounds__(WN* WM* PULSE_WAVE) void moe_tile_kernel(GroupArgs 
                         *reinterpret_cast<float4*>(mine + (lane % 32) * PITCH + (f * 32 + q * 8 + h * 4) * 4) = v;
                     }
                 tile_wave_sync();
-                constexpr int PCS = W_COLS / 4, ROWS = PULSE_WAVE / PCS;
+                constexpr int PCS = W_COLS / 4;
 #pragma unroll
-                for (int it = 0; it < 32 / ROWS; ++it) {
-                    const int row = it * ROWS + lane / PCS, pc = lane % PCS;
+                for (int it = 0; it < 32 * PCS / PULSE_WAVE; ++it) {
+                    const int row = (it * PULSE_WAVE + lane) / PCS, pc = (it * PULSE_WAVE + lane) % PCS;
                     const float4 v = *reinterpret_cast<const float4*>(mine + row * PITCH + pc * 16);
                     const int p = pair_s[m_base + row], n = n_wave + f0 * 32 + pc * 4;
                     if (p >= 0 && n < a.N)
@@ -499,35 +503,35 @@ __global__ __launch_bounds__(WN* WM* PULSE_WAVE) void moe_tile_kernel(GroupArgs 
     }
 }
 
-template <bool DOWN, int WR, int XR, int WN, int WM, int S, bool NT>
+template <bool DOWN, int WR, int XR, int WN, int WM, int S, bool NT, int SX = S>
 void launch_tiles(GroupArgs a, int max_tiles, hipStream_t stream) {
     constexpr int COLS = DOWN ? WR : WR / 2;
     a.tiles_n = (a.N + COLS - 1) / COLS;
     const int64_t grid = (static_cast<int64_t>(max_tiles) * a.tiles_n + 7) / 8 * 8;
-    hipLaunchKernelGGL((moe_tile_kernel<DOWN, WR, XR, WN, WM, S, NT>), dim3(static_cast<unsigned>(grid)), dim3(WN * WM * PULSE_WAVE), 0,
+    hipLaunchKernelGGL((moe_tile_kernel<DOWN, WR, XR, WN, WM, S, SX, NT>), dim3(static_cast<unsigned>(grid)), dim3(WN * WM * PULSE_WAVE), 0,
                        stream, a);
 }
 
-// Which shape a list's tiles take: lists of 32 rows (decoding) and of 64 are bound by the weights' way from memory, lists of
-// 128 by the matrix cores.  `once`: an expert's weights are read for one tile or hardly more, and go past the caches; where
-// two tiles of an expert follow each other they find each other's weights there.  Measured, 16 experts of 1,536 x 4,096, 4
-// chosen a token, gate and up alone / with down in us, at 8, 64, 130, 211, 300, 400, 500, 600, 1,024, 2,048 tokens:
-//   32 rows (weights 128, 3 stages)         79/115  84/125  109/159
-//     once                                  71/103  74/110  116/168
-//     once, weights 64 (2 wavefronts, 4)    68/101  70/110  105/161
-//   64 rows (weights 128, 3 stages)         79/115  85/126   89/131   88/142  108/178  101/168  124/199  148/238  215/335  348/561
-//     once                                  70/103  75/111   77/117   86/139  135/213  124/201  154/241  211/319  257/405  501/755
-//   128 rows (weights 256, 3 stages)                96/138  101/147  102/150  104/154  107/158  151/227  164/236  132/239  259/425
-//     once                                          90/130   94/134   95/139   95/144   97/145  154/220  163/239  143/246  271/432
-//   the kernels above, 32 rows, K shared    78/111 110/167  219/351
-//   the kernels above, 128 rows            150/231 150/231           184/288           370/688 (at 400 tokens)
+// Which shape a list's tiles take.  Lists of up to 128 rows are for experts of one tile mostly: bound by the weights' way from
+// memory, which go past the caches; where two tiles of an expert follow each other (192 rows) they find each other's weights
+// there, and the wider the tile the less a compute unit copies.  Measured, 16 experts of 1,536 x 4,096, 4 chosen a token, gate
+// and up alone / with down in us, at 8, 64, 130, 211, 300, 400, 600, 1,024, 1,300, 2,048, 4,096 tokens:
+//   32 rows (weights 64, 2 wavefronts, 4 stages)   68/101  70/110 105/161
+//     not past the caches (weights 128, 3 stages)  79/115  84/125 109/159
+//   64 rows (weights 128, 3 stages)                70/103  75/111  77/117   86/139  135/213 124/201  211/319
+//     not past the caches                          79/115  85/126   89/131  88/142  108/178 101/168  148/238  215/335
+//   128 rows (weights 256, 3 stages)                       90/130   94/134  95/139   95/144  97/145  163/239  143/246
+//     not past the caches                                  96/138  101/147 102/150  104/154 107/158  164/236  138/241  199/309  276/452  480/786
+//   192 rows (weights 192, down 256; X for down in 2 stages)                                         109/175  156/240  155/241  229/368  450/704
+//   the kernels above, 32 rows, K shared           78/111 110/167  219/351
+//   the kernels above, 128 rows                   150/231 150/231                                   370/688
 template <bool DOWN>
-void launch_tiles_for(const GroupArgs& a, int max_tiles, int rows, bool once, hipStream_t stream) {
+void launch_tiles_for(const GroupArgs& a, int max_tiles, int rows, hipStream_t stream) {
     if (rows <= 32) launch_tiles<DOWN, 64, 32, 2, 1, 4, true>(a, max_tiles, stream);
-    else if (rows <= 64 && once) launch_tiles<DOWN, 128, 64, 4, 1, 3, true>(a, max_tiles, stream);
-    else if (rows <= 64) launch_tiles<DOWN, 128, 64, 4, 1, 3, false>(a, max_tiles, stream);
-    else if (once) launch_tiles<DOWN, 256, 128, 2, 2, 3, true>(a, max_tiles, stream);
-    else launch_tiles<DOWN, 256, 128, 2, 2, 3, false>(a, max_tiles, stream);
+    else if (rows <= 64) launch_tiles<DOWN, 128, 64, 4, 1, 3, true>(a, max_tiles, stream);
+    else if (rows <= 128) launch_tiles<DOWN, 256, 128, 2, 2, 3, true>(a, max_tiles, stream);
+    else if constexpr (DOWN) launch_tiles<DOWN, 256, 192, 2, 2, 3, false, 2>(a, max_tiles, stream);
+    else launch_tiles<DOWN, 192, 192, 2, 2, 3, false>(a, max_tiles, stream);
 }
 
 }  // namespace
@@ -551,25 +555,25 @@ static bool aligned16(const void* p) { return reinterpret_cast<uintptr_t>(p) % 1
 
 extern "C" int pulse_moe_gate_up_grouped(const void* x, const void* wg, const void* wu, const int* order,
                                          const int* tile_expert, const int* tile_row0, const int* tile_rows,
-                                         const int* num_tiles, int max_tiles, int tile_rows_max, int once, void* act, int hidden,
+                                         const int* num_tiles, int max_tiles, int tile_rows_max, void* act, int hidden,
                                          int ff, int top, const float* in_weight, int act_kind, float limit,
                                          hipStream_t stream) {
     PULSE_REQUIRE(act_kind == 0 || act_kind == 1, "moe_gate_up_grouped: unknown activation %d", act_kind);
     PULSE_REQUIRE(hidden > 0 && ff > 0 && top > 0 && max_tiles > 0, "moe_gate_up_grouped: bad sizes");
     PULSE_REQUIRE(hidden % 8 == 0 && aligned16(x) && aligned16(wg) && aligned16(wu),
                   "moe_gate_up_grouped: rows must be multiples of 8 values and 16-byte aligned");
-    PULSE_REQUIRE(tile_rows_max == 32 || tile_rows_max == 64 || tile_rows_max == 128, "moe_gate_up_grouped: tiles of 32, 64 or 128 rows");
+    PULSE_REQUIRE(tile_rows_max == 32 || tile_rows_max == 64 || tile_rows_max == 128 || tile_rows_max == 192, "moe_gate_up_grouped: tiles of 32, 64, 128 or 192 rows");
     PULSE_REQUIRE(x && wg && wu && order && tile_expert && tile_row0 && tile_rows && num_tiles && act,
                   "moe_gate_up_grouped: null pointer");
     PULSE_REQUIRE((ff + 15) / 16 < 65536, "moe_gate_up_grouped: an inner width of %d is too large", ff);
     if (hidden % 64 == 0 && ff % 8 == 0 && aligned16(act)) {   // (the loop walks K in whole steps of 64; rows leave in 16-byte pieces)
         launch_tiles_for<false>({static_cast<const bf16_t*>(x), {static_cast<const bf16_t*>(wg), static_cast<const bf16_t*>(wu)},
                                  act, order, tile_expert, tile_row0, tile_rows, num_tiles, in_weight, hidden, ff, top, 0,
-                                 act_kind, limit}, max_tiles, tile_rows_max, once != 0, stream);
+                                 act_kind, limit}, max_tiles, tile_rows_max, stream);
         PULSE_LAUNCH_CHECK("moe_gate_up_grouped");
         return 0;
     }
-    const dim3 grid(max_tiles, (ff + 63) / 64);
+    const dim3 grid(max_tiles, (ff + 63) / 64, (tile_rows_max + 127) / 128);
     if (tile_rows_max == 32)
         hipLaunchKernelGGL(moe_gate_up_grouped_kernel<2>, dim3(max_tiles, (ff + 15) / 16), dim3(256), 0, stream, static_cast<const bf16_t*>(x),
                            static_cast<const bf16_t*>(wg), static_cast<const bf16_t*>(wu), order, tile_expert, tile_row0,
@@ -584,22 +588,21 @@ extern "C" int pulse_moe_gate_up_grouped(const void* x, const void* wg, const vo
 
 extern "C" int pulse_moe_down_grouped(const void* act, const void* wd, const int* order, const int* tile_expert,
                                       const int* tile_row0, const int* tile_rows, const int* num_tiles, int max_tiles,
-                                      int tile_rows_max, int once, float* y, int hidden, int ff, hipStream_t stream) {
+                                      int tile_rows_max, float* y, int hidden, int ff, hipStream_t stream) {
     PULSE_REQUIRE(hidden > 0 && ff > 0 && max_tiles > 0, "moe_down_grouped: bad sizes");
     PULSE_REQUIRE(ff % 8 == 0 && aligned16(act) && aligned16(wd),
                   "moe_down_grouped: rows must be multiples of 8 values and 16-byte aligned");
-    PULSE_REQUIRE(tile_rows_max == 32 || tile_rows_max == 64 || tile_rows_max == 128, "moe_down_grouped: tiles of 32, 64 or 128 rows");
+    PULSE_REQUIRE(tile_rows_max == 32 || tile_rows_max == 64 || tile_rows_max == 128 || tile_rows_max == 192, "moe_down_grouped: tiles of 32, 64, 128 or 192 rows");
     PULSE_REQUIRE(act && wd && order && tile_expert && tile_row0 && tile_rows && num_tiles && y,
                   "moe_down_grouped: null pointer");
     PULSE_REQUIRE((hidden + 15) / 16 < 65536, "moe_down_grouped: a width of %d is too large", hidden);
     if (ff % 64 == 0 && hidden % 4 == 0 && aligned16(y)) {
         launch_tiles_for<true>({static_cast<const bf16_t*>(act), {static_cast<const bf16_t*>(wd), nullptr}, y, order, tile_expert,
-                                tile_row0, tile_rows, num_tiles, nullptr, ff, hidden, 1, 0, 0, 0.f}, max_tiles, tile_rows_max,
-                               once != 0, stream);
+                                tile_row0, tile_rows, num_tiles, nullptr, ff, hidden, 1, 0, 0, 0.f}, max_tiles, tile_rows_max, stream);
         PULSE_LAUNCH_CHECK("moe_down_grouped");
         return 0;
     }
-    const dim3 grid(max_tiles, (hidden + 63) / 64);
+    const dim3 grid(max_tiles, (hidden + 63) / 64, (tile_rows_max + 127) / 128);
     if (tile_rows_max == 32)
         hipLaunchKernelGGL(moe_down_grouped_kernel<2>, dim3(max_tiles, (hidden + 15) / 16), dim3(256), 0, stream, static_cast<const bf16_t*>(act),
                            static_cast<const bf16_t*>(wd), order, tile_expert, tile_row0, tile_rows, num_tiles, y, hidden, ff);

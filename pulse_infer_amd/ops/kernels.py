@@ -1681,25 +1681,17 @@ def moe_down(x: torch.Tensor, act: torch.Tensor, w_down: torch.Tensor, idx: torc
          _ptr(idx), _ptr(weight), _ptr(out), _i32(tokens), _i32(hidden), _i32(ff), _i32(experts), _i32(top), _stream())
 
 
-MOE_TILE_ROWS = (32, 64, 128)   # rows of an expert's tile in the grouped products
+MOE_TILE_ROWS = (32, 64, 128, 192)   # rows of an expert's tile in the grouped products
 
 
 def moe_tile_rows(pairs: int, experts: int) -> int:
-    """Rows of the tiles for a step of ``pairs`` (token, choice) pairs, by how many an expert gets on average: up to some
-    fifty, the weights' way from memory is the time, and one tile should hold them all; 128 rows read the weights once up to
-    about 112; from there to about 160 an expert has two tiles of 128 mostly empty, or three of 64 (16 experts of 1,536 x
-    4,096, 4 chosen a token, gate, up and down in tiles of 64 / 128 rows: at 300 tokens 178 / 144 us, at 400 168 / 145,
-    at 500 199 / 220, at 600 238 / 236, at 700 258 / 215)."""
-    if pairs <= 16 * experts:
-        return MOE_TILE_ROWS[0]
-    return MOE_TILE_ROWS[1] if pairs <= 56 * experts or 112 * experts < pairs < 160 * experts else MOE_TILE_ROWS[2]
-
-
-def moe_weights_once(pairs: int, experts: int, tile_rows: int) -> bool:
-    """Whether an expert of such a step has one tile mostly: its weights then need not stay in the caches (16 experts of
-    1,536 x 4,096: tiles of 64 rows for 53 pairs an expert 142 us and 139 past the caches, for 75 178 and 213; tiles of 128
-    for 100 158 and 145, for 150 236 and 239, for 256 239 and 246)."""
-    return pairs <= tile_rows * 7 // 8 * experts
+    """Rows of the tiles for a step of ``pairs`` (token, choice) pairs, by how many an expert gets on average: while the
+    weights' way from memory is the time, one tile should hold them all, up to about 112 rows in one of 128; beyond, tiles of
+    192 rows (16 experts of 1,536 x 4,096, 4 chosen a token, gate, up and down in tiles of 64 / 128 / 192 rows: at 211 tokens
+    139 / 139 us, at 300 213 / 144, at 400 201 / 145 / 147, at 600 238 / 228 / 175, at 850 316 / 221 / 239, at 1,300
+    309 / 241 with 128 and 192, at 2,048 452 / 368)."""
+    per = pairs / experts
+    return MOE_TILE_ROWS[0 if per <= 16 else 1 if per <= 56 else 2 if per <= 112 else 3]
 
 
 def moe_grouped_takes(x: torch.Tensor, w_gate: torch.Tensor, w_down: torch.Tensor) -> bool:
@@ -1746,15 +1738,14 @@ def moe_grouped(x: torch.Tensor, w_gate: torch.Tensor, w_up: torch.Tensor, w_dow
     base = scratch.data_ptr()
     at = lambda n: ctypes.c_void_p(base + 4 * n)
     rank, order = at(0), at(pairs)
-    once = _i32(1 if moe_weights_once(pairs, experts, tile_rows) else 0)
     t_expert, t_row0, t_rows, count = at(2 * pairs), at(2 * pairs + tiles), at(2 * pairs + 2 * tiles), at(2 * pairs + 3 * tiles)
     call("pulse_moe_group", _ptr(idx), _i32(pairs), _i32(experts), _i32(tile_rows), _i32(tiles), rank, order, t_expert,
          t_row0, t_rows, count, _stream())
     call("pulse_moe_gate_up_grouped", _ptr(x), _ptr(w_gate), _ptr(w_up), order, t_expert, t_row0, t_rows, count, _i32(tiles),
-         _i32(tile_rows), once, _ptr(act), _i32(hidden), _i32(ff), _i32(top), _ptr(weight if weight_on_input else None),
+         _i32(tile_rows), _ptr(act), _i32(hidden), _i32(ff), _i32(top), _ptr(weight if weight_on_input else None),
          _i32(EXPERT_ACTIVATIONS[activation]), _f32(limit), _stream())
     call("pulse_moe_down_grouped", _ptr(act), _ptr(w_down), order, t_expert, t_row0, t_rows, count, _i32(tiles),
-         _i32(tile_rows), once, _ptr(y), _i32(hidden), _i32(ff), _stream())
+         _i32(tile_rows), _ptr(y), _i32(hidden), _i32(ff), _stream())
     if out is None:
         return
     call("pulse_moe_combine", _ptr(x), _i32(_tag(x, "moe_grouped")), _ptr(y), _ptr(idx),
