@@ -72,12 +72,13 @@ __device__ __forceinline__ void by_mask(const RowView& row, F f) {
 
 // f(i, value) for i = first, first + step, .. below end, in that order; the values of AHEAD entries are asked for
 // before the first is used (a workgroup alone on its row otherwise waits out a trip to memory for every entry).  32 rows of
-// 151,936 with all options among them: 565 us with the masks' branches beside every load, 503 without.
-template <typename F>
+// 151,936 with all options among them: 565 us with the masks' branches beside every load, 503 without.  MOST: entries ahead
+// in a row without masks, no more than a thread has.
+template <int MOST = 16, typename F>
 __device__ __forceinline__ void sweep(const RowView& row, int first, int end, int step, F f) {
     by_mask(row, [&](auto masked) __attribute__((always_inline)) {
         constexpr bool MASKED = decltype(masked)::value;
-        constexpr int AHEAD = MASKED ? 8 : 16;
+        constexpr int AHEAD = MASKED ? 8 : MOST;
         int i = first;
         for (; i + (AHEAD - 1) * step < end; i += AHEAD * step) {
             float x[AHEAD];
@@ -590,7 +591,7 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
             // Top-p alone: the histogram's masses say near which token the sum reaches `want`; the tokens of that bin and
             // its neighbours are ranked, and M is summed, in its own order, for the five (or fifteen) round that place side by side.
             // (A search for the threshold's bits, four a pass, takes eight such passes.  32 rows of 151,936, this kernel:
-            // 661 us with the search, 377 with this, 158 with the mass and the histogram made by the kernels in front.)
+            // 661 us with the search, 377 with this, 141 with the mass and the histogram made by the kernels in front.)
             want = p * whole;
             found = nucleus_edge(row, want, best, inv_t, bin_scale, hist, hist_w, sf, si, list_i, list_x, cand, &nearest, thr);
         } else {
@@ -747,16 +748,18 @@ __device__ __forceinline__ RowView simple_row(const float* logits, int r, int64_
 __global__ __launch_bounds__(SIMPLE_THREADS) void simple_max_kernel(
     const float* __restrict__ logits, int vocab, int64_t row_stride, const float* __restrict__ penalty,
     const int* __restrict__ seen_row, const uint32_t* __restrict__ seen_masks, const uint32_t* __restrict__ banned,
-    int mask_words, float* __restrict__ part_max, int* __restrict__ part_idx) {
+    int mask_words, float* __restrict__ part_max, int* __restrict__ part_idx, float* __restrict__ part_min) {
     __shared__ float sv[SIMPLE_THREADS / PULSE_WAVE];
     __shared__ int si[SIMPLE_THREADS / PULSE_WAVE];
+    __shared__ float sl[SIMPLE_THREADS / PULSE_WAVE];
     const int r = blockIdx.y, chunk = blockIdx.x, chunks = gridDim.x;
     const RowView row = simple_row(logits, r, row_stride, vocab, penalty, seen_row, seen_masks, banned, mask_words);
     const int begin = chunk * SIMPLE_CHUNK, end = min(vocab, begin + SIMPLE_CHUNK);
-    float best = -INFINITY;
+    float best = -INFINITY, lowest = INFINITY;
     int best_i = 0x7fffffff;
-    sweep(row, begin + static_cast<int>(threadIdx.x), end, SIMPLE_THREADS, [&](int i, float x) {
+    sweep<SIMPLE_CHUNK / SIMPLE_THREADS>(row, begin + static_cast<int>(threadIdx.x), end, SIMPLE_THREADS, [&](int i, float x) {
         if (x > best) { best = x; best_i = i; }   // a thread's indices rise: the first of equals stays
+        if (x != -INFINITY) lowest = fminf(lowest, x);
     });
     const int lane = threadIdx.x % PULSE_WAVE, wave = threadIdx.x / PULSE_WAVE;
 #pragma unroll
@@ -765,11 +768,16 @@ __global__ __launch_bounds__(SIMPLE_THREADS) void simple_max_kernel(
         const int oi = __shfl_xor(best_i, off, PULSE_WAVE);
         if (ov > best || (ov == best && oi < best_i)) { best = ov; best_i = oi; }
     }
-    if (lane == 0) { sv[wave] = best; si[wave] = best_i; }
+    if (part_min) lowest = -wave_max(-lowest);
+    if (lane == 0) { sv[wave] = best; si[wave] = best_i; sl[wave] = lowest; }
     __syncthreads();
     if (threadIdx.x == 0) {
         for (int w = 1; w < SIMPLE_THREADS / PULSE_WAVE; ++w)
             if (sv[w] > best || (sv[w] == best && si[w] < best_i)) { best = sv[w]; best_i = si[w]; }
+        if (part_min) {
+            for (int w = 1; w < SIMPLE_THREADS / PULSE_WAVE; ++w) lowest = fminf(lowest, sl[w]);
+            part_min[r * chunks + chunk] = lowest;
+        }
         part_max[r * chunks + chunk] = best;
         part_idx[r * chunks + chunk] = best_i;
     }
@@ -801,7 +809,7 @@ __global__ __launch_bounds__(SIMPLE_THREADS) void simple_mass_kernel(
     const RowView row = simple_row(logits, r, row_stride, vocab, penalty, seen_row, seen_masks, banned, mask_words);
     const int begin = chunk * SIMPLE_CHUNK, end = min(vocab, begin + SIMPLE_CHUNK);
     float mass = 0.f;
-    sweep(row, begin + static_cast<int>(threadIdx.x), end, SIMPLE_THREADS, [&](int, float x) {
+    sweep<SIMPLE_CHUNK / SIMPLE_THREADS>(row, begin + static_cast<int>(threadIdx.x), end, SIMPLE_THREADS, [&](int, float x) {
         if (x != -INFINITY) mass += expf((x - best) * inv_t);
     });
     const int lane = threadIdx.x % PULSE_WAVE, wave = threadIdx.x / PULSE_WAVE;
@@ -923,6 +931,11 @@ __global__ __launch_bounds__(SIMPLE_THREADS) void topk_collect_kernel(
     if (threadIdx.x == 0) *my_n = total;   // more than TOPK_SEGMENT: the row does not fit
 }
 
+// What rest_kernel adds a row's histogram to.
+__device__ __forceinline__ void clear_histogram(int* rest, int lane) {
+    for (int b = lane; b < 2 * HIST_BINS; b += PULSE_WAVE) rest[b] = 0;
+}
+
 // The choice of every row from what the kernels before left, a wavefront a row: the largest logit for greedy rows;
 // for rows with top-k the candidates' segments strung together in LDS and finished there; for rows that draw from the
 // whole vocabulary the chunk in which u * mass falls (chunk masses in chunk order), walked alone.  done[r] says
@@ -934,7 +947,7 @@ __global__ __launch_bounds__(PULSE_WAVE) void chunked_choose_kernel(
     const uint32_t* __restrict__ banned, int mask_words, const float* __restrict__ part_max,
     const int* __restrict__ part_idx, const float* __restrict__ part_mass, const int* __restrict__ seg_i,
     const float* __restrict__ seg_x, const int* __restrict__ seg_n, int chunks, int* __restrict__ out,
-    int* __restrict__ done) {
+    int* __restrict__ done, int* __restrict__ left) {
     __shared__ int list_i[LIST_CAP];
     __shared__ float list_x[LIST_CAP];
     const int r = blockIdx.x, lane = threadIdx.x;
@@ -980,6 +993,7 @@ __global__ __launch_bounds__(PULSE_WAVE) void chunked_choose_kernel(
         const int n = first + __shfl(pre1, PULSE_WAVE - 1, PULSE_WAVE);
         if (k > chunks || chunks > 2 * PULSE_WAVE || __ballot(over) != 0ull || n > LIST_CAP || n < k || n == 0) {
             if (lane == 0) done[r] = 0;   // not a row for these kernels: sample_kernel takes it
+            clear_histogram(left + static_cast<int64_t>(r) * REST_WORDS, lane);
             return;
         }
         float whole = 0.f;   // without top-k: the mass of the whole row, chunk masses in chunk order
@@ -1002,6 +1016,7 @@ __global__ __launch_bounds__(PULSE_WAVE) void chunked_choose_kernel(
             if (enough) out[r] = token;
             done[r] = enough ? 1 : 0;
         }
+        if (!__shfl(enough ? 1 : 0, 0, PULSE_WAVE)) clear_histogram(left + static_cast<int64_t>(r) * REST_WORDS, lane);
         return;
     }
     // a draw from the whole vocabulary: the chunk in which it falls, chunk masses in chunk order
@@ -1044,66 +1059,54 @@ __global__ __launch_bounds__(PULSE_WAVE) void chunked_choose_kernel(
 }
 
 // ---- the rows that are left, before sample_kernel ---------------------------------------------------------------
-// A workgroup a row goes over its row at the rate of one compute unit; of what sample_kernel needs to know of the whole row,
-// the mass (a wavefront of it summed by a wavefront here, entries and order as there), the smallest number and the
-// histogram are made by as many workgroups as there are wavefronts in it: 17 and 30 us for 13 rows of 151,936,
-// where the passes inside sample_kernel took 220.
-__global__ __launch_bounds__(PULSE_WAVE) void rest_mass_kernel(
+// A workgroup a row goes over its row at the rate of one compute unit; what sample_kernel needs to know of the whole row, its
+// mass (a wavefront of it summed by a wavefront here, entries and order as there) and the histogram over [lowest, best], is
+// made by many workgroups, in one launch: 18 us for 6 rows of 151,936 and 32 for 26, where the passes inside sample_kernel
+// took 220 and two launches, the histogram behind the mass and the lowest value, 34 for 13.  (The lowest value comes with the maxima, and the
+// histogram is cleared by the kernel that leaves the row.)
+constexpr int REST_GROUPS = 16;                                             // workgroups for a row's histogram
+constexpr int MASS_GROUPS = SAMPLE_WAVES * PULSE_WAVE / SIMPLE_THREADS;     // and for its mass
+
+__global__ __launch_bounds__(SIMPLE_THREADS) void rest_kernel(
     const float* __restrict__ logits, int vocab, int64_t row_stride, const float* __restrict__ temperature,
     const int* __restrict__ top_k, const float* __restrict__ penalty, const int* __restrict__ seen_row,
     const uint32_t* __restrict__ seen_masks, const uint32_t* __restrict__ banned, int mask_words,
-    const float* __restrict__ part_max, int chunks, const int* __restrict__ done, int* __restrict__ rest) {
-    const int r = blockIdx.y, wave = blockIdx.x, lane = threadIdx.x;
-    if (done[r]) return;
-    rest += static_cast<int64_t>(r) * REST_WORDS;
-    constexpr int SLICE = 2 * HIST_BINS / SAMPLE_WAVES;
-    for (int b = lane; b < SLICE; b += PULSE_WAVE) rest[wave * SLICE + b] = 0;
-    const float best = simple_row_max(part_max + static_cast<int64_t>(r) * chunks, chunks);
-    const float inv_t = 1.0f / temperature[r];
-    const int k = top_k ? top_k[r] : 0;
-    const RowView row = simple_row(logits, r, row_stride, vocab, penalty, seen_row, seen_masks, banned, mask_words);
-    float mass = 0.f, lowest = INFINITY;
-    if (k > 0 && k < vocab) {
-        sweep(row, wave * PULSE_WAVE + lane, vocab, SAMPLE_THREADS, [&](int, float x) {
-            if (x != -INFINITY) lowest = fminf(lowest, x);
-        });
-    } else {
-        sweep(row, wave * PULSE_WAVE + lane, vocab, SAMPLE_THREADS, [&](int, float x) {
-            if (x != -INFINITY) { mass += expf((x - best) * inv_t); lowest = fminf(lowest, x); }
-        });
-    }
-    mass = wave_sum(mass);
-    lowest = -wave_max(-lowest);
-    if (lane == 0) {
-        rest[REST_MASS + wave] = __float_as_int(mass);
-        rest[REST_LOWEST + wave] = __float_as_int(lowest);
-    }
-}
-
-constexpr int REST_GROUPS = 16;
-
-__global__ __launch_bounds__(SIMPLE_THREADS) void rest_histogram_kernel(
-    const float* __restrict__ logits, int vocab, int64_t row_stride, const float* __restrict__ temperature,
-    const int* __restrict__ top_k, const float* __restrict__ penalty, const int* __restrict__ seen_row,
-    const uint32_t* __restrict__ seen_masks, const uint32_t* __restrict__ banned, int mask_words,
-    const float* __restrict__ part_max, int chunks, const int* __restrict__ done, int* __restrict__ rest) {
+    const float* __restrict__ part_max, const float* __restrict__ part_min, int chunks, const int* __restrict__ done,
+    int* __restrict__ rest) {
     __shared__ int hist[HIST_BINS];
     __shared__ float hist_w[HIST_BINS];
-    const int r = blockIdx.y;
+    const int r = blockIdx.y, lane = threadIdx.x % PULSE_WAVE;
     if (done[r]) return;
     rest += static_cast<int64_t>(r) * REST_WORDS;
-    for (int b = threadIdx.x; b < HIST_BINS; b += SIMPLE_THREADS) { hist[b] = 0; hist_w[b] = 0.f; }
     const float best = simple_row_max(part_max + static_cast<int64_t>(r) * chunks, chunks);
-    float lowest = INFINITY;
-    for (int w = 0; w < SAMPLE_WAVES; ++w) lowest = fminf(lowest, __int_as_float(rest[REST_LOWEST + w]));
     const float inv_t = 1.0f / temperature[r];
     const int k = top_k ? top_k[r] : 0;
     const bool by_k = k > 0 && k < vocab;
+    const RowView row = simple_row(logits, r, row_stride, vocab, penalty, seen_row, seen_masks, banned, mask_words);
+    if (blockIdx.x < MASS_GROUPS) {
+        const int wave = blockIdx.x * (SIMPLE_THREADS / PULSE_WAVE) + threadIdx.x / PULSE_WAVE;
+        float mass = 0.f, lowest = INFINITY;
+        if (!by_k)
+            sweep(row, wave * PULSE_WAVE + lane, vocab, SAMPLE_THREADS, [&](int, float x) {
+                if (x != -INFINITY) mass += expf((x - best) * inv_t);
+            });
+        for (int c = lane; c < chunks; c += PULSE_WAVE) lowest = fminf(lowest, part_min[static_cast<int64_t>(r) * chunks + c]);
+        mass = wave_sum(mass);
+        lowest = -wave_max(-lowest);
+        if (lane == 0) {
+            rest[REST_MASS + wave] = __float_as_int(mass);
+            rest[REST_LOWEST + wave] = __float_as_int(lowest);
+        }
+        return;
+    }
+    for (int b = threadIdx.x; b < HIST_BINS; b += SIMPLE_THREADS) { hist[b] = 0; hist_w[b] = 0.f; }
+    float lowest = INFINITY;
+    for (int c = lane; c < chunks; c += PULSE_WAVE) lowest = fminf(lowest, part_min[static_cast<int64_t>(r) * chunks + c]);
+    lowest = -wave_max(-lowest);
     const float scale = static_cast<float>(HIST_BINS) / (best - lowest);
     __syncthreads();
     if (!(best > lowest && scale < INFINITY)) return;    // (as sample_kernel: no histogram)
-    const RowView row = simple_row(logits, r, row_stride, vocab, penalty, seen_row, seen_masks, banned, mask_words);
-    sweep(row, blockIdx.x * SIMPLE_THREADS + threadIdx.x, vocab, REST_GROUPS * SIMPLE_THREADS, [&](int, float x) {
+    sweep(row, (blockIdx.x - MASS_GROUPS) * SIMPLE_THREADS + threadIdx.x, vocab, REST_GROUPS * SIMPLE_THREADS, [&](int, float x) {
         if (x != -INFINITY) {
             const int b = min(HIST_BINS - 1, static_cast<int>((best - x) * scale));
             atomicAdd(&hist[b], 1);
@@ -1217,8 +1220,8 @@ extern "C" int pulse_sample(const float* logits, int rows, int vocab, int64_t ro
 // equal values around the k-th largest, a distribution too flat for top-p alone) by the kernel of pulse_sample behind
 // them, which skips the rows that are done.  What a row's choice is does not depend on the
 // other rows.  Scratch, with chunks = pulse_sample_chunks(vocab): part_max, part_mass (float32), part_idx, seg_n
-// (int32) of rows * chunks entries; seg_i (int32), seg_x (float32) of rows * chunks * pulse_sample_segment()
-// entries; done (int32) of rows entries; rest (int32) of rows * pulse_sample_rest() entries.
+// (int32) of rows * chunks entries; seg_x (float32) of rows * chunks * pulse_sample_segment() entries, seg_i (int32) of
+// rows * (pulse_sample_rest() + chunks) more; done (int32) of rows entries.
 extern "C" int pulse_sample_rest() { return REST_WORDS; }
 extern "C" int pulse_sample_chunks(int vocab) { return (vocab + SIMPLE_CHUNK - 1) / SIMPLE_CHUNK; }
 extern "C" int pulse_sample_segment() { return TOPK_SEGMENT; }
@@ -1227,18 +1230,22 @@ extern "C" int pulse_sample_chunked(const float* logits, int rows, int vocab, in
                                     const int* top_k, const float* top_p, const float* uniform, const float* penalty,
                                     const int* seen_row, const uint32_t* seen_masks, const uint32_t* banned,
                                     int mask_words, float* part_max, int* part_idx, float* part_mass, int* seg_i,
-                                    float* seg_x, int* seg_n, int* done, int* rest, int* out, hipStream_t stream) {
+                                    float* seg_x, int* seg_n, int* done, int* out, hipStream_t stream) {
     PULSE_REQUIRE(rows >= 0 && vocab > 0 && row_stride >= vocab, "sample_chunked: bad sizes rows=%d V=%d", rows, vocab);
     PULSE_REQUIRE(rows < 65536, "sample_chunked: at most 65535 rows");
-    PULSE_REQUIRE(logits && out && part_max && part_idx && part_mass && seg_i && seg_x && seg_n && done && rest,
+    PULSE_REQUIRE(logits && out && part_max && part_idx && part_mass && seg_i && seg_x && seg_n && done,
                   "sample_chunked: null pointer");
     PULSE_REQUIRE(!temperature || uniform, "sample_chunked: temperature sampling needs uniform numbers");
     PULSE_REQUIRE((!seen_masks && !banned) || mask_words * 32 >= vocab, "sample_chunked: masks cover %d tokens, "
                   "vocabulary has %d", mask_words * 32, vocab);
     if (rows == 0) return 0;
     const int chunks = pulse_sample_chunks(vocab);
+    // behind the segments: what is made of the rows that are left, and the chunks' smallest numbers
+    const bool leaves = temperature && (top_k || top_p);    // (without them every row is done)
+    int* rest = leaves ? seg_i + static_cast<int64_t>(rows) * chunks * TOPK_SEGMENT : nullptr;
+    float* part_min = leaves ? reinterpret_cast<float*>(rest + static_cast<int64_t>(rows) * REST_WORDS) : nullptr;
     hipLaunchKernelGGL(simple_max_kernel, dim3(chunks, rows), dim3(SIMPLE_THREADS), 0, stream, logits, vocab, row_stride,
-                       penalty, seen_row, seen_masks, banned, mask_words, part_max, part_idx);
+                       penalty, seen_row, seen_masks, banned, mask_words, part_max, part_idx, part_min);
     PULSE_LAUNCH_CHECK("sample_chunked (maxima)");
     if (temperature) {
         hipLaunchKernelGGL(simple_mass_kernel, dim3(chunks, rows), dim3(SIMPLE_THREADS), 0, stream, logits, vocab,
@@ -1254,17 +1261,13 @@ extern "C" int pulse_sample_chunked(const float* logits, int rows, int vocab, in
     }
     hipLaunchKernelGGL(chunked_choose_kernel, dim3(rows), dim3(PULSE_WAVE), 0, stream, logits, vocab, row_stride,
                        temperature, top_k, top_p, uniform, penalty, seen_row, seen_masks, banned, mask_words, part_max,
-                       part_idx, part_mass, seg_i, seg_x, seg_n, chunks, out, done);
+                       part_idx, part_mass, seg_i, seg_x, seg_n, chunks, out, done, rest);
     PULSE_LAUNCH_CHECK("sample_chunked (choice)");
-    if (temperature && (top_k || top_p)) {   // (without them every row is done)
-        hipLaunchKernelGGL(rest_mass_kernel, dim3(SAMPLE_WAVES, rows), dim3(PULSE_WAVE), 0, stream, logits, vocab, row_stride,
-                           temperature, top_k, penalty, seen_row, seen_masks, banned, mask_words, part_max, chunks,
-                           static_cast<const int*>(done), rest);
-        PULSE_LAUNCH_CHECK("sample_chunked (masses of the rest)");
-        hipLaunchKernelGGL(rest_histogram_kernel, dim3(REST_GROUPS, rows), dim3(SIMPLE_THREADS), 0, stream, logits, vocab,
+    if (leaves) {
+        hipLaunchKernelGGL(rest_kernel, dim3(MASS_GROUPS + REST_GROUPS, rows), dim3(SIMPLE_THREADS), 0, stream, logits, vocab,
                            row_stride, temperature, top_k, penalty, seen_row, seen_masks, banned, mask_words, part_max,
-                           chunks, static_cast<const int*>(done), rest);
-        PULSE_LAUNCH_CHECK("sample_chunked (histograms of the rest)");
+                           part_min, chunks, static_cast<const int*>(done), rest);
+        PULSE_LAUNCH_CHECK("sample_chunked (what is left)");
         hipLaunchKernelGGL(sample_kernel, dim3(rows), dim3(SAMPLE_THREADS), 0, stream, logits, vocab, row_stride,
                            temperature, top_k, top_p, uniform, penalty, seen_row, seen_masks, banned, mask_words, out,
                            static_cast<const int*>(done), part_max, part_idx, chunks, static_cast<const int*>(rest));

@@ -480,16 +480,16 @@ def gemm_stages(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, swiglu: boo
         splits = out.shape[0]
         _need(not swiglu and out.dim() == 3 and tuple(out.shape[1:]) == (m, n) and out.is_contiguous() and n % 4 == 0
               and k % (64 * splits) == 0, f"gemm_stages: float32 results go to contiguous [shares, {m}, {n}]")
-        mode, ldc, part_stride = 2, n, m * n if splits > 1 else 0
+        mode, ldc = 1, n
     else:
         cols = n // 2 if swiglu else n
         _need(gemm_stages_takes(m, n, k, swiglu) and out.dtype == torch.bfloat16 and out.dim() == 2
               and tuple(out.shape) == (m, cols) and out.stride(1) == 1,
               f"gemm_stages: M={m} N={n} K={k} is not a shape it takes, or out is not bfloat16 [{m}, {cols}]")
-        mode, ldc, part_stride, splits = (1 if swiglu else 0), (out.stride(0) if m > 1 else cols), 0, 1
-    call("pulse_gemm_stages", _ptr(a), _i64(a.stride(0) if m > 1 else k), _ptr(w), _i64(w.stride(0) if n > 1 else k),
-         _ptr(out), _i64(ldc), _i32(m), _i32(n), _i32(k), _i32(mode), _i32(splits), _i64(part_stride), _stream(),
-         label=f"N={n} K={k}")
+        mode, ldc, splits = 0, (out.stride(0) if m > 1 else cols), 1
+    call("pulse_gemm_mid", _ptr(a), _i64(a.stride(0) if m > 1 else k), _ptr(w), _i64(w.stride(0) if n > 1 else k),
+         _ptr(out), _i64(ldc), _i32(m), _i32(n), _i32(k), _i32(mode), _i32(1 if swiglu else 0), _i32(splits),
+         _i32(-1), _stream(), label=f"N={n} K={k}")
 
 
 MID_MAX_ROWS = 192
@@ -1047,8 +1047,8 @@ def sample_chunked_scratch(rows: int, vocab: int, device) -> dict:
     f32 = lambda n: torch.empty(n, dtype=torch.float32, device=device)
     i32 = lambda n: torch.empty(n, dtype=torch.int32, device=device)
     return {"part_max": f32(rows * per_row), "part_idx": i32(rows * per_row), "part_mass": f32(rows * per_row),
-            "seg_n": i32(rows * per_row), "done": i32(rows), "seg_i": i32(rows * per_row * SAMPLE_SEGMENT),
-            "seg_x": f32(rows * per_row * SAMPLE_SEGMENT), "rest": i32(rows * SAMPLE_REST)}
+            "seg_n": i32(rows * per_row), "done": i32(rows), "seg_i": i32(rows * (per_row * (SAMPLE_SEGMENT + 1) + SAMPLE_REST)),
+            "seg_x": f32(rows * per_row * SAMPLE_SEGMENT)}
 
 
 def sample_chunked(logits: torch.Tensor, out: torch.Tensor, scratch: dict, temperature: Optional[torch.Tensor] = None,
@@ -1059,9 +1059,9 @@ def sample_chunked(logits: torch.Tensor, out: torch.Tensor, scratch: dict, tempe
     """``sample`` in chunks of the vocabulary with a workgroup each instead of a workgroup a row: greedy rows, rows
     that draw from the whole vocabulary and rows with top-k (k at most the number of chunks) are chosen from what the
     chunks leave; rows with top-p alone, and what does not fit, go through the kernel of ``sample`` behind them,
-    which two more have prepared.
+    which one more has prepared.
     Which way a row goes depends on the row alone.  ``scratch`` as ``sample_chunked_scratch`` makes it."""
-    names = ("part_max", "part_idx", "part_mass", "seg_i", "seg_x", "seg_n", "done", "rest")
+    names = ("part_max", "part_idx", "part_mass", "seg_i", "seg_x", "seg_n", "done")
     _gpu("sample_chunked", logits, out, temperature, top_k, top_p, uniform, penalty, seen_row, seen_masks, banned,
          *(scratch[n] for n in names))
     _need(logits.dim() == 2 and logits.dtype == torch.float32 and logits.stride(1) == 1,
@@ -1076,9 +1076,9 @@ def sample_chunked(logits: torch.Tensor, out: torch.Tensor, scratch: dict, tempe
     per_row = sample_chunks(vocab)
     for name, dt, need in (("part_max", torch.float32, rows * per_row), ("part_idx", torch.int32, rows * per_row),
                            ("part_mass", torch.float32, rows * per_row), ("seg_n", torch.int32, rows * per_row),
-                           ("done", torch.int32, rows), ("seg_i", torch.int32, rows * per_row * SAMPLE_SEGMENT),
-                           ("seg_x", torch.float32, rows * per_row * SAMPLE_SEGMENT),
-                           ("rest", torch.int32, rows * SAMPLE_REST)):
+                           ("done", torch.int32, rows),
+                           ("seg_i", torch.int32, rows * (per_row * (SAMPLE_SEGMENT + 1) + SAMPLE_REST)),
+                           ("seg_x", torch.float32, rows * per_row * SAMPLE_SEGMENT)):
         t = scratch[name]
         _need(t.dtype == dt and t.is_contiguous() and t.numel() >= need, f"sample_chunked: {name} must hold {need} {dt}")
     words = 0
@@ -1092,7 +1092,7 @@ def sample_chunked(logits: torch.Tensor, out: torch.Tensor, scratch: dict, tempe
          _ptr(temperature), _ptr(top_k), _ptr(top_p), _ptr(uniform), _ptr(penalty), _ptr(seen_row), _ptr(seen_masks),
          _ptr(banned), _i32(words), _ptr(scratch["part_max"]), _ptr(scratch["part_idx"]), _ptr(scratch["part_mass"]),
          _ptr(scratch["seg_i"]), _ptr(scratch["seg_x"]), _ptr(scratch["seg_n"]), _ptr(scratch["done"]),
-         _ptr(scratch["rest"]), _ptr(out), _stream())
+         _ptr(out), _stream())
 
 
 def argmax(logits: torch.Tensor, out: torch.Tensor, part_val: torch.Tensor, part_idx: torch.Tensor) -> None:
