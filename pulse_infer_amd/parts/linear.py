@@ -280,6 +280,8 @@ class Linear:
             return False
         if rows <= self.STAGE_ROWS[1]:
             return True
+        if self.takes_tiles(x, w, swiglu):      # (what ``OWN_MANY_ROWS`` asks for)
+            return False
         if not swiglu:
             return n <= 32 * compute_units() and rows <= self.STAGE_ROWS_NARROW
         return ((n <= 192 * compute_units() and rows <= self.STAGE_ROWS_SWIGLU[0])
@@ -291,6 +293,8 @@ class Linear:
         rows, n, k = x.shape[0], self.out_features, self.in_features
         if not (self.library and x.dtype == torch.bfloat16 and self.STAGE_ROWS[0] <= rows <= self.STAGE_ROWS_SHARES
                 and n * k >= self.STAGE_MIN_WEIGHT and self.operands_ok(x)) or n % 4 or k % 64:
+            return 0
+        if rows > self.STAGE_ROWS[1] and self.tile_shares_for(x):
             return 0
         return kernels.gemm_stages_shares(rows, n, k)
 
