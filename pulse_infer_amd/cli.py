@@ -62,10 +62,10 @@ def build_parser() -> argparse.ArgumentParser:
                         "config.json (for Qwen3: rope_pairing=half, the channels a rotation pairs); may be repeated")
     p.add_argument("--strict", action="store_true", help="a tensor that no part of the model asks for is an error")
     p.add_argument("--stats", action="store_true")
-    p.add_argument("--own-products", choices=["none", "swiglu", "all"], default=None,
-                   help="which bfloat16 products of 256 and more rows run as this package's tiled product instead of the "
-                        "vendor library's: gate and up with SwiGLU inside, all of them, or none "
-                        "(default: $PULSE_OWN_PRODUCTS, else none)")
+    p.add_argument("--own-products", choices=["none", "stages", "swiglu", "all"], default=None,
+                   help="which bfloat16 products of 256 and more rows run as this package's instead of the vendor "
+                        "library's: those that its product in stages is faster at, gate and up with SwiGLU inside or all of "
+                        "them in its tiled product, or none (default: $PULSE_OWN_PRODUCTS, else stages)")
     p.add_argument("--log-level", default=None, help="trace, debug, info, warn, error, critical or off "
                                                      "(default: $PULSE_LOG_LEVEL, else info); messages go to standard error")
     return p

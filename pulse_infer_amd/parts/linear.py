@@ -27,18 +27,18 @@ from ..ops.device import compute_units
 from .base import LazyNorm, RowStats, Workspace
 
 
-# Which products of many rows (256 and more) run as this package's tiled product instead of the library's: "none";
-# "swiglu": gate and up with SwiGLU inside, which saves the pass over twice the feed-forward's width; "all": every
-# product of bfloat16 (a step then makes no library call).  PULSE_OWN_PRODUCTS sets it.  Measured through the
-# serving loop: a prompt of 2,048 tokens of the 8B shape 73.9K tokens/s with "none", 72.9K with "swiglu", 71.6K with
-# "all" (alone and with the chip warm, gate+up with SwiGLU inside takes 310 us against the library's 328 + 30 for
-# the pass; between the other kernels of a step the library's product takes 278); serving of the 8B shape 4,334 /
-# 4,313 / 4,248 tokens/s, of the 14B shape 2,695 / 2,688 (means of two runs each, "none" and "swiglu"), of the 32B shape
-# 1,258 / 1,264.  So the library stays the default.
-OWN_MANY_ROWS = os.environ.get("PULSE_OWN_PRODUCTS", "none")
-if OWN_MANY_ROWS not in ("none", "swiglu", "all"):
-    raise ValueError(f"PULSE_OWN_PRODUCTS must be none, swiglu or all, not '{OWN_MANY_ROWS}'")
-
+# Which products of many rows (256 and more) run as this package's instead of the library's: "stages", the product in
+# stages where it is the faster one (``takes_stages``); or the tiled product, "swiglu": for gate and up with SwiGLU inside,
+# which saves the pass over twice the feed-forward's width (the others as with "stages"), "all": for every product of
+# bfloat16 (a step then makes no library call); "none": no product of more than 256 rows.  PULSE_OWN_PRODUCTS sets it.
+# Measured: a prompt of 509 tokens of the 8B shape 9.2 ms with "stages", 9.6 with "none".  Through the serving loop, a prompt of
+# 2,048 tokens 73.9K tokens/s with "none", 72.9K with "swiglu", 71.6K with "all" (alone and with the chip warm, gate+up
+# with SwiGLU inside takes 310 us against the library's 328 + 30 for the pass; between the other kernels of a step the
+# library's product takes 278); serving of the 8B shape 4,334 / 4,313 / 4,248 tokens/s, of the 14B shape 2,695 / 2,688 (means
+# of two runs each, "none" and "swiglu"), of the 32B shape 1,258 / 1,264.  So the library stays for the largest.
+OWN_MANY_ROWS = os.environ.get("PULSE_OWN_PRODUCTS", "stages")
+if OWN_MANY_ROWS not in ("none", "stages", "swiglu", "all"):
+    raise ValueError(f"PULSE_OWN_PRODUCTS must be none, stages, swiglu or all, not '{OWN_MANY_ROWS}'")
 library_calls = 0   # products that went to the vendor library so far (a step that made none can be recorded as a graph)
 
 
@@ -280,7 +280,7 @@ class Linear:
             return False
         if rows <= self.STAGE_ROWS[1]:
             return True
-        if self.takes_tiles(x, w, swiglu):      # (what ``OWN_MANY_ROWS`` asks for)
+        if OWN_MANY_ROWS == "none" or self.takes_tiles(x, w, swiglu):
             return False
         if not swiglu:
             return n <= 32 * compute_units() and rows <= self.STAGE_ROWS_NARROW
@@ -294,7 +294,7 @@ class Linear:
         if not (self.library and x.dtype == torch.bfloat16 and self.STAGE_ROWS[0] <= rows <= self.STAGE_ROWS_SHARES
                 and n * k >= self.STAGE_MIN_WEIGHT and self.operands_ok(x)) or n % 4 or k % 64:
             return 0
-        if rows > self.STAGE_ROWS[1] and self.tile_shares_for(x):
+        if rows > self.STAGE_ROWS[1] and (OWN_MANY_ROWS == "none" or self.tile_shares_for(x)):
             return 0
         return kernels.gemm_stages_shares(rows, n, k)
 
@@ -303,7 +303,7 @@ class Linear:
     def takes_tiles(self, x: torch.Tensor, w: Optional[torch.Tensor] = None, swiglu: bool = False) -> bool:
         """Whether a product of this many rows runs as this package's tiled product (``OWN_MANY_ROWS`` allowing)."""
         w = self.weight if w is None else w
-        if OWN_MANY_ROWS == "none" or (OWN_MANY_ROWS == "swiglu" and not swiglu):
+        if OWN_MANY_ROWS in ("none", "stages") or (OWN_MANY_ROWS == "swiglu" and not swiglu):
             return False
         return (self.library and x.dtype == torch.bfloat16 and x.shape[0] >= self.TILE_MIN_ROWS and self.operands_ok(x)
                 and kernels.gemm_tile_takes(x.shape[0], w.shape[0], w.shape[1], swiglu=swiglu))
