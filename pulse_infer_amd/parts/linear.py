@@ -261,8 +261,9 @@ class Linear:
     # 279 and 396); otherwise, up to 1,536 rows, where its tiles fill their rounds, which its estimate tells: at least 1.1
     # PFLOP/s (24,576 x 4,096 at 1,024 rows 176 against 184, but at 800 173 against 154; 34,816 x 5,120 at 1,024 322
     # against 410).  Plain products as long as the library leaves compute units idle (6,144 x 4,096 at 1,024 rows 51
-    # against 53), updates in shares up to 512 rows (4,096 x 4,096 at 512 rows 25 against 31, 4,096 x 12,288 at 357 47
-    # against 52, 2,560 x 9,728 27 against 41).  Small products stay where they are.
+    # against 53), updates in shares up to 512 rows unless the library's shares fill half the units (4,096 x 4,096 at 512 rows 25
+    # against 31, 2,560 x 9,728 at 357 27 against 41; 4,096 x 12,288 at 357 and 509 rows takes as long either way, 45 and 60,
+    # but in eight shares at 357, which cost the norm behind 2 more).  Small products stay where they are.
     STAGE_ROWS = (65, 256)              # any of these
     STAGE_ROWS_SWIGLU = (768, 1536)
     STAGE_SWIGLU_RATE = 1100            # flops a nanosecond
@@ -294,8 +295,13 @@ class Linear:
         if not (self.library and x.dtype == torch.bfloat16 and self.STAGE_ROWS[0] <= rows <= self.STAGE_ROWS_SHARES
                 and n * k >= self.STAGE_MIN_WEIGHT and self.operands_ok(x)) or n % 4 or k % 64:
             return 0
-        if rows > self.STAGE_ROWS[1] and (OWN_MANY_ROWS == "none" or self.tile_shares_for(x)):
-            return 0
+        if rows > self.STAGE_ROWS[1]:
+            if OWN_MANY_ROWS == "none" or self.tile_shares_for(x):
+                return 0
+            tile = self.LIBRARY_TILE
+            tiles = ((rows + tile - 1) // tile) * ((n + tile - 1) // tile) * self.library_shares_for(x)
+            if 2 * tiles >= compute_units():
+                return 0
         return kernels.gemm_stages_shares(rows, n, k)
 
     TILE_MIN_ROWS = 256          # from here on the tiled product for many rows is a candidate
