@@ -334,8 +334,7 @@ __global__ __launch_bounds__(256) void attn_rows_f32_kernel(const float* __restr
         if (c % 4 != wave) continue;
         f32x4 v = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int w = 0; w < 4; ++w)
-            if (factor[w] != 0.f) v += acc_s[w][c][lane] * factor[w];
+        for (int w = 0; w < 4; ++w) v += acc_s[w][c][lane] * factor[w];     // (NaN stays NaN whatever its share weighs)
         v *= rescale * inv;
         const int ch = 16 * c + 4 * kg;
         if (grow && a.gate_per_channel) {

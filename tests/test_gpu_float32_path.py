@@ -122,3 +122,42 @@ def test_float32_attention_of_whole_rows(k, d, nq, nkv, page, form):
         # more rounding a key and a handful for the exponentials and the gate
         bound = (2 * (d + 8) * U * float(size) + (int(see.sum()) + 64) * U) * float(vs[see].abs().max())
         assert float((got - want).abs().max()) <= bound, (t, e, p)
+
+
+@pytest.mark.parametrize("tokens", [1, 70])
+def test_float32_attention_hides_no_value_that_is_not_a_number(k, tokens):
+    """A query that is NaN, sixteen keys in a row that are (all that one wavefront sees of a request), and a value that is one
+    whose weight is nothing beside the others': what a token sees of them makes its row NaN, and no other."""
+    nq, nkv, d, page, before = 2, 1, 64, 16, 63
+    total = before + tokens
+    pages = (total + page - 1) // page
+    q = rnd(tokens, nq * d, seed=1)
+    ks, vs = rnd(3, total, d, seed=2), rnd(3, total, d, seed=3)
+    ks[1, 32:48] = float("nan")                   # request 1: every key of the third block
+    ks[2, :16] = 0.0
+    ks[2, 16:] = 40.0 * q[0, :d]                  # request 2: its first block's scores lie hundreds below the others
+    q[:, d:] = q[:, :d]
+    q[1:] = q[0]
+    vs[2, 5] = float("nan")
+    kc = torch.zeros(3 * pages, nkv, page, d)
+    vc = torch.zeros(3 * pages, nkv, d, page)
+    for r in range(3):
+        for j in range(total):
+            kc[r * pages + j // page, 0, j % page] = ks[r, j]
+            vc[r * pages + j // page, 0, :, j % page] = vs[r, j]
+    table = torch.arange(3 * pages, dtype=torch.int32).view(3, pages)
+
+    def run(entry, queries):
+        out = torch.full((tokens, nq * d), 7.0, device=DEV)
+        k.attn_generic(queries.to(DEV), out, nq, nkv, d, kc.to(DEV), vc.to(DEV),
+                       torch.arange(before, total, dtype=torch.int32, device=DEV),
+                       torch.full((tokens,), entry, dtype=torch.int32, device=DEV), table.to(DEV), 1.0)
+        return out.cpu().view(tokens, nq, d)
+
+    assert not torch.isnan(run(0, q)).any()
+    bad = q.clone()
+    bad[tokens - 1, d:] = float("nan")            # (the last token's second head)
+    out = run(0, bad)
+    assert torch.isnan(out[-1, 1]).all() and not torch.isnan(out[-1, 0]).any() and not torch.isnan(out[:-1]).any()
+    assert torch.isnan(run(1, q)).all()
+    assert torch.isnan(run(2, q)).all()
