@@ -328,7 +328,7 @@ __global__ void attn_wide_merge_kernel(const float* __restrict__ part, const flo
     const float l = lane < n_splits ? part_ml[2 * (at + lane) + 1] : 0.f;
     const float m_all = wave_max(m);
     const float f = m == -INFINITY ? 0.f : expf(m - m_all);
-    float l_all = wave_sum(f == 0.f ? 0.f : l * f);
+    float l_all = wave_sum(m == -INFINITY ? 0.f : l * f);
     if (threadIdx.x < PULSE_WAVE) factor[lane] = f;
     __syncthreads();
     float scale_out = 1.f;
@@ -349,10 +349,8 @@ __global__ void attn_wide_merge_kernel(const float* __restrict__ part, const flo
 #pragma unroll
             for (int u = 0; u < AHEAD; ++u) v[u] = from[static_cast<int64_t>(min(s0 + u, n_splits - 1)) * w];
 #pragma unroll
-            for (int u = 0; u < AHEAD; ++u) {      // (a split without keys has left nothing)
-                const float fu = s0 + u < n_splits ? factor[s0 + u] : 0.f;
-                if (fu != 0.f) sum = fmaf(v[u], fu, sum);
-            }
+            for (int u = 0; u < AHEAD; ++u)        // (a split without keys has left zeros; NaN stays NaN whatever it weighs)
+                if (s0 + u < n_splits) sum = fmaf(v[u], factor[s0 + u], sum);
         }
         orow[ch] = sum * inv;
     }
