@@ -114,7 +114,9 @@ __global__ __launch_bounds__(256) void gemm_stages_kernel(StageArgs a) {
 #pragma unroll
                         for (int i = 0; i < 4; ++i) {
                             const float gate = acc[q * 4 + i], up = acc[8 + q * 4 + i];
-                            v[i] = (__bf16)(gate * __builtin_amdgcn_rcpf(1.0f + __expf(-gate)) * up);
+                            // (a quarter of 1 + exp(-gate): its reciprocal is a normal number as long as the exponential is
+                            // finite.  expf and a division, no nearer to 64 bits behind the rounding to bfloat16, cost 2 to 16 %.)
+                            v[i] = (__bf16)(0.25f * gate * __builtin_amdgcn_rcpf(fmaf(0.25f, __expf(-gate), 0.25f)) * up);
                         }
                         *reinterpret_cast<tile_bf16x4*>(at + (f * 16 + q * 8 + h * 4) * 2) = v;
                     }

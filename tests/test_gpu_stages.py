@@ -57,3 +57,25 @@ def test_product_in_stages_refuses_what_it_cannot_read():
     assert not kernels.gemm_stages_takes(70, 64, 96) and kernels.gemm_stages_shares(70, 64, 96) == 0
     with pytest.raises((KernelError, ValueError)):
         kernels.gemm_stages(x, w, torch.empty(70, 64, dtype=torch.bfloat16, device=DEV))
+
+
+def test_product_in_stages_applies_silu_where_its_exponential_is_largest():
+    """Gates down to -88.6, where 1 / (1 + exp(-gate)) is smaller than any normal float32 number: silu(gate) is still one, and
+    so is its product with a large up."""
+    from pulse_infer_amd.ops import kernels
+
+    m, n, k = 65, 64, 64
+    gates = torch.linspace(-88.6, 88.6, m)
+    x, w = torch.zeros(m, k, dtype=torch.bfloat16), torch.zeros(n, k, dtype=torch.bfloat16)
+    high = gates.to(torch.bfloat16)
+    x[:, 0], x[:, 1], x[:, 2] = high, (gates - high.float()).to(torch.bfloat16), 1024.0
+    gate_rows = torch.arange(n) // 16 % 2 == 0
+    w[gate_rows, 0] = w[gate_rows, 1] = 1.0
+    w[~gate_rows, 2] = 1.0
+    act = torch.full((m, n // 2), float("nan"), dtype=torch.bfloat16, device=DEV)
+    kernels.gemm_stages(x.to(DEV), w.to(DEV), act, swiglu=True)
+    g = (x[:, 0].to(F64) + x[:, 1].to(F64)).view(m, 1)
+    want = (g / (1.0 + torch.exp(-g)) * 1024.0).expand(m, n // 2)
+    # the exponential of a number good to 2^-24 of up to 89 (2^-17), a reciprocal, one rounding to bfloat16
+    bound = (2.0 ** -8 + 2.0 ** -16) * want.abs() + 1024.0 * 2.0 ** -149
+    assert ((act.cpu().to(F64) - want).abs() <= bound).all()
