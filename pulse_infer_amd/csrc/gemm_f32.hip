@@ -268,6 +268,9 @@ __global__ __launch_bounds__(SHARES* PULSE_WAVE) void gemm_f32_staged_kernel(Gem
     int stage = 0;
     for (int b = b0; b < b_end; ++b) {
         const int next = stage == 0 ? S - 1 : stage - 1;
+        // (the reads of the stage that this copy goes to, those of the block before, have returned: the products that use
+        // them may be placed behind the copy, and the compiler does not know that it writes there)
+        asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");
         copy(b + S - 1, next);
         asm volatile("s_waitcnt vmcnt(%0)" : : "n"((S - 1) * (BN + BM)) : "memory");
         multiply(stage, b, b < b_full);

@@ -491,6 +491,28 @@ def test_top_p_alone_on_flat_rows_at_the_edges_of_the_passes(k, vocab, ties):
         assert ok, (r, t, other)
 
 
+def test_sampling_in_chunks_takes_scratch_without_room_for_what_is_left(k):
+    """Scratch of the segments alone, as a caller may have sized it by the chunks and the segment: the rows that the chunks
+    cannot choose for are then gone over by their own workgroup; the tokens are the same."""
+    rows, vocab = 6, 40000
+    gen = torch.Generator().manual_seed(9)
+    logits = (torch.randn(rows, vocab, generator=gen) * 1.5).to(DEV)
+    kw = dict(temperature=torch.full((rows,), 0.9).to(DEV), top_p=torch.tensor([0.9, 0.3, 1.0, 0.99, 0.5, 0.9]).to(DEV),
+              top_k=torch.tensor([0, 0, 0, 300, 40, 0], dtype=torch.int32).to(DEV), uniform=torch.rand(rows, generator=gen).to(DEV))
+    chunks = k.sample_chunks(vocab)
+    f32 = lambda n: torch.full((n,), float("nan"), device=DEV)
+    i32 = lambda n: torch.full((n,), -77, dtype=torch.int32, device=DEV)
+    guarded = i32(rows * chunks * k.SAMPLE_SEGMENT + 4096)
+    scratch = {"part_max": f32(rows * chunks), "part_idx": i32(rows * chunks), "part_mass": f32(rows * chunks),
+               "seg_n": i32(rows * chunks), "done": i32(rows), "seg_i": guarded[: rows * chunks * k.SAMPLE_SEGMENT],
+               "seg_x": f32(rows * chunks * k.SAMPLE_SEGMENT)}
+    few, usual = (torch.full((rows,), -9, dtype=torch.int32, device=DEV) for _ in range(2))
+    k.sample_chunked(logits, few, scratch, **kw)
+    k.sample_chunked(logits, usual, _chunked_scratch(k, rows, vocab), **kw)
+    assert few.tolist() == usual.tolist() and min(few.tolist()) >= 0
+    assert (guarded[rows * chunks * k.SAMPLE_SEGMENT:] == -77).all()      # nothing is written behind it
+
+
 def _chunked_scratch(k, rows, vocab):
     scratch = k.sample_chunked_scratch(rows, vocab, DEV)
     for t in scratch.values():                             # nothing that was not written is used
