@@ -16,6 +16,7 @@
 // (106 TFLOP/s), 16,384 x 2,048 at 333 rows 699 -> 202 (110), 2,048 x 8,192 at 1,024 rows 271 (127), 32,000 x 2,048 at one
 // row 276 -> 55 (4.7 TB/s).  The error against 64 bits halves (K of 2,048: 8e-7 -> 4e-7): four shorter sums.
 #include "common.h"
+#include "tile_loop.h"
 
 namespace {
 
@@ -35,25 +36,20 @@ struct GemmArgs {
     int tiles_m, tiles_n;
 };
 
-// Values k .. k + 3 of a row.  VEC: the row can be read in pieces of four, and K is a multiple of 4; a piece past the end is
-// then the row's last piece, read for nobody, so that no lane branches round a load.
-template <typename T, bool VEC>
+// Values k .. k + 3 of a row that can be read in pieces of four, K a multiple of 4; a piece past the end is the row's last
+// piece, read for nobody, so that no lane branches round a load.
+template <typename T>
 __device__ __forceinline__ f32x4 load4(const T* row, int k, int K) {
     f32x4 v;
-    if constexpr (VEC) {
-        const int at = min(k, K - 4);
-        if constexpr (sizeof(T) == 4) {
-            v = *reinterpret_cast<const f32x4*>(row + at);
-        } else {
-            const uint2 raw = *reinterpret_cast<const uint2*>(row + at);
-            v[0] = __uint_as_float(raw.x << 16);
-            v[1] = __uint_as_float(raw.x & 0xffff0000u);
-            v[2] = __uint_as_float(raw.y << 16);
-            v[3] = __uint_as_float(raw.y & 0xffff0000u);
-        }
+    const int at = min(k, K - 4);
+    if constexpr (sizeof(T) == 4) {
+        v = *reinterpret_cast<const f32x4*>(row + at);
     } else {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = k + e < K ? to_f32<T>(row[k + e]) : 0.f;
+        const uint2 raw = *reinterpret_cast<const uint2*>(row + at);
+        v[0] = __uint_as_float(raw.x << 16);
+        v[1] = __uint_as_float(raw.x & 0xffff0000u);
+        v[2] = __uint_as_float(raw.y << 16);
+        v[3] = __uint_as_float(raw.y & 0xffff0000u);
     }
     return v;
 }
@@ -80,7 +76,7 @@ __device__ __forceinline__ void store_tile(const GemmArgs& a, int m, int n, f32x
 
 // A workgroup's tile is 16 * BN weight rows (the row operand) by 16 * BM rows of A (the column operand); U blocks of k
 // are a stage.
-template <typename TA, typename TW, bool VEC, int BM, int BN, int U>
+template <typename TA, typename TW, int BM, int BN, int U>
 __global__ __launch_bounds__(SHARES* PULSE_WAVE) void gemm_f32_kernel(GemmArgs a) {
     constexpr int TILES = BM * BN;
     constexpr int PASS = TILES % 8 == 0 ? 8 : TILES % 6 == 0 ? 6 : TILES % 9 == 0 ? 9 : TILES;     // tiles of the matrix instruction a pass of the meeting in LDS
@@ -122,9 +118,9 @@ __global__ __launch_bounds__(SHARES* PULSE_WAVE) void gemm_f32_kernel(GemmArgs a
         for (int u = 0; u < U; ++u) {
             const int k = (block + u) * KB + 4 * kg;
 #pragma unroll
-            for (int j = 0; j < BN; ++j) wv[set][u][j] = load4<TW, VEC>(wrow[j], k, a.K);
+            for (int j = 0; j < BN; ++j) wv[set][u][j] = load4<TW>(wrow[j], k, a.K);
 #pragma unroll
-            for (int i = 0; i < BM; ++i) av[set][u][i] = load4<TA, VEC>(arow[i], k, a.K);
+            for (int i = 0; i < BM; ++i) av[set][u][i] = load4<TA>(arow[i], k, a.K);
         }
         __builtin_amdgcn_sched_barrier(0);   // (the loads stay ahead of the products that they hide behind)
     };
@@ -297,6 +293,123 @@ __global__ __launch_bounds__(SHARES* PULSE_WAVE) void gemm_f32_staged_kernel(Gem
     }
 }
 
+// The same walk for rows that cannot be read in pieces of four (their length or distance is no multiple of four values):
+// a block's 16 rows are read four rows an instruction, the 16 values of each side by side, so that an instruction touches
+// four to eight lines where value e of every lane's piece touches sixteen, and go through LDS of the wavefront's own into the
+// operands' order.  2,050 weight rows of 1,001, float32 and bfloat16: 4,096 rows 273 and 265 us, straight into registers 734
+// and 783 (scalar multiply-adds on a 64 x 64 tile in LDS 527 and 460); 17 rows 10.8 and 10.7, 21.5 and 31.3 (177 and 128).
+template <typename TA, typename TW, int BM, int BN>
+__global__ __launch_bounds__(SHARES* PULSE_WAVE) void gemm_f32_ragged_kernel(GemmArgs a) {
+    constexpr int TILES = BM * BN, T = BM + BN;
+    constexpr int PASS = TILES % 8 == 0 ? 8 : TILES % 6 == 0 ? 6 : TILES % 9 == 0 ? 9 : TILES;
+    constexpr int STAGE = T * 1024, MEET = SHARES * PASS * PULSE_WAVE * 16;
+    __shared__ __attribute__((aligned(1024))) char lds[SHARES * STAGE > MEET ? SHARES * STAGE : MEET];
+
+    const int total = a.tiles_m * a.tiles_n;
+    const int per_die = (total + 7) / 8;
+    const int tile = (blockIdx.x % 8) * per_die + blockIdx.x / 8;
+    if (static_cast<int>(blockIdx.x / 8) >= per_die || tile >= total) return;
+    const int m0 = tile % a.tiles_m * (16 * BM), n0 = tile / a.tiles_m * (16 * BN);
+
+    const int lane = threadIdx.x % PULSE_WAVE;
+    const int share = __builtin_amdgcn_readfirstlane(threadIdx.x / PULSE_WAVE);
+    const int r = lane % 16, kg = lane / 16;
+    const int blocks = (a.K + KB - 1) / KB;
+    const int b_end = static_cast<int>(static_cast<int64_t>(blocks) * (share + 1) / SHARES);
+    const int b0 = static_cast<int>(static_cast<int64_t>(blocks) * share / SHARES);
+
+    // raw[t][e]: value lane % 16 of row 4 e + lane / 16 of the t-th sixteen rows; piece c of row q sits at place c ^ (q / 4 % 4)
+    float raw[T][4];
+    auto fetch = [&](int block) __attribute__((always_inline)) {
+        const int k = block * KB + r;
+        const bool in = k < a.K;
+        const int at = in ? k : a.K - 1;
+#pragma unroll
+        for (int t = 0; t < T; ++t)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int row = 4 * e + kg;
+                if (t < BN)
+                    raw[t][e] = to_f32<TW>(static_cast<const TW*>(a.W)[static_cast<int64_t>(min(n0 + 16 * t + row, a.N - 1)) * a.ldw + at]);
+                else
+                    raw[t][e] = to_f32<TA>(static_cast<const TA*>(a.A)[static_cast<int64_t>(min(m0 + 16 * (t - BN) + row, a.M - 1)) * a.lda + at]);
+                raw[t][e] = in ? raw[t][e] : 0.f;
+            }
+        __builtin_amdgcn_sched_barrier(0);   // (the loads stay ahead of the products that they hide behind)
+    };
+    float* mine = reinterpret_cast<float*>(lds + share * STAGE);
+    f32x4 v[T];
+    auto turn = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int t = 0; t < T; ++t)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) mine[t * 256 + (4 * e + kg) * 16 + ((r / 4) ^ e) * 4 + r % 4] = raw[t][e];
+        tile_wave_sync();
+#pragma unroll
+        for (int t = 0; t < T; ++t) v[t] = *reinterpret_cast<const f32x4*>(mine + t * 256 + r * 16 + (kg ^ (r / 4 % 4)) * 4);
+        tile_wave_sync();
+    };
+
+    f32x4 acc[BN][BM];
+#pragma unroll
+    for (int j = 0; j < BN; ++j)
+#pragma unroll
+        for (int i = 0; i < BM; ++i) acc[j][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (b0 < b_end) {
+        fetch(b0);
+        turn();
+        for (int b = b0; b < b_end; ++b) {
+            if (b + 1 < b_end) fetch(b + 1);
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int j = 0; j < BN; ++j)
+#pragma unroll
+                    for (int i = 0; i < BM; ++i)
+                        acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[j][e], v[BN + i][e], acc[j][i], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            if (b + 1 < b_end) turn();
+        }
+    }
+    __syncthreads();
+
+    f32x4* meet = reinterpret_cast<f32x4*>(lds);          // [SHARES][PASS][64]
+#pragma unroll
+    for (int t0 = 0; t0 < TILES; t0 += PASS) {
+        if (t0 > 0) __syncthreads();
+#pragma unroll
+        for (int t = 0; t < PASS; ++t) meet[(share * PASS + t) * PULSE_WAVE + lane] = acc[(t0 + t) / BM][(t0 + t) % BM];
+        __syncthreads();
+#pragma unroll
+        for (int t = 0; t < PASS; ++t) {
+            if (t % SHARES != share) continue;
+            f32x4 sum = meet[t * PULSE_WAVE + lane];
+#pragma unroll
+            for (int s = 1; s < SHARES; ++s) sum += meet[(s * PASS + t) * PULSE_WAVE + lane];
+            store_tile(a, m0 + 16 * ((t0 + t) % BM) + r, n0 + 16 * ((t0 + t) / BM) + 4 * kg, sum);
+        }
+    }
+}
+
+template <typename TA, typename TW, int BM, int BN>
+void launch_ragged(GemmArgs a, hipStream_t stream) {
+    a.tiles_m = (a.M + 16 * BM - 1) / (16 * BM);
+    a.tiles_n = (a.N + 16 * BN - 1) / (16 * BN);
+    const unsigned grid = static_cast<unsigned>((static_cast<int64_t>(a.tiles_m) * a.tiles_n + 7) / 8 * 8);
+    hipLaunchKernelGGL((gemm_f32_ragged_kernel<TA, TW, BM, BN>), dim3(grid), dim3(SHARES * PULSE_WAVE), 0, stream, a);
+}
+
+// Up to 128 rows tiles of 16 x 32, of which there are enough (100 rows, 2,050 x 1,001: 14.5 us, 19.1 with 32 x 32); beyond, 32
+// x 64 where a compute unit gets eight or more of them (4,096 rows: 273 us, 313 with 32 x 32), else 32 x 32 (1,024 rows: 81, 85
+// with 32 x 64; 48 x 64 and 64 x 64 were slower throughout, 334 and 301 at 4,096 rows).
+template <typename TA, typename TW>
+void launch_ragged_for(const GemmArgs& a, hipStream_t stream) {
+    const int64_t wide = static_cast<int64_t>((a.M + 31) / 32) * ((a.N + 63) / 64);
+    if (a.M <= 128) launch_ragged<TA, TW, 1, 2>(a, stream);
+    else if (wide >= 8 * static_cast<int64_t>(pulse_compute_units())) launch_ragged<TA, TW, 2, 4>(a, stream);
+    else launch_ragged<TA, TW, 2, 2>(a, stream);
+}
+
 template <int BM, int BN, int S>
 void launch_staged(GemmArgs a, hipStream_t stream) {
     a.tiles_m = (a.M + 16 * BM - 1) / (16 * BM);
@@ -305,12 +418,12 @@ void launch_staged(GemmArgs a, hipStream_t stream) {
     hipLaunchKernelGGL((gemm_f32_staged_kernel<BM, BN, S>), dim3(grid), dim3(SHARES * PULSE_WAVE), 0, stream, a);
 }
 
-template <typename TA, typename TW, bool VEC, int BM, int BN, int U>
+template <typename TA, typename TW, int BM, int BN, int U>
 void launch(GemmArgs a, hipStream_t stream) {
     a.tiles_m = (a.M + 16 * BM - 1) / (16 * BM);
     a.tiles_n = (a.N + 16 * BN - 1) / (16 * BN);
     const unsigned grid = static_cast<unsigned>((static_cast<int64_t>(a.tiles_m) * a.tiles_n + 7) / 8 * 8);
-    hipLaunchKernelGGL((gemm_f32_kernel<TA, TW, VEC, BM, BN, U>), dim3(grid), dim3(SHARES * PULSE_WAVE), 0, stream, a);
+    hipLaunchKernelGGL((gemm_f32_kernel<TA, TW, BM, BN, U>), dim3(grid), dim3(SHARES * PULSE_WAVE), 0, stream, a);
 }
 
 }  // namespace
@@ -335,10 +448,10 @@ extern "C" int pulse_gemm_f32(const void* A, int a_dtype, const void* W, int w_d
     // 38 -> 30 us; 2,048 x 8,192 29 -> 74).
     if (M <= 16 || !vec || a_size != 4 || w_size != 4) {
         PULSE_DISPATCH_DTYPE(a_dtype, TA, PULSE_DISPATCH_DTYPE(w_dtype, TW,
-            if (!vec) launch<TA, TW, false, 2, 2, 1>(a, stream);
-            else if (M > 16) launch<TA, TW, true, 2, 2, 2>(a, stream);
-            else if (N >= 64 * pulse_compute_units()) launch<TA, TW, true, 1, 4, 2>(a, stream);
-            else launch<TA, TW, true, 1, 1, 4>(a, stream)));
+            if (!vec) launch_ragged_for<TA, TW>(a, stream);
+            else if (M > 16) launch<TA, TW, 2, 2, 2>(a, stream);
+            else if (N >= 64 * pulse_compute_units()) launch<TA, TW, 1, 4, 2>(a, stream);
+            else launch<TA, TW, 1, 1, 4>(a, stream)));
     } else {
         // The tile whose fullest compute unit ends first: workgroups on it x (pairs of blocks in a tile + 2, what a
         // workgroup costs beside its products).  Measured at 333 rows: 2,048 weight rows of 8,192 133 / 144 / 105 / 134 us

@@ -22,9 +22,9 @@ def rnd(*shape, seed):
 
 # rows x weight rows x K: one and sixteen rows with few and many weight rows; every staged tile (the rule's 2 x 2, 2 x 4,
 # 3 x 4 and 4 x 4 blocks), with remainders of rows, weight rows and K; shares of K of no, one and unequal numbers of blocks;
-# rows that are no multiple of four, which take scalar loads
+# rows that are no multiple of four, which are read value by value: tiles of 16 x 32, 32 x 32 and 32 x 64, K below one block
 @pytest.mark.parametrize("shape", [(1, 100, 4), (1, 16400, 20), (16, 33, 68), (17, 40, 16), (40, 90, 300), (49, 2050, 1028),
-                                   (97, 2048, 52), (333, 2048, 100), (333, 5000, 84), (1030, 4100, 36), (65, 70, 257)])
+                                   (97, 2048, 52), (333, 2048, 100), (333, 5000, 84), (1030, 4100, 36), (65, 70, 257), (1, 33, 3), (130, 1010, 67), (129, 100, 1001), (2050, 2100, 18)])
 @pytest.mark.parametrize("types", [(torch.float32, torch.float32, torch.float32), (torch.bfloat16, torch.float32, torch.float32),
                                    (torch.float32, torch.bfloat16, torch.bfloat16)])
 def test_float32_product_at_the_edges_of_its_tiles(k, shape, types):
