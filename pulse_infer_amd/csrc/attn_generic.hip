@@ -165,8 +165,18 @@ __global__ __launch_bounds__(64) void attn_generic_kernel(const TX* __restrict__
 // row, 28 us with this.
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 
+// f over the values of the first sixteen lanes.
+template <typename F>
+__device__ __forceinline__ int of_sixteen(int v, F f) {
+    v = f(v, __builtin_amdgcn_update_dpp(v, v, 0x128, 0xf, 0xf, false));    // (row_ror:8, then 4, 2, 1)
+    v = f(v, __builtin_amdgcn_update_dpp(v, v, 0x124, 0xf, 0xf, false));
+    v = f(v, __builtin_amdgcn_update_dpp(v, v, 0x122, 0xf, 0xf, false));
+    v = f(v, __builtin_amdgcn_update_dpp(v, v, 0x121, 0xf, 0xf, false));
+    return __builtin_amdgcn_readfirstlane(v);
+}
+
 template <int DB>
-__global__ __launch_bounds__(256) void attn_rows_f32_kernel(const float* __restrict__ q, float* __restrict__ out,
+__global__ __launch_bounds__(256, DB == 2 ? 5 : DB == 4 ? 4 : 1) void attn_rows_f32_kernel(const float* __restrict__ q, float* __restrict__ out,
                                                             const float* __restrict__ kcache,
                                                             const float* __restrict__ vcache,
                                                             const int* __restrict__ positions,
@@ -174,21 +184,29 @@ __global__ __launch_bounds__(256) void attn_rows_f32_kernel(const float* __restr
                                                             const int* __restrict__ block_table,
                                                             const float* __restrict__ gate, int64_t gate_stride,
                                                             const float* __restrict__ sink, AttnArgs a, int tokens, int tp,
-                                                            int hp) {
+                                                            int hp, int takers) {
     constexpr int D = 16 * DB;
     __shared__ f32x4 acc_s[4][DB][PULSE_WAVE];
     __shared__ float m_s[4][16], l_s[4][16];
 
     const int group = a.nq / a.nkv;
     const int t0 = blockIdx.x * tp;
-    const int kvh = blockIdx.y, h0 = kvh * group + blockIdx.z * hp;
+    const int kvh = blockIdx.y, parts = (group + hp - 1) / hp, turn = blockIdx.z / parts, first_head = blockIdx.z % parts * hp, h0 = kvh * group + first_head;
     const int lane = threadIdx.x % PULSE_WAVE;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / PULSE_WAVE);
     const int r = lane % 16, kg = lane / 16;
     const int t_end = min(t0 + tp, tokens);
 
+    // A tile may hold tokens of several entries: every one's rows are a walk of their own, which begin where `begins` has a
+    // bit, and the workgroups of the tile take them in turn.  (Lane i looks at the tile's i-th token.)
+    const int n = t_end - t0, own = t0 + min(lane, n - 1);
+    const int own_entry = token_entry[own], own_pos = positions[own];
+    const int entry_before = __shfl_up(own_entry, 1, PULSE_WAVE);
+    unsigned long long begins = __ballot(lane < n && (lane == 0 || own_entry != entry_before));
+    if (turn > 0 && __popcll(begins) <= turn) return;       // (the first has a walk for sure and need not wait to know it)
+
     // this lane's row (a row past the end is row 0 of the tile, sees nothing and is not written)
-    const bool live = r / hp < tp && t0 + r / hp < t_end && blockIdx.z * hp + r % hp < group;
+    bool live = r / hp < tp && t0 + r / hp < t_end && first_head + r % hp < group;
     const int t = live ? t0 + r / hp : t0;
     const int h = live ? h0 + r % hp : h0;
     const int pos = live ? positions[t] : -1;
@@ -281,23 +299,26 @@ __global__ __launch_bounds__(256) void attn_rows_f32_kernel(const float* __restr
         }
     };
 
-    for (int ta = t0; ta < t_end;) {      // a tile may hold tokens of several entries: one after the other
-        const int entry = token_entry[ta];
-        int hi = -1, low = 0x7fffffff, kept = 0, tb = ta;
-        for (; tb < t_end && token_entry[tb] == entry; ++tb) {
-            const int p = positions[tb];
-            const int l0 = a.chunk > 0 ? p - p % a.chunk : (a.window > 0 && p - a.window + 1 > 0) ? p - a.window + 1 : 0;
-            hi = max(hi, p);
-            low = min(low, l0);
-            kept = max(kept, min(a.keep_first, l0));
-        }
-        const int* bt = block_table + static_cast<int64_t>(entry) * a.bt_width;
-        const bool in_entry = t >= ta && t < tb;
+    const int own_lo = a.chunk > 0 ? own_pos - own_pos % a.chunk : (a.window > 0 && own_pos - a.window + 1 > 0) ? own_pos - a.window + 1 : 0;
+    bool took = false;
+    for (int run = 0; begins != 0; ++run) {
+        const int ia = __builtin_ctzll(begins);
+        begins &= begins - 1;
+        const int ib = begins != 0 ? __builtin_ctzll(begins) : n;
+        if (run % takers != turn) continue;
+        const bool in_walk = lane >= ia && lane < ib;
+        int hi = in_walk ? own_pos : -1, low = in_walk ? own_lo : 0x7fffffff, kept = in_walk ? min(a.keep_first, own_lo) : 0;
+        hi = of_sixteen(hi, [](int x, int y) { return max(x, y); });
+        low = of_sixteen(low, [](int x, int y) { return min(x, y); });
+        kept = of_sixteen(kept, [](int x, int y) { return max(x, y); });
+        const int* bt = block_table + static_cast<int64_t>(__builtin_amdgcn_readlane(own_entry, ia)) * a.bt_width;
+        const bool in_entry = t >= t0 + ia && t < t0 + ib;
         const int first = (kept + 15) / 16, from = max(low / 16, first), to = hi / 16;
         for (int b = wave; b < first && b <= to; b += 4) block(b, bt, in_entry);
         for (int b = from + ((wave - from) & 3); b <= to; b += 4) block(b, bt, in_entry);
-        ta = tb;
+        took = took || in_entry;
     }
+    live = live && took;
 
     l += __shfl_xor(l, 16, PULSE_WAVE);
     l += __shfl_xor(l, 32, PULSE_WAVE);
@@ -360,12 +381,18 @@ int launch_rows_f32(const void* q, void* out, const void* kcache, const void* vc
     const int hp = group < 16 ? group : 16;
     // Few tokens (decoding) get a tile each: their keys are those of one request or another, and more tiles fill the chip.
     const int tp = tokens <= 64 ? 1 : 16 / hp;
-    const dim3 grid((tokens + tp - 1) / tp, a.nkv, (group + hp - 1) / hp);
+    // More tokens may still be as many requests, whose walks one workgroup would do one behind the other (80 requests of 1,000
+    // keys, 8 heads of 256 with keys of their own: 1,870 us): as many workgroups a tile as the chip has room for take them in
+    // turn (398 us), and in a prompt, where a tile is one walk, all but the first of them leave at once.
+    const int tiles = (tokens + tp - 1) / tp, z = (group + hp - 1) / hp;
+    const int64_t walks = static_cast<int64_t>(tiles) * a.nkv * z, room = 8 * static_cast<int64_t>(pulse_compute_units());
+    const int takers = static_cast<int>(walks * tp <= room ? tp : walks < room ? room / walks : 1);
+    const dim3 grid(tiles, a.nkv, z * takers);     // (those that leave at once come last)
 #define PULSE_ROWS_LAUNCH(DB)                                                                                            \
     hipLaunchKernelGGL((attn_rows_f32_kernel<DB>), grid, dim3(256), 0, stream, static_cast<const float*>(q),             \
                        static_cast<float*>(out), static_cast<const float*>(kcache), static_cast<const float*>(vcache),  \
                        positions, token_entry, block_table, static_cast<const float*>(gate), gate_stride, sink, a, tokens, \
-                       tp, hp)
+                       tp, hp, takers)
     if (a.d == 32) PULSE_ROWS_LAUNCH(2);
     else if (a.d == 64) PULSE_ROWS_LAUNCH(4);
     else if (a.d == 128) PULSE_ROWS_LAUNCH(8);

@@ -124,6 +124,34 @@ def test_float32_attention_of_whole_rows(k, d, nq, nkv, page, form):
         assert float((got - want).abs().max()) <= bound, (t, e, p)
 
 
+@pytest.mark.parametrize("requests", [65, 1100])
+def test_float32_attention_of_many_requests_at_once(k, requests):
+    """A step of single tokens whose tiles hold sixteen requests each, with a workgroup a request and, where the chip has no room
+    for that many, with several each; portions of two tokens among them."""
+    nq, d, page = 8, 32, 16
+    gen = torch.Generator().manual_seed(4)
+    last = torch.randint(1, 3 * page, (requests,), generator=gen)
+    counts = [2 if i % 7 == 3 else 1 for i in range(requests)]
+    entry = [i for i, c in enumerate(counts) for _ in range(c)]
+    positions = [int(last[i]) - c + 1 + j for i, c in enumerate(counts) for j in range(c)]
+    ks, vs = rnd(requests, 3 * page, nq, d, seed=5), rnd(requests, 3 * page, nq, d, seed=6)
+    q = rnd(len(entry), nq * d, seed=7)
+    kc = ks.view(requests * 3, page, nq, d).transpose(1, 2).contiguous()
+    vc = vs.view(requests * 3, page, nq, d).permute(0, 2, 3, 1).contiguous()
+    out = torch.full((len(entry), nq * d), 7.0, device=DEV)
+    ints = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    k.attn_generic(q.to(DEV), out, nq, nq, d, kc.to(DEV), vc.to(DEV), ints(positions), ints(entry),
+                   torch.arange(requests * 3, dtype=torch.int32, device=DEV).view(requests, 3), 0.3)
+    e, p = torch.tensor(entry), torch.tensor(positions)
+    s = (q.view(-1, 1, nq, d).to(F64) * ks[e].to(F64)).sum(-1) * 0.3                       # [tokens, keys, heads]
+    s = s.masked_fill((torch.arange(3 * page).view(1, -1) > p.view(-1, 1)).unsqueeze(-1), float("-inf"))
+    want = (torch.softmax(s, 1).unsqueeze(-1) * vs[e].to(F64)).sum(1).reshape(len(entry), nq * d)
+    size = float((q.view(-1, 1, nq, d).abs() * ks[e].abs()).sum(-1).max()) * 0.3
+    # (as above: scores off by (d + 8) u of their size, weights by twice that, a rounding a key and some for the exponentials)
+    bound = (2 * (d + 8) * U * size + (3 * page + 64) * U) * float(vs.abs().max())
+    assert float((out.cpu().to(F64) - want).abs().max()) <= bound
+
+
 @pytest.mark.parametrize("tokens", [1, 70])
 def test_float32_attention_hides_no_value_that_is_not_a_number(k, tokens):
     """A query that is NaN, sixteen keys in a row that are (all that one wavefront sees of a request), and a value that is one
