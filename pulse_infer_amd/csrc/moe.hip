@@ -189,16 +189,22 @@ __global__ __launch_bounds__(1024) void moe_router_kernel(const TX* __restrict__
 }
 
 // The same for bfloat16 rows and weights, sixteen tokens a workgroup: the logits are products of 16 outputs with 16 tokens
-// on the matrix cores (exact products, float32 sums), K shared out over sixteen wavefronts in steps of 32, whose sums meet
-// in LDS in their order; then a wavefront a token routes.  A token's logits do not depend on its neighbours.
+// on the matrix cores (exact products, float32 sums).  The sixteen wavefronts take a block of outputs each, or share a block's
+// K out in steps of 32 where there are fewer blocks, and meet in LDS in their order; then a wavefront a token routes.  A
+// token's logits do not depend on its neighbours.
 //
-// A workgroup a token reads every output's weights for one row: 2,048 tokens of 4,096 with 16 outputs 83 us, 17 with
-// this; 8 tokens 21 us (its dot products read the row from LDS eight lanes a bank, and the choice took sixteen values a
-// lane whatever the number of outputs), 13.
+// What bounds it: what a compute unit takes in, every output's weights for sixteen tokens (a workgroup a token: for one), and
+// the trips to memory of a walk.  us at 1 / 16 / 256 / 2,048 tokens:
+//   outputs x width               16 x 4,096            64 x 2,048            128 x 2,048            256 x 7,168
+//   a workgroup a token           24 / 24 / 25 / 81     31 / 32 / 33 / 141    46 / 47 / 48 / 259     214 / 215 / 218 / 1,615
+//   a block behind the other      12 / 16 / 17 / 17     27 / 39 / 39 / 40     49 / 71 / 72 / 72      157 / 245 / 246 / 248
+//   this                          13 / 17 / 17 / 17     17 / 23 / 24 / 24     28 / 40 / 40 / 41      132 / 204 / 205 / 207
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 constexpr int TILE_TOKENS = 16;
 constexpr int TILE_WAVES = 16;
+template <int V>
+struct Steps { static constexpr int value = V; };
 
 template <int PER>
 __global__ __launch_bounds__(1024) void moe_router_tile_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
@@ -211,33 +217,48 @@ __global__ __launch_bounds__(1024) void moe_router_tile_kernel(const bf16_t* __r
     const int r = lane % 16, kg = lane / 16;
     const int t0 = blockIdx.x * TILE_TOKENS;
     const bf16_t* xrow = x + static_cast<int64_t>(min(t0 + r, tokens - 1)) * hidden + kg * 8;
-    const int steps = hidden / 32;
-    for (int o0 = 0; o0 < n; o0 += 16) {
-        const bf16_t* wrow = w + static_cast<int64_t>(min(o0 + r, n - 1)) * hidden + kg * 8;
+    const int steps = hidden / 32, blocks = (n + 15) / 16;
+    int shares = TILE_WAVES;
+    while (shares > 1 && shares * blocks > TILE_WAVES) shares /= 2;
+    const int share = wave % shares;
+    for (int b0 = 0; b0 < blocks; b0 += TILE_WAVES / shares) {       // (with shares: once)
+        const int block = b0 + wave / shares, o0 = 16 * block;
         f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-        constexpr int AHEAD = 8;
-        for (int s0 = wave; s0 < steps; s0 += AHEAD * TILE_WAVES) {
-            bf16x8 wv[AHEAD], xv[AHEAD];
+        if (block < blocks) {
+            const bf16_t* wrow = w + static_cast<int64_t>(min(o0 + r, n - 1)) * hidden + kg * 8;
+            auto walk = [&](int s0, auto ahead) __attribute__((always_inline)) {
+                constexpr int AHEAD = decltype(ahead)::value;
+                bf16x8 wv[AHEAD], xv[AHEAD];
 #pragma unroll
-            for (int u = 0; u < AHEAD; ++u) {        // (past the end: the first step's again, for nobody)
-                const int s = s0 + u * TILE_WAVES, at = (s < steps ? s : s0) * 32;
-                wv[u] = *reinterpret_cast<const bf16x8*>(wrow + at);
-                xv[u] = *reinterpret_cast<const bf16x8*>(xrow + at);
+                for (int u = 0; u < AHEAD; ++u) {        // (past the end: the first step's again, for nobody)
+                    const int s = s0 + u * shares, at = (s < steps ? s : s0) * 32;
+                    wv[u] = *reinterpret_cast<const bf16x8*>(wrow + at);
+                    xv[u] = *reinterpret_cast<const bf16x8*>(xrow + at);
+                }
+#pragma unroll
+                for (int u = 0; u < AHEAD; ++u)
+                    if (s0 + u * shares < steps) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv[u], xv[u], acc, 0, 0, 0);
+            };
+            for (int s0 = share; s0 < steps;) {
+                if (s0 + 4 * shares < steps) {
+                    walk(s0, Steps<8>());
+                    s0 += 8 * shares;
+                } else {
+                    walk(s0, Steps<4>());
+                    s0 += 4 * shares;
+                }
             }
-#pragma unroll
-            for (int u = 0; u < AHEAD; ++u)
-                if (s0 + u * TILE_WAVES < steps) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv[u], xv[u], acc, 0, 0, 0);
         }
-        if (o0 > 0) __syncthreads();
-        meet[wave][lane] = acc;
-        __syncthreads();
-        if (wave == 0) {     // lane l holds outputs 4 * (l / 16) + e of token l % 16
-            f32x4 v = meet[0][lane];
-#pragma unroll
-            for (int i = 1; i < TILE_WAVES; ++i) v += meet[i][lane];
+        if (shares > 1) {
+            meet[wave][lane] = acc;
+            __syncthreads();
+            if (share == 0)
+                for (int i = 1; i < shares; ++i) acc += meet[wave + i][lane];
+        }
+        if (share == 0) {    // lane l holds outputs 4 * (l / 16) + e of token l % 16
 #pragma unroll
             for (int e = 0; e < 4; ++e)
-                if (o0 + 4 * kg + e < n) z_s[r * n + o0 + 4 * kg + e] = v[e];
+                if (o0 + 4 * kg + e < n) z_s[r * n + o0 + 4 * kg + e] = acc[e];
         }
     }
     __syncthreads();

@@ -1,4 +1,4 @@
-"""Experts' products grouped by expert where their tiles end."""
+"""The router on the matrix cores and the experts' products grouped by expert, where their tiles end."""
 import pytest
 import torch
 
@@ -52,3 +52,34 @@ def test_grouped_experts_at_the_edges_of_their_tiles(hidden, ff, rows, form):
     if form == "silu":
         want, size = want * weight, size * weight
     assert ((out.cpu().to(F64) - want).abs() <= (ff + 4) * 2.0 ** -24 * size).all()
+
+
+# one block of outputs for all sixteen wavefronts to share, two, five (two wavefronts a block), nine and seventeen (one, and a
+# second round); widths of fewer steps of 32 than wavefronts, of a whole round of eight ahead, of a remainder, of several rounds
+@pytest.mark.parametrize("n", [8, 17, 65, 130, 257, 1000])
+@pytest.mark.parametrize("hidden", [64, 544, 4096, 4128, 5120])
+@pytest.mark.parametrize("tokens", [1, 17])
+def test_router_logits_at_the_edges_of_its_blocks(n, hidden, tokens):
+    """The scores of every output: a correction that is far above all scores names the outputs that are chosen."""
+    from pulse_infer_amd.ops import kernels
+
+    x, w = rnd(tokens, hidden, seed=1).to(torch.bfloat16), (rnd(n, hidden, seed=2) * hidden ** -0.5).to(torch.bfloat16)
+    z = x.to(F64) @ w.to(F64).T
+    # a float32 sum of `hidden` exact products in any order, through a sigmoid of slope 1/4 and a few roundings of its own
+    bound = (hidden + 2) * 2.0 ** -24 * (x.to(F64).abs() @ w.to(F64).abs().T) / 4 + 2.0 ** -21
+    top = 8
+    order = torch.randperm(n, generator=torch.Generator().manual_seed(3)).tolist()
+    for first in range(0, n, top):
+        some = (order + order[:top])[first:first + top]
+        correction = torch.zeros(n)
+        correction[some] = 1024.0
+        idx = torch.full((tokens, top), -5, dtype=torch.int32, device=DEV)
+        weight = torch.full((tokens, top), float("nan"), device=DEV)
+        kernels.moe_router(x.to(DEV), w.to(DEV), correction.to(torch.bfloat16).to(DEV), top, idx, weight, score="sigmoid",
+                           renormalize=False)
+        got, chosen = weight.cpu().to(F64), idx.cpu().long()
+        assert (chosen.sort(1).values == torch.tensor(sorted(some))).all()
+        want = torch.sigmoid(z).gather(1, chosen)
+        assert ((got - want).abs() <= bound.gather(1, chosen)).all()
+        if n > 200 and first >= 8 * top:      # (enough of them to meet every block)
+            break
