@@ -94,6 +94,9 @@ template <> __device__ __forceinline__ ushort4 narrow4<bf16_t>(float4 v) {
     return make_ushort4(f32_to_bf16(v.x), f32_to_bf16(v.y), f32_to_bf16(v.z), f32_to_bf16(v.w));
 }
 
+template <int V>
+struct Ahead { static constexpr int value = V; };
+
 // THREADS threads a row: 256, or 1024 for few rows and for an update in parts (a row then has enough loads in
 // flight to be read at more than the rate of one wavefront's round trips).
 // PARTS: the update may come in parts (kept apart so that the kernel for one update needs no more registers than it did).
@@ -134,30 +137,34 @@ __global__ __launch_bounds__(THREADS) void add_rmsnorm_vec_kernel(float* __restr
             const int i = threadIdx.x + c * THREADS;
             if (i < nvec) v[c] = hrow[i];
         }
-        // The parts of an update (shares of a product's inner dimension) are added in their order; the loads of
-        // four parts are asked for before the first is added, since few rows are bound by the trips to memory.  (A loop
-        // unrolled by eight over a number of parts known only here takes four parts one at a time: 97 rows of 4,096 and 4
-        // to 8 parts 6.6 us, 5.9 so; 32 rows and 4 parts 5.1 either way.)
-        constexpr int AHEAD = 4;
-        for (int p0 = 0; p0 < parts; p0 += AHEAD) {
+        // The parts of an update (shares of a product's inner dimension) are added in their order; the loads of four parts, and of
+        // all that are left behind the fours, are asked for before the first is added, since few rows are bound by the trips to
+        // memory.  97 rows of 4,096, 2 / 3 / 4 / 8 parts: 3.7 / 3.9 / 3.9 / 4.4 us; in a loop unrolled by eight, which takes what
+        // is left behind the eights one at a time, 3.8 / 3.9 / 4.1 / 4.7 (and, of twice the registers, 2,048 rows of 5,120 in 8
+        // parts 88, 77 so); with fours that repeat the last part, 4.0 / 4.1 / 4.1 / 4.9.
+        auto add = [&](int p0, auto ahead) __attribute__((always_inline)) {
+            constexpr int AHEAD = decltype(ahead)::value;
             float4 d[AHEAD][CHUNKS];
 #pragma unroll
             for (int u = 0; u < AHEAD; ++u)
 #pragma unroll
                 for (int c = 0; c < CHUNKS; ++c) {
                     const int i = threadIdx.x + c * THREADS;
-                    if (i < nvec) d[u][c] = widen4(drow[min(p0 + u, parts - 1) * (part_stride / 4) + i]);
+                    if (i < nvec) d[u][c] = widen4(drow[(p0 + u) * (part_stride / 4) + i]);
                 }
 #pragma unroll
-            for (int u = 0; u < AHEAD; ++u) {
-                if (p0 + u >= parts) break;
+            for (int u = 0; u < AHEAD; ++u)
 #pragma unroll
                 for (int c = 0; c < CHUNKS; ++c) {
                     const int i = threadIdx.x + c * THREADS;
                     if (i < nvec) { v[c].x += dscale * d[u][c].x; v[c].y += dscale * d[u][c].y; v[c].z += dscale * d[u][c].z; v[c].w += dscale * d[u][c].w; }
                 }
-            }
-        }
+        };
+        int p = 0;
+        for (; p + 4 <= parts; p += 4) add(p, Ahead<4>());
+        if (parts - p == 3) add(p, Ahead<3>());
+        else if (parts - p == 2) add(p, Ahead<2>());
+        else if (parts - p == 1) add(p, Ahead<1>());
 #pragma unroll
         for (int c = 0; c < CHUNKS; ++c) {
             const int i = threadIdx.x + c * THREADS;

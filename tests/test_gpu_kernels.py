@@ -443,6 +443,24 @@ def test_sampling_at_a_real_vocabulary(k, mode, vocab, chunked):
     assert again.item() == got[5]
 
 
+@pytest.mark.parametrize("parts", [1, 2, 3, 4, 5, 6, 7, 8, 9, 16])
+@pytest.mark.parametrize("hidden", [64, 4100, 8192])
+def test_norm_adds_the_parts_of_an_update_in_their_order(k, parts, hidden):
+    """Groups of four parts and one to three behind them: the residual is the float32 sum part by part, to the bit."""
+    rows, eps = 5, 1e-6
+    gen = torch.Generator().manual_seed(parts)
+    h, delta = torch.randn(rows, hidden, generator=gen), torch.randn(parts, rows, hidden, generator=gen)
+    w = torch.rand(hidden, generator=gen) + 0.5
+    hd, out = h.to(DEV), torch.full((rows, hidden), float("nan"), device=DEV)
+    k.add_rmsnorm(hd, delta.to(DEV), w.to(DEV), eps, out)
+    for p in range(parts):
+        h = h + delta[p]
+    assert torch.equal(hd.cpu(), h)
+    x = h.to(F64)
+    want = x / torch.sqrt((x * x).mean(1, keepdim=True) + eps) * w.to(F64)
+    assert ((out.cpu().to(F64) - want).abs() <= (hidden / 1024 + 16) * 2.0 ** -24 * want.abs()).all()
+
+
 @pytest.mark.parametrize("vocab", [3, 65, 1025, 2049, 40000])
 @pytest.mark.parametrize("ties", [False, True])
 def test_top_p_alone_on_flat_rows_at_the_edges_of_the_passes(k, vocab, ties):
