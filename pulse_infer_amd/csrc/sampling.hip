@@ -87,7 +87,14 @@ __device__ __forceinline__ void sweep(const RowView& row, int first, int end, in
 #pragma unroll
             for (int u = 0; u < AHEAD; ++u) f(i + u * step, x[u]);
         }
-        for (; i < end; i += step) f(i, row.at<MASKED>(i));
+        if (i < end) {        // what is left, asked for together too (past the end: the last entry again, for nobody)
+            float x[AHEAD];
+#pragma unroll
+            for (int u = 0; u < AHEAD; ++u) x[u] = row.at<MASKED>(min(i + u * step, end - 1));
+#pragma unroll
+            for (int u = 0; u < AHEAD; ++u)
+                if (i + u * step < end) f(i + u * step, x[u]);
+        }
     });
 }
 
@@ -476,16 +483,12 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
         if (ranged) {
             for (int b = threadIdx.x; b < HIST_BINS; b += SAMPLE_THREADS) {
                 hist[b] = rest ? rest[b] : 0;
-                hist_w[b] = rest ? __int_as_float(rest[HIST_BINS + b]) : 0.f;
+                if (!by_k) hist_w[b] = rest ? __int_as_float(rest[HIST_BINS + b]) : 0.f;
             }
             __syncthreads();
             if (!rest) {
                 sweep(row, threadIdx.x, vocab, SAMPLE_THREADS, [&](int, float x) {
-                    if (x != -INFINITY) {
-                        const int b = bin_of(x);
-                        atomicAdd(&hist[b], 1);
-                        if (!by_k) add_in_group(&hist_w[b], expf((x - best) * inv_t));
-                    }
+                    if (x != -INFINITY) atomicAdd(&hist[bin_of(x)], 1);
                 });
                 __syncthreads();
             }
@@ -508,7 +511,7 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
             }
         }
         bool may_hold = true;    // whether the list can hold top_p of the row (its mass is known to a thousandth at least)
-        if (!by_k && edge >= 0) {
+        if (rest && !by_k && edge >= 0) {
             float above = 0.f;
             for (int b = threadIdx.x; b <= edge; b += SAMPLE_THREADS) above += hist_w[b];
             may_hold = block_sum_f(above, sf) >= 0.999f * p * whole;
@@ -591,8 +594,16 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
             // Top-p alone: the histogram's masses say near which token the sum reaches `want`; the tokens of that bin and
             // its neighbours are ranked, and M is summed, in its own order, for the five (or fifteen) round that place side by side.
             // (A search for the threshold's bits, four a pass, takes eight such passes.  32 rows of 151,936, this kernel:
-            // 661 us with the search, 377 with this, 141 with the mass and the histogram made by the kernels in front.)
+            // 661 us with the search, 377 with this, 141 with the mass and the histogram made by the kernels in front.  The masses
+            // are summed for the rows that come here alone: every row's cost those whose list holds top_p 1.7 to 2.5 times.)
             want = p * whole;
+            if (!rest) {
+                sweep(row, threadIdx.x, vocab, SAMPLE_THREADS, [&](int, float x) {
+                    if (x != -INFINITY)
+                        add_in_group(&hist_w[min(HIST_BINS - 1, static_cast<int>((best - x) * bin_scale))], expf((x - best) * inv_t));
+                });
+                __syncthreads();
+            }
             found = nucleus_edge(row, want, best, inv_t, bin_scale, hist, hist_w, sf, si, list_i, list_x, cand, &nearest, thr);
         } else {
             float mass = 0.f;
@@ -993,7 +1004,7 @@ __global__ __launch_bounds__(PULSE_WAVE) void chunked_choose_kernel(
         const int n = first + __shfl(pre1, PULSE_WAVE - 1, PULSE_WAVE);
         if (k > chunks || chunks > 2 * PULSE_WAVE || __ballot(over) != 0ull || n > LIST_CAP || n < k || n == 0) {
             if (lane == 0) done[r] = 0;   // not a row for these kernels: sample_kernel takes it
-            clear_histogram(left + static_cast<int64_t>(r) * REST_WORDS, lane);
+            if (left) clear_histogram(left + static_cast<int64_t>(r) * REST_WORDS, lane);
             return;
         }
         float whole = 0.f;   // without top-k: the mass of the whole row, chunk masses in chunk order
@@ -1016,7 +1027,7 @@ __global__ __launch_bounds__(PULSE_WAVE) void chunked_choose_kernel(
             if (enough) out[r] = token;
             done[r] = enough ? 1 : 0;
         }
-        if (!__shfl(enough ? 1 : 0, 0, PULSE_WAVE)) clear_histogram(left + static_cast<int64_t>(r) * REST_WORDS, lane);
+        if (left && !__shfl(enough ? 1 : 0, 0, PULSE_WAVE)) clear_histogram(left + static_cast<int64_t>(r) * REST_WORDS, lane);
         return;
     }
     // a draw from the whole vocabulary: the chunk in which it falls, chunk masses in chunk order
@@ -1242,8 +1253,12 @@ extern "C" int pulse_sample_chunked(const float* logits, int rows, int vocab, in
     const int chunks = pulse_sample_chunks(vocab);
     // behind the segments: what is made of the rows that are left, and the chunks' smallest numbers
     const bool leaves = temperature && (top_k || top_p);    // (without them every row is done)
-    int* rest = leaves ? seg_i + static_cast<int64_t>(rows) * chunks * TOPK_SEGMENT : nullptr;
-    float* part_min = leaves ? reinterpret_cast<float*>(rest + static_cast<int64_t>(rows) * REST_WORDS) : nullptr;
+    // They are made while a workgroup a row leaves most of the chip idle and its passes are long: 32,000 values, flat rows
+    // under top-p and others, 16 rows 103 and 80 us with them (272 and 87 without any of it), 64 rows 128 and 108, 159 and
+    // 92 without; 151,936 values, 64 rows 427 and 291 (947 and 776).
+    const bool prepare = leaves && vocab >= 1024 * static_cast<int64_t>(rows);
+    int* rest = prepare ? seg_i + static_cast<int64_t>(rows) * chunks * TOPK_SEGMENT : nullptr;
+    float* part_min = prepare ? reinterpret_cast<float*>(rest + static_cast<int64_t>(rows) * REST_WORDS) : nullptr;
     hipLaunchKernelGGL(simple_max_kernel, dim3(chunks, rows), dim3(SIMPLE_THREADS), 0, stream, logits, vocab, row_stride,
                        penalty, seen_row, seen_masks, banned, mask_words, part_max, part_idx, part_min);
     PULSE_LAUNCH_CHECK("sample_chunked (maxima)");
@@ -1263,11 +1278,13 @@ extern "C" int pulse_sample_chunked(const float* logits, int rows, int vocab, in
                        temperature, top_k, top_p, uniform, penalty, seen_row, seen_masks, banned, mask_words, part_max,
                        part_idx, part_mass, seg_i, seg_x, seg_n, chunks, out, done, rest);
     PULSE_LAUNCH_CHECK("sample_chunked (choice)");
-    if (leaves) {
+    if (prepare) {
         hipLaunchKernelGGL(rest_kernel, dim3(MASS_GROUPS + REST_GROUPS, rows), dim3(SIMPLE_THREADS), 0, stream, logits, vocab,
                            row_stride, temperature, top_k, penalty, seen_row, seen_masks, banned, mask_words, part_max,
                            part_min, chunks, static_cast<const int*>(done), rest);
         PULSE_LAUNCH_CHECK("sample_chunked (what is left)");
+    }
+    if (leaves) {
         hipLaunchKernelGGL(sample_kernel, dim3(rows), dim3(SAMPLE_THREADS), 0, stream, logits, vocab, row_stride,
                            temperature, top_k, top_p, uniform, penalty, seen_row, seen_masks, banned, mask_words, out,
                            static_cast<const int*>(done), part_max, part_idx, chunks, static_cast<const int*>(rest));
