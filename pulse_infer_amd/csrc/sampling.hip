@@ -1231,17 +1231,19 @@ extern "C" int pulse_sample(const float* logits, int rows, int vocab, int64_t ro
 // equal values around the k-th largest, a distribution too flat for top-p alone) by the kernel of pulse_sample behind
 // them, which skips the rows that are done.  What a row's choice is does not depend on the
 // other rows.  Scratch, with chunks = pulse_sample_chunks(vocab): part_max, part_mass (float32), part_idx, seg_n
-// (int32) of rows * chunks entries; seg_x (float32) of rows * chunks * pulse_sample_segment() entries, seg_i (int32) of
-// rows * (pulse_sample_rest() + chunks) more; done (int32) of rows entries.
+// (int32) of rows * chunks entries; seg_i (int32), seg_x (float32) of rows * chunks * pulse_sample_segment()
+// entries; done (int32) of rows entries; and, optional (null: the rows that are left are gone over by their own workgroups
+// alone, with the same choices), rest (int32) of rows * (pulse_sample_rest() + chunks) entries.
 extern "C" int pulse_sample_rest() { return REST_WORDS; }
 extern "C" int pulse_sample_chunks(int vocab) { return (vocab + SIMPLE_CHUNK - 1) / SIMPLE_CHUNK; }
 extern "C" int pulse_sample_segment() { return TOPK_SEGMENT; }
 
-extern "C" int pulse_sample_chunked(const float* logits, int rows, int vocab, int64_t row_stride, const float* temperature,
+extern "C" int pulse_sample_chunked_rest(const float* logits, int rows, int vocab, int64_t row_stride, const float* temperature,
                                     const int* top_k, const float* top_p, const float* uniform, const float* penalty,
                                     const int* seen_row, const uint32_t* seen_masks, const uint32_t* banned,
                                     int mask_words, float* part_max, int* part_idx, float* part_mass, int* seg_i,
-                                    float* seg_x, int* seg_n, int* done, int* out, hipStream_t stream) {
+                                    float* seg_x, int* seg_n, int* done, int* rest, int* out,
+                                         hipStream_t stream) {
     PULSE_REQUIRE(rows >= 0 && vocab > 0 && row_stride >= vocab, "sample_chunked: bad sizes rows=%d V=%d", rows, vocab);
     PULSE_REQUIRE(rows < 65536, "sample_chunked: at most 65535 rows");
     PULSE_REQUIRE(logits && out && part_max && part_idx && part_mass && seg_i && seg_x && seg_n && done,
@@ -1251,13 +1253,13 @@ extern "C" int pulse_sample_chunked(const float* logits, int rows, int vocab, in
                   "vocabulary has %d", mask_words * 32, vocab);
     if (rows == 0) return 0;
     const int chunks = pulse_sample_chunks(vocab);
-    // behind the segments: what is made of the rows that are left, and the chunks' smallest numbers
     const bool leaves = temperature && (top_k || top_p);    // (without them every row is done)
     // They are made while a workgroup a row leaves most of the chip idle and its passes are long: 32,000 values, flat rows
     // under top-p and others, 16 rows 103 and 80 us with them (272 and 87 without any of it), 64 rows 128 and 108, 159 and
     // 92 without; 151,936 values, 64 rows 427 and 291 (947 and 776).
-    const bool prepare = leaves && vocab >= 1024 * static_cast<int64_t>(rows);
-    int* rest = prepare ? seg_i + static_cast<int64_t>(rows) * chunks * TOPK_SEGMENT : nullptr;
+    const bool prepare = rest && leaves && vocab >= 1024 * static_cast<int64_t>(rows);
+    if (!prepare) rest = nullptr;
+    // (behind what is made of the rows: the chunks' smallest numbers)
     float* part_min = prepare ? reinterpret_cast<float*>(rest + static_cast<int64_t>(rows) * REST_WORDS) : nullptr;
     hipLaunchKernelGGL(simple_max_kernel, dim3(chunks, rows), dim3(SIMPLE_THREADS), 0, stream, logits, vocab, row_stride,
                        penalty, seen_row, seen_masks, banned, mask_words, part_max, part_idx, part_min);
@@ -1291,6 +1293,16 @@ extern "C" int pulse_sample_chunked(const float* logits, int rows, int vocab, in
         PULSE_LAUNCH_CHECK("sample_chunked (the rest)");
     }
     return 0;
+}
+
+extern "C" int pulse_sample_chunked(const float* logits, int rows, int vocab, int64_t row_stride, const float* temperature,
+                                    const int* top_k, const float* top_p, const float* uniform, const float* penalty,
+                                    const int* seen_row, const uint32_t* seen_masks, const uint32_t* banned,
+                                    int mask_words, float* part_max, int* part_idx, float* part_mass, int* seg_i,
+                                    float* seg_x, int* seg_n, int* done, int* out, hipStream_t stream) {
+    return pulse_sample_chunked_rest(logits, rows, vocab, row_stride, temperature, top_k, top_p, uniform, penalty, seen_row,
+                                     seen_masks, banned, mask_words, part_max, part_idx, part_mass, seg_i, seg_x, seg_n, done,
+                                     nullptr, out, stream);
 }
 
 // Set the bit of tokens[i] in the mask row rows[i] (the per-request "seen" set of the presence penalty).

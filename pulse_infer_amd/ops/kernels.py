@@ -1047,8 +1047,8 @@ def sample_chunked_scratch(rows: int, vocab: int, device) -> dict:
     f32 = lambda n: torch.empty(n, dtype=torch.float32, device=device)
     i32 = lambda n: torch.empty(n, dtype=torch.int32, device=device)
     return {"part_max": f32(rows * per_row), "part_idx": i32(rows * per_row), "part_mass": f32(rows * per_row),
-            "seg_n": i32(rows * per_row), "done": i32(rows), "seg_i": i32(rows * (per_row * (SAMPLE_SEGMENT + 1) + SAMPLE_REST)),
-            "seg_x": f32(rows * per_row * SAMPLE_SEGMENT)}
+            "seg_n": i32(rows * per_row), "done": i32(rows), "seg_i": i32(rows * per_row * SAMPLE_SEGMENT),
+            "seg_x": f32(rows * per_row * SAMPLE_SEGMENT), "rest": i32(rows * (per_row + SAMPLE_REST))}
 
 
 def sample_chunked(logits: torch.Tensor, out: torch.Tensor, scratch: dict, temperature: Optional[torch.Tensor] = None,
@@ -1060,10 +1060,11 @@ def sample_chunked(logits: torch.Tensor, out: torch.Tensor, scratch: dict, tempe
     that draw from the whole vocabulary and rows with top-k (k at most the number of chunks) are chosen from what the
     chunks leave; rows with top-p alone, and what does not fit, go through the kernel of ``sample`` behind them,
     which one more has prepared.
-    Which way a row goes depends on the row alone.  ``scratch`` as ``sample_chunked_scratch`` makes it."""
+    Which way a row goes depends on the row alone.  ``scratch`` as ``sample_chunked_scratch`` makes it; without its
+    ``rest`` that one does not run, and the choices are the same."""
     names = ("part_max", "part_idx", "part_mass", "seg_i", "seg_x", "seg_n", "done")
     _gpu("sample_chunked", logits, out, temperature, top_k, top_p, uniform, penalty, seen_row, seen_masks, banned,
-         *(scratch[n] for n in names))
+         *(scratch[n] for n in names), scratch.get("rest"))
     _need(logits.dim() == 2 and logits.dtype == torch.float32 and logits.stride(1) == 1,
           "sample_chunked: logits must be float32 [R, V]")
     rows, vocab = logits.shape
@@ -1076,9 +1077,11 @@ def sample_chunked(logits: torch.Tensor, out: torch.Tensor, scratch: dict, tempe
     per_row = sample_chunks(vocab)
     for name, dt, need in (("part_max", torch.float32, rows * per_row), ("part_idx", torch.int32, rows * per_row),
                            ("part_mass", torch.float32, rows * per_row), ("seg_n", torch.int32, rows * per_row),
-                           ("done", torch.int32, rows),
-                           ("seg_i", torch.int32, rows * (per_row * (SAMPLE_SEGMENT + 1) + SAMPLE_REST)),
-                           ("seg_x", torch.float32, rows * per_row * SAMPLE_SEGMENT)):
+                           ("done", torch.int32, rows), ("seg_i", torch.int32, rows * per_row * SAMPLE_SEGMENT),
+                           ("seg_x", torch.float32, rows * per_row * SAMPLE_SEGMENT),
+                           ("rest", torch.int32, rows * (per_row + SAMPLE_REST))):
+        if name not in scratch and name == "rest":
+            continue
         t = scratch[name]
         _need(t.dtype == dt and t.is_contiguous() and t.numel() >= need, f"sample_chunked: {name} must hold {need} {dt}")
     words = 0
@@ -1088,11 +1091,11 @@ def sample_chunked(logits: torch.Tensor, out: torch.Tensor, scratch: dict, tempe
             w = t.shape[-1]
             _need(words in (0, w), "sample_chunked: masks differ in width")
             words = w
-    call("pulse_sample_chunked", _ptr(logits), _i32(rows), _i32(vocab), _i64(logits.stride(0) if rows > 1 else vocab),
+    call("pulse_sample_chunked_rest", _ptr(logits), _i32(rows), _i32(vocab), _i64(logits.stride(0) if rows > 1 else vocab),
          _ptr(temperature), _ptr(top_k), _ptr(top_p), _ptr(uniform), _ptr(penalty), _ptr(seen_row), _ptr(seen_masks),
          _ptr(banned), _i32(words), _ptr(scratch["part_max"]), _ptr(scratch["part_idx"]), _ptr(scratch["part_mass"]),
          _ptr(scratch["seg_i"]), _ptr(scratch["seg_x"]), _ptr(scratch["seg_n"]), _ptr(scratch["done"]),
-         _ptr(out), _stream())
+         _ptr(scratch.get("rest")), _ptr(out), _stream())
 
 
 def argmax(logits: torch.Tensor, out: torch.Tensor, part_val: torch.Tensor, part_idx: torch.Tensor) -> None:
