@@ -297,19 +297,9 @@ extern "C" int pulse_gemm_mid_takes(int M, int N, int K, int splits) {
 // products of the shares of K, to be added up by the consumer in split order.  swiglu != 0 (mode 0, splits 1): W holds
 // gate and up rows interleaved in slabs of 16 (gate slab, up slab, ...), N counts both, C is bfloat16 [M, N / 2] =
 // silu(gate) * up.
-// waves: wavefronts (of 16 weight rows) a workgroup, 2, 3, 4, 6 or 10 (4 or 6 above 64 rows); 0 lets the entry point choose;
-// -1: the product in stages of gemm_stages.hip, which takes other sizes (pulse_gemm_stages_takes) and knows silu only.
-extern "C" int pulse_gemm_stages(const void* X, int64_t ldx, const void* W, int64_t ldw, void* C, int64_t ldc, int M, int N,
-                                 int K, int mode, int splits, int64_t part_stride, hipStream_t stream);
-
+// waves: wavefronts (of 16 weight rows) a workgroup, 2, 3, 4, 6 or 10 (4 or 6 above 64 rows); 0 lets the entry point choose.
 extern "C" int pulse_gemm_mid(const void* X, int64_t ldx, const void* W, int64_t ldw, void* C, int64_t ldc, int M, int N,
                               int K, int mode, int swiglu, int splits, int waves, hipStream_t stream) {
-    if (waves == -1) {
-        PULSE_REQUIRE((mode == MID_BF16 || mode == MID_PARTS) && (swiglu == 0 || (swiglu == 1 && mode == MID_BF16)),
-                      "gemm_mid: in stages, a bfloat16 result, with silu or without, or float32 shares (mode %d, swiglu %d)", mode, swiglu);
-        return pulse_gemm_stages(X, ldx, W, ldw, C, ldc, M, N, K, swiglu ? 1 : mode == MID_PARTS ? 2 : 0, splits,
-                                 splits > 1 ? static_cast<int64_t>(M) * ldc : 0, stream);
-    }
     PULSE_REQUIRE(pulse_gemm_mid_takes(M, N, K, splits), "gemm_mid: M=%d (1..192) N=%d K=%d in %d shares (multiples of %d)",
                   M, N, K, splits, KC_MIN);
     PULSE_REQUIRE(X && W && C, "gemm_mid: null pointer");

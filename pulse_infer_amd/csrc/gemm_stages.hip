@@ -145,24 +145,23 @@ void launch(StageArgs a, hipStream_t stream) {
 }
 
 // weight rows and rows of X a tile (the kernels below, in this order)
-constexpr int SHAPES[][2] = {{32, 128}, {64, 64}, {64, 128}, {96, 128}, {128, 64}, {128, 128}, {192, 128}, {256, 128},
+constexpr int SHAPES[][2] = {{64, 64}, {64, 128}, {96, 128}, {128, 64}, {128, 128}, {192, 128}, {256, 128},
                                {192, 192}, {192, 256}, {256, 192}, {256, 256}};
 constexpr int NUM_SHAPES = sizeof(SHAPES) / sizeof(SHAPES[0]);
 
 template <int MODE>
 void launch_shape(int shape, const StageArgs& a, hipStream_t s) {
     switch (shape) {
-        case 0: return launch<MODE, 32, 128, 1, 4, 4>(a, s);
-        case 1: return launch<MODE, 64, 64, 2, 2, 6>(a, s);
-        case 2: return launch<MODE, 64, 128, 2, 2, 6>(a, s);
-        case 3: return launch<MODE, 96, 128, 1, 4, 5>(a, s);
-        case 4: return launch<MODE, 128, 64, 4, 1, 3>(a, s);
-        case 5: return launch<MODE, 128, 128, 2, 2, 4>(a, s);
-        case 6: return launch<MODE, 192, 128, 2, 2, 3>(a, s);
-        case 7: return launch<MODE, 256, 128, 2, 2, 3>(a, s);
-        case 8: return launch<MODE, 192, 192, 2, 2, 3, 3, false>(a, s);
-        case 9: return launch<MODE, 192, 256, 2, 2, 3, 2, false>(a, s);
-        case 10: return launch<MODE, 256, 192, 2, 2, 3, 2, false>(a, s);
+        case 0: return launch<MODE, 64, 64, 2, 2, 6>(a, s);
+        case 1: return launch<MODE, 64, 128, 2, 2, 6>(a, s);
+        case 2: return launch<MODE, 96, 128, 1, 4, 5>(a, s);
+        case 3: return launch<MODE, 128, 64, 4, 1, 3>(a, s);
+        case 4: return launch<MODE, 128, 128, 2, 2, 4>(a, s);
+        case 5: return launch<MODE, 192, 128, 2, 2, 3>(a, s);
+        case 6: return launch<MODE, 256, 128, 2, 2, 3>(a, s);
+        case 7: return launch<MODE, 192, 192, 2, 2, 3, 3, false>(a, s);
+        case 8: return launch<MODE, 192, 256, 2, 2, 3, 2, false>(a, s);
+        case 9: return launch<MODE, 256, 192, 2, 2, 3, 2, false>(a, s);
         default: return launch<MODE, 256, 256, 2, 2, 3, 2, false>(a, s);
     }
 }
@@ -211,13 +210,20 @@ extern "C" int pulse_gemm_stages_takes(int M, int N, int K, int mode, int splits
     if (K % (64 * splits)) return 0;
     const int n_step = mode == OUT_SWIGLU ? 32 : (mode == OUT_BF16 ? 8 : 4);
     if (N % n_step) return 0;
-    return static_cast<int64_t>((M + 63) / 64) * ((N + 31) / 32) * splits <= (1 << 28);
+    return static_cast<int64_t>((M + 63) / 64) * ((N + 63) / 64) * splits <= (1 << 27);
 }
 
 // How many shares of K float32 results are best made in (0: a shape that the product does not take).
 extern "C" int pulse_gemm_stages_shares(int M, int N, int K) {
     if (!pulse_gemm_stages_takes(M, N, K, OUT_F32, 1)) return 0;
     return plan_for(M, N, K, 0).splits;
+}
+
+// The tile of a product in so many shares: weight rows * 1,024 + rows of X (0: a shape that the product does not take).
+extern "C" int pulse_gemm_stages_tile(int M, int N, int K, int splits) {
+    if (!pulse_gemm_stages_takes(M, N, K, OUT_F32, splits) && !(splits == 1 && pulse_gemm_stages_takes(M, N, K, OUT_BF16, 1))) return 0;
+    const int shape = plan_for(M, N, K, splits).shape;
+    return SHAPES[shape][0] * 1024 + SHAPES[shape][1];
 }
 
 // The estimated time of bfloat16 results in nanoseconds, at most 2 s (0: a shape that the product

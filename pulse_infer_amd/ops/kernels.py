@@ -457,6 +457,14 @@ def gemm_stages_shares(m: int, n: int, k: int) -> int:
 
 
 @functools.lru_cache(maxsize=4096)
+def gemm_stages_tile(m: int, n: int, k: int, shares: int = 1) -> tuple:
+    """(weight rows, rows of x) of the tile that ``gemm_stages`` takes (a function of the sizes alone); (0, 0): it does not
+    take the shape."""
+    code = int(library.load().pulse_gemm_stages_tile(_i32(m), _i32(n), _i32(k), _i32(shares)))
+    return code // 1024, code % 1024
+
+
+@functools.lru_cache(maxsize=4096)
 def gemm_stages_time(m: int, n: int, k: int) -> int:
     """What ``gemm_stages`` is estimated to take for bfloat16 results, nanoseconds (a function of the sizes alone)."""
     return int(library.load().pulse_gemm_stages_time(_i32(m), _i32(n), _i32(k)))
@@ -480,16 +488,16 @@ def gemm_stages(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, swiglu: boo
         splits = out.shape[0]
         _need(not swiglu and out.dim() == 3 and tuple(out.shape[1:]) == (m, n) and out.is_contiguous() and n % 4 == 0
               and k % (64 * splits) == 0, f"gemm_stages: float32 results go to contiguous [shares, {m}, {n}]")
-        mode, ldc = 1, n
+        mode, ldc, part_stride = 2, n, m * n
     else:
         cols = n // 2 if swiglu else n
         _need(gemm_stages_takes(m, n, k, swiglu) and out.dtype == torch.bfloat16 and out.dim() == 2
               and tuple(out.shape) == (m, cols) and out.stride(1) == 1,
               f"gemm_stages: M={m} N={n} K={k} is not a shape it takes, or out is not bfloat16 [{m}, {cols}]")
-        mode, ldc, splits = 0, (out.stride(0) if m > 1 else cols), 1
-    call("pulse_gemm_mid", _ptr(a), _i64(a.stride(0) if m > 1 else k), _ptr(w), _i64(w.stride(0) if n > 1 else k),
-         _ptr(out), _i64(ldc), _i32(m), _i32(n), _i32(k), _i32(mode), _i32(1 if swiglu else 0), _i32(splits),
-         _i32(-1), _stream(), label=f"N={n} K={k}")
+        mode, ldc, splits, part_stride = 1 if swiglu else 0, (out.stride(0) if m > 1 else cols), 1, 0
+    call("pulse_gemm_stages", _ptr(a), _i64(a.stride(0) if m > 1 else k), _ptr(w), _i64(w.stride(0) if n > 1 else k),
+         _ptr(out), _i64(ldc), _i32(m), _i32(n), _i32(k), _i32(mode), _i32(splits), _i64(part_stride), _stream(),
+         label=f"N={n} K={k}")
 
 
 MID_MAX_ROWS = 192

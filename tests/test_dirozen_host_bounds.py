@@ -122,6 +122,13 @@ def check(name, args):
             need(room(c) >= (splits - 1) * m * val(ldc) + (m - 1) * val(ldc) + (n // 2 if swiglu else n), "out")
         else:
             need(room(c) >= (m - 1) * val(ldc) + n, "out")
+    elif name == "pulse_gemm_stages":
+        a, ldx, w, ldw, c, ldc, m, n, k, mode, splits, part_stride, _ = args
+        m, n, k, mode, splits = (val(v) for v in (m, n, k, mode, splits))
+        need(room(a) >= (m - 1) * val(ldx) + k and room(w) >= (n - 1) * val(ldw) + k, "operands")
+        need(k % (64 * splits) == 0 and (splits == 1 or mode == 2), "shares")
+        need(room(c) >= (splits - 1) * val(part_stride) + (m - 1) * val(ldc) + (n // 2 if mode == 1 else n), "out")
+        need(splits == 1 or val(part_stride) >= (m - 1) * val(ldc) + n, "shares that overlap")
     elif name == "pulse_swiglu":
         gu, out, _, tokens, inter, _, _, _ = args
         need(room(gu) >= val(tokens) * 2 * val(inter) and room(out) >= val(tokens) * val(inter), "operands")
@@ -210,3 +217,23 @@ def test_every_entry_point_stays_inside_its_tensors(checked_kernels, seed):
                 runner.free_request(k)
         runner.cache.check()
     assert {"pulse_qk_rope_kv", "pulse_add_rmsnorm", "pulse_embed_gather"} <= set(checked_kernels)
+
+
+@pytest.mark.parametrize("rows", [65, 130, 255, 300, 512])
+def test_products_in_stages_stay_inside_their_tensors(checked_kernels, rows):
+    """The product for some tens to some hundreds of rows has an entry point of its own: plain, with SwiGLU inside, and in
+    shares that the next norm adds up."""
+    from pulse_infer_amd.ops import kernels
+    from pulse_infer_amd.parts.base import Workspace
+
+    x, w = torch.zeros(rows, 2048, dtype=torch.bfloat16), torch.zeros(4096, 2048, dtype=torch.bfloat16)
+    wide = torch.zeros(rows, 4096 + 24, dtype=torch.bfloat16)[:, :4096]
+    kernels.gemm_stages(x, w, wide)
+    kernels.gemm_stages(x, w, torch.zeros(rows, 2048, dtype=torch.bfloat16), swiglu=True)
+    for shares in {1, kernels.gemm_stages_shares(rows, 4096, 2048), 32}:
+        kernels.gemm_stages(x, w, Workspace(torch.device("cpu")).buffer("parts", shares * rows, 4096, torch.float32).view(shares, rows, 4096))
+    assert checked_kernels and set(checked_kernels) == {"pulse_gemm_stages"}
+    for n, k, splits in ((4096, 2048, 1), (4096, 2048, 4), (24576, 4096, 1)):
+        tile = kernels.gemm_stages_tile(rows, n, k, splits)
+        assert tile[0] in (64, 96, 128, 192, 256) and tile[1] in (64, 128, 192, 256)
+    assert kernels.gemm_stages_tile(rows, 4096, 96) == (0, 0)
