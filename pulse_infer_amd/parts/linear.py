@@ -30,7 +30,8 @@ from .base import LazyNorm, RowStats, Workspace
 # Which products of many rows (256 and more) run as this package's instead of the library's: "stages", the product in
 # stages where it is the faster one (``takes_stages``); or the tiled product, "swiglu": for gate and up with SwiGLU inside,
 # which saves the pass over twice the feed-forward's width (the others as with "stages"), "all": for every product of
-# bfloat16 (a step then makes no library call); "none": no product of more than 256 rows.  PULSE_OWN_PRODUCTS sets it.
+# bfloat16 (a step then makes no library call); "none": none of them.  (Products of fewer rows are not its business: 65 to 255
+# of them run in stages whatever it says, where they did not go to the library by rules of their own before.)  PULSE_OWN_PRODUCTS sets it.
 # Measured: a prompt of 509 tokens of the 8B shape 9.2 ms with "stages", 9.6 with "none".  Through the serving loop, a prompt of
 # 2,048 tokens 73.9K tokens/s with "none", 72.9K with "swiglu", 71.6K with "all" (alone and with the chip warm, gate+up
 # with SwiGLU inside takes 310 us against the library's 328 + 30 for the pass; between the other kernels of a step the
@@ -264,7 +265,7 @@ class Linear:
     # against 53), updates in shares up to 512 rows unless the library's shares fill half the units (4,096 x 4,096 at 512 rows 25
     # against 31, 2,560 x 9,728 at 357 27 against 41; 4,096 x 12,288 at 357 and 509 rows takes as long either way, 45 and 60,
     # but in eight shares at 357, which cost the norm behind 2 more).  Small products stay where they are.
-    STAGE_ROWS = (65, 256)              # any of these
+    STAGE_ROWS = (65, 256)              # any of these (from ``TILE_MIN_ROWS`` on if ``OWN_MANY_ROWS`` leaves them to it)
     STAGE_ROWS_SWIGLU = (768, 1536)
     STAGE_SWIGLU_RATE = 1100            # flops a nanosecond
     STAGE_ROWS_SHARES = 512
@@ -279,10 +280,10 @@ class Linear:
         if not (self.library and x.dtype == torch.bfloat16 and self.STAGE_ROWS[0] <= rows <= self.STAGE_ROWS_SWIGLU[1]
                 and n * k >= self.STAGE_MIN_WEIGHT and self.operands_ok(x) and kernels.gemm_stages_takes(rows, n, k, swiglu)):
             return False
+        if rows >= self.TILE_MIN_ROWS and (OWN_MANY_ROWS == "none" or self.takes_tiles(x, w, swiglu)):
+            return False
         if rows <= self.STAGE_ROWS[1]:
             return True
-        if OWN_MANY_ROWS == "none" or self.takes_tiles(x, w, swiglu):
-            return False
         if not swiglu:
             return n <= 32 * compute_units() and rows <= self.STAGE_ROWS_NARROW
         return ((n <= 192 * compute_units() and rows <= self.STAGE_ROWS_SWIGLU[0])
@@ -295,16 +296,16 @@ class Linear:
         if not (self.library and x.dtype == torch.bfloat16 and self.STAGE_ROWS[0] <= rows <= self.STAGE_ROWS_SHARES
                 and n * k >= self.STAGE_MIN_WEIGHT and self.operands_ok(x)) or n % 4 or k % 64:
             return 0
+        if rows >= self.TILE_MIN_ROWS and (OWN_MANY_ROWS == "none" or self.tile_shares_for(x)):
+            return 0
         if rows > self.STAGE_ROWS[1]:
-            if OWN_MANY_ROWS == "none" or self.tile_shares_for(x):
-                return 0
             tile = self.LIBRARY_TILE
             tiles = ((rows + tile - 1) // tile) * ((n + tile - 1) // tile) * self.library_shares_for(x)
             if 2 * tiles >= compute_units():
                 return 0
         return kernels.gemm_stages_shares(rows, n, k)
 
-    TILE_MIN_ROWS = 256          # from here on the tiled product for many rows is a candidate
+    TILE_MIN_ROWS = 256          # from here on the tiled product for many rows is a candidate, and ``OWN_MANY_ROWS`` decides
 
     def takes_tiles(self, x: torch.Tensor, w: Optional[torch.Tensor] = None, swiglu: bool = False) -> bool:
         """Whether a product of this many rows runs as this package's tiled product (``OWN_MANY_ROWS`` allowing)."""

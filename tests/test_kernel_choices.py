@@ -133,3 +133,34 @@ def test_own_products_share_out_their_inner_dimension_evenly(units):
                 groups = -(-n // (16 * waves))
                 fullest = -(-groups // units) * 16 * waves
                 assert fullest * units < 1.5 * n + 1.5 * units * (m // 2)
+
+
+def test_which_products_of_many_rows_the_option_decides(units, monkeypatch):
+    """Up to 255 rows the product in stages whatever the option says; from 256 on as it says: none of this package's, the tiled
+    product for gate and up or for all, the product in stages where it takes them."""
+    import torch
+    from pulse_infer_amd.parts import linear
+    from pulse_infer_amd.parts.linear import Linear
+
+    gate_up = Linear(torch.empty(24576, 4096, dtype=torch.bfloat16, device="meta"), "bfloat16")
+    o = Linear(torch.empty(4096, 4096, dtype=torch.bfloat16, device="meta"), "bfloat16")
+    rows = lambda m: torch.empty(m, 4096, dtype=torch.bfloat16, device="meta")
+    for policy in ("none", "stages", "swiglu", "all"):
+        monkeypatch.setattr(linear, "OWN_MANY_ROWS", policy)
+        for m in (64, 65, 255):
+            assert gate_up.takes_stages(rows(m), swiglu=True) == (m >= 65) and not gate_up.takes_tiles(rows(m), swiglu=True)
+            assert bool(o.stage_shares_for(rows(m))) == (m >= 65)
+        for m in (256, 257, 512, 513, 768, 769, 1024, 1536, 1537):
+            assert gate_up.takes_tiles(rows(m), swiglu=True) == (policy in ("swiglu", "all"))
+            assert o.takes_tiles(rows(m)) == (policy == "all") == bool(o.tile_shares_for(rows(m)))
+            if policy != "stages":
+                assert not gate_up.takes_stages(rows(m), swiglu=True)
+            if policy in ("none", "all"):
+                assert not o.takes_stages(rows(m)) and not o.stage_shares_for(rows(m))
+            if m > Linear.STAGE_ROWS_SHARES:
+                assert not o.stage_shares_for(rows(m))
+            if m > Linear.STAGE_ROWS_SWIGLU[1]:
+                assert not gate_up.takes_stages(rows(m), swiglu=True)
+    monkeypatch.setattr(linear, "OWN_MANY_ROWS", "stages")
+    for m in (256, 257, 512, 768):
+        assert gate_up.takes_stages(rows(m), swiglu=True) or (24576 > 192 * units and m > 256)
