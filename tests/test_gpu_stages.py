@@ -79,3 +79,19 @@ def test_product_in_stages_applies_silu_where_its_exponential_is_largest():
     # the exponential of a number good to 2^-24 of up to 89 (2^-17), a reciprocal, one rounding to bfloat16
     bound = (2.0 ** -8 + 2.0 ** -16) * want.abs() + 1024.0 * 2.0 ** -149
     assert ((act.cpu().to(F64) - want).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("n,k", [(4096, 1024), (1028, 4096), (2048, 2048)])
+def test_an_update_in_stages_does_not_depend_on_the_rows_beside_it(n, k):
+    """65 to 192 rows: the same shares, every tile walks a share in the same order; to the bit."""
+    from pulse_infer_amd.parts.base import Workspace
+    from pulse_infer_amd.parts.linear import Linear
+
+    lin = Linear((rnd(n, k, seed=3) * k ** -0.5).to(torch.bfloat16).to(DEV), "bfloat16")
+    x = rnd(192, k, seed=4).to(torch.bfloat16).to(DEV)
+    ws, h = Workspace(torch.device(DEV)), torch.zeros(192, n, device=DEV)
+    scratch = torch.empty(192, n, dtype=torch.bfloat16, device=DEV)
+    whole = lin.add_into(x, h, scratch, ws).clone()
+    assert whole.dim() == 3
+    for m in (65, 97, 128, 160, 191):
+        assert torch.equal(lin.add_into(x[:m], h[:m], scratch[:m], ws), whole[:, :m])

@@ -164,3 +164,19 @@ def test_which_products_of_many_rows_the_option_decides(units, monkeypatch):
     monkeypatch.setattr(linear, "OWN_MANY_ROWS", "stages")
     for m in (256, 257, 512, 768):
         assert gate_up.takes_stages(rows(m), swiglu=True) or (24576 > 192 * units and m > 256)
+
+
+def test_shares_of_an_update_depend_on_the_weight_alone_up_to_192_rows(units):
+    """17 to 64 rows (shared out over workgroups) and 65 to 192 (in stages): one cut each."""
+    import torch
+    from pulse_infer_amd.parts.linear import Linear
+
+    for n, k in ((4096, 4096), (4096, 12288), (2560, 9728), (5120, 17408), (2048, 8192), (7168, 2048), (1000, 8192)):
+        lin = Linear(torch.empty(n, k, dtype=torch.bfloat16, device="meta"), "bfloat16")
+        rows = lambda m: torch.empty(m, k, dtype=torch.bfloat16, device="meta")
+        assert len({lin.shares_and_waves_for(rows(m)) for m in (17, 33, 64, 100, 192)}) == 1
+        cuts = {lin.stage_shares_for(rows(m)) for m in range(65, 193)}
+        assert len(cuts) == 1 and cuts != {0}
+        for m in (193, 255, 256, 300, 512):
+            shares = lin.stage_shares_for(rows(m))
+            assert 0 <= shares <= 16 and (shares == 0 or k % (64 * shares) == 0)
