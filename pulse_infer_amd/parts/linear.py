@@ -31,7 +31,7 @@ from .base import LazyNorm, RowStats, Workspace
 # stages where it is the faster one (``takes_stages``); or the tiled product, "swiglu": for gate and up with SwiGLU inside,
 # which saves the pass over twice the feed-forward's width (the others as with "stages"), "all": for every product of
 # bfloat16 (a step then makes no library call); "none": none of them.  (Products of fewer rows are not its business: 65 to 255
-# of them run in stages whatever it says, where they did not go to the library by rules of their own before.)  PULSE_OWN_PRODUCTS sets it.
+# of them run in stages, where that is the faster one, whatever it says.)  PULSE_OWN_PRODUCTS sets it.
 # Measured: a prompt of 509 tokens of the 8B shape 9.2 ms with "stages", 9.6 with "none".  Through the serving loop, a prompt of
 # 2,048 tokens 73.9K tokens/s with "none", 72.9K with "swiglu", 71.6K with "all" (alone and with the chip warm, gate+up
 # with SwiGLU inside takes 310 us against the library's 328 + 30 for the pass; between the other kernels of a step the
@@ -261,11 +261,10 @@ class Linear:
     # 5,120 153, 196 and 247 against 171, 201 and 282; of 51,200 x 5,120, wider than that, 202, 312 and 384 against 212,
     # 279 and 396); otherwise, up to 1,536 rows, where its tiles fill their rounds, which its estimate tells: at least 1.1
     # PFLOP/s (24,576 x 4,096 at 1,024 rows 176 against 184, but at 800 173 against 154; 34,816 x 5,120 at 1,024 322
-    # against 410).  Plain products as long as the library leaves compute units idle (6,144 x 4,096 at 1,024 rows 51
-    # against 53), updates in shares up to 512 rows unless the library's shares fill half the units (4,096 x 4,096 at 512 rows 25
+    # against 410).  Plain products: see ``fills_stages``.  Updates in shares up to 512 rows unless the library's shares fill half the units (4,096 x 4,096 at 512 rows 25
     # against 31, 2,560 x 9,728 at 357 27 against 41; 4,096 x 12,288 at 357 and 509 rows takes as long either way, 45 and 60,
     # but in eight shares at 357, which cost the norm behind 2 more).  Small products stay where they are.
-    STAGE_ROWS = (65, 256)              # any of these (from ``TILE_MIN_ROWS`` on if ``OWN_MANY_ROWS`` leaves them to it)
+    STAGE_ROWS = (65, 256)              # with SwiGLU and in shares any of these (the last one if ``OWN_MANY_ROWS`` leaves it to it)
     STAGE_ROWS_SWIGLU = (768, 1536)
     STAGE_SWIGLU_RATE = 1100            # flops a nanosecond
     STAGE_ROWS_SHARES = 512
@@ -283,12 +282,35 @@ class Linear:
             return False
         if rows >= self.TILE_MIN_ROWS and (OWN_MANY_ROWS == "none" or self.takes_tiles(x, w, swiglu)):
             return False
+        if not swiglu:
+            return self.fills_stages(rows, n, k)
         if rows <= self.STAGE_ROWS[1]:
             return True
-        if not swiglu:
-            return n <= 32 * compute_units() and rows <= self.STAGE_ROWS_NARROW
         return ((n <= 192 * compute_units() and rows <= self.STAGE_ROWS_SWIGLU[0])
                 or kernels.gemm_stages_time(rows, n, k) * self.STAGE_SWIGLU_RATE <= 2 * rows * n * k)
+
+    def fills_stages(self, rows: int, n: int, k: int) -> bool:
+        """Whether a plain product's tiles keep enough compute units busy: its inner dimension cannot be cut (the result is
+        bfloat16), as the library's can, so it is the slower one where most units have no tile.
+
+        Measured over 28 weights of 576 to 65,536 rows and 1,024 to 8,192 columns (tiles a unit and round: us, library / this):
+        576 x 8,192 at 128 rows (0.07) 14 / 36, 1,536 x 7,168 at 97 (0.19) 19 / 28, 2,048 x 4,096 at 128 (0.25) 12.5 / 20,
+        4,096 x 4,096 at 97 (0.50) 16 / 18, 10,240 x 5,120 at 97 (0.62) 34 / 39; 6,144 x 4,096 at 97 (0.75) 23 / 19, 4,096 x 4,096
+        at 160 (0.75) 27 / 19, 7,168 x 4,096 at 192 (0.88) 35 / 28, 8,192 x 2,048 at 224 (1.0) 24 / 17; of 2,048 columns and
+        fewer already 3,072 x 2,048 at 97 (0.38) 12 / 11, 4,096 x 1,024 at 65 (0.50) 11 / 7.  Beyond 256 rows the library's own
+        tiles fill: 4,096 x 4,096 at 700 (0.75) 35 / 39, 8,192 x 8,192 at 333 (0.75) 66 / 75, 6,144 x 2,560 at 300 (0.94) 22 / 24, but 6,144 x 4,096 at 357 (0.75, tiles
+        of 96 x 128) 38 / 33, 8,192 x 2,048 at 300 (0.75) 24 / 21, 6,144 x 4,096 at 512 (1.0) 39 / 37.  (The library's times jump with the rows,
+        28 us at 255 and 42 at 256 for 6,144 x 4,096, so a rule of sizes leaves some on the wrong side: 5 to 15 % at a twentieth of the 375
+        sizes measured, 6,144 x 2,560 at 255 20 / 23, 4,608 x 3,072 at 444 25 / 29.)"""
+        tile_n, tile_m = kernels.gemm_stages_tile(rows, n, k)
+        tiles, units = ((n + tile_n - 1) // tile_n) * ((rows + tile_m - 1) // tile_m), compute_units()
+        fill = tiles / (((tiles + units - 1) // units) * units)
+        if rows <= self.STAGE_ROWS[1]:
+            return fill >= 0.7 or (k <= 2048 and fill >= 0.33)
+        if n > 32 * units or rows > self.STAGE_ROWS_NARROW:
+            return False
+        return fill >= 0.95 or (rows <= self.STAGE_ROWS_SHARES and fill >= 0.7
+                                and (k <= 2048 or (k <= 4096 and tile_n * tile_m >= 96 * 128)))
 
     def stage_shares_for(self, x: torch.Tensor) -> int:
         """Into how many shares of the inner dimension the product in stages cuts an update that the next norm adds up; 0:

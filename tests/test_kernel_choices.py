@@ -180,3 +180,29 @@ def test_shares_of_an_update_depend_on_the_weight_alone_up_to_192_rows(units):
         for m in (193, 255, 256, 300, 512):
             shares = lin.stage_shares_for(rows(m))
             assert 0 <= shares <= 16 and (shares == 0 or k % (64 * shares) == 0)
+
+
+def test_plain_products_in_stages_keep_the_compute_units_busy(monkeypatch):
+    """Narrow weights whose tiles leave most units idle stay with the library, whose product can cut their inner dimension;
+    what fills the chip goes in stages, up to 255 rows and, while the weight is narrow, to 1,024."""
+    import torch
+    from pulse_infer_amd.ops import device, kernels
+    from pulse_infer_amd.parts import linear
+    from pulse_infer_amd.parts.linear import Linear
+
+    monkeypatch.setattr(device, "_units", 256)
+    monkeypatch.setattr(linear, "OWN_MANY_ROWS", "stages")
+    takes = lambda m, n, k: Linear(torch.empty(n, k, dtype=torch.bfloat16, device="meta"), "bfloat16").takes_stages(
+        torch.empty(m, k, dtype=torch.bfloat16, device="meta"))
+    for n, k in ((576, 8192), (1536, 7168), (2048, 4096), (1024, 4096)):
+        assert not any(takes(m, n, k) for m in (65, 97, 128, 192, 255))
+    for n, k in ((6144, 4096), (7168, 4096), (8192, 2048), (12288, 4096)):
+        assert all(takes(m, n, k) for m in (65, 97, 128, 192, 255))
+    assert takes(357, 6144, 4096) and takes(512, 6144, 4096) and not takes(700, 4096, 4096) and not takes(1100, 6144, 4096)
+    assert not takes(64, 6144, 4096) and not takes(300, 12288, 4096)
+    for m in (65, 255, 256, 1024):
+        for n, k in ((2112, 7168), (5120, 8192), (3072, 2048), (24576, 1536)):
+            tile = kernels.gemm_stages_tile(m, n, k)
+            if takes(m, n, k):
+                tiles = -(-n // tile[0]) * -(-m // tile[1])
+                assert tiles >= 0.33 * 256
