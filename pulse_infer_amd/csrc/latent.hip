@@ -163,47 +163,62 @@ template <> __device__ __forceinline__ hp_bf16x8 load8<float>(const float* p) {
 
 // A workgroup takes 16 TT tokens of one head and 4 / KW tiles of 16 output channels; KW of its wavefronts share a tile's K out
 // in steps of 32 and meet in LDS in their order.  W rows are the matrix cores' row operand (m = output channel), the tokens'
-// rows of x the column operand, so a lane ends up with four neighbouring channels of its token.
+// rows of x the column operand, so a lane ends up with four neighbouring channels of its token.  K is summed in KW * CH chains,
+// step s in chain s % (KW * CH), which are added in their order: KW * CH goes with K alone, so a token's sums do not depend
+// on how many tokens there are.
 //
 // What bounds it for few tokens: trips to memory.  A workgroup a head walked all its tiles a piece of 32 values at a time: 8
-// tokens, 32 heads, 512 x 128 and 128 x 512 18 us each, 5.3 and 5.2 with a workgroup a few tiles and the pieces of
+// tokens, 32 heads, 512 x 128 and 128 x 512 10.2 and 8.3 us, 3.0 and 3.1 with a workgroup a few tiles and the pieces of
 // AHEAD steps asked for together.
-template <typename TX, int TT, int KW>
+template <typename TX, int TT, int KW, int CH>
 __global__ __launch_bounds__(256) void heads_product_kernel(const TX* __restrict__ x, int64_t x_stride, int x_head,
                                                             const bf16_t* __restrict__ w, const bf16_t* __restrict__ gate,
                                                             int64_t gate_stride, bf16_t* __restrict__ y, int64_t y_stride,
                                                             int y_head, int tokens, int m_out, int k_in, float scale, int gate_heads) {
+    static_assert(KW == 1 || CH == 1, "the chains are the wavefronts' or one wavefront's");
     __shared__ hp_f32x4 meet[KW > 1 ? 4 : 1][TT][PULSE_WAVE];
     const int t0 = blockIdx.x * (16 * TT), h = blockIdx.y;
     const int lane = threadIdx.x % PULSE_WAVE, wave = threadIdx.x / PULSE_WAVE;
     const int r = lane % 16, g = lane / 16;
-    const int m0 = (static_cast<int>(blockIdx.z) * (4 / KW) + wave / KW) * 16, share = wave % KW;
+    const int share = wave % KW;
     const TX* xrow[TT];
 #pragma unroll
     for (int u = 0; u < TT; ++u)
         xrow[u] = x + static_cast<int64_t>(min(t0 + 16 * u + r, tokens - 1)) * x_stride + static_cast<int64_t>(h) * x_head;
     const hp_bf16x8 zero = __builtin_bit_cast(hp_bf16x8, make_uint4(0u, 0u, 0u, 0u));
+    const int m0 = (static_cast<int>(blockIdx.z) * (4 / KW) + wave / KW) * 16;
     const int m = m0 + r;
     const bf16_t* wrow = m < m_out ? w + (static_cast<int64_t>(h) * m_out + m) * k_in : nullptr;
-    hp_f32x4 acc[TT];
+    hp_f32x4 chain[CH][TT];
 #pragma unroll
-    for (int u = 0; u < TT; ++u) acc[u] = hp_f32x4{0.f, 0.f, 0.f, 0.f};
-    constexpr int AHEAD = TT == 1 ? 4 : 2;
-    for (int k0 = share * 32; k0 < k_in; k0 += 32 * KW * AHEAD) {
-        hp_bf16x8 wa[AHEAD], xb[AHEAD][TT];
+    for (int c = 0; c < CH; ++c)
 #pragma unroll
-        for (int v = 0; v < AHEAD; ++v) {
-            const int k = k0 + 32 * KW * v + 8 * g;
-            const bool in = k < k_in;
-            wa[v] = (in && wrow) ? *reinterpret_cast<const hp_bf16x8*>(wrow + k) : zero;
+        for (int u = 0; u < TT; ++u) chain[c][u] = hp_f32x4{0.f, 0.f, 0.f, 0.f};
+    constexpr int AHEAD = TT == 1 ? 4 : 2, ROUND = CH > AHEAD ? CH : AHEAD;
+    for (int k0 = share * 32; k0 < k_in; k0 += 32 * KW * ROUND) {
 #pragma unroll
-            for (int u = 0; u < TT; ++u) xb[v][u] = in ? load8<TX>(xrow[u] + k) : zero;
+        for (int v0 = 0; v0 < ROUND; v0 += AHEAD) {
+            hp_bf16x8 wa[AHEAD], xb[AHEAD][TT];
+#pragma unroll
+            for (int v = 0; v < AHEAD; ++v) {
+                const int k = k0 + 32 * KW * (v0 + v) + 8 * g;
+                const bool in = k < k_in;
+                wa[v] = (in && wrow) ? *reinterpret_cast<const hp_bf16x8*>(wrow + k) : zero;
+#pragma unroll
+                for (int u = 0; u < TT; ++u) xb[v][u] = in ? load8<TX>(xrow[u] + k) : zero;
+            }
+#pragma unroll
+            for (int v = 0; v < AHEAD; ++v)
+#pragma unroll
+                for (int u = 0; u < TT; ++u)
+                    chain[(v0 + v) % CH][u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa[v], xb[v][u], chain[(v0 + v) % CH][u], 0, 0, 0);
         }
-#pragma unroll
-        for (int v = 0; v < AHEAD; ++v)
-#pragma unroll
-            for (int u = 0; u < TT; ++u) acc[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa[v], xb[v][u], acc[u], 0, 0, 0);
     }
+    hp_f32x4 (&acc)[TT] = chain[0];
+#pragma unroll
+    for (int c = 1; c < CH; ++c)
+#pragma unroll
+        for (int u = 0; u < TT; ++u) acc[u] += chain[c][u];
     if constexpr (KW > 1) {
 #pragma unroll
         for (int u = 0; u < TT; ++u) meet[wave][u][lane] = acc[u];
@@ -435,20 +450,23 @@ extern "C" int pulse_heads_product(const void* x, int64_t x_stride, int x_head, 
     PULSE_REQUIRE(reinterpret_cast<uintptr_t>(x) % 16 == 0 && (x_stride * xb) % 16 == 0 && (static_cast<int64_t>(x_head) * xb) % 16 == 0 &&
                   reinterpret_cast<uintptr_t>(w) % 16 == 0, "heads_product: operands must be 16-byte aligned");
     if (tokens == 0) return 0;
-    // K shared out from 256 values on, while there are few tokens: there the walk along K is what a workgroup waits for.
-    const int kw = tokens < 256 && k_in >= 256 ? 4 : 1;
+    // K in four chains from 256 values on: while there are few tokens the wavefronts' (the walk along K is what a workgroup
+    // waits for), then one wavefront's.
+    const bool chains = k_in >= 256;
+    const int kw = tokens < 256 && chains ? 4 : 1, tt = tokens >= 256 ? 4 : 1;
     const unsigned tiles_m = (m_out + 15) / 16, groups = (tiles_m + 4 / kw - 1) / (4 / kw);
     PULSE_REQUIRE(groups < 65536, "heads_product: %d output channels are too many", m_out);
-#define PULSE_HEADS(TT_, KW_)                                                                                            \
+#define PULSE_HEADS(TT_, KW_, CH_)                                                                                       \
     PULSE_DISPATCH_DTYPE(x_dtype, TX,                                                                                    \
-        hipLaunchKernelGGL((heads_product_kernel<TX, TT_, KW_>), dim3((tokens + 16 * TT_ - 1) / (16 * TT_), heads, groups), \
-                           dim3(256), 0,                                                                                 \
-                           stream, static_cast<const TX*>(x), x_stride, x_head, static_cast<const bf16_t*>(w),           \
+        hipLaunchKernelGGL((heads_product_kernel<TX, TT_, KW_, CH_>), dim3((tokens + 16 * TT_ - 1) / (16 * TT_), heads,  \
+                           groups), dim3(256), 0, stream, static_cast<const TX*>(x), x_stride, x_head,                   \
+                           static_cast<const bf16_t*>(w),                                                                \
                            static_cast<const bf16_t*>(gate), gate_stride, static_cast<bf16_t*>(y), y_stride, y_head,     \
                            tokens, m_out, k_in, scale, gate_heads))
-    if (tokens >= 256) PULSE_HEADS(4, 1);
-    else if (kw == 4) PULSE_HEADS(1, 4);
-    else PULSE_HEADS(1, 1);
+    if (tt == 4 && chains) PULSE_HEADS(4, 1, 4);
+    else if (tt == 4) PULSE_HEADS(4, 1, 1);
+    else if (chains) PULSE_HEADS(1, 4, 1);
+    else PULSE_HEADS(1, 1, 1);
 #undef PULSE_HEADS
     PULSE_LAUNCH_CHECK("heads_product");
     return 0;

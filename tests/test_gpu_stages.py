@@ -95,3 +95,27 @@ def test_an_update_in_stages_does_not_depend_on_the_rows_beside_it(n, k):
     assert whole.dim() == 3
     for m in (65, 97, 128, 160, 191):
         assert torch.equal(lin.add_into(x[:m], h[:m], scratch[:m], ws), whole[:, :m])
+
+
+@pytest.mark.parametrize("m_out,k_in", [(512, 128), (40, 256), (128, 512), (72, 264), (200, 1000)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_a_product_a_head_does_not_depend_on_the_tokens_beside_it(m_out, k_in, dtype):
+    """A token by itself, a few, and enough for tiles of 64 tokens: the same bits."""
+    from pulse_infer_amd.ops import kernels
+
+    heads, tokens = 5, 1100
+    w = (rnd(heads, m_out, k_in, seed=1) * k_in ** -0.5).to(torch.bfloat16).to(DEV)
+    x = rnd(tokens, heads * k_in, seed=2).to(dtype).to(DEV)
+
+    def run(rows):
+        out = torch.full((rows.shape[0], heads * m_out), float("nan"), dtype=torch.bfloat16, device=DEV)
+        kernels.heads_product(rows, k_in, w, None, out, m_out, 0.5)
+        return out
+
+    whole = run(x)
+    for a, b in ((0, 1), (3, 20), (100, 355), (500, 756), (700, 1001)):
+        assert torch.equal(run(x[a:b].contiguous()), whole[a:b]), (a, b)
+    xr = x.to(torch.bfloat16).cpu().to(F64).view(tokens, heads, k_in)
+    want = 0.5 * torch.stack([xr[:, h] @ w[h].cpu().to(F64).T for h in range(heads)], 1).reshape(tokens, -1)
+    size = 0.5 * torch.stack([xr[:, h].abs() @ w[h].cpu().to(F64).abs().T for h in range(heads)], 1).reshape(tokens, -1)
+    assert ((whole.cpu().to(F64) - want).abs() <= (k_in + 4) * 2.0 ** -24 * size + 2.0 ** -8 * want.abs()).all()
