@@ -379,11 +379,12 @@ __global__ __launch_bounds__(VEC_THREADS) void qk_rope_kv_vec_kernel(bf16_t* __r
                                                                      int tokens, int per_token, int rope_groups) {
     const int b = blockIdx.x;
     if (b < rope_groups) {
-        const int64_t row = static_cast<int64_t>(b) * (VEC_THREADS / PULSE_WAVE) + threadIdx.x / PULSE_WAVE;
-        if (row >= static_cast<int64_t>(tokens) * per_token) return;
-        qk_rope_rows<TW, PAIRING, LPH>(static_cast<int>(row / per_token), static_cast<int>(row % per_token),
-                                       threadIdx.x % PULSE_WAVE, qkv, q_w, k_w, cos_t, sin_t, kcache, positions, token_entry,
-                                       block_table, a);
+        // (fewer than 2^30 rows, see the entry point: a division of 32 bits, by one number for the whole wavefront)
+        const unsigned row = __builtin_amdgcn_readfirstlane(b * (VEC_THREADS / PULSE_WAVE) + threadIdx.x / PULSE_WAVE);
+        const unsigned t = row / static_cast<unsigned>(per_token);
+        if (t >= static_cast<unsigned>(tokens)) return;
+        qk_rope_rows<TW, PAIRING, LPH>(static_cast<int>(t), static_cast<int>(row - t * per_token), threadIdx.x % PULSE_WAVE, qkv, q_w,
+                                       k_w, cos_t, sin_t, kcache, positions, token_entry, block_table, a);
     } else {
         v_page_rows((b - rope_groups) / a.nkv, (b - rope_groups) % a.nkv, qkv, vcache, positions, token_entry, block_table, a,
                     tokens);
