@@ -225,11 +225,13 @@ def test_benchmark_layer_sizes(layer_shape, dtype):
     torch.cuda.empty_cache()
 
 
-@pytest.mark.parametrize("policy", ["swiglu", "all"])
+@pytest.mark.parametrize("policy", ["stages", "swiglu", "all"])
 def test_benchmark_layer_sizes_with_this_packages_products_for_many_rows(layer_shape, policy, monkeypatch):
     """A prompt of 600 tokens at the benchmark's layer sizes, whole and in portions of 300, 260 and 40 tokens, with the
-    products of 256 and more rows in this package's tiled product (gate and up with SwiGLU inside; or all of them, o
-    and down in shares of the inner dimension) against the plain implementation and against the library's products."""
+    products of 256 and more rows as the default has them (in stages where that is the faster one: gate and up with SwiGLU
+    inside, o in shares that the next norm adds up) or in this package's tiled product (gate and up with SwiGLU inside; or
+    all of them, o and down in shares of the inner dimension) against the plain implementation and against the library's
+    products."""
     from pulse_infer_amd.engine.runner import ModelRunner
     from pulse_infer_amd.models.factory import load_model
     from pulse_infer_amd.parts import linear

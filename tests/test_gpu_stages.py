@@ -11,10 +11,12 @@ def rnd(*shape, seed):
     return torch.randn(shape, generator=torch.Generator().manual_seed(seed))
 
 
-# every tile the plan knows, with remainders of rows and weight rows, one step of K and many, one row and several panels
+# remainders of rows and weight rows, one step of K and many, one row and several panels; bfloat16 results, float32 shares of one
+# step each and of the plan's number, SwiGLU (which tile runs is the plan's choice: every one of them, with the stages of K going
+# round, is in the tests behind this one)
 @pytest.mark.parametrize("shape", [(1, 32, 64), (65, 96, 128), (97, 6144, 192), (97, 24576, 64), (128, 4096, 1024),
                                    (130, 24608, 128), (193, 12288, 64), (256, 4128, 320), (357, 6176, 64), (1030, 2080, 128),
-                                   # tiles of 192 and 256 rows of X: 192 x 192, 192 x 256, 256 x 192, 256 x 256, panels of them
+                                   # tiles of 192 and 256 rows of X, panels of them
                                    (357, 24544, 64), (509, 24544, 1024), (357, 24608, 64), (509, 24608, 64), (2100, 8224, 128)])
 def test_product_in_stages_at_the_edges_of_its_tiles(shape):
     from pulse_infer_amd.ops import kernels
@@ -47,6 +49,58 @@ def test_product_in_stages_at_the_edges_of_its_tiles(shape):
         wanted = gate * torch.sigmoid(gate) * up
         # hardware exponential and reciprocal (relative 2^-21 each), one rounding to bfloat16
         assert ((act.cpu().to(F64) - wanted).abs() <= 2.0 ** -7.9 * wanted.abs() + 1e-5).all()
+
+
+STEPS = 13      # more than twice the stages of any tile: every stage is filled, read and filled again
+
+
+def product(m, n, k):
+    x, w = rnd(m, k, seed=1).to(torch.bfloat16).to(DEV), (rnd(n, k, seed=2) * k ** -0.5).to(torch.bfloat16).to(DEV)
+    want, size = x.to(F64) @ w.to(F64).T, x.to(F64).abs() @ w.to(F64).abs().T
+    return x, w, want, (k + 2) * 2.0 ** -24 * size          # (a float32 sum of k exact products, in any order)
+
+
+# the tile that the plan takes for these rows and weight rows on 256 compute units, remainders of both
+@pytest.mark.parametrize("tile,m,n", [((64, 64), 70, 672), ((64, 128), 70, 8288), ((96, 128), 70, 16928), ((128, 64), 130, 8288),
+                                      ((128, 128), 130, 12960), ((192, 128), 130, 16928), ((256, 128), 130, 24864),
+                                      ((192, 192), 130, 32800), ((192, 256), 193, 32800), ((256, 192), 300, 24864),
+                                      ((256, 256), 600, 16928)])
+def test_every_tile_of_the_product_in_stages(tile, m, n):
+    from pulse_infer_amd.ops import kernels
+
+    k = 64 * STEPS
+    assert kernels.gemm_stages_tile(m, n, k) == tile and m % tile[1] and n % tile[0]
+    x, w, want, exact = product(m, n, k)
+    out = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device=DEV)
+    kernels.gemm_stages(x, w, out)
+    assert ((out.to(F64) - want).abs() <= exact + 2.0 ** -8 * want.abs()).all()
+    act = torch.full((m, n // 2), float("nan"), dtype=torch.bfloat16, device=DEV)
+    kernels.gemm_stages(x, w, act, swiglu=True)
+    slab = torch.arange(n, device=DEV) // 16 % 2
+    gate, up, gate_off, up_off = want[:, slab == 0], want[:, slab == 1], exact[:, slab == 0], exact[:, slab == 1]
+    silu = gate * torch.sigmoid(gate)
+    # (silu's slope is 1.1 at most; the exponential and the reciprocal, one rounding to bfloat16)
+    bound = (2.0 ** -8 + 2.0 ** -16) * (silu * up).abs() + 1.1 * gate_off * (up.abs() + up_off) + silu.abs() * up_off
+    assert ((act.to(F64) - silu * up).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("tile,m,n,shares", [((64, 64), 70, 356, 2), ((64, 128), 70, 4232, 2), ((96, 128), 70, 8336, 2),
+                                             ((128, 64), 130, 4232, 2), ((128, 128), 130, 3092, 4), ((192, 128), 130, 8336, 2),
+                                             ((256, 128), 130, 12440, 2), ((192, 192), 130, 16544, 2), ((192, 256), 193, 16544, 2),
+                                             ((256, 192), 130, 12440, 4), ((256, 256), 193, 12440, 4)])
+def test_every_tile_of_the_product_in_stages_in_shares(tile, m, n, shares):
+    from pulse_infer_amd.ops import kernels
+
+    k = 64 * STEPS * shares
+    assert kernels.gemm_stages_tile(m, n, k, shares) == tile and m % tile[1] and n % tile[0]
+    x, w, want, exact = product(m, n, k)
+    parts = torch.full((shares, m, n), float("nan"), device=DEV)
+    kernels.gemm_stages(x, w, parts)
+    assert ((parts.to(F64).sum(0) - want).abs() <= exact).all()
+    part = k // shares
+    for i in range(shares):
+        a, b = x[:, i * part:(i + 1) * part].to(F64), w[:, i * part:(i + 1) * part].to(F64)
+        assert ((parts[i].to(F64) - a @ b.T).abs() <= (part + 2) * 2.0 ** -24 * (a.abs() @ b.abs().T)).all(), i
 
 
 def test_product_in_stages_refuses_what_it_cannot_read():
