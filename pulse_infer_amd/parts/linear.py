@@ -136,14 +136,16 @@ class Linear:
     def add_into(self, x: torch.Tensor, residual: torch.Tensor, scratch: torch.Tensor,
                  workspace: Optional[Workspace] = None, next_scale: Optional[torch.Tensor] = None,
                  next_offset: float = 0.0, leave_stats: bool = True):
-        """residual += x W^T, in one of five ways.  Few rows: the kernel adds into the residual itself and None is
+        """residual += x W^T, in one of six ways.  Few rows: the kernel adds into the residual itself and None is
         returned, or, given a workspace and a shape the fused kernel takes, the ``RowStats`` of the updated rows (their
         sums of squares and a rounded copy, multiplied column by column by ``next_scale``, the weight of the norm that
         reads the residual next, ``next_offset`` added to each in float32: with these the next product can do without a
         norm kernel before it).  17 to
         192 rows, given a workspace: the product's inner dimension is shared out over workgroups and the shares' float32
-        results [parts, rows, out] are returned as the update, which the next norm adds up in order; more rows of a
-        product with a wide inner dimension and a narrow output: the same through the library's batched product.
+        results [parts, rows, out] are returned as the update, which the next norm adds up in order; 65 to 512 rows of a
+        weight that is not small: the same from the product in stages (``stage_shares_for``); more rows of a product with a
+        wide inner dimension and a narrow output: the same through the library's batched product, or, if all products are to
+        be this package's, the tiled one.
         Otherwise the product is written to ``scratch`` and returned for the caller to add.  ``leave_stats=False``:
         no ``RowStats`` are made (their buffers are the workspace's, one set a width: a caller that still reads the
         set of the rows as they were before this update says so)."""
@@ -204,7 +206,7 @@ class Linear:
     MID_ROWS = (17, 64)          # where the product with X shared through LDS and SwiGLU inside beats the library's
                                  # product followed by the SwiGLU kernel
     SHARES_ROWS = (17, 192)      # where a product that adds into the residual has its inner dimension shared out over
-                                 # workgroups (measured on the 8B shape: 1% of a decoding step at 17 to 32 rows, 4% at
+                                 # workgroups, from 65 rows on if the product in stages does not take it (measured on the 8B shape: 1% of a decoding step at 17 to 32 rows, 4% at
                                  # 48, 6% at 64; at 96 to 192 rows the library takes 22 to 33 us for o and 55 to 90 us
                                  # for down, the shared-out product 16 to 22 and 33 to 47.  Up to 16 rows the few-rows
                                  # kernel stands: it leaves what the next product needs to do without a norm kernel,
