@@ -143,9 +143,9 @@ class Linear:
         norm kernel before it).  17 to
         192 rows, given a workspace: the product's inner dimension is shared out over workgroups and the shares' float32
         results [parts, rows, out] are returned as the update, which the next norm adds up in order; 65 to 512 rows of a
-        weight that is not small: the same from the product in stages (``stage_shares_for``); more rows of a product with a
-        wide inner dimension and a narrow output: the same through the library's batched product, or, if all products are to
-        be this package's, the tiled one.
+        weight that is not small, and more rows of a product with a wide inner dimension and a narrow output: the same from
+        the product in stages (``stage_shares_for``), from the tiled one if all products are to be it, or from the library's
+        if none of them is to be this package's.
         Otherwise the product is written to ``scratch`` and returned for the caller to add.  ``leave_stats=False``:
         no ``RowStats`` are made (their buffers are the workspace's, one set a width: a caller that still reads the
         set of the rows as they were before this update says so)."""
@@ -170,20 +170,21 @@ class Linear:
                                      self.out_features, torch.float32).view(splits, rows, self.out_features)
             kernels.gemm_tile(x, self.weight, parts)
             return parts
-        splits = self.library_shares_for(x) if workspace is not None else 0
+        splits = self.library_shares_for(x) if workspace is not None and self.operands_ok(x) else 0
         if splits:
-            # Many rows but few output tiles (down: a wide inner dimension, a narrow output): the library's product
-            # leaves most compute units idle (14B shape, 544 rows: 179 us), so it runs as a batch over shares of the
-            # inner dimension (102 us) whose float32 results the next norm adds up in order.
+            # Many rows but few output tiles (down: a wide inner dimension, a narrow output) that the product in stages is
+            # not to take: the library's product, a share of the inner dimension after the other, with float32 results
+            # that the next norm adds up in order.  (Not as one batched product: its right operand would be a transposed
+            # view of bfloat16, a form that is unsafe on this stack, and a copy of the weight costs more than it gains.)
             rows, share = x.shape[0], self.in_features // splits
             parts = workspace.buffer(f"linear.parts.{self.out_features}.{self.in_features}", splits * rows,
                                      self.out_features, torch.float32).view(splits, rows, self.out_features)
-            xa = x.view(rows, splits, share).transpose(0, 1)
-            wb = self.weight.view(self.out_features, splits, share).permute(1, 2, 0)
             global library_calls
             library_calls += 1
-            with timing.region("library batched matmul"):
-                torch.bmm(xa, wb, out_dtype=torch.float32, out=parts)
+            with timing.region("library matmul in shares"):
+                for s in range(splits):
+                    cut = slice(s * share, (s + 1) * share)
+                    torch.mm(x[:, cut], self.weight[:, cut].t(), out_dtype=torch.float32, out=parts[s])
             return parts
         if (self.library and x.dtype == torch.bfloat16 and x.shape[0] <= kernels.SKINNY_FAST_ROWS
                 and kernels.gemm_skinny_ok(x, self.weight)):
@@ -212,15 +213,16 @@ class Linear:
                                  # kernel stands: it leaves what the next product needs to do without a norm kernel,
                                  # and a step of 13 rows is 3% faster with it, one of 16 rows as fast)
 
-    LIBRARY_SHARES_MIN_K = 8192  # inner dimensions from here on are worth sharing out in the library's product
-    LIBRARY_TILE = 256           # its output tiles are about this large in both directions
+    LIBRARY_SHARES_MIN_K = 8192  # inner dimensions from here on are worth sharing out beyond 192 rows
+    LIBRARY_TILE = 256           # the library's output tiles are about this large in both directions
 
     def library_shares_for(self, x: torch.Tensor) -> int:
-        """Into how many shares the library's product of more than 192 rows is cut; 0: not at all.  Measured (8B,
-        14B and 32B shapes of down, 272 to 2,048 rows): 4 shares win up to about 50 output tiles, 2 shares up to
-        about 140 (8B shape at 2,048 rows: 182 -> 157 us, which the wider update costs again in the norm that adds
-        it up, so the rule stops at 100 tiles), none beyond; products with an inner dimension of 4,096 to 8,192 (o)
-        gain 5 us at most."""
+        """Whether an update of more than 192 rows has so few output tiles and so wide an inner dimension that it is to be
+        made in shares beyond the sizes that go in stages anyway, and into how many the library's is cut (``OWN_MANY_ROWS``
+        "none"); 0: not at all.  Measured (8B, 14B and 32B shapes of down, 272 to 2,048 rows): up to about 100 tiles shares
+        win (14B shape at 544 rows 179 -> 102 us with the library's products side by side, 90 in stages); the 8B shape at
+        2,048 rows gains in the product (182 -> 157 us) what the wider update costs again in the norm that adds it up;
+        products with an inner dimension of 4,096 to 8,192 (o) gain 5 us at most."""
         rows = x.shape[0]
         if not (self.library and x.dtype == torch.bfloat16 and rows > self.SHARES_ROWS[1]
                 and self.in_features >= self.LIBRARY_SHARES_MIN_K and x.is_contiguous()
@@ -263,13 +265,14 @@ class Linear:
     # 5,120 153, 196 and 247 against 171, 201 and 282; of 51,200 x 5,120, wider than that, 202, 312 and 384 against 212,
     # 279 and 396); otherwise, up to 1,536 rows, where its tiles fill their rounds, which its estimate tells: at least 1.1
     # PFLOP/s (24,576 x 4,096 at 1,024 rows 176 against 184, but at 800 173 against 154; 34,816 x 5,120 at 1,024 322
-    # against 410).  Plain products: see ``fills_stages``.  Updates in shares up to 512 rows unless the library's shares fill half the units (4,096 x 4,096 at 512 rows 25
-    # against 31, 2,560 x 9,728 at 357 27 against 41; 4,096 x 12,288 at 357 and 509 rows takes as long either way, 45 and 60,
-    # but in eight shares at 357, which cost the norm behind 2 more).  Small products stay where they are.
+    # against 410).  Plain products: see ``fills_stages``.  Updates in shares: up to 512 rows all that are not small (4,096 x 4,096 at 512 rows 25 us against
+    # the library's 31, 2,560 x 9,728 at 357 27 against 41), beyond those of a wide inner dimension and few tiles
+    # (``library_shares_for``): us without the norm behind, rows 544 / 768 / 1,024: 4,096 x 12,288 65 / 69 / 90, 5,120 x 17,408
+    # 90 / 122 / 162 (the library's in shares side by side 102 at 544).  Small products stay where they are.
     STAGE_ROWS = (65, 256)              # with SwiGLU and in shares any of these (the last one if ``OWN_MANY_ROWS`` leaves it to it)
     STAGE_ROWS_SWIGLU = (768, 1536)
     STAGE_SWIGLU_RATE = 1100            # flops a nanosecond
-    STAGE_ROWS_SHARES = 512
+    STAGE_ROWS_SHARES = 512             # beyond, only where ``library_shares_for`` says so
     STAGE_CUT_ROWS = 128                # the rows that updates of up to 192 rows are cut into shares for
     STAGE_ROWS_NARROW = 1024            # plain products of at most 32 weight rows a compute unit
     STAGE_MIN_WEIGHT = 1 << 22
@@ -318,18 +321,15 @@ class Linear:
         """Into how many shares of the inner dimension the product in stages cuts an update that the next norm adds up; 0:
         not this product.  Up to 192 rows the cut depends on the weight's shape alone, as that of the shared-out product, so
         a row's sums do not depend on how many rows are beside it (the best cut for 128 rows: as fast as one by the rows, but
-        2,560 x 4,096 at 192 rows 23 us against 19); beyond, as in the library's product, it goes with the rows."""
+        2,560 x 4,096 at 192 rows 23 us against 19); beyond it goes with the rows."""
         rows, n, k = x.shape[0], self.out_features, self.in_features
-        if not (self.library and x.dtype == torch.bfloat16 and self.STAGE_ROWS[0] <= rows <= self.STAGE_ROWS_SHARES
-                and n * k >= self.STAGE_MIN_WEIGHT and self.operands_ok(x)) or n % 4 or k % 64:
+        if not (self.library and x.dtype == torch.bfloat16 and self.STAGE_ROWS[0] <= rows and self.operands_ok(x)) \
+                or n % 4 or k % 64 or (n * k < self.STAGE_MIN_WEIGHT and not self.library_shares_for(x)):
             return 0
         if rows >= self.TILE_MIN_ROWS and (OWN_MANY_ROWS == "none" or self.tile_shares_for(x)):
             return 0
-        if rows > self.STAGE_ROWS[1]:
-            tile = self.LIBRARY_TILE
-            tiles = ((rows + tile - 1) // tile) * ((n + tile - 1) // tile) * self.library_shares_for(x)
-            if 2 * tiles >= compute_units():
-                return 0
+        if rows > self.STAGE_ROWS_SHARES and not self.library_shares_for(x):
+            return 0
         return kernels.gemm_stages_shares(self.STAGE_CUT_ROWS if rows <= self.SHARES_ROWS[1] else rows, n, k)
 
     TILE_MIN_ROWS = 256          # from here on the tiled product for many rows is a candidate, and ``OWN_MANY_ROWS`` decides

@@ -173,3 +173,30 @@ def test_a_product_a_head_does_not_depend_on_the_tokens_beside_it(m_out, k_in, d
     want = 0.5 * torch.stack([xr[:, h] @ w[h].cpu().to(F64).T for h in range(heads)], 1).reshape(tokens, -1)
     size = 0.5 * torch.stack([xr[:, h].abs() @ w[h].cpu().to(F64).abs().T for h in range(heads)], 1).reshape(tokens, -1)
     assert ((whole.cpu().to(F64) - want).abs() <= (k_in + 4) * 2.0 ** -24 * size + 2.0 ** -8 * want.abs()).all()
+
+
+@pytest.mark.parametrize("policy", ["stages", "none"])
+@pytest.mark.parametrize("rows,n", [(193, 256), (257, 256), (513, 768), (1100, 1028), (2560, 256)])
+def test_updates_in_shares_make_no_batched_product(rows, n, policy, monkeypatch):
+    """The batched product in bfloat16 with a transposed view as its right operand is a call that has faulted: no update
+    makes it, whoever makes the shares."""
+    from pulse_infer_amd.parts import linear
+    from pulse_infer_amd.parts.base import Workspace
+
+    def never(*args, **kwargs):
+        raise AssertionError("a batched product was called")
+    for name in ("bmm", "baddbmm", "matmul", "einsum"):
+        monkeypatch.setattr(torch, name, never)
+    monkeypatch.setattr(linear, "OWN_MANY_ROWS", policy)
+    k = 8192
+    g = torch.Generator().manual_seed(rows)
+    x = torch.randn(rows, k, generator=g).bfloat16().to(DEV)
+    w = (torch.randn(n, k, generator=g) * k ** -0.5).bfloat16().to(DEV)
+    lin = linear.Linear(w, "bfloat16")
+    assert lin.library_shares_for(x)
+    parts = lin.add_into(x, torch.zeros(rows, n, device=DEV), torch.empty(rows, n, dtype=torch.bfloat16, device=DEV),
+                         Workspace(torch.device(DEV)))
+    want = torch.mm(x.double(), w.double().t())
+    bound = (k + 2) * 2.0 ** -24 * torch.mm(x.double().abs(), w.double().abs().t())     # as above, the shares' sum in 64 bits
+    assert parts.dtype == torch.float32 and parts.shape[1:] == (rows, n)
+    assert ((parts.double().sum(0) - want).abs() <= bound).all()

@@ -182,6 +182,28 @@ def test_shares_of_an_update_depend_on_the_weight_alone_up_to_192_rows(units):
             assert 0 <= shares <= 16 and (shares == 0 or k % (64 * shares) == 0)
 
 
+def test_updates_in_shares_of_many_rows_are_this_packages(units, monkeypatch):
+    """Wherever an update beyond 192 rows is worth making in shares, the product in stages makes them, also of small
+    weights, unless the option gives it to the tiled product or to the library."""
+    import torch
+    from pulse_infer_amd.parts import linear
+    from pulse_infer_amd.parts.linear import Linear
+
+    for n, k in ((4096, 12288), (5120, 17408), (2560, 9728), (1024, 8192), (256, 8192), (100, 8192)):
+        lin = Linear(torch.empty(n, k, dtype=torch.bfloat16, device="meta"), "bfloat16")
+        for m in (193, 256, 257, 357, 512, 513, 1024, 1536, 2048, 6400, 30000):
+            x = torch.empty(m, k, dtype=torch.bfloat16, device="meta")
+            for policy in ("stages", "swiglu"):
+                monkeypatch.setattr(linear, "OWN_MANY_ROWS", policy)
+                shares = lin.stage_shares_for(x)
+                assert shares or not lin.library_shares_for(x)
+                assert shares <= 16 and (not shares or k % (64 * shares) == 0)
+                if m > Linear.STAGE_ROWS_SHARES:
+                    assert bool(shares) == bool(lin.library_shares_for(x))
+            monkeypatch.setattr(linear, "OWN_MANY_ROWS", "none")
+            assert m < 256 or not lin.stage_shares_for(x)
+
+
 def test_plain_products_in_stages_keep_the_compute_units_busy(monkeypatch):
     """Narrow weights whose tiles leave most units idle stay with the library, whose product can cut their inner dimension;
     what fills the chip goes in stages, up to 255 rows and, while the weight is narrow, to 1,024."""
