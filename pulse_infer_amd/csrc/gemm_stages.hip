@@ -2,15 +2,21 @@
 // bfloat16 operands, float32 sums on the matrix cores, on the loop of tile_loop.h.
 // (reference: cuBLAS for every product, src/ops/kernels/cuda/matmul_kernel.cu:132-154)
 //
-// What bounds it: the bytes that the fullest compute unit copies into LDS.  A unit takes in 40 to 65 bytes a nanosecond
-// whatever the tile's shape, less where they are weights that come from memory, so the shape and the shares of K are
-// chosen for the least of them (`plan_for`).  Measured with weights from memory, us, against the vendor library's product
-// (gate and up: with its pass for SwiGLU behind it) and this package's shared-out product for up to 192 rows:
+// What bounds it: the bytes that the fullest compute unit copies into LDS.  A unit takes in 30 to 55 bytes a nanosecond over a
+// launch, least where they are weights that come from memory, and the matrix cores are busy for 13 to 47 % of it, LDS waits
+// make 1 to 4 % (counters at 97, 357 and 509 rows), so the shape and the shares of K are chosen for the least bytes
+// (`plan_for`).  Measured alone with weights from memory, us, against the vendor library's product (gate and up: with its
+// pass for SwiGLU behind it) and this package's shared-out product for up to 192 rows; in brackets behind a figure, what it
+// takes inside a step, between other kernels and with the chip warm:
 //                                   97 rows              192                  357                 509
-//   gate + up, 24,576 x 4,096       44 (library 54)      54 (64)              71 (84)             87 (96)
-//   qkv, 6,144 x 4,096              20 (25)              26 (36)              30 (41)             33 (42)
-//   o, 4,096 x 4,096, shares        13 (25; 16 shared)   17 (37; 21 shared)   22 (29)             24 (32)
-//   down, 4,096 x 12,288, shares    25 (44; 34 shared)   33 (92; 47 shared)   42 (52 shared)      51 (59 shared)
+//   gate + up, 24,576 x 4,096       45 [44]              54                   71 [74]             88 [101]
+//     library                       54                   64                   84                  96
+//   qkv, 6,144 x 4,096              19 [20]              26                   34 [34]             35 [38]
+//     library                       25                   36                   41                  42
+//   o, 4,096 x 4,096, shares        12 [13]              17                   22 [24]             24 [28]
+//     library / shared out          25 / 16              37 / 21              29                  32
+//   down, 4,096 x 12,288, shares    24 [25]              33                   41 [43]             52 [62]
+//     library / shared out          44 / 34              92 / 47              52, shared [46]     59, shared [60]
 // From some 260 rows on tiles of 192 or 256 rows of X (their weights through three stages, X, which comes from L2, through
 // two where LDS holds no third) take the place of the library's: 357 rows of gate + up ran 96 us in tiles of 192 x 128.
 // Steps of 32 of K in twice the stages, the other way to fit such tiles, bring 64 bytes of a row at a time, which a unit

@@ -32,11 +32,11 @@ from .base import LazyNorm, RowStats, Workspace
 # which saves the pass over twice the feed-forward's width (the others as with "stages"), "all": for every product of
 # bfloat16 (a step then makes no library call); "none": none of them.  (Products of fewer rows are not its business: 65 to 255
 # of them run in stages, where that is the faster one, whatever it says.)  PULSE_OWN_PRODUCTS sets it.
-# Measured: a prompt of 509 tokens of the 8B shape 9.2 ms with "stages", 9.6 with "none".  Through the serving loop, a prompt of
+# Measured: a prompt of 509 tokens of the 8B shape 9.0 ms with "stages", 11.3 with "none" (whose updates in shares are made one
+# after the other, see ``add_into``; 9.6 before, side by side).  Through the serving loop, a prompt of
 # 2,048 tokens 73.9K tokens/s with "none", 72.9K with "swiglu", 71.6K with "all" (alone and with the chip warm, gate+up
 # with SwiGLU inside takes 310 us against the library's 328 + 30 for the pass; between the other kernels of a step the
-# library's product takes 278); serving of the 8B shape 4,334 / 4,313 / 4,248 tokens/s, of the 14B shape 2,695 / 2,688 (means
-# of two runs each, "none" and "swiglu"), of the 32B shape 1,258 / 1,264.  So the library stays for the largest.
+# library's product takes 278): prompts of that size make no updates in shares.  So the library stays for the largest.
 OWN_MANY_ROWS = os.environ.get("PULSE_OWN_PRODUCTS", "stages")
 if OWN_MANY_ROWS not in ("none", "stages", "swiglu", "all"):
     raise ValueError(f"PULSE_OWN_PRODUCTS must be none, stages, swiglu or all, not '{OWN_MANY_ROWS}'")
