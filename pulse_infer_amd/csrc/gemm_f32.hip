@@ -1,9 +1,9 @@
 // C[M, N] = A[M, K] * W[N, K]^T in float32, every output added up in an order of its own that M has no part in.
 //
-// This is the matrix product of the true 32-bit path.  Products and sums are float32 throughout: the matrix
-// instruction is v_mfma_f32_16x16x4_f32, which multiplies and accumulates in float32 (no reduced-precision mode).
-// Inputs may be stored as bfloat16 (they are widened exactly).  (reference: cublasSgemm,
-// src/ops/kernels/cuda/matmul_kernel.cu:70-88)
+// This is the matrix product of the true 32-bit path.  Float32 operands with a large weight are multiplied as parts on the
+// bfloat16 instruction (gemm_split.hip, which is no less exact), whatever the number of rows; all others here on
+// v_mfma_f32_16x16x4_f32, which multiplies and accumulates in float32 (no reduced-precision mode).  Inputs may be stored as
+// bfloat16 (they are widened exactly).  (reference: cublasSgemm, src/ops/kernels/cuda/matmul_kernel.cu:70-88)
 //
 // The order: K is cut into blocks of 16 and the blocks into four shares, one a wavefront of the workgroup that owns the
 // output; a share is added up block after block, and the four shares in their order.  The cut depends on K alone and
@@ -11,11 +11,11 @@
 //
 // What bounds it: the matrix cores (256 float32 operations a clock and compute unit) from about 100 rows on, the weights'
 // way from memory below.  Wavefronts that share K instead of the tile fetch nothing twice in a workgroup and walk without
-// a barrier; the next blocks are asked for before these are multiplied.  Measured, weight rows x K at a number of rows,
-// against scalar multiply-adds on a 64 x 64 tile in LDS (16 k a barrier), in us: 2,048 x 8,192 at 333 rows 830 -> 105
-// (106 TFLOP/s), 16,384 x 2,048 at 333 rows 699 -> 202 (110), 2,048 x 8,192 at 1,024 rows 271 (127), 32,000 x 2,048 at one
-// row 276 -> 55 (4.7 TB/s).  The error against 64 bits halves (K of 2,048: 8e-7 -> 4e-7): four shorter sums.
+// a barrier; the next blocks are asked for before these are multiplied.  Measured against scalar multiply-adds on a 64 x 64 tile
+// in LDS (16 k a barrier): 2,048 x 8,192 at 333 rows 830 -> 105 us (106 TFLOP/s).  The error against 64 bits is half that of one sum
+// (K of 2,048: 8e-7 -> 4e-7): four shorter sums.
 #include "common.h"
+#include "gemm_split.h"
 #include "tile_loop.h"
 
 namespace {
@@ -428,8 +428,8 @@ void launch(GemmArgs a, hipStream_t stream) {
 
 }  // namespace
 
-extern "C" int pulse_gemm_f32(const void* A, int a_dtype, const void* W, int w_dtype, void* C, int c_dtype,
-                              int M, int N, int K, int64_t lda, int64_t ldw, int64_t ldc, hipStream_t stream) {
+static int gemm_f32(const void* A, int a_dtype, const void* W, int w_dtype, void* C, int c_dtype, int M, int N, int K, int64_t lda,
+                    int64_t ldw, int64_t ldc, void* scratch, hipStream_t stream) {
     PULSE_REQUIRE(M >= 0 && N > 0 && K > 0, "gemm_f32: bad sizes M=%d N=%d K=%d", M, N, K);
     PULSE_REQUIRE(lda >= K && ldw >= K && ldc >= N, "gemm_f32: leading dimensions too small");
     PULSE_REQUIRE(pulse_dtype_ok(a_dtype) && pulse_dtype_ok(w_dtype) && pulse_dtype_ok(c_dtype), "gemm_f32: bad dtype tag");
@@ -443,6 +443,12 @@ extern "C" int pulse_gemm_f32(const void* A, int a_dtype, const void* W, int w_d
     const int a_size = a_dtype == PULSE_BF16 ? 2 : 4, w_size = w_dtype == PULSE_BF16 ? 2 : 4;
     const bool vec = K % 4 == 0 && lda % 4 == 0 && ldw % 4 == 0 && reinterpret_cast<uintptr_t>(A) % (4 * a_size) == 0 &&
                      reinterpret_cast<uintptr_t>(W) % (4 * w_size) == 0;
+    if (a_size == 4 && w_size == 4 && vec && pulse_split_takes(N, K)) {
+        pulse_split_launch(static_cast<const float*>(A), static_cast<const float*>(W), C, a.c_bf16 != 0, wide, M, N, K, lda, ldw, ldc,
+                           ldw < (1 << 25) ? scratch : nullptr, -1, stream);
+        PULSE_LAUNCH_CHECK("gemm_f32");
+        return 0;
+    }
     // Up to 16 rows a product is the weights' way from memory: tiles of one block of weight rows with four blocks of k a
     // stage, four blocks of weight rows where there are enough of them for every compute unit (16,384 x 2,048 at 12 rows
     // 38 -> 30 us; 2,048 x 8,192 29 -> 74).
@@ -474,4 +480,21 @@ extern "C" int pulse_gemm_f32(const void* A, int a_dtype, const void* W, int w_d
     }
     PULSE_LAUNCH_CHECK("gemm_f32");
     return 0;
+}
+
+extern "C" int pulse_gemm_f32(const void* A, int a_dtype, const void* W, int w_dtype, void* C, int c_dtype,
+                              int M, int N, int K, int64_t lda, int64_t ldw, int64_t ldc, hipStream_t stream) {
+    return gemm_f32(A, a_dtype, W, w_dtype, C, c_dtype, M, N, K, lda, ldw, ldc, nullptr, stream);
+}
+
+// How many bytes of scratch make the product of float32 operands of these sizes fastest (0: none).
+extern "C" int64_t pulse_gemm_f32_scratch(int M, int N, int K) { return M > 0 && N > 0 && K > 0 && K % 4 == 0 ? pulse_split_scratch(M, N, K) : 0; }
+
+// The same product, bit for bit, with that many bytes of scratch.
+extern "C" int pulse_gemm_f32_scratched(const void* A, int a_dtype, const void* W, int w_dtype, void* C, int c_dtype, int M, int N, int K,
+                                        int64_t lda, int64_t ldw, int64_t ldc, void* scratch, int64_t scratch_bytes, hipStream_t stream) {
+    PULSE_REQUIRE(scratch != nullptr && reinterpret_cast<uintptr_t>(scratch) % 16 == 0, "gemm_f32: the scratch must be 16-byte aligned");
+    PULSE_REQUIRE(scratch_bytes >= pulse_gemm_f32_scratch(M, N, K), "gemm_f32: %lld bytes of scratch, %lld are needed",
+                  static_cast<long long>(scratch_bytes), static_cast<long long>(pulse_gemm_f32_scratch(M, N, K)));
+    return gemm_f32(A, a_dtype, W, w_dtype, C, c_dtype, M, N, K, lda, ldw, ldc, scratch, stream);
 }

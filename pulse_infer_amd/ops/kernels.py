@@ -3,7 +3,8 @@
 Each function checks on the host that devices, storage types, shapes and
 strides are what its kernel assumes, then launches on torch's current stream.
 Tensors are passed as raw device pointers; nothing here allocates unless a
-result tensor is asked for, and nothing falls back to another implementation.
+result tensor is asked for (or, ``gemm_f32`` of many rows, scratch from torch's
+pool), and nothing falls back to another implementation.
 """
 from __future__ import annotations
 
@@ -257,9 +258,23 @@ def gemm_f32(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor) -> None:
     _need(k == k2, f"gemm_f32: inner sizes differ: a is [{m}, {k}], w is [{n}, {k2}]")
     _need(tuple(out.shape) == (m, n), f"gemm_f32: out must be [{m}, {n}], got {tuple(out.shape)}")
     _need(a.stride(1) == 1 and w.stride(1) == 1 and out.stride(1) == 1, "gemm_f32: rows must be contiguous")
-    call("pulse_gemm_f32", _ptr(a), _i32(_tag(a, "gemm_f32")), _ptr(w), _i32(_tag(w, "gemm_f32")), _ptr(out),
-         _i32(_tag(out, "gemm_f32")), _i32(m), _i32(n), _i32(k), _i64(a.stride(0) if m > 1 else k),
-         _i64(w.stride(0) if n > 1 else k), _i64(out.stride(0) if m > 1 else n), _stream())
+    args = (_ptr(a), _i32(_tag(a, "gemm_f32")), _ptr(w), _i32(_tag(w, "gemm_f32")), _ptr(out), _i32(_tag(out, "gemm_f32")),
+            _i32(m), _i32(n), _i32(k), _i64(a.stride(0) if m > 1 else k), _i64(w.stride(0) if n > 1 else k),
+            _i64(out.stride(0) if m > 1 else n))
+    size = _gemm_f32_scratch(m, n, k) if a.dtype == w.dtype == torch.float32 else 0
+    if size:     # from torch's pool, which hands it out again in the order of this stream
+        scratch = torch.empty(size, dtype=torch.uint8, device=a.device)
+        call("pulse_gemm_f32_scratched", *args, _ptr(scratch), _i64(size), _stream())
+    else:
+        call("pulse_gemm_f32", *args, _stream())
+
+
+@functools.lru_cache(maxsize=1024)
+def _gemm_f32_scratch(m: int, n: int, k: int) -> int:
+    """Bytes of scratch that make a product of float32 operands of these sizes fastest (0: none)."""
+    entry = library.load().pulse_gemm_f32_scratch
+    entry.restype = ctypes.c_int64
+    return entry(_i32(m), _i32(n), _i32(k))
 
 
 SKINNY_MAX_ROWS = 64           # what the kernel takes
