@@ -17,6 +17,7 @@ typedef __attribute__((ext_vector_type(8))) __bf16 tile_bf16x8;
 typedef __attribute__((ext_vector_type(4))) __bf16 tile_bf16x4;
 typedef __attribute__((ext_vector_type(16))) float tile_f32x16;
 
+
 template <int WR, int XR, int WN, int WM, int S, bool NT = false, int SX = S>
 struct TileLoop {
     static constexpr int BK = 64;
@@ -28,6 +29,12 @@ struct TileLoop {
     static constexpr int PER = PER_W + PER_X;
     static constexpr int KK = BK / 16;                               // products of the matrix instruction's depth a step
     static constexpr int LDS = X0 + SX * STAGE_X;
+    // The next products' operand reads go out between these, over the first READS of them, so that the last is here in time: a
+    // lone wavefront a SIMD issues no product while it issues reads.  (All of them ahead of the products, 24,576 x 4,096 with
+    // SwiGLU alone: 357 rows in tiles of 192 x 192 74 us, so 70; 509 rows in 192 x 256 91 and 86.  Inside a step, at the power
+    // limit, a prompt of 509 gains 0.6 %.)  Where a step has few products the reads go ahead of them (0): behind the first they
+    // are late (experts of 8 tokens in 64 x 32, a step 1 % slower).
+    static constexpr int READS = TN * TM < 6 ? 0 : TN * TM == 6 ? 4 : TN * TM - 3;
     static_assert(WR % (8 * NW) == 0 && XR % (8 * NW) == 0 && TN >= 1 && TM >= 1 && SX >= 2 && S >= SX,
                   "whole chunks and pieces a wavefront");
 
@@ -86,34 +93,43 @@ struct TileLoop {
 #pragma unroll
         for (int j = 0; j < FIRST; ++j) copy(S - 1, S - 1, SX - 1, SX - 1, j);
         tile_bf16x8 wf[2][TN], xf[2][TM];
-        auto read = [&](int slot_w, int slot_x, int kk, int buf) __attribute__((always_inline)) {
-#pragma unroll
-            for (int g = 0; g < TM; ++g) xf[buf][g] = *reinterpret_cast<const tile_bf16x8*>(lds + slot_x * STAGE_X + x_at[kk] + g * 32 * ROW_BYTES);
-#pragma unroll
-            for (int f = 0; f < TN; ++f) wf[buf][f] = *reinterpret_cast<const tile_bf16x8*>(lds + slot_w * STAGE_W + w_at[kk] + f * 32 * ROW_BYTES);
-        };
         asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" : : "n"(LATER + FIRST) : "memory");
-        read(0, 0, 0, 0);
+#pragma unroll
+        for (int g = 0; g < TM; ++g) xf[0][g] = *reinterpret_cast<const tile_bf16x8*>(lds + x_at[0] + g * 32 * ROW_BYTES);
+#pragma unroll
+        for (int f = 0; f < TN; ++f) wf[0][f] = *reinterpret_cast<const tile_bf16x8*>(lds + w_at[0] + f * 32 * ROW_BYTES);
         int sw = 0, sx = 0;
         for (int s = 0; s < steps; ++s) {
             const int next_w = sw == S - 1 ? 0 : sw + 1, before_w = sw == 0 ? S - 1 : sw - 1;
             const int next_x = sx == SX - 1 ? 0 : sx + 1, before_x = sx == 0 ? SX - 1 : sx - 1;
 #pragma unroll
             for (int kk = 0; kk < KK; ++kk) {
+                const int buf = kk & 1, then = kk == KK - 1 ? 0 : kk + 1;
+                const char* const lds_w = lds + (kk == KK - 1 ? next_w : sw) * STAGE_W + w_at[then];
+                const char* const lds_x = lds + (kk == KK - 1 ? next_x : sx) * STAGE_X + x_at[then];
                 __builtin_amdgcn_sched_barrier(0);
-                if (kk == KK - 1) {
-                    // this wavefront's copies of the next step have landed and its operands are here; behind the barrier
-                    // that holds for everyone
-                    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"(LATER) : "memory");
-                    read(next_w, next_x, 0, (kk + 1) & 1);
-                } else {
-                    read(sw, sx, kk + 1, (kk + 1) & 1);
+                // before a step's last products: this wavefront's copies of the next step have landed and its operands are
+                // here; behind the barrier that holds for everyone
+                if (kk == KK - 1) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"(LATER) : "memory");
+                // (the operands of the products behind these, in the order in which those ask for them)
+                auto read = [&](int i) __attribute__((always_inline)) {
+                    if (i < TM) xf[buf ^ 1][i] = *reinterpret_cast<const tile_bf16x8*>(lds_x + i * 32 * ROW_BYTES);
+                    else wf[buf ^ 1][i - TM] = *reinterpret_cast<const tile_bf16x8*>(lds_w + (i - TM) * 32 * ROW_BYTES);
+                };
+                if constexpr (READS == 0) {
+#pragma unroll
+                    for (int i = 0; i < TN + TM; ++i) read(i);
                 }
                 __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                 for (int p = 0; p < TN * TM; ++p) {
-                    acc[p / TM][p % TM] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[kk & 1][p / TM], xf[kk & 1][p % TM],
+                    acc[p / TM][p % TM] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[buf][p / TM], xf[buf][p % TM],
                                                                                   acc[p / TM][p % TM], 0, 0, 0);
+                    __builtin_amdgcn_sched_barrier(0);
+                    if constexpr (READS > 0) {
+#pragma unroll
+                        for (int i = min(p, READS) * (TN + TM) / READS; i < min(p + 1, READS) * (TN + TM) / READS; ++i) read(i);
+                    }
                     __builtin_amdgcn_sched_barrier(0);
                     // the copies, spread evenly over the products
                     const int q = (kk == KK - 1 ? 0 : kk + 1) * TN * TM + p;
