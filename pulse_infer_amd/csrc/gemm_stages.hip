@@ -75,7 +75,7 @@ __global__ __launch_bounds__(256) void gemm_stages_kernel(StageArgs a) {
                   k0 + Loop::piece_of(row, lane) * 8;
     }
     Loop loop;
-    loop.run(from, lds, wave, lane, a.K);
+    loop.run(from, lds, wave, lane, a.K, MODE == OUT_SWIGLU ? tile_first_step(n0 / TILE_BLOCK, a.K / Loop::BK) : 0);
 
     // Results leave through LDS, a wavefront's 32 rows at a time, in whole 16-byte pieces of rows.
     constexpr int TN = Loop::TN, TM = Loop::TM;

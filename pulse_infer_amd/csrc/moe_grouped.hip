@@ -424,7 +424,8 @@ __global__ __launch_bounds__(WN* WM* PULSE_WAVE) void moe_tile_kernel(GroupArgs 
         }
     }
     Loop loop;
-    loop.run(from, lds, wave, lane, a.K);
+    constexpr int BLOCK = DOWN ? TILE_BLOCK : TILE_BLOCK / 2;
+    loop.run(from, lds, wave, lane, a.K, tile_first_step(e * ((a.N + BLOCK - 1) / BLOCK) + n0 / BLOCK, a.K / Loop::BK));
 
     // Results leave through LDS, a wavefront's 32 rows at a time, in whole 16-byte pieces of rows.
     constexpr int TN = Loop::TN, TM = Loop::TM;

@@ -18,6 +18,14 @@ typedef __attribute__((ext_vector_type(4))) __bf16 tile_bf16x4;
 typedef __attribute__((ext_vector_type(16))) float tile_f32x16;
 
 
+// Where along K (of so many steps) the tiles of a block of TILE_BLOCK weight rows start.  Rows of a power of two bytes, at the
+// same place in all of a launch's workgroups at a time, fall on few of the memory's channels; blocks that start elsewhere, in
+// turns of five steps, spread over them.  A function of the weight's row alone, and every tile lies inside a block: a result's
+// sums have one order, whatever the tile.  (24,576 x 4,096 with SwiGLU: 70 / 97 / 128 rows 44 / 45.5 / 47 us -> 37.5 / 38.6 / 41,
+// more rows the same; the 8B shape's other products lose or gain less than half a microsecond.)
+constexpr int TILE_BLOCK = 768;
+__device__ __forceinline__ int tile_first_step(int block, int steps) { return static_cast<int>(block * 5u % static_cast<uint32_t>(steps)); }
+
 template <int WR, int XR, int WN, int WM, int S, bool NT = false, int SX = S>
 struct TileLoop {
     static constexpr int BK = 64;
@@ -37,6 +45,7 @@ struct TileLoop {
     static constexpr int READS = TN * TM < 6 ? 0 : TN * TM == 6 ? 4 : TN * TM - 3;
     static_assert(WR % (8 * NW) == 0 && XR % (8 * NW) == 0 && TN >= 1 && TM >= 1 && SX >= 2 && S >= SX,
                   "whole chunks and pieces a wavefront");
+    static_assert(TILE_BLOCK % WR == 0, "a tile lies inside a block of weight rows");
 
     // Piece c (16 bytes) of row r of a stage sits at place c ^ swz(r): the rows that neighbouring lanes read together then
     // lie in different places of what LDS serves at once.
@@ -50,18 +59,22 @@ struct TileLoop {
     }
     static __device__ __forceinline__ int piece_of(int row, int lane) { return (lane % 8) ^ swz(row); }
 
-    // from[j]: where that piece lies in memory at k = 0.
-    __device__ __forceinline__ void run(const bf16_t* const (&from)[PER], char* lds, int wave, int lane, int K) {
+    // from[j]: where that piece lies in memory at k = 0.  The walk along K starts at step `first` and goes round its end.
+    __device__ __forceinline__ void run(const bf16_t* const (&from)[PER], char* lds, int wave, int lane, int K, int first = 0) {
         const int wave_n = wave % WN, wave_m = wave / WN;
         const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(
             (void __attribute__((address_space(3)))*)(lds)));
         const int steps = K / BK;
+        auto place = [&](int step) __attribute__((always_inline)) {      // (steps past the last: copies that nobody reads)
+            const int at = min(step, steps - 1) + first;
+            return (at >= steps ? at - steps : at) * BK;
+        };
         // The j-th copy of a batch, X first; a batch: W of one step into its slot, X of another into its.
         auto copy = [&](int step_w, int slot_w, int step_x, int slot_x, int j) __attribute__((always_inline)) {
             if (j < PER_X) {
-                load_to_lds(from[PER_W + j] + min(step_x, steps - 1) * BK, lds0 + X0 + slot_x * STAGE_X + (wave * PER_X + j) * 1024);
+                load_to_lds(from[PER_W + j] + place(step_x), lds0 + X0 + slot_x * STAGE_X + (wave * PER_X + j) * 1024);
             } else {
-                const bf16_t* at = from[j - PER_X] + min(step_w, steps - 1) * BK;
+                const bf16_t* at = from[j - PER_X] + place(step_w);
                 const uint32_t to = lds0 + slot_w * STAGE_W + (wave * PER_W + j - PER_X) * 1024;
                 if constexpr (NT) stream_to_lds(at, to);
                 else load_to_lds(at, to);

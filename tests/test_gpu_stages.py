@@ -200,3 +200,20 @@ def test_updates_in_shares_make_no_batched_product(rows, n, policy, monkeypatch)
     bound = (k + 2) * 2.0 ** -24 * torch.mm(x.double().abs(), w.double().abs().t())     # as above, the shares' sum in 64 bits
     assert parts.dtype == torch.float32 and parts.shape[1:] == (rows, n)
     assert ((parts.double().sum(0) - want).abs() <= bound).all()
+
+
+def test_gate_and_up_in_stages_do_not_depend_on_the_rows_beside_them():
+    """Where a block of weight rows starts its walk along K is a matter of the weight alone: every tile, the same bits."""
+    from pulse_infer_amd.ops import kernels
+
+    n, k = 24608, 64 * STEPS
+    x, w, _, _ = product(600, n, k)
+    whole = torch.empty((600, n // 2), dtype=torch.bfloat16, device=DEV)
+    kernels.gemm_stages(x, w, whole, swiglu=True)
+    tiles = set()
+    for m in (1, 65, 97, 130, 193, 357, 509):
+        tiles.add(kernels.gemm_stages_tile(m, n, k))
+        act = torch.full((m, n // 2), float("nan"), dtype=torch.bfloat16, device=DEV)
+        kernels.gemm_stages(x[:m], w, act, swiglu=True)
+        assert torch.equal(act, whole[:m]), m
+    assert len(tiles) >= 4
