@@ -251,8 +251,7 @@ __global__ __launch_bounds__(256, DB == 2 ? 5 : DB == 4 ? 4 : 1) void attn_rows_
             s[e] = seen[e] ? s[e] : -INFINITY;
             top = fmaxf(top, s[e]);
         }
-        top = fmaxf(top, __shfl_xor(top, 16, PULSE_WAVE));
-        top = fmaxf(top, __shfl_xor(top, 32, PULSE_WAVE));
+        top = across_rows(top, LaneMax());
         const float m_new = fmaxf(m, top);
         const float alpha = m_new == -INFINITY ? 1.f : expf(m - m_new);
         f32x4 p;
@@ -320,8 +319,7 @@ __global__ __launch_bounds__(256, DB == 2 ? 5 : DB == 4 ? 4 : 1) void attn_rows_
     }
     live = live && took;
 
-    l += __shfl_xor(l, 16, PULSE_WAVE);
-    l += __shfl_xor(l, 32, PULSE_WAVE);
+    l = across_rows(l, LaneSum());
     if (kg == 0) {
         m_s[wave][r] = m;
         l_s[wave][r] = l;

@@ -173,8 +173,7 @@ __global__ __launch_bounds__(256, PER_SIMD) void attn_wide_kernel(const bf16_t* 
                     v[t][i] = seen ? x : -INFINITY;
                     mx = fmaxf(mx, v[t][i]);
                 }
-            mx = fmaxf(mx, __shfl_xor(mx, 16, PULSE_WAVE));
-            mx = fmaxf(mx, __shfl_xor(mx, 32, PULSE_WAVE));
+            mx = across_rows(mx, LaneMax());
             const float m_new = fmaxf(m_run[rr], mx);
             alpha[rr] = (m_new == -INFINITY) ? 1.f : expf(m_run[rr] - m_new);
             float sum = 0.f;
@@ -228,8 +227,7 @@ __global__ __launch_bounds__(256, PER_SIMD) void attn_wide_kernel(const bf16_t* 
 #pragma unroll
     for (int rr = 0; rr < R; ++rr) {
         float l = l_run[rr];
-        l += __shfl_xor(l, 16, PULSE_WAVE);
-        l += __shfl_xor(l, 32, PULSE_WAVE);
+        l = across_rows(l, LaneSum());
         __syncthreads();   // (the row tile before has been read)
         if (g == 0) { ml[wave][r][0] = m_run[rr]; ml[wave][r][1] = l; }
         __syncthreads();

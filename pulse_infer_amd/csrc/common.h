@@ -74,16 +74,74 @@ template <typename T> __device__ __forceinline__ T from_f32(float v);
 template <> __device__ __forceinline__ float from_f32<float>(float v) { return v; }
 template <> __device__ __forceinline__ bf16_t from_f32<bf16_t>(float v) { return f32_to_bf16(v); }
 
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-    for (int off = PULSE_WAVE / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, PULSE_WAVE);
-    return v;
+// The two operands of a step of a reduction over the wavefront: what lanes i and i ^ STEP hold, the same pair (in one order or the
+// other) for both.  Steps go 32, 16, 8, 4, 2, 1; below 8 the pair is right once the steps before have been taken (lanes that
+// differ in the higher bits then hold the same).  By lane moves in the vector unit: a trip through LDS, which `__shfl_xor` takes,
+// is waited for six times a sum.  (Steps of the 8B shape, the same bits: decoding 32 requests 4,786 -> 4,744 us, one 3,265 -> 3,242,
+// 24 beside a portion of 333 tokens 8,996 -> 8,834, the norms, the attention's maxima and the sums of squares among it.)
+struct WaveTwo { uint32_t a, b; };
+template <int STEP>
+__device__ __forceinline__ WaveTwo wave_two(uint32_t v) {
+    if constexpr (STEP == 32 || STEP == 16) {
+        const auto both = STEP == 32 ? __builtin_amdgcn_permlane32_swap(v, v, false, false) : __builtin_amdgcn_permlane16_swap(v, v, false, false);
+        return {both[0], both[1]};
+    } else {
+        return {v, static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x120 + STEP /* row_ror:STEP */, 0xF, 0xF, true))};
+    }
 }
 
-__device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-    for (int off = PULSE_WAVE / 2; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, PULSE_WAVE));
+// op over all lanes, lanes 32 apart first (every lane gets it; op must not care for its operands' order)
+template <typename T, typename F>
+__device__ __forceinline__ T wave_reduce(T v, F op) {
+    static_assert(sizeof(T) == 4, "a register a lane");
+    auto step = [&](WaveTwo t) __attribute__((always_inline)) { v = op(__builtin_bit_cast(T, t.a), __builtin_bit_cast(T, t.b)); };
+    step(wave_two<32>(__builtin_bit_cast(uint32_t, v)));
+    step(wave_two<16>(__builtin_bit_cast(uint32_t, v)));
+    step(wave_two<8>(__builtin_bit_cast(uint32_t, v)));
+    step(wave_two<4>(__builtin_bit_cast(uint32_t, v)));
+    step(wave_two<2>(__builtin_bit_cast(uint32_t, v)));
+    step(wave_two<1>(__builtin_bit_cast(uint32_t, v)));
     return v;
+}
+// op over the sixteen lanes of a row of lanes, 8 apart first.
+template <typename F>
+__device__ __forceinline__ float row_reduce(float v, F op) {
+    auto step = [&](WaveTwo t) __attribute__((always_inline)) { v = op(__uint_as_float(t.a), __uint_as_float(t.b)); };
+    step(wave_two<8>(__float_as_uint(v)));
+    step(wave_two<4>(__float_as_uint(v)));
+    step(wave_two<2>(__float_as_uint(v)));
+    step(wave_two<1>(__float_as_uint(v)));
+    return v;
+}
+// op over the four lanes that hold the same place of their row of sixteen, neighbouring rows first.
+template <typename F>
+__device__ __forceinline__ float across_rows(float v, F op) {
+    const WaveTwo near = wave_two<16>(__float_as_uint(v));
+    const WaveTwo far = wave_two<32>(__float_as_uint(op(__uint_as_float(near.a), __uint_as_float(near.b))));
+    return op(__uint_as_float(far.a), __uint_as_float(far.b));
+}
+struct LaneSum { __device__ __forceinline__ float operator()(float a, float b) const { return a + b; } };
+struct LaneMax { __device__ __forceinline__ float operator()(float a, float b) const { return fmaxf(a, b); } };
+__device__ __forceinline__ float wave_sum(float v) { return wave_reduce(v, LaneSum()); }
+__device__ __forceinline__ float wave_max(float v) { return wave_reduce(v, LaneMax()); }
+
+__device__ __forceinline__ int wave_sum(int v) { return wave_reduce(v, [](int a, int b) { return a + b; }); }
+
+// The largest value over all lanes and its number, the lowest among equals (numbers only: no NaN).
+__device__ __forceinline__ void wave_argmax(float& v, int& i) {
+    auto step = [&](WaveTwo x, WaveTwo n) __attribute__((always_inline)) {
+        const float a = __uint_as_float(x.a), b = __uint_as_float(x.b);
+        const int ia = static_cast<int>(n.a), ib = static_cast<int>(n.b);
+        const bool second = b > a || (b == a && ib < ia);
+        v = second ? b : a;
+        i = second ? ib : ia;
+    };
+    step(wave_two<32>(__float_as_uint(v)), wave_two<32>(static_cast<uint32_t>(i)));
+    step(wave_two<16>(__float_as_uint(v)), wave_two<16>(static_cast<uint32_t>(i)));
+    step(wave_two<8>(__float_as_uint(v)), wave_two<8>(static_cast<uint32_t>(i)));
+    step(wave_two<4>(__float_as_uint(v)), wave_two<4>(static_cast<uint32_t>(i)));
+    step(wave_two<2>(__float_as_uint(v)), wave_two<2>(static_cast<uint32_t>(i)));
+    step(wave_two<1>(__float_as_uint(v)), wave_two<1>(static_cast<uint32_t>(i)));
 }
 
 // Sum over a block of up to 1024 threads; `scratch` holds one float per wave (>= 16).

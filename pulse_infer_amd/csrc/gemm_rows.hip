@@ -225,8 +225,7 @@ __global__ __launch_bounds__(SL* KW* PULSE_WAVE) void gemm_rows_kernel(RowsArgs 
             }
         }
         if (a.sumsq_out) {   // the four lanes of a row hold its 16 columns
-            sq += __shfl_xor(sq, 16, PULSE_WAVE);
-            sq += __shfl_xor(sq, 32, PULSE_WAVE);
+            sq = across_rows(sq, LaneSum());
             if (kg == 0 && m < M && n_base < N) a.sumsq_out[static_cast<int64_t>(m) * a.parts_out + n_base / 16] = sq;
         }
     }

@@ -109,10 +109,7 @@ __device__ __forceinline__ void epilogue(float (*red)[SLABS * MT][16][17], void*
             }
             if (sumsq) {  // the 16 lanes of a row of lanes hold the 16 columns of one row of the tile
                 float sq = updated * updated;
-                sq += __shfl_xor(sq, 8, 16);
-                sq += __shfl_xor(sq, 4, 16);
-                sq += __shfl_xor(sq, 2, 16);
-                sq += __shfl_xor(sq, 1, 16);
+                sq = row_reduce(sq, LaneSum());
                 // (a slab that lies beyond N altogether, the second of a pair when N is no multiple of 32, has no part)
                 if (n_in == 0 && m < M && n_base + (tile / MT) * 16 < N)
                     sumsq[static_cast<int64_t>(m) * parts + n_base / 16 + tile / MT] = sq;

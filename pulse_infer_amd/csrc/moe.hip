@@ -115,12 +115,7 @@ __device__ __forceinline__ void route_row(const float* row, const TW* __restrict
             const int j = lane + r * PULSE_WAVE;
             if (c[r] > best || (c[r] == best && j < best_j && c[r] > -INFINITY)) { best = c[r]; best_j = j; }
         }
-#pragma unroll
-        for (int off = PULSE_WAVE / 2; off > 0; off >>= 1) {
-            const float ob = __shfl_xor(best, off, PULSE_WAVE);
-            const int oj = __shfl_xor(best_j, off, PULSE_WAVE);
-            if (ob > best || (ob == best && oj < best_j)) { best = ob; best_j = oj; }
-        }
+        wave_argmax(best, best_j);
         // the owner of best_j gives its score and retires the output
         float sc = 0.f;
 #pragma unroll

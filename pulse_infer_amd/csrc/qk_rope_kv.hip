@@ -300,8 +300,12 @@ __device__ __forceinline__ void qk_rope_rows(int t, int y, int lane, bf16_t* __r
         float ss = 0.f;
 #pragma unroll
         for (int i = 0; i < 8; ++i) ss += e[i] * e[i];
+        if constexpr (LPH == 16) {
+            ss = row_reduce(ss, LaneSum());
+        } else {
 #pragma unroll
-        for (int off = LPH / 2; off > 0; off >>= 1) ss += __shfl_xor(ss, off, PULSE_WAVE);
+            for (int off = LPH / 2; off > 0; off >>= 1) ss += __shfl_xor(ss, off, PULSE_WAVE);
+        }
         inv = 1.0f / sqrtf(ss / static_cast<float>(d) + a.eps);
 #pragma unroll
         for (int i = 0; i < 8; ++i) e[i] = e[i] * inv * wv[i];

@@ -102,8 +102,7 @@ __device__ float block_sum_f(float v, float* scratch) { return block_sum(v, scra
 
 __device__ float block_max_f(float v, float* scratch) {
     const int lane = threadIdx.x % PULSE_WAVE, wave = threadIdx.x / PULSE_WAVE;
-#pragma unroll
-    for (int off = PULSE_WAVE / 2; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, PULSE_WAVE));
+    v = wave_max(v);
     __syncthreads();
     if (lane == 0) scratch[wave] = v;
     __syncthreads();
@@ -114,8 +113,7 @@ __device__ float block_max_f(float v, float* scratch) {
 
 __device__ int block_sum_i(int v, int* scratch) {
     const int lane = threadIdx.x % PULSE_WAVE, wave = threadIdx.x / PULSE_WAVE;
-#pragma unroll
-    for (int off = PULSE_WAVE / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, PULSE_WAVE);
+    v = wave_sum(v);
     __syncthreads();
     if (lane == 0) scratch[wave] = v;
     __syncthreads();
@@ -127,12 +125,7 @@ __device__ int block_sum_i(int v, int* scratch) {
 // (value, index) maximum with the lowest index among equal values
 __device__ void block_argmax(float& v, int& idx, float* sv, int* si) {
     const int lane = threadIdx.x % PULSE_WAVE, wave = threadIdx.x / PULSE_WAVE;
-#pragma unroll
-    for (int off = PULSE_WAVE / 2; off > 0; off >>= 1) {
-        const float ov = __shfl_xor(v, off, PULSE_WAVE);
-        const int oi = __shfl_xor(idx, off, PULSE_WAVE);
-        if (ov > v || (ov == v && oi < idx)) { v = ov; idx = oi; }
-    }
+    wave_argmax(v, idx);
     __syncthreads();
     if (lane == 0) { sv[wave] = v; si[wave] = idx; }
     __syncthreads();
@@ -195,16 +188,6 @@ template <int PER>
 __device__ bool finish_on_list(const int* list_i, float* list_x, int n, bool by_k, int k, bool use_p, float p, float whole,
                                float best, float inv_t, float u, int best_i, int& token) {
     const int lane = threadIdx.x % PULSE_WAVE;
-    auto lane_sum_i = [&](int v) {
-#pragma unroll
-        for (int off = PULSE_WAVE / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, PULSE_WAVE);
-        return v;
-    };
-    auto lane_sum_f = [&](float v) {
-#pragma unroll
-        for (int off = PULSE_WAVE / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, PULSE_WAVE);
-        return v;
-    };
     uint32_t keys[PER];
     float wts[PER];
 #pragma unroll
@@ -221,14 +204,14 @@ __device__ bool finish_on_list(const int* list_i, float* list_x, int n, bool by_
             int c = 0;
 #pragma unroll
             for (int j = 0; j < PER; ++j) c += (lane + j * PULSE_WAVE < n && keys[j] >= cand) ? 1 : 0;
-            if (lane_sum_i(c) >= k) keep = cand;
+            if (wave_sum(c) >= k) keep = cand;
         }
     }
     if (use_p) {
         float mass = 0.f;
 #pragma unroll
         for (int j = 0; j < PER; ++j) mass += keys[j] >= keep ? wts[j] : 0.f;
-        mass = lane_sum_f(mass);
+        mass = wave_sum(mass);
         const float want = p * (by_k ? mass : whole);
         if (!by_k && !(mass >= want)) return false;   // without top-k the list must hold all of the top_p set
         uint32_t thr = 0u;
@@ -238,7 +221,7 @@ __device__ bool finish_on_list(const int* list_i, float* list_x, int n, bool by_
             float part_mass = 0.f;
 #pragma unroll
             for (int j = 0; j < PER; ++j) part_mass += keys[j] >= lim ? wts[j] : 0.f;
-            if (lane_sum_f(part_mass) >= want) thr = cand;
+            if (wave_sum(part_mass) >= want) thr = cand;
         }
         if (thr > keep) keep = thr;
     }
@@ -251,7 +234,7 @@ __device__ bool finish_on_list(const int* list_i, float* list_x, int n, bool by_
         if (e < n) list_x[e] = w;
         kept += w;
     }
-    kept = lane_sum_f(kept);
+    kept = wave_sum(kept);
     int last;
     const int e = wave_walk(0, n, u * kept, [&](int q) { return list_x[q]; }, last);
     token = e >= 0 ? list_i[e] : (last >= 0 ? list_i[last] : best_i);
@@ -497,8 +480,7 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
             constexpr int SHARE = HIST_BINS / SAMPLE_WAVES;
             int mine = 0;
             for (int b = wave * SHARE + lane; b < (wave + 1) * SHARE; b += PULSE_WAVE) mine += hist[b];
-#pragma unroll
-            for (int off = PULSE_WAVE / 2; off > 0; off >>= 1) mine += __shfl_xor(mine, off, PULSE_WAVE);
+            mine = wave_sum(mine);
             if (lane == 0) wave_bins[wave] = mine;
             __syncthreads();
             int w = 0;
@@ -638,8 +620,7 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
     // the kept mass of every wavefront's part, then the part in which the draw falls is walked by its wavefront
     float mine = 0.f;
     sweep(row, part_begin + lane, part_end, PULSE_WAVE, [&](int, float x) { mine += weight_of(x); });
-#pragma unroll
-    for (int off = PULSE_WAVE / 2; off > 0; off >>= 1) mine += __shfl_xor(mine, off, PULSE_WAVE);
+    mine = wave_sum(mine);
     if (lane == 0) part_sum[wave] = mine;
     __syncthreads();
     float kept = 0.f;
@@ -697,12 +678,7 @@ __global__ __launch_bounds__(ARGMAX_THREADS) void argmax_chunks_kernel(const flo
         if (x > best) { best = x; best_i = i; }   // NaN never wins; ascending i keeps the lowest index among equals
     }
     const int lane = threadIdx.x % PULSE_WAVE, wave = threadIdx.x / PULSE_WAVE;
-#pragma unroll
-    for (int off = PULSE_WAVE / 2; off > 0; off >>= 1) {
-        const float ov = __shfl_xor(best, off, PULSE_WAVE);
-        const int oi = __shfl_xor(best_i, off, PULSE_WAVE);
-        if (ov > best || (ov == best && oi < best_i)) { best = ov; best_i = oi; }
-    }
+    wave_argmax(best, best_i);
     if (lane == 0) { sv[wave] = best; si[wave] = best_i; }
     __syncthreads();
     if (threadIdx.x == 0) {
@@ -724,12 +700,7 @@ __global__ __launch_bounds__(PULSE_WAVE) void argmax_merge_kernel(const float* _
         const int i = part_idx[r * chunks + c];
         if (v > best || (v == best && i < best_i)) { best = v; best_i = i; }
     }
-#pragma unroll
-    for (int off = PULSE_WAVE / 2; off > 0; off >>= 1) {
-        const float ov = __shfl_xor(best, off, PULSE_WAVE);
-        const int oi = __shfl_xor(best_i, off, PULSE_WAVE);
-        if (ov > best || (ov == best && oi < best_i)) { best = ov; best_i = oi; }
-    }
+    wave_argmax(best, best_i);
     if (threadIdx.x == 0) out[r] = best_i == 0x7fffffff ? -1 : best_i;
 }
 
@@ -773,12 +744,7 @@ __global__ __launch_bounds__(SIMPLE_THREADS) void simple_max_kernel(
         if (x != -INFINITY) lowest = fminf(lowest, x);
     });
     const int lane = threadIdx.x % PULSE_WAVE, wave = threadIdx.x / PULSE_WAVE;
-#pragma unroll
-    for (int off = PULSE_WAVE / 2; off > 0; off >>= 1) {
-        const float ov = __shfl_xor(best, off, PULSE_WAVE);
-        const int oi = __shfl_xor(best_i, off, PULSE_WAVE);
-        if (ov > best || (ov == best && oi < best_i)) { best = ov; best_i = oi; }
-    }
+    wave_argmax(best, best_i);
     if (part_min) lowest = -wave_max(-lowest);
     if (lane == 0) { sv[wave] = best; si[wave] = best_i; sl[wave] = lowest; }
     __syncthreads();
@@ -798,8 +764,7 @@ __global__ __launch_bounds__(SIMPLE_THREADS) void simple_max_kernel(
 __device__ __forceinline__ float simple_row_max(const float* part_max, int chunks) {
     float best = -INFINITY;
     for (int c = threadIdx.x % PULSE_WAVE; c < chunks; c += PULSE_WAVE) best = fmaxf(best, part_max[c]);
-#pragma unroll
-    for (int off = PULSE_WAVE / 2; off > 0; off >>= 1) best = fmaxf(best, __shfl_xor(best, off, PULSE_WAVE));
+    best = wave_max(best);
     return best;
 }
 
@@ -824,8 +789,7 @@ __global__ __launch_bounds__(SIMPLE_THREADS) void simple_mass_kernel(
         if (x != -INFINITY) mass += expf((x - best) * inv_t);
     });
     const int lane = threadIdx.x % PULSE_WAVE, wave = threadIdx.x / PULSE_WAVE;
-#pragma unroll
-    for (int off = PULSE_WAVE / 2; off > 0; off >>= 1) mass += __shfl_xor(mass, off, PULSE_WAVE);
+    mass = wave_sum(mass);
     if (lane == 0) sf[wave] = mass;
     __syncthreads();
     if (threadIdx.x == 0) {
@@ -895,10 +859,7 @@ __global__ __launch_bounds__(SIMPLE_THREADS) void topk_collect_kernel(
         uint32_t bound = 0u;
         for (int bit = 31; bit >= 0; --bit) {
             const uint32_t cand = bound | (1u << bit);
-            int c = (keys[0] >= cand ? 1 : 0) + (keys[1] >= cand ? 1 : 0);
-#pragma unroll
-            for (int off = PULSE_WAVE / 2; off > 0; off >>= 1) c += __shfl_xor(c, off, PULSE_WAVE);
-            if (c >= k) bound = cand;
+            if (__builtin_popcountll(__ballot(keys[0] >= cand)) + __builtin_popcountll(__ballot(keys[1] >= cand)) >= k) bound = cand;
         }
         // back to the value whose key it is (a maximum of -inf, a chunk with nothing left, has the key of -inf)
         float value = -INFINITY;
@@ -907,8 +868,7 @@ __global__ __launch_bounds__(SIMPLE_THREADS) void topk_collect_kernel(
             const int c = lane + j * PULSE_WAVE;
             if (c < chunks && keys[j] == bound) value = part_max[r * chunks + c];
         }
-#pragma unroll
-        for (int off = PULSE_WAVE / 2; off > 0; off >>= 1) value = fmaxf(value, __shfl_xor(value, off, PULSE_WAVE));
+        value = wave_max(value);
         if (lane == 0) s_bound = value;
     }
     __syncthreads();
@@ -974,12 +934,7 @@ __global__ __launch_bounds__(PULSE_WAVE) void chunked_choose_kernel(
         const int i = part_idx[c];
         if (v > best || (v == best && i < best_i)) { best = v; best_i = i; }
     }
-#pragma unroll
-    for (int off = PULSE_WAVE / 2; off > 0; off >>= 1) {
-        const float ov = __shfl_xor(best, off, PULSE_WAVE);
-        const int oi = __shfl_xor(best_i, off, PULSE_WAVE);
-        if (ov > best || (ov == best && oi < best_i)) { best = ov; best_i = oi; }
-    }
+    wave_argmax(best, best_i);
     const float temp = temperature ? temperature[r] : 0.f;
     if (best_i == 0x7fffffff || !(temp > 0.f)) {   // everything banned or NaN, or the largest logit wins
         if (lane == 0) { out[r] = best_i == 0x7fffffff ? -1 : best_i; done[r] = 1; }
@@ -1010,8 +965,7 @@ __global__ __launch_bounds__(PULSE_WAVE) void chunked_choose_kernel(
         float whole = 0.f;   // without top-k: the mass of the whole row, chunk masses in chunk order
         if (!by_k) {
             for (int c = lane; c < chunks; c += PULSE_WAVE) whole += part_mass[c];
-#pragma unroll
-            for (int off = PULSE_WAVE / 2; off > 0; off >>= 1) whole += __shfl_xor(whole, off, PULSE_WAVE);
+            whole = wave_sum(whole);
         }
         const int64_t seg0 = (static_cast<int64_t>(r) * chunks + lane) * TOPK_SEGMENT;
         for (int e = 0; e < n0; ++e) { list_i[pre0 - n0 + e] = seg_i[seg0 + e]; list_x[pre0 - n0 + e] = seg_x[seg0 + e]; }
@@ -1033,8 +987,7 @@ __global__ __launch_bounds__(PULSE_WAVE) void chunked_choose_kernel(
     // a draw from the whole vocabulary: the chunk in which it falls, chunk masses in chunk order
     float total = 0.f;
     for (int c = lane; c < chunks; c += PULSE_WAVE) total += part_mass[c];
-#pragma unroll
-    for (int off = PULSE_WAVE / 2; off > 0; off >>= 1) total += __shfl_xor(total, off, PULSE_WAVE);
+    total = wave_sum(total);
     const float target = uniform[r] * total;
     float run = 0.f;
     int who = -1, last_chunk = -1;

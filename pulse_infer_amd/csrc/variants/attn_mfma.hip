@@ -253,8 +253,7 @@ __device__ __forceinline__ void prepare_head(bf16x8 (&x)[NCHUNK], const HeadTabl
             ss += f[ch][e] * f[ch][e];
         }
     if (normed) {
-        ss += __shfl_xor(ss, 16, PULSE_WAVE);
-        ss += __shfl_xor(ss, 32, PULSE_WAVE);
+        ss = across_rows(ss, LaneSum());
         const float inv = 1.0f / sqrtf(ss / static_cast<float>(D) + eps);
 #pragma unroll
         for (int ch = 0; ch < NCHUNK; ++ch)
@@ -568,8 +567,7 @@ __global__ __launch_bounds__(WAVES* PULSE_WAVE) PULSE_ATTN_WAVES_PER_EU void att
                 p[t][i] = v;
                 mx = fmaxf(mx, v);
             }
-        mx = fmaxf(mx, __shfl_xor(mx, 16, PULSE_WAVE));
-        mx = fmaxf(mx, __shfl_xor(mx, 32, PULSE_WAVE));
+        mx = across_rows(mx, LaneMax());
         const float m_new = fmaxf(m, mx);
         const float alpha = (m_new == -INFINITY) ? 1.f : exp2f(m - m_new);
         float psum = 0.f;
@@ -655,8 +653,7 @@ __global__ __launch_bounds__(WAVES* PULSE_WAVE) PULSE_ATTN_WAVES_PER_EU void att
     }
 
     // the column's sum sits in four lanes
-    l_part += __shfl_xor(l_part, 16, PULSE_WAVE);
-    l_part += __shfl_xor(l_part, 32, PULSE_WAVE);
+    l_part = across_rows(l_part, LaneSum());
     if (kg == 0) {
         s_m[wave][r] = m;
         s_l[wave][r] = l_part;
@@ -872,8 +869,7 @@ __global__ __launch_bounds__(WAVES* PULSE_WAVE) PULSE_ATTN_WAVES_PER_EU void att
                 mx = fmaxf(mx, v);
             }
         if (inner && !col_ok) mx = -INFINITY;
-        mx = fmaxf(mx, __shfl_xor(mx, 16, PULSE_WAVE));
-        mx = fmaxf(mx, __shfl_xor(mx, 32, PULSE_WAVE));
+        mx = across_rows(mx, LaneMax());
         const float m_new = fmaxf(m, mx);
         const bool dead = m_new == -INFINITY;  // no key of this column so far
         const float alpha = dead ? 1.f : __builtin_amdgcn_exp2f((m - m_new) * c2);
@@ -941,8 +937,7 @@ __global__ __launch_bounds__(WAVES* PULSE_WAVE) PULSE_ATTN_WAVES_PER_EU void att
         __syncthreads();
     }
 
-    l_part += __shfl_xor(l_part, 16, PULSE_WAVE);
-    l_part += __shfl_xor(l_part, 32, PULSE_WAVE);
+    l_part = across_rows(l_part, LaneSum());
     if (col_ok) {
         l_part = with_sink(l_part, m == -INFINITY ? -INFINITY : m * c2, a.sink, col_head);
         const float inv = gated(l_part > 0.f ? 1.0f / l_part : 0.f, a.gate, a.gate_stride, col_row, col_head, a.gate_width);
@@ -1238,8 +1233,7 @@ __global__ __launch_bounds__(NW* PULSE_WAVE) PULSE_WIDE_WAVES_PER_EU void attn_p
             for (int t = 0; t < KT; ++t)
 #pragma unroll
                 for (int i = 0; i < 4; ++i) mx = fmaxf(mx, s[ct][t][i]);
-            mx = fmaxf(mx, __shfl_xor(mx, 16, PULSE_WAVE));
-            mx = fmaxf(mx, __shfl_xor(mx, 32, PULSE_WAVE));
+            mx = across_rows(mx, LaneMax());
             // The reference point of the exponents follows the maximum only when that has grown by more than
             // 2^LAZY_BITS in the weights' units: until then weights may exceed 1 (by at most that factor, which float32
             // sums and bfloat16 weights hold with the same relative precision), and the accumulators, which are most of
@@ -1338,8 +1332,7 @@ __global__ __launch_bounds__(NW* PULSE_WAVE) PULSE_WIDE_WAVES_PER_EU void attn_p
 #pragma unroll
     for (int ct = 0; ct < CT; ++ct) {
         float l = l_part[ct];
-        l += __shfl_xor(l, 16, PULSE_WAVE);
-        l += __shfl_xor(l, 32, PULSE_WAVE);
+        l = across_rows(l, LaneSum());
         if (col_ok[ct] && direct) {
             l = with_sink(l, m[ct] == -INFINITY ? -INFINITY : m[ct] * c2, a.sink, col_head);
             const float inv = gated(l > 0.f ? 1.0f / l : 0.f, a.gate, a.gate_stride, col_row[ct], col_head, a.gate_width);
