@@ -134,6 +134,20 @@ __device__ void block_argmax(float& v, int& idx, float* sv, int* si) {
         if (sv[w] > v || (sv[w] == v && si[w] < idx)) { v = sv[w]; idx = si[w]; }
 }
 
+// The sum of a step's 64 weights is the prefix's at its last lane, to the bit, and a third of the prefix's instructions without a trip
+// through LDS: the prefix is made for the step in which the sum comes near `rest` only (chunked_choose_kernel, 32 rows of 151,936,
+// 28 -> 22 us).
+__device__ __forceinline__ float pairs_sum(float v) {     // neighbours first, then pairs of neighbours, ..
+    const auto moved = [&](auto code) __attribute__((always_inline)) {
+        return __uint_as_float(static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, __float_as_int(v), decltype(code)::value, 0xF, 0xF, true)));
+    };
+    v += moved(Int<0xB1>());      // quad_perm [1, 0, 3, 2]
+    v += moved(Int<0x4E>());      // quad_perm [2, 3, 0, 1]
+    v += moved(Int<0x141>());     // row_half_mirror: the other four of eight
+    v += moved(Int<0x140>());     // row_mirror: the other eight of sixteen
+    return across_rows(v, LaneSum());
+}
+
 // ---- the walk along the cumulative sum, a wavefront over 64 consecutive entries at a time ---------------------
 // `weight(i)` is the weight of entry i of [begin, end) (0 for what is not kept), entries in vocabulary order.  The
 // wavefront finds the first entry at which the running sum exceeds `rest` and returns its number, or -1 if the sum
@@ -152,6 +166,9 @@ __device__ int wave_walk(int begin, int end, float rest, Weight weight, int& las
             const int i = first + u * PULSE_WAVE + lane;
             ws[u] = i < end ? weight(i) : 0.f;
         }
+        float sums[AHEAD];
+#pragma unroll
+        for (int u = 0; u < AHEAD; ++u) sums[u] = pairs_sum(ws[u]);
 #pragma unroll
         for (int u = 0; u < AHEAD; ++u) {
             const int base = first + u * PULSE_WAVE;
@@ -159,6 +176,11 @@ __device__ int wave_walk(int begin, int end, float rest, Weight weight, int& las
             const unsigned long long has = __ballot(w > 0.f);
             if (has == 0ull) continue;
             last = base + (63 - __builtin_clzll(has));
+            // (a prefix may round up to a few units in its last place beyond the sum)
+            if (!(rest < (run + sums[u]) * 1.00001f)) {
+                run += sums[u];
+                continue;
+            }
             // inclusive prefix over the lanes, in lane order
             float pre = w;
 #pragma unroll
@@ -241,132 +263,107 @@ __device__ bool finish_on_list(const int* list_i, float* list_x, int n, bool by_
     return true;
 }
 
-// What the kernels in front of sample_kernel leave of a row that the chunks could not choose for: the histogram's counts and
-// masses, then the mass of each of sample_kernel's wavefronts (as it would sum it) and the smallest number of each.
-constexpr int REST_MASS = 2 * HIST_BINS, REST_LOWEST = REST_MASS + SAMPLE_WAVES;
-constexpr int REST_WORDS = REST_LOWEST + SAMPLE_WAVES;
+// ---- top-p alone on rows whose share is no short list -------------------------------------------------------------
+// The masses here are whole numbers: an entry's weight, at most 1, in units of 2^-40 (2^-31 from 2^23 entries on, so that a row's
+// sum fits 64 bits).  Their sums are the same in any order, so a row's threshold and draw are one choice whoever sums, a
+// workgroup a row or many, and need no second pass over the row in one fixed order; and they are nearer to the exact masses
+// than float32 sums: 152,000 roundings of 2^-41 against sums good to 2^-24.
+typedef unsigned long long mass_t;
 
-__device__ __forceinline__ void add_in_group(float* p, float v) {
-    __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+struct Weigh {
+    float best, inv_t, low_scale;
+    int low;
+    __device__ __forceinline__ Weigh(float best_, float inv_t_, int vocab) : best(best_), inv_t(inv_t_) {
+        low = vocab < (1 << 23) ? 20 : 11;
+        low_scale = static_cast<float>(1 << low);
+    }
+    __device__ __forceinline__ mass_t operator()(float x) const {
+        const float w = expf((x - best) * inv_t) * 1048576.f;
+        const uint32_t high = static_cast<uint32_t>(w);      // (the rest of w is exact)
+        return (static_cast<mass_t>(high) << low) + static_cast<uint32_t>(rintf((w - static_cast<float>(high)) * low_scale));
+    }
+};
+
+__device__ __forceinline__ mass_t mass_sum(mass_t v) {
+#pragma unroll
+    for (int off = PULSE_WAVE / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, PULSE_WAVE);
+    return v;
 }
-
-constexpr int CANDIDATES = 15;   // most thresholds whose masses are summed side by side in a pass
-
-// The largest threshold t with M(t) >= want (see sample_kernel), from the histogram of a row under top-p alone; false where
-// the bracket does not hold it (or too many tokens share the bins), and then nothing is said.  Called by a whole workgroup.
-__device__ bool nucleus_edge(const RowView& row, float want, float best, float inv_t, float scale, const int* hist,
-                             const float* hist_w, float* sf, int* si, int* list_i, float* list_x, uint32_t* cand,
-                             unsigned long long* nearest, uint32_t& thr) {
-    const int lane = threadIdx.x % PULSE_WAVE, wave = threadIdx.x / PULSE_WAVE;
-    // the first bin at which the masses from the top reach `want`: thread t sums bins 2 t and 2 t + 1
-    constexpr int PER = HIST_BINS / SAMPLE_THREADS;
-    static_assert(PER == 2, "two bins a thread");
-    const float w0 = hist_w[2 * threadIdx.x], w1 = hist_w[2 * threadIdx.x + 1];
-    float pre = w0 + w1;
+// The sum over the lanes up to this one.
+__device__ __forceinline__ mass_t mass_through(mass_t v) {
 #pragma unroll
     for (int off = 1; off < PULSE_WAVE; off <<= 1) {
-        const float up = __shfl_up(pre, off, PULSE_WAVE);
-        if (lane >= off) pre += up;
+        const mass_t up = __shfl_up(v, off, PULSE_WAVE);
+        if (static_cast<int>(threadIdx.x % PULSE_WAVE) >= off) v += up;
     }
-    __syncthreads();
-    if (lane == PULSE_WAVE - 1) sf[wave] = pre;
-    if (threadIdx.x == 0) { si[0] = HIST_BINS; si[1] = 0; *nearest = ~0ull; }
-    __syncthreads();
-    float before = 0.f;
-    for (int w = 0; w < wave; ++w) before += sf[w];
-    const float through1 = before + pre, through0 = through1 - w1;     // masses through this thread's bins
-    if (through0 >= want) atomicMin(&si[0], 2 * static_cast<int>(threadIdx.x));
-    else if (through1 >= want) atomicMin(&si[0], 2 * static_cast<int>(threadIdx.x) + 1);
-    __syncthreads();
-    const int at = si[0];
-    if (at >= HIST_BINS) return false;
-    const int b0 = max(0, at - 1), b1 = min(HIST_BINS - 1, at + 1);
-    int count = 0;
-    for (int b = b0; b <= b1; ++b) count += hist[b];
-    if (count > LIST_CAP) return false;
-    float mine = 0.f;
-    for (int b = threadIdx.x; b < b0; b += SAMPLE_THREADS) mine += hist_w[b];
-    const float base = block_sum_f(mine, sf);       // the mass above the three bins
-    // their tokens, in any order: keys and weights
-    sweep(row, threadIdx.x, row.vocab, SAMPLE_THREADS, [&](int, float x) {
-        if (x == -INFINITY) return;
-        const int b = min(HIST_BINS - 1, static_cast<int>((best - x) * scale));
-        if (b < b0 || b > b1) return;
-        const int e = atomicAdd(&si[1], 1);
-        if (e < LIST_CAP) {
-            list_i[e] = static_cast<int>(order_key(x));
-            list_x[e] = expf((x - best) * inv_t);
-        }
-    });
-    __syncthreads();
-    const int n = si[1];
-    if (n > LIST_CAP || n == 0) return false;
-    // every token's place among them and the mass through it; of those that reach `want`, the one placed first
-    int place[LIST_CAP / SAMPLE_THREADS];
-    uint32_t keys[LIST_CAP / SAMPLE_THREADS];
-#pragma unroll
-    for (int u = 0; u < LIST_CAP / SAMPLE_THREADS; ++u) {
-        const int e = threadIdx.x + u * SAMPLE_THREADS;
-        place[u] = -1;
-        keys[u] = 0u;
-        if (e >= n) continue;
-        const uint32_t key = static_cast<uint32_t>(list_i[e]);
-        float through = base;
-        int higher = 0;
-        for (int j = 0; j < n; ++j) {
-            const uint32_t other = static_cast<uint32_t>(list_i[j]);
-            through += other >= key ? list_x[j] : 0.f;
-            higher += other > key ? 1 : 0;
-        }
-        place[u] = higher;
-        keys[u] = key;
-        if (through >= want) atomicMin(nearest, static_cast<unsigned long long>(higher));
-    }
-    __syncthreads();
-    if (*nearest == ~0ull) return false;
-    // M at the places round that one.  The histogram's masses are good to a few units in the last place of the whole, which is
-    // less than a token there unless the row is very flat: two places to either side first, seven where those do not hold it.
-    auto try_round = [&](auto count) __attribute__((always_inline)) {
-        constexpr int C = decltype(count)::value;
-        const int first = static_cast<int>(*nearest) - C / 2;
-        __syncthreads();
-        if (threadIdx.x < C) cand[threadIdx.x] = 0u;
-        __syncthreads();
-#pragma unroll
-        for (int u = 0; u < LIST_CAP / SAMPLE_THREADS; ++u)
-            if (place[u] >= first && place[u] >= 0 && place[u] < first + C) cand[place[u] - first] = keys[u];
-        __syncthreads();
-        // (equal tokens share a place, and the places behind it stay empty: 0)
-        uint32_t t[C], least = 0xffffffffu;
-        float above[C];
-#pragma unroll
-        for (int j = 0; j < C; ++j) {
-            t[j] = cand[j];
-            above[j] = 0.f;
-            if (t[j] != 0u && t[j] < least) least = t[j];
-        }
-        sweep(row, threadIdx.x, row.vocab, SAMPLE_THREADS, [&](int, float x) {
-            if (x == -INFINITY) return;
-            const uint32_t key = order_key(x);
-            if (key < least) return;
-            const float w = expf((x - best) * inv_t);
-#pragma unroll
-            for (int j = 0; j < C; ++j)
-                if (key >= t[j]) above[j] += w;
-        });
-        bool below = false, found = false, open = true;      // a larger candidate's mass falls short; the first that does not is known
-#pragma unroll
-        for (int j = 0; j < C; ++j) {
-            const float m = block_sum_f(above[j], sf);
-            if (t[j] == 0u || found || !open) continue;
-            if (m < want) below = true;
-            else if (below) { found = true; thr = t[j]; }
-            else open = false;                               // (the same for every thread)
-        }
-        return found;
-    };
-    return try_round(Int<5>()) || try_round(Int<CANDIDATES>());
+    return v;
 }
+
+// What the kernels in front of sample_kernel leave of a row that the chunks could not choose for, in 32-bit words: the histogram
+// over [lowest, best] (rows with top-k: counts; top-p alone: masses; 64 bits each), the row's smallest number, whether its token is
+// chosen after all, the mass of the bins above the one with top-p's edge, that of the row, and every chunk's of the former.
+constexpr int REST_LOWEST = 2 * HIST_BINS, REST_CHOSEN = REST_LOWEST + 1, REST_BASE = REST_LOWEST + 2, REST_WHOLE = REST_LOWEST + 4;
+constexpr int REST_CHUNKS = REST_LOWEST + 6, REST_MOST_CHUNKS = 2 * PULSE_WAVE;
+constexpr int REST_WORDS = REST_CHUNKS + 2 * REST_MOST_CHUNKS;
+static_assert(REST_WORDS % 2 == 0 && REST_CHUNKS % 2 == 0, "64-bit words");
+
+__device__ __forceinline__ int bin_at(float x, float best, float scale) { return min(HIST_BINS - 1, static_cast<int>((best - x) * scale)); }
+
+// The bin in which the masses from the top reach p of the whole (or, k > 0, the counts reach k), the mass above it and the whole:
+// thread t of THREADS sums HIST_BINS / THREADS neighbouring bins.  -1 if they do not.  Called by a whole workgroup.
+template <int THREADS>
+__device__ int edge_bin(const mass_t* hist, float p, int k, mass_t* waves, int* at, mass_t* above, mass_t& base, mass_t& whole) {
+    constexpr int PER = HIST_BINS / THREADS, WAVES = THREADS / PULSE_WAVE;
+    const int lane = threadIdx.x % PULSE_WAVE, wave = threadIdx.x / PULSE_WAVE;
+    mass_t bins[PER], mine = 0;
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+        bins[j] = hist[threadIdx.x * PER + j];
+        mine += bins[j];
+    }
+    const mass_t through = mass_through(mine);
+    if (lane == PULSE_WAVE - 1) waves[wave] = through;
+    if (threadIdx.x == 0) *at = -1;
+    __syncthreads();
+    mass_t before = through - mine;
+    whole = 0;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) {
+        if (w < wave) before += waves[w];
+        whole += waves[w];
+    }
+    const double want = k > 0 ? static_cast<double>(k) : static_cast<double>(p) * static_cast<double>(whole);
+    if (static_cast<double>(before) < want && static_cast<double>(before + mine) >= want) {      // one thread
+        int j = 0;
+        while (j < PER - 1 && static_cast<double>(before + bins[j]) < want) before += bins[j++];
+        *at = threadIdx.x * PER + j;
+        *above = before;
+    }
+    __syncthreads();
+    base = *above;
+    return *at;
+}
+
+// The largest of the keys at or above which the mass is at least p of the whole: `n` tokens of the edge's bin, `base` the mass
+// above it (the masses through the bin reach that share, so there is one).  Every token's own sum, no order: called by a whole workgroup,
+// `best` (LDS) cleared before and read behind a barrier.
+__device__ void edge_key(const uint32_t* keys, const mass_t* masses, int n, int threads, mass_t base, mass_t whole, float p, uint32_t* best) {
+    const double want = static_cast<double>(p) * static_cast<double>(whole);
+    for (int e = threadIdx.x; e < n; e += threads) {
+        const uint32_t key = keys[e];
+        mass_t through = base;
+        for (int j = 0; j < n; ++j) through += keys[j] >= key ? masses[j] : 0;
+        if (static_cast<double>(through) >= want) atomicMax(best, key);
+    }
+}
+
+// u of the kept mass, as a number below it.
+__device__ __forceinline__ mass_t draw_from(float u, mass_t kept) {
+    const mass_t t = static_cast<mass_t>(static_cast<double>(u) * static_cast<double>(kept));
+    return t < kept ? t : kept - 1;
+}
+
+constexpr int EDGE_CAP = 1024;   // tokens of the edge's bin that are ranked
 
 __global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
     const float* __restrict__ logits, int vocab, int64_t row_stride, const float* __restrict__ temperature,
@@ -376,9 +373,11 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
     const float* __restrict__ part_max, const int* __restrict__ part_idx, int chunks, const int* __restrict__ rest) {
     __shared__ float sf[SAMPLE_WAVES];
     __shared__ int si[SAMPLE_WAVES];
-    __shared__ int hist[HIST_BINS];
-    __shared__ float hist_w[HIST_BINS];     // top-p alone: the bins' masses (in the order of arrival: good for a bracket)
-    if (done && done[blockIdx.x]) return;   // the kernels that work in chunks have chosen this row's token already
+    __shared__ mass_t hist_m[HIST_BINS];    // top-p alone: the bins' masses
+    int* const hist = reinterpret_cast<int*>(hist_m);
+    if (rest) rest += static_cast<int64_t>(blockIdx.x) * REST_WORDS;
+    // the kernels that work in chunks have chosen this row's token already
+    if (done && (done[blockIdx.x] || (rest && rest[REST_CHOSEN]))) return;
     __shared__ int wave_bins[SAMPLE_WAVES];
     __shared__ int region_i[SAMPLE_WAVES][WAVE_CAP];
     __shared__ float region_x[SAMPLE_WAVES][WAVE_CAP];
@@ -387,8 +386,9 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
     __shared__ float list_x[LIST_CAP];
     __shared__ float part_sum[SAMPLE_WAVES];
     __shared__ int list_done;
-    __shared__ uint32_t cand[CANDIDATES];
-    __shared__ unsigned long long nearest;
+    __shared__ mass_t edge_m[EDGE_CAP], part_m[SAMPLE_WAVES], edge_above;
+    __shared__ uint32_t edge_best;
+    __shared__ int edge_n;
 
     const int r = blockIdx.x;
     const int lane = threadIdx.x % PULSE_WAVE, wave = threadIdx.x / PULSE_WAVE;
@@ -436,17 +436,15 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
     // ---- with top-k: locate the k-th largest with a histogram over [lowest, best], collect what lies at or above
     // its bin (in vocabulary order), and finish on that short list in LDS.  Falls through to the passes over the
     // whole vocabulary when the list would not fit (many equal values) or the range is empty.
-    // Top-p alone takes the same way with the LIST_TRY largest values, if their mass reaches top_p of the whole.
+    // Top-p alone takes the same way with the LIST_TRY largest values, if their mass reaches top_p of the whole.  (Behind the
+    // kernels in chunks it does not: their list was as long.)
     constexpr int LIST_TRY = 1024;
     const bool by_k = k > 0 && k < vocab;
     const int k_list = by_k ? k : min(vocab - 1, LIST_TRY);
     float whole = 0.f;   // without top-k: the mass of the whole vocabulary, which top_p refers to
-    float bin_scale = 0.f;
-    if (by_k || (use_p && k_list > 0)) {
-        if (rest) {      // (the kernels before have been over the row for both, and for the histogram)
-            rest += static_cast<int64_t>(r) * REST_WORDS;
-            for (int w = 0; w < SAMPLE_WAVES; ++w) whole += __int_as_float(rest[REST_MASS + w]);
-            lowest = __int_as_float(rest[REST_LOWEST + threadIdx.x % SAMPLE_WAVES]);
+    if (by_k || (use_p && k_list > 0 && !done)) {
+        if (rest) {      // (the kernels before have been over the row)
+            lowest = __int_as_float(rest[REST_LOWEST]);
         } else if (!by_k) {
             float mass = 0.f;
             sweep(row, threadIdx.x, vocab, SAMPLE_THREADS, [&](int, float x) {
@@ -465,8 +463,7 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
         int edge = -1, listed = 0;
         if (ranged) {
             for (int b = threadIdx.x; b < HIST_BINS; b += SAMPLE_THREADS) {
-                hist[b] = rest ? rest[b] : 0;
-                if (!by_k) hist_w[b] = rest ? __int_as_float(rest[HIST_BINS + b]) : 0.f;
+                hist[b] = rest ? rest[2 * b] : 0;
             }
             __syncthreads();
             if (!rest) {
@@ -475,7 +472,6 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
                 });
                 __syncthreads();
             }
-            if (!by_k) bin_scale = scale;
             // the bin in which the count from the top reaches k: first by wavefronts' shares of the bins, then by bins
             constexpr int SHARE = HIST_BINS / SAMPLE_WAVES;
             int mine = 0;
@@ -492,13 +488,7 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
                 edge = b;
             }
         }
-        bool may_hold = true;    // whether the list can hold top_p of the row (its mass is known to a thousandth at least)
-        if (rest && !by_k && edge >= 0) {
-            float above = 0.f;
-            for (int b = threadIdx.x; b <= edge; b += SAMPLE_THREADS) above += hist_w[b];
-            may_hold = block_sum_f(above, sf) >= 0.999f * p * whole;
-        }
-        if (edge >= 0 && listed <= LIST_CAP && may_hold) {
+        if (edge >= 0 && listed <= LIST_CAP) {
             int count = 0;
             by_mask(row, [&](auto masked) __attribute__((always_inline)) {
             constexpr int AHEAD = 8;   // steps of 64 entries whose values are asked for together
@@ -555,6 +545,121 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
     }
 
     // ---- passes over the whole vocabulary
+    if (use_p && !by_k) {
+        const Weigh weigh(best, inv_t, vocab);
+        float least = rest ? __int_as_float(rest[REST_LOWEST]) : lowest;
+        if (least == INFINITY) {      // (nobody has been over the row for it)
+            sweep(row, threadIdx.x, vocab, SAMPLE_THREADS, [&](int, float x) {
+                if (x != -INFINITY) least = fminf(least, x);
+            });
+            least = -block_max_f(-least, sf);
+        }
+        const float scale = static_cast<float>(HIST_BINS) / (best - least);
+        mass_t base = 0, whole_m = 0;
+        uint32_t thr = 0u;
+        bool found = false;
+        if (best > least && scale < INFINITY) {
+            // The bin in which the masses from the top reach top-p's share, and of its tokens the one that does it.  (Whole
+            // masses and one pass for that token take the place of float32 sums, good for a bracket only, and of a pass over
+            // the row for the sums at the five or fifteen tokens round that place.)
+            __syncthreads();
+            for (int b = threadIdx.x; b < HIST_BINS; b += SAMPLE_THREADS) hist_m[b] = rest ? reinterpret_cast<const mass_t*>(rest)[b] : 0;
+            if (threadIdx.x == 0) { edge_n = 0; edge_best = 0u; }
+            __syncthreads();
+            if (!rest) {
+                sweep(row, threadIdx.x, vocab, SAMPLE_THREADS, [&](int, float x) {
+                    if (x != -INFINITY) atomicAdd(&hist_m[bin_at(x, best, scale)], weigh(x));
+                });
+                __syncthreads();
+            }
+            const int at = edge_bin<SAMPLE_THREADS>(hist_m, p, 0, part_m, si, &edge_above, base, whole_m);
+            if (at >= 0) {
+                uint32_t* const keys = reinterpret_cast<uint32_t*>(list_i);
+                sweep(row, threadIdx.x, vocab, SAMPLE_THREADS, [&](int, float x) {
+                    if (x == -INFINITY || bin_at(x, best, scale) != at) return;
+                    const int e = atomicAdd(&edge_n, 1);
+                    if (e < EDGE_CAP) { keys[e] = order_key(x); edge_m[e] = weigh(x); }
+                });
+                __syncthreads();
+                const int n = edge_n;
+                if (n <= EDGE_CAP) {
+                    edge_key(keys, edge_m, n, SAMPLE_THREADS, base, whole_m, p, &edge_best);
+                    __syncthreads();
+                    thr = edge_best;
+                    found = thr != 0u;
+                }
+            }
+        }
+        auto block_mass = [&](mass_t v) {
+            v = mass_sum(v);
+            __syncthreads();
+            if (lane == 0) part_m[wave] = v;
+            __syncthreads();
+            mass_t total = 0;
+            for (int w = 0; w < SAMPLE_WAVES; ++w) total += part_m[w];
+            return total;
+        };
+        if (!found) {       // too many tokens in a bin, or no range: four bits of the threshold a pass
+            mass_t mass = 0;
+            sweep(row, threadIdx.x, vocab, SAMPLE_THREADS, [&](int, float x) { if (x != -INFINITY) mass += weigh(x); });
+            const double want = static_cast<double>(p) * static_cast<double>(block_mass(mass));
+            thr = 0u;
+            for (int shift = 28; shift >= 0; shift -= 4) {
+                mass_t above[15];
+#pragma unroll
+                for (int j = 0; j < 15; ++j) above[j] = 0;
+                sweep<8>(row, threadIdx.x, vocab, SAMPLE_THREADS, [&](int, float x) {
+                    if (x == -INFINITY) return;
+                    const uint32_t key = order_key(x);
+                    if (key < (thr | (1u << shift))) return;
+                    const mass_t w = weigh(x);
+#pragma unroll
+                    for (int j = 0; j < 15; ++j)
+                        if (key >= (thr | (static_cast<uint32_t>(j + 1) << shift))) above[j] += w;
+                });
+                uint32_t digit = 0u;
+#pragma unroll
+                for (int j = 0; j < 15; ++j)
+                    if (static_cast<double>(block_mass(above[j])) >= want) digit = static_cast<uint32_t>(j + 1);
+                thr |= digit << shift;
+            }
+        }
+        // the kept mass of every wavefront's part, then the part in which the draw falls is walked by its wavefront
+        mass_t mine = 0;
+        sweep(row, part_begin + lane, part_end, PULSE_WAVE, [&](int, float x) { if (x != -INFINITY && order_key(x) >= thr) mine += weigh(x); });
+        const mass_t kept = block_mass(mine);
+        if (kept == 0) {     // (an infinite logit: no weight is a number)
+            if (threadIdx.x == 0) out[r] = best_i;
+            return;
+        }
+        const mass_t target = draw_from(uniform[r], kept);
+        mass_t run = 0;
+        int who = 0;
+        while (target >= run + part_m[who]) run += part_m[who++];      // (target < kept: there is such a part)
+        if (wave != who) return;
+        int token = -1;
+        by_mask(row, [&](auto masked) __attribute__((always_inline)) {
+            constexpr int AHEAD = 8;     // steps of 64 entries whose values are asked for together
+            for (int first = part_begin; first < part_end && token < 0; first += AHEAD * PULSE_WAVE) {
+                float xs[AHEAD];
+#pragma unroll
+                for (int q = 0; q < AHEAD; ++q) {
+                    const int i = first + q * PULSE_WAVE + lane;
+                    xs[q] = i < part_end ? row.at<decltype(masked)::value>(i) : -INFINITY;
+                }
+#pragma unroll
+                for (int q = 0; q < AHEAD; ++q) {
+                    if (token >= 0) continue;
+                    const mass_t through = run + mass_through(xs[q] != -INFINITY && order_key(xs[q]) >= thr ? weigh(xs[q]) : 0);
+                    const unsigned long long hit = __ballot(target < through);
+                    if (hit != 0ull) token = first + q * PULSE_WAVE + __builtin_ctzll(hit);
+                    run = __shfl(through, PULSE_WAVE - 1, PULSE_WAVE);
+                }
+            }
+        });
+        if (lane == 0) out[r] = token;
+        return;
+    }
     // top-k threshold: the k-th largest key, found bit by bit
     uint32_t keep = 0u;
     if (k > 0 && k < vocab) {
@@ -567,36 +672,14 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
     }
     auto weight_of = [&](float x) { return (x != -INFINITY && order_key(x) >= keep) ? expf((x - best) * inv_t) : 0.f; };
     if (use_p) {
-        // M(t), the mass at or above a threshold t as this kernel sums it (every thread its entries in their order, then the
-        // threads): no larger for a larger t, so the largest t with M(t) >= want is one value however it is looked for.
-        uint32_t thr = 0u;
-        bool found = false;
-        float want;
-        if (!by_k && bin_scale > 0.f) {
-            // Top-p alone: the histogram's masses say near which token the sum reaches `want`; the tokens of that bin and
-            // its neighbours are ranked, and M is summed, in its own order, for the five (or fifteen) round that place side by side.
-            // (A search for the threshold's bits, four a pass, takes eight such passes.  32 rows of 151,936, this kernel:
-            // 661 us with the search, 377 with this, 141 with the mass and the histogram made by the kernels in front.  The masses
-            // are summed for the rows that come here alone: every row's cost those whose list holds top_p 1.7 to 2.5 times.)
-            want = p * whole;
-            if (!rest) {
-                sweep(row, threadIdx.x, vocab, SAMPLE_THREADS, [&](int, float x) {
-                    if (x != -INFINITY)
-                        add_in_group(&hist_w[min(HIST_BINS - 1, static_cast<int>((best - x) * bin_scale))], expf((x - best) * inv_t));
-                });
-                __syncthreads();
-            }
-            found = nucleus_edge(row, want, best, inv_t, bin_scale, hist, hist_w, sf, si, list_i, list_x, cand, &nearest, thr);
-        } else {
-            float mass = 0.f;
-            sweep(row, threadIdx.x, vocab, SAMPLE_THREADS, [&](int, float x) { mass += weight_of(x); });
-            want = p * block_sum_f(mass, sf);
-        }
-        // Else the largest threshold whose kept mass still reaches `want`, four bits of it a pass over the row: the masses
+        float mass = 0.f;
+        sweep(row, threadIdx.x, vocab, SAMPLE_THREADS, [&](int, float x) { mass += weight_of(x); });
+        const float want = p * block_sum_f(mass, sf);
+        // The largest threshold whose kept mass still reaches `want`, four bits of it a pass over the row: the masses
         // above the fifteen candidates of a digit are summed side by side (each in the order in which a pass for it
         // alone would sum it, so the choice is that of a search bit by bit, in an eighth of the passes).
-        if (!found) thr = 0u;
-        for (int shift = 28; shift >= 0 && !found; shift -= 4) {
+        uint32_t thr = 0u;
+        for (int shift = 28; shift >= 0; shift -= 4) {
             float above[15];
 #pragma unroll
             for (int j = 0; j < 15; ++j) above[j] = 0.f;
@@ -902,9 +985,30 @@ __global__ __launch_bounds__(SIMPLE_THREADS) void topk_collect_kernel(
     if (threadIdx.x == 0) *my_n = total;   // more than TOPK_SEGMENT: the row does not fit
 }
 
-// What rest_kernel adds a row's histogram to.
-__device__ __forceinline__ void clear_histogram(int* rest, int lane) {
-    for (int b = lane; b < 2 * HIST_BINS; b += PULSE_WAVE) rest[b] = 0;
+// The chunks' segments strung together in LDS: chunk c's entries go to places first[c] .. first[c + 1] - 1.  Eight a thread are asked
+// for together (a lane that fetched its chunk's entries one after the other took 15 of the choice's 26 us).
+template <int THREADS>
+__device__ __forceinline__ void string_segments(const int* seg_i, const float* seg_x, const int* first, int chunks, int* list_i, float* list_x) {
+    constexpr int AHEAD = 8;
+    for (int q0 = threadIdx.x; q0 < chunks * TOPK_SEGMENT; q0 += AHEAD * THREADS) {
+        int to[AHEAD], i[AHEAD];
+        float x[AHEAD];
+#pragma unroll
+        for (int u = 0; u < AHEAD; ++u) {
+            const int q = q0 + u * THREADS, c = min(q / TOPK_SEGMENT, chunks - 1), e = q - c * TOPK_SEGMENT;
+            to[u] = e < first[c + 1] - first[c] ? first[c] + e : -1;
+            i[u] = to[u] >= 0 ? seg_i[q] : 0;
+            x[u] = to[u] >= 0 ? seg_x[q] : 0.f;
+        }
+#pragma unroll
+        for (int u = 0; u < AHEAD; ++u)
+            if (to[u] >= 0) { list_i[to[u]] = i[u]; list_x[to[u]] = x[u]; }
+    }
+}
+
+// What rest_kernel adds a row's histogram to, and that the row's token is not chosen.
+__device__ __forceinline__ void clear_rest(int* rest, int lane) {
+    for (int b = lane; b <= REST_CHOSEN; b += PULSE_WAVE) rest[b] = 0;
 }
 
 // The choice of every row from what the kernels before left, a wavefront a row: the largest logit for greedy rows;
@@ -921,6 +1025,7 @@ __global__ __launch_bounds__(PULSE_WAVE) void chunked_choose_kernel(
     int* __restrict__ done, int* __restrict__ left) {
     __shared__ int list_i[LIST_CAP];
     __shared__ float list_x[LIST_CAP];
+    __shared__ int first_s[2 * PULSE_WAVE + 1];
     const int r = blockIdx.x, lane = threadIdx.x;
     part_max += r * chunks;
     part_idx += r * chunks;
@@ -959,7 +1064,7 @@ __global__ __launch_bounds__(PULSE_WAVE) void chunked_choose_kernel(
         const int n = first + __shfl(pre1, PULSE_WAVE - 1, PULSE_WAVE);
         if (k > chunks || chunks > 2 * PULSE_WAVE || __ballot(over) != 0ull || n > LIST_CAP || n < k || n == 0) {
             if (lane == 0) done[r] = 0;   // not a row for these kernels: sample_kernel takes it
-            if (left) clear_histogram(left + static_cast<int64_t>(r) * REST_WORDS, lane);
+            if (left) clear_rest(left + static_cast<int64_t>(r) * REST_WORDS, lane);
             return;
         }
         float whole = 0.f;   // without top-k: the mass of the whole row, chunk masses in chunk order
@@ -967,21 +1072,25 @@ __global__ __launch_bounds__(PULSE_WAVE) void chunked_choose_kernel(
             for (int c = lane; c < chunks; c += PULSE_WAVE) whole += part_mass[c];
             whole = wave_sum(whole);
         }
-        const int64_t seg0 = (static_cast<int64_t>(r) * chunks + lane) * TOPK_SEGMENT;
-        for (int e = 0; e < n0; ++e) { list_i[pre0 - n0 + e] = seg_i[seg0 + e]; list_x[pre0 - n0 + e] = seg_x[seg0 + e]; }
-        const int64_t seg1 = seg0 + static_cast<int64_t>(PULSE_WAVE) * TOPK_SEGMENT;
-        for (int e = 0; e < n1; ++e) { list_i[first + pre1 - n1 + e] = seg_i[seg1 + e]; list_x[first + pre1 - n1 + e] = seg_x[seg1 + e]; }
+        first_s[lane] = pre0 - n0;
+        first_s[lane + PULSE_WAVE] = first + pre1 - n1;
+        if (lane == 0) first_s[2 * PULSE_WAVE] = n;
+        __syncthreads();
+        const int64_t segment = static_cast<int64_t>(r) * chunks * TOPK_SEGMENT;
+        string_segments<PULSE_WAVE>(seg_i + segment, seg_x + segment, first_s, chunks, list_i, list_x);
         __syncthreads();
         int token;
         const bool enough =   // (false only without top-k: the list does not hold top_p of the row)
-            n <= 4 * PULSE_WAVE   // the usual case with top-k: a few dozen candidates, a few a lane
+            n <= 4 * PULSE_WAVE   // the usual case with top-k: a few dozen candidates, a few a lane; top-p alone has some hundreds
                 ? finish_on_list<4>(list_i, list_x, n, by_k, k, use_p, p, whole, best, inv_t, uniform[r], best_i, token)
+                : n <= 12 * PULSE_WAVE
+                ? finish_on_list<12>(list_i, list_x, n, by_k, k, use_p, p, whole, best, inv_t, uniform[r], best_i, token)
                 : finish_on_list<LIST_PER_LANE>(list_i, list_x, n, by_k, k, use_p, p, whole, best, inv_t, uniform[r], best_i, token);
         if (lane == 0) {
             if (enough) out[r] = token;
             done[r] = enough ? 1 : 0;
         }
-        if (left && !__shfl(enough ? 1 : 0, 0, PULSE_WAVE)) clear_histogram(left + static_cast<int64_t>(r) * REST_WORDS, lane);
+        if (left && !__shfl(enough ? 1 : 0, 0, PULSE_WAVE)) clear_rest(left + static_cast<int64_t>(r) * REST_WORDS, lane);
         return;
     }
     // a draw from the whole vocabulary: the chunk in which it falls, chunk masses in chunk order
@@ -997,7 +1106,7 @@ __global__ __launch_bounds__(PULSE_WAVE) void chunked_choose_kernel(
         const float mine = base + lane < chunks ? part_mass[base + lane] : 0.f;
         const int n = min(PULSE_WAVE, chunks - base);
         for (int j = 0; j < n; ++j) {
-            const float m = __shfl(mine, j, PULSE_WAVE);
+            const float m = __uint_as_float(static_cast<uint32_t>(__builtin_amdgcn_readlane(__float_as_int(mine), j)));
             if (m > 0.f) {
                 last_chunk = base + j;
                 if (target < run + m) { who = base + j; break; }
@@ -1023,66 +1132,244 @@ __global__ __launch_bounds__(PULSE_WAVE) void chunked_choose_kernel(
 }
 
 // ---- the rows that are left, before sample_kernel ---------------------------------------------------------------
-// A workgroup a row goes over its row at the rate of one compute unit; what sample_kernel needs to know of the whole row, its
-// mass (a wavefront of it summed by a wavefront here, entries and order as there) and the histogram over [lowest, best], is
-// made by many workgroups, in one launch: 18 us for 6 rows of 151,936 and 32 for 26, where the passes inside sample_kernel
-// took 220 and two launches, the histogram behind the mass and the lowest value, 34 for 13.  (The lowest value comes with the maxima, and the
-// histogram is cleared by the kernel that leaves the row.)
-constexpr int REST_GROUPS = 16;                                             // workgroups for a row's histogram
-constexpr int MASS_GROUPS = SAMPLE_WAVES * PULSE_WAVE / SIMPLE_THREADS;     // and for its mass
+// A workgroup a row goes over its row at the rate of one compute unit.  What has to be known of the whole row, the histogram
+// over [lowest, best], is made by many (the lowest value comes with the maxima, and the histogram is cleared by the kernel that
+// leaves the row); with it a row is finished in chunks as well (left_collect_kernel, left_choose_kernel), unless a chunk has more
+// tokens at the edge than its segment holds: those rows are sample_kernel's.
+// 32 rows of 151,936, six of them flat under top-p alone and six with a k above the number of chunks: these three kernels 41 us,
+// where the histogram with float32 masses and sample_kernel's passes took 31 and 128.
+constexpr int REST_GROUPS = 32;                                             // workgroups for a row's histogram
+
+// Whether a row is left, and what is known of it.
+struct LeftRow {
+    bool by_p, ranged;
+    int k;               // 0: without top-k
+    float p, best, lowest, inv_t, scale;
+    __device__ __forceinline__ LeftRow(int r, int vocab, int chunks, const float* temperature, const int* top_k, const float* top_p,
+                                       const float* part_max, const float* part_min) {
+        const int lane = threadIdx.x % PULSE_WAVE;
+        k = top_k ? top_k[r] : 0;
+        if (k < 0 || k >= vocab) k = 0;
+        p = top_p ? top_p[r] : 0.f;
+        by_p = k == 0 && p > 0.f && p < 1.f;
+        inv_t = 1.0f / temperature[r];
+        best = simple_row_max(part_max + static_cast<int64_t>(r) * chunks, chunks);
+        lowest = INFINITY;
+        for (int c = lane; c < chunks; c += PULSE_WAVE) lowest = fminf(lowest, part_min[static_cast<int64_t>(r) * chunks + c]);
+        lowest = -wave_max(-lowest);
+        scale = static_cast<float>(HIST_BINS) / (best - lowest);
+        ranged = best > lowest && scale < INFINITY;
+    }
+};
 
 __global__ __launch_bounds__(SIMPLE_THREADS) void rest_kernel(
     const float* __restrict__ logits, int vocab, int64_t row_stride, const float* __restrict__ temperature,
-    const int* __restrict__ top_k, const float* __restrict__ penalty, const int* __restrict__ seen_row,
+    const int* __restrict__ top_k, const float* __restrict__ top_p, const float* __restrict__ penalty, const int* __restrict__ seen_row,
     const uint32_t* __restrict__ seen_masks, const uint32_t* __restrict__ banned, int mask_words,
     const float* __restrict__ part_max, const float* __restrict__ part_min, int chunks, const int* __restrict__ done,
     int* __restrict__ rest) {
-    __shared__ int hist[HIST_BINS];
-    __shared__ float hist_w[HIST_BINS];
-    const int r = blockIdx.y, lane = threadIdx.x % PULSE_WAVE;
+    __shared__ mass_t hist[HIST_BINS];
+    const int r = blockIdx.y;
     if (done[r]) return;
     rest += static_cast<int64_t>(r) * REST_WORDS;
-    const float best = simple_row_max(part_max + static_cast<int64_t>(r) * chunks, chunks);
-    const float inv_t = 1.0f / temperature[r];
-    const int k = top_k ? top_k[r] : 0;
-    const bool by_k = k > 0 && k < vocab;
+    for (int b = threadIdx.x; b < HIST_BINS; b += SIMPLE_THREADS) hist[b] = 0;
+    const LeftRow left(r, vocab, chunks, temperature, top_k, top_p, part_max, part_min);
+    if (blockIdx.x == 0 && threadIdx.x == 0) rest[REST_LOWEST] = __float_as_int(left.lowest);
+    __syncthreads();
+    if (!left.ranged) return;    // (as sample_kernel: no histogram)
     const RowView row = simple_row(logits, r, row_stride, vocab, penalty, seen_row, seen_masks, banned, mask_words);
-    if (blockIdx.x < MASS_GROUPS) {
-        const int wave = blockIdx.x * (SIMPLE_THREADS / PULSE_WAVE) + threadIdx.x / PULSE_WAVE;
-        float mass = 0.f, lowest = INFINITY;
-        if (!by_k)
-            sweep(row, wave * PULSE_WAVE + lane, vocab, SAMPLE_THREADS, [&](int, float x) {
-                if (x != -INFINITY) mass += expf((x - best) * inv_t);
-            });
-        for (int c = lane; c < chunks; c += PULSE_WAVE) lowest = fminf(lowest, part_min[static_cast<int64_t>(r) * chunks + c]);
-        mass = wave_sum(mass);
-        lowest = -wave_max(-lowest);
-        if (lane == 0) {
-            rest[REST_MASS + wave] = __float_as_int(mass);
-            rest[REST_LOWEST + wave] = __float_as_int(lowest);
-        }
+    const Weigh weigh(left.best, left.inv_t, vocab);
+    const int first = blockIdx.x * SIMPLE_THREADS + threadIdx.x;
+    if (left.k > 0)
+        sweep(row, first, vocab, REST_GROUPS * SIMPLE_THREADS, [&](int, float x) {
+            if (x != -INFINITY) atomicAdd(&hist[bin_at(x, left.best, left.scale)], static_cast<mass_t>(1));
+        });
+    else
+        sweep(row, first, vocab, REST_GROUPS * SIMPLE_THREADS, [&](int, float x) {
+            if (x != -INFINITY) atomicAdd(&hist[bin_at(x, left.best, left.scale)], weigh(x));
+        });
+    __syncthreads();
+    for (int b = threadIdx.x; b < HIST_BINS; b += SIMPLE_THREADS)
+        if (hist[b] != 0) atomicAdd(reinterpret_cast<mass_t*>(rest) + b, hist[b]);
+}
+
+// A workgroup a chunk, into the chunk's segment.  Rows with top-k: the entries in the bin in which the k-th largest lies and above
+// it, in vocabulary order.  Top-p alone: the entries in the bin of the edge, in any order, and the mass of those above it.  (More
+// entries than a segment holds, or no edge: the number says so.)
+__global__ __launch_bounds__(SIMPLE_THREADS) void left_collect_kernel(
+    const float* __restrict__ logits, int vocab, int64_t row_stride, const float* __restrict__ temperature,
+    const int* __restrict__ top_k, const float* __restrict__ top_p, const float* __restrict__ penalty, const int* __restrict__ seen_row,
+    const uint32_t* __restrict__ seen_masks, const uint32_t* __restrict__ banned, int mask_words,
+    const float* __restrict__ part_max, const float* __restrict__ part_min, const int* __restrict__ done,
+    int* __restrict__ seg_i, float* __restrict__ seg_x, int* __restrict__ seg_n, int* __restrict__ rest) {
+    constexpr int WAVES = SIMPLE_THREADS / PULSE_WAVE, PER = SIMPLE_CHUNK / SIMPLE_THREADS;
+    __shared__ mass_t waves[WAVES], above_s;
+    __shared__ int at_s, counts[WAVES];
+    const int r = blockIdx.y, chunk = blockIdx.x, chunks = gridDim.x;
+    const int lane = threadIdx.x % PULSE_WAVE, wave = threadIdx.x / PULSE_WAVE;
+    if (done[r]) return;
+    const RowView row = simple_row(logits, r, row_stride, vocab, penalty, seen_row, seen_masks, banned, mask_words);
+    const int begin = chunk * SIMPLE_CHUNK + static_cast<int>(threadIdx.x) * PER;
+    float xs[PER];        // (asked for first: they travel while the edge is searched)
+    by_mask(row, [&](auto masked) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < PER; ++j) xs[j] = begin + j < vocab ? row.at<decltype(masked)::value>(begin + j) : -INFINITY;
+    });
+    const LeftRow left(r, vocab, chunks, temperature, top_k, top_p, part_max, part_min);
+    if (left.k == 0 && !left.by_p) return;
+    rest += static_cast<int64_t>(r) * REST_WORDS;
+    mass_t base = 0, whole = 0;
+    const int at = edge_bin<SIMPLE_THREADS>(reinterpret_cast<const mass_t*>(rest), left.p, left.k, waves, &at_s, &above_s, base, whole);
+    int* const my_n = seg_n + static_cast<int64_t>(r) * chunks + chunk;
+    if (at < 0) {
+        if (threadIdx.x == 0) *my_n = TOPK_SEGMENT + 1;
         return;
     }
-    for (int b = threadIdx.x; b < HIST_BINS; b += SIMPLE_THREADS) { hist[b] = 0; hist_w[b] = 0.f; }
-    float lowest = INFINITY;
-    for (int c = lane; c < chunks; c += PULSE_WAVE) lowest = fminf(lowest, part_min[static_cast<int64_t>(r) * chunks + c]);
-    lowest = -wave_max(-lowest);
-    const float scale = static_cast<float>(HIST_BINS) / (best - lowest);
+    const Weigh weigh(left.best, left.inv_t, vocab);
+    int bins[PER], mine = 0;
+    mass_t mass = 0;
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+        bins[j] = xs[j] == -INFINITY ? HIST_BINS : bin_at(xs[j], left.best, left.scale);
+        if (bins[j] == at || (left.k > 0 && bins[j] < at)) ++mine;
+        else if (bins[j] < at) mass += weigh(xs[j]);
+    }
+    // where this thread's entries go: an exclusive sum over the threads, in thread order (vocabulary order)
+    int pre = mine;
+#pragma unroll
+    for (int off = 1; off < PULSE_WAVE; off <<= 1) {
+        const int up = __shfl_up(pre, off, PULSE_WAVE);
+        if (lane >= off) pre += up;
+    }
+    mass = mass_sum(mass);
+    __syncthreads();      // (what edge_bin left has been read)
+    if (lane == PULSE_WAVE - 1) { counts[wave] = pre; waves[wave] = mass; }
     __syncthreads();
-    if (!(best > lowest && scale < INFINITY)) return;    // (as sample_kernel: no histogram)
-    sweep(row, (blockIdx.x - MASS_GROUPS) * SIMPLE_THREADS + threadIdx.x, vocab, REST_GROUPS * SIMPLE_THREADS, [&](int, float x) {
-        if (x != -INFINITY) {
-            const int b = min(HIST_BINS - 1, static_cast<int>((best - x) * scale));
-            atomicAdd(&hist[b], 1);
-            if (!by_k) add_in_group(&hist_w[b], expf((x - best) * inv_t));
+    int to = pre - mine, total = 0;
+    mass = 0;
+    for (int w = 0; w < WAVES; ++w) {
+        if (w < wave) to += counts[w];
+        total += counts[w];
+        mass += waves[w];
+    }
+    const int64_t segment = (static_cast<int64_t>(r) * chunks + chunk) * TOPK_SEGMENT;
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+        if (bins[j] == at || (left.k > 0 && bins[j] < at)) {
+            if (to < TOPK_SEGMENT) { seg_i[segment + to] = begin + j; seg_x[segment + to] = xs[j]; }
+            ++to;
+        }
+    }
+    if (threadIdx.x != 0) return;
+    *my_n = total;
+    *reinterpret_cast<mass_t*>(rest + REST_CHUNKS + 2 * chunk) = mass;
+    if (chunk == 0) {
+        *reinterpret_cast<mass_t*>(rest + REST_BASE) = base;
+        *reinterpret_cast<mass_t*>(rest + REST_WHOLE) = whole;
+    }
+}
+
+// The choice of such a row.  Top-k: on the strung segments, as sample_kernel's.  Top-p alone: the edge among the collected tokens,
+// the chunk in which the draw falls, its token.
+__global__ __launch_bounds__(SIMPLE_THREADS) void left_choose_kernel(
+    const float* __restrict__ logits, int vocab, int64_t row_stride, const float* __restrict__ temperature,
+    const int* __restrict__ top_k, const float* __restrict__ top_p, const float* __restrict__ uniform,
+    const float* __restrict__ penalty, const int* __restrict__ seen_row, const uint32_t* __restrict__ seen_masks,
+    const uint32_t* __restrict__ banned, int mask_words, const float* __restrict__ part_max, const float* __restrict__ part_min,
+    int chunks, const int* __restrict__ done, const int* __restrict__ seg_i, const float* __restrict__ seg_x,
+    const int* __restrict__ seg_n, int* __restrict__ rest, int* __restrict__ out) {
+    constexpr int WAVES = SIMPLE_THREADS / PULSE_WAVE, PER = SIMPLE_CHUNK / SIMPLE_THREADS;
+    __shared__ int list_i[LIST_CAP];
+    __shared__ float list_x[LIST_CAP];
+    __shared__ int first_s[REST_MOST_CHUNKS + 1], n_s;
+    __shared__ mass_t masses[EDGE_CAP], chunk_m[REST_MOST_CHUNKS], waves[WAVES], target_s;
+    __shared__ uint32_t keys[EDGE_CAP], best_s;
+    __shared__ int who_s;
+    const int r = blockIdx.x, lane = threadIdx.x % PULSE_WAVE, wave = threadIdx.x / PULSE_WAVE;
+    if (done[r]) return;
+    const LeftRow left(r, vocab, chunks, temperature, top_k, top_p, part_max, part_min);
+    if (left.k == 0 && !left.by_p) return;
+    rest += static_cast<int64_t>(r) * REST_WORDS;
+    seg_n += static_cast<int64_t>(r) * chunks;
+    const int64_t segment = static_cast<int64_t>(r) * chunks * TOPK_SEGMENT;
+    if (wave == 0) {      // the segments' places in the list, two neighbouring chunks a lane
+        const int n0 = 2 * lane < chunks ? seg_n[2 * lane] : 0, n1 = 2 * lane + 1 < chunks ? seg_n[2 * lane + 1] : 0;
+        int pre = n0 + n1;
+#pragma unroll
+        for (int off = 1; off < PULSE_WAVE; off <<= 1) {
+            const int up = __shfl_up(pre, off, PULSE_WAVE);
+            if (lane >= off) pre += up;
+        }
+        first_s[2 * lane] = pre - n0 - n1;
+        first_s[2 * lane + 1] = pre - n1;
+        const bool over = __ballot(n0 > TOPK_SEGMENT || n1 > TOPK_SEGMENT) != 0ull;
+        if (lane == PULSE_WAVE - 1) { n_s = over ? LIST_CAP + 1 : pre; first_s[REST_MOST_CHUNKS] = pre; }
+        if (lane == 0) best_s = 0u;
+    }
+    if (static_cast<int>(threadIdx.x) < chunks) chunk_m[threadIdx.x] = *reinterpret_cast<const mass_t*>(rest + REST_CHUNKS + 2 * threadIdx.x);
+    __syncthreads();
+    const int n = n_s;
+    if (n == 0 || n > (left.k > 0 ? LIST_CAP : EDGE_CAP)) return;
+    string_segments<SIMPLE_THREADS>(seg_i + segment, seg_x + segment, first_s, chunks, list_i, list_x);
+    __syncthreads();
+    if (left.k > 0) {
+        if (wave != 0) return;
+        int token;            // (with top-k every list is enough)
+        if (n <= 8 * PULSE_WAVE) finish_on_list<8>(list_i, list_x, n, true, left.k, left.p > 0.f && left.p < 1.f, left.p, 0.f, left.best, left.inv_t, uniform[r], list_i[0], token);
+        else finish_on_list<LIST_PER_LANE>(list_i, list_x, n, true, left.k, left.p > 0.f && left.p < 1.f, left.p, 0.f, left.best, left.inv_t, uniform[r], list_i[0], token);
+        if (lane == 0) { out[r] = token; rest[REST_CHOSEN] = 1; }
+        return;
+    }
+    const Weigh weigh(left.best, left.inv_t, vocab);
+    const float p = left.p;
+    for (int e = threadIdx.x; e < n; e += SIMPLE_THREADS) {
+        keys[e] = order_key(list_x[e]);
+        masses[e] = weigh(list_x[e]);
+    }
+    __syncthreads();
+    edge_key(keys, masses, n, SIMPLE_THREADS, *reinterpret_cast<const mass_t*>(rest + REST_BASE),
+             *reinterpret_cast<const mass_t*>(rest + REST_WHOLE), p, &best_s);
+    __syncthreads();
+    const uint32_t thr = best_s;
+    if (thr == 0u) return;
+    for (int e = threadIdx.x; e < n; e += SIMPLE_THREADS)
+        if (keys[e] >= thr) atomicAdd(&chunk_m[list_i[e] / SIMPLE_CHUNK], masses[e]);
+    __syncthreads();
+    if (wave == 0) {      // the chunk in which u of the kept mass falls, two chunks a lane
+        const mass_t m0 = 2 * lane < chunks ? chunk_m[2 * lane] : 0, m1 = 2 * lane + 1 < chunks ? chunk_m[2 * lane + 1] : 0;
+        const mass_t through = mass_through(m0 + m1), target = draw_from(uniform[r], __shfl(through, PULSE_WAVE - 1, PULSE_WAVE));
+        mass_t before = through - m0 - m1;
+        if (target >= before && target < through) {                    // (target is less than all of it: one lane)
+            const bool second = target >= before + m0;
+            who_s = 2 * lane + (second ? 1 : 0);
+            target_s = target - before - (second ? m0 : 0);
+        }
+    }
+    __syncthreads();
+    const int begin = who_s * SIMPLE_CHUNK + static_cast<int>(threadIdx.x) * PER;
+    const RowView row = simple_row(logits, r, row_stride, vocab, penalty, seen_row, seen_masks, banned, mask_words);
+    mass_t ms[PER], mine = 0;
+    by_mask(row, [&](auto masked) __attribute__((always_inline)) {
+        float xs[PER];
+#pragma unroll
+        for (int j = 0; j < PER; ++j) xs[j] = begin + j < vocab ? row.at<decltype(masked)::value>(begin + j) : -INFINITY;
+#pragma unroll
+        for (int j = 0; j < PER; ++j) {
+            ms[j] = xs[j] != -INFINITY && order_key(xs[j]) >= thr ? weigh(xs[j]) : 0;
+            mine += ms[j];
         }
     });
+    const mass_t through = mass_through(mine);
+    if (lane == PULSE_WAVE - 1) waves[wave] = through;
     __syncthreads();
-    for (int b = threadIdx.x; b < HIST_BINS; b += SIMPLE_THREADS) {
-        if (hist[b] == 0) continue;
-        atomicAdd(&rest[b], hist[b]);
-        if (!by_k) unsafeAtomicAdd(reinterpret_cast<float*>(rest) + HIST_BINS + b, hist_w[b]);
-    }
+    mass_t before = through - mine;
+    for (int w = 0; w < wave; ++w) before += waves[w];
+    const mass_t target = target_s;
+    if (target < before || target >= before + mine) return;            // one thread has it
+    int j = 0;
+    while (target >= before + ms[j]) before += ms[j++];
+    out[r] = begin + j;
+    rest[REST_CHOSEN] = 1;
 }
 
 }  // namespace
@@ -1180,13 +1467,15 @@ extern "C" int pulse_sample(const float* logits, int rows, int vocab, int64_t ro
 // The same in chunks of the vocabulary with a workgroup each, which reads a row many times faster than the
 // workgroup a row of pulse_sample does.  Greedy rows, rows that draw from the whole vocabulary at their temperature
 // rows with top-k (and top-p on what it keeps) whose k is at most the number of chunks and rows with top-p alone whose
-// top_p share lies in some hundreds of the largest logits are chosen by these kernels; rows that do not fit (many
-// equal values around the k-th largest, a distribution too flat for top-p alone) by the kernel of pulse_sample behind
-// them, which skips the rows that are done.  What a row's choice is does not depend on the
-// other rows.  Scratch, with chunks = pulse_sample_chunks(vocab): part_max, part_mass (float32), part_idx, seg_n
+// top_p share lies in some hundreds of the largest logits are chosen by these kernels; rows that do not fit (a larger k, a
+// distribution too flat for top-p alone) by three more that go by a histogram of the row, and what does not fit these either (many
+// equal values at the edge) by the kernel of pulse_sample behind them, which skips the rows that are done.  What a row's choice is
+// does not depend on the other rows.  Whole calls, us, before the histogram's kernels finished rows: 32,000 values, 3 / 16 / 64 rows
+// 136 / 150 / 187 -> 94 / 119 / 161; 151,936 values 208 / 241 / 327 -> 103 / 131 / 200.  Scratch, with chunks = pulse_sample_chunks(vocab): part_max, part_mass (float32), part_idx, seg_n
 // (int32) of rows * chunks entries; seg_i (int32), seg_x (float32) of rows * chunks * pulse_sample_segment()
 // entries; done (int32) of rows entries; and, optional (null: the rows that are left are gone over by their own workgroups
-// alone, with the same choices), rest (int32) of rows * (pulse_sample_rest() + chunks) entries.
+// alone, with the same choices, as where it does not start at a multiple of 8 bytes), rest (int32) of rows *
+// (pulse_sample_rest() + chunks) entries.
 extern "C" int pulse_sample_rest() { return REST_WORDS; }
 extern "C" int pulse_sample_chunks(int vocab) { return (vocab + SIMPLE_CHUNK - 1) / SIMPLE_CHUNK; }
 extern "C" int pulse_sample_segment() { return TOPK_SEGMENT; }
@@ -1207,10 +1496,7 @@ extern "C" int pulse_sample_chunked_rest(const float* logits, int rows, int voca
     if (rows == 0) return 0;
     const int chunks = pulse_sample_chunks(vocab);
     const bool leaves = temperature && (top_k || top_p);    // (without them every row is done)
-    // They are made while a workgroup a row leaves most of the chip idle and its passes are long: 32,000 values, flat rows
-    // under top-p and others, 16 rows 103 and 80 us with them (272 and 87 without any of it), 64 rows 128 and 108, 159 and
-    // 92 without; 151,936 values, 64 rows 427 and 291 (947 and 776).
-    const bool prepare = rest && leaves && vocab >= 1024 * static_cast<int64_t>(rows);
+    const bool prepare = rest && leaves && reinterpret_cast<uintptr_t>(rest) % alignof(mass_t) == 0;
     if (!prepare) rest = nullptr;
     // (behind what is made of the rows: the chunks' smallest numbers)
     float* part_min = prepare ? reinterpret_cast<float*>(rest + static_cast<int64_t>(rows) * REST_WORDS) : nullptr;
@@ -1234,9 +1520,18 @@ extern "C" int pulse_sample_chunked_rest(const float* logits, int rows, int voca
                        part_idx, part_mass, seg_i, seg_x, seg_n, chunks, out, done, rest);
     PULSE_LAUNCH_CHECK("sample_chunked (choice)");
     if (prepare) {
-        hipLaunchKernelGGL(rest_kernel, dim3(MASS_GROUPS + REST_GROUPS, rows), dim3(SIMPLE_THREADS), 0, stream, logits, vocab,
-                           row_stride, temperature, top_k, penalty, seen_row, seen_masks, banned, mask_words, part_max,
-                           part_min, chunks, static_cast<const int*>(done), rest);
+        hipLaunchKernelGGL(rest_kernel, dim3(REST_GROUPS, rows), dim3(SIMPLE_THREADS), 0, stream, logits, vocab, row_stride, temperature,
+                           top_k, top_p, penalty, seen_row, seen_masks, banned, mask_words, part_max, part_min, chunks,
+                           static_cast<const int*>(done), rest);
+        if (chunks <= REST_MOST_CHUNKS) {
+            hipLaunchKernelGGL(left_collect_kernel, dim3(chunks, rows), dim3(SIMPLE_THREADS), 0, stream, logits, vocab, row_stride,
+                               temperature, top_k, top_p, penalty, seen_row, seen_masks, banned, mask_words, part_max, part_min,
+                               static_cast<const int*>(done), seg_i, seg_x, seg_n, rest);
+            hipLaunchKernelGGL(left_choose_kernel, dim3(rows), dim3(SIMPLE_THREADS), 0, stream, logits, vocab, row_stride,
+                               temperature, top_k, top_p, uniform, penalty, seen_row, seen_masks, banned, mask_words, part_max, part_min,
+                               chunks, static_cast<const int*>(done), static_cast<const int*>(seg_i), static_cast<const float*>(seg_x),
+                               static_cast<const int*>(seg_n), rest, out);
+        }
         PULSE_LAUNCH_CHECK("sample_chunked (what is left)");
     }
     if (leaves) {

@@ -1056,7 +1056,7 @@ def sample(logits: torch.Tensor, out: torch.Tensor, temperature: Optional[torch.
 
 SAMPLE_CHUNK = 2048      # as SIMPLE_CHUNK of sampling.hip
 SAMPLE_SEGMENT = 32      # as TOPK_SEGMENT of sampling.hip
-SAMPLE_REST = 2 * 2048 + 2 * 16   # as REST_WORDS of sampling.hip
+SAMPLE_REST = 2 * 2048 + 6 + 2 * 128   # as REST_WORDS of sampling.hip
 
 
 def sample_chunks(vocab: int) -> int:

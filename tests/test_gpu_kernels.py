@@ -1529,3 +1529,41 @@ def test_two_stage_argmax(k):
         single = torch.empty(rows, dtype=torch.int32, device=DEV)
         k.sample(logits, single)
         assert single.tolist() == want
+
+
+@pytest.mark.parametrize("vocab", [5, 2049, 40000, 151936, 2048 * 128, 2048 * 128 + 3])
+def test_rows_left_by_the_chunks_are_chosen_the_same_with_and_without_many_workgroups(k, vocab):
+    """Flat rows under top-p and rows with more top-k than chunks, masks and ties among them: the kernels that take a row's chunks
+    to a workgroup each, and the workgroup a row that does without their scratch, to the token (the masses are whole numbers);
+    a row that holds an infinity chooses it."""
+    rows = 20
+    gen = torch.Generator().manual_seed(vocab)
+    logits = torch.randn(rows, vocab, generator=gen) * torch.linspace(0.2, 3.0, rows).view(-1, 1)
+    logits[3] = (logits[3] * 2).round() / 2                # so many equal values that no segment holds the edge's bin
+    logits[4] = 1.0
+    logits[5, vocab // 2] = float("inf")
+    logits[6, : vocab - 1] = float("-inf")
+    top_k = torch.zeros(rows, dtype=torch.int32)
+    top_k[10:] = torch.tensor([129, 140, 200, 300, 500, 1000, 1900, 3000, vocab, vocab + 7], dtype=torch.int32)
+    top_p = torch.linspace(0.3, 0.9999, rows)
+    top_p[14:16] = 0.0
+    words = (vocab + 31) // 32
+    seen = torch.randint(-2 ** 31, 2 ** 31 - 1, (rows, words), generator=gen).to(torch.int32)
+    banned = torch.zeros(words, dtype=torch.int32)
+    banned[0] = 2
+    dev = lambda t: t.to(DEV)
+    kw = dict(temperature=dev(torch.linspace(0.5, 1.5, rows)), top_k=dev(top_k), top_p=dev(top_p),
+              uniform=dev(torch.rand(rows, generator=gen)), penalty=dev(torch.where(torch.arange(rows) % 2 == 1, 0.5, 0.0)),
+              seen_row=torch.arange(rows, dtype=torch.int32, device=DEV), seen_masks=dev(seen), banned=dev(banned))
+    many, one = (torch.full((rows,), -9, dtype=torch.int32, device=DEV) for _ in range(2))
+    scratch = _chunked_scratch(k, rows, vocab)
+    k.sample_chunked(dev(logits), many, scratch, **kw)
+    without = _chunked_scratch(k, rows, vocab)
+    del without["rest"]
+    k.sample_chunked(dev(logits), one, without, **kw)
+    assert many.tolist() == one.tolist() and min(many.tolist()) >= 0 and max(many.tolist()) < vocab
+    assert many[5].item() == vocab // 2 and many[6].item() == vocab - 1
+    if vocab == 151936:
+        chosen = scratch["rest"].view(-1)[: rows * k.SAMPLE_REST].view(rows, k.SAMPLE_REST)[:, 2 * 2048 + 1].cpu()
+        left = scratch["done"][:rows].cpu() == 0
+        assert left.sum() >= 8 and (chosen[left] == 1).sum() >= 6        # most of them did not need the workgroup a row
