@@ -50,7 +50,7 @@ __device__ __forceinline__ bf16x8 zeros8() {
     return __builtin_bit_cast(bf16x8, u32x4{0u, 0u, 0u, 0u});
 }
 
-template <int R, int CT, int AHEAD, int PER_SIMD>
+template <int R, int CT, int AHEAD, int PER_SIMD, bool EARLY>
 __global__ __launch_bounds__(256, PER_SIMD) void attn_wide_kernel(const bf16_t* __restrict__ q, float* __restrict__ out,
                                                         const bf16_t* __restrict__ kcache,
                                                         const bf16_t* __restrict__ vcache,
@@ -122,6 +122,31 @@ __global__ __launch_bounds__(256, PER_SIMD) void attn_wide_kernel(const bf16_t* 
         }
         ahead[0] = lookup(step + 4, 0);
         ahead[1] = lookup(step + 4, 1);
+        // Where the values lie.  Keys of the operand that have never been stored are cleared:
+        // one mask a 32-bit half of the lane's eight values, the same for every tile.
+        unsigned int keep_bits[4];
+        const bf16_t* vbase[2];
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            const int j = jbase[t] + 4 * g;
+            const bool there = page[t] >= 0;
+            keep_bits[2 * t] = (there && j <= pos_last ? 0x0000FFFFu : 0u) | (there && j + 1 <= pos_last ? 0xFFFF0000u : 0u);
+            keep_bits[2 * t + 1] = (there && j + 2 <= pos_last ? 0x0000FFFFu : 0u) | (there && j + 3 <= pos_last ? 0xFFFF0000u : 0u);
+            // (value head c's channel e lies (c * d + e) * page_size behind kv head 0's: with all values side by side the
+            // channel number is c * d + e itself)
+            vbase[t] = vcache + static_cast<int64_t>(there ? page[t] : 0) * a.nkv * d * a.page_size + off[t] + 4 * g
+                       + static_cast<int64_t>((a.all_values ? 0 : kvh * d) + chunk0 + r) * a.page_size;
+        }
+        const int tile_stride = 16 * a.page_size;
+        // (EARLY: the values are asked for before the keys, so that one trip to memory serves both)
+        u32x2 early[EARLY ? CT : 1][2];
+        if constexpr (EARLY) {
+#pragma unroll
+            for (int c = 0; c < CT; ++c)
+#pragma unroll
+                for (int t = 0; t < 2; ++t) early[c][t] = *reinterpret_cast<const u32x2*>(vbase[t] + min(c, tiles - 1) * tile_stride);
+            __builtin_amdgcn_sched_barrier(0);
+        }
         // S^T: keys x rows, for every row tile from the same key operands
         f32x4 s[R][2];
 #pragma unroll
@@ -129,22 +154,30 @@ __global__ __launch_bounds__(256, PER_SIMD) void attn_wide_kernel(const bf16_t* 
         const bf16_t* krow[2];
 #pragma unroll
         for (int t = 0; t < 2; ++t)
-            krow[t] = page[t] >= 0 ? kcache + ((static_cast<int64_t>(page[t]) * a.nkv + kvh) * a.page_size + off[t] + r) * d
-                                   : nullptr;
-        // (the operands of AHEAD pieces of 32 channels are asked for together: a piece by itself waits out a trip to
-        // memory, and a wavefront of a step of few tokens has a block or two of keys in all.  8 requests of 1,500 tokens,
-        // a latent row of 576 channels: 28 us a piece at a time, 26 so.)
+            krow[t] = kcache + ((static_cast<int64_t>(max(page[t], 0)) * a.nkv + kvh) * a.page_size + off[t] + r) * d;
+        // (the operands of AHEAD pieces of 32 channels are asked for together, from addresses that always hold keys (what is no key's
+        // or no channel's is masked behind): a piece by itself waits out a trip to memory, and a wavefront of a step of few tokens
+        // has a block or two of keys in all.)
         for (int e0 = 0; e0 < d; e0 += 32 * AHEAD) {
             bf16x8 ka[AHEAD][2], qb[AHEAD][R];
 #pragma unroll
             for (int u = 0; u < AHEAD; ++u) {
-                const int e = e0 + 32 * u + 8 * g;
-                const bool in = e < d;
+                const int e = min(e0 + 32 * u + 8 * g, d - 8);
 #pragma unroll
-                for (int t = 0; t < 2; ++t)
-                    ka[u][t] = (in && krow[t]) ? *reinterpret_cast<const bf16x8*>(krow[t] + e) : zeros8();
+                for (int t = 0; t < 2; ++t) ka[u][t] = *reinterpret_cast<const bf16x8*>(krow[t] + e);
 #pragma unroll
-                for (int rr = 0; rr < R; ++rr) qb[u][rr] = in ? *reinterpret_cast<const bf16x8*>(qrow[rr] + e) : zeros8();
+                for (int rr = 0; rr < R; ++rr) qb[u][rr] = *reinterpret_cast<const bf16x8*>(qrow[rr] + e);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            if (e0 + 32 * AHEAD > d) {          // pieces behind the head's channels
+#pragma unroll
+                for (int u = 0; u < AHEAD; ++u) {
+                    const bool in = e0 + 32 * u + 8 * g < d;
+#pragma unroll
+                    for (int t = 0; t < 2; ++t) ka[u][t] = in ? ka[u][t] : zeros8();
+#pragma unroll
+                    for (int rr = 0; rr < R; ++rr) qb[u][rr] = in ? qb[u][rr] : zeros8();
+                }
             }
 #pragma unroll
             for (int u = 0; u < AHEAD; ++u)
@@ -188,29 +221,14 @@ __global__ __launch_bounds__(256, PER_SIMD) void attn_wide_kernel(const bf16_t* 
             l_run[rr] = l_run[rr] * alpha[rr] + sum;
             m_run[rr] = m_new;
         }
-        // O^T += V^T P^T, channel tile by channel tile.  Keys of the operand that have never been stored are cleared:
-        // one mask a 32-bit half of the lane's eight values, the same for every tile.
-        unsigned int keep_bits[4];
-        const bf16_t* vbase[2];
-#pragma unroll
-        for (int t = 0; t < 2; ++t) {
-            const int j = jbase[t] + 4 * g;
-            const bool there = page[t] >= 0;
-            keep_bits[2 * t] = (there && j <= pos_last ? 0x0000FFFFu : 0u) | (there && j + 1 <= pos_last ? 0xFFFF0000u : 0u);
-            keep_bits[2 * t + 1] = (there && j + 2 <= pos_last ? 0x0000FFFFu : 0u) | (there && j + 3 <= pos_last ? 0xFFFF0000u : 0u);
-            // (value head c's channel e lies (c * d + e) * page_size behind kv head 0's: with all values side by side the
-            // channel number is c * d + e itself)
-            vbase[t] = vcache + static_cast<int64_t>(there ? page[t] : 0) * a.nkv * d * a.page_size + off[t] + 4 * g
-                       + static_cast<int64_t>((a.all_values ? 0 : kvh * d) + chunk0 + r) * a.page_size;
-        }
-        const int tile_stride = 16 * a.page_size;
+        // O^T += V^T P^T, channel tile by channel tile
 #pragma unroll
         for (int c = 0; c < CT; ++c) {
             if (c < tiles) {
                 u32x4 raw;
 #pragma unroll
                 for (int t = 0; t < 2; ++t) {
-                    const u32x2 two = *reinterpret_cast<const u32x2*>(vbase[t] + c * tile_stride);
+                    const u32x2 two = EARLY ? early[EARLY ? c : 0][t] : *reinterpret_cast<const u32x2*>(vbase[t] + c * tile_stride);
                     raw[2 * t] = two[0] & keep_bits[2 * t];
                     raw[2 * t + 1] = two[1] & keep_bits[2 * t + 1];
                 }
@@ -391,19 +409,22 @@ extern "C" int pulse_attn_wide(const void* q, int64_t q_stride, float* out, int6
     a.n_splits = n_splits; a.part = part; a.part_ml = part_ml;
     if (row_tiles == 4) {
         const dim3 grid(n_items, (wv + 127) / 128, n_splits);
-        hipLaunchKernelGGL((attn_wide_kernel<4, 8, 1, 1>), grid, dim3(256), 0, stream, static_cast<const bf16_t*>(q), out,
+        hipLaunchKernelGGL((attn_wide_kernel<4, 8, 1, 1, false>), grid, dim3(256), 0, stream, static_cast<const bf16_t*>(q), out,
                            static_cast<const bf16_t*>(kcache), static_cast<const bf16_t*>(vcache), positions, token_entry,
                            block_table, items, sink, a);
     } else {
         const dim3 grid(n_items, (wv + 255) / 256, n_splits);
-        // Steps of few tokens, whose keys are shared out, ask for six pieces of a key ahead and need the registers of a
-        // wavefront and a half for it; prompt portions have enough wavefronts to wait for one another (three a SIMD).
-#define PULSE_WIDE(AHEAD, PER_SIMD)                                                                                      \
-    hipLaunchKernelGGL((attn_wide_kernel<1, MAX_TILES, AHEAD, PER_SIMD>), grid, dim3(256), 0, stream,                    \
+        // Steps of few tokens, whose keys are shared out, ask for the values and four pieces of a key ahead and need the registers of
+        // a wavefront and a half for it; prompt portions have enough wavefronts to wait for one another (three a SIMD).  A latent
+        // row of 576 channels, with the merge, six pieces ahead and the values behind the scores -> this, us: one request of 600
+        // tokens 20.0 -> 19.4, 8 of 300 22.6 -> 19.3, 8 of 1,500 in 16 splits 30.0 -> 28.2, 8 of 4,000 56.4 -> 50.7, 32 of 1,500
+        // 73.9 -> 65.7.  (Six pieces beside the values do not fit 256 registers.)
+#define PULSE_WIDE(AHEAD, PER_SIMD, EARLY)                                                                                      \
+    hipLaunchKernelGGL((attn_wide_kernel<1, MAX_TILES, AHEAD, PER_SIMD, EARLY>), grid, dim3(256), 0, stream,                    \
                        static_cast<const bf16_t*>(q), out, static_cast<const bf16_t*>(kcache),                           \
                        static_cast<const bf16_t*>(vcache), positions, token_entry, block_table, items, sink, a)
-        if (n_splits > 1) PULSE_WIDE(6, 2);
-        else PULSE_WIDE(1, 3);
+        if (n_splits > 1) PULSE_WIDE(4, 2, true);
+        else PULSE_WIDE(1, 3, false);
 #undef PULSE_WIDE
     }
     PULSE_LAUNCH_CHECK("attn_wide");
