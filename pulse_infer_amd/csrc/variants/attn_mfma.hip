@@ -306,10 +306,19 @@ __device__ __forceinline__ void prepare_head(bf16x8 (&x)[NCHUNK], const HeadTabl
 // token's position also prepares the token's key, puts key and value into the registers of the block they belong
 // to (their page is written from here and never read back), so that the launch before this one is saved.
 template <bool FUSED>
-__global__ __launch_bounds__(WAVES* PULSE_WAVE) PULSE_ATTN_WAVES_PER_EU void attn_mfma_kernel(MfmaArgs a) {
-    __shared__ float s_m[WAVES][16];
-    __shared__ float s_l[WAVES][16];
-    __shared__ float s_o[WAVES][D][17];
+struct MfmaShared {
+    float m[WAVES][16];
+    float l[WAVES][16];
+    float o[WAVES][D][17];
+    u32x4 newk[FUSED ? WAVES : 1][D / 8];
+    bf16_t newv[FUSED ? WAVES : 1][D];
+};
+
+template <bool FUSED>
+__device__ __forceinline__ void attn_mfma_workgroup(const MfmaArgs& a, const int block, MfmaShared<FUSED>& shared) {
+    float (&s_m)[WAVES][16] = shared.m;
+    float (&s_l)[WAVES][16] = shared.l;
+    float (&s_o)[WAVES][D][17] = shared.o;
 
     // Workgroups that follow each other in the grid go to different XCDs, each with its own L2 and its own share of
     // the way to memory (about an eighth of the chip's rate), and inside an XCD to different compute units, each of
@@ -317,11 +326,11 @@ __global__ __launch_bounds__(WAVES* PULSE_WAVE) PULSE_ATTN_WAVES_PER_EU void att
     // splits, then the items: a request with a long context among short ones is then read through every XCD and by
     // as many compute units as it has workgroups.
     const int heads = a.nkv * a.head_chunks;
-    const int hy = blockIdx.x % heads;
-    int split = (blockIdx.x / heads) % a.n_splits;
-    int item = blockIdx.x / heads / a.n_splits;
+    const int hy = block % heads;
+    int split = (block / heads) % a.n_splits;
+    int item = block / heads / a.n_splits;
     if (a.plan) {
-        const int k = blockIdx.x / heads;
+        const int k = block / heads;
         if (k >= a.plan[0]) return;
         const int s = a.plan[1 + k];
         item = s / a.n_splits;
@@ -413,10 +422,8 @@ __global__ __launch_bounds__(WAVES* PULSE_WAVE) PULSE_ATTN_WAVES_PER_EU void att
     };
     // FUSED: the token's key and value wait in LDS, a copy for each wavefront (so that no barrier is needed), until
     // the block they belong to is computed.
-    __shared__ u32x4 s_newk[FUSED ? WAVES : 1][D / 8];
-    __shared__ bf16_t s_newv[FUSED ? WAVES : 1][D];
-    u32x4* stash_k = s_newk[FUSED ? wave : 0];
-    bf16_t* stash_v = s_newv[FUSED ? wave : 0];
+    u32x4* stash_k = shared.newk[FUSED ? wave : 0];
+    bf16_t* stash_v = shared.newv[FUSED ? wave : 0];
     auto prepare = [&](bool own_key) {
         const float temp = a.temp_every > 0
             ? 1.f + a.temp_coef * logf(static_cast<float>((max(pos_c, 0) + 1) / a.temp_every) + 1.f) : 1.f;
@@ -706,6 +713,12 @@ __global__ __launch_bounds__(WAVES* PULSE_WAVE) PULSE_ATTN_WAVES_PER_EU void att
             a.part_ml[2 * slot + 1] = ll;
         }
     }
+}
+
+template <bool FUSED>
+__global__ __launch_bounds__(WAVES* PULSE_WAVE) PULSE_ATTN_WAVES_PER_EU void attn_mfma_kernel(MfmaArgs a) {
+    __shared__ __attribute__((aligned(16))) MfmaShared<FUSED> shared;
+    attn_mfma_workgroup<FUSED>(a, blockIdx.x, shared);
 }
 
 // ---------------------------------------------------------------------------------------------------------
@@ -1002,21 +1015,22 @@ struct WideShape {
 #else
 #define PULSE_WIDE_WAVES_PER_EU PULSE_ATTN_WAVES_PER_EU
 #endif
+// s_kv: 2 * Shape::STAGE values of LDS, a stage after the other, the K block first; (bx, by, bz) of (items, heads, splits): the workgroup.
 template <int CT, int KT, int NW>
-__global__ __launch_bounds__(NW* PULSE_WAVE) PULSE_WIDE_WAVES_PER_EU void attn_prefill_wide_kernel(MfmaArgs a, int per) {
+__device__ __forceinline__ void attn_prefill_wide_workgroup(const MfmaArgs& a, const int per, const int bx, const int by, const int bz,
+                                                            const int items, const int heads, bf16_t* const s_kv) {
     using Shape = WideShape<CT, KT, NW>;
     constexpr int BK = Shape::BK;
     static_assert(KT % 2 == 0, "the second product takes pairs of key tiles");
     static_assert(D == 32 || D == 64 || D == 128 || D == 192, "whole 1 KB chunks, and key rows that start at the same place of 128 bytes or divide them");
     constexpr int P = Shape::P;
-    __shared__ __attribute__((aligned(1024))) bf16_t s_kv[2 * Shape::STAGE];  // stage: K block, then V block
 
     // The second half of the kv heads walks the items backwards: a long item (a late portion of a prompt) then
     // shares its compute unit with a short one instead of another long one, and the longest workgroups, which set
     // the kernel's time, run at a lone workgroup's speed.
-    const int item = (blockIdx.y * 2 / gridDim.y) & 1 ? gridDim.x - 1 - blockIdx.x : blockIdx.x;
-    const int g = blockIdx.y / a.head_chunks;
-    const int chunk = blockIdx.y % a.head_chunks;
+    const int item = (by * 2 / heads) & 1 ? items - 1 - bx : bx;
+    const int g = by / a.head_chunks;
+    const int chunk = by % a.head_chunks;
     const int tid = threadIdx.x;
     const int wave = uniform(tid / PULSE_WAVE);
     const int lane = tid % PULSE_WAVE;
@@ -1030,7 +1044,7 @@ __global__ __launch_bounds__(NW* PULSE_WAVE) PULSE_WIDE_WAVES_PER_EU void attn_p
     // keys of its split only.  An item all of whose keys lie in the first split is finished here as without
     // splits; the others leave unnormalised partial results for attn_prefill_reduce_kernel.
     const bool splits = a.n_splits > 1;
-    const int split = splits ? static_cast<int>(blockIdx.z) : 0;
+    const int split = splits ? bz : 0;
     const int split_begin = splits ? split * a.split_size : 0;
     if (split_begin > hi) return;                            // no key of the item here; the merge does not read this split
     const int split_last = splits ? min(hi, split_begin + a.split_size - 1) : hi;
@@ -1365,6 +1379,34 @@ __global__ __launch_bounds__(NW* PULSE_WAVE) PULSE_WIDE_WAVES_PER_EU void attn_p
     }
 }
 
+template <int CT, int KT, int NW>
+__global__ __launch_bounds__(NW* PULSE_WAVE) PULSE_WIDE_WAVES_PER_EU void attn_prefill_wide_kernel(MfmaArgs a, int per) {
+    __shared__ __attribute__((aligned(1024))) bf16_t s_kv[2 * WideShape<CT, KT, NW>::STAGE];
+    attn_prefill_wide_workgroup<CT, KT, NW>(a, per, blockIdx.x, blockIdx.y, blockIdx.z, gridDim.x, gridDim.y, s_kv);
+}
+
+#define PULSE_BESIDE (PULSE_HEAD_DIM <= 128)
+#if PULSE_BESIDE
+// A step's decoded tokens and its prompt portions in one launch, the decoded tokens' workgroups first: they wait for memory while
+// the portions' compute, and both leave compute units idle when alone.  (Head sizes whose portions leave two workgroups a unit.)
+// 24 tokens at contexts of 200 to 1,300 beside a portion of 333, 8 kv heads of 4, in a step: 31.5 + 15.8 us -> 38.5; with the
+// tokens' keys cut in two or three 36.4 + 4.7 and 36.1 + 5.6 for their merge.
+template <int CT, int KT, int NW>
+__global__ __launch_bounds__(NW* PULSE_WAVE) PULSE_ATTN_WAVES_PER_EU void attn_beside_kernel(MfmaArgs tokens, MfmaArgs portions, int per,
+                                                                                            int token_blocks, int items, int heads) {
+    static_assert(NW == WAVES, "workgroups of one size");
+    constexpr int KV = 2 * WideShape<CT, KT, NW>::STAGE * static_cast<int>(sizeof(bf16_t)), MERGE = sizeof(MfmaShared<false>);
+    __shared__ __attribute__((aligned(1024))) char lds[KV > MERGE ? KV : MERGE];
+    const int block = blockIdx.x;
+    if (block < token_blocks) {
+        attn_mfma_workgroup<false>(tokens, block, *reinterpret_cast<MfmaShared<false>*>(lds));
+    } else {
+        const int at = block - token_blocks;
+        attn_prefill_wide_workgroup<CT, KT, NW>(portions, per, at % items, at / items, 0, items, heads, reinterpret_cast<bf16_t*>(lds));
+    }
+}
+#endif
+
 // The merge of the prompt-portion kernel's splits: out[row, head, :] = sum_z w_z o_z / sum_z w_z l_z with
 // w_z = exp2(m_z - max m) over the splits that begin at or below the row's position, in the order of the splits.
 // A thread takes four channels of one head; rows of items that were finished in the first split are left alone.
@@ -1689,7 +1731,7 @@ int launch_attn_mfma(const void* q, int64_t q_stride, void* out, int64_t o_strid
                      int n_items, int tokens, int nq, int nkv, int page_size, int num_pages, float scale, int window,
                      int split_size, int n_splits, int max_context, float* part_o, float* part_ml,
                      const Preparation* prep, const int* live_context, const int* plan, const PulseAttnExtras* ex,
-                     hipStream_t stream) {
+                     hipStream_t stream, const MfmaArgs* portions = nullptr) {
     PULSE_REQUIRE(tokens >= 0 && n_items >= 0 && nq > 0 && nkv > 0, "attn_mfma: bad sizes");
     PULSE_REQUIRE(nq % nkv == 0, "attn_mfma: %d query heads are not a multiple of %d kv heads", nq, nkv);
     PULSE_REQUIRE(page_size > 0 && page_size % 16 == 0, "attn_mfma: page size %d must be a multiple of 16", page_size);
@@ -1746,6 +1788,12 @@ int launch_attn_mfma(const void* q, int64_t q_stride, void* out, int64_t o_strid
         a.pairing = prep->pairing; a.new_key = prep->new_key;
         hipLaunchKernelGGL(attn_mfma_kernel<true>, dim3(n_items * nkv * a.head_chunks * n_splits), dim3(WAVES * PULSE_WAVE),
                            0, stream, a);
+#if PULSE_WIDE && PULSE_BESIDE
+    } else if (portions) {
+        const int blocks = n_items * nkv * a.head_chunks * n_splits, heads = nkv * a.head_chunks;
+        hipLaunchKernelGGL((attn_beside_kernel<WIDE_CT, 4, WIDE_NW>), dim3(blocks + portions->n_items * heads), dim3(WAVES * PULSE_WAVE),
+                           0, stream, a, *portions, 16 / gp, blocks, portions->n_items, heads);
+#endif
     } else {
         hipLaunchKernelGGL(attn_mfma_kernel<false>, dim3(n_items * nkv * a.head_chunks * n_splits), dim3(WAVES * PULSE_WAVE),
                            0, stream, a);
@@ -1765,18 +1813,99 @@ int launch_attn_mfma(const void* q, int64_t q_stride, void* out, int64_t o_strid
 
 }  // namespace
 
+extern "C" int pulse_attn_prefill(const void* q, int64_t q_stride, void* out, int64_t o_stride, const void* kcache, const void* vcache,
+                                  const int* positions, const int* block_table, int bt_width, const int* items, int n_items, int tokens,
+                                  int nq, int nkv, int page_size, int num_pages, float scale, int window, int split_size, int n_splits,
+                                  float* part_o, float* part_ml, const PulseAttnExtras* extras, hipStream_t stream);
+
+// Extras of pulse_attn_mfma with a list of prompt portions behind them, told by plain_norm (which that entry point does not use).
+constexpr int ATTN_BESIDE = 2;
+struct PulseAttnBeside {
+    PulseAttnExtras extras;
+    const int* long_items;
+    int n_long;
+};
+
+namespace {
+
+constexpr int SPLIT_KEYS = PULSE_WIDE ? 64 : 0;
+
+// The arguments of the prompt-portion kernel, checked.
+int fill_portions(MfmaArgs& a, const void* q, int64_t q_stride, void* out, int64_t o_stride, const void* kcache, const void* vcache,
+                  const int* positions, const int* block_table, int bt_width, const int* items, int n_items, int tokens, int nq,
+                  int nkv, int page_size, int num_pages, float scale, int window, int split_size, int n_splits, float* part_o,
+                  float* part_ml, const PulseAttnExtras* extras) {
+    PULSE_REQUIRE(n_splits >= 1 && n_splits < 65536, "attn_prefill: bad number of splits %d", n_splits);
+    if (n_splits > 1) {
+        PULSE_REQUIRE(SPLIT_KEYS > 0, "attn_prefill: head size %d has no split variant", D);
+        PULSE_REQUIRE(split_size > 0 && split_size % SPLIT_KEYS == 0,
+                      "attn_prefill: split size %d must be a positive multiple of %d", split_size, SPLIT_KEYS);
+        PULSE_REQUIRE(part_o && part_ml && (reinterpret_cast<uintptr_t>(part_o) % 16) == 0,
+                      "attn_prefill: scratch for the split results is missing or not 16-byte aligned");
+    }
+    PULSE_REQUIRE(tokens >= 0 && n_items >= 0 && nq > 0 && nkv > 0, "attn_prefill: bad sizes");
+    PULSE_REQUIRE(nq % nkv == 0, "attn_prefill: %d query heads are not a multiple of %d kv heads", nq, nkv);
+    PULSE_REQUIRE(page_size > 0 && page_size % 16 == 0, "attn_prefill: page size %d must be a multiple of 16", page_size);
+    PULSE_REQUIRE(num_pages > 0 && bt_width > 0 && window >= 0, "attn_prefill: bad cache geometry");
+    PULSE_REQUIRE(q_stride % 8 == 0 && o_stride % 4 == 0 && q_stride >= static_cast<int64_t>(nq) * D &&
+                  o_stride >= static_cast<int64_t>(nq) * D, "attn_prefill: row strides must cover the heads and keep alignment");
+    PULSE_REQUIRE((reinterpret_cast<uintptr_t>(q) % 16) == 0 && (reinterpret_cast<uintptr_t>(kcache) % 16) == 0 &&
+                  (reinterpret_cast<uintptr_t>(vcache) % 16) == 0 && (reinterpret_cast<uintptr_t>(out) % 8) == 0,
+                  "attn_prefill: pointers must be 16-byte aligned");
+    PULSE_REQUIRE(static_cast<int64_t>(nkv) * ((nq / nkv + 15) / 16) < 65536, "attn_prefill: grid too large");
+    PULSE_REQUIRE(q && out && kcache && vcache && positions && block_table && items, "attn_prefill: null pointer");
+    const int group = nq / nkv;
+    int gp = 1;
+    while (gp < group && gp < 16) gp *= 2;
+    a.q = static_cast<const bf16_t*>(q); a.q_stride = q_stride;
+    a.out = static_cast<bf16_t*>(out); a.o_stride = o_stride;
+    a.part_o = nullptr; a.part_ml = nullptr;
+    a.kc = static_cast<const bf16_t*>(kcache); a.vc = static_cast<const bf16_t*>(vcache);
+    a.positions = positions; a.block_table = block_table; a.items = items;
+    a.bt_width = bt_width; a.nq = nq; a.nkv = nkv; a.group = group; a.gp = gp; a.head_chunks = (group + 15) / 16;
+    a.page_size = page_size; a.num_pages = num_pages;
+    a.page_shift = (page_size & (page_size - 1)) == 0 ? __builtin_ctz(page_size) : -1;
+    a.scale_log2e = scale * 1.4426950408889634f;
+    a.window = window; a.split_size = n_splits > 1 ? split_size : 0; a.n_splits = n_splits;
+    a.n_items = n_items;
+    a.live_context = nullptr;
+    a.plan = nullptr;
+    a.part_o = n_splits > 1 ? part_o : nullptr; a.part_ml = n_splits > 1 ? part_ml : nullptr;
+    if (tokens == 0 || n_items == 0) return 0;
+    return take_gate(a, extras, nq, scale);
+}
+
+}  // namespace
+
 // Scratch needed for `tokens` rows cut into `n_splits`: tokens * nq * n_splits * D floats of part_o, * 2 of part_ml.
 // live_context (device, or null): the longest context (last position + 1) among ALL items of this call as the step
 // has it; split_size and n_splits say what the launch is made for (max_context), and with live_context the kernel cuts
 // the keys that are there evenly into the same number of splits.  A value below an item's context loses keys.
 // plan (device, or null): what pulse_attn_plan made of these items and positions for this n_splits; it takes the
 // place of that even cut (every item then has a split size of its own and the workgroups an order).
+// extras with the tag of a PulseAttnBeside: its list of prompt portions (as pulse_attn_prefill's, every walk whole) goes in the same
+// launch where the head size has a kernel for both, else in one before it; the results are those of the two calls.
 extern "C" int pulse_attn_mfma(const void* q, int64_t q_stride, void* out, int64_t o_stride, const void* kcache,
                                const void* vcache, const int* positions, const int* block_table, int bt_width,
                                const int* items, int n_items, int tokens, int nq,
                                int nkv, int page_size, int num_pages, float scale, int window, int split_size,
                                int n_splits, int max_context, float* part_o, float* part_ml, const int* live_context,
                                const int* plan, const PulseAttnExtras* extras, hipStream_t stream) {
+    if (extras && extras->plain_norm == ATTN_BESIDE) {
+        const PulseAttnBeside* more = reinterpret_cast<const PulseAttnBeside*>(extras);
+        MfmaArgs portions;
+        if (fill_portions(portions, q, q_stride, out, o_stride, kcache, vcache, positions, block_table, bt_width, more->long_items,
+                          more->n_long, tokens, nq, nkv, page_size, num_pages, scale, window, 0, 1, nullptr, nullptr, extras)) return 1;
+        const int64_t heads = static_cast<int64_t>(nkv) * ((nq / nkv + 15) / 16);
+        const bool both = PULSE_WIDE && PULSE_HEAD_DIM <= 128 && tokens > 0 && n_items > 0 && more->n_long > 0 &&
+                          (static_cast<int64_t>(n_items) * n_splits + more->n_long) * heads < (int64_t{1} << 31);
+        if (both)
+            return launch_attn_mfma(q, q_stride, out, o_stride, kcache, vcache, positions, block_table, bt_width, items, n_items, tokens,
+                                    nq, nkv, page_size, num_pages, scale, window, split_size, n_splits, max_context, part_o, part_ml,
+                                    nullptr, live_context, plan, extras, stream, &portions);
+        if (pulse_attn_prefill(q, q_stride, out, o_stride, kcache, vcache, positions, block_table, bt_width, more->long_items, more->n_long,
+                               tokens, nq, nkv, page_size, num_pages, scale, window, 0, 1, nullptr, nullptr, extras, stream)) return 1;
+    }
     return launch_attn_mfma(q, q_stride, out, o_stride, kcache, vcache, positions, block_table, bt_width, items, n_items,
                             tokens, nq, nkv, page_size, num_pages, scale, window, split_size, n_splits, max_context,
                             part_o, part_ml, nullptr, live_context, plan, extras, stream);
@@ -1839,7 +1968,7 @@ extern "C" int pulse_attn_decode(const void* qkv, int64_t qkv_stride, void* out,
 }
 
 // Keys a split of the prompt-portion kernel must be a multiple of; 0 when this head size's kernel has no splits.
-extern "C" int pulse_attn_prefill_split_keys() { return PULSE_WIDE ? 64 : 0; }
+extern "C" int pulse_attn_prefill_split_keys() { return SPLIT_KEYS; }
 
 // Prompt portions: items of up to 4 * pulse_attn_prefill_tiles() * pulse_attn_mfma_tokens_per_item(group) tokens of one
 // request, a workgroup each (and per split), keys shared through LDS.  With n_splits > 1 (head sizes for which
@@ -1851,44 +1980,11 @@ extern "C" int pulse_attn_prefill(const void* q, int64_t q_stride, void* out, in
                                   int nq, int nkv, int page_size, int num_pages, float scale, int window,
                                   int split_size, int n_splits, float* part_o, float* part_ml,
                                   const PulseAttnExtras* extras, hipStream_t stream) {
-    PULSE_REQUIRE(n_splits >= 1 && n_splits < 65536, "attn_prefill: bad number of splits %d", n_splits);
-    if (n_splits > 1) {
-        PULSE_REQUIRE(pulse_attn_prefill_split_keys() > 0, "attn_prefill: head size %d has no split variant", D);
-        PULSE_REQUIRE(split_size > 0 && split_size % pulse_attn_prefill_split_keys() == 0,
-                      "attn_prefill: split size %d must be a positive multiple of %d", split_size, pulse_attn_prefill_split_keys());
-        PULSE_REQUIRE(part_o && part_ml && (reinterpret_cast<uintptr_t>(part_o) % 16) == 0,
-                      "attn_prefill: scratch for the split results is missing or not 16-byte aligned");
-    }
-    PULSE_REQUIRE(tokens >= 0 && n_items >= 0 && nq > 0 && nkv > 0, "attn_prefill: bad sizes");
-    PULSE_REQUIRE(nq % nkv == 0, "attn_prefill: %d query heads are not a multiple of %d kv heads", nq, nkv);
-    PULSE_REQUIRE(page_size > 0 && page_size % 16 == 0, "attn_prefill: page size %d must be a multiple of 16", page_size);
-    PULSE_REQUIRE(num_pages > 0 && bt_width > 0 && window >= 0, "attn_prefill: bad cache geometry");
-    PULSE_REQUIRE(q_stride % 8 == 0 && o_stride % 4 == 0 && q_stride >= static_cast<int64_t>(nq) * D &&
-                  o_stride >= static_cast<int64_t>(nq) * D, "attn_prefill: row strides must cover the heads and keep alignment");
-    PULSE_REQUIRE((reinterpret_cast<uintptr_t>(q) % 16) == 0 && (reinterpret_cast<uintptr_t>(kcache) % 16) == 0 &&
-                  (reinterpret_cast<uintptr_t>(vcache) % 16) == 0 && (reinterpret_cast<uintptr_t>(out) % 8) == 0,
-                  "attn_prefill: pointers must be 16-byte aligned");
-    PULSE_REQUIRE(static_cast<int64_t>(nkv) * ((nq / nkv + 15) / 16) < 65536, "attn_prefill: grid too large");
-    PULSE_REQUIRE(q && out && kcache && vcache && positions && block_table && items, "attn_prefill: null pointer");
-    if (tokens == 0 || n_items == 0) return 0;
-    const int group = nq / nkv;
-    int gp = 1;
-    while (gp < group && gp < 16) gp *= 2;
     MfmaArgs a;
-    a.q = static_cast<const bf16_t*>(q); a.q_stride = q_stride;
-    a.out = static_cast<bf16_t*>(out); a.o_stride = o_stride;
-    a.part_o = nullptr; a.part_ml = nullptr;
-    a.kc = static_cast<const bf16_t*>(kcache); a.vc = static_cast<const bf16_t*>(vcache);
-    a.positions = positions; a.block_table = block_table; a.items = items;
-    a.bt_width = bt_width; a.nq = nq; a.nkv = nkv; a.group = group; a.gp = gp; a.head_chunks = (group + 15) / 16;
-    a.page_size = page_size; a.num_pages = num_pages;
-    a.page_shift = (page_size & (page_size - 1)) == 0 ? __builtin_ctz(page_size) : -1;
-    a.scale_log2e = scale * 1.4426950408889634f;
-    a.window = window; a.split_size = n_splits > 1 ? split_size : 0; a.n_splits = n_splits;
-    a.live_context = nullptr;
-    a.plan = nullptr;
-    a.part_o = n_splits > 1 ? part_o : nullptr; a.part_ml = n_splits > 1 ? part_ml : nullptr;
-    if (take_gate(a, extras, nq, scale)) return 1;
+    if (fill_portions(a, q, q_stride, out, o_stride, kcache, vcache, positions, block_table, bt_width, items, n_items, tokens, nq, nkv,
+                      page_size, num_pages, scale, window, split_size, n_splits, part_o, part_ml, extras)) return 1;
+    if (tokens == 0 || n_items == 0) return 0;
+    const int gp = a.gp;
 #if PULSE_WIDE
     hipLaunchKernelGGL((attn_prefill_wide_kernel<WIDE_CT, 4, WIDE_NW>), dim3(n_items, nkv * a.head_chunks, n_splits),
                        dim3(WIDE_NW * PULSE_WAVE), 0, stream, a, 16 / gp);

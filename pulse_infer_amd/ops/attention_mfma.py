@@ -28,9 +28,15 @@ class _Extras(ctypes.Structure):
                 ("chunk", ctypes.c_int)]
 
 
+class _Beside(_Extras):
+    # as PulseAttnBeside of the kernel source: told by plain_norm = 2
+    _fields_ = [("long_items", ctypes.c_void_p), ("n_long", ctypes.c_int)]
+
+
 def _extras(what: str, tokens: int, nq: int, gate: Optional[torch.Tensor] = None, plain_norm: bool = False,
             v_head0: int = -1, q_temperature: Optional[Tuple[float, int]] = None, gate_width: int = 0,
-            sink: Optional[torch.Tensor] = None, softcap: float = 0.0, chunk: int = 0):
+            sink: Optional[torch.Tensor] = None, softcap: float = 0.0, chunk: int = 0,
+            long_items: Optional[torch.Tensor] = None):
     """What the entry points take besides their lists, or a null pointer when there is none of it.  ``gate``: bfloat16
     [tokens, nq] (rows may be strided), the logits of an output gate: head h of token t leaves the kernel multiplied
     by sigmoid(gate[t, h]).  The rest is for ``attn_decode``: a norm of q and k without weights, the head number at
@@ -38,11 +44,17 @@ def _extras(what: str, tokens: int, nq: int, gate: Optional[torch.Tensor] = None
     q *= 1 + coef * ln(floor((position + 1) / every) + 1).  ``gate_width`` > 0: the gate holds a logit for each of the
     first ``gate_width`` channels of every head ([tokens, nq * gate_width]).  ``sink`` float32 [nq]: exp(sink[h]) is one
     more term of head h's softmax denominator; ``softcap`` > 0: scaled scores become cap * tanh(score / cap); ``chunk`` > 0:
-    a token sees only the keys of its own chunk of that many positions, counted from 0."""
+    a token sees only the keys of its own chunk of that many positions, counted from 0; ``long_items`` (``attn_mfma``
+    only): the items of prompt portions that go with the others."""
     if (gate is None and not plain_norm and v_head0 < 0 and q_temperature is None and sink is None and not softcap
-            and not chunk):
+            and not chunk and long_items is None):
         return None
-    ex = _Extras()
+    ex = _Extras() if long_items is None else _Beside()
+    if long_items is not None:
+        _gpu(what, long_items)
+        _need(not plain_norm and long_items.dtype == torch.int32 and long_items.is_contiguous()
+              and long_items.numel() % ITEM_INTS == 0, f"{what}: items must be int32 quadruples")
+        ex.long_items, ex.n_long = long_items.data_ptr(), long_items.numel() // ITEM_INTS
     if gate is not None:
         _gpu(what, gate)
         cols = nq * max(1, gate_width)
@@ -60,7 +72,7 @@ def _extras(what: str, tokens: int, nq: int, gate: Optional[torch.Tensor] = None
     ex.softcap = float(softcap)
     _need(chunk >= 0, f"{what}: a chunk must not be negative")
     ex.chunk = int(chunk)
-    ex.plain_norm = 1 if plain_norm else 0
+    ex.plain_norm = 2 if long_items is not None else 1 if plain_norm else 0
     ex.v_head0 = int(v_head0)
     if q_temperature is not None:
         coef, every = q_temperature
@@ -167,11 +179,13 @@ def attn_mfma(q: torch.Tensor, out: torch.Tensor, nq: int, nkv: int, d: int, kca
               part_o: Optional[torch.Tensor], part_ml: Optional[torch.Tensor],
               live_context: Optional[torch.Tensor] = None, plan: Optional[torch.Tensor] = None,
               gate: Optional[torch.Tensor] = None, gate_width: int = 0, sink: Optional[torch.Tensor] = None,
-              softcap: float = 0.0, chunk: int = 0) -> None:
+              softcap: float = 0.0, chunk: int = 0, long_items: Optional[torch.Tensor] = None) -> None:
     """Attention of decoded tokens and short portions.  ``split_size`` x ``n_splits`` is what the launch is made for
     (contexts up to ``max_context``); ``live_context`` (one int32 on the device: the longest context among the step's
     entries as it is now) lets the kernel cut the keys that are there evenly into the same number of splits;
-    ``plan`` (what ``attn_plan`` made of these items for this ``n_splits``) takes the place of that even cut."""
+    ``plan`` (what ``attn_plan`` made of these items for this ``n_splits``) takes the place of that even cut.
+    ``long_items``: the items of prompt portions (as for ``attn_prefill``, every walk whole), in the same launch where the
+    head size has a kernel for both."""
     _gpu("attn_mfma", q, out, kcache, vcache, positions, block_table, items, part_o, part_ml, live_context, plan)
     _live(live_context)
     _planned(plan, items.numel() // ITEM_INTS, n_splits)
@@ -199,7 +213,7 @@ def attn_mfma(q: torch.Tensor, out: torch.Tensor, nq: int, nkv: int, d: int, kca
             _ptr(items), _i32(n_items), _i32(tokens), _i32(nq), _i32(nkv), _i32(page_size), _i32(pages), _f32(scale),
             _i32(window), _i32(split_size), _i32(n_splits), _i32(max_context), _ptr(part_o), _ptr(part_ml),
             _ptr(live_context), _ptr(plan), _extras("attn_mfma", tokens, nq, gate, gate_width=gate_width, sink=sink, softcap=softcap,
-            chunk=chunk), _stream())
+            chunk=chunk, long_items=long_items), _stream())
 
 
 PLAN_MIN_KEYS = 256      # no split of a plan is shorter (what a workgroup costs beside its walk, in keys walked)

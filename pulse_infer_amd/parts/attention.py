@@ -268,6 +268,7 @@ class PagedAttention(Part):
                 dev(attention_mfma.build_items(long, portion)),
                 max((e.start + e.count for _, e in short), default=0))
         short_items, long_items, short_context = ctx.extras[key]
+        beside = False
         if long_items is not None:
             skey = f"static:attention.portion_splits:{portion}:{window or self.chunk}:{self.nkv}:{group}:{self.d}"
             if skey not in ctx.extras:
@@ -276,14 +277,17 @@ class PagedAttention(Part):
                     window or self.chunk)
             split_size, n_splits = ctx.extras[skey]
             part_o = part_ml = None
+            # (portions whose walks are whole go in the launch of the single tokens and short portions, if there are any)
+            beside = short_items is not None and n_splits == 1
             if n_splits > 1:
                 rows = ctx.num_tokens * self.nq * n_splits
                 part_o = ctx.workspace.buffer("attention.portion_part_o", rows, self.d, torch.float32)
                 part_ml = ctx.workspace.buffer("attention.portion_part_ml", rows, 2, torch.float32)
-            attention_mfma.attn_prefill(q, out, self.nq, self.nkv, self.d, cache.keys, cache.values, ctx.positions,
-                                        table, long_items, self.scale, window, split_size, n_splits, part_o, part_ml,
-                                        gate=gate, gate_width=self.gate_width, sink=self.sink, softcap=self.score_cap,
-                                        chunk=self.chunk)
+            if not beside:
+                attention_mfma.attn_prefill(q, out, self.nq, self.nkv, self.d, cache.keys, cache.values, ctx.positions,
+                                            table, long_items, self.scale, window, split_size, n_splits, part_o, part_ml,
+                                            gate=gate, gate_width=self.gate_width, sink=self.sink, softcap=self.score_cap,
+                                            chunk=self.chunk)
         if short_items is not None:
             # a recorded step passes its context bucket as max_context: its splits must cover that
             max_context = ctx.max_context if long_items is None else short_context
@@ -328,4 +332,5 @@ class PagedAttention(Part):
                                      table, short_items, self.scale, window, split_size, n_splits,
                                      max_context, part_o, part_ml,
                                      live_context=ctx.live_context if plan is None else None, plan=plan, gate=gate,
-                                     gate_width=self.gate_width, sink=self.sink, softcap=self.score_cap, chunk=self.chunk)
+                                     gate_width=self.gate_width, sink=self.sink, softcap=self.score_cap, chunk=self.chunk,
+                                     long_items=long_items if beside else None)

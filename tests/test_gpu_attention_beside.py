@@ -1,0 +1,46 @@
+"""Decoded tokens, short portions and prompt portions in one attention launch: the bits of the two launches it stands for."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+class Entry:
+    def __init__(self, start, count, first_row):
+        self.start, self.count, self.first_row = start, count, first_row
+
+
+# head sizes with a kernel for both and without; whole walks and splits of the tokens' keys, one item and many, a window, chunks
+@pytest.mark.parametrize("d", [128, 64, 32, 192, 80])
+@pytest.mark.parametrize("nq,nkv,splits,window,chunk", [(8, 2, 1, 0, 0), (32, 8, 4, 0, 0), (4, 4, 3, 0, 0), (8, 2, 1, 40, 0),
+                                                       (8, 2, 1, 0, 96)])
+def test_tokens_and_portions_in_one_launch(d, nq, nkv, splits, window, chunk):
+    from pulse_infer_amd.ops import attention_mfma as am
+
+    page, lengths = 16, [(0, 1), (300, 1), (77, 3), (0, 200), (130, 33), (511, 1), (5, 16)]
+    gen = torch.Generator().manual_seed(d + nq)
+    entries, rows = [], 0
+    for start, count in lengths:
+        entries.append(Entry(start, count, rows))
+        rows += count
+    width = max((e.start + e.count + page - 1) // page for e in entries)
+    pages = len(entries) * width
+    table = torch.randperm(pages, generator=gen).to(torch.int32).view(len(entries), width).to(DEV)
+    bf = lambda *s: torch.randn(s, generator=gen).to(torch.bfloat16).to(DEV)
+    q, kc, vc = bf(rows, nq * d), bf(pages, nkv, page, d), bf(pages, nkv, d, page)
+    positions = torch.tensor([e.start + i for e in entries for i in range(e.count)], dtype=torch.int32, device=DEV)
+    group = nq // nkv
+    short, long = am.split_entries(entries)
+    dev = lambda flat: torch.tensor(flat, dtype=torch.int32, device=DEV)
+    short_items = dev(am.build_items(short, am.tokens_per_item(group)))
+    long_items = dev(am.build_items(long, am.portion_tokens(group, d)))
+    context = max(e.start + e.count for _, e in short)
+    size = ((context + splits - 1) // splits + 31) // 32 * 32
+    part_o, part_ml = torch.empty(rows * nq * splits * d, device=DEV), torch.empty(rows * nq * splits * 2, device=DEV)
+    one, two = (torch.full((rows, nq * d), float("nan"), dtype=torch.bfloat16, device=DEV) for _ in range(2))
+    tail = (d ** -0.5, window, size, splits, context, part_o, part_ml)
+    am.attn_prefill(q, two, nq, nkv, d, kc, vc, positions, table, long_items, d ** -0.5, window, chunk=chunk)
+    am.attn_mfma(q, two, nq, nkv, d, kc, vc, positions, table, short_items, *tail, chunk=chunk)
+    am.attn_mfma(q, one, nq, nkv, d, kc, vc, positions, table, short_items, *tail, chunk=chunk, long_items=long_items)
+    assert not torch.isnan(two).any() and torch.equal(one, two)
