@@ -999,14 +999,16 @@ __device__ __forceinline__ constexpr int piece_rot(int j, int P) {
     return P >= 8 ? ((j & 3) | (((j >> 3) & 1) << 2)) : (((j >> 1) & 1) | (((j >> 3) & 1) << 1));
 }
 
-template <int CT, int KT, int NW>
+// VD: the value channels of a head that are not fill (a multiple of 32); only these are read and computed.
+template <int CT, int KT, int NW, int VD = D>
 struct WideShape {
     static constexpr int BK = KT * 16;                    // keys a block
     static constexpr int P = D / 8;                       // 16-byte pieces a key row
     static constexpr int STAGE_K = BK * D;                // bfloat16 elements
-    static constexpr int STAGE_V = KT * D * 16;
+    static constexpr int STAGE_V = KT * VD * 16;
     static constexpr int STAGE = STAGE_K + STAGE_V;
-    static constexpr int TILE_CHUNKS = 16 * P / 64;       // 1 KB chunks (one load of a wavefront) of a key tile; as many of a value tile
+    static constexpr int TILE_CHUNKS = 16 * P / 64;       // 1 KB chunks (one load of a wavefront) of a key tile
+    static constexpr int VALUE_CHUNKS = VD / 32;          // and of a value tile
     static_assert(KT == NW, "a wavefront copies one key tile and one value tile of every block");
 };
 
@@ -1016,10 +1018,11 @@ struct WideShape {
 #define PULSE_WIDE_WAVES_PER_EU PULSE_ATTN_WAVES_PER_EU
 #endif
 // s_kv: 2 * Shape::STAGE values of LDS, a stage after the other, the K block first; (bx, by, bz) of (items, heads, splits): the workgroup.
-template <int CT, int KT, int NW>
+template <int CT, int KT, int NW, int VD>
 __device__ __forceinline__ void attn_prefill_wide_workgroup(const MfmaArgs& a, const int per, const int bx, const int by, const int bz,
                                                             const int items, const int heads, bf16_t* const s_kv) {
-    using Shape = WideShape<CT, KT, NW>;
+    using Shape = WideShape<CT, KT, NW, VD>;
+    constexpr int NVT = VD / 16;            // tiles of 16 value channels
     constexpr int BK = Shape::BK;
     static_assert(KT % 2 == 0, "the second product takes pairs of key tiles");
     static_assert(D == 32 || D == 64 || D == 128 || D == 192, "whole 1 KB chunks, and key rows that start at the same place of 128 bytes or divide them");
@@ -1092,12 +1095,12 @@ __device__ __forceinline__ void attn_prefill_wide_workgroup(const MfmaArgs& a, c
             bq[ct][ch] = (col_ok[ct] && off < D) ? *reinterpret_cast<const bf16x8*>(qrow + off) : zero8();
         }
     }
-    f32x4 acc[CT][NDT];
+    f32x4 acc[CT][NVT];
     float m[CT], l_part[CT];
 #pragma unroll
     for (int ct = 0; ct < CT; ++ct) {
 #pragma unroll
-        for (int dt = 0; dt < NDT; ++dt) acc[ct][dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int dt = 0; dt < NVT; ++dt) acc[ct][dt] = f32x4{0.f, 0.f, 0.f, 0.f};
         m[ct] = -INFINITY;
         l_part[ct] = 0.f;
     }
@@ -1107,13 +1110,17 @@ __device__ __forceinline__ void attn_prefill_wide_workgroup(const MfmaArgs& a, c
     // wavefront's tile changes from block to block.
     const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(
         (void __attribute__((address_space(3)))*)(&s_kv[0])));  // the array's address inside LDS
-    int k_from[Shape::TILE_CHUNKS], v_from[Shape::TILE_CHUNKS];
+    int k_from[Shape::TILE_CHUNKS], v_from[Shape::VALUE_CHUNKS];
 #pragma unroll
     for (int i = 0; i < Shape::TILE_CHUNKS; ++i) {
         const int slot = 64 * i + lane;         // within the tile's 16 * P slots
         const int key = slot / P, pos = slot % P;
         const int c8 = (pos - piece_rot(key, P) + P) % P;
         k_from[i] = key * D + c8 * 8;
+    }
+#pragma unroll
+    for (int i = 0; i < Shape::VALUE_CHUNKS; ++i) {
+        const int slot = 64 * i + lane;
         const int blk = slot / 32, half = (slot / 16) % 2, chr = slot % 16;
         v_from[i] = (blk * 16 + chr) * a.page_size + half * 8;
     }
@@ -1150,11 +1157,12 @@ __device__ __forceinline__ void attn_prefill_wide_workgroup(const MfmaArgs& a, c
         const int64_t base = page * page_elems + head_elems;
         const bf16_t* kfrom = a.kc + base + slot0 * D;
         const bf16_t* vfrom = a.vc + base + slot0;
-        const uint32_t to = lds0 + stage * (Shape::STAGE * 2) + wave * (Shape::TILE_CHUNKS * 1024);
+        const uint32_t stage0 = lds0 + stage * (Shape::STAGE * 2), to = stage0 + wave * (Shape::TILE_CHUNKS * 1024);
+        const uint32_t values_to = stage0 + Shape::STAGE_K * 2 + wave * (Shape::VALUE_CHUNKS * 1024);
 #pragma unroll
         for (int i = 0; i < Shape::TILE_CHUNKS; ++i) load_to_lds(kfrom + k_from[i], to + i * 1024);
 #pragma unroll
-        for (int i = 0; i < Shape::TILE_CHUNKS; ++i) load_to_lds(vfrom + v_from[i], to + Shape::STAGE_K * 2 + i * 1024);
+        for (int i = 0; i < Shape::VALUE_CHUNKS; ++i) load_to_lds(vfrom + v_from[i], values_to + i * 1024);
     };
     // Operand reads.  Row r of score tile t is not key 16 t + r but key 32 (t / 2) + 8 (r / 4) + 4 (t % 2) + r % 4 of
     // the block: the four rows that lane group kg gets back of tiles 2 ks and 2 ks + 1 are then the eight
@@ -1168,7 +1176,7 @@ __device__ __forceinline__ void attn_prefill_wide_workgroup(const MfmaArgs& a, c
 #pragma unroll
         for (int ch = 0; ch < NCHUNK; ++ch) k_at[par][ch] = (row * P + (4 * ch + kg + piece_rot(row, P)) % P) * 8;
     }
-    const int v_at = (kg >> 1) * D * 16 + ((kg & 1) * 16 + r) * 8;
+    const int v_at = (kg >> 1) * VD * 16 + ((kg & 1) * 16 + r) * 8;
 
     const float c2 = a.scale_log2e;
     constexpr float LAZY_BITS = 8.f;
@@ -1203,10 +1211,10 @@ __device__ __forceinline__ void attn_prefill_wide_workgroup(const MfmaArgs& a, c
             }
         }
         // the first value operands are asked for before the weights are computed, the rest as the products go
-        constexpr int V_STEPS = (KT / 2) * NDT;
+        constexpr int V_STEPS = (KT / 2) * NVT;
         auto v_read = [&](int i) {
-            const int ks = i / NDT, dt = i % NDT;
-            return *reinterpret_cast<const u32x4*>(&s_v[(2 * ks) * D * 16 + dt * 256 + v_at]);
+            const int ks = i / NVT, dt = i % NVT;
+            return *reinterpret_cast<const u32x4*>(&s_v[(2 * ks) * VD * 16 + dt * 256 + v_at]);
         };
         u32x4 vw[V_STEPS];
 #pragma unroll
@@ -1276,13 +1284,13 @@ __device__ __forceinline__ void attn_prefill_wide_workgroup(const MfmaArgs& a, c
 #pragma unroll
             for (int ct = 0; ct < CT; ++ct)
 #pragma unroll
-                for (int dt = 0; dt < NDT; ++dt) acc[ct][dt] = acc[ct][dt] * alpha[ct];
+                for (int dt = 0; dt < NVT; ++dt) acc[ct][dt] = acc[ct][dt] * alpha[ct];
         }
         // (values under keys outside [lo_item, hi] have been cleared in LDS by clear_stale before this block is computed)
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int i = 0; i < V_STEPS; ++i) {
-            const int ks = i / NDT, dt = i % NDT;
+            const int ks = i / NVT, dt = i % NVT;
             if (i + AHEAD < V_STEPS) vw[i + AHEAD] = v_read(i + AHEAD);
 #pragma unroll
             for (int ct = 0; ct < CT; ++ct)
@@ -1299,14 +1307,14 @@ __device__ __forceinline__ void attn_prefill_wide_workgroup(const MfmaArgs& a, c
         bf16_t* s_v = s_kv + stage * Shape::STAGE + Shape::STAGE_K;
 #pragma unroll
         for (int t = 0; t < KT; ++t)
-            for (int piece = tid; piece < 2 * D; piece += NW * PULSE_WAVE) {
+            for (int piece = tid; piece < 2 * VD; piece += NW * PULSE_WAVE) {
                 const int j = b * BK + 16 * t + 8 * ((piece / 16) % 2);    // the piece's first key
                 u32x4 mask;
 #pragma unroll
                 for (int w = 0; w < 4; ++w)
                     mask[w] = ((j + 2 * w <= hi && j + 2 * w >= lo_item) ? 0x0000ffffu : 0u) |
                               ((j + 2 * w + 1 <= hi && j + 2 * w + 1 >= lo_item) ? 0xffff0000u : 0u);
-                u32x4* at = reinterpret_cast<u32x4*>(s_v + t * D * 16 + piece * 8);
+                u32x4* at = reinterpret_cast<u32x4*>(s_v + t * VD * 16 + piece * 8);
                 *at = *at & mask;
             }
     };
@@ -1352,7 +1360,7 @@ __device__ __forceinline__ void attn_prefill_wide_workgroup(const MfmaArgs& a, c
             const float inv = gated(l > 0.f ? 1.0f / l : 0.f, a.gate, a.gate_stride, col_row[ct], col_head, a.gate_width);
             bf16_t* dst = a.out + static_cast<int64_t>(col_row[ct]) * a.o_stride + static_cast<int64_t>(col_head) * D;
 #pragma unroll
-            for (int dt = 0; dt < NDT; ++dt) {
+            for (int dt = 0; dt < NVT; ++dt) {
                 if (a.gate_width > 0) {
 #pragma unroll
                     for (int i = 0; i < 4; ++i)
@@ -1370,7 +1378,7 @@ __device__ __forceinline__ void attn_prefill_wide_workgroup(const MfmaArgs& a, c
             const int64_t slot = (static_cast<int64_t>(col_row[ct]) * a.nq + col_head) * a.n_splits + split;
             float* dst = a.part_o + slot * D;
 #pragma unroll
-            for (int dt = 0; dt < NDT; ++dt) *reinterpret_cast<f32x4*>(dst + dt * 16 + 4 * kg) = acc[ct][dt];
+            for (int dt = 0; dt < NVT; ++dt) *reinterpret_cast<f32x4*>(dst + dt * 16 + 4 * kg) = acc[ct][dt];
             if (kg == 0) {
                 a.part_ml[2 * slot] = m[ct] == -INFINITY ? -INFINITY : m[ct] * c2;
                 a.part_ml[2 * slot + 1] = l;
@@ -1382,8 +1390,21 @@ __device__ __forceinline__ void attn_prefill_wide_workgroup(const MfmaArgs& a, c
 template <int CT, int KT, int NW>
 __global__ __launch_bounds__(NW* PULSE_WAVE) PULSE_WIDE_WAVES_PER_EU void attn_prefill_wide_kernel(MfmaArgs a, int per) {
     __shared__ __attribute__((aligned(1024))) bf16_t s_kv[2 * WideShape<CT, KT, NW>::STAGE];
-    attn_prefill_wide_workgroup<CT, KT, NW>(a, per, blockIdx.x, blockIdx.y, blockIdx.z, gridDim.x, gridDim.y, s_kv);
+    attn_prefill_wide_workgroup<CT, KT, NW, D>(a, per, blockIdx.x, blockIdx.y, blockIdx.z, gridDim.x, gridDim.y, s_kv);
 }
+
+#define PULSE_NARROW_VALUES (PULSE_HEAD_DIM == 192 && PULSE_WIDE_CT == 2)
+#if PULSE_NARROW_VALUES
+// Heads of 192 channels whose values fill 128 of them at most (the latent rows' expanded form): the stages are then 80 KB instead of
+// 96, so that two workgroups share a unit, two wavefronts a SIMD, and a sixth of the products falls away.  32 heads, a prompt of
+// 2,048: 192 -> 79 us, with the same bits.
+constexpr int NARROW_VALUES = 128;
+template <int CT, int KT, int NW>
+__global__ __launch_bounds__(NW* PULSE_WAVE) __attribute__((amdgpu_waves_per_eu(2))) void attn_prefill_values_kernel(MfmaArgs a, int per) {
+    __shared__ __attribute__((aligned(1024))) bf16_t s_kv[2 * WideShape<CT, KT, NW, NARROW_VALUES>::STAGE];
+    attn_prefill_wide_workgroup<CT, KT, NW, NARROW_VALUES>(a, per, blockIdx.x, blockIdx.y, blockIdx.z, gridDim.x, gridDim.y, s_kv);
+}
+#endif
 
 #define PULSE_BESIDE (PULSE_HEAD_DIM <= 128)
 #if PULSE_BESIDE
@@ -1402,7 +1423,7 @@ __global__ __launch_bounds__(NW* PULSE_WAVE) PULSE_ATTN_WAVES_PER_EU void attn_b
         attn_mfma_workgroup<false>(tokens, block, *reinterpret_cast<MfmaShared<false>*>(lds));
     } else {
         const int at = block - token_blocks;
-        attn_prefill_wide_workgroup<CT, KT, NW>(portions, per, at % items, at / items, 0, items, heads, reinterpret_cast<bf16_t*>(lds));
+        attn_prefill_wide_workgroup<CT, KT, NW, D>(portions, per, at % items, at / items, 0, items, heads, reinterpret_cast<bf16_t*>(lds));
     }
 }
 #endif
@@ -1818,8 +1839,13 @@ extern "C" int pulse_attn_prefill(const void* q, int64_t q_stride, void* out, in
                                   int nq, int nkv, int page_size, int num_pages, float scale, int window, int split_size, int n_splits,
                                   float* part_o, float* part_ml, const PulseAttnExtras* extras, hipStream_t stream);
 
-// Extras of pulse_attn_mfma with a list of prompt portions behind them, told by plain_norm (which that entry point does not use).
-constexpr int ATTN_BESIDE = 2;
+// Extras with more behind them, told by plain_norm, which these entry points do not use: for pulse_attn_mfma a list of prompt portions;
+// for pulse_attn_prefill how many of a head's value channels are no fill (those behind them need not be computed).
+constexpr int ATTN_BESIDE = 2, ATTN_VALUES = 3;
+struct PulseAttnValues {
+    PulseAttnExtras extras;
+    int values;
+};
 struct PulseAttnBeside {
     PulseAttnExtras extras;
     const int* long_items;
@@ -1985,6 +2011,14 @@ extern "C" int pulse_attn_prefill(const void* q, int64_t q_stride, void* out, in
                       page_size, num_pages, scale, window, split_size, n_splits, part_o, part_ml, extras)) return 1;
     if (tokens == 0 || n_items == 0) return 0;
     const int gp = a.gp;
+    const int values = extras && extras->plain_norm == ATTN_VALUES ? reinterpret_cast<const PulseAttnValues*>(extras)->values : D;
+    PULSE_REQUIRE(values > 0 && values <= D, "attn_prefill: %d value channels of a head of %d", values, D);
+#if PULSE_WIDE && PULSE_NARROW_VALUES
+    if (values <= NARROW_VALUES)
+        hipLaunchKernelGGL((attn_prefill_values_kernel<WIDE_CT, 4, WIDE_NW>), dim3(n_items, nkv * a.head_chunks, n_splits),
+                           dim3(WIDE_NW * PULSE_WAVE), 0, stream, a, 16 / gp);
+    else
+#endif
 #if PULSE_WIDE
     hipLaunchKernelGGL((attn_prefill_wide_kernel<WIDE_CT, 4, WIDE_NW>), dim3(n_items, nkv * a.head_chunks, n_splits),
                        dim3(WIDE_NW * PULSE_WAVE), 0, stream, a, 16 / gp);

@@ -33,10 +33,15 @@ class _Beside(_Extras):
     _fields_ = [("long_items", ctypes.c_void_p), ("n_long", ctypes.c_int)]
 
 
+class _Values(_Extras):
+    # as PulseAttnValues of the kernel source: told by plain_norm = 3
+    _fields_ = [("values", ctypes.c_int)]
+
+
 def _extras(what: str, tokens: int, nq: int, gate: Optional[torch.Tensor] = None, plain_norm: bool = False,
             v_head0: int = -1, q_temperature: Optional[Tuple[float, int]] = None, gate_width: int = 0,
             sink: Optional[torch.Tensor] = None, softcap: float = 0.0, chunk: int = 0,
-            long_items: Optional[torch.Tensor] = None):
+            long_items: Optional[torch.Tensor] = None, values: int = 0):
     """What the entry points take besides their lists, or a null pointer when there is none of it.  ``gate``: bfloat16
     [tokens, nq] (rows may be strided), the logits of an output gate: head h of token t leaves the kernel multiplied
     by sigmoid(gate[t, h]).  The rest is for ``attn_decode``: a norm of q and k without weights, the head number at
@@ -45,16 +50,20 @@ def _extras(what: str, tokens: int, nq: int, gate: Optional[torch.Tensor] = None
     first ``gate_width`` channels of every head ([tokens, nq * gate_width]).  ``sink`` float32 [nq]: exp(sink[h]) is one
     more term of head h's softmax denominator; ``softcap`` > 0: scaled scores become cap * tanh(score / cap); ``chunk`` > 0:
     a token sees only the keys of its own chunk of that many positions, counted from 0; ``long_items`` (``attn_mfma``
-    only): the items of prompt portions that go with the others."""
+    only): the items of prompt portions that go with the others; ``values`` > 0 (``attn_prefill`` only): so many of a head's
+    value channels are wanted, those behind them may be left out."""
     if (gate is None and not plain_norm and v_head0 < 0 and q_temperature is None and sink is None and not softcap
-            and not chunk and long_items is None):
+            and not chunk and long_items is None and not values):
         return None
-    ex = _Extras() if long_items is None else _Beside()
+    ex = _Beside() if long_items is not None else _Values() if values else _Extras()
     if long_items is not None:
         _gpu(what, long_items)
         _need(not plain_norm and long_items.dtype == torch.int32 and long_items.is_contiguous()
               and long_items.numel() % ITEM_INTS == 0, f"{what}: items must be int32 quadruples")
         ex.long_items, ex.n_long = long_items.data_ptr(), long_items.numel() // ITEM_INTS
+    if values:
+        _need(not plain_norm and long_items is None, f"{what}: value channels are for prompt portions alone")
+        ex.values = int(values)
     if gate is not None:
         _gpu(what, gate)
         cols = nq * max(1, gate_width)
@@ -72,7 +81,7 @@ def _extras(what: str, tokens: int, nq: int, gate: Optional[torch.Tensor] = None
     ex.softcap = float(softcap)
     _need(chunk >= 0, f"{what}: a chunk must not be negative")
     ex.chunk = int(chunk)
-    ex.plain_norm = 2 if long_items is not None else 1 if plain_norm else 0
+    ex.plain_norm = 2 if long_items is not None else 3 if values else 1 if plain_norm else 0
     ex.v_head0 = int(v_head0)
     if q_temperature is not None:
         coef, every = q_temperature
@@ -341,13 +350,14 @@ def attn_prefill(q: torch.Tensor, out: torch.Tensor, nq: int, nkv: int, d: int, 
                  items: torch.Tensor, scale: float, window: int, split_size: int = 0, n_splits: int = 1,
                  part_o: Optional[torch.Tensor] = None, part_ml: Optional[torch.Tensor] = None,
                  gate: Optional[torch.Tensor] = None, gate_width: int = 0, sink: Optional[torch.Tensor] = None,
-                 softcap: float = 0.0, chunk: int = 0) -> None:
+                 softcap: float = 0.0, chunk: int = 0, values: int = 0) -> None:
     """Attention for prompt portions: items of up to portion_tokens(group, d) tokens, keys shared through LDS.
     With ``n_splits > 1`` the keys are walked in splits of ``split_size`` (a multiple of 64) by workgroups of their
     own and merged by a second kernel; ``part_o`` / ``part_ml`` are float32 scratch of tokens * nq * n_splits * d
-    and * 2 elements."""
+    and * 2 elements.  ``values`` > 0: the first ``values`` channels of a head are wanted, ``out`` holds anything in the others."""
     _gpu("attn_prefill", q, out, kcache, vcache, positions, block_table, items, part_o, part_ml)
     tokens = q.shape[0]
+    _need(0 <= values <= d, f"attn_prefill: {values} value channels of a head of {d}")
     if n_splits > 1:
         _need(d in PREFILL_SPLIT_HEAD_DIMS, f"attn_prefill: head size {d} has no split variant")
         _need(split_size > 0 and split_size % PREFILL_SPLIT_KEYS == 0,
@@ -374,7 +384,7 @@ def attn_prefill(q: torch.Tensor, out: torch.Tensor, nq: int, nkv: int, d: int, 
             _f32(scale), _i32(window), _i32(split_size if n_splits > 1 else 0), _i32(n_splits),
             _ptr(part_o if n_splits > 1 else None), _ptr(part_ml if n_splits > 1 else None),
             _extras("attn_prefill", tokens, nq, gate, gate_width=gate_width, sink=sink, softcap=softcap,
-            chunk=chunk), _stream())
+            chunk=chunk, values=values), _stream())
 
 
 def decode_takes(d: int, rotary_dim: int, pairing: int) -> bool:

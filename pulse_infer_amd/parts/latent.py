@@ -340,7 +340,7 @@ class LatentAttention(PagedAttention):
                                     self.scale, int(self.window) if self.window is not None else 0, plan["split_size"],
                                     plan["splits"], part_o, part_ml, gate=gate,
                                     gate_width=0 if self.gate_heads else (self.v_dim if gate is not None else 0),
-                                    sink=self.sink, softcap=self.score_cap)
+                                    sink=self.sink, softcap=self.score_cap, values=0 if direct else self.v_dim)
         if not direct:
             for a, b in plan["spans"]:
                 kernels.latent_compact(o[a:b], w, out[a:b], self.nq, self.v_dim, self.out_scale)

@@ -44,3 +44,39 @@ def test_tokens_and_portions_in_one_launch(d, nq, nkv, splits, window, chunk):
     am.attn_mfma(q, two, nq, nkv, d, kc, vc, positions, table, short_items, *tail, chunk=chunk)
     am.attn_mfma(q, one, nq, nkv, d, kc, vc, positions, table, short_items, *tail, chunk=chunk, long_items=long_items)
     assert not torch.isnan(two).any() and torch.equal(one, two)
+
+
+@pytest.mark.parametrize("values", [1, 96, 128, 129, 192])
+@pytest.mark.parametrize("splits,window,gated", [(1, 0, False), (3, 0, True), (1, 90, False)])
+def test_portions_of_heads_whose_values_are_narrower(values, splits, window, gated):
+    """Heads of 192 channels whose values fill ``values`` of them: the bits of the kernel that computes them all, stale values
+    (not a number) under keys that nobody sees among it."""
+    from pulse_infer_amd.ops import attention_mfma as am
+
+    page, nq, d, lengths = 16, 6, 192, [(0, 333), (70, 64), (500, 17)]
+    gen = torch.Generator().manual_seed(values)
+    entries, rows = [], 0
+    for start, count in lengths:
+        entries.append(Entry(start, count, rows))
+        rows += count
+    width = max((e.start + e.count + page - 1) // page for e in entries)
+    pages = len(entries) * width
+    table = torch.randperm(pages, generator=gen).to(torch.int32).view(len(entries), width).to(DEV)
+    bf = lambda *s: torch.randn(s, generator=gen).to(torch.bfloat16).to(DEV)
+    q, kc, vc = bf(rows, nq * d), bf(pages, nq, page, d), bf(pages, nq, d, page)
+    vc[:, :, values:] = 0.0
+    for i, e in enumerate(entries):                         # behind a request's last position
+        end = e.start + e.count
+        if end % page:
+            vc[int(table[i, end // page]), :, :values, end % page:] = float("nan")
+    positions = torch.tensor([e.start + i for e in entries for i in range(e.count)], dtype=torch.int32, device=DEV)
+    items = torch.tensor(am.build_items(list(enumerate(entries)), am.portion_tokens(1, d)), dtype=torch.int32, device=DEV)
+    size = 192 if splits > 1 else 0
+    part_o, part_ml = torch.zeros(rows * nq * splits * d, device=DEV), torch.empty(rows * nq * splits * 2, device=DEV)
+    gate = bf(rows, nq) if gated else None
+    one, two = (torch.zeros((rows, nq * d), dtype=torch.bfloat16, device=DEV) for _ in range(2))
+    args = (nq, nq, d, kc, vc, positions, table, items, d ** -0.5, window, size, splits, part_o, part_ml)
+    am.attn_prefill(q, two, *args, gate=gate)
+    am.attn_prefill(q, one, *args, gate=gate, values=values)
+    wanted = lambda t: t.view(rows, nq, d)[:, :, :values]
+    assert not torch.isnan(wanted(two)).any() and torch.equal(wanted(one), wanted(two))
