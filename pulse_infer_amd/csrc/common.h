@@ -158,6 +158,26 @@ __device__ __forceinline__ float block_sum(float v, float* scratch) {
     return total;
 }
 
+// Eight neighbouring bfloat16 channels of a head, rotated: (u, p) -> u cos - p sin for a pair's first channel, u cos + p sin for
+// its second.  Pairs are neighbours (`other` unused; cs, sn: four angles) or, `apart`, half the rotated channels apart (`other`: the
+// partners' eight; eight angles; `lower`: the first channels).  The angles come in whole pieces: one by one, each was waited for.
+__device__ __forceinline__ uint4 turned_piece(uint4 own, uint4 other, bool apart, bool lower, const float* cs, const float* sn) {
+    const float4 c0 = *reinterpret_cast<const float4*>(cs), c1 = *reinterpret_cast<const float4*>(cs + (apart ? 4 : 0));
+    const float4 s0 = *reinterpret_cast<const float4*>(sn), s1 = *reinterpret_cast<const float4*>(sn + (apart ? 4 : 0));
+    const uint32_t u[4] = {own.x, own.y, own.z, own.w}, o[4] = {other.x, other.y, other.z, other.w};
+    const float c[8] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w}, s[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
+    uint32_t to[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const float a = __uint_as_float(u[j] << 16), b = __uint_as_float(u[j] & 0xffff0000u);
+        const float pa = apart ? __uint_as_float(o[j] << 16) : b, pb = apart ? __uint_as_float(o[j] & 0xffff0000u) : a;
+        const float ca = apart ? c[2 * j] : c[j], cb = apart ? c[2 * j + 1] : c[j], sa = apart ? s[2 * j] : s[j], sb = apart ? s[2 * j + 1] : s[j];
+        const float qa = !apart || lower ? -pa : pa, qb = apart && lower ? -pb : pb;
+        to[j] = static_cast<uint32_t>(f32_to_bf16(a * ca + qa * sa)) | (static_cast<uint32_t>(f32_to_bf16(b * cb + qb * sb)) << 16);
+    }
+    return make_uint4(to[0], to[1], to[2], to[3]);
+}
+
 // Dispatch a two-way storage tag to a template argument.
 #define PULSE_DISPATCH_DTYPE(tag, T, ...)                 \
     do {                                                  \

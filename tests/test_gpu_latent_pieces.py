@@ -56,3 +56,34 @@ def test_queries_pages_and_results_in_pieces(heads, d, rot, dv, width, pairing):
     kernels.latent_compact(o, width, y[0], heads, dv)
     kernels.latent_compact(shifted(o), width, y[1], heads, dv)
     assert torch.equal(y[0], y[1]) and torch.equal(y[0], o.view(tokens, heads, width)[..., :dv].reshape(tokens, -1))
+
+
+@pytest.mark.parametrize("tokens", [1, 5, 700])
+@pytest.mark.parametrize("d,stored,rotary,pairing", [(128, 128, 128, 1), (64, 96, 16, 1), (24, 32, 8, 0), (40, 40, 0, 0)])
+def test_rows_of_queries_and_keys_in_pieces(tokens, d, stored, rotary, pairing):
+    """Queries and keys without biases and norms: 16 bytes a thread, and value by value (from an address that is no multiple of 16)."""
+    from pulse_infer_amd.ops import kernels
+
+    nq, nkv, dv, page = 5, 2, 24, 16
+    x = bf(tokens, nq * d + nkv * (d + dv), seed=7)
+    angle = torch.randn(tokens, max(1, rotary // 2), generator=torch.Generator().manual_seed(8)).to(DEV)
+    cos, sin = (angle.cos(), angle.sin()) if rotary else (None, None)
+    entries = 3
+    width = (tokens + page - 1) // page + 1
+    table = torch.randperm(entries * width, generator=torch.Generator().manual_seed(9)).to(torch.int32).view(entries, width).to(DEV)
+    table[2, 0] = -1                                        # no page: nothing is written there
+    entry = (torch.arange(tokens) % entries).to(torch.int32).to(DEV)
+    positions = torch.arange(tokens, dtype=torch.int32, device=DEV)
+    got = []
+    for src in (x, shifted(x)):
+        q = torch.full((tokens, nq * stored), float("nan"), dtype=BF, device=DEV)
+        k = torch.full((entries * width, nkv, page, stored), 7.0, dtype=BF, device=DEV)
+        v = torch.full((entries * width, nkv, stored, page), 7.0, dtype=BF, device=DEV)
+        kernels.qkv_rows(src, q, nq, nkv, d, dv, stored, None, None, 1e-6, cos, sin, rotary, pairing, k, v, positions, entry, table,
+                         norm=False)
+        got.append((q, k, v))
+    # (the two products' sum may be contracted differently: a float32 rounding before that to bfloat16)
+    for one, two in zip(*got):
+        assert ((one.double() - two.double()).abs() <= 2.0 ** -7 * two.double().abs() + 2.0 ** -20).all()
+    if rotary == 0:
+        assert torch.equal(got[0][0].view(tokens, nq, stored)[..., :d].reshape(tokens, -1), x[:, :nq * d])
