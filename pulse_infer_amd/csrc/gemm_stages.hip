@@ -4,12 +4,13 @@
 //
 // What bounds it: the bytes that the fullest compute unit copies into LDS.  A unit takes in 30 to 55 bytes a nanosecond over a
 // launch, least where they are weights that come from memory, and the matrix cores are busy for 13 to 47 % of it, LDS waits
-// make 1 to 4 % (counters at 97, 357 and 509 rows), so the shape and the shares of K are chosen for the least bytes
+// make 1 to 4 % (counters at 97, 357 and 509 rows; from 300 rows on the power limit comes near: 357 rows of gate + up take 57 us with
+// operands of zeros, 70 with others), so the shape and the shares of K are chosen for the least bytes
 // (`plan_for`).  Measured alone with weights from memory, us, against the vendor library's product (gate and up: with its
 // pass for SwiGLU behind it) and this package's shared-out product for up to 192 rows; in brackets behind a figure, what it
 // takes inside a step, between other kernels and with the chip warm:
 //                                   97 rows              192                  357                 509
-//   gate + up, 24,576 x 4,096       45 [44]              54                   71 [74]             88 [101]
+//   gate + up, 24,576 x 4,096       39 [39]              54                   70 [72]             86 [95]
 //     library                       54                   64                   84                  96
 //   qkv, 6,144 x 4,096              19 [20]              26                   34 [34]             35 [38]
 //     library                       25                   36                   41                  42
