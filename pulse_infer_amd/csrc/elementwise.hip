@@ -26,12 +26,47 @@ __global__ void embed_gather_kernel(const int* __restrict__ ids, const TW* __res
     for (int i = threadIdx.x; i < hidden; i += blockDim.x) dst[i] = to_f32<TW>(src[i]) * scale;
 }
 
+// The same for widths in fours and aligned rows: four values a thread, a row's pieces asked for together (one after the other each
+// waits out a trip to memory: 8 / 357 rows of 4,096 inside a step 10 / 11 us -> 4).
+template <typename TW>
+__global__ __launch_bounds__(256) void embed_gather_vec_kernel(const int* __restrict__ ids, const TW* __restrict__ table,
+                                                               float* __restrict__ out, int hidden, int vocab, int* bad_id, float scale) {
+    struct __attribute__((aligned(4 * sizeof(TW)))) Four { TW v[4]; };
+    constexpr int AHEAD = 4;
+    const int t = blockIdx.x, id = ids[t], pieces = hidden / 4;
+    const bool good = id >= 0 && id < vocab;
+    float4* dst = reinterpret_cast<float4*>(out + static_cast<int64_t>(t) * hidden);
+    const Four* src = reinterpret_cast<const Four*>(table + static_cast<int64_t>(good ? id : 0) * hidden);
+    for (int i0 = threadIdx.x; i0 < pieces; i0 += AHEAD * 256) {
+        Four f[AHEAD];
+#pragma unroll
+        for (int u = 0; u < AHEAD; ++u) f[u] = src[min(i0 + u * 256, pieces - 1)];
+#pragma unroll
+        for (int u = 0; u < AHEAD; ++u) {
+            const int i = i0 + u * 256;
+            const float nan = __builtin_nanf("");
+            if (i < pieces)
+                dst[i] = good ? make_float4(to_f32<TW>(f[u].v[0]) * scale, to_f32<TW>(f[u].v[1]) * scale, to_f32<TW>(f[u].v[2]) * scale,
+                                            to_f32<TW>(f[u].v[3]) * scale)
+                              : make_float4(nan, nan, nan, nan);
+        }
+    }
+    if (!good && threadIdx.x == 0) *bad_id = 1;
+}
+
 extern "C" int pulse_embed_gather(const int* ids, const void* table, int table_dtype, float* out,
                                   int tokens, int hidden, int vocab, int* bad_id, float scale, hipStream_t stream) {
     PULSE_REQUIRE(tokens >= 0 && hidden > 0 && vocab > 0, "embed_gather: bad sizes T=%d H=%d V=%d", tokens, hidden, vocab);
     PULSE_REQUIRE(pulse_dtype_ok(table_dtype), "embed_gather: bad dtype tag %d", table_dtype);
     PULSE_REQUIRE(ids && table && out && bad_id, "embed_gather: null pointer");
     if (tokens == 0) return 0;
+    if (hidden % 4 == 0 && reinterpret_cast<uintptr_t>(table) % 16 == 0 && reinterpret_cast<uintptr_t>(out) % 16 == 0) {
+        PULSE_DISPATCH_DTYPE(table_dtype, TW,
+            hipLaunchKernelGGL(embed_gather_vec_kernel<TW>, dim3(tokens), dim3(256), 0, stream, ids, static_cast<const TW*>(table), out,
+                               hidden, vocab, bad_id, scale));
+        PULSE_LAUNCH_CHECK("embed_gather");
+        return 0;
+    }
     PULSE_DISPATCH_DTYPE(table_dtype, TW,
         hipLaunchKernelGGL(embed_gather_kernel<TW>, dim3(tokens), dim3(256), 0, stream, ids,
                            static_cast<const TW*>(table), out, hidden, vocab, bad_id, scale));

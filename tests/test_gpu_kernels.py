@@ -51,6 +51,18 @@ def test_embed_gather(k, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("hidden", [4, 1020, 4096, 5004])
+def test_embed_gather_in_pieces_of_four(k, dtype, hidden):
+    table, ref = as_stored(rnd(11, hidden), dtype)
+    ids = torch.tensor([10, 0, -1, 11, 3], dtype=torch.int32, device=DEV)
+    out, bad = torch.full((6, hidden), 7.0, device=DEV), torch.zeros(1, dtype=torch.int32, device=DEV)
+    k.embed_gather(ids, table, out[:5], bad, 0.5)
+    assert bad.item() == 1 and bool(out[2:4].isnan().all()) and bool((out[5] == 7.0).all())
+    good = [0, 1, 4]
+    assert torch.equal(out[good].cpu().to(F64), 0.5 * ref[ids[good].cpu().long()])
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("hidden", [48, 1000, 4100])
 def test_add_rmsnorm(k, dtype, hidden):
     rows, eps = 9, 3e-5
