@@ -1276,7 +1276,7 @@ __global__ __launch_bounds__(SIMPLE_THREADS) void left_choose_kernel(
     const int* __restrict__ top_k, const float* __restrict__ top_p, const float* __restrict__ uniform,
     const float* __restrict__ penalty, const int* __restrict__ seen_row, const uint32_t* __restrict__ seen_masks,
     const uint32_t* __restrict__ banned, int mask_words, const float* __restrict__ part_max, const float* __restrict__ part_min,
-    int chunks, const int* __restrict__ done, const int* __restrict__ seg_i, const float* __restrict__ seg_x,
+    const int* __restrict__ part_idx, int chunks, const int* __restrict__ done, const int* __restrict__ seg_i, const float* __restrict__ seg_x,
     const int* __restrict__ seg_n, int* __restrict__ rest, int* __restrict__ out) {
     constexpr int WAVES = SIMPLE_THREADS / PULSE_WAVE, PER = SIMPLE_CHUNK / SIMPLE_THREADS;
     __shared__ int list_i[LIST_CAP];
@@ -1314,9 +1314,19 @@ __global__ __launch_bounds__(SIMPLE_THREADS) void left_choose_kernel(
     __syncthreads();
     if (left.k > 0) {
         if (wave != 0) return;
+        // (where no weight is a number above zero, the largest logit)
+        float largest = -INFINITY;
+        int best_i = 0x7fffffff;
+        for (int c = lane; c < chunks; c += PULSE_WAVE) {
+            const float v = part_max[static_cast<int64_t>(r) * chunks + c];
+            const int i = part_idx[static_cast<int64_t>(r) * chunks + c];
+            if (v > largest || (v == largest && i < best_i)) { largest = v; best_i = i; }
+        }
+        wave_argmax(largest, best_i);
+        const bool use_p = left.p > 0.f && left.p < 1.f;
         int token;            // (with top-k every list is enough)
-        if (n <= 8 * PULSE_WAVE) finish_on_list<8>(list_i, list_x, n, true, left.k, left.p > 0.f && left.p < 1.f, left.p, 0.f, left.best, left.inv_t, uniform[r], list_i[0], token);
-        else finish_on_list<LIST_PER_LANE>(list_i, list_x, n, true, left.k, left.p > 0.f && left.p < 1.f, left.p, 0.f, left.best, left.inv_t, uniform[r], list_i[0], token);
+        if (n <= 8 * PULSE_WAVE) finish_on_list<8>(list_i, list_x, n, true, left.k, use_p, left.p, 0.f, left.best, left.inv_t, uniform[r], best_i, token);
+        else finish_on_list<LIST_PER_LANE>(list_i, list_x, n, true, left.k, use_p, left.p, 0.f, left.best, left.inv_t, uniform[r], best_i, token);
         if (lane == 0) { out[r] = token; rest[REST_CHOSEN] = 1; }
         return;
     }
@@ -1529,7 +1539,7 @@ extern "C" int pulse_sample_chunked_rest(const float* logits, int rows, int voca
                                static_cast<const int*>(done), seg_i, seg_x, seg_n, rest);
             hipLaunchKernelGGL(left_choose_kernel, dim3(rows), dim3(SIMPLE_THREADS), 0, stream, logits, vocab, row_stride,
                                temperature, top_k, top_p, uniform, penalty, seen_row, seen_masks, banned, mask_words, part_max, part_min,
-                               chunks, static_cast<const int*>(done), static_cast<const int*>(seg_i), static_cast<const float*>(seg_x),
+                               static_cast<const int*>(part_idx), chunks, static_cast<const int*>(done), static_cast<const int*>(seg_i), static_cast<const float*>(seg_x),
                                static_cast<const int*>(seg_n), rest, out);
         }
         PULSE_LAUNCH_CHECK("sample_chunked (what is left)");

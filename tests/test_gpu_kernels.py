@@ -1579,3 +1579,32 @@ def test_rows_left_by_the_chunks_are_chosen_the_same_with_and_without_many_workg
         chosen = scratch["rest"].view(-1)[: rows * k.SAMPLE_REST].view(rows, k.SAMPLE_REST)[:, 2 * 2048 + 1].cpu()
         left = scratch["done"][:rows].cpu() == 0
         assert left.sum() >= 8 and (chosen[left] == 1).sum() >= 6        # most of them did not need the workgroup a row
+
+
+@pytest.mark.parametrize("vocab", [5, 40, 2049, 32000, 151936])
+@pytest.mark.parametrize("p", [0.0, 0.9])
+def test_rows_whose_weights_are_no_numbers_choose_the_largest_logit(k, vocab, p):
+    """Top-k above the number of chunks where no weight is a number above zero: a temperature whose inverse is infinite, and an
+    infinite logit among few others.  The largest logit, which is not the first of those kept, whichever kernels choose."""
+    top_k = k.sample_chunks(vocab) + 2
+    logits = torch.full((3, vocab), float("-inf"))
+    gen = torch.Generator().manual_seed(vocab)
+    logits[0] = torch.randn(vocab, generator=gen)
+    for r in (1, 2):                                  # twenty values a chunk of 2,048 at most
+        for first in range(0, vocab, 2048):
+            at = first + torch.randperm(min(2048, vocab - first), generator=gen)[:20]
+            logits[r, at] = torch.randn(len(at), generator=gen)
+    logits[0, :2] = logits[1, :2] = logits[2, :2] = torch.tensor([4.0, 3.5])
+    largest = [vocab - 1, vocab // 2, vocab - 2]
+    logits[0, largest[0]], logits[1, largest[1]], logits[2, largest[2]] = 5.0, 5.0, float("inf")
+    dev = lambda t: t.to(DEV)
+    kw = dict(temperature=torch.tensor([1e-39, 2e-39, 0.7]), top_k=torch.full((3,), top_k, dtype=torch.int32),
+              top_p=torch.full((3,), p), uniform=torch.tensor([0.1, 0.5, 0.9]))
+    kw = {name: dev(t) for name, t in kw.items()}
+    scratch, without = _chunked_scratch(k, 3, vocab), _chunked_scratch(k, 3, vocab)
+    del without["rest"]
+    for choose in (lambda o: k.sample(dev(logits), o, **kw), lambda o: k.sample_chunked(dev(logits), o, without, **kw),
+                   lambda o: k.sample_chunked(dev(logits), o, scratch, **kw)):
+        out = torch.full((3,), -9, dtype=torch.int32, device=DEV)
+        choose(out)
+        assert out.tolist() == largest
