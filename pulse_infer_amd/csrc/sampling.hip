@@ -719,6 +719,10 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
         if (who < 0) run += part_sum[w];
     }
     if (who < 0) {  // rounding left the target beyond the last part: its last kept entry
+        if (last_part < 0) {      // (no weight is a number above zero)
+            if (threadIdx.x == 0) out[r] = best_i;
+            return;
+        }
         who = last_part;
         run = INFINITY;
     }

@@ -1583,10 +1583,12 @@ def test_rows_left_by_the_chunks_are_chosen_the_same_with_and_without_many_workg
 
 @pytest.mark.parametrize("vocab", [5, 40, 2049, 32000, 151936])
 @pytest.mark.parametrize("p", [0.0, 0.9])
-def test_rows_whose_weights_are_no_numbers_choose_the_largest_logit(k, vocab, p):
+@pytest.mark.parametrize("more", [2, 60])
+def test_rows_whose_weights_are_no_numbers_choose_the_largest_logit(k, vocab, p, more):
     """Top-k above the number of chunks where no weight is a number above zero: a temperature whose inverse is infinite, and an
-    infinite logit among few others.  The largest logit, which is not the first of those kept, whichever kernels choose."""
-    top_k = k.sample_chunks(vocab) + 2
+    infinite logit among few others, in one chunk fewer than k.  The largest logit, which is not the first of those kept, whichever
+    kernels choose."""
+    top_k = min(k.sample_chunks(vocab) + more, vocab - 1)
     logits = torch.full((3, vocab), float("-inf"))
     gen = torch.Generator().manual_seed(vocab)
     logits[0] = torch.randn(vocab, generator=gen)
