@@ -1834,27 +1834,14 @@ int launch_attn_mfma(const void* q, int64_t q_stride, void* out, int64_t o_strid
 
 }  // namespace
 
-extern "C" int pulse_attn_prefill(const void* q, int64_t q_stride, void* out, int64_t o_stride, const void* kcache, const void* vcache,
-                                  const int* positions, const int* block_table, int bt_width, const int* items, int n_items, int tokens,
-                                  int nq, int nkv, int page_size, int num_pages, float scale, int window, int split_size, int n_splits,
-                                  float* part_o, float* part_ml, const PulseAttnExtras* extras, hipStream_t stream);
-
-// Extras with more behind them, told by plain_norm, which these entry points do not use: for pulse_attn_mfma a list of prompt portions;
-// for pulse_attn_prefill how many of a head's value channels are no fill (those behind them need not be computed).
-constexpr int ATTN_BESIDE = 2, ATTN_VALUES = 3;
-struct PulseAttnValues {
-    PulseAttnExtras extras;
-    int values;
-};
-struct PulseAttnBeside {
-    PulseAttnExtras extras;
-    const int* long_items;
-    int n_long;
-};
-
 namespace {
 
 constexpr int SPLIT_KEYS = PULSE_WIDE ? 64 : 0;
+#if PULSE_WIDE
+constexpr bool BESIDE = PULSE_BESIDE;
+#else
+constexpr bool BESIDE = false;
+#endif
 
 // The arguments of the prompt-portion kernel, checked.
 int fill_portions(MfmaArgs& a, const void* q, int64_t q_stride, void* out, int64_t o_stride, const void* kcache, const void* vcache,
@@ -1901,6 +1888,39 @@ int fill_portions(MfmaArgs& a, const void* q, int64_t q_stride, void* out, int64
     return take_gate(a, extras, nq, scale);
 }
 
+int attn_prefill(const void* q, int64_t q_stride, void* out, int64_t o_stride, const void* kcache, const void* vcache,
+                 const int* positions, const int* block_table, int bt_width, const int* items, int n_items, int tokens, int nq,
+                 int nkv, int page_size, int num_pages, float scale, int window, int split_size, int n_splits, float* part_o,
+                 float* part_ml, const PulseAttnExtras* extras, [[maybe_unused]] int values, hipStream_t stream) {
+    MfmaArgs a;
+    if (fill_portions(a, q, q_stride, out, o_stride, kcache, vcache, positions, block_table, bt_width, items, n_items, tokens, nq, nkv,
+                      page_size, num_pages, scale, window, split_size, n_splits, part_o, part_ml, extras)) return 1;
+    if (tokens == 0 || n_items == 0) return 0;
+    const int gp = a.gp;
+#if PULSE_WIDE && PULSE_NARROW_VALUES
+    if (values <= NARROW_VALUES)
+        hipLaunchKernelGGL((attn_prefill_values_kernel<WIDE_CT, 4, WIDE_NW>), dim3(n_items, nkv * a.head_chunks, n_splits),
+                           dim3(WIDE_NW * PULSE_WAVE), 0, stream, a, 16 / gp);
+    else
+#endif
+#if PULSE_WIDE
+    hipLaunchKernelGGL((attn_prefill_wide_kernel<WIDE_CT, 4, WIDE_NW>), dim3(n_items, nkv * a.head_chunks, n_splits),
+                       dim3(WIDE_NW * PULSE_WAVE), 0, stream, a, 16 / gp);
+    if (n_splits > 1) {
+        PULSE_LAUNCH_CHECK("attn_prefill");
+        const int item_tokens = WIDE_NW * WIDE_CT * (16 / gp);
+        hipLaunchKernelGGL(attn_prefill_reduce_kernel, dim3(n_items * item_tokens, (nq + PR_HEADS - 1) / PR_HEADS),
+                           dim3(PR_THREADS), 0, stream, part_o, part_ml, positions, items, item_tokens, a.out, o_stride, nq,
+                           n_splits, split_size, a.gate, a.gate_stride, a.gate_width, a.sink);
+    }
+#else
+    hipLaunchKernelGGL(attn_prefill_kernel, dim3(n_items, nkv * a.head_chunks), dim3(WAVES * PULSE_WAVE), 0, stream, a,
+                       16 / gp);
+#endif
+    PULSE_LAUNCH_CHECK("attn_prefill");
+    return 0;
+}
+
 }  // namespace
 
 // Scratch needed for `tokens` rows cut into `n_splits`: tokens * nq * n_splits * D floats of part_o, * 2 of part_ml.
@@ -1909,32 +1929,37 @@ int fill_portions(MfmaArgs& a, const void* q, int64_t q_stride, void* out, int64
 // the keys that are there evenly into the same number of splits.  A value below an item's context loses keys.
 // plan (device, or null): what pulse_attn_plan made of these items and positions for this n_splits; it takes the
 // place of that even cut (every item then has a split size of its own and the workgroups an order).
-// extras with the tag of a PulseAttnBeside: its list of prompt portions (as pulse_attn_prefill's, every walk whole) goes in the same
-// launch where the head size has a kernel for both, else in one before it; the results are those of the two calls.
 extern "C" int pulse_attn_mfma(const void* q, int64_t q_stride, void* out, int64_t o_stride, const void* kcache,
                                const void* vcache, const int* positions, const int* block_table, int bt_width,
                                const int* items, int n_items, int tokens, int nq,
                                int nkv, int page_size, int num_pages, float scale, int window, int split_size,
                                int n_splits, int max_context, float* part_o, float* part_ml, const int* live_context,
                                const int* plan, const PulseAttnExtras* extras, hipStream_t stream) {
-    if (extras && extras->plain_norm == ATTN_BESIDE) {
-        const PulseAttnBeside* more = reinterpret_cast<const PulseAttnBeside*>(extras);
-        MfmaArgs portions;
-        if (fill_portions(portions, q, q_stride, out, o_stride, kcache, vcache, positions, block_table, bt_width, more->long_items,
-                          more->n_long, tokens, nq, nkv, page_size, num_pages, scale, window, 0, 1, nullptr, nullptr, extras)) return 1;
-        const int64_t heads = static_cast<int64_t>(nkv) * ((nq / nkv + 15) / 16);
-        const bool both = PULSE_WIDE && PULSE_HEAD_DIM <= 128 && tokens > 0 && n_items > 0 && more->n_long > 0 &&
-                          (static_cast<int64_t>(n_items) * n_splits + more->n_long) * heads < (int64_t{1} << 31);
-        if (both)
-            return launch_attn_mfma(q, q_stride, out, o_stride, kcache, vcache, positions, block_table, bt_width, items, n_items, tokens,
-                                    nq, nkv, page_size, num_pages, scale, window, split_size, n_splits, max_context, part_o, part_ml,
-                                    nullptr, live_context, plan, extras, stream, &portions);
-        if (pulse_attn_prefill(q, q_stride, out, o_stride, kcache, vcache, positions, block_table, bt_width, more->long_items, more->n_long,
-                               tokens, nq, nkv, page_size, num_pages, scale, window, 0, 1, nullptr, nullptr, extras, stream)) return 1;
-    }
     return launch_attn_mfma(q, q_stride, out, o_stride, kcache, vcache, positions, block_table, bt_width, items, n_items,
                             tokens, nq, nkv, page_size, num_pages, scale, window, split_size, n_splits, max_context,
                             part_o, part_ml, nullptr, live_context, plan, extras, stream);
+}
+
+// The same with a list of prompt portions (as pulse_attn_prefill's, every walk whole) beside the items: in the same launch where the
+// head size has a kernel for both, else in one before it; the results are those of the two calls.
+extern "C" int pulse_attn_mfma_beside(const void* q, int64_t q_stride, void* out, int64_t o_stride, const void* kcache,
+                                      const void* vcache, const int* positions, const int* block_table, int bt_width,
+                                      const int* items, int n_items, int tokens, int nq,
+                                      int nkv, int page_size, int num_pages, float scale, int window, int split_size,
+                                      int n_splits, int max_context, float* part_o, float* part_ml, const int* live_context,
+                                      const int* plan, const PulseAttnExtras* extras, const int* long_items, int n_long,
+                                      hipStream_t stream) {
+    MfmaArgs portions;
+    if (fill_portions(portions, q, q_stride, out, o_stride, kcache, vcache, positions, block_table, bt_width, long_items, n_long, tokens,
+                      nq, nkv, page_size, num_pages, scale, window, 0, 1, nullptr, nullptr, extras)) return 1;
+    const int64_t heads = static_cast<int64_t>(nkv) * ((nq / nkv + 15) / 16);
+    const bool both = BESIDE && tokens > 0 && n_items > 0 && n_long > 0 &&
+                      (static_cast<int64_t>(n_items) * n_splits + n_long) * heads < (int64_t{1} << 31);
+    if (!both && attn_prefill(q, q_stride, out, o_stride, kcache, vcache, positions, block_table, bt_width, long_items, n_long, tokens, nq,
+                              nkv, page_size, num_pages, scale, window, 0, 1, nullptr, nullptr, extras, D, stream)) return 1;
+    return launch_attn_mfma(q, q_stride, out, o_stride, kcache, vcache, positions, block_table, bt_width, items, n_items, tokens, nq, nkv,
+                            page_size, num_pages, scale, window, split_size, n_splits, max_context, part_o, part_ml, nullptr,
+                            live_context, plan, extras, stream, both ? &portions : nullptr);
 }
 
 // The plan of a step (see attn_plan_kernel) for pulse_attn_mfma / pulse_attn_decode with the same items and n_splits:
@@ -2006,35 +2031,20 @@ extern "C" int pulse_attn_prefill(const void* q, int64_t q_stride, void* out, in
                                   int nq, int nkv, int page_size, int num_pages, float scale, int window,
                                   int split_size, int n_splits, float* part_o, float* part_ml,
                                   const PulseAttnExtras* extras, hipStream_t stream) {
-    MfmaArgs a;
-    if (fill_portions(a, q, q_stride, out, o_stride, kcache, vcache, positions, block_table, bt_width, items, n_items, tokens, nq, nkv,
-                      page_size, num_pages, scale, window, split_size, n_splits, part_o, part_ml, extras)) return 1;
-    if (tokens == 0 || n_items == 0) return 0;
-    const int gp = a.gp;
-    const int values = extras && extras->plain_norm == ATTN_VALUES ? reinterpret_cast<const PulseAttnValues*>(extras)->values : D;
-    PULSE_REQUIRE(values > 0 && values <= D, "attn_prefill: %d value channels of a head of %d", values, D);
-#if PULSE_WIDE && PULSE_NARROW_VALUES
-    if (values <= NARROW_VALUES)
-        hipLaunchKernelGGL((attn_prefill_values_kernel<WIDE_CT, 4, WIDE_NW>), dim3(n_items, nkv * a.head_chunks, n_splits),
-                           dim3(WIDE_NW * PULSE_WAVE), 0, stream, a, 16 / gp);
-    else
-#endif
-#if PULSE_WIDE
-    hipLaunchKernelGGL((attn_prefill_wide_kernel<WIDE_CT, 4, WIDE_NW>), dim3(n_items, nkv * a.head_chunks, n_splits),
-                       dim3(WIDE_NW * PULSE_WAVE), 0, stream, a, 16 / gp);
-    if (n_splits > 1) {
-        PULSE_LAUNCH_CHECK("attn_prefill");
-        const int item_tokens = WIDE_NW * WIDE_CT * (16 / gp);
-        hipLaunchKernelGGL(attn_prefill_reduce_kernel, dim3(n_items * item_tokens, (nq + PR_HEADS - 1) / PR_HEADS),
-                           dim3(PR_THREADS), 0, stream, part_o, part_ml, positions, items, item_tokens, a.out, o_stride, nq,
-                           n_splits, split_size, a.gate, a.gate_stride, a.gate_width, a.sink);
-    }
-#else
-    hipLaunchKernelGGL(attn_prefill_kernel, dim3(n_items, nkv * a.head_chunks), dim3(WAVES * PULSE_WAVE), 0, stream, a,
-                       16 / gp);
-#endif
-    PULSE_LAUNCH_CHECK("attn_prefill");
-    return 0;
+    return attn_prefill(q, q_stride, out, o_stride, kcache, vcache, positions, block_table, bt_width, items, n_items, tokens, nq, nkv,
+                        page_size, num_pages, scale, window, split_size, n_splits, part_o, part_ml, extras, D, stream);
+}
+
+// The same for callers that want the first `values` channels of every head: `out` holds anything in the others.
+extern "C" int pulse_attn_prefill_values(const void* q, int64_t q_stride, void* out, int64_t o_stride, const void* kcache,
+                                         const void* vcache, const int* positions, const int* block_table, int bt_width,
+                                         const int* items, int n_items, int tokens,
+                                         int nq, int nkv, int page_size, int num_pages, float scale, int window,
+                                         int split_size, int n_splits, float* part_o, float* part_ml,
+                                         const PulseAttnExtras* extras, int values, hipStream_t stream) {
+    PULSE_REQUIRE(values > 0 && values <= D, "attn_prefill_values: %d value channels of a head of %d", values, D);
+    return attn_prefill(q, q_stride, out, o_stride, kcache, vcache, positions, block_table, bt_width, items, n_items, tokens, nq, nkv,
+                        page_size, num_pages, scale, window, split_size, n_splits, part_o, part_ml, extras, values, stream);
 }
 
 // Column tiles a wavefront of the prompt-portion kernel takes: its items hold 4 * this * tokens_per_item tokens.

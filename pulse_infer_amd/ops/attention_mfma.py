@@ -28,20 +28,9 @@ class _Extras(ctypes.Structure):
                 ("chunk", ctypes.c_int)]
 
 
-class _Beside(_Extras):
-    # as PulseAttnBeside of the kernel source: told by plain_norm = 2
-    _fields_ = [("long_items", ctypes.c_void_p), ("n_long", ctypes.c_int)]
-
-
-class _Values(_Extras):
-    # as PulseAttnValues of the kernel source: told by plain_norm = 3
-    _fields_ = [("values", ctypes.c_int)]
-
-
 def _extras(what: str, tokens: int, nq: int, gate: Optional[torch.Tensor] = None, plain_norm: bool = False,
             v_head0: int = -1, q_temperature: Optional[Tuple[float, int]] = None, gate_width: int = 0,
-            sink: Optional[torch.Tensor] = None, softcap: float = 0.0, chunk: int = 0,
-            long_items: Optional[torch.Tensor] = None, values: int = 0):
+            sink: Optional[torch.Tensor] = None, softcap: float = 0.0, chunk: int = 0):
     """What the entry points take besides their lists, or a null pointer when there is none of it.  ``gate``: bfloat16
     [tokens, nq] (rows may be strided), the logits of an output gate: head h of token t leaves the kernel multiplied
     by sigmoid(gate[t, h]).  The rest is for ``attn_decode``: a norm of q and k without weights, the head number at
@@ -49,21 +38,11 @@ def _extras(what: str, tokens: int, nq: int, gate: Optional[torch.Tensor] = None
     q *= 1 + coef * ln(floor((position + 1) / every) + 1).  ``gate_width`` > 0: the gate holds a logit for each of the
     first ``gate_width`` channels of every head ([tokens, nq * gate_width]).  ``sink`` float32 [nq]: exp(sink[h]) is one
     more term of head h's softmax denominator; ``softcap`` > 0: scaled scores become cap * tanh(score / cap); ``chunk`` > 0:
-    a token sees only the keys of its own chunk of that many positions, counted from 0; ``long_items`` (``attn_mfma``
-    only): the items of prompt portions that go with the others; ``values`` > 0 (``attn_prefill`` only): so many of a head's
-    value channels are wanted, those behind them may be left out."""
+    a token sees only the keys of its own chunk of that many positions, counted from 0."""
     if (gate is None and not plain_norm and v_head0 < 0 and q_temperature is None and sink is None and not softcap
-            and not chunk and long_items is None and not values):
+            and not chunk):
         return None
-    ex = _Beside() if long_items is not None else _Values() if values else _Extras()
-    if long_items is not None:
-        _gpu(what, long_items)
-        _need(not plain_norm and long_items.dtype == torch.int32 and long_items.is_contiguous()
-              and long_items.numel() % ITEM_INTS == 0, f"{what}: items must be int32 quadruples")
-        ex.long_items, ex.n_long = long_items.data_ptr(), long_items.numel() // ITEM_INTS
-    if values:
-        _need(not plain_norm and long_items is None, f"{what}: value channels are for prompt portions alone")
-        ex.values = int(values)
+    ex = _Extras()
     if gate is not None:
         _gpu(what, gate)
         cols = nq * max(1, gate_width)
@@ -81,7 +60,7 @@ def _extras(what: str, tokens: int, nq: int, gate: Optional[torch.Tensor] = None
     ex.softcap = float(softcap)
     _need(chunk >= 0, f"{what}: a chunk must not be negative")
     ex.chunk = int(chunk)
-    ex.plain_norm = 2 if long_items is not None else 3 if values else 1 if plain_norm else 0
+    ex.plain_norm = 1 if plain_norm else 0
     ex.v_head0 = int(v_head0)
     if q_temperature is not None:
         coef, every = q_temperature
@@ -195,7 +174,7 @@ def attn_mfma(q: torch.Tensor, out: torch.Tensor, nq: int, nkv: int, d: int, kca
     ``plan`` (what ``attn_plan`` made of these items for this ``n_splits``) takes the place of that even cut.
     ``long_items``: the items of prompt portions (as for ``attn_prefill``, every walk whole), in the same launch where the
     head size has a kernel for both."""
-    _gpu("attn_mfma", q, out, kcache, vcache, positions, block_table, items, part_o, part_ml, live_context, plan)
+    _gpu("attn_mfma", q, out, kcache, vcache, positions, block_table, items, part_o, part_ml, live_context, plan, long_items)
     _live(live_context)
     _planned(plan, items.numel() // ITEM_INTS, n_splits)
     tokens = q.shape[0]
@@ -208,8 +187,9 @@ def attn_mfma(q: torch.Tensor, out: torch.Tensor, nq: int, nkv: int, d: int, kca
     _int_vec("attn_mfma: positions", positions, tokens)
     _need(block_table.dim() == 2 and block_table.dtype == torch.int32 and block_table.is_contiguous(),
           "attn_mfma: block_table must be contiguous int32 [entries, width]")
-    _need(items.dtype == torch.int32 and items.is_contiguous() and items.numel() % ITEM_INTS == 0,
-          "attn_mfma: items must be int32 quadruples")
+    for listed in (items, long_items):
+        _need(listed is None or (listed.dtype == torch.int32 and listed.is_contiguous() and listed.numel() % ITEM_INTS == 0),
+              "attn_mfma: items must be int32 quadruples")
     n_items = items.numel() // ITEM_INTS
     if n_splits > 1:
         need = tokens * nq * n_splits
@@ -217,12 +197,16 @@ def attn_mfma(q: torch.Tensor, out: torch.Tensor, nq: int, nkv: int, d: int, kca
               and part_ml.dtype == torch.float32 and part_o.numel() >= need * d and part_ml.numel() >= need * 2,
               "attn_mfma: scratch for the split results is too small")
     lib = load_variant("attn_mfma", {"PULSE_HEAD_DIM": d})
-    call_in(lib, "pulse_attn_mfma", _ptr(q), _i64(q.stride(0)), _ptr(out), _i64(out.stride(0)), _ptr(kcache),
+    args = (_ptr(q), _i64(q.stride(0)), _ptr(out), _i64(out.stride(0)), _ptr(kcache),
             _ptr(vcache), _ptr(positions), _ptr(block_table), _i32(block_table.shape[1]),
             _ptr(items), _i32(n_items), _i32(tokens), _i32(nq), _i32(nkv), _i32(page_size), _i32(pages), _f32(scale),
             _i32(window), _i32(split_size), _i32(n_splits), _i32(max_context), _ptr(part_o), _ptr(part_ml),
             _ptr(live_context), _ptr(plan), _extras("attn_mfma", tokens, nq, gate, gate_width=gate_width, sink=sink, softcap=softcap,
-            chunk=chunk, long_items=long_items), _stream())
+            chunk=chunk))
+    if long_items is None:
+        call_in(lib, "pulse_attn_mfma", *args, _stream())
+    else:
+        call_in(lib, "pulse_attn_mfma_beside", *args, _ptr(long_items), _i32(long_items.numel() // ITEM_INTS), _stream())
 
 
 PLAN_MIN_KEYS = 256      # no split of a plan is shorter (what a workgroup costs beside its walk, in keys walked)
@@ -378,13 +362,16 @@ def attn_prefill(q: torch.Tensor, out: torch.Tensor, nq: int, nkv: int, d: int, 
     _need(items.dtype == torch.int32 and items.is_contiguous() and items.numel() % ITEM_INTS == 0,
           "attn_prefill: items must be int32 quadruples")
     lib = load_variant("attn_mfma", {"PULSE_HEAD_DIM": d})
-    call_in(lib, "pulse_attn_prefill", _ptr(q), _i64(q.stride(0)), _ptr(out), _i64(out.stride(0)), _ptr(kcache),
+    args = (_ptr(q), _i64(q.stride(0)), _ptr(out), _i64(out.stride(0)), _ptr(kcache),
             _ptr(vcache), _ptr(positions), _ptr(block_table), _i32(block_table.shape[1]),
             _ptr(items), _i32(items.numel() // ITEM_INTS), _i32(tokens), _i32(nq), _i32(nkv), _i32(page_size), _i32(pages),
             _f32(scale), _i32(window), _i32(split_size if n_splits > 1 else 0), _i32(n_splits),
             _ptr(part_o if n_splits > 1 else None), _ptr(part_ml if n_splits > 1 else None),
-            _extras("attn_prefill", tokens, nq, gate, gate_width=gate_width, sink=sink, softcap=softcap,
-            chunk=chunk, values=values), _stream())
+            _extras("attn_prefill", tokens, nq, gate, gate_width=gate_width, sink=sink, softcap=softcap, chunk=chunk))
+    if values:
+        call_in(lib, "pulse_attn_prefill_values", *args, _i32(values), _stream())
+    else:
+        call_in(lib, "pulse_attn_prefill", *args, _stream())
 
 
 def decode_takes(d: int, rotary_dim: int, pairing: int) -> bool:

@@ -80,3 +80,38 @@ def test_portions_of_heads_whose_values_are_narrower(values, splits, window, gat
     am.attn_prefill(q, one, *args, gate=gate, values=values)
     wanted = lambda t: t.view(rows, nq, d)[:, :, :values]
     assert not torch.isnan(wanted(two)).any() and torch.equal(wanted(one), wanted(two))
+
+
+def test_options_of_other_entry_points_are_not_read_here():
+    """``plain_norm`` of the options is for decoded tokens that are prepared on the way: whatever it holds, the entry points of prepared
+    queries do as without it, and read nothing behind the options."""
+    import ctypes
+
+    from pulse_infer_amd.ops import attention_mfma as am
+    from pulse_infer_amd.ops.library import call_in
+    from pulse_infer_amd.ops.kernels import _f32, _i32, _i64, _ptr, _stream
+
+    d, nq, nkv, page, context = 64, 4, 2, 16, 50
+    gen = torch.Generator().manual_seed(3)
+    bf = lambda *s: torch.randn(s, generator=gen).to(torch.bfloat16).to(DEV)
+    pages = (context + page - 1) // page
+    q, kc, vc = bf(context, nq * d), bf(pages, nkv, page, d), bf(pages, nkv, d, page)
+    positions = torch.arange(context, dtype=torch.int32, device=DEV)
+    table = torch.arange(pages, dtype=torch.int32, device=DEV).view(1, pages)
+    entry = [(0, Entry(0, context, 0))]
+    lib = am.load_variant("attn_mfma", {"PULSE_HEAD_DIM": d})
+    for name, per, tail in (("pulse_attn_mfma", am.tokens_per_item(nq // nkv), (_i32(context),)),
+                            ("pulse_attn_prefill", am.portion_tokens(nq // nkv, d), ())):
+        items = torch.tensor(am.build_items(entry, per), dtype=torch.int32, device=DEV)
+        results = []
+        for plain_norm in (0, 1, 2, 3, -1):
+            ex = am._Extras()
+            ex.plain_norm, ex.v_head0 = plain_norm, -1
+            out = torch.full((context, nq * d), float("nan"), dtype=torch.bfloat16, device=DEV)
+            split = (_i32(64), _i32(1)) if tail else (_i32(0), _i32(1))
+            call_in(lib, name, _ptr(q), _i64(nq * d), _ptr(out), _i64(nq * d), _ptr(kc), _ptr(vc), _ptr(positions), _ptr(table),
+                    _i32(pages), _ptr(items), _i32(items.numel() // am.ITEM_INTS), _i32(context), _i32(nq), _i32(nkv), _i32(page),
+                    _i32(pages), _f32(d ** -0.5), _i32(0), *split, *tail, _ptr(None), _ptr(None),
+                    *((_ptr(None), _ptr(None)) if tail else ()), ctypes.byref(ex), _stream())
+            results.append(out)
+        assert not torch.isnan(results[0]).any() and all(torch.equal(results[0], r) for r in results[1:])
