@@ -309,10 +309,11 @@ static_assert(REST_WORDS % 2 == 0 && REST_CHUNKS % 2 == 0, "64-bit words");
 
 __device__ __forceinline__ int bin_at(float x, float best, float scale) { return min(HIST_BINS - 1, static_cast<int>((best - x) * scale)); }
 
-// The bin in which the masses from the top reach p of the whole (or, k > 0, the counts reach k), the mass above it and the whole:
-// thread t of THREADS sums HIST_BINS / THREADS neighbouring bins.  -1 if they do not.  Called by a whole workgroup.
+// The bin in which the masses from the top reach p of the whole (or, k > 0, the counts reach k; or, given, `want`), the mass above it
+// and the whole: thread t of THREADS sums HIST_BINS / THREADS neighbouring bins.  `base` is on the way in the mass above them all, on
+// the way out that above the bin.  -1 if there is no such bin.  Called by a whole workgroup.
 template <int THREADS>
-__device__ int edge_bin(const mass_t* hist, float p, int k, mass_t* waves, int* at, mass_t* above, mass_t& base, mass_t& whole) {
+__device__ int edge_bin(const mass_t* hist, float p, int k, mass_t* waves, int* at, mass_t* above, mass_t& base, mass_t& whole, double want = -1.) {
     constexpr int PER = HIST_BINS / THREADS, WAVES = THREADS / PULSE_WAVE;
     const int lane = threadIdx.x % PULSE_WAVE, wave = threadIdx.x / PULSE_WAVE;
     mass_t bins[PER], mine = 0;
@@ -325,14 +326,14 @@ __device__ int edge_bin(const mass_t* hist, float p, int k, mass_t* waves, int* 
     if (lane == PULSE_WAVE - 1) waves[wave] = through;
     if (threadIdx.x == 0) *at = -1;
     __syncthreads();
-    mass_t before = through - mine;
+    mass_t before = base + through - mine;
     whole = 0;
 #pragma unroll
     for (int w = 0; w < WAVES; ++w) {
         if (w < wave) before += waves[w];
         whole += waves[w];
     }
-    const double want = k > 0 ? static_cast<double>(k) : static_cast<double>(p) * static_cast<double>(whole);
+    if (want < 0.) want = k > 0 ? static_cast<double>(k) : static_cast<double>(p) * static_cast<double>(whole);
     if (static_cast<double>(before) < want && static_cast<double>(before + mine) >= want) {      // one thread
         int j = 0;
         while (j < PER - 1 && static_cast<double>(before + bins[j]) < want) before += bins[j++];
@@ -599,29 +600,36 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
             for (int w = 0; w < SAMPLE_WAVES; ++w) total += part_m[w];
             return total;
         };
-        if (!found) {       // too many tokens in a bin, or no range: four bits of the threshold a pass
-            mass_t mass = 0;
-            sweep(row, threadIdx.x, vocab, SAMPLE_THREADS, [&](int, float x) { if (x != -INFINITY) mass += weigh(x); });
-            const double want = static_cast<double>(p) * static_cast<double>(block_mass(mass));
+        if (!found) {
+            // Too many tokens in a bin, or no range: the threshold's bits, eleven a pass, by a histogram over them.  (Four bits a pass,
+            // the masses above the fifteen candidates of a digit side by side in 64 bits, took eight passes and spilled 395 registers:
+            // a row of 151,936 with ties at the edge 1,855 us, so XXX; float32 sums, a quarter of the registers, 960.)
+            double want = -1.;
+            base = 0;
             thr = 0u;
-            for (int shift = 28; shift >= 0; shift -= 4) {
-                mass_t above[15];
-#pragma unroll
-                for (int j = 0; j < 15; ++j) above[j] = 0;
+            for (int pass = 0; pass < 3; ++pass) {
+                const int shift = pass == 0 ? 21 : pass == 1 ? 10 : 0, known = pass == 0 ? 32 : pass == 1 ? 21 : 10;
+                const uint32_t most = pass == 2 ? 1023u : 2047u;
+                __syncthreads();
+                for (int b = threadIdx.x; b < HIST_BINS; b += SAMPLE_THREADS) hist_m[b] = 0;
+                __syncthreads();
                 sweep<8>(row, threadIdx.x, vocab, SAMPLE_THREADS, [&](int, float x) {
-                    if (x == -INFINITY) return;
                     const uint32_t key = order_key(x);
-                    if (key < (thr | (1u << shift))) return;
-                    const mass_t w = weigh(x);
-#pragma unroll
-                    for (int j = 0; j < 15; ++j)
-                        if (key >= (thr | (static_cast<uint32_t>(j + 1) << shift))) above[j] += w;
+                    if (x == -INFINITY || (known < 32 && (key ^ thr) >> known != 0u)) return;
+                    mass_t w = weigh(x);
+                    // (one entry for lanes that all hold the same value, which would wait for one another)
+                    const unsigned long long here = __ballot(1);
+                    if (__ballot(key == static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(key))) == here) {
+                        if (lane != __builtin_ctzll(here)) return;
+                        w *= static_cast<mass_t>(__builtin_popcountll(here));
+                    }
+                    atomicAdd(&hist_m[most - ((key >> shift) & most)], w);
                 });
-                uint32_t digit = 0u;
-#pragma unroll
-                for (int j = 0; j < 15; ++j)
-                    if (static_cast<double>(block_mass(above[j])) >= want) digit = static_cast<uint32_t>(j + 1);
-                thr |= digit << shift;
+                __syncthreads();
+                const int at = edge_bin<SAMPLE_THREADS>(hist_m, p, 0, part_m, si, &edge_above, base, whole_m, want);
+                if (at < 0) { thr = 0xffffffffu; break; }     // (no weight is a number)
+                if (pass == 0) want = static_cast<double>(p) * static_cast<double>(whole_m);
+                thr |= (most - at) << shift;
             }
         }
         // the kept mass of every wavefront's part, then the part in which the draw falls is walked by its wavefront
