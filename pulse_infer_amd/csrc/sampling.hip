@@ -299,7 +299,7 @@ __device__ __forceinline__ mass_t mass_through(mass_t v) {
     return v;
 }
 
-// What the kernels in front of sample_kernel leave of a row that the chunks could not choose for, in 32-bit words: the histogram
+// What the kernels in front of left_kernel leave of a row that the chunks could not choose for, in 32-bit words: the histogram
 // over [lowest, best] (rows with top-k: counts; top-p alone: masses; 64 bits each), the row's smallest number, whether its token is
 // chosen after all, the mass of the bins above the one with top-p's edge, that of the row, and every chunk's of the former.
 constexpr int REST_LOWEST = 2 * HIST_BINS, REST_CHOSEN = REST_LOWEST + 1, REST_BASE = REST_LOWEST + 2, REST_WHOLE = REST_LOWEST + 4;
@@ -366,19 +366,19 @@ __device__ __forceinline__ mass_t draw_from(float u, mass_t kept) {
 
 constexpr int EDGE_CAP = 1024;   // tokens of the edge's bin that are ranked
 
-__global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
+// A row by a workgroup of SAMPLE_THREADS.  `chunked`: behind the kernels that work in chunks, which left the chunks' maxima, and in
+// `rest` what they have been over the row for, or null.
+__device__ __forceinline__ void sample_row(
     const float* __restrict__ logits, int vocab, int64_t row_stride, const float* __restrict__ temperature,
     const int* __restrict__ top_k, const float* __restrict__ top_p, const float* __restrict__ uniform,
     const float* __restrict__ penalty, const int* __restrict__ seen_row, const uint32_t* __restrict__ seen_masks,
-    const uint32_t* __restrict__ banned, int mask_words, int* __restrict__ out, const int* __restrict__ done,
+    const uint32_t* __restrict__ banned, int mask_words, int* __restrict__ out, const bool chunked,
     const float* __restrict__ part_max, const int* __restrict__ part_idx, int chunks, const int* __restrict__ rest) {
     __shared__ float sf[SAMPLE_WAVES];
     __shared__ int si[SAMPLE_WAVES];
     __shared__ mass_t hist_m[HIST_BINS];    // top-p alone: the bins' masses
     int* const hist = reinterpret_cast<int*>(hist_m);
     if (rest) rest += static_cast<int64_t>(blockIdx.x) * REST_WORDS;
-    // the kernels that work in chunks have chosen this row's token already
-    if (done && (done[blockIdx.x] || (rest && rest[REST_CHOSEN]))) return;
     __shared__ int wave_bins[SAMPLE_WAVES];
     __shared__ int region_i[SAMPLE_WAVES][WAVE_CAP];
     __shared__ float region_x[SAMPLE_WAVES][WAVE_CAP];
@@ -443,7 +443,7 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
     const bool by_k = k > 0 && k < vocab;
     const int k_list = by_k ? k : min(vocab - 1, LIST_TRY);
     float whole = 0.f;   // without top-k: the mass of the whole vocabulary, which top_p refers to
-    if (by_k || (use_p && k_list > 0 && !done)) {
+    if (by_k || (use_p && k_list > 0 && !chunked)) {
         if (rest) {      // (the kernels before have been over the row)
             lowest = __int_as_float(rest[REST_LOWEST]);
         } else if (!by_k) {
@@ -603,7 +603,7 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
         if (!found) {
             // Too many tokens in a bin, or no range: the threshold's bits, eleven a pass, by a histogram over them.  (Four bits a pass,
             // the masses above the fifteen candidates of a digit side by side in 64 bits, took eight passes and spilled 395 registers:
-            // a row of 151,936 with ties at the edge 1,855 us, so XXX; float32 sums, a quarter of the registers, 960.)
+            // a row of 151,936 with ties at the edge 1,855 us, so 408.)
             double want = -1.;
             base = 0;
             thr = 0u;
@@ -743,6 +743,15 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
     if (lane == 0) out[r] = e >= 0 ? e : (last >= 0 ? last : best_i);
 }
 
+__global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
+    const float* __restrict__ logits, int vocab, int64_t row_stride, const float* __restrict__ temperature,
+    const int* __restrict__ top_k, const float* __restrict__ top_p, const float* __restrict__ uniform,
+    const float* __restrict__ penalty, const int* __restrict__ seen_row, const uint32_t* __restrict__ seen_masks,
+    const uint32_t* __restrict__ banned, int mask_words, int* __restrict__ out) {
+    sample_row(logits, vocab, row_stride, temperature, top_k, top_p, uniform, penalty, seen_row, seen_masks, banned, mask_words, out,
+               false, nullptr, nullptr, 0, nullptr);
+}
+
 __global__ void mark_seen_kernel(uint32_t* __restrict__ masks, int mask_words, const int* __restrict__ rows,
                                  const int* __restrict__ tokens, int n, int vocab) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -804,7 +813,7 @@ __global__ __launch_bounds__(PULSE_WAVE) void argmax_merge_kernel(const float* _
 // known about the row as a whole but its maximum and its mass, so the row is cut into chunks of SIMPLE_CHUNK logits
 // with a workgroup each: the chunk's maximum (with its lowest index); then, the row's maximum known, the chunk's
 // mass; then one wavefront a row finds the chunk in which u * mass falls (chunk masses summed in chunk order) and
-// walks that chunk alone (chunked_choose_kernel).  The steps and their meaning are those of sample_kernel; sums are
+// walks that chunk alone (chunked_choose_kernel).  The steps and their meaning are those of sample_row; sums are
 // taken in another order.
 constexpr int SIMPLE_CHUNK = 2048;
 constexpr int SIMPLE_THREADS = 256;
@@ -899,15 +908,15 @@ __global__ __launch_bounds__(SIMPLE_THREADS) void simple_mass_kernel(
 // lower bound of the k-th largest logit (that many logits, the maxima themselves, reach it), so everything that
 // top-k keeps lies at or above it, and little else: a workgroup a chunk collects what it has there, in vocabulary
 // order, into its own short segment; a wavefront a row strings the segments together in LDS and finishes on that list
-// as sample_kernel does on its own (finish_on_list).  A row that does not fit (k above the number of chunks, a chunk
-// with more candidates than its segment holds: many equal values) is left to sample_kernel, which runs behind and
+// as sample_row does on its own (finish_on_list).  A row that does not fit (k above the number of chunks, a chunk
+// with more candidates than its segment holds: many equal values) is left to left_kernel, which runs behind and
 // skips the rows that are done.
 constexpr int TOPK_SEGMENT = 32;   // candidates a chunk may leave
 
 // A row with top-p alone takes the same way with what lies at or above one of the lower chunk maxima (seven eighths
 // of the chunks have a larger one): some hundreds of the largest logits of a vocabulary of 150,000, which hold the
 // top_p share of a distribution as peaked as a language model's; if they do not (or a chunk has more than its segment
-// holds), the row is left to sample_kernel too.  The mass of the whole row, which top_p refers to, comes from
+// holds), the row is left to left_kernel too.  The mass of the whole row, which top_p refers to, comes from
 // simple_mass_kernel.
 __device__ __forceinline__ int top_p_bound_rank(int chunks) { return max(1, chunks - chunks / 8); }
 
@@ -1018,6 +1027,11 @@ __device__ __forceinline__ void string_segments(const int* seg_i, const float* s
     }
 }
 
+// How the choice in chunks leaves a row, in `done`: its token is chosen; left; left with so large a k that no segments will hold its
+// list (half full on average), for a workgroup alone, which goes by the histogram of the whole row, or, where a workgroup's own
+// passes over a short row cost no more than that, without it.
+enum { LEFT = 0, CHOSEN = 1, LEFT_COUNTED = 2, LEFT_ALONE = 3 };
+
 // What rest_kernel adds a row's histogram to, and that the row's token is not chosen.
 __device__ __forceinline__ void clear_rest(int* rest, int lane) {
     for (int b = lane; b <= REST_CHOSEN; b += PULSE_WAVE) rest[b] = 0;
@@ -1026,7 +1040,7 @@ __device__ __forceinline__ void clear_rest(int* rest, int lane) {
 // The choice of every row from what the kernels before left, a wavefront a row: the largest logit for greedy rows;
 // for rows with top-k the candidates' segments strung together in LDS and finished there; for rows that draw from the
 // whole vocabulary the chunk in which u * mass falls (chunk masses in chunk order), walked alone.  done[r] says
-// whether the row's token is chosen; the others (rows that did not fit) are sample_kernel's.
+// whether the row's token is chosen; the others (rows that did not fit) are left_kernel's.
 __global__ __launch_bounds__(PULSE_WAVE) void chunked_choose_kernel(
     const float* __restrict__ logits, int vocab, int64_t row_stride, const float* __restrict__ temperature,
     const int* __restrict__ top_k, const float* __restrict__ top_p, const float* __restrict__ uniform,
@@ -1075,7 +1089,8 @@ __global__ __launch_bounds__(PULSE_WAVE) void chunked_choose_kernel(
         const int first = __shfl(pre0, PULSE_WAVE - 1, PULSE_WAVE);      // candidates of chunks 0 .. 63
         const int n = first + __shfl(pre1, PULSE_WAVE - 1, PULSE_WAVE);
         if (k > chunks || chunks > 2 * PULSE_WAVE || __ballot(over) != 0ull || n > LIST_CAP || n < k || n == 0) {
-            if (lane == 0) done[r] = 0;   // not a row for these kernels: sample_kernel takes it
+            // not a row for these kernels
+            if (lane == 0) done[r] = !by_k || k <= chunks * (TOPK_SEGMENT / 2) ? LEFT : vocab >= 1024 * static_cast<int64_t>(gridDim.x) ? LEFT_COUNTED : LEFT_ALONE;
             if (left) clear_rest(left + static_cast<int64_t>(r) * REST_WORDS, lane);
             return;
         }
@@ -1143,11 +1158,12 @@ __global__ __launch_bounds__(PULSE_WAVE) void chunked_choose_kernel(
     if (lane == 0) { out[r] = e >= 0 ? e : (last >= 0 ? last : best_i); done[r] = 1; }
 }
 
-// ---- the rows that are left, before sample_kernel ---------------------------------------------------------------
+// ---- the rows that are left ---------------------------------------------------------------------------------------
 // A workgroup a row goes over its row at the rate of one compute unit.  What has to be known of the whole row, the histogram
 // over [lowest, best], is made by many (the lowest value comes with the maxima, and the histogram is cleared by the kernel that
-// leaves the row); with it a row is finished in chunks as well (left_collect_kernel, left_choose_kernel), unless a chunk has more
-// tokens at the edge than its segment holds: those rows are sample_kernel's.
+// leaves the row); with it a row is finished in chunks as well (left_collect_kernel, left_choose), unless a chunk has more
+// tokens at the edge than its segment holds: those rows a workgroup goes over alone (sample_row), in the launch that chooses.
+// (left_choose by a kernel of its own: every call waits for one launch more, top-p or top-k in 33 to 37 us, 37 to 41.)
 // 32 rows of 151,936, six of them flat under top-p alone and six with a k above the number of chunks: these three kernels 41 us,
 // where the histogram with float32 masses and sample_kernel's passes took 31 and 128.
 constexpr int REST_GROUPS = 32;                                             // workgroups for a row's histogram
@@ -1182,13 +1198,13 @@ __global__ __launch_bounds__(SIMPLE_THREADS) void rest_kernel(
     int* __restrict__ rest) {
     __shared__ mass_t hist[HIST_BINS];
     const int r = blockIdx.y;
-    if (done[r]) return;
+    if (done[r] == CHOSEN || done[r] == LEFT_ALONE) return;
     rest += static_cast<int64_t>(r) * REST_WORDS;
     for (int b = threadIdx.x; b < HIST_BINS; b += SIMPLE_THREADS) hist[b] = 0;
     const LeftRow left(r, vocab, chunks, temperature, top_k, top_p, part_max, part_min);
     if (blockIdx.x == 0 && threadIdx.x == 0) rest[REST_LOWEST] = __float_as_int(left.lowest);
     __syncthreads();
-    if (!left.ranged) return;    // (as sample_kernel: no histogram)
+    if (!left.ranged) return;    // (as sample_row: no histogram)
     const RowView row = simple_row(logits, r, row_stride, vocab, penalty, seen_row, seen_masks, banned, mask_words);
     const Weigh weigh(left.best, left.inv_t, vocab);
     const int first = blockIdx.x * SIMPLE_THREADS + threadIdx.x;
@@ -1219,7 +1235,7 @@ __global__ __launch_bounds__(SIMPLE_THREADS) void left_collect_kernel(
     __shared__ int at_s, counts[WAVES];
     const int r = blockIdx.y, chunk = blockIdx.x, chunks = gridDim.x;
     const int lane = threadIdx.x % PULSE_WAVE, wave = threadIdx.x / PULSE_WAVE;
-    if (done[r]) return;
+    if (done[r] != LEFT) return;
     const RowView row = simple_row(logits, r, row_stride, vocab, penalty, seen_row, seen_masks, banned, mask_words);
     const int begin = chunk * SIMPLE_CHUNK + static_cast<int>(threadIdx.x) * PER;
     float xs[PER];        // (asked for first: they travel while the edge is searched)
@@ -1281,16 +1297,17 @@ __global__ __launch_bounds__(SIMPLE_THREADS) void left_collect_kernel(
     }
 }
 
-// The choice of such a row.  Top-k: on the strung segments, as sample_kernel's.  Top-p alone: the edge among the collected tokens,
-// the chunk in which the draw falls, its token.
-__global__ __launch_bounds__(SIMPLE_THREADS) void left_choose_kernel(
+// The choice of such a row by a workgroup of THREADS; false if it does not fit.  Top-k: on the strung segments, as sample_row's.
+// Top-p alone: the edge among the collected tokens, the chunk in which the draw falls, its token.
+template <int THREADS>
+__device__ __forceinline__ bool left_choose(
     const float* __restrict__ logits, int vocab, int64_t row_stride, const float* __restrict__ temperature,
     const int* __restrict__ top_k, const float* __restrict__ top_p, const float* __restrict__ uniform,
     const float* __restrict__ penalty, const int* __restrict__ seen_row, const uint32_t* __restrict__ seen_masks,
     const uint32_t* __restrict__ banned, int mask_words, const float* __restrict__ part_max, const float* __restrict__ part_min,
-    const int* __restrict__ part_idx, int chunks, const int* __restrict__ done, const int* __restrict__ seg_i, const float* __restrict__ seg_x,
+    const int* __restrict__ part_idx, int chunks, const int* __restrict__ seg_i, const float* __restrict__ seg_x,
     const int* __restrict__ seg_n, int* __restrict__ rest, int* __restrict__ out) {
-    constexpr int WAVES = SIMPLE_THREADS / PULSE_WAVE, PER = SIMPLE_CHUNK / SIMPLE_THREADS;
+    constexpr int WAVES = THREADS / PULSE_WAVE, PER = SIMPLE_CHUNK / THREADS;
     __shared__ int list_i[LIST_CAP];
     __shared__ float list_x[LIST_CAP];
     __shared__ int first_s[REST_MOST_CHUNKS + 1], n_s;
@@ -1298,9 +1315,8 @@ __global__ __launch_bounds__(SIMPLE_THREADS) void left_choose_kernel(
     __shared__ uint32_t keys[EDGE_CAP], best_s;
     __shared__ int who_s;
     const int r = blockIdx.x, lane = threadIdx.x % PULSE_WAVE, wave = threadIdx.x / PULSE_WAVE;
-    if (done[r]) return;
     const LeftRow left(r, vocab, chunks, temperature, top_k, top_p, part_max, part_min);
-    if (left.k == 0 && !left.by_p) return;
+    if (left.k == 0 && !left.by_p) return false;
     rest += static_cast<int64_t>(r) * REST_WORDS;
     seg_n += static_cast<int64_t>(r) * chunks;
     const int64_t segment = static_cast<int64_t>(r) * chunks * TOPK_SEGMENT;
@@ -1321,11 +1337,11 @@ __global__ __launch_bounds__(SIMPLE_THREADS) void left_choose_kernel(
     if (static_cast<int>(threadIdx.x) < chunks) chunk_m[threadIdx.x] = *reinterpret_cast<const mass_t*>(rest + REST_CHUNKS + 2 * threadIdx.x);
     __syncthreads();
     const int n = n_s;
-    if (n == 0 || n > (left.k > 0 ? LIST_CAP : EDGE_CAP)) return;
-    string_segments<SIMPLE_THREADS>(seg_i + segment, seg_x + segment, first_s, chunks, list_i, list_x);
+    if (n == 0 || n > (left.k > 0 ? LIST_CAP : EDGE_CAP)) return false;
+    string_segments<THREADS>(seg_i + segment, seg_x + segment, first_s, chunks, list_i, list_x);
     __syncthreads();
     if (left.k > 0) {
-        if (wave != 0) return;
+        if (wave != 0) return true;
         // (where no weight is a number above zero, the largest logit)
         float largest = -INFINITY;
         int best_i = 0x7fffffff;
@@ -1340,21 +1356,21 @@ __global__ __launch_bounds__(SIMPLE_THREADS) void left_choose_kernel(
         if (n <= 8 * PULSE_WAVE) finish_on_list<8>(list_i, list_x, n, true, left.k, use_p, left.p, 0.f, left.best, left.inv_t, uniform[r], best_i, token);
         else finish_on_list<LIST_PER_LANE>(list_i, list_x, n, true, left.k, use_p, left.p, 0.f, left.best, left.inv_t, uniform[r], best_i, token);
         if (lane == 0) { out[r] = token; rest[REST_CHOSEN] = 1; }
-        return;
+        return true;
     }
     const Weigh weigh(left.best, left.inv_t, vocab);
     const float p = left.p;
-    for (int e = threadIdx.x; e < n; e += SIMPLE_THREADS) {
+    for (int e = threadIdx.x; e < n; e += THREADS) {
         keys[e] = order_key(list_x[e]);
         masses[e] = weigh(list_x[e]);
     }
     __syncthreads();
-    edge_key(keys, masses, n, SIMPLE_THREADS, *reinterpret_cast<const mass_t*>(rest + REST_BASE),
+    edge_key(keys, masses, n, THREADS, *reinterpret_cast<const mass_t*>(rest + REST_BASE),
              *reinterpret_cast<const mass_t*>(rest + REST_WHOLE), p, &best_s);
     __syncthreads();
     const uint32_t thr = best_s;
-    if (thr == 0u) return;
-    for (int e = threadIdx.x; e < n; e += SIMPLE_THREADS)
+    if (thr == 0u) return false;
+    for (int e = threadIdx.x; e < n; e += THREADS)
         if (keys[e] >= thr) atomicAdd(&chunk_m[list_i[e] / SIMPLE_CHUNK], masses[e]);
     __syncthreads();
     if (wave == 0) {      // the chunk in which u of the kept mass falls, two chunks a lane
@@ -1387,11 +1403,31 @@ __global__ __launch_bounds__(SIMPLE_THREADS) void left_choose_kernel(
     mass_t before = through - mine;
     for (int w = 0; w < wave; ++w) before += waves[w];
     const mass_t target = target_s;
-    if (target < before || target >= before + mine) return;            // one thread has it
-    int j = 0;
-    while (target >= before + ms[j]) before += ms[j++];
-    out[r] = begin + j;
-    rest[REST_CHOSEN] = 1;
+    if (target >= before && target < before + mine) {                  // one thread has it
+        int j = 0;
+        while (target >= before + ms[j]) before += ms[j++];
+        out[r] = begin + j;
+        rest[REST_CHOSEN] = 1;
+    }
+    return true;
+}
+
+// The rows that are left: by what the kernels before collected, else by their workgroup alone.
+__global__ __launch_bounds__(SAMPLE_THREADS) void left_kernel(
+    const float* __restrict__ logits, int vocab, int64_t row_stride, const float* __restrict__ temperature,
+    const int* __restrict__ top_k, const float* __restrict__ top_p, const float* __restrict__ uniform,
+    const float* __restrict__ penalty, const int* __restrict__ seen_row, const uint32_t* __restrict__ seen_masks,
+    const uint32_t* __restrict__ banned, int mask_words, const float* __restrict__ part_max, const float* __restrict__ part_min,
+    const int* __restrict__ part_idx, int chunks, const int* __restrict__ done, const int* __restrict__ seg_i, const float* __restrict__ seg_x,
+    const int* __restrict__ seg_n, int* __restrict__ rest, int* __restrict__ out) {
+    const int how = done[blockIdx.x];
+    if (how == CHOSEN) return;
+    if (rest && how == LEFT && chunks <= REST_MOST_CHUNKS &&
+        left_choose<SAMPLE_THREADS>(logits, vocab, row_stride, temperature, top_k, top_p, uniform, penalty, seen_row, seen_masks, banned,
+                                    mask_words, part_max, part_min, part_idx, chunks, seg_i, seg_x, seg_n, rest, out)) return;
+    __syncthreads();
+    sample_row(logits, vocab, row_stride, temperature, top_k, top_p, uniform, penalty, seen_row, seen_masks, banned, mask_words, out, true,
+               part_max, part_idx, chunks, how == LEFT_ALONE ? nullptr : rest);
 }
 
 }  // namespace
@@ -1479,9 +1515,7 @@ extern "C" int pulse_sample(const float* logits, int rows, int vocab, int64_t ro
                   mask_words * 32, vocab);
     if (rows == 0) return 0;
     hipLaunchKernelGGL(sample_kernel, dim3(rows), dim3(SAMPLE_THREADS), 0, stream, logits, vocab, row_stride,
-                       temperature, top_k, top_p, uniform, penalty, seen_row, seen_masks, banned, mask_words, out,
-                       static_cast<const int*>(nullptr), static_cast<const float*>(nullptr),
-                       static_cast<const int*>(nullptr), 0, static_cast<const int*>(nullptr));
+                       temperature, top_k, top_p, uniform, penalty, seen_row, seen_masks, banned, mask_words, out);
     PULSE_LAUNCH_CHECK("sample");
     return 0;
 }
@@ -1490,9 +1524,9 @@ extern "C" int pulse_sample(const float* logits, int rows, int vocab, int64_t ro
 // workgroup a row of pulse_sample does.  Greedy rows, rows that draw from the whole vocabulary at their temperature
 // rows with top-k (and top-p on what it keeps) whose k is at most the number of chunks and rows with top-p alone whose
 // top_p share lies in some hundreds of the largest logits are chosen by these kernels; rows that do not fit (a larger k, a
-// distribution too flat for top-p alone) by three more that go by a histogram of the row, and what does not fit these either (many
-// equal values at the edge) by the kernel of pulse_sample behind them, which skips the rows that are done.  What a row's choice is
-// does not depend on the other rows.  Whole calls, us, before the histogram's kernels finished rows: 32,000 values, 3 / 16 / 64 rows
+// distribution too flat for top-p alone) by three more that go by a histogram of the row, the last of which takes what does not fit
+// these either (many equal values at the edge, a k beyond half of what the segments hold) as pulse_sample does.  What a row's choice
+// is does not depend on the other rows.  Whole calls, us, before the histogram's kernels finished rows: 32,000 values, 3 / 16 / 64 rows
 // 136 / 150 / 187 -> 94 / 119 / 161; 151,936 values 208 / 241 / 327 -> 103 / 131 / 200.  Scratch, with chunks = pulse_sample_chunks(vocab): part_max, part_mass (float32), part_idx, seg_n
 // (int32) of rows * chunks entries; seg_i (int32), seg_x (float32) of rows * chunks * pulse_sample_segment()
 // entries; done (int32) of rows entries; and, optional (null: the rows that are left are gone over by their own workgroups
@@ -1549,17 +1583,14 @@ extern "C" int pulse_sample_chunked_rest(const float* logits, int rows, int voca
             hipLaunchKernelGGL(left_collect_kernel, dim3(chunks, rows), dim3(SIMPLE_THREADS), 0, stream, logits, vocab, row_stride,
                                temperature, top_k, top_p, penalty, seen_row, seen_masks, banned, mask_words, part_max, part_min,
                                static_cast<const int*>(done), seg_i, seg_x, seg_n, rest);
-            hipLaunchKernelGGL(left_choose_kernel, dim3(rows), dim3(SIMPLE_THREADS), 0, stream, logits, vocab, row_stride,
-                               temperature, top_k, top_p, uniform, penalty, seen_row, seen_masks, banned, mask_words, part_max, part_min,
-                               static_cast<const int*>(part_idx), chunks, static_cast<const int*>(done), static_cast<const int*>(seg_i), static_cast<const float*>(seg_x),
-                               static_cast<const int*>(seg_n), rest, out);
         }
         PULSE_LAUNCH_CHECK("sample_chunked (what is left)");
     }
     if (leaves) {
-        hipLaunchKernelGGL(sample_kernel, dim3(rows), dim3(SAMPLE_THREADS), 0, stream, logits, vocab, row_stride,
-                           temperature, top_k, top_p, uniform, penalty, seen_row, seen_masks, banned, mask_words, out,
-                           static_cast<const int*>(done), part_max, part_idx, chunks, static_cast<const int*>(rest));
+        hipLaunchKernelGGL(left_kernel, dim3(rows), dim3(SAMPLE_THREADS), 0, stream, logits, vocab, row_stride,
+                           temperature, top_k, top_p, uniform, penalty, seen_row, seen_masks, banned, mask_words, part_max, part_min,
+                           static_cast<const int*>(part_idx), chunks, static_cast<const int*>(done), static_cast<const int*>(seg_i),
+                           static_cast<const float*>(seg_x), static_cast<const int*>(seg_n), rest, out);
         PULSE_LAUNCH_CHECK("sample_chunked (the rest)");
     }
     return 0;

@@ -1081,11 +1081,12 @@ def sample_chunked(logits: torch.Tensor, out: torch.Tensor, scratch: dict, tempe
                    seen_row: Optional[torch.Tensor] = None, seen_masks: Optional[torch.Tensor] = None,
                    banned: Optional[torch.Tensor] = None) -> None:
     """``sample`` in chunks of the vocabulary with a workgroup each instead of a workgroup a row: greedy rows, rows
-    that draw from the whole vocabulary and rows with top-k (k at most the number of chunks) are chosen from what the
-    chunks leave; rows with top-p alone, and what does not fit, go through the kernel of ``sample`` behind them,
-    which one more has prepared.
-    Which way a row goes depends on the row alone.  ``scratch`` as ``sample_chunked_scratch`` makes it; without its
-    ``rest`` that one does not run, and the choices are the same."""
+    that draw from the whole vocabulary, rows with top-k (k at most the number of chunks) and rows with top-p alone whose
+    share lies in some hundreds of the largest logits are chosen from what the chunks leave.  Three more kernels take the others:
+    they go by a histogram of the row and collect in chunks what lies at its edge; what fits no segments (many equal values, a
+    large k) the last of them goes over with a workgroup a row, as ``sample``.
+    Which way a row goes depends on the row alone (for a large k in a short row, on the number of rows).  ``scratch`` as ``sample_chunked_scratch`` makes it; without its
+    ``rest`` there is no histogram and the last kernel takes every row that is left, with the same choices."""
     names = ("part_max", "part_idx", "part_mass", "seg_i", "seg_x", "seg_n", "done")
     _gpu("sample_chunked", logits, out, temperature, top_k, top_p, uniform, penalty, seen_row, seen_masks, banned,
          *(scratch[n] for n in names), scratch.get("rest"))
