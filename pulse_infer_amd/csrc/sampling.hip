@@ -1142,6 +1142,10 @@ __global__ __launch_bounds__(PULSE_WAVE) void chunked_choose_kernel(
         }
     }
     float rest = target - run;
+    if (who < 0 && last_chunk < 0) {      // (no weight is a number above zero)
+        if (lane == 0) { out[r] = best_i; done[r] = CHOSEN; }
+        return;
+    }
     if (who < 0) {  // rounding left the target beyond the last chunk with mass: its last kept entry
         who = last_chunk;
         rest = INFINITY;

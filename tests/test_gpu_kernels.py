@@ -1610,3 +1610,19 @@ def test_rows_whose_weights_are_no_numbers_choose_the_largest_logit(k, vocab, p,
         out = torch.full((3,), -9, dtype=torch.int32, device=DEV)
         choose(out)
         assert out.tolist() == largest
+
+
+@pytest.mark.parametrize("vocab", [5, 2049, 40000])
+def test_draws_from_the_whole_vocabulary_without_weights_choose_the_largest_logit(k, vocab):
+    """Rows at a temperature alone whose weights are no numbers above zero (a temperature whose inverse is infinite, an infinite
+    logit), the first row of all among them: the largest logit, in chunks and by a workgroup a row."""
+    gen = torch.Generator().manual_seed(vocab)
+    logits = torch.randn(3, vocab, generator=gen)
+    largest = [vocab // 2, vocab - 1, vocab // 3]
+    for r, at in enumerate(largest):
+        logits[r, at] = float("inf") if r == 2 else 9.0
+    kw = dict(temperature=torch.tensor([1e-39, 2e-40, 0.7]).to(DEV), uniform=torch.tensor([0.0, 0.5, 0.9]).to(DEV))
+    chunked, whole = (torch.full((3,), -9, dtype=torch.int32, device=DEV) for _ in range(2))
+    k.sample_chunked(logits.to(DEV), chunked, _chunked_scratch(k, 3, vocab), **kw)
+    k.sample(logits.to(DEV), whole, **kw)
+    assert chunked.tolist() == largest and whole.tolist() == largest
