@@ -746,12 +746,15 @@ def attn_wide(q: torch.Tensor, out: torch.Tensor, nq: int, nkv: int, d: int, wv:
 
 def attn_wide_splits(n_items: int, chunks: int, keys: int) -> int:
     """Over how many workgroups ``attn_wide`` shares an item's keys out: enough that the launch has about two
-    workgroups a compute unit, every one with three steps of 32 keys or more (the last with what is left).  A step a
-    wavefront of four: 8 requests of 1,500 tokens in 8 / 11 / 12 / 16 splits (6, 5, 4, 3 steps) 28 / 37 / 31 / 28 us, one of 600 in 4 / 8 25 / 19."""
+    workgroups a compute unit, every one with three steps of 32 keys or so (129 to 160 keys in three and two, the last of more
+    with what is left).  A step a wavefront of four: 8 requests of 1,500 tokens in 8 / 11 / 12 / 16 splits (6, 5, 4, 3 steps)
+    28 / 37 / 31 / 28 us, one of 600 in 4 / 8 25 / 19.  Up to four steps a workgroup has a wavefront for each, and a cut costs the
+    second kernel for nothing: 97 and 128 keys whole / in two 15.6 / 19.1 and 15.9 / 19.5 us; 160 keys 22.7 / 19.4."""
     from .device import compute_units
     base = max(1, n_items * chunks)
     want = (2 * compute_units() + base - 1) // base
-    return max(1, min(want, 16, (keys + 95) // 96))
+    steps = (keys + 31) // 32
+    return max(1, min(want, 16, 1 if steps <= 4 else (steps + 2) // 3))
 
 
 def head_mix(x: torch.Tensor, mix: torch.Tensor, out: torch.Tensor, heads: int, kv_heads: int, d: int, dv: int,

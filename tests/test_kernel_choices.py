@@ -228,3 +228,14 @@ def test_plain_products_in_stages_keep_the_compute_units_busy(monkeypatch):
             if takes(m, n, k):
                 tiles = -(-n // tile[0]) * -(-m // tile[1])
                 assert tiles >= 0.33 * 256
+
+
+def test_keys_of_four_steps_are_not_cut_over_workgroups(units):
+    """attn_wide's splits: none up to a step of 32 keys for each of a workgroup's wavefronts; beyond, two to three steps or more each."""
+    from pulse_infer_amd.ops import kernels as K
+
+    assert all(K.attn_wide_splits(items, 2, keys) == 1 for items in (1, 4, 8, 32, 1000) for keys in (1, 32, 96, 97, 128))
+    for items, keys in itertools.product((1, 4, 8, 32), (129, 160, 161, 256, 600, 1500, 40000)):
+        n, steps = K.attn_wide_splits(items, 2, keys), (keys + 31) // 32
+        assert 1 <= n <= 16 and (steps + n - 1) // n >= 3
+        assert n == 1 or items * 2 * (n - 1) < 2 * units
