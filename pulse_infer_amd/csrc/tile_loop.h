@@ -17,14 +17,15 @@ typedef __attribute__((ext_vector_type(8))) __bf16 tile_bf16x8;
 typedef __attribute__((ext_vector_type(4))) __bf16 tile_bf16x4;
 typedef __attribute__((ext_vector_type(16))) float tile_f32x16;
 
-
 // Where along K (of so many steps) the tiles of a block of TILE_BLOCK weight rows start.  Rows of a power of two bytes, at the
 // same place in all of a launch's workgroups at a time, fall on few of the memory's channels; blocks that start elsewhere, in
 // turns of five steps, spread over them.  A function of the weight's row alone, and every tile lies inside a block: a result's
-// sums have one order, whatever the tile.  (24,576 x 4,096 with SwiGLU: 70 / 97 / 128 rows 44 / 45.5 / 47 us -> 37.5 / 38.6 / 41,
-// more rows the same; the 8B shape's other products lose or gain less than half a microsecond.)
+// sums have one order, whatever the tile.  (All at the start -> this: 22,016 x 4,096 with SwiGLU at 70 / 97 / 128 / 256 rows 39.6 /
+// 41.5 / 43.9 / 57.7 us -> 34.1 / 36.9 / 39.4 / 54.5; 64 experts of 1,024 x 2,048, 8 chosen a token, 32 / 211 tokens 150 / 168 -> 137 /
+// 152.  Rows of other lengths lie on channels of their own as it is, and their blocks start together: 34,816 x 5,120 at 70 / 128
+// rows 69.9 / 73.6 so, 71.0 / 75.0 in turns; 19,456 x 2,560 26.1 / 31.1 and 26.8 / 31.7.)
 constexpr int TILE_BLOCK = 768;
-__device__ __forceinline__ int tile_first_step(int block, int steps) { return static_cast<int>(block * 5u % static_cast<uint32_t>(steps)); }
+__device__ __forceinline__ int tile_first_step(int block, int steps) { return (steps & (steps - 1)) == 0 ? (block * 5) & (steps - 1) : 0; }
 
 template <int WR, int XR, int WN, int WM, int S, bool NT = false, int SX = S>
 struct TileLoop {

@@ -217,3 +217,16 @@ def test_gate_and_up_in_stages_do_not_depend_on_the_rows_beside_them():
         kernels.gemm_stages(x[:m], w, act, swiglu=True)
         assert torch.equal(act, whole[:m]), m
     assert len(tiles) >= 4
+
+
+@pytest.mark.parametrize("k", [320, 2560])
+@pytest.mark.parametrize("rows", [70, 300])
+def test_blocks_of_weight_rows_start_together_where_their_rows_are_no_power_of_two(rows, k):
+    """Rows of another length lie on channels of their own: their sums have the one order of K, whichever block they lie in."""
+    from pulse_infer_amd.ops import kernels
+
+    x, block = rnd(rows, k, seed=5).to(torch.bfloat16).to(DEV), rnd(768, k, seed=6).to(torch.bfloat16).to(DEV)
+    w = block.repeat(4, 1).contiguous()
+    act = torch.full((rows, 1536), float("nan"), dtype=torch.bfloat16, device=DEV)
+    kernels.gemm_stages(x, w, act, swiglu=True)
+    assert not torch.isnan(act).any() and torch.equal(act[:, :768], act[:, 768:])
