@@ -194,6 +194,13 @@ __device__ __forceinline__ int live_split_size(int live, int n_splits, int split
 // scalar work and uniform branches.
 __device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
 
+// A number of a list that the launch only reads, the same for every lane.  Said to lie in constant memory, so that the scalar unit
+// reads it whatever else the kernel holds: beside another body the compiler took it for something that may be written, read a
+// step's pages through the vector unit, and so waited for all keys and values in flight with every one of them.
+__device__ __forceinline__ int listed_int(const int* p) {
+    return *(const int __attribute__((address_space(4)))*)(reinterpret_cast<uintptr_t>(p));
+}
+
 // Page index and slot of a key: a shift when the page size is a power of two (divisions by a run-time
 // number cost dozens of scalar instructions in the inner loop).
 __device__ __forceinline__ void page_of(int j, int page_size, int page_shift, int& pi, int& slot) {
@@ -331,8 +338,8 @@ __device__ __forceinline__ void attn_mfma_workgroup(const MfmaArgs& a, const int
     int item = block / heads / a.n_splits;
     if (a.plan) {
         const int k = block / heads;
-        if (k >= a.plan[0]) return;
-        const int s = a.plan[1 + k];
+        if (k >= listed_int(a.plan)) return;
+        const int s = listed_int(a.plan + 1 + k);
         item = s / a.n_splits;
         split = s % a.n_splits;
     }
@@ -348,13 +355,13 @@ __device__ __forceinline__ void attn_mfma_workgroup(const MfmaArgs& a, const int
     // dependent trips to memory before a workgroup streams is item -> block table -> keys.  The positions (which only
     // decide masks and the end of the walk) and q travel at the same time.
     const bool listed = a.items != nullptr;
-    const int row0 = listed ? a.items[4 * item] : item;
-    const int ntok = listed ? a.items[4 * item + 1] : 1;
-    const int* bt = a.block_table + static_cast<int64_t>(listed ? a.items[4 * item + 2] : item) * a.bt_width;
-    const int hi = a.positions[row0 + ntok - 1];    // last key any column of the item may see
-    const int split_size = a.plan ? a.plan[1 + a.n_items * a.n_splits + item]
+    const int row0 = listed ? listed_int(a.items + 4 * item) : item;
+    const int ntok = listed ? listed_int(a.items + 4 * item + 1) : 1;
+    const int* bt = a.block_table + static_cast<int64_t>(listed ? listed_int(a.items + 4 * item + 2) : item) * a.bt_width;
+    const int hi = listed_int(a.positions + row0 + ntok - 1);    // last key any column of the item may see
+    const int split_size = a.plan ? listed_int(a.plan + 1 + a.n_items * a.n_splits + item)
                            : (a.live_context && a.n_splits > 1)
-                               ? live_split_size(uniform(*a.live_context), a.n_splits, a.split_size) : a.split_size;
+                               ? live_split_size(listed_int(a.live_context), a.n_splits, a.split_size) : a.split_size;
     int split_end = 0;                              // set once hi has arrived
 
     // this lane's column: a token of the item and a head of the group
@@ -366,7 +373,7 @@ __device__ __forceinline__ void attn_mfma_workgroup(const MfmaArgs& a, const int
     const int pos_c = col_ok ? a.positions[col_row] : -1;
     const int lo_c = low_key(a.window, a.chunk, pos_c);
     // lowest key any column needs (the first token's window)
-    const int pos_first = a.positions[row0];
+    const int pos_first = listed_int(a.positions + row0);
     const int lo_item = low_key(a.window, a.chunk, pos_first);
     const int split_begin = splits_from(a.chunk, lo_item) + split * split_size;
 
@@ -452,7 +459,7 @@ __device__ __forceinline__ void attn_mfma_workgroup(const MfmaArgs& a, const int
         // where key and value go, for the steps to come: asked for now, written when the walk over the keys is over
         int pi, slot;
         page_of(hi, a.page_size, a.page_shift, pi, slot);
-        own_page = pi < a.bt_width ? bt[pi] : -1;
+        own_page = pi < a.bt_width ? listed_int(bt + pi) : -1;
     };
     // FUSED: the first wavefront of the split that holds the token writes its key and value to their page
     auto store_own = [&]() {
@@ -516,7 +523,7 @@ __device__ __forceinline__ void attn_mfma_workgroup(const MfmaArgs& a, const int
         for (int t = 0; t < 2; ++t) {
             int pi, slot0;
             page_of(b * BLOCK_KEYS + 16 * t, a.page_size, a.page_shift, pi, slot0);
-            p.page[t] = bt[min(pi, a.bt_width - 1)];
+            p.page[t] = listed_int(bt + min(pi, a.bt_width - 1));
         }
         return p;
     };
@@ -1410,8 +1417,9 @@ __global__ __launch_bounds__(NW* PULSE_WAVE) __attribute__((amdgpu_waves_per_eu(
 #if PULSE_BESIDE
 // A step's decoded tokens and its prompt portions in one launch, the decoded tokens' workgroups first: they wait for memory while
 // the portions' compute, and both leave compute units idle when alone.  (Head sizes whose portions leave two workgroups a unit.)
-// 24 tokens at contexts of 200 to 1,300 beside a portion of 333, 8 kv heads of 4, in a step: 31.5 + 15.8 us -> 38.5; with the
-// tokens' keys cut in two or three 36.4 + 4.7 and 36.1 + 5.6 for their merge.
+// Two launches -> one, us, 8 kv heads of 4, heads of 128 / 64 / 32 channels: 24 tokens at contexts of 1,000 beside a portion of 512
+// 47.4 / 32.3 / 28.1 -> 35.8 / 19.6 / 16.5, 64 at 3,000 beside 40 152 / 83.0 / 49.6 -> 144 / 75.0 / 44.6; 0.57 to 0.95 times over 8 to 128
+// tokens, contexts of 200 to 3,000 and portions of 40 to 512.  With the tokens' keys cut in two or three and a merge behind: no gain.
 template <int CT, int KT, int NW>
 __global__ __launch_bounds__(NW* PULSE_WAVE) PULSE_ATTN_WAVES_PER_EU void attn_beside_kernel(MfmaArgs tokens, MfmaArgs portions, int per,
                                                                                             int token_blocks, int items, int heads) {
