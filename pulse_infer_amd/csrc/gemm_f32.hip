@@ -445,7 +445,7 @@ static int gemm_f32(const void* A, int a_dtype, const void* W, int w_dtype, void
                      reinterpret_cast<uintptr_t>(W) % (4 * w_size) == 0;
     if (a_size == 4 && w_size == 4 && vec && pulse_split_takes(N, K)) {
         pulse_split_launch(static_cast<const float*>(A), static_cast<const float*>(W), C, a.c_bf16 != 0, wide, M, N, K, lda, ldw, ldc,
-                           ldw < (1 << 25) ? scratch : nullptr, -1, stream);
+                           ldw < (1 << 25) ? scratch : nullptr, stream);
         PULSE_LAUNCH_CHECK("gemm_f32");
         return 0;
     }

@@ -8,6 +8,6 @@ bool pulse_split_takes(int N, int K);
 // How many bytes of scratch the fastest way for these sizes takes (0: none).
 int64_t pulse_split_scratch(int M, int N, int K);
 
-// Operands that are read four values at a time; `scratch` null: the way that takes none; `way`: -1, or one by its number.
+// Operands that are read four values at a time; `scratch` null: a way that takes none.
 void pulse_split_launch(const float* A, const float* W, void* C, bool c_bf16, bool c_wide, int M, int N, int K, int64_t lda, int64_t ldw,
-                        int64_t ldc, void* scratch, int way, hipStream_t stream);
+                        int64_t ldc, void* scratch, hipStream_t stream);

@@ -2,8 +2,8 @@
 // (reference: cublasSgemm, src/ops/kernels/cuda/matmul_kernel.cu:70-88)
 //
 // A float32 value is the sum of three bfloat16 parts, exactly: the value rounded, what that leaves rounded, the rest (8 + 8 + 8
-// bits).  Of the nine products of two values' parts the six largest are made (second x second and third x third and the like
-// below: at most 2^-26 of the product are left out, a quarter of a float32 rounding), each exact, on v_mfma_f32_16x16x32_bf16
+// bits).  Of the nine products of two values' parts the six largest are made (second x third, third x second and third x third are
+// not: at most 2^-26 of the product are left out, a quarter of a float32 rounding), each exact, on v_mfma_f32_16x16x32_bf16
 // with float32 sums.  That instruction does sixteen times the arithmetic of v_mfma_f32_16x16x4_f32, so six of it take 3/8 of the
 // time.  Error against 64 bits, relative, normal operands, K of 2,048 / 8,192: 2.4e-7 / 5.1e-7, the float32 instruction with
 // four shares of K 4.1e-7 / 8.1e-7; largest difference over the result's root mean square 1.7e-6 / 3.1e-6 against 3.3e-6 /
@@ -13,26 +13,32 @@
 // product after product as `w_part` and `x_part` say, and the shares in their order.  The cut depends on K alone and every way
 // below does the same, so a row's result does not depend on what else is in the batch, bit for bit.
 //
-// Range: parts are as exact as said for rows (of a share) whose largest value is at least 2^-100 and below 2^60, or that are
-// zeros.  Any other row, one with an infinity or NaN among them, is flagged, and results of flagged rows are made anew on the
-// float32 instruction (`replace_flagged`): products of parts would overflow, or make a NaN of an infinity times zero.
+// Range: so exact for rows (of a share) whose largest value is at least 2^-100 and below 2^60, or that are zeros.  Any other row,
+// one with an infinity or NaN among them, is flagged, and results of flagged rows are made anew on the float32 instruction
+// (`replace_flagged`): products of parts would overflow, or make a NaN of an infinity times zero.  In a row that is not flagged what is
+// lost of a value is below 2^-126: a value below 2^-110 loses of its third part, which shows only where every larger value of
+// the row meets a zero (values of 2^-110 / 2^-115 / 2^-118 alone: 2.9e-7 / 4.9e-7 / 3.1e-6, the float32 instruction 4.1e-7).
 //
-// Ways: few rows straight from memory into registers (gemm_split_rows_kernel); from there on X is taken apart once
-// (gemm_split_prepare_kernel) and multiplied in tiles of up to 96 x 256, whose wavefronts take the weights apart as they go
-// (gemm_split_tile_kernel), K in one go or its shares over workgroups, added up by gemm_split_sum_kernel.
+// Ways: up to some hundreds of rows both operands are taken apart as they go (gemm_split_staged_kernel); from there on X once
+// (gemm_split_prepare_kernel), multiplied in tiles of 64 or 96 x 256 whose wavefronts take the weights apart
+// (gemm_split_tile_kernel), K in one go or its shares over workgroups, added up by gemm_split_sum_kernel.  `way_for` chooses.
 // What bounds the tiles: 333 x 16,384 x 2,048 takes 125 us, its matrix instructions alone 91 (the power limit: 1.47 PFLOP/s);
 // the difference is the issue of the weights' arithmetic, 104 instructions a wavefront and block beside 72 products.  Two
-// wavefronts a SIMD are what hides it: with one, 160 us.  Taking X apart in the tiles, as its weights, 146 to 160.
-// Measured, weight rows x K, us, float32 instruction -> parts:
-//                        12 rows       32           64           97           200           333           1,024
-//   16,384 x 2,048       54 -> 50      56 -> 56     62 -> 71     84 -> 81     155 -> 100    237 -> 123    602 -> 340
-//   3,072 x 2,048        13 -> 14      18 -> 17     19 -> 22     26 -> 29     35 -> 41      60 -> 48
-//   2,048 x 8,192        38 -> 37      64 -> 40     62 -> 43     55 -> 48     83 -> 65      110 -> 79     264 -> 205
-// (At 40 to 200 rows the smallest of these lose by the two kernels beside the tiles what the others of a layer gain; a choice by
-// the rows would make a row's sums depend on the batch.)
+// wavefronts a SIMD are what hides it: with one, 160 us.  Taking X apart in the tiles, as its weights, 146 to 160.  What bounds the
+// staged way: the weights' way from memory up to 32 rows (5.3 TB/s at 16,384 x 2,048), the issue of that arithmetic beyond.
+// Measured, weight rows x K from memory, us, float32 instruction -> parts:
+//                     1 row         12 rows       24            64            97            200           333           1,024
+//   16,384 x 2,048    28 -> 25      30 -> 26      31 -> 29      44 -> 39      77 -> 66      144 -> 96     203 -> 123    584 -> 346
+//   3,072 x 2,048     7.8 -> 8.3    10.0 -> 8.9   14.4 -> 11.2  14.8 -> 14.3  22 -> 22      30 -> 27      58 -> 42      110 -> 87
+//   2,048 x 8,192     21 -> 23      30 -> 25      49 -> 25      50 -> 34      45 -> 42      76 -> 57      106 -> 73     270 -> 200
+//   12,288 x 4,096    40 -> 36      52 -> 38      56 -> 50      74 -> 61      126 -> 96     209 -> 155    324 -> 198    828 -> 532
+//   6,144 x 1,024     8.9 -> 8.8    11.4 -> 9.8   9.4 -> 10.1   14.2 -> 14.9  22 -> 21      33 -> 33      49 -> 47      122 -> 99
+// (Read straight into registers by eight wavefronts a workgroup, up to 64 rows took 1.1 to 1.4 times the float32 instruction's time,
+// and tiles at 40 to 200 rows of the smallest weights 1.1 to 1.7 times, by the two kernels beside them.)
 #include "gemm_split.h"
 #include "tile_loop.h"
 #include <algorithm>
+#include <cmath>
 
 namespace {
 
@@ -410,105 +416,145 @@ void launch_tile(SplitArgs a, hipStream_t stream) {
     hipLaunchKernelGGL((gemm_split_tile_kernel<TM, ALL>), dim3(grid), dim3(TILE_WAVES * PULSE_WAVE), 0, stream, a);
 }
 
-// Few rows, where the weights' way from memory is the time: a workgroup has 16 * BM rows of X and 16 * BN weight rows, its
-// wavefronts a share of K each, straight from memory into registers, U blocks a set, the next set on its way.
-template <int BM, int BN, int U>
-__global__ __launch_bounds__(SHARES* PULSE_WAVE) void gemm_split_rows_kernel(SplitArgs a) {
-    constexpr int T = BM + BN;
-    __shared__ f32x4 meet[SHARES][BN * BM][PULSE_WAVE];
-    const int n0 = blockIdx.x * (16 * BN), m0 = blockIdx.y * (16 * BM);
+// Up to some hundreds of rows, without anything made of X before: a workgroup has 16 * BM rows of X and 16 * BN weight rows, its
+// WAVES wavefronts a share or two of K each.  A wavefront copies its own blocks (128 bytes of eight rows an instruction: read
+// straight into registers, the lanes that are served together touch sixteen rows) into two stages of its own, reads the next block
+// while this one is multiplied, and takes both operands apart; no barrier until the shares meet.
+template <int BM, int BN, int WAVES>
+__global__ __launch_bounds__(WAVES* PULSE_WAVE) void gemm_split_staged_kernel(SplitArgs a) {
+    constexpr int S = 2, T = BM + BN, TILES = BM * BN, STAGE = T * 2048, PER = SHARES / WAVES;
+    constexpr int RING = WAVES * S * STAGE, MEET = SHARES * TILES * PULSE_WAVE * 16;
+    __shared__ __attribute__((aligned(1024))) char lds[RING > MEET ? RING : MEET];
+
+    // (the workgroups of a die, every eighth, take neighbouring tiles: those of one span of weight rows)
+    const int total = a.tiles_m * a.tiles_n;
+    const int per_die = (total + 7) / 8;
+    const int tile = (blockIdx.x % 8) * per_die + blockIdx.x / 8;
+    if (static_cast<int>(blockIdx.x / 8) >= per_die || tile >= total) return;
+    const int m0 = tile % a.tiles_m * (16 * BM), n0 = tile / a.tiles_m * (16 * BN);
+
     const int lane = threadIdx.x % PULSE_WAVE;
-    const int share = __builtin_amdgcn_readfirstlane(threadIdx.x / PULSE_WAVE);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / PULSE_WAVE);
     const int r = lane % 16, kg = lane / 16;
-    const int blocks = (a.K + KB - 1) / KB;
-    const int b0 = share > 0 ? share_end(blocks, share - 1) : 0, b_end = share_end(blocks, share);
+    const int blocks = (a.K + KB - 1) / KB, s0 = wave * PER;
+    const int first = s0 > 0 ? share_end(blocks, s0 - 1) : 0, last = share_end(blocks, s0 + PER - 1);
 
-    // (rows past the end are the last row again: their results are not written)
-    const float* row[T];
+    // Copies: half h of tile t is its rows 8 h .. 8 h + 7, 128 bytes each; piece c of row q sits at place c ^ (q % 8).  (Rows past
+    // the end are the last row again, their results are not written; a piece behind K is the row's last, and zeros once read.)
+    const int crow = lane / 8, cpiece = (lane % 8) ^ crow;
+    const float* from[T][2];
 #pragma unroll
-    for (int j = 0; j < BN; ++j) row[j] = a.W + static_cast<int64_t>(min(n0 + 16 * j + r, a.N - 1)) * a.ldw;
+    for (int h = 0; h < 2; ++h) {
 #pragma unroll
-    for (int i = 0; i < BM; ++i) row[BN + i] = a.A + static_cast<int64_t>(min(m0 + 16 * i + r, a.M - 1)) * a.lda;
-
-    f32x4 acc[BN][BM];
-    uint32_t most[T];
+        for (int j = 0; j < BN; ++j) from[j][h] = a.W + static_cast<int64_t>(min(n0 + 16 * j + 8 * h + crow, a.N - 1)) * a.ldw;
 #pragma unroll
-    for (int j = 0; j < BN; ++j)
+        for (int i = 0; i < BM; ++i) from[BN + i][h] = a.A + static_cast<int64_t>(min(m0 + 16 * i + 8 * h + crow, a.M - 1)) * a.lda;
+    }
+    char* const mine = lds + wave * S * STAGE;
+    const uint32_t mine_at = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((void __attribute__((address_space(3)))*)(mine)));
+    auto copy = [&](int block, int stage) __attribute__((always_inline)) {
+        const int at = min(min(block, last - 1) * KB + 4 * cpiece, a.K - 4);
+        const uint32_t to = __builtin_amdgcn_readfirstlane(mine_at + stage * STAGE);
 #pragma unroll
-        for (int i = 0; i < BM; ++i) acc[j][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int t = 0; t < T; ++t)
 #pragma unroll
-    for (int j = 0; j < T; ++j) most[j] = 0;
-
-    f32x4 raw[2][U][T][2];       // values 8 kg .. of a block
-    auto fetch = [&](int set, int block) __attribute__((always_inline)) {
+            for (int h = 0; h < 2; ++h) load_to_lds(from[t][h] + at, to + t * 2048 + h * 1024);
+    };
+    f32x4 raw[T][2];             // values 8 kg .. of a block
+    auto read = [&](int stage) __attribute__((always_inline)) {
 #pragma unroll
-        for (int u = 0; u < U; ++u)
+        for (int t = 0; t < T; ++t)
 #pragma unroll
             for (int q = 0; q < 2; ++q)
-#pragma unroll
-                for (int j = 0; j < T; ++j) raw[set][u][j][q] = load4(row[j], (block + u) * KB + 8 * kg + 4 * q, a.K);
-        __builtin_amdgcn_sched_barrier(0);   // (the loads stay ahead of the products that they hide behind)
+                raw[t][q] = *reinterpret_cast<const f32x4*>(mine + stage * STAGE + t * 2048 + r * 128 + ((2 * kg + q) ^ (r % 8)) * 16);
     };
-    auto multiply = [&](int set, int block) __attribute__((always_inline)) {
+
+    f32x4 acc[PER][BN][BM];
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            if (block + u >= b_end) continue;
-            if ((block + u + 1) * KB > a.K) {                    // behind K: zeros
+    for (int p = 0; p < PER; ++p)
+#pragma unroll
+        for (int j = 0; j < BN; ++j)
+#pragma unroll
+            for (int i = 0; i < BM; ++i) acc[p][j][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    int stage = 0;               // of block b
+    if (first < last) {
+#pragma unroll
+        for (int s = 0; s < S; ++s) copy(first + s, s);
+        asm volatile("s_waitcnt vmcnt(%0)" : : "n"((S - 1) * T * 2) : "memory");
+        read(0);
+    }
+#pragma unroll
+    for (int p = 0; p < PER; ++p) {
+        const int b0 = s0 + p > 0 ? share_end(blocks, s0 + p - 1) : 0, b_end = share_end(blocks, s0 + p);
+        uint32_t most[T];
+#pragma unroll
+        for (int t = 0; t < T; ++t) most[t] = 0;
+        for (int b = b0; b < b_end; ++b) {
+            if ((b + 1) * KB > a.K) {                                // behind K: zeros
 #pragma unroll
                 for (int q = 0; q < 2; ++q)
-                    if ((block + u) * KB + 8 * kg + 4 * q >= a.K) {
+                    if (b * KB + 8 * kg + 4 * q >= a.K) {
 #pragma unroll
-                        for (int j = 0; j < T; ++j) raw[set][u][j][q] = f32x4{0.f, 0.f, 0.f, 0.f};
+                        for (int t = 0; t < T; ++t) raw[t][q] = f32x4{0.f, 0.f, 0.f, 0.f};
                     }
             }
             tile_bf16x8 parts[T][3];
 #pragma unroll
-            for (int j = 0; j < T; ++j) {
+            for (int t = 0; t < T; ++t) {
                 uint32_t v[3][4];
-                each<SPLIT_STEPS>([&](auto n) __attribute__((always_inline)) { split_step<decltype(n)::value>(raw[set][u][j], v, most[j]); });
+                each<SPLIT_STEPS>([&](auto n) __attribute__((always_inline)) { split_step<decltype(n)::value>(raw[t], v, most[t]); });
 #pragma unroll
-                for (int p = 0; p < 3; ++p) parts[j][p] = __builtin_bit_cast(tile_bf16x8, uint4{v[p][0], v[p][1], v[p][2], v[p][3]});
+                for (int x = 0; x < 3; ++x) parts[t][x] = __builtin_bit_cast(tile_bf16x8, uint4{v[x][0], v[x][1], v[x][2], v[x][3]});
             }
+            // this block's values are in registers, so its stage is free; the next block's copies have landed
+            asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");
+            copy(b + S, stage);
+            asm volatile("s_waitcnt vmcnt(%0)" : : "n"((S - 1) * T * 2) : "memory");
+            stage = stage == S - 1 ? 0 : stage + 1;
+            read(stage);
 #pragma unroll
-            for (int q = 0; q < 6; ++q)
+            for (int i = 0; i < BM; ++i)
 #pragma unroll
-                for (int j = 0; j < BN; ++j)
+                for (int q = 0; q < 6; ++q)
 #pragma unroll
-                    for (int i = 0; i < BM; ++i)
-                        acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(parts[j][w_part(q)], parts[BN + i][x_part(q)], acc[j][i], 0, 0, 0);
+                    for (int j = 0; j < BN; ++j)
+                        acc[p][j][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(parts[j][w_part(q)], parts[BN + i][x_part(q)], acc[p][j][i], 0, 0, 0);
         }
-        __builtin_amdgcn_sched_barrier(0);
-    };
-    fetch(0, b0);
-    for (int b = b0; b < b_end; b += 2 * U) {
-        fetch(1, b + U);
-        multiply(0, b);
-        fetch(0, b + 2 * U);
-        multiply(1, b + U);
+        uint32_t bad[T], any = 0;
+#pragma unroll
+        for (int t = 0; t < T; ++t) {
+            uint32_t top = max(most[t] & 0xffffu, most[t] >> 16);
+            top = max(top, static_cast<uint32_t>(__shfl_xor(top, 16)));
+            top = max(top, static_cast<uint32_t>(__shfl_xor(top, 32)));
+            any |= bad[t] = static_cast<uint32_t>(__ballot(outside(top))) & 0xffffu;
+        }
+        if (any != 0) {
+#pragma unroll
+            for (int j = 0; j < BN; ++j)
+#pragma unroll
+                for (int i = 0; i < BM; ++i)
+                    if ((bad[j] | bad[BN + i]) != 0)
+                        replace_flagged(acc[p][j][i], bad[j], bad[BN + i], a.A + static_cast<int64_t>(min(m0 + 16 * i + r, a.M - 1)) * a.lda,
+                                        a.W + static_cast<int64_t>(min(n0 + 16 * j + r, a.N - 1)) * a.ldw, b0 * KB, min(b_end * KB, a.K), lane);
+        }
     }
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" : : : "memory");   // the last copies, which nobody reads, must not land in what follows
+    __syncthreads();
 
-    uint32_t bad[T];
+    f32x4* const meet = reinterpret_cast<f32x4*>(lds);              // [SHARES][TILES][64]
 #pragma unroll
-    for (int j = 0; j < T; ++j) {
-        u16x2 top = __builtin_bit_cast(u16x2, most[j]);
+    for (int p = 0; p < PER; ++p)
 #pragma unroll
-        for (int x = 16; x <= 32; x *= 2) top = __builtin_elementwise_max(top, __builtin_bit_cast(u16x2, __shfl_xor(__builtin_bit_cast(uint32_t, top), x)));
-        bad[j] = static_cast<uint32_t>(__ballot(outside(__builtin_bit_cast(uint32_t, top)))) & 0xffffu;
-    }
+        for (int j = 0; j < BN; ++j)
 #pragma unroll
-    for (int j = 0; j < BN; ++j)
-#pragma unroll
-        for (int i = 0; i < BM; ++i) {
-            if ((bad[j] | bad[BN + i]) != 0) replace_flagged(acc[j][i], bad[j], bad[BN + i], row[BN + i], row[j], b0 * KB, min(b_end * KB, a.K), lane);
-            meet[share][j * BM + i][lane] = acc[j][i];
-        }
+            for (int i = 0; i < BM; ++i) meet[((s0 + p) * TILES + j * BM + i) * PULSE_WAVE + lane] = acc[p][j][i];
     __syncthreads();
 #pragma unroll
-    for (int t = 0; t < BN * BM; ++t) {
-        if (t % SHARES != share) continue;
-        f32x4 v = meet[0][t][lane];
+    for (int t = 0; t < TILES; ++t) {
+        if (t % WAVES != wave) continue;
+        f32x4 v = meet[t * PULSE_WAVE + lane];
 #pragma unroll
-        for (int s = 1; s < SHARES; ++s) v += meet[s][t][lane];
+        for (int s = 1; s < SHARES; ++s) v += meet[(s * TILES + t) * PULSE_WAVE + lane];
         store_four(a, static_cast<char*>(a.C), m0 + 16 * (t % BM) + r, n0 + 16 * (t / BM) + 4 * kg, v);
     }
 }
@@ -523,115 +569,152 @@ __global__ __launch_bounds__(256) void gemm_split_sum_kernel(const float* parts,
     store_four(a, static_cast<char*>(a.C), static_cast<int>(at / a.N), static_cast<int>(at % a.N), v);
 }
 
-template <int BM, int BN, int U>
-void launch_rows(const SplitArgs& a, hipStream_t stream) {
-    hipLaunchKernelGGL((gemm_split_rows_kernel<BM, BN, U>), dim3((a.N + 16 * BN - 1) / (16 * BN), (a.M + 16 * BM - 1) / (16 * BM)),
-                       dim3(SHARES * PULSE_WAVE), 0, stream, a);
+template <int BM, int BN, int WAVES>
+void launch_staged(SplitArgs a, hipStream_t stream) {
+    a.tiles_m = (a.M + 16 * BM - 1) / (16 * BM);
+    a.tiles_n = (a.N + 16 * BN - 1) / (16 * BN);
+    const unsigned grid = static_cast<unsigned>((static_cast<int64_t>(a.tiles_m) * a.tiles_n + 7) / 8 * 8);
+    hipLaunchKernelGGL((gemm_split_staged_kernel<BM, BN, WAVES>), dim3(grid), dim3(WAVES * PULSE_WAVE), 0, stream, a);
 }
 
-struct Way { int tiles, groups; double block; };    // tiles of 16 rows a workgroup, workgroups that share K, ns a block of k
-constexpr Way WAYS[] = {{6, 1, 1900.}, {4, 1, 1450.}, {2, 1, 1050.}, {6, 8, 1900.}, {4, 8, 1450.}, {2, 8, 1050.},
-                        {6, 4, 1900.}, {4, 4, 1450.}, {2, 4, 1050.}};
 constexpr int CHUNK = 2016;                          // rows whose parts are in scratch at a time
 constexpr int64_t RESULTS_AT_MOST = 128ll << 20;     // bytes of the shares' results
 
 int64_t parts_bytes(int M, int K) { return static_cast<int64_t>((M + 15) / 16) * ((K + KB - 1) / KB) * 3072; }
 int64_t flags_bytes(int M) { return (static_cast<int64_t>((M + 15) / 16) * 16 * SHARES + 255) / 256 * 256; }
 
-// The tiles of the least estimated time: rounds of workgroups x blocks of k (three more for a workgroup's start) x the time of
-// one, as measured with the chip full; shares over workgroups cost the second kernel and their results' way to memory and back.
-int way_for(int M, int N, int K) {
-    const int64_t units = pulse_compute_units(), blocks = (K + KB - 1) / KB;
+// The ways, of the least estimated time.  All give the same bits, so the choice is free; its figures are fitted to 6,900 times of 14 weights
+// (128 to 12,288 long, 2,048 to 151,936 of them) at 1 to 1,024 rows, weights from memory: the way it takes is 1 % slower than
+// the best one on average, 19 % at most, and 0.80 times the float32 instruction's time on average (slower by more than 3 % at 12 of
+// 425 sizes, most at 49,152 x 128; 2,048 x 8,192 at one row 20.8 -> 23.3 us, 6,144 x 1,024 at 17 to 64 rows by 5 %).
+// A block of k takes a lone workgroup `alone` us and a unit that is full of its kind `full` us for each SIMD's wavefront; `rate`:
+// bytes a ps from memory.
+struct Staged { int bm, bn, waves; double alone, full, rate; };
+constexpr Staged STAGED[] = {{1, 1, 8, 0.40, 0.30, 5.82}, {1, 2, 4, 0.42, 0.47, 5.75}, {1, 2, 8, 0.49, 0.44, 5.24}, {2, 1, 8, 0.44, 0.44, 4.51},
+                             {2, 2, 8, 0.62, 0.60, 4.70}, {2, 2, 4, 0.50, 0.60, 5.09}, {2, 4, 4, 0.75, 0.89, 5.20}, {3, 2, 4, 0.59, 0.78, 4.63},
+                             {3, 4, 4, 0.95, 1.09, 4.99}, {4, 4, 4, 1.16, 1.27, 4.67}};
+constexpr int STAGED_WAYS = sizeof(STAGED) / sizeof(STAGED[0]);
+// Tiles of 96 or 64 rows by 256 weight rows, `groups` workgroups that share K.
+struct Tiled { int tiles, groups; double block; };
+constexpr Tiled TILED[] = {{6, 1, 1.29}, {4, 1, 1.06}, {6, 8, 1.29}, {4, 8, 1.06}, {6, 4, 1.29}, {4, 4, 1.06}};
+constexpr int TILED_WAYS = sizeof(TILED) / sizeof(TILED[0]);
+
+double larger_of(double a, double b, double c) {     // (a little more than the largest where others come near)
+    a *= a; b *= b; c *= c;
+    return std::sqrt(std::sqrt(a * a + b * b + c * c));
+}
+
+double staged_us(const Staged& w, int M, int N, int K, double bytes, int units) {
+    const int64_t wgs = static_cast<int64_t>((M + 16 * w.bm - 1) / (16 * w.bm)) * ((N + 16 * w.bn - 1) / (16 * w.bn));
+    const int64_t a_unit = (wgs + units - 1) / units;
+    const int lds = std::max(w.waves * 2 * (w.bm + w.bn) * 2048, SHARES * w.bm * w.bn * 1024);
+    const int together = std::min(160 * 1024 / lds, 16 / w.waves);
+    const double walk = (K + KB - 1) / KB / static_cast<double>(w.waves);
+    return 2.1 + larger_of(a_unit * walk * w.waves / 4 * w.full, (a_unit + together - 1) / together * (walk + 7.6) * w.alone, bytes / (w.rate * 1e6));
+}
+
+double tiled_us(const Tiled& w, int M, int N, int K, double bytes, int units) {
+    const int64_t blocks = (K + KB - 1) / KB;
+    const int64_t wgs = static_cast<int64_t>((M + 16 * w.tiles - 1) / (16 * w.tiles)) * ((N + TILE_N - 1) / TILE_N) * w.groups;
+    double us = larger_of((wgs + units - 1) / units * ((blocks + w.groups - 1) / w.groups + 4.0) * w.block, bytes / 4.05e6, 0.);
+    if (w.groups > 1) us += 2. * M * N * SHARES * 4 / 6.07e6;
+    return us + 8.7 + M * (K * 4.) / 1.28e6;
+}
+
+// The number of a staged way, or STAGED_WAYS + that of tiles (`scratch`: they may be chosen; `results`: so may shares over workgroups).
+int way_for(int M, int N, int K, bool scratch, bool results) {
+    const double bytes = 4. * (static_cast<double>(N) * K + static_cast<double>(M) * K + static_cast<double>(M) * N);
+    const int units = pulse_compute_units();
     int best = 0;
-    double least = 0.0;
-    for (int i = 0; i < 9; ++i) {
-        const Way& w = WAYS[i];
-        const int64_t results = static_cast<int64_t>(M) * N * SHARES * 4;
-        if (w.groups > 1 && (blocks < 2 * SHARES || N % 4 != 0 || results > RESULTS_AT_MOST)) continue;
-        const int64_t wgs = static_cast<int64_t>((M + 16 * w.tiles - 1) / (16 * w.tiles)) * ((N + TILE_N - 1) / TILE_N) * w.groups;
-        double cost = ((wgs + units - 1) / units) * ((blocks + w.groups - 1) / w.groups + 3) * w.block;
-        if (w.groups > 1) cost += 3000. + 2 * results / 4500.;
-        if (i == 0 || cost < least) { best = i; least = cost; }
+    double least = 0.;
+    for (int i = 0; i < STAGED_WAYS; ++i) {
+        if (i > 0 && STAGED[i].bm > std::max(1, (M + 15) / 16)) continue;
+        const double us = staged_us(STAGED[i], M, N, K, bytes, units);
+        if (i == 0 || us < least) { best = i; least = us; }
+    }
+    if (!scratch || M <= 16 || parts_bytes(M, K) >= (1ll << 32)) return best;
+    for (int i = 0; i < TILED_WAYS; ++i) {
+        if (TILED[i].groups > 1 && (!results || (K + KB - 1) / KB < 2 * SHARES || N % 4 != 0 ||
+                                    static_cast<int64_t>(M) * N * SHARES * 4 > RESULTS_AT_MOST)) continue;
+        const double us = tiled_us(TILED[i], M, N, K, bytes, units);
+        if (us < least) { best = STAGED_WAYS + i; least = us; }
     }
     return best;
 }
 
-// Few rows, whose weights go straight into registers: always up to 16; up to 32 of a weight of many rows (16,384 x 2,048 at 32
-// rows 56 us, tiles 65); more where the workgroups of 32 rows by 16 or 32 weight rows find a compute unit each and K is short
-// (3,072 x 2,048 at 64 rows 22 us, tiles 25; but 2,048 x 8,192 52 us, tiles 43).
-// Weight rows a workgroup (in sixteens) of this way, or 0: tiles.
-int rows_way_for(int M, int N, int K) {
-    const int64_t units = pulse_compute_units();
-    if (M <= 16) return N >= 64 * units ? 4 : 1;
-    if (M <= 32 && N >= 64 * units) return 4;
-    if (K >= 4096) return 0;
-    for (int bn = 1; bn <= 2; ++bn)
-        if (static_cast<int64_t>((M + 31) / 32) * ((N + 16 * bn - 1) / (16 * bn)) <= units) return bn;
-    return 0;
+void launch_staged_way(int way, const SplitArgs& a, hipStream_t stream) {
+    switch (way) {
+        case 0: launch_staged<1, 1, 8>(a, stream); break;
+        case 1: launch_staged<1, 2, 4>(a, stream); break;
+        case 2: launch_staged<1, 2, 8>(a, stream); break;
+        case 3: launch_staged<2, 1, 8>(a, stream); break;
+        case 4: launch_staged<2, 2, 8>(a, stream); break;
+        case 5: launch_staged<2, 2, 4>(a, stream); break;
+        case 6: launch_staged<2, 4, 4>(a, stream); break;
+        case 7: launch_staged<3, 2, 4>(a, stream); break;
+        case 8: launch_staged<3, 4, 4>(a, stream); break;
+        default: launch_staged<4, 4, 4>(a, stream); break;
+    }
 }
 
 }  // namespace
 
 // A rule of the weight alone, so that a row's sums do not depend on the batch.  Smaller products than this stay with the float32
-// instruction: the kernels beside the tiles cost what the tiles gain (2,048 x 2,048 at 97 / 333 rows 18 / 33 us there, 22 / 35
-// here; 1,024 x 512 at 300 rows 11 against 14; 3,072 x 2,048, the first that is made here, 26 against 29 and 60 against 48).
+// instruction: those of a few hundred thousand values gain nothing (1,024 x 512 at 512 / 1,024 rows 8.3 / 13.0 us there, 9.3 / 13.6
+// here), and between them and this line little (2,048 x 2,048 at 12 / 97 / 200 / 333 rows 9.9 / 14.0 / 22.1 / 30.2 and 8.4 / 14.1 / 21.5 /
+// 26.5), so that the line has stayed where tiles alone begin to pay (3,072 x 2,048 at 333 rows 58 and 45).
 bool pulse_split_takes(int N, int K) { return static_cast<int64_t>(N) * K >= 6ll << 20; }
 
 int64_t pulse_split_scratch(int M, int N, int K) {
     if (!pulse_split_takes(N, K)) return 0;
     M = M < CHUNK ? M : CHUNK;
-    if (rows_way_for(M, N, K) != 0 || parts_bytes(M, K) >= (1ll << 32)) return 0;
-    return parts_bytes(M, K) + flags_bytes(M) + (WAYS[way_for(M, N, K)].groups > 1 ? static_cast<int64_t>(SHARES) * M * N * 4 : 0);
+    const int way = way_for(M, N, K, true, true) - STAGED_WAYS;
+    if (way < 0) return 0;
+    return parts_bytes(M, K) + flags_bytes(M) + (TILED[way].groups > 1 ? static_cast<int64_t>(SHARES) * M * N * 4 : 0);
 }
 
 void pulse_split_launch(const float* A, const float* W, void* C, bool c_bf16, bool c_wide, int M, int N, int K, int64_t lda, int64_t ldw,
-                        int64_t ldc, void* scratch, int way, hipStream_t stream) {
+                        int64_t ldc, void* scratch, hipStream_t stream) {
     SplitArgs a{A, W, C, c_bf16 ? 1 : 0, c_wide ? 1 : 0, M, N, K, lda, ldw, ldc, 0, 0, 1, 0, nullptr, nullptr};
-    if (scratch == nullptr || (way < 0 && pulse_split_scratch(M, N, K) == 0)) {
-        const int bn = rows_way_for(M, N, K);
-        if (M <= 16) {
-            if (bn == 4) launch_rows<1, 4, 1>(a, stream);
-            else if (K >= 4096) launch_rows<1, 1, 4>(a, stream);    // (2,048 x 8,192 at 12 rows 37 us against 40 with two blocks a set,
-            else launch_rows<1, 1, 2>(a, stream);                   //  3,072 x 2,048 14.7 against 13.6)
-        } else if (bn == 4) {
-            launch_rows<2, 4, 1>(a, stream);
-        } else if (bn == 2) {
-            launch_rows<2, 2, 1>(a, stream);
-        } else if (bn == 1) {
-            launch_rows<2, 1, 1>(a, stream);
-        } else {
-            launch_rows<4, 2, 1>(a, stream);                        // (no scratch was given)
-        }
+    const int whole = way_for(M < CHUNK ? M : CHUNK, N, K, scratch != nullptr, true);
+    if (whole < STAGED_WAYS) {
+        launch_staged_way(M <= CHUNK ? whole : way_for(M, N, K, false, false), a, stream);
         return;
     }
+    // (the scratch is that of the largest chunk: a way whose results it holds)
+    const bool results = TILED[whole - STAGED_WAYS].groups > 1;
     for (int m = 0; m < M; m += CHUNK) {
         SplitArgs c = a;
         c.M = M - m < CHUNK ? M - m : CHUNK;
         c.A = A + static_cast<int64_t>(m) * lda;
         c.C = static_cast<char*>(C) + static_cast<int64_t>(m) * ldc * (c_bf16 ? 2 : 4);
-        // (the scratch is that of the largest chunk: a way whose results it holds)
-        const int which = way >= 0 ? way : m == 0 ? way_for(c.M, N, K) : WAYS[way_for(CHUNK, N, K)].groups > 1 ? way_for(c.M, N, K) : way_for(CHUNK, N, K);
+        const int way = m == 0 ? whole : way_for(c.M, N, K, true, results);
+        if (way < STAGED_WAYS) {
+            launch_staged_way(way, c, stream);
+            continue;
+        }
+        const Tiled& w = TILED[way - STAGED_WAYS];
         char* parts = static_cast<char*>(scratch);
         uint8_t* flags = reinterpret_cast<uint8_t*>(parts + parts_bytes(c.M, K));
-        float* results = reinterpret_cast<float*>(parts + parts_bytes(c.M, K) + flags_bytes(c.M));
+        float* shares = reinterpret_cast<float*>(parts + parts_bytes(c.M, K) + flags_bytes(c.M));
         hipLaunchKernelGGL(gemm_split_prepare_kernel, dim3((c.M + 15) / 16, SHARES), dim3(PREPARE_WAVES * PULSE_WAVE), 0, stream, c, parts, flags);
         c.xparts = parts;
         c.xflags = flags;
+        if (w.groups == 1) {
+            if (w.tiles == 6) launch_tile<6, true>(c, stream);
+            else launch_tile<4, true>(c, stream);
+            continue;
+        }
         SplitArgs p = c;
-        p.C = results;
+        p.C = shares;
         p.c_bf16 = 0;
         p.c_wide = 1;
         p.ldc = N;
-        p.groups = WAYS[which].groups;
+        p.groups = w.groups;
         p.part_stride = static_cast<int64_t>(c.M) * N;
-        if (which == 0) launch_tile<6, true>(c, stream);
-        else if (which == 1) launch_tile<4, true>(c, stream);
-        else if (which == 2) launch_tile<2, true>(c, stream);
-        else if (WAYS[which].tiles == 6) launch_tile<6, false>(p, stream);
-        else if (WAYS[which].tiles == 4) launch_tile<4, false>(p, stream);
-        else launch_tile<2, false>(p, stream);
-        if (WAYS[which].groups > 1)
-            hipLaunchKernelGGL(gemm_split_sum_kernel, dim3(static_cast<unsigned>((p.part_stride / 4 + 255) / 256)), dim3(256), 0, stream,
-                               results, p.part_stride, c);
+        if (w.tiles == 6) launch_tile<6, false>(p, stream);
+        else launch_tile<4, false>(p, stream);
+        hipLaunchKernelGGL(gemm_split_sum_kernel, dim3(static_cast<unsigned>((p.part_stride / 4 + 255) / 256)), dim3(256), 0, stream,
+                           shares, p.part_stride, c);
     }
 }

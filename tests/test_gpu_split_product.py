@@ -119,3 +119,21 @@ def test_parts_are_no_less_exact_than_the_float32_instruction(k):
             want = a.to(F64) @ w.to(F64).T
             errors.append(float((out.to(F64) - want).norm() / want.norm()))
         assert errors[0] <= 0.8 * errors[1]        # (measured 0.4 to 0.6)
+
+
+# weights past the line whose rows and K end inside tiles and blocks, long and short of both
+@pytest.mark.parametrize("n,kk", [(3074, 2052), (16390, 516), (1030, 8196), (6150, 1028), (40003, 164), (4099, 4100)])
+def test_parts_of_some_rows_are_the_same_bits_whatever_the_tile(k, n, kk):
+    """Every number of rows up to some hundreds goes its own way (tiles of 16 to 64 rows by 16 to 64 weight rows, of 64 and 96 by 256,
+    with K in one go or over workgroups): each row's results are those of the largest batch, and within a float32 sum's bound."""
+    most = 200
+    a, w = rnd(most, kk, seed=11).to(DEV), rnd(n, kk, seed=12).to(DEV)
+    whole = torch.full((most, n), float("nan"), device=DEV)
+    k.gemm_f32(a, w, whole)
+    assert ((whole.to(F64) - a.to(F64) @ w.to(F64).T).abs() <= bound(a, w)).all()
+    for m in (1, 4, 15, 16, 17, 31, 32, 33, 47, 48, 49, 63, 64, 65, 96, 97, 129, 160, 161):
+        some = torch.full((m, n), float("nan"), device=DEV)
+        k.gemm_f32(a[most - m:], w, some)
+        assert torch.equal(some, whole[most - m:]), m
+        without_scratch(a[:m], w, some)
+        assert torch.equal(some, whole[:m]), m
