@@ -47,6 +47,16 @@ def check(name, args):
     def need(cond, what):
         assert cond, f"{name}: {what}"
 
+    if name == "pulse_attn_mfma_beside":  # the arguments of the tokens' entry point, and the portions beside them before the stream
+        *args, portions, n_portions, stream = args
+        it = portions.tensor.view(-1, 4)
+        need(it.shape[0] == val(n_portions) and int((it[:, 0] + it[:, 1]).max()) <= val(args[11])
+             and int(it[:, 2].max()) < args[7].tensor.shape[0], "portions")
+        name, args = "pulse_attn_mfma", [*args, stream]
+    elif name == "pulse_attn_prefill_values":  # the arguments of the portions' entry point, and the values' channels before the stream
+        *args, values, stream = args
+        need(0 < val(values) <= args[4].tensor.shape[-1], "channels of a value")
+        name, args = "pulse_attn_prefill", [*args, stream]
     if name == "pulse_qk_rope_kv":
         (qkv, _, stride, _, _, _, _, _, _, _, _, kc, vc, _, pos, ent, bt, width, tokens, nq, nkv, d, page, pages, write,
          _, vh0, _, _, _) = args
