@@ -77,8 +77,9 @@ template <> __device__ __forceinline__ bf16_t from_f32<bf16_t>(float v) { return
 // The two operands of a step of a reduction over the wavefront: what lanes i and i ^ STEP hold, the same pair (in one order or the
 // other) for both.  Steps go 32, 16, 8, 4, 2, 1; below 8 the pair is right once the steps before have been taken (lanes that
 // differ in the higher bits then hold the same).  By lane moves in the vector unit: a trip through LDS, which `__shfl_xor` takes,
-// is waited for six times a sum.  (Steps of the 8B shape, the same bits: decoding 32 requests 4,786 -> 4,744 us, one 3,265 -> 3,242,
-// 24 beside a portion of 333 tokens 8,996 -> 8,834, the norms, the attention's maxima and the sums of squares among it.)
+// is waited for six times a sum.  (The same bits.  Decoding steps of the 8B shape, the norms, the attention's maxima and the sums of
+// squares among it: 32 requests 4,790 -> 4,749 us, one 3,263 -> 3,239 where runs of one side differ by 2 us; less than runs differ by on
+// a card where that is more.)
 struct WaveTwo { uint32_t a, b; };
 template <int STEP>
 __device__ __forceinline__ WaveTwo wave_two(uint32_t v) {

@@ -662,7 +662,7 @@ void launch_staged_way(int way, const SplitArgs& a, hipStream_t stream) {
 // A rule of the weight alone, so that a row's sums do not depend on the batch.  Smaller products than this stay with the float32
 // instruction: those of a few hundred thousand values gain nothing (1,024 x 512 at 512 / 1,024 rows 8.3 / 13.0 us there, 9.3 / 13.6
 // here), and between them and this line little (2,048 x 2,048 at 12 / 97 / 200 / 333 rows 9.9 / 14.0 / 22.1 / 30.2 and 8.4 / 14.1 / 21.5 /
-// 26.5), so that the line has stayed where tiles alone begin to pay (3,072 x 2,048 at 333 rows 58 and 45).
+// 26.5), so that the line has stayed where tiles alone begin to pay (3,072 x 2,048 at 333 rows 58 and 42).
 bool pulse_split_takes(int N, int K) { return static_cast<int64_t>(N) * K >= 6ll << 20; }
 
 int64_t pulse_split_scratch(int M, int N, int K) {

@@ -2,21 +2,21 @@
 // bfloat16 operands, float32 sums on the matrix cores, on the loop of tile_loop.h.
 // (reference: cuBLAS for every product, src/ops/kernels/cuda/matmul_kernel.cu:132-154)
 //
-// What bounds it: the bytes that the fullest compute unit copies into LDS.  A unit takes in 30 to 55 bytes a nanosecond over a
-// launch, least where they are weights that come from memory, and the matrix cores are busy for 13 to 47 % of it, LDS waits
-// make 1 to 4 % (counters at 97, 357 and 509 rows; from 300 rows on the power limit comes near: 357 rows of gate + up take 57 us with
-// operands of zeros, 70 with others), so the shape and the shares of K are chosen for the least bytes
+// What bounds it: the bytes that the fullest compute unit copies into LDS.  A unit takes in 28 to 54 bytes a nanosecond over a
+// launch, least where they are weights that come from memory, and the matrix cores are busy for 13 to 46 % of it, LDS waits
+// make 1 to 6 % (counters at 97, 357 and 509 rows; from 300 rows on the power limit comes near: 357 rows of gate + up take 57 us with
+// operands of zeros, 70 to 73 with others), so the shape and the shares of K are chosen for the least bytes
 // (`plan_for`).  Measured alone with weights from memory, us, against the vendor library's product (gate and up: with its
 // pass for SwiGLU behind it) and this package's shared-out product for up to 192 rows; in brackets behind a figure, what it
 // takes inside a step, between other kernels and with the chip warm:
 //                                   97 rows              192                  357                 509
-//   gate + up, 24,576 x 4,096       39 [39]              54                   70 [72]             86 [95]
+//   gate + up, 24,576 x 4,096       43 [41]              55                   73 [70]             90 [86]
 //     library                       54                   64                   84                  96
-//   qkv, 6,144 x 4,096              19 [20]              26                   34 [34]             35 [38]
+//   qkv, 6,144 x 4,096              19 [20]              26                   33 [33]             36 [36]
 //     library                       25                   36                   41                  42
-//   o, 4,096 x 4,096, shares        12 [13]              17                   22 [24]             24 [28]
+//   o, 4,096 x 4,096, shares        13 [14]              17                   21 [22]             25 [25]
 //     library / shared out          25 / 16              37 / 21              29                  32
-//   down, 4,096 x 12,288, shares    24 [25]              33                   41 [43]             52 [62]
+//   down, 4,096 x 12,288, shares    25 [27]              31                   43 [46]             53 [52]
 //     library / shared out          44 / 34              92 / 47              52, shared [46]     59, shared [60]
 // From some 260 rows on tiles of 192 or 256 rows of X (their weights through three stages, X, which comes from L2, through
 // two where LDS holds no third) take the place of the library's: 357 rows of gate + up ran 96 us in tiles of 192 x 128.

@@ -1530,9 +1530,10 @@ extern "C" int pulse_sample(const float* logits, int rows, int vocab, int64_t ro
 // top_p share lies in some hundreds of the largest logits are chosen by these kernels; rows that do not fit (a larger k, a
 // distribution too flat for top-p alone) by three more that go by a histogram of the row, the last of which takes what does not fit
 // these either (many equal values at the edge, a k beyond half of what the segments hold) as pulse_sample does.  What a row's choice
-// is does not depend on the other rows.  Whole calls, us, before the histogram's kernels finished rows: 32,000 values, 3 / 16 / 64 rows
-// 136 / 150 / 187 -> 94 / 119 / 161; 151,936 values 208 / 241 / 327 -> 103 / 131 / 200.  Scratch, with chunks = pulse_sample_chunks(vocab): part_max, part_mass (float32), part_idx, seg_n
-// (int32) of rows * chunks entries; seg_i (int32), seg_x (float32) of rows * chunks * pulse_sample_segment()
+// is does not depend on the other rows.  Whole steps of rows with
+// mixed options, the host's part among it, us, before the histogram's kernels finished rows: 32,000 values, 3 / 16 / 64 rows
+// 139 / 155 / 191 -> 93 / 119 / 162; 151,936 values 212 / 247 / 331 -> 101 / 130 / 202.
+// Scratch, with chunks = pulse_sample_chunks(vocab): part_max, part_mass (float32), part_idx, seg_n (int32) of rows * chunks entries; seg_i (int32), seg_x (float32) of rows * chunks * pulse_sample_segment()
 // entries; done (int32) of rows entries; and, optional (null: the rows that are left are gone over by their own workgroups
 // alone, with the same choices, as where it does not start at a multiple of 8 bytes), rest (int32) of rows *
 // (pulse_sample_rest() + chunks) entries.
