@@ -137,3 +137,23 @@ def test_parts_of_some_rows_are_the_same_bits_whatever_the_tile(k, n, kk):
         assert torch.equal(some, whole[most - m:]), m
         without_scratch(a[:m], w, some)
         assert torch.equal(some, whole[:m]), m
+
+
+# members whose third part, second part, all parts but the first are below the smallest normal number
+@pytest.mark.parametrize("e", [-60, -108, -112, -118, -124])
+def test_members_far_below_their_row_s_largest(k, e):
+    """A row whose largest value is in range is taken apart whatever its other members are: of these, parts below 2^-126 are lost
+    (less than 2^-126 of a value), and products and sums below it may be flushed, six a pair of values.  It shows where
+    the large values meet zeros."""
+    n, kk = 3074, 2052
+    w = rnd(n, kk, seed=14)
+    w[:, 0] = 0.0
+    for m in (1, 33, 333):
+        a = rnd(m, kk, seed=13) * 2.0 ** e
+        a[:, 0] = 1.0
+        out = torch.empty(m, n, device=DEV)
+        k.gemm_f32(a.to(DEV), w.to(DEV), out)
+        small = a.clone()
+        small[:, 0] = 0.0
+        limit = bound(small, w) + 2.0 ** -126 * (w.abs().to(F64).sum(1) + 6 * kk)
+        assert ((out.cpu().to(F64) - small.to(F64) @ w.to(F64).T).abs() <= limit).all(), m
