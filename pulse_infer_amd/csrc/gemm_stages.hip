@@ -47,9 +47,9 @@ struct StageArgs {
 
 constexpr int PANEL = 8;  // tiles of rows a panel of the tile order
 
-template <int MODE, int WR, int XR, int WN, int WM, int S, int SX, bool NT>
+template <int MODE, int WR, int XR, int WN, int WM, int S, int SX, bool NT, bool FAR>
 __global__ __launch_bounds__(256) void gemm_stages_kernel(StageArgs a) {
-    using Loop = TileLoop<WR, XR, WN, WM, S, NT, SX>;
+    using Loop = TileLoop<WR, XR, WN, WM, S, NT, SX, FAR>;
     __shared__ __attribute__((aligned(1024))) char lds[Loop::LDS];
 
     // The workgroups of a die (every eighth) take neighbouring tiles, in panels of eight tiles of rows, which share
@@ -67,97 +67,89 @@ __global__ __launch_bounds__(256) void gemm_stages_kernel(StageArgs a) {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / PULSE_WAVE);
     const int lane = threadIdx.x % PULSE_WAVE;
     const int64_t k0 = static_cast<int64_t>(split) * a.K;
-    const bf16_t* from[Loop::PER];       // (rows past an operand's end are its last row: their results are not written)
+    typename Loop::Offset from[Loop::PER];       // (rows past an operand's end are its last row: their results are not written)
 #pragma unroll
     for (int j = 0; j < Loop::PER; ++j) {
         const int row = Loop::row_of(j, wave, lane);
-        from[j] = (j < Loop::PER_W ? a.W + static_cast<int64_t>(min(n0 + row, a.N - 1)) * a.ldw
-                                   : a.X + static_cast<int64_t>(min(m0 + row, a.M - 1)) * a.ldx) +
-                  k0 + Loop::piece_of(row, lane) * 8;
+        const int64_t at = j < Loop::PER_W ? min(row, a.N - 1 - n0) * a.ldw : min(row, a.M - 1 - m0) * a.ldx;
+        from[j] = Loop::offset_of(j, at + Loop::piece_of(row, lane) * 8);
     }
+    const bf16_t* const w_rows = a.W + n0 * a.ldw + k0;
+    const bf16_t* const x_rows = a.X + m0 * a.ldx + k0;
     Loop loop;
-    loop.run(from, lds, wave, lane, a.K, MODE == OUT_SWIGLU ? tile_first_step(n0 / TILE_BLOCK, a.K / Loop::BK) : 0);
+    loop.run([&](int j) __attribute__((always_inline)) { return j < Loop::PER_W ? w_rows : x_rows; }, from, lds, wave, lane, a.K,
+             MODE == OUT_SWIGLU ? tile_first_step(n0 / TILE_BLOCK, a.K / Loop::BK) : 0);
 
     // Results leave through LDS, a wavefront's 32 rows at a time, in whole 16-byte pieces of rows.
     constexpr int TN = Loop::TN, TM = Loop::TM;
-    constexpr int FP = TN % 4 == 0 ? (MODE == OUT_F32 ? 2 : 4) : TN % 2 == 0 ? 2 : 1;     // 32-row pieces of W a pass
     constexpr int SIZE = MODE == OUT_F32 ? 4 : 2;
-    constexpr int COLS = MODE == OUT_SWIGLU ? FP * 16 : FP * 32, PITCH = COLS * SIZE + 16;
-    constexpr int PCS = COLS * SIZE / 16, ROWS = PULSE_WAVE / PCS;
+    constexpr int COLS = TN * (MODE == OUT_SWIGLU ? 8 : 16), PITCH = COLS * SIZE + 16, PCS = COLS * SIZE / 16;
     constexpr int WAVE_LDS = Loop::LDS / 4;
-    static_assert(32 * PITCH <= WAVE_LDS && TN % FP == 0, "a wavefront's piece of LDS holds 32 rows of a pass");
+    static_assert(32 * PITCH <= WAVE_LDS && TN % 2 == 0, "a wavefront's piece of LDS holds 32 rows of its part of the tile");
     char* mine = lds + wave * WAVE_LDS;
-    const int wave_n = wave % WN, wave_m = wave / WN, h = lane / 32;
-    const int n_wave = (n0 + wave_n * TN * 32) / (MODE == OUT_SWIGLU ? 2 : 1);
+    const int wave_n = wave % WN, wave_m = wave / WN, h = lane / 16;
+    const int n_wave = (n0 + wave_n * TN * 16) / (MODE == OUT_SWIGLU ? 2 : 1);
     const int n_end = MODE == OUT_SWIGLU ? a.N / 2 : a.N;
     char* out = static_cast<char*>(a.C) + (MODE == OUT_F32 ? split * a.part_stride * 4 : 0);
 #pragma unroll
-    for (int g = 0; g < TM; ++g) {
-        const int m_base = m0 + (wave_m * TM + g) * 32;
+    for (int g0 = 0; g0 < TM; g0 += 2) {
+        const int m_base = m0 + (wave_m * TM + g0) * 16;
         if (m_base >= a.M) break;
 #pragma unroll
-        for (int f0 = 0; f0 < TN; f0 += FP) {
+        for (int g = g0; g < g0 + 2; ++g) {
+            char* at = mine + ((g - g0) * 16 + lane % 16) * PITCH + h * 4 * SIZE;
 #pragma unroll
-            for (int f = 0; f < FP; ++f) {
-                const tile_f32x16& acc = loop.acc[f0 + f][g];
-                char* at = mine + (lane % 32) * PITCH;
+            for (int f = 0; f < TN; f += MODE == OUT_SWIGLU ? 2 : 1) {
+                const tile_f32x4& acc = loop.acc[f][g];
                 if constexpr (MODE == OUT_F32) {
+                    *reinterpret_cast<float4*>(at + f * 64) = float4{acc[0], acc[1], acc[2], acc[3]};
+                } else {
+                    tile_bf16x4 v;
 #pragma unroll
-                    for (int q = 0; q < 4; ++q)
-                        *reinterpret_cast<float4*>(at + (f * 32 + q * 8 + h * 4) * 4) =
-                            float4{acc[q * 4], acc[q * 4 + 1], acc[q * 4 + 2], acc[q * 4 + 3]};
-                } else if constexpr (MODE == OUT_BF16) {
-#pragma unroll
-                    for (int q = 0; q < 4; ++q) {
-                        tile_bf16x4 v;
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) v[i] = (__bf16)acc[q * 4 + i];
-                        *reinterpret_cast<tile_bf16x4*>(at + (f * 32 + q * 8 + h * 4) * 2) = v;
-                    }
-                } else {     // weight rows alternate in slabs of 16: the gate rows of 16 outputs, their up rows behind
-#pragma unroll
-                    for (int q = 0; q < 2; ++q) {
-                        tile_bf16x4 v;
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) {
-                            const float gate = acc[q * 4 + i], up = acc[8 + q * 4 + i];
+                    for (int i = 0; i < 4; ++i) {
+                        if constexpr (MODE == OUT_BF16) {
+                            v[i] = (__bf16)acc[i];
+                        } else {     // weight rows alternate in slabs of 16: the gate rows of 16 outputs, their up rows behind
+                            const float gate = acc[i], up = loop.acc[f + 1][g][i];
                             // (a quarter of 1 + exp(-gate): its reciprocal is a normal number as long as the exponential is
                             // finite.  expf and a division, no nearer to 64 bits behind the rounding to bfloat16, cost 2 to 16 %.)
                             v[i] = (__bf16)(0.25f * gate * __builtin_amdgcn_rcpf(fmaf(0.25f, __expf(-gate), 0.25f)) * up);
                         }
-                        *reinterpret_cast<tile_bf16x4*>(at + (f * 16 + q * 8 + h * 4) * 2) = v;
                     }
+                    *reinterpret_cast<tile_bf16x4*>(at + f * (MODE == OUT_SWIGLU ? 16 : 32)) = v;
                 }
             }
-            tile_wave_sync();
-#pragma unroll
-            for (int it = 0; it < 32 / ROWS; ++it) {
-                const int row = it * ROWS + lane / PCS, pc = lane % PCS;
-                const uint4 v = *reinterpret_cast<const uint4*>(mine + row * PITCH + pc * 16);
-                const int m = m_base + row, n = n_wave + f0 * (MODE == OUT_SWIGLU ? 16 : 32) + pc * (16 / SIZE);
-                if (m < a.M && n < n_end)
-                    *reinterpret_cast<uint4*>(out + (static_cast<int64_t>(m) * a.ldc + n) * SIZE) = v;
-            }
-            tile_wave_sync();
         }
+        tile_wave_sync();
+#pragma unroll
+        for (int it = 0; it < PCS / 2; ++it) {
+            const int row = (it * PULSE_WAVE + lane) / PCS, pc = (it * PULSE_WAVE + lane) % PCS;
+            const uint4 v = *reinterpret_cast<const uint4*>(mine + row * PITCH + pc * 16);
+            const int m = m_base + row, n = n_wave + pc * (16 / SIZE);
+            if (m < a.M && n < n_end) *reinterpret_cast<uint4*>(out + (m * a.ldc + n) * SIZE) = v;
+        }
+        tile_wave_sync();
     }
 }
 
-template <int MODE, int WR, int XR, int WN, int WM, int S, int SX = S, bool NT = true>
+template <int MODE, int WR, int XR, int WN, int WM, int S, int SX = S, bool NT = true, bool FAR = false>
 void launch(StageArgs a, hipStream_t stream) {
     a.tiles_m = (a.M + XR - 1) / XR;
     a.tiles_n = (a.N + WR - 1) / WR;
     const int64_t grid = (static_cast<int64_t>(a.tiles_m) * a.tiles_n * a.splits + 7) / 8 * 8;
-    hipLaunchKernelGGL((gemm_stages_kernel<MODE, WR, XR, WN, WM, S, SX, NT>), dim3(static_cast<unsigned>(grid)), dim3(256), 0, stream, a);
+    hipLaunchKernelGGL((gemm_stages_kernel<MODE, WR, XR, WN, WM, S, SX, NT, FAR>), dim3(static_cast<unsigned>(grid)), dim3(256), 0, stream, a);
 }
 
 // weight rows and rows of X a tile (the kernels below, in this order)
 constexpr int SHAPES[][2] = {{64, 64}, {64, 128}, {96, 128}, {128, 64}, {128, 128}, {192, 128}, {256, 128},
                                {192, 192}, {192, 256}, {256, 192}, {256, 256}};
+constexpr int64_t FAR_ROWS = 1 << 22;   // values between rows: 256 of them come to 2 GB
 constexpr int NUM_SHAPES = sizeof(SHAPES) / sizeof(SHAPES[0]);
 
 template <int MODE>
 void launch_shape(int shape, const StageArgs& a, hipStream_t s) {
+    // (a tile's last row must lie less than 4 GB behind its first; what does not goes by pointers, in the smallest tiles)
+    if (a.ldx >= FAR_ROWS || a.ldw >= FAR_ROWS) return launch<MODE, 64, 64, 2, 2, 6, 6, true, true>(a, s);
     switch (shape) {
         case 0: return launch<MODE, 64, 64, 2, 2, 6>(a, s);
         case 1: return launch<MODE, 64, 128, 2, 2, 6>(a, s);

@@ -410,46 +410,52 @@ __global__ __launch_bounds__(WN* WM* PULSE_WAVE) void moe_tile_kernel(GroupArgs 
     __syncthreads();
 
     // (rows past the end are the tile's first row, weight rows past the end the last one: their results are not written)
-    const bf16_t* from[Loop::PER];
+    // A chunk is eight rows of one weight: gate and up alternate in slabs of 16.
+    const int64_t first_row = static_cast<int64_t>(e) * a.N + n0;
+    typename Loop::Offset from[Loop::PER];
 #pragma unroll
     for (int j = 0; j < Loop::PER; ++j) {
-        const int row = Loop::row_of(j, wave, lane), piece = Loop::piece_of(row, lane);
-        if (j < Loop::PER_W) {
-            const int n = DOWN ? n0 + row : n0 + row / 32 * 16 + row % 16;
-            const bf16_t* w = DOWN ? a.w[0] : (row & 16) ? a.w[1] : a.w[0];
-            from[j] = w + (static_cast<int64_t>(e) * a.N + min(n, a.N - 1)) * a.K + piece * 8;
-        } else {
-            const int p = pair_s[row] < 0 ? pair_s[0] : pair_s[row];
-            from[j] = a.x + static_cast<int64_t>(DOWN ? p : p / a.top) * a.K + piece * 8;
-        }
+        const int row = Loop::row_of(j, wave, lane);
+        int64_t at;
+        if (j < Loop::PER_W) at = min(DOWN ? row : row / 32 * 16 + row % 16, a.N - 1 - n0);
+        else at = (pair_s[row] < 0 ? pair_s[0] : pair_s[row]) / (DOWN ? 1 : a.top);
+        from[j] = Loop::offset_of(j, at * a.K + Loop::piece_of(row, lane) * 8);
     }
     Loop loop;
     constexpr int BLOCK = DOWN ? TILE_BLOCK : TILE_BLOCK / 2;
-    loop.run(from, lds, wave, lane, a.K, tile_first_step(e * ((a.N + BLOCK - 1) / BLOCK) + n0 / BLOCK, a.K / Loop::BK));
+    loop.run([&](int j) __attribute__((always_inline)) {
+                 if (j >= Loop::PER_W) return a.x;
+                 return (!DOWN && (wave * Loop::PER_W + j) & 2 ? a.w[1] : a.w[0]) + first_row * a.K;
+             }, from, lds, wave, lane, a.K, tile_first_step(e * ((a.N + BLOCK - 1) / BLOCK) + n0 / BLOCK, a.K / Loop::BK));
 
     // Results leave through LDS, a wavefront's 32 rows at a time, in whole 16-byte pieces of rows.
     constexpr int TN = Loop::TN, TM = Loop::TM;
+    constexpr int SIZE = DOWN ? 4 : 2, W_COLS = TN * (DOWN ? 16 : 8), PITCH = W_COLS * SIZE + 16, PCS = W_COLS * SIZE / 16;
     constexpr int WAVE_LDS = Loop::LDS / Loop::NW;
+    static_assert(32 * PITCH <= WAVE_LDS && TN % 2 == 0, "a wavefront's piece of LDS holds 32 rows of its part of the tile");
     char* mine = lds + wave * WAVE_LDS;
-    const int wave_n = wave % WN, wave_m = wave / WN, h = lane / 32;
-    const int n_wave = n0 + wave_n * TN * (DOWN ? 32 : 16);
+    const int wave_n = wave % WN, wave_m = wave / WN, h = lane / 16;
+    const int n_wave = n0 + wave_n * W_COLS;
 #pragma unroll
-    for (int g = 0; g < TM; ++g) {
-        const int m_base = (wave_m * TM + g) * 32;
+    for (int g0 = 0; g0 < TM; g0 += 2) {
+        const int m_base = (wave_m * TM + g0) * 16;
         if (m_base >= rows) break;
-        if constexpr (!DOWN) {
-            constexpr int W_COLS = TN * 16, PITCH = W_COLS * 2 + 16;
-            static_assert(32 * PITCH <= WAVE_LDS, "a wavefront's piece of LDS holds 32 rows of its part of the tile");
-            const float wgt = weight_s[m_base + lane % 32];
 #pragma unroll
-            for (int f = 0; f < TN; ++f)
+        for (int g = g0; g < g0 + 2; ++g) {
+            char* at = mine + ((g - g0) * 16 + lane % 16) * PITCH + h * 4 * SIZE;
+            if constexpr (DOWN) {
 #pragma unroll
-                for (int q = 0; q < 2; ++q) {
+                for (int f = 0; f < TN; ++f)
+                    *reinterpret_cast<float4*>(at + f * 64) = float4{loop.acc[f][g][0], loop.acc[f][g][1], loop.acc[f][g][2], loop.acc[f][g][3]};
+            } else {
+                const float wgt = weight_s[(wave_m * TM + g) * 16 + lane % 16];
+#pragma unroll
+                for (int f = 0; f < TN; f += 2) {
                     tile_bf16x4 v;
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
                         // an expert that is fed weight * x: both products are linear, so the factor goes onto their results
-                        float gate = loop.acc[f][g][q * 4 + i] * wgt, up = loop.acc[f][g][8 + q * 4 + i] * wgt;
+                        float gate = loop.acc[f][g][i] * wgt, up = loop.acc[f + 1][g][i] * wgt;
                         if (a.act_kind == 1) {   // clamped: min(g, limit) * sigmoid(1.702 g) * (clamp(u) + 1)
                             gate = fminf(gate, a.limit);
                             up = fminf(fmaxf(up, -a.limit), a.limit);
@@ -458,49 +464,20 @@ __global__ __launch_bounds__(WN* WM* PULSE_WAVE) void moe_tile_kernel(GroupArgs 
                             v[i] = (__bf16)(gate / (1.0f + expf(-gate)) * up);
                         }
                     }
-                    *reinterpret_cast<tile_bf16x4*>(mine + (lane % 32) * PITCH + (f * 16 + q * 8 + h * 4) * 2) = v;
+                    *reinterpret_cast<tile_bf16x4*>(at + f * 16) = v;
                 }
-            tile_wave_sync();
-            constexpr int PCS = W_COLS / 8;
-#pragma unroll
-            for (int it = 0; it < 32 * PCS / PULSE_WAVE; ++it) {
-                const int row = (it * PULSE_WAVE + lane) / PCS, pc = (it * PULSE_WAVE + lane) % PCS;
-                const uint4 v = *reinterpret_cast<const uint4*>(mine + row * PITCH + pc * 16);
-                const int p = pair_s[m_base + row], n = n_wave + pc * 8;
-                if (p >= 0 && n < a.N)
-                    *reinterpret_cast<uint4*>(static_cast<bf16_t*>(a.out) + static_cast<int64_t>(p) * a.N + n) = v;
-            }
-            tile_wave_sync();
-        } else {
-            constexpr int FP = TN % 2 == 0 ? 2 : TN;   // 32-row pieces of W a pass
-            constexpr int W_COLS = FP * 32, PITCH = W_COLS * 4 + 16;
-            static_assert(32 * PITCH <= WAVE_LDS && TN % FP == 0, "a wavefront's piece of LDS holds 32 rows of a pass");
-#pragma unroll
-            for (int f0 = 0; f0 < TN; f0 += FP) {
-#pragma unroll
-                for (int f = 0; f < FP; ++f)
-#pragma unroll
-                    for (int q = 0; q < 4; ++q) {
-                        float4 v;
-                        v.x = loop.acc[f0 + f][g][q * 4];
-                        v.y = loop.acc[f0 + f][g][q * 4 + 1];
-                        v.z = loop.acc[f0 + f][g][q * 4 + 2];
-                        v.w = loop.acc[f0 + f][g][q * 4 + 3];
-                        *reinterpret_cast<float4*>(mine + (lane % 32) * PITCH + (f * 32 + q * 8 + h * 4) * 4) = v;
-                    }
-                tile_wave_sync();
-                constexpr int PCS = W_COLS / 4;
-#pragma unroll
-                for (int it = 0; it < 32 * PCS / PULSE_WAVE; ++it) {
-                    const int row = (it * PULSE_WAVE + lane) / PCS, pc = (it * PULSE_WAVE + lane) % PCS;
-                    const float4 v = *reinterpret_cast<const float4*>(mine + row * PITCH + pc * 16);
-                    const int p = pair_s[m_base + row], n = n_wave + f0 * 32 + pc * 4;
-                    if (p >= 0 && n < a.N)
-                        *reinterpret_cast<float4*>(static_cast<float*>(a.out) + static_cast<int64_t>(p) * a.N + n) = v;
-                }
-                tile_wave_sync();
             }
         }
+        tile_wave_sync();
+#pragma unroll
+        for (int it = 0; it < PCS / 2; ++it) {
+            const int row = (it * PULSE_WAVE + lane) / PCS, pc = (it * PULSE_WAVE + lane) % PCS;
+            const uint4 v = *reinterpret_cast<const uint4*>(mine + row * PITCH + pc * 16);
+            const int p = pair_s[m_base + row], n = n_wave + pc * (16 / SIZE);
+            if (p >= 0 && n < a.N)
+                *reinterpret_cast<uint4*>(static_cast<char*>(a.out) + (static_cast<int64_t>(p) * a.N + n) * SIZE) = v;
+        }
+        tile_wave_sync();
     }
 }
 
@@ -554,6 +531,9 @@ extern "C" int pulse_moe_group(const int* idx, int pairs, int experts, int tile_
 
 static bool aligned16(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
 
+// Whether `rows` rows of K values, and a tile's rows of a weight, lie less than 4 GB behind the first (moe_tile_kernel's offsets).
+static bool near_rows(int64_t rows, int K) { return K < (1 << 22) && rows * K < (1ll << 30); }
+
 extern "C" int pulse_moe_gate_up_grouped(const void* x, const void* wg, const void* wu, const int* order,
                                          const int* tile_expert, const int* tile_row0, const int* tile_rows,
                                          const int* num_tiles, int max_tiles, int tile_rows_max, void* act, int hidden,
@@ -567,7 +547,8 @@ extern "C" int pulse_moe_gate_up_grouped(const void* x, const void* wg, const vo
     PULSE_REQUIRE(x && wg && wu && order && tile_expert && tile_row0 && tile_rows && num_tiles && act,
                   "moe_gate_up_grouped: null pointer");
     PULSE_REQUIRE((ff + 15) / 16 < 65536, "moe_gate_up_grouped: an inner width of %d is too large", ff);
-    if (hidden % 64 == 0 && ff % 8 == 0 && aligned16(act)) {   // (the loop walks K in whole steps of 64; rows leave in 16-byte pieces)
+    // (the loop walks K in whole steps of 64; rows leave in 16-byte pieces; the tiles have room for every pair)
+    if (hidden % 64 == 0 && ff % 8 == 0 && aligned16(act) && near_rows(static_cast<int64_t>(max_tiles) * tile_rows_max / top + 1, hidden)) {
         launch_tiles_for<false>({static_cast<const bf16_t*>(x), {static_cast<const bf16_t*>(wg), static_cast<const bf16_t*>(wu)},
                                  act, order, tile_expert, tile_row0, tile_rows, num_tiles, in_weight, hidden, ff, top, 0,
                                  act_kind, limit}, max_tiles, tile_rows_max, stream);
@@ -597,7 +578,7 @@ extern "C" int pulse_moe_down_grouped(const void* act, const void* wd, const int
     PULSE_REQUIRE(act && wd && order && tile_expert && tile_row0 && tile_rows && num_tiles && y,
                   "moe_down_grouped: null pointer");
     PULSE_REQUIRE((hidden + 15) / 16 < 65536, "moe_down_grouped: a width of %d is too large", hidden);
-    if (ff % 64 == 0 && hidden % 4 == 0 && aligned16(y)) {
+    if (ff % 64 == 0 && hidden % 4 == 0 && aligned16(y) && near_rows(static_cast<int64_t>(max_tiles) * tile_rows_max, ff)) {
         launch_tiles_for<true>({static_cast<const bf16_t*>(act), {static_cast<const bf16_t*>(wd), nullptr}, y, order, tile_expert,
                                 tile_row0, tile_rows, num_tiles, nullptr, ff, hidden, 1, 0, 0, 0.f}, max_tiles, tile_rows_max, stream);
         PULSE_LAUNCH_CHECK("moe_down_grouped");

@@ -1,5 +1,5 @@
 // The loop of a matrix product on an output tile of WR weight rows x XR rows of X, bfloat16 operands, float32 sums:
-// WN wavefronts along the weight rows by WM along the rows of X, on v_mfma_f32_32x32x16_bf16.
+// WN wavefronts along the weight rows by WM along the rows of X, on v_mfma_f32_16x16x32_bf16.
 //
 // K goes in steps of 64 through S stages of LDS for the tile's rows of W and SX for those of X (128 bytes a row), filled
 // straight from memory; S - 1 steps are on their way while one is multiplied, and there is one barrier a step, before its
@@ -8,14 +8,25 @@
 // rows, the weights' way from memory: a compute unit must have some tens of kilobytes on their way all the time (6 TB/s x
 // 2 us over 256 units: 48 KB).  X comes from L2 and may have one stage less: it goes out first.
 //
-// The tile of the matrix instruction is D[n][m] = W . X^T: lane l holds column m = l % 32 and rows n = 8 (i / 4) +
-// 4 (l / 32) + i % 4, i = 0 .. 15, of a 32 x 32 piece.
+// The tile of the matrix instruction is D[n][m] = W . X^T: lane l holds column m = l % 16 and rows n = 4 (l / 16) + i, i = 0 .. 3, of
+// a 16 x 16 piece.
+//
+// The instruction: from some 300 rows on a product takes what the card's power allows, and v_mfma_f32_16x16x32_bf16 reads and writes half
+// as many sums a product as v_mfma_f32_32x32x16_bf16, on which this loop ran before: 2,048 rows of 24,576 x 4,096 with SwiGLU in tiles
+// of 256 x 256 314 -> 282 us (with operands of zeros, which cost little power, 227 and 224), 509 rows in 192 x 256 84 -> 81.
+// Neighbouring products share an operand (two rows of X's pieces in turns): 285 -> 281 us against one row after the other.
+//
+// The copies: a base in scalar registers, which moves along K, and a lane's byte offset from it, which does not; a wavefront's eight
+// chunks of 1 KB lie in a row in LDS and are told apart by the instruction's own offset, so a copy is one instruction in the loop (with a
+// pointer a lane and M0 set for each, six: 324 -> 306 us at 2,048 rows, 85 -> 81 at 357 in 192 x 256, before the other instruction).
 #pragma once
 #include "common.h"
+#include <type_traits>
+#include <utility>
 
 typedef __attribute__((ext_vector_type(8))) __bf16 tile_bf16x8;
 typedef __attribute__((ext_vector_type(4))) __bf16 tile_bf16x4;
-typedef __attribute__((ext_vector_type(16))) float tile_f32x16;
+typedef __attribute__((ext_vector_type(4))) float tile_f32x4;
 
 // Where along K (of so many steps) the tiles of a block of TILE_BLOCK weight rows start.  Rows of a power of two bytes, at the
 // same place in all of a launch's workgroups at a time, fall on few of the memory's channels; blocks that start elsewhere, in
@@ -27,24 +38,30 @@ typedef __attribute__((ext_vector_type(16))) float tile_f32x16;
 constexpr int TILE_BLOCK = 768;
 __device__ __forceinline__ int tile_first_step(int block, int steps) { return (steps & (steps - 1)) == 0 ? (block * 5) & (steps - 1) : 0; }
 
-template <int WR, int XR, int WN, int WM, int S, bool NT = false, int SX = S>
+// f(0), f(1) .. f(N - 1) with constants (an unrolled loop whatever its size).
+template <typename F, int... I>
+__device__ __forceinline__ void tile_each(F&& f, std::integer_sequence<int, I...>) { (f(std::integral_constant<int, I>()), ...); }
+template <int N, typename F>
+__device__ __forceinline__ void tile_each(F&& f) { tile_each(f, std::make_integer_sequence<int, N>()); }
+
+// FAR: rows further than 4 GB from their base (a pointer a lane, as slow as that is).
+template <int WR, int XR, int WN, int WM, int S, bool NT = false, int SX = S, bool FAR = false>
 struct TileLoop {
     static constexpr int BK = 64;
     static constexpr int ROW_BYTES = BK * 2;
     static constexpr int STAGE_W = WR * ROW_BYTES, STAGE_X = XR * ROW_BYTES, X0 = S * STAGE_W;
     static constexpr int NW = WN * WM;
-    static constexpr int TN = WR / 32 / WN, TM = XR / 32 / WM;       // 32-row pieces a wavefront
+    static constexpr int TN = WR / 16 / WN, TM = XR / 16 / WM;       // 16-row pieces a wavefront
     static constexpr int PER_W = WR / 8 / NW, PER_X = XR / 8 / NW;   // chunks of 1 KB (8 rows) a wavefront copies
     static constexpr int PER = PER_W + PER_X;
-    static constexpr int KK = BK / 16;                               // products of the matrix instruction's depth a step
+    static constexpr int KK = BK / 32;                               // products of the matrix instruction's depth a step
+    static constexpr int P = TN * TM, ALL = KK * P;                  // products a depth, and a step
     static constexpr int LDS = X0 + SX * STAGE_X;
     // The next products' operand reads go out between these, over the first READS of them, so that the last is here in time: a
-    // lone wavefront a SIMD issues no product while it issues reads.  (All of them ahead of the products, 24,576 x 4,096 with
-    // SwiGLU alone: 357 rows in tiles of 192 x 192 74 us, so 70; 509 rows in 192 x 256 91 and 86.  Inside a step, at the power
-    // limit, a prompt of 509 gains 0.6 %.)  Where a step has few products the reads go ahead of them (0): behind the first they
-    // are late (experts of 8 tokens in 64 x 32, a step 1 % slower).
-    static constexpr int READS = TN * TM < 6 ? 0 : TN * TM == 6 ? 4 : TN * TM - 3;
-    static_assert(WR % (8 * NW) == 0 && XR % (8 * NW) == 0 && TN >= 1 && TM >= 1 && SX >= 2 && S >= SX,
+    // lone wavefront a SIMD issues no product while it issues reads.  Where a step has few products the reads go ahead of them (0):
+    // behind the first they are late (experts of 8 tokens in 64 x 32, a step 1 % slower).
+    static constexpr int READS = P < 24 ? 0 : P * 3 / 4;
+    static_assert(WR % (8 * NW) == 0 && XR % (8 * NW) == 0 && TN >= 1 && TM % 2 == 0 && SX >= 2 && S >= SX,
                   "whole chunks and pieces a wavefront");
     static_assert(TILE_BLOCK % WR == 0, "a tile lies inside a block of weight rows");
 
@@ -52,7 +69,7 @@ struct TileLoop {
     // lie in different places of what LDS serves at once.
     static __device__ __forceinline__ int swz(int row) { return (row & 7) ^ ((row >> 3) & 1); }
 
-    tile_f32x16 acc[TN][TM];
+    tile_f32x4 acc[TN][TM];
 
     // Row (of the tile's W for j < PER_W, else of its X) and piece that this lane brings with the wavefront's j-th chunk.
     static __device__ __forceinline__ int row_of(int j, int wave, int lane) {
@@ -60,103 +77,131 @@ struct TileLoop {
     }
     static __device__ __forceinline__ int piece_of(int row, int lane) { return (lane % 8) ^ swz(row); }
 
-    // from[j]: where that piece lies in memory at k = 0.  The walk along K starts at step `first` and goes round its end.
-    __device__ __forceinline__ void run(const bf16_t* const (&from)[PER], char* lds, int wave, int lane, int K, int first = 0) {
+    // A lane's offset for its j-th chunk from that piece's place in memory at k = 0, in values from the chunk's base.  (Less what the
+    // copy's instruction adds, which moves both the place in LDS and the one in memory; BACK keeps it from below zero.)
+    typedef std::conditional_t<FAR, uint64_t, uint32_t> Offset;
+    static constexpr int BACK = FAR ? 0 : 3072;
+    static constexpr int inside(int j) { return FAR ? 0 : ((j < PER_W ? j : j - PER_W) % 8 - 4) * 1024; }
+    static __device__ __forceinline__ Offset offset_of(int j, int64_t values) { return static_cast<Offset>(values * 2 + BACK - inside(j)); }
+
+    // base(j): where the wavefront's j-th chunk counts its offsets from, the same for all lanes.  The walk along K starts at step
+    // `first` and goes round its end.
+    template <typename Base>
+    __device__ __forceinline__ void run(Base&& base, const Offset (&from)[PER], char* lds, int wave, int lane, int K, int first = 0) {
         const int wave_n = wave % WN, wave_m = wave / WN;
         const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(
             (void __attribute__((address_space(3)))*)(lds)));
         const int steps = K / BK;
         auto place = [&](int step) __attribute__((always_inline)) {      // (steps past the last: copies that nobody reads)
             const int at = min(step, steps - 1) + first;
-            return (at >= steps ? at - steps : at) * BK;
+            return (at >= steps ? at - steps : at) * ROW_BYTES;
         };
+        // The batch of step s, W of step s + S and X of step s + SX, goes out behind that step's barrier: FIRST copies of it
+        // between the step's last products, the others between the next step's.
+        constexpr int FIRST = P * PER / ALL;
+        constexpr int LATER = (SX - 2) * PER + (S > SX ? PER_W : 0);   // copies behind the last that the next step needs
         // The j-th copy of a batch, X first; a batch: W of one step into its slot, X of another into its.
-        auto copy = [&](int step_w, int slot_w, int step_x, int slot_x, int j) __attribute__((always_inline)) {
-            if (j < PER_X) {
-                load_to_lds(from[PER_W + j] + place(step_x), lds0 + X0 + slot_x * STAGE_X + (wave * PER_X + j) * 1024);
+        auto copy = [&](int step_w, int slot_w, int step_x, int slot_x, auto jc) __attribute__((always_inline)) {
+            constexpr int j = jc;
+            constexpr bool is_x = j < PER_X;
+            constexpr int i = is_x ? j : j - PER_X, c = is_x ? PER_W + j : j - PER_X;
+            const Offset off = from[c];
+            const char* at = reinterpret_cast<const char*>(base(c)) - BACK + place(is_x ? step_x : step_w);
+            const uint32_t to = lds0 + (is_x ? X0 + slot_x * STAGE_X + wave * PER_X * 1024 : slot_w * STAGE_W + wave * PER_W * 1024);
+            if constexpr (FAR) {
+                if constexpr (NT && !is_x) stream_to_lds(at + off, to + i * 1024);
+                else load_to_lds(at + off, to + i * 1024);
             } else {
-                const bf16_t* at = from[j - PER_X] + place(step_w);
-                const uint32_t to = lds0 + slot_w * STAGE_W + (wave * PER_W + j - PER_X) * 1024;
-                if constexpr (NT) stream_to_lds(at, to);
-                else load_to_lds(at, to);
+                // M0, the place in LDS, holds for the eight chunks behind it (nothing that the compiler makes of this loop uses M0)
+                if constexpr (i % 8 == 0 || j == FIRST)
+                    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0" : : "s"(to + (i / 8 * 8 + 4) * 1024) : "memory", "m0");
+                if constexpr (NT && !is_x)
+                    asm volatile("global_load_lds_dwordx4 %0, %1 offset:%c2 nt" : : "v"(off), "s"(at), "n"(inside(c)) : "memory");
+                else
+                    asm volatile("global_load_lds_dwordx4 %0, %1 offset:%c2" : : "v"(off), "s"(at), "n"(inside(c)) : "memory");
             }
         };
-        const int h = lane / 32, e = h ^ swz(lane % 32);
+        const int h = lane / 16, e = h ^ swz(lane % 16);
         int w_at[KK], x_at[KK];
 #pragma unroll
         for (int kk = 0; kk < KK; ++kk) {
-            const int place = (e ^ (kk << 1)) * 16;
-            w_at[kk] = (wave_n * TN * 32 + lane % 32) * ROW_BYTES + place;
-            x_at[kk] = X0 + (wave_m * TM * 32 + lane % 32) * ROW_BYTES + place;
+            const int piece = (e ^ (kk << 2)) * 16;
+            w_at[kk] = (wave_n * TN * 16 + lane % 16) * ROW_BYTES + piece;
+            x_at[kk] = X0 + (wave_m * TM * 16 + lane % 16) * ROW_BYTES + piece;
         }
 #pragma unroll
         for (int f = 0; f < TN; ++f)
 #pragma unroll
             for (int g = 0; g < TM; ++g)
 #pragma unroll
-                for (int i = 0; i < 16; ++i) acc[f][g][i] = 0.f;
+                for (int i = 0; i < 4; ++i) acc[f][g][i] = 0.f;
 
-        // The batch of step s, W of step s + S and X of step s + SX, goes out behind that step's barrier: FIRST copies of it
-        // between the step's last products, the others between the next step's.
-        constexpr int ALL = KK * TN * TM, FIRST = TN * TM * PER / ALL;
-        constexpr int LATER = (SX - 2) * PER + (S > SX ? PER_W : 0);   // copies behind the last that the next step needs
-#pragma unroll
-        for (int s = -S; s < -1; ++s)
-#pragma unroll
-            for (int j = s + SX >= 0 ? 0 : PER_X; j < PER; ++j) copy(s + S, s + S, s + SX, s + SX, j);
-#pragma unroll
-        for (int j = 0; j < FIRST; ++j) copy(S - 1, S - 1, SX - 1, SX - 1, j);
+        tile_each<S - 1>([&](auto sc) __attribute__((always_inline)) {
+            constexpr int s = sc - S;
+            tile_each<PER>([&](auto j) __attribute__((always_inline)) {
+                if constexpr (s + SX >= 0 || j >= PER_X) copy(s + S, s + S, s + SX, s + SX, j);
+            });
+        });
+        tile_each<FIRST>([&](auto j) __attribute__((always_inline)) { copy(S - 1, S - 1, SX - 1, SX - 1, j); });
         tile_bf16x8 wf[2][TN], xf[2][TM];
         asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" : : "n"(LATER + FIRST) : "memory");
 #pragma unroll
-        for (int g = 0; g < TM; ++g) xf[0][g] = *reinterpret_cast<const tile_bf16x8*>(lds + x_at[0] + g * 32 * ROW_BYTES);
+        for (int g = 0; g < TM; ++g) xf[0][g] = *reinterpret_cast<const tile_bf16x8*>(lds + x_at[0] + g * 16 * ROW_BYTES);
 #pragma unroll
-        for (int f = 0; f < TN; ++f) wf[0][f] = *reinterpret_cast<const tile_bf16x8*>(lds + w_at[0] + f * 32 * ROW_BYTES);
+        for (int f = 0; f < TN; ++f) wf[0][f] = *reinterpret_cast<const tile_bf16x8*>(lds + w_at[0] + f * 16 * ROW_BYTES);
         int sw = 0, sx = 0;
         for (int s = 0; s < steps; ++s) {
             const int next_w = sw == S - 1 ? 0 : sw + 1, before_w = sw == 0 ? S - 1 : sw - 1;
             const int next_x = sx == SX - 1 ? 0 : sx + 1, before_x = sx == 0 ? SX - 1 : sx - 1;
-#pragma unroll
-            for (int kk = 0; kk < KK; ++kk) {
-                const int buf = kk & 1, then = kk == KK - 1 ? 0 : kk + 1;
+            tile_each<KK>([&](auto kc) __attribute__((always_inline)) {
+                constexpr int kk = kc, buf = kk & 1, then = kk == KK - 1 ? 0 : kk + 1;
                 const char* const lds_w = lds + (kk == KK - 1 ? next_w : sw) * STAGE_W + w_at[then];
                 const char* const lds_x = lds + (kk == KK - 1 ? next_x : sx) * STAGE_X + x_at[then];
                 __builtin_amdgcn_sched_barrier(0);
                 // before a step's last products: this wavefront's copies of the next step have landed and its operands are
                 // here; behind the barrier that holds for everyone
-                if (kk == KK - 1) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"(LATER) : "memory");
-                // (the operands of the products behind these, in the order in which those ask for them)
+                if constexpr (kk == KK - 1) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"(LATER) : "memory");
+                // (the operands of the products behind these)
                 auto read = [&](int i) __attribute__((always_inline)) {
-                    if (i < TM) xf[buf ^ 1][i] = *reinterpret_cast<const tile_bf16x8*>(lds_x + i * 32 * ROW_BYTES);
-                    else wf[buf ^ 1][i - TM] = *reinterpret_cast<const tile_bf16x8*>(lds_w + (i - TM) * 32 * ROW_BYTES);
+                    if (i < TM) xf[buf ^ 1][i] = *reinterpret_cast<const tile_bf16x8*>(lds_x + i * 16 * ROW_BYTES);
+                    else wf[buf ^ 1][i - TM] = *reinterpret_cast<const tile_bf16x8*>(lds_w + (i - TM) * 16 * ROW_BYTES);
                 };
                 if constexpr (READS == 0) {
 #pragma unroll
                     for (int i = 0; i < TN + TM; ++i) read(i);
                 }
                 __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                for (int p = 0; p < TN * TM; ++p) {
-                    acc[p / TM][p % TM] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[buf][p / TM], xf[buf][p % TM],
-                                                                                  acc[p / TM][p % TM], 0, 0, 0);
+                tile_each<P>([&](auto pc) __attribute__((always_inline)) {
+                    // two pieces of X in turns along the pieces of W, and back with the next two
+                    constexpr int p = pc, pair = p / (2 * TN), f = p % (2 * TN) / 2, g = 2 * pair + (p % 2 ^ f % 2), n = pair % 2 ? TN - 1 - f : f;
+                    acc[n][g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[buf][n], xf[buf][g], acc[n][g], 0, 0, 0);
                     __builtin_amdgcn_sched_barrier(0);
                     if constexpr (READS > 0) {
+                        constexpr int from_i = (p < READS ? p : READS) * (TN + TM) / READS, to_i = (p + 1 < READS ? p + 1 : READS) * (TN + TM) / READS;
 #pragma unroll
-                        for (int i = min(p, READS) * (TN + TM) / READS; i < min(p + 1, READS) * (TN + TM) / READS; ++i) read(i);
+                        for (int i = from_i; i < to_i; ++i) read(i);
                     }
                     __builtin_amdgcn_sched_barrier(0);
                     // the copies, spread evenly over the products
-                    const int q = (kk == KK - 1 ? 0 : kk + 1) * TN * TM + p;
-#pragma unroll
-                    for (int j = q * PER / ALL; j < (q + 1) * PER / ALL; ++j) {
-                        if (kk == KK - 1) copy(s + S, sw, s + SX, sx, j);
+                    constexpr int q = (kk == KK - 1 ? 0 : kk + 1) * P + p;
+                    tile_each<(q + 1) * PER / ALL - q * PER / ALL>([&](auto jc) __attribute__((always_inline)) {
+                        constexpr std::integral_constant<int, q * PER / ALL + jc> j{};
+                        if constexpr (kk == KK - 1) copy(s + S, sw, s + SX, sx, j);
                         else copy(s + S - 1, before_w, s + SX - 1, before_x, j);
-                    }
+                    });
                     __builtin_amdgcn_sched_barrier(0);
-                }
-            }
+                });
+            });
             sw = next_w, sx = next_x;
         }
+        // the sums stay in the registers they are made in up to here (where their stores want them elsewhere, the compiler moved them in the loop)
+#pragma unroll
+        for (int f = 0; f < TN; ++f)
+#pragma unroll
+            for (int g = 0; g < TM; ++g) {
+                if constexpr (P >= 24) asm volatile("" : "+a"(acc[f][g]));
+                else asm volatile("" : "+v"(acc[f][g]));
+            }
         // the last copies, which nobody reads, must not land in what follows
         asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" : : : "memory");
     }

@@ -83,3 +83,36 @@ def test_router_logits_at_the_edges_of_its_blocks(n, hidden, tokens):
         assert ((got - want).abs() <= bound.gather(1, chosen)).all()
         if n > 200 and first >= 8 * top:      # (enough of them to meet every block)
             break
+
+
+def test_grouped_experts_with_room_for_more_pairs_than_offsets_reach():
+    """Lists with room for so many pairs that their rows may lie more than 4 GB apart take the kernels that go by pointers."""
+    from pulse_infer_amd.ops import kernels
+
+    hidden, ff, experts, pairs, rows = 64, 64, 3, 200, 192
+    x = rnd(pairs, hidden, seed=2).to(torch.bfloat16).to(DEV)
+    wg, wu = ((rnd(experts, ff, hidden, seed=3 + i) * hidden ** -0.5).to(torch.bfloat16).to(DEV) for i in range(2))
+    wd = (rnd(experts, hidden, ff, seed=5) * ff ** -0.5).to(torch.bfloat16).to(DEV)
+    idx = (torch.arange(pairs, dtype=torch.int32) % experts).to(DEV)
+    few = kernels.moe_max_tiles(pairs, experts, rows)
+    many = (1 << 24) // rows + few
+    rank, order = (torch.empty(pairs, dtype=torch.int32, device=DEV) for _ in range(2))
+    tile_expert, tile_row0, tile_rows = (torch.empty(many, dtype=torch.int32, device=DEV) for _ in range(3))
+    num = torch.empty(1, dtype=torch.int32, device=DEV)
+    p, i32 = kernels._ptr, kernels._i32
+    kernels.call("pulse_moe_group", p(idx), i32(pairs), i32(experts), i32(rows), i32(few), p(rank), p(order), p(tile_expert), p(tile_row0),
+                 p(tile_rows), p(num), kernels._stream())
+    lists = [p(order), p(tile_expert), p(tile_row0), p(tile_rows), p(num)]
+    e = idx.long().cpu()
+    g = torch.einsum("th,tfh->tf", x.cpu().to(F64), wg.cpu().to(F64)[e])
+    want = g * torch.sigmoid(g) * torch.einsum("th,tfh->tf", x.cpu().to(F64), wu.cpu().to(F64)[e])
+    for tiles in (few, many):
+        act = torch.full((pairs, ff), float("nan"), dtype=torch.bfloat16, device=DEV)
+        kernels.call("pulse_moe_gate_up_grouped", p(x), p(wg), p(wu), *lists, i32(tiles), i32(rows), p(act), i32(hidden), i32(ff), i32(1),
+                     p(None), i32(0), kernels._f32(0.0), kernels._stream())
+        got = act.cpu().to(F64)
+        assert ((got - want).abs() <= 2.0 ** -8 * want.abs() + 1e-5 * (1.0 + want.abs().max())).all(), tiles
+        y = torch.full((pairs, hidden), float("nan"), device=DEV)
+        kernels.call("pulse_moe_down_grouped", p(act), p(wd), *lists, i32(tiles), i32(rows), p(y), i32(hidden), i32(ff), kernels._stream())
+        out, size = (torch.einsum("tf,thf->th", a, b) for a, b in ((got, wd.cpu().to(F64)[e]), (got.abs(), wd.cpu().to(F64)[e].abs())))
+        assert ((y.cpu().to(F64) - out).abs() <= (ff + 4) * 2.0 ** -24 * size).all(), tiles

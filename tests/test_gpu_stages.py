@@ -230,3 +230,24 @@ def test_blocks_of_weight_rows_start_together_where_their_rows_are_no_power_of_t
     act = torch.full((rows, 1536), float("nan"), dtype=torch.bfloat16, device=DEV)
     kernels.gemm_stages(x, w, act, swiglu=True)
     assert not torch.isnan(act).any() and torch.equal(act[:, :768], act[:, 768:])
+
+
+@pytest.mark.parametrize("far", ["x", "w", "both"])
+def test_product_in_stages_of_rows_gigabytes_apart(far):
+    """A tile's rows more than 4 GB behind its first: by pointers, the same bits as of rows that lie together."""
+    from pulse_infer_amd.ops import kernels
+
+    m, n, k = 70, 160, 192
+    x, w, _, _ = product(m, n, k)
+    apart = (1 << 22) + 8
+    xf, wf = (torch.empty_strided(t.shape, (apart, 1), dtype=t.dtype, device=DEV).copy_(t) if far in (name, "both") else t
+              for name, t in (("x", x), ("w", w)))
+    for swiglu, width in ((False, n), (True, n // 2)):
+        near, out = (torch.full((m, width), float("nan"), dtype=torch.bfloat16, device=DEV) for _ in range(2))
+        kernels.gemm_stages(x, w, near, swiglu=swiglu)
+        kernels.gemm_stages(xf, wf, out, swiglu=swiglu)
+        assert torch.equal(out, near)
+    near, out = (torch.full((3, m, n), float("nan"), device=DEV) for _ in range(2))
+    kernels.gemm_stages(x, w, near)
+    kernels.gemm_stages(xf, wf, out)
+    assert torch.equal(out, near)
