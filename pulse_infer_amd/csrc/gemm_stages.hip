@@ -4,8 +4,8 @@
 //
 // What bounds it: the bytes that the fullest compute unit copies into LDS.  A unit takes in 28 to 54 bytes a nanosecond over a
 // launch, least where they are weights that come from memory, and the matrix cores are busy for 13 to 46 % of it, LDS waits
-// make 1 to 6 % (counters at 97, 357 and 509 rows; from 300 rows on the power limit comes near: 357 rows of gate + up take 57 us with
-// operands of zeros, 70 to 73 with others), so the shape and the shares of K are chosen for the least bytes
+// make 1 to 6 % (counters at 97, 357 and 509 rows; from 300 rows on the power limit comes near: 357 rows of gate + up take 58 us with
+// operands of zeros, 62 to 65 with others, 2,048 rows 224 and 284), so the shape and the shares of K are chosen for the least bytes
 // (`plan_for`).  Measured alone with weights from memory, us, against the vendor library's product (gate and up: with its
 // pass for SwiGLU behind it) and this package's shared-out product for up to 192 rows; in brackets behind a figure, what it
 // takes inside a step, between other kernels and with the chip warm:
@@ -171,10 +171,12 @@ struct Plan { int shape, splits; double ns; };
 // row of a stage (128 bytes) takes a compute unit 3.1 ns.  Tiles of more than 128 rows of X hold weights long enough for
 // their further rounds to find them near: 2 ns a row then, or what its products take on the matrix cores (1.13 x their
 // time at the rate of a large product, 5.5 flops a picosecond a unit), and 0.75 of that for a last round that leaves half
-// the units idle.  Every share adds its results' way to memory and back to whoever adds them up (8 bytes a value at 4
-// TB/s).  Estimated / measured, 24,576 x 4,096 with SwiGLU, us: 97 rows 96 x 128 44 / 44, 128 x 128 51 / 50; 357 rows
-// 192 x 192 76 / 71, 192 x 256 89 / 82; 509 rows 192 x 256 89 / 87, 256 x 256 111 / 104, 192 x 192 123 / 120; 700 rows
-// 192 x 192 139 / 132, 192 x 256 151 / 152; 1,024 rows 192 x 256 172 / 181.
+// the units idle.  Beyond 512 rows, where several tiles read a weight's rows, large tiles take 2.6 ns a row from the first round on, or
+// 0.94 x their products' time, and small ones 3.5.  Every share adds its results' way to memory and back to whoever adds them up (8
+// bytes a value at 4 TB/s).  Estimated / measured, 24,576 x 4,096 with SwiGLU, us: 97 rows 96 x 128 44 / 38, 128 x 128 51 / 41; 357 rows
+// 192 x 192 76 / 62, 192 x 256 89 / 78; 512 rows 192 x 256 89 / 80, 256 x 256 111 / 85; 1,024 rows 192 x 256 149 / 157; 2,048 rows 256 x 256
+// 269 / 284.  (Which shape is best follows from it: over the 288 sizes measured from 257 rows on, of 18 weights, its choices take
+// 0.3 % longer than the best shape's; without the figures for 512 rows and more 0.6 %, and shares of K that pay were not seen.)
 Plan plan_for(int M, int N, int K, int shares) {
     const int64_t units = pulse_compute_units();
     Plan best{0, 1, 0.0};
@@ -185,10 +187,12 @@ Plan plan_for(int M, int N, int K, int shares) {
             const int wr = SHAPES[i][0], xr = SHAPES[i][1];
             const int64_t tiles = static_cast<int64_t>((M + xr - 1) / xr) * ((N + wr - 1) / wr) * splits;
             const int64_t rounds = (tiles + units - 1) / units, last = tiles - (rounds - 1) * units;
-            double row = rounds * 3.1;
+            const bool many = M > 512;
+            double row = rounds * (many ? 3.5 : 3.1);
             if (xr > 128) {
-                const double later = std::max(2.0, 1.13 * wr * xr * 128.0 / (wr + xr) / 5500.0);
-                row = std::max(3.1, later) + (rounds - 1) * later - (rounds > 1 && 2 * last <= units ? 0.25 * later : 0.0);
+                const double later = std::max(many ? 2.6 : 2.0, (many ? 0.94 : 1.13) * wr * xr * 128.0 / (wr + xr) / 5500.0);
+                row = std::max(many ? 2.6 : 3.1, later) + (rounds - 1) * later;
+                if (rounds > 1 && 2 * last <= units) row -= (many ? 0.2 : 0.25) * later;
             }
             const double ns = row * (wr + xr) * (K / splits / 64) + (shares == 1 ? 0.0 : splits * 8.0 / 4000.0 * M * N);
             if (!any || ns < best.ns) { best = {i, splits, ns}; any = true; }
@@ -231,29 +235,58 @@ extern "C" int pulse_gemm_stages_time(int M, int N, int K) {
     return pulse_gemm_stages_takes(M, N, K, OUT_BF16, 1) ? static_cast<int>(std::min(plan_for(M, N, K, 1).ns, 2e9)) : 0;
 }
 
+// What both products check before they launch: operands there and aligned, rows that hold K values, results that hold N.
+static int check_operands(const char* name, const void* X, int64_t ldx, const void* W, int64_t ldw, const void* C, int64_t ldc, int M, int N,
+                          int K, int mode, int splits, int64_t part_stride) {
+    PULSE_REQUIRE(pulse_gemm_stages_takes(M, N, K, mode, splits),
+                  "%s: %d rows x %d weight rows x inner dimension %d, mode %d, %d shares: the inner dimension must "
+                  "be a multiple of 64 a share, the weight rows a multiple of 8 (32 with SwiGLU, 4 for float32 results), "
+                  "shares need float32 results", name, M, N, K, mode, splits);
+    PULSE_REQUIRE(X && W && C && aligned16(X) && aligned16(W) && aligned16(C), "%s: operands must be aligned to 16 bytes", name);
+    PULSE_REQUIRE(ldx >= K && ldw >= K && ldx % 8 == 0 && ldw % 8 == 0, "%s: rows of X and W must be K long at "
+                  "least and start at multiples of 16 bytes (strides %lld, %lld)", name, (long long)ldx, (long long)ldw);
+    const int out_cols = mode == OUT_SWIGLU ? N / 2 : N;
+    PULSE_REQUIRE(ldc >= out_cols && ldc % (mode == OUT_F32 ? 4 : 8) == 0, "%s: rows of the result must be %d long "
+                  "at least and start at multiples of 16 bytes (stride %lld)", name, out_cols, (long long)ldc);
+    PULSE_REQUIRE(splits == 1 || (part_stride >= static_cast<int64_t>(M - 1) * ldc + N && part_stride % 4 == 0),
+                  "%s: the shares' results overlap (stride %lld)", name, (long long)part_stride);
+    return 0;
+}
+
+static void launch_mode(int mode, int shape, const StageArgs& a, hipStream_t stream) {
+    if (mode == OUT_BF16) launch_shape<OUT_BF16>(shape, a, stream);
+    else if (mode == OUT_SWIGLU) launch_shape<OUT_SWIGLU>(shape, a, stream);
+    else launch_shape<OUT_F32>(shape, a, stream);
+}
+
 // mode 0: C [M, N] bfloat16.  mode 1: the rows of W alternate in slabs of 16 gate rows and their 16 up rows;
 // C [M, N / 2] bfloat16 = silu(gate) * up.  mode 2: float32, one result [M, N] for every share of K, `part_stride`
 // elements apart (the shares are added up by whoever reads them, in order).
 extern "C" int pulse_gemm_stages(const void* X, int64_t ldx, const void* W, int64_t ldw, void* C, int64_t ldc, int M, int N,
                                  int K, int mode, int splits, int64_t part_stride, hipStream_t stream) {
-    PULSE_REQUIRE(pulse_gemm_stages_takes(M, N, K, mode, splits),
-                  "gemm_stages: %d rows x %d weight rows x inner dimension %d, mode %d, %d shares: the inner dimension must "
-                  "be a multiple of 64 a share, the weight rows a multiple of 8 (32 with SwiGLU, 4 for float32 results), "
-                  "shares need float32 results", M, N, K, mode, splits);
-    PULSE_REQUIRE(X && W && C && aligned16(X) && aligned16(W) && aligned16(C), "gemm_stages: operands must be aligned to 16 bytes");
-    PULSE_REQUIRE(ldx >= K && ldw >= K && ldx % 8 == 0 && ldw % 8 == 0, "gemm_stages: rows of X and W must be K long at "
-                  "least and start at multiples of 16 bytes (strides %lld, %lld)", (long long)ldx, (long long)ldw);
-    const int out_cols = mode == OUT_SWIGLU ? N / 2 : N;
-    PULSE_REQUIRE(ldc >= out_cols && ldc % (mode == OUT_F32 ? 4 : 8) == 0, "gemm_stages: rows of the result must be %d long "
-                  "at least and start at multiples of 16 bytes (stride %lld)", out_cols, (long long)ldc);
-    PULSE_REQUIRE(splits == 1 || (part_stride >= static_cast<int64_t>(M - 1) * ldc + N && part_stride % 4 == 0),
-                  "gemm_stages: the shares' results overlap (stride %lld)", (long long)part_stride);
-    StageArgs a{static_cast<const bf16_t*>(X), ldx, static_cast<const bf16_t*>(W), ldw, C, ldc, M, N, K / splits, 0, 0, splits,
-                splits > 1 ? part_stride : 0};
-    const int shape = plan_for(M, N, K, splits).shape;
-    if (mode == OUT_BF16) launch_shape<OUT_BF16>(shape, a, stream);
-    else if (mode == OUT_SWIGLU) launch_shape<OUT_SWIGLU>(shape, a, stream);
-    else launch_shape<OUT_F32>(shape, a, stream);
+    if (const int bad = check_operands("gemm_stages", X, ldx, W, ldw, C, ldc, M, N, K, mode, splits, part_stride)) return bad;
+    launch_mode(mode, plan_for(M, N, K, splits).shape,
+                {static_cast<const bf16_t*>(X), ldx, static_cast<const bf16_t*>(W), ldw, C, ldc, M, N, K / splits, 0, 0, splits,
+                 splits > 1 ? part_stride : 0}, stream);
     PULSE_LAUNCH_CHECK("gemm_stages");
+    return 0;
+}
+
+// The same in tiles of 256 x 256 whatever the rows (fewer sizes: at most 2^24 tiles, rows less than 4M values apart).
+extern "C" int pulse_gemm_tile_takes(int M, int N, int K, int mode, int splits) {
+    if (!pulse_gemm_stages_takes(M, N, K, mode, splits)) return 0;
+    return static_cast<int64_t>((M + 255) / 256) * ((N + 255) / 256) * splits <= (1 << 24);
+}
+
+extern "C" int pulse_gemm_tile(const void* X, int64_t ldx, const void* W, int64_t ldw, void* C, int64_t ldc, int M, int N,
+                               int K, int mode, int splits, int64_t part_stride, void* stream) {
+    if (const int bad = check_operands("gemm_tile", X, ldx, W, ldw, C, ldc, M, N, K, mode, splits, part_stride)) return bad;
+    PULSE_REQUIRE(pulse_gemm_tile_takes(M, N, K, mode, splits) && ldx < FAR_ROWS && ldw < FAR_ROWS,
+                  "gemm_tile: at most 2^24 tiles, and rows of X and W less than 4M elements apart (strides %lld, %lld)",
+                  (long long)ldx, (long long)ldw);
+    launch_mode(mode, NUM_SHAPES - 1,
+                {static_cast<const bf16_t*>(X), ldx, static_cast<const bf16_t*>(W), ldw, C, ldc, M, N, K / splits, 0, 0, splits,
+                 splits > 1 ? part_stride : 0}, static_cast<hipStream_t>(stream));
+    PULSE_LAUNCH_CHECK("gemm_tile");
     return 0;
 }

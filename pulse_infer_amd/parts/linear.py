@@ -4,14 +4,14 @@ Four products stand behind it:
 
 * few rows (decoding, short portions) of bfloat16: this package's weight-streaming
   matrix-core kernel, which can also add into the float32 residual or apply SwiGLU;
-* 65 rows to some hundreds of bfloat16: this package's product with several stages of its
-  operands on their way through LDS (``takes_stages`` says where it is the faster one);
-* more rows of bfloat16: the vendor library's product (torch.matmul / torch.mm,
-  i.e. hipBLASLt/rocBLAS, float32 accumulation, bfloat16 or float32 output), as
-  the reference uses cuBLAS (src/ops/kernels/cuda/matmul_kernel.cu:132-154), or this
-  package's product in output tiles of 256 x 256, which can apply SwiGLU on the way
-  out or leave float32 results of shares of the inner dimension (``OWN_MANY_ROWS``
-  says which products go there);
+* 65 rows and more of bfloat16: this package's product with several stages of its
+  operands on their way through LDS, which can apply SwiGLU on the way out or leave
+  float32 results of shares of the inner dimension (``takes_stages`` and
+  ``stage_shares_for`` say where it is the faster one);
+* else the vendor library's product (torch.matmul / torch.mm, i.e. hipBLASLt/rocBLAS,
+  float32 accumulation, bfloat16 or float32 output), as the reference uses cuBLAS
+  (src/ops/kernels/cuda/matmul_kernel.cu:132-154); ``OWN_MANY_ROWS`` says which
+  products of many rows go where;
 * the float32 run, and any weight kept in 32-bit: this package's own kernel on the
   float32 matrix instruction, with no reduced-precision mode anywhere.
 """
@@ -28,15 +28,12 @@ from .base import LazyNorm, RowStats, Workspace
 
 
 # Which products of many rows (256 and more) run as this package's instead of the library's: "stages", the product in
-# stages where it is the faster one (``takes_stages``); or the tiled product, "swiglu": for gate and up with SwiGLU inside,
-# which saves the pass over twice the feed-forward's width (the others as with "stages"), "all": for every product of
-# bfloat16 (a step then makes no library call); "none": none of them.  (Products of fewer rows are not its business: 65 to 255
+# stages where it is the faster one (``takes_stages``); or the same in tiles of 256 x 256 throughout, "swiglu": for gate and up with
+# SwiGLU inside (the others as with "stages"), "all": for every product of bfloat16 (a step then makes no library call); "none": none of
+# them.  (Products of fewer rows are not its business: 65 to 255
 # of them run in stages, where that is the faster one, whatever it says.)  PULSE_OWN_PRODUCTS sets it.
-# Measured: a prompt of 509 tokens of the 8B shape 9.0 ms with "stages", 11.3 with "none" (whose updates in shares are made one
-# after the other, see ``add_into``; 9.6 before, side by side).  Through the serving loop, a prompt of
-# 2,048 tokens 73.9K tokens/s with "none", 72.9K with "swiglu", 71.6K with "all" (alone and with the chip warm, gate+up
-# with SwiGLU inside takes 310 us against the library's 328 + 30 for the pass; between the other kernels of a step the
-# library's product takes 278): prompts of that size make no updates in shares.  So the library stays for the largest.
+# Measured, prompts of the 8B shape: 509 tokens 8.7 ms with "stages", 11.3 with "none" (whose updates in shares are made one
+# after the other, see ``add_into``); 2,048 tokens 24.9 with "stages", 26.9 with "none"; 8,192 106.5 and 108.8.
 OWN_MANY_ROWS = os.environ.get("PULSE_OWN_PRODUCTS", "stages")
 if OWN_MANY_ROWS not in ("none", "stages", "swiglu", "all"):
     raise ValueError(f"PULSE_OWN_PRODUCTS must be none, stages, swiglu or all, not '{OWN_MANY_ROWS}'")
@@ -220,9 +217,10 @@ class Linear:
         """Whether an update of more than 192 rows has so few output tiles and so wide an inner dimension that it is to be
         made in shares beyond the sizes that go in stages anyway, and into how many the library's is cut (``OWN_MANY_ROWS``
         "none"); 0: not at all.  Measured (8B, 14B and 32B shapes of down, 272 to 2,048 rows): up to about 100 tiles shares
-        win (14B shape at 544 rows 179 -> 102 us with the library's products side by side, 90 in stages); the 8B shape at
-        2,048 rows gains in the product (182 -> 157 us) what the wider update costs again in the norm that adds it up;
-        products with an inner dimension of 4,096 to 8,192 (o) gain 5 us at most."""
+        win (14B shape at 544 rows 179 -> 102 us with the library's products side by side, 84 in stages); in stages also while two
+        shares fill the chip once, half as many tiles as compute units (us, shares with their cost in the next norm / the library's:
+        4,096 x 12,288 at 2,048 rows 150 / 175, 5,120 x 17,408 at 1,536 203 / 349, 2,560 x 9,728 at 3,000 116 / 133; beyond, 5,120 x
+        17,408 at 2,048 303 / 273, 5,120 x 8,192 159 / 134).  Products with an inner dimension of 4,096 to 8,192 (o) gain 5 us at most."""
         rows = x.shape[0]
         if not (self.library and x.dtype == torch.bfloat16 and rows > self.SHARES_ROWS[1]
                 and self.in_features >= self.LIBRARY_SHARES_MIN_K and x.is_contiguous()
@@ -230,7 +228,7 @@ class Linear:
             return 0
         tile = self.LIBRARY_TILE
         tiles = ((rows + tile - 1) // tile) * ((self.out_features + tile - 1) // tile)
-        splits = 4 if tiles <= 50 else (2 if tiles <= 100 else 0)
+        splits = 4 if tiles <= 50 else (2 if tiles <= (100 if OWN_MANY_ROWS == "none" else compute_units() // 2) else 0)
         while splits > 1 and (self.in_features % splits or (self.in_features // splits) % 64):
             splits //= 2
         return splits if splits > 1 else 0
@@ -259,22 +257,18 @@ class Linear:
             return out.is_contiguous() and out.data_ptr() % 16 == 0 and w.shape[0] % 4 == 0
         return out.dtype == torch.bfloat16 and out.stride(1) == 1 and out.stride(0) % 4 == 0 and out.data_ptr() % 16 == 0
 
-    # Where the product in stages is the fastest (more figures are beside its kernel).  With SwiGLU inside: up to 768 rows
-    # where a compute unit gets 192 weight rows at most (gate and up of 24,576 x 4,096 at
-    # 357, 512 and 700 rows 74, 97 and 139 us, the library's product and the pass behind it 97, 105 and 165; of 34,816 x
-    # 5,120 153, 196 and 247 against 171, 201 and 282; of 51,200 x 5,120, wider than that, 202, 312 and 384 against 212,
-    # 279 and 396); otherwise, up to 1,536 rows, where its tiles fill their rounds, which its estimate tells: at least 1.1
-    # PFLOP/s (24,576 x 4,096 at 1,024 rows 176 against 184, but at 800 173 against 154; 34,816 x 5,120 at 1,024 322
-    # against 410).  Plain products: see ``fills_stages``.  Updates in shares: up to 512 rows all that are not small (4,096 x 4,096 at 512 rows 25 us against
-    # the library's 31, 2,560 x 9,728 at 357 27 against 41), beyond those of a wide inner dimension and few tiles
-    # (``library_shares_for``): us without the norm behind, rows 544 / 768 / 1,024: 4,096 x 12,288 65 / 69 / 90, 5,120 x 17,408
-    # 90 / 122 / 162 (the library's in shares side by side 102 at 544).  Small products stay where they are.
+    # Where the product in stages is the fastest (more figures are beside its kernel).  With SwiGLU inside: wherever it takes the
+    # shape (us against the library's product and the pass behind it: 24,576 x 4,096 at 357 / 512 / 800 / 2,048 / 8,192 rows 62 / 80 /
+    # 147 / 284 / 1,116 against 91 / 104 / 165 / 337 / 1,305; 34,816 x 5,120 at 544 / 2,048 183 / 549 against 218 / 664; 51,200 x 5,120 at
+    # 300 / 640 / 4,096 185 / 318 / 1,472 against 203 / 359 / 1,880; 19,456 x 2,560 at 257 / 3,000 40 / 231 against 54 / 290).  Plain products:
+    # see ``fills_stages``.  Updates in shares: up to 512 rows all that are not small (4,096 x 4,096 at 512 rows 25 us against
+    # the library's 28, 2,560 x 9,728 at 357 28 against 40), beyond those of a wide inner dimension and few tiles
+    # (``library_shares_for``).  Small products stay where they are.
     STAGE_ROWS = (65, 256)              # with SwiGLU and in shares any of these (the last one if ``OWN_MANY_ROWS`` leaves it to it)
-    STAGE_ROWS_SWIGLU = (768, 1536)
-    STAGE_SWIGLU_RATE = 1100            # flops a nanosecond
+    STAGE_ROWS_SWIGLU = (256, 1 << 30)
     STAGE_ROWS_SHARES = 512             # beyond, only where ``library_shares_for`` says so
     STAGE_CUT_ROWS = 128                # the rows that updates of up to 192 rows are cut into shares for
-    STAGE_ROWS_NARROW = 1024            # plain products of at most 32 weight rows a compute unit
+    STAGE_RATE = 875                    # plain products of more rows: estimated flops a picosecond
     STAGE_MIN_WEIGHT = 1 << 22
 
     def takes_stages(self, x: torch.Tensor, w: Optional[torch.Tensor] = None, swiglu: bool = False) -> bool:
@@ -287,12 +281,7 @@ class Linear:
             return False
         if rows >= self.TILE_MIN_ROWS and (OWN_MANY_ROWS == "none" or self.takes_tiles(x, w, swiglu)):
             return False
-        if not swiglu:
-            return self.fills_stages(rows, n, k)
-        if rows <= self.STAGE_ROWS[1]:
-            return True
-        return ((n <= 192 * compute_units() and rows <= self.STAGE_ROWS_SWIGLU[0])
-                or kernels.gemm_stages_time(rows, n, k) * self.STAGE_SWIGLU_RATE <= 2 * rows * n * k)
+        return swiglu or self.fills_stages(rows, n, k)
 
     def fills_stages(self, rows: int, n: int, k: int) -> bool:
         """Whether a plain product's tiles keep enough compute units busy: its inner dimension cannot be cut (the result is
@@ -303,8 +292,15 @@ class Linear:
         4,096 x 4,096 at 97 (0.50) 16 / 18, 10,240 x 5,120 at 97 (0.62) 34 / 39; 6,144 x 4,096 at 97 (0.75) 23 / 19, 4,096 x 4,096
         at 160 (0.75) 27 / 19, 7,168 x 4,096 at 192 (0.88) 35 / 28, 8,192 x 2,048 at 224 (1.0) 24 / 17; of 2,048 columns and
         fewer already 3,072 x 2,048 at 97 (0.38) 12 / 11, 4,096 x 1,024 at 65 (0.50) 11 / 7.  Beyond 256 rows the library's own
-        tiles fill: 4,096 x 4,096 at 700 (0.75) 35 / 39, 8,192 x 8,192 at 333 (0.75) 66 / 75, 6,144 x 2,560 at 300 (0.94) 22 / 24, but 6,144 x 4,096 at 357 (0.75, tiles
-        of 96 x 128) 38 / 33, 8,192 x 2,048 at 300 (0.75) 24 / 21, 6,144 x 4,096 at 512 (1.0) 39 / 37.  (The library's times jump with the rows,
+        tiles fill: 8,192 x 8,192 at 333 (0.75) 66 / 75, 6,144 x 2,560 at 300 (0.94) 22 / 24, but 6,144 x 4,096 at 357 (0.75, tiles
+        of 96 x 128) 36 / 32, 8,192 x 2,048 at 300 (0.75) 24 / 21, 6,144 x 4,096 at 512 (1.0) 37 / 34.
+
+        Beyond 512 rows its estimate decides, that is how far its tiles fill their rounds and how large they are (estimated flops a
+        picosecond: us, library / this): 4,096 x 8,192 at 1,536 (807) 92 / 102, 2,048 x 2,048 at 1,536 (449) 19 / 23, 5,120 x 5,120 at 800
+        (525) 57 / 59, 10,240 x 5,120 at 544 (714) 64 / 69; 6,144 x 4,096 at 1,200 (945) 57 / 57, 1,536 (1,210) 70 / 59, 2,048 (1,383) 81 / 74
+        and 8,192 (1,498) 267 / 276, 5,120 x 5,120 at 1,536 (1,008) 76 / 70 and 8,192 (1,337) 454 / 309, 10,240 x 5,120 at 1,200 (1,097) 128 /
+        107, 4,096 x 4,096 at 2,048 (1,075) 59 / 57.  Over the sizes measured beyond 512 rows the rule comes to 0.967 of the library's
+        time.  (The library's times jump with the rows,
         28 us at 255 and 42 at 256 for 6,144 x 4,096, so a rule of sizes leaves some on the wrong side: 5 to 15 % at a twentieth of the 375
         sizes measured, 6,144 x 2,560 at 255 20 / 23, 4,608 x 3,072 at 444 25 / 29.)"""
         tile_n, tile_m = kernels.gemm_stages_tile(rows, n, k)
@@ -312,10 +308,9 @@ class Linear:
         fill = tiles / (((tiles + units - 1) // units) * units)
         if rows <= self.STAGE_ROWS[1]:
             return fill >= 0.7 or (k <= 2048 and fill >= 0.33)
-        if n > 32 * units or rows > self.STAGE_ROWS_NARROW:
-            return False
-        return fill >= 0.95 or (rows <= self.STAGE_ROWS_SHARES and fill >= 0.7
-                                and (k <= 2048 or (k <= 4096 and tile_n * tile_m >= 96 * 128)))
+        if rows > self.STAGE_ROWS_SHARES:
+            return kernels.gemm_stages_time(rows, n, k) * 1000 * self.STAGE_RATE <= 2 * rows * n * k
+        return n <= 32 * units and (fill >= 0.95 or (fill >= 0.7 and (k <= 2048 or (k <= 4096 and tile_n * tile_m >= 96 * 128))))
 
     def stage_shares_for(self, x: torch.Tensor) -> int:
         """Into how many shares of the inner dimension the product in stages cuts an update that the next norm adds up; 0:
