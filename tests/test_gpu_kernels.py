@@ -782,6 +782,13 @@ def test_attn_mfma(k, case, split):
     _mfma_case(k, split=split, **case)
 
 
+# several heads a workgroup of the merge (2 to 8 splits, by the head size), one; a split a lane, one more, and many
+@pytest.mark.parametrize("d", [16, 112, 128, 224])
+@pytest.mark.parametrize("splits", [2, 3, 4, 5, 8, 9, 33, 63, 64, 65, 150])
+def test_attn_mfma_merges_any_number_of_splits(k, splits, d):
+    _mfma_case(k, nq=6, nkv=2, d=d, bs=16, window=0, lens=[splits * 32 - 3, 1, 32, 33, splits * 16 + 1], portion=1, split=32)
+
+
 @pytest.mark.parametrize("case", [
     dict(nq=32, nkv=8, d=128, bs=16, window=0, lens=[300, 513, 512, 31], portion=3),
     dict(nq=6, nkv=3, d=48, bs=32, window=24, lens=[170, 90, 24, 25], portion=1),
