@@ -456,13 +456,16 @@ __global__ __launch_bounds__(WN* WM* PULSE_WAVE) void moe_tile_kernel(GroupArgs 
                     for (int i = 0; i < 4; ++i) {
                         // an expert that is fed weight * x: both products are linear, so the factor goes onto their results
                         float gate = loop.acc[f][g][i] * wgt, up = loop.acc[f + 1][g][i] * wgt;
+                        float slope = 1.0f;
                         if (a.act_kind == 1) {   // clamped: min(g, limit) * sigmoid(1.702 g) * (clamp(u) + 1)
                             gate = fminf(gate, a.limit);
-                            up = fminf(fmaxf(up, -a.limit), a.limit);
-                            v[i] = (__bf16)(gate / (1.0f + expf(-1.702f * gate)) * (up + 1.0f));
-                        } else {
-                            v[i] = (__bf16)(gate / (1.0f + expf(-gate)) * up);
+                            up = fminf(fmaxf(up, -a.limit), a.limit) + 1.0f;
+                            slope = 1.702f;
                         }
+                        // (as in the products in stages: the reciprocal of a quarter is a normal number as long as the exponential is
+                        // finite; expf and a division, no nearer to 64 bits behind the rounding, took 12 us more: 16 experts of
+                        // 1,536 x 4,096, 8,192 pairs, 209 -> 197 us.)
+                        v[i] = (__bf16)(0.25f * gate * __builtin_amdgcn_rcpf(fmaf(0.25f, __expf(-slope * gate), 0.25f)) * up);
                     }
                     *reinterpret_cast<tile_bf16x4*>(at + f * 16) = v;
                 }

@@ -116,3 +116,29 @@ def test_grouped_experts_with_room_for_more_pairs_than_offsets_reach():
         kernels.call("pulse_moe_down_grouped", p(act), p(wd), *lists, i32(tiles), i32(rows), p(y), i32(hidden), i32(ff), kernels._stream())
         out, size = (torch.einsum("tf,thf->th", a, b) for a, b in ((got, wd.cpu().to(F64)[e]), (got.abs(), wd.cpu().to(F64)[e].abs())))
         assert ((y.cpu().to(F64) - out).abs() <= (ff + 4) * 2.0 ** -24 * size).all(), tiles
+
+
+@pytest.mark.parametrize("hidden,ff", [(64, 64), (1024, 448)])
+@pytest.mark.parametrize("form", ["silu", "clamped_on_input"])
+def test_grouped_experts_do_not_depend_on_the_tiles_of_their_rows(hidden, ff, form):
+    """Lists of 32, 64, 128 and 192 rows, and what their last tiles are rounded up to: the same bits."""
+    from pulse_infer_amd.ops import kernels
+
+    counts = [1, 31, 33, 63, 64, 65, 96, 127, 128, 129, 191, 193, 192 + 64, 192 + 65, 320, 321, 0, 384 + 128]
+    experts, pairs = len(counts), sum(counts)
+    idx = torch.cat([torch.full((c,), e, dtype=torch.int32) for e, c in enumerate(counts)]).view(pairs, 1).to(DEV)
+    x = rnd(pairs, hidden, seed=2).to(torch.bfloat16).to(DEV)
+    wg, wu = ((rnd(experts, ff, hidden, seed=3 + i) * hidden ** -0.5).to(torch.bfloat16).to(DEV) for i in range(2))
+    wd = (rnd(experts, hidden, ff, seed=5) * ff ** -0.5).to(torch.bfloat16).to(DEV)
+    weight = torch.rand(pairs, 1, generator=torch.Generator().manual_seed(6)).to(DEV) + 0.5
+    kw = dict(weight_on_input=True, activation="clamped_swish", limit=0.8) if form != "silu" else {}
+    results = []
+    for rows in (32, 64, 128, 192):
+        act = torch.full((pairs, ff), float("nan"), dtype=torch.bfloat16, device=DEV)
+        y = torch.full((pairs, hidden), float("nan"), device=DEV)
+        ints = torch.full((2 * pairs + 3 * kernels.moe_max_tiles(pairs, experts, rows) + 1,), -5, dtype=torch.int32, device=DEV)
+        kernels.moe_grouped(x, wg, wu, wd, idx, weight, act, y, None, ints, rows, **kw)
+        results.append((act, y))
+    assert not torch.isnan(results[0][0]).any() and not torch.isnan(results[0][1]).any()
+    for act, y in results[1:]:
+        assert torch.equal(act, results[0][0]) and torch.equal(y, results[0][1])
