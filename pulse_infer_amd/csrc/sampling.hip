@@ -196,6 +196,37 @@ __device__ int wave_walk(int begin, int end, float rest, Weight weight, int& las
     return -1;
 }
 
+// The same over STEPS * 64 weights in LDS whose steps' sums (as pairs_sum makes them) are there, step q's in lane q.
+template <int STEPS>
+__device__ int wave_walk_summed(const float* weights, float sums, float rest, int& last) {
+    const int lane = threadIdx.x % PULSE_WAVE;
+    float run = 0.f;
+    last = -1;
+    for (int q = 0; q < STEPS; ++q) {
+        const float sum = __uint_as_float(static_cast<uint32_t>(__builtin_amdgcn_readlane(__float_as_int(sums), q)));
+        if (sum == 0.f) continue;      // (no weight above zero)
+        if (!(rest < (run + sum) * 1.00001f)) {
+            run += sum;
+            continue;
+        }
+        const float w = weights[q * PULSE_WAVE + lane];
+        float pre = w;
+#pragma unroll
+        for (int off = 1; off < PULSE_WAVE; off <<= 1) {
+            const float up = __shfl_up(pre, off, PULSE_WAVE);
+            if (lane >= off) pre += up;
+        }
+        const unsigned long long hit = __ballot(w > 0.f && rest < run + pre);
+        if (hit != 0ull) return q * PULSE_WAVE + __builtin_ctzll(hit);
+        run += __shfl(pre, PULSE_WAVE - 1, PULSE_WAVE);
+    }
+    for (int q = STEPS - 1; q >= 0 && last < 0; --q) {
+        const unsigned long long has = __ballot(weights[q * PULSE_WAVE + lane] > 0.f);
+        if (has != 0ull) last = q * PULSE_WAVE + 63 - __builtin_clzll(has);
+    }
+    return -1;
+}
+
 constexpr int HIST_BINS = 2048;                         // bins of the value histogram that locates the k-th largest
 constexpr int WAVE_CAP = 128;                           // candidates a wavefront may collect
 constexpr int LIST_CAP = SAMPLE_WAVES * WAVE_CAP;       // candidates of a row
@@ -872,37 +903,6 @@ __device__ __forceinline__ float simple_row_max(const float* part_max, int chunk
     return best;
 }
 
-__global__ __launch_bounds__(SIMPLE_THREADS) void simple_mass_kernel(
-    const float* __restrict__ logits, int vocab, int64_t row_stride, const float* __restrict__ temperature,
-    const int* __restrict__ top_k,
-    const float* __restrict__ penalty, const int* __restrict__ seen_row, const uint32_t* __restrict__ seen_masks,
-    const uint32_t* __restrict__ banned, int mask_words, const float* __restrict__ part_max,
-    float* __restrict__ part_mass) {
-    __shared__ float sf[SIMPLE_THREADS / PULSE_WAVE];
-    const int r = blockIdx.y, chunk = blockIdx.x, chunks = gridDim.x;
-    const float temp = temperature ? temperature[r] : 0.f;
-    if (!(temp > 0.f)) return;   // the largest logit wins: no mass is asked for
-    if (top_k && top_k[r] > 0) return;   // what top-k keeps is weighed on the short list
-    const float best = simple_row_max(part_max + r * chunks, chunks);
-    if (best == -INFINITY) return;
-    const float inv_t = 1.0f / temp;
-    const RowView row = simple_row(logits, r, row_stride, vocab, penalty, seen_row, seen_masks, banned, mask_words);
-    const int begin = chunk * SIMPLE_CHUNK, end = min(vocab, begin + SIMPLE_CHUNK);
-    float mass = 0.f;
-    sweep<SIMPLE_CHUNK / SIMPLE_THREADS>(row, begin + static_cast<int>(threadIdx.x), end, SIMPLE_THREADS, [&](int, float x) {
-        if (x != -INFINITY) mass += expf((x - best) * inv_t);
-    });
-    const int lane = threadIdx.x % PULSE_WAVE, wave = threadIdx.x / PULSE_WAVE;
-    mass = wave_sum(mass);
-    if (lane == 0) sf[wave] = mass;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        float total = 0.f;
-        for (int w = 0; w < SIMPLE_THREADS / PULSE_WAVE; ++w) total += sf[w];
-        part_mass[r * chunks + chunk] = total;
-    }
-}
-
 // ---- rows with top-k, in chunks -------------------------------------------------------------------------------
 // With a small k the candidates can be found chunk by chunk as well.  The k-th largest of the chunks' maxima is a
 // lower bound of the k-th largest logit (that many logits, the maxima themselves, reach it), so everything that
@@ -916,44 +916,76 @@ constexpr int TOPK_SEGMENT = 32;   // candidates a chunk may leave
 // A row with top-p alone takes the same way with what lies at or above one of the lower chunk maxima (seven eighths
 // of the chunks have a larger one): some hundreds of the largest logits of a vocabulary of 150,000, which hold the
 // top_p share of a distribution as peaked as a language model's; if they do not (or a chunk has more than its segment
-// holds), the row is left to left_kernel too.  The mass of the whole row, which top_p refers to, comes from
-// simple_mass_kernel.
+// holds), the row is left to left_kernel too.  The mass of the whole row, which top_p refers to, is the chunks' masses'.
 __device__ __forceinline__ int top_p_bound_rank(int chunks) { return max(1, chunks - chunks / 8); }
 
-__global__ __launch_bounds__(SIMPLE_THREADS) void topk_collect_kernel(
+// Where a chunk's entries go that are taken, entry u * SIMPLE_THREADS + t being thread t's u-th: the number of those before it in that
+// order (vocabulary order), -1 for what is not taken; `total`: all of them.  Called by a whole workgroup, `counts` of its own each time.
+constexpr int CHUNK_PER = SIMPLE_CHUNK / SIMPLE_THREADS;
+__device__ __forceinline__ void chunk_places(const bool (&taken)[CHUNK_PER], int (*counts)[SIMPLE_THREADS / PULSE_WAVE], int (&place)[CHUNK_PER], int& total) {
+    constexpr int WAVES = SIMPLE_THREADS / PULSE_WAVE;
+    const int lane = threadIdx.x % PULSE_WAVE, wave = threadIdx.x / PULSE_WAVE;
+    unsigned long long has[CHUNK_PER];
+#pragma unroll
+    for (int u = 0; u < CHUNK_PER; ++u) {
+        has[u] = __ballot(taken[u]);
+        if (lane == u) counts[u][wave] = __builtin_popcountll(has[u]);
+    }
+    __syncthreads();
+    total = 0;
+#pragma unroll
+    for (int u = 0; u < CHUNK_PER; ++u) {
+        place[u] = total + __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(has[u] >> 32), __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(has[u]), 0u));
+#pragma unroll
+        for (int w = 0; w < WAVES; ++w) {
+            if (w < wave) place[u] += counts[u][w];
+            total += counts[u][w];
+        }
+        if (!taken[u]) place[u] = -1;
+    }
+}
+
+// A chunk's logits, entry u * SIMPLE_THREADS + t with thread t (-inf past the end), all asked for together.
+__device__ __forceinline__ void chunk_values(const RowView& row, int begin, float (&xs)[CHUNK_PER]) {
+    by_mask(row, [&](auto masked) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < CHUNK_PER; ++u) {
+            const int i = begin + u * SIMPLE_THREADS + static_cast<int>(threadIdx.x);
+            const float x = row.at<decltype(masked)::value>(min(i, row.vocab - 1));
+            xs[u] = i < row.vocab ? x : -INFINITY;
+        }
+    });
+}
+
+// What a chunk adds, the row's maxima known: its mass (rows without top-k) and its candidates (rows with top-k or top-p), from one reading
+// of its logits.  What bounds it: the trips to memory of 9 workgroups a unit; the logits are asked for first, in whole lines.  (Two
+// kernels, the candidates' a thread with eight neighbouring logits, 32 rows of 151,936: all options 5.6 + 11.0 us, 8.9 in one; top-p alone
+// 6.8 + 18.8 and 12.6.)
+__global__ __launch_bounds__(SIMPLE_THREADS) void chunk_kernel(
     const float* __restrict__ logits, int vocab, int64_t row_stride, const float* __restrict__ temperature,
     const int* __restrict__ top_k, const float* __restrict__ top_p, const float* __restrict__ penalty,
     const int* __restrict__ seen_row, const uint32_t* __restrict__ seen_masks, const uint32_t* __restrict__ banned,
-    int mask_words, const float* __restrict__ part_max, int* __restrict__ seg_i, float* __restrict__ seg_x,
+    int mask_words, const float* __restrict__ part_max, float* __restrict__ part_mass, int* __restrict__ seg_i, float* __restrict__ seg_x,
     int* __restrict__ seg_n) {
     constexpr int WAVES = SIMPLE_THREADS / PULSE_WAVE;
-    constexpr int PER = SIMPLE_CHUNK / SIMPLE_THREADS;   // consecutive logits a thread takes
-    __shared__ float s_bound;
-    __shared__ int s_count[WAVES];
+    __shared__ float s_bound, s_mass[WAVES];
+    __shared__ int s_count[CHUNK_PER][WAVES];
     const int r = blockIdx.y, chunk = blockIdx.x, chunks = gridDim.x;
     const int lane = threadIdx.x % PULSE_WAVE, wave = threadIdx.x / PULSE_WAVE;
-    int k = top_k ? top_k[r] : 0;
-    const float p = top_p ? top_p[r] : 0.f;
-    if (k <= 0 && p > 0.f && p < 1.f) k = top_p_bound_rank(chunks);   // top-p alone: see top_p_bound_rank
-    const float temp = temperature ? temperature[r] : 0.f;
-    int* my_n = seg_n + r * chunks + chunk;
-    if (!(temp > 0.f) || k <= 0 || k > chunks || chunks > 2 * PULSE_WAVE) {   // greedy rows need no candidates; the others are not for these kernels
-        if (threadIdx.x == 0) *my_n = 0;
-        return;
-    }
-    // the chunk's logits are asked for first: they travel while the bound is searched
+    const int own_k = top_k ? top_k[r] : 0;
+    const float p = top_p ? top_p[r] : 0.f, temp = temperature[r];
     const RowView row = simple_row(logits, r, row_stride, vocab, penalty, seen_row, seen_masks, banned, mask_words);
-    const int begin = chunk * SIMPLE_CHUNK + static_cast<int>(threadIdx.x) * PER;
-    float xs[PER];
-    by_mask(row, [&](auto masked) __attribute__((always_inline)) {
-#pragma unroll
-        for (int j = 0; j < PER; ++j) {
-            const int i = begin + j;
-            xs[j] = i < vocab ? row.at<decltype(masked)::value>(i) : -INFINITY;
-        }
-    });
-    // the k-th largest of the chunks' maxima, bit by bit (chunks <= 2 * 64: two a lane)
-    if (wave == 0) {
+    const bool any = top_k || top_p, weighed = temp > 0.f && own_k <= 0;      // (what top-k keeps is weighed on the short list)
+    const int k = own_k <= 0 && p > 0.f && p < 1.f ? top_p_bound_rank(chunks) : own_k;      // top-p alone: see top_p_bound_rank
+    int* my_n = seg_n + r * chunks + chunk;
+    // (greedy rows need no candidates; k beyond the chunks is not for these kernels)
+    const bool listed = any && temp > 0.f && k > 0 && k <= chunks && chunks <= 2 * PULSE_WAVE;
+    if (any && !listed && threadIdx.x == 0) *my_n = 0;
+    if (!listed && !weighed) return;
+    float xs[CHUNK_PER];
+    chunk_values(row, chunk * SIMPLE_CHUNK, xs);
+    const float best = simple_row_max(part_max + r * chunks, chunks);
+    if (listed && wave == 0) {     // the k-th largest of the chunks' maxima, bit by bit (chunks <= 2 * 64: two a lane)
         uint32_t keys[2];
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
@@ -975,34 +1007,35 @@ __global__ __launch_bounds__(SIMPLE_THREADS) void topk_collect_kernel(
         value = wave_max(value);
         if (lane == 0) s_bound = value;
     }
+    if (weighed && best != -INFINITY) {
+        const float inv_t = 1.0f / temp;
+        float mass = 0.f;
+#pragma unroll
+        for (int u = 0; u < CHUNK_PER; ++u)
+            if (xs[u] != -INFINITY) mass += expf((xs[u] - best) * inv_t);
+        mass = wave_sum(mass);
+        if (lane == 0) s_mass[wave] = mass;
+    }
     __syncthreads();
+    if (weighed && best != -INFINITY && threadIdx.x == 0) {
+        float total = 0.f;
+        for (int w = 0; w < WAVES; ++w) total += s_mass[w];
+        part_mass[r * chunks + chunk] = total;
+    }
+    if (!listed) return;
     const float bound = s_bound;
-    int mine = 0;
+    bool taken[CHUNK_PER];
 #pragma unroll
-    for (int j = 0; j < PER; ++j) mine += (xs[j] != -INFINITY && xs[j] >= bound) ? 1 : 0;
-    // where this thread's candidates go: an exclusive sum over the threads, in thread order (vocabulary order)
-    int pre = mine;
+    for (int u = 0; u < CHUNK_PER; ++u) taken[u] = xs[u] != -INFINITY && xs[u] >= bound;
+    int place[CHUNK_PER], total;
+    chunk_places(taken, s_count, place, total);
+    const int64_t segment = (static_cast<int64_t>(r) * chunks + chunk) * TOPK_SEGMENT;
 #pragma unroll
-    for (int off = 1; off < PULSE_WAVE; off <<= 1) {
-        const int up = __shfl_up(pre, off, PULSE_WAVE);
-        if (lane >= off) pre += up;
-    }
-    if (lane == PULSE_WAVE - 1) s_count[wave] = pre;
-    __syncthreads();
-    int at = pre - mine, total = 0;
-    for (int w = 0; w < WAVES; ++w) {
-        if (w < wave) at += s_count[w];
-        total += s_count[w];
-    }
-    int* out_i = seg_i + (static_cast<int64_t>(r) * chunks + chunk) * TOPK_SEGMENT;
-    float* out_x = seg_x + (static_cast<int64_t>(r) * chunks + chunk) * TOPK_SEGMENT;
-#pragma unroll
-    for (int j = 0; j < PER; ++j) {
-        if (xs[j] != -INFINITY && xs[j] >= bound) {
-            if (at < TOPK_SEGMENT) { out_i[at] = begin + j; out_x[at] = xs[j]; }
-            ++at;
+    for (int u = 0; u < CHUNK_PER; ++u)
+        if (place[u] >= 0 && place[u] < TOPK_SEGMENT) {
+            seg_i[segment + place[u]] = chunk * SIMPLE_CHUNK + u * SIMPLE_THREADS + static_cast<int>(threadIdx.x);
+            seg_x[segment + place[u]] = xs[u];
         }
-    }
     if (threadIdx.x == 0) *my_n = total;   // more than TOPK_SEGMENT: the row does not fit
 }
 
@@ -1033,15 +1066,20 @@ __device__ __forceinline__ void string_segments(const int* seg_i, const float* s
 enum { LEFT = 0, CHOSEN = 1, LEFT_COUNTED = 2, LEFT_ALONE = 3 };
 
 // What rest_kernel adds a row's histogram to, and that the row's token is not chosen.
-__device__ __forceinline__ void clear_rest(int* rest, int lane) {
-    for (int b = lane; b <= REST_CHOSEN; b += PULSE_WAVE) rest[b] = 0;
+__device__ __forceinline__ void clear_rest(int* rest) {
+    for (int b = threadIdx.x; b <= REST_CHOSEN; b += blockDim.x) rest[b] = 0;
 }
 
-// The choice of every row from what the kernels before left, a wavefront a row: the largest logit for greedy rows;
+// The choice of every row from what the kernels before left, a workgroup a row: the largest logit for greedy rows;
 // for rows with top-k the candidates' segments strung together in LDS and finished there; for rows that draw from the
 // whole vocabulary the chunk in which u * mass falls (chunk masses in chunk order), walked alone.  done[r] says
 // whether the row's token is chosen; the others (rows that did not fit) are left_kernel's.
-__global__ __launch_bounds__(PULSE_WAVE) void chunked_choose_kernel(
+// The four wavefronts fetch (segments, the walked chunk's logits and their weights) and make the steps' sums; what is chosen is one
+// wavefront's business, the others reach the same decisions up to there.  (A wavefront alone on its row waited out five trips to memory
+// for the segments and branched on every chunk's mass: 32 rows 20.6 -> 10.9 us at a temperature, 13.1 -> 10.6 with top-k 50, 21.7 -> 11.7
+// with all options.)
+constexpr int CHOOSE_THREADS = 256;
+__global__ __launch_bounds__(CHOOSE_THREADS) void chunked_choose_kernel(
     const float* __restrict__ logits, int vocab, int64_t row_stride, const float* __restrict__ temperature,
     const int* __restrict__ top_k, const float* __restrict__ top_p, const float* __restrict__ uniform,
     const float* __restrict__ penalty, const int* __restrict__ seen_row, const uint32_t* __restrict__ seen_masks,
@@ -1052,11 +1090,23 @@ __global__ __launch_bounds__(PULSE_WAVE) void chunked_choose_kernel(
     __shared__ int list_i[LIST_CAP];
     __shared__ float list_x[LIST_CAP];
     __shared__ int first_s[2 * PULSE_WAVE + 1];
-    const int r = blockIdx.x, lane = threadIdx.x;
+    constexpr int STEPS = SIMPLE_CHUNK / PULSE_WAVE, MINE = STEPS / (CHOOSE_THREADS / PULSE_WAVE);
+    static_assert(LIST_CAP >= SIMPLE_CHUNK && STEPS <= PULSE_WAVE, "a chunk's weights fit the list, its steps' sums a wavefront");
+    __shared__ float sums_s[STEPS];
+    const int r = blockIdx.x, lane = threadIdx.x % PULSE_WAVE, wave = threadIdx.x / PULSE_WAVE;
+    // (the row's options, and what its chunks left, are asked for together)
+    const float temp = temperature ? temperature[r] : 0.f;
+    const int k = top_k ? top_k[r] : 0;
+    const float p = top_p ? top_p[r] : 0.f;
+    const float u = temperature ? uniform[r] : 0.f;
+    const RowView row = simple_row(logits, r, row_stride, vocab, penalty, seen_row, seen_masks, banned, mask_words);
     part_max += r * chunks;
     part_idx += r * chunks;
     part_mass += r * chunks;
     seg_n += r * chunks;
+    const int at1 = lane + PULSE_WAVE;
+    const float mass0 = lane < chunks ? part_mass[lane] : 0.f, mass1 = at1 < chunks ? part_mass[at1] : 0.f;     // (a greedy row's: not written, not used)
+    const int n0 = lane < chunks ? seg_n[lane] : 0, n1 = at1 < chunks ? seg_n[at1] : 0;                         // (without top-k and top-p: nor these)
     // the largest logit, the lowest index among equals
     float best = -INFINITY;
     int best_i = 0x7fffffff;
@@ -1066,19 +1116,15 @@ __global__ __launch_bounds__(PULSE_WAVE) void chunked_choose_kernel(
         if (v > best || (v == best && i < best_i)) { best = v; best_i = i; }
     }
     wave_argmax(best, best_i);
-    const float temp = temperature ? temperature[r] : 0.f;
     if (best_i == 0x7fffffff || !(temp > 0.f)) {   // everything banned or NaN, or the largest logit wins
-        if (lane == 0) { out[r] = best_i == 0x7fffffff ? -1 : best_i; done[r] = 1; }
+        if (threadIdx.x == 0) { out[r] = best_i == 0x7fffffff ? -1 : best_i; done[r] = 1; }
         return;
     }
-    const int k = top_k ? top_k[r] : 0;
-    const float p = top_p ? top_p[r] : 0.f;
     const bool use_p = p > 0.f && p < 1.f;
     const float inv_t = 1.0f / temp;
     if (k > 0 || use_p) {
         const bool by_k = k > 0;
         // the segments' places in the list: an exclusive sum over the chunks, in chunk order (two chunks a lane)
-        const int n0 = lane < chunks ? seg_n[lane] : 0, n1 = lane + PULSE_WAVE < chunks ? seg_n[lane + PULSE_WAVE] : 0;
         const bool over = n0 > TOPK_SEGMENT || n1 > TOPK_SEGMENT;
         int pre0 = n0, pre1 = n1;
 #pragma unroll
@@ -1090,76 +1136,93 @@ __global__ __launch_bounds__(PULSE_WAVE) void chunked_choose_kernel(
         const int n = first + __shfl(pre1, PULSE_WAVE - 1, PULSE_WAVE);
         if (k > chunks || chunks > 2 * PULSE_WAVE || __ballot(over) != 0ull || n > LIST_CAP || n < k || n == 0) {
             // not a row for these kernels
-            if (lane == 0) done[r] = !by_k || k <= chunks * (TOPK_SEGMENT / 2) ? LEFT : vocab >= 1024 * static_cast<int64_t>(gridDim.x) ? LEFT_COUNTED : LEFT_ALONE;
-            if (left) clear_rest(left + static_cast<int64_t>(r) * REST_WORDS, lane);
+            if (threadIdx.x == 0) done[r] = !by_k || k <= chunks * (TOPK_SEGMENT / 2) ? LEFT : vocab >= 1024 * static_cast<int64_t>(gridDim.x) ? LEFT_COUNTED : LEFT_ALONE;
+            if (left) clear_rest(left + static_cast<int64_t>(r) * REST_WORDS);
             return;
         }
         float whole = 0.f;   // without top-k: the mass of the whole row, chunk masses in chunk order
         if (!by_k) {
-            for (int c = lane; c < chunks; c += PULSE_WAVE) whole += part_mass[c];
-            whole = wave_sum(whole);
+            whole = wave_sum(mass0 + mass1);     // (at most 2 * 64 chunks here)
         }
-        first_s[lane] = pre0 - n0;
-        first_s[lane + PULSE_WAVE] = first + pre1 - n1;
-        if (lane == 0) first_s[2 * PULSE_WAVE] = n;
+        if (wave == 0) {
+            first_s[lane] = pre0 - n0;
+            first_s[lane + PULSE_WAVE] = first + pre1 - n1;
+            if (lane == 0) first_s[2 * PULSE_WAVE] = n;
+        }
         __syncthreads();
         const int64_t segment = static_cast<int64_t>(r) * chunks * TOPK_SEGMENT;
-        string_segments<PULSE_WAVE>(seg_i + segment, seg_x + segment, first_s, chunks, list_i, list_x);
+        string_segments<CHOOSE_THREADS>(seg_i + segment, seg_x + segment, first_s, chunks, list_i, list_x);
         __syncthreads();
+        if (wave != 0) return;
         int token;
         const bool enough =   // (false only without top-k: the list does not hold top_p of the row)
             n <= 4 * PULSE_WAVE   // the usual case with top-k: a few dozen candidates, a few a lane; top-p alone has some hundreds
-                ? finish_on_list<4>(list_i, list_x, n, by_k, k, use_p, p, whole, best, inv_t, uniform[r], best_i, token)
+                ? finish_on_list<4>(list_i, list_x, n, by_k, k, use_p, p, whole, best, inv_t, u, best_i, token)
                 : n <= 12 * PULSE_WAVE
-                ? finish_on_list<12>(list_i, list_x, n, by_k, k, use_p, p, whole, best, inv_t, uniform[r], best_i, token)
-                : finish_on_list<LIST_PER_LANE>(list_i, list_x, n, by_k, k, use_p, p, whole, best, inv_t, uniform[r], best_i, token);
+                ? finish_on_list<12>(list_i, list_x, n, by_k, k, use_p, p, whole, best, inv_t, u, best_i, token)
+                : finish_on_list<LIST_PER_LANE>(list_i, list_x, n, by_k, k, use_p, p, whole, best, inv_t, u, best_i, token);
         if (lane == 0) {
             if (enough) out[r] = token;
             done[r] = enough ? 1 : 0;
         }
-        if (left && !__shfl(enough ? 1 : 0, 0, PULSE_WAVE)) clear_rest(left + static_cast<int64_t>(r) * REST_WORDS, lane);
+        if (left && !enough)      // (by this wavefront alone)
+            for (int b = lane; b <= REST_CHOSEN; b += PULSE_WAVE) left[static_cast<int64_t>(r) * REST_WORDS + b] = 0;
         return;
     }
     // a draw from the whole vocabulary: the chunk in which it falls, chunk masses in chunk order
-    float total = 0.f;
-    for (int c = lane; c < chunks; c += PULSE_WAVE) total += part_mass[c];
+    float total = mass0;
+    for (int c = lane + PULSE_WAVE; c < chunks; c += PULSE_WAVE) total += c < 2 * PULSE_WAVE ? mass1 : part_mass[c];
     total = wave_sum(total);
-    const float target = uniform[r] * total;
-    float run = 0.f;
+    const float target = u * total;
+    float run = 0.f, rest = 0.f;
     int who = -1, last_chunk = -1;
-    // (every lane the same few dozen additions; the masses come 64 at a time, one a lane, so that the additions do
-    // not each wait for a trip to memory)
+    // (every lane the same additions, 64 masses at a time, lane j keeping the sum before the j-th: a branch an addition took three times as long)
     for (int base = 0; base < chunks && who < 0; base += PULSE_WAVE) {
-        const float mine = base + lane < chunks ? part_mass[base + lane] : 0.f;
-        const int n = min(PULSE_WAVE, chunks - base);
-        for (int j = 0; j < n; ++j) {
-            const float m = __uint_as_float(static_cast<uint32_t>(__builtin_amdgcn_readlane(__float_as_int(mine), j)));
-            if (m > 0.f) {
-                last_chunk = base + j;
-                if (target < run + m) { who = base + j; break; }
-            }
-            run += m;
+        const float mine = base == 0 ? mass0 : base == PULSE_WAVE ? mass1 : base + lane < chunks ? part_mass[base + lane] : 0.f;
+        float before = 0.f;
+#pragma unroll 8
+        for (int j = 0; j < PULSE_WAVE; ++j) {
+            before = lane == j ? run : before;
+            run += __uint_as_float(static_cast<uint32_t>(__builtin_amdgcn_readlane(__float_as_int(mine), j)));
+        }
+        const unsigned long long has = __ballot(mine > 0.f), hit = __ballot(mine > 0.f && target < before + mine);
+        if (hit != 0ull) {
+            const int j = __builtin_ctzll(hit);
+            who = base + j;
+            rest = target - __shfl(before, j, PULSE_WAVE);
+        } else if (has != 0ull) {
+            last_chunk = base + 63 - __builtin_clzll(has);
         }
     }
-    float rest = target - run;
     if (who < 0 && last_chunk < 0) {      // (no weight is a number above zero)
-        if (lane == 0) { out[r] = best_i; done[r] = CHOSEN; }
+        if (threadIdx.x == 0) { out[r] = best_i; done[r] = CHOSEN; }
         return;
     }
     if (who < 0) {  // rounding left the target beyond the last chunk with mass: its last kept entry
         who = last_chunk;
         rest = INFINITY;
     }
-    const RowView row = simple_row(logits, r, row_stride, vocab, penalty, seen_row, seen_masks, banned, mask_words);
-    const int begin = who * SIMPLE_CHUNK, end = min(vocab, begin + SIMPLE_CHUNK);
-    int last, e;
+    // The chunk's walk, as wave_walk's: the wavefronts make the weights and the sums of a share of its steps each.
+    const int begin = who * SIMPLE_CHUNK;
+    float* const weights = list_x;
+    float ws[MINE];
     by_mask(row, [&](auto masked) __attribute__((always_inline)) {
-        e = wave_walk(begin, end, rest, [&](int i) {
-            const float x = row.at<decltype(masked)::value>(i);
-            return x != -INFINITY ? expf((x - best) * inv_t) : 0.f;
-        }, last);
+#pragma unroll
+        for (int j = 0; j < MINE; ++j) ws[j] = row.at<decltype(masked)::value>(min(begin + (wave * MINE + j) * PULSE_WAVE + lane, vocab - 1));
     });
-    if (lane == 0) { out[r] = e >= 0 ? e : (last >= 0 ? last : best_i); done[r] = 1; }
+#pragma unroll
+    for (int j = 0; j < MINE; ++j) {
+        const int at = (wave * MINE + j) * PULSE_WAVE + lane;
+        ws[j] = begin + at < vocab && ws[j] != -INFINITY ? expf((ws[j] - best) * inv_t) : 0.f;
+        weights[at] = ws[j];
+        const float sum = pairs_sum(ws[j]);
+        if (lane == 0) sums_s[wave * MINE + j] = sum;
+    }
+    __syncthreads();
+    if (wave != 0) return;
+    int last;
+    const int e = wave_walk_summed<STEPS>(weights, sums_s[min(lane, STEPS - 1)], rest, last);
+    if (lane == 0) { out[r] = e >= 0 ? begin + e : (last >= 0 ? begin + last : best_i); done[r] = 1; }
 }
 
 // ---- the rows that are left ---------------------------------------------------------------------------------------
@@ -1234,19 +1297,15 @@ __global__ __launch_bounds__(SIMPLE_THREADS) void left_collect_kernel(
     const uint32_t* __restrict__ seen_masks, const uint32_t* __restrict__ banned, int mask_words,
     const float* __restrict__ part_max, const float* __restrict__ part_min, const int* __restrict__ done,
     int* __restrict__ seg_i, float* __restrict__ seg_x, int* __restrict__ seg_n, int* __restrict__ rest) {
-    constexpr int WAVES = SIMPLE_THREADS / PULSE_WAVE, PER = SIMPLE_CHUNK / SIMPLE_THREADS;
+    constexpr int WAVES = SIMPLE_THREADS / PULSE_WAVE, PER = CHUNK_PER;
     __shared__ mass_t waves[WAVES], above_s;
-    __shared__ int at_s, counts[WAVES];
+    __shared__ int at_s, counts[PER][WAVES];
     const int r = blockIdx.y, chunk = blockIdx.x, chunks = gridDim.x;
     const int lane = threadIdx.x % PULSE_WAVE, wave = threadIdx.x / PULSE_WAVE;
     if (done[r] != LEFT) return;
     const RowView row = simple_row(logits, r, row_stride, vocab, penalty, seen_row, seen_masks, banned, mask_words);
-    const int begin = chunk * SIMPLE_CHUNK + static_cast<int>(threadIdx.x) * PER;
     float xs[PER];        // (asked for first: they travel while the edge is searched)
-    by_mask(row, [&](auto masked) __attribute__((always_inline)) {
-#pragma unroll
-        for (int j = 0; j < PER; ++j) xs[j] = begin + j < vocab ? row.at<decltype(masked)::value>(begin + j) : -INFINITY;
-    });
+    chunk_values(row, chunk * SIMPLE_CHUNK, xs);
     const LeftRow left(r, vocab, chunks, temperature, top_k, top_p, part_max, part_min);
     if (left.k == 0 && !left.by_p) return;
     rest += static_cast<int64_t>(r) * REST_WORDS;
@@ -1258,40 +1317,28 @@ __global__ __launch_bounds__(SIMPLE_THREADS) void left_collect_kernel(
         return;
     }
     const Weigh weigh(left.best, left.inv_t, vocab);
-    int bins[PER], mine = 0;
+    bool taken[PER];
     mass_t mass = 0;
 #pragma unroll
     for (int j = 0; j < PER; ++j) {
-        bins[j] = xs[j] == -INFINITY ? HIST_BINS : bin_at(xs[j], left.best, left.scale);
-        if (bins[j] == at || (left.k > 0 && bins[j] < at)) ++mine;
-        else if (bins[j] < at) mass += weigh(xs[j]);
-    }
-    // where this thread's entries go: an exclusive sum over the threads, in thread order (vocabulary order)
-    int pre = mine;
-#pragma unroll
-    for (int off = 1; off < PULSE_WAVE; off <<= 1) {
-        const int up = __shfl_up(pre, off, PULSE_WAVE);
-        if (lane >= off) pre += up;
+        const int bin = xs[j] == -INFINITY ? HIST_BINS : bin_at(xs[j], left.best, left.scale);
+        taken[j] = bin == at || (left.k > 0 && bin < at);
+        if (!taken[j] && bin < at) mass += weigh(xs[j]);
     }
     mass = mass_sum(mass);
     __syncthreads();      // (what edge_bin left has been read)
-    if (lane == PULSE_WAVE - 1) { counts[wave] = pre; waves[wave] = mass; }
-    __syncthreads();
-    int to = pre - mine, total = 0;
+    if (lane == PULSE_WAVE - 1) waves[wave] = mass;
+    int place[PER], total;
+    chunk_places(taken, counts, place, total);
     mass = 0;
-    for (int w = 0; w < WAVES; ++w) {
-        if (w < wave) to += counts[w];
-        total += counts[w];
-        mass += waves[w];
-    }
+    for (int w = 0; w < WAVES; ++w) mass += waves[w];
     const int64_t segment = (static_cast<int64_t>(r) * chunks + chunk) * TOPK_SEGMENT;
 #pragma unroll
-    for (int j = 0; j < PER; ++j) {
-        if (bins[j] == at || (left.k > 0 && bins[j] < at)) {
-            if (to < TOPK_SEGMENT) { seg_i[segment + to] = begin + j; seg_x[segment + to] = xs[j]; }
-            ++to;
+    for (int j = 0; j < PER; ++j)
+        if (place[j] >= 0 && place[j] < TOPK_SEGMENT) {
+            seg_i[segment + place[j]] = chunk * SIMPLE_CHUNK + j * SIMPLE_THREADS + static_cast<int>(threadIdx.x);
+            seg_x[segment + place[j]] = xs[j];
         }
-    }
     if (threadIdx.x != 0) return;
     *my_n = total;
     *reinterpret_cast<mass_t*>(rest + REST_CHUNKS + 2 * chunk) = mass;
@@ -1565,18 +1612,11 @@ extern "C" int pulse_sample_chunked_rest(const float* logits, int rows, int voca
                        penalty, seen_row, seen_masks, banned, mask_words, part_max, part_idx, part_min);
     PULSE_LAUNCH_CHECK("sample_chunked (maxima)");
     if (temperature) {
-        hipLaunchKernelGGL(simple_mass_kernel, dim3(chunks, rows), dim3(SIMPLE_THREADS), 0, stream, logits, vocab,
-                           row_stride, temperature, top_k, penalty, seen_row, seen_masks, banned, mask_words,
-                           part_max, part_mass);
-        PULSE_LAUNCH_CHECK("sample_chunked (masses)");
-        if (top_k || top_p) {
-            hipLaunchKernelGGL(topk_collect_kernel, dim3(chunks, rows), dim3(SIMPLE_THREADS), 0, stream, logits, vocab,
-                               row_stride, temperature, top_k, top_p, penalty, seen_row, seen_masks, banned, mask_words,
-                               part_max, seg_i, seg_x, seg_n);
-            PULSE_LAUNCH_CHECK("sample_chunked (candidates)");
-        }
+        hipLaunchKernelGGL(chunk_kernel, dim3(chunks, rows), dim3(SIMPLE_THREADS), 0, stream, logits, vocab, row_stride, temperature,
+                           top_k, top_p, penalty, seen_row, seen_masks, banned, mask_words, part_max, part_mass, seg_i, seg_x, seg_n);
+        PULSE_LAUNCH_CHECK("sample_chunked (masses and candidates)");
     }
-    hipLaunchKernelGGL(chunked_choose_kernel, dim3(rows), dim3(PULSE_WAVE), 0, stream, logits, vocab, row_stride,
+    hipLaunchKernelGGL(chunked_choose_kernel, dim3(rows), dim3(CHOOSE_THREADS), 0, stream, logits, vocab, row_stride,
                        temperature, top_k, top_p, uniform, penalty, seen_row, seen_masks, banned, mask_words, part_max,
                        part_idx, part_mass, seg_i, seg_x, seg_n, chunks, out, done, rest);
     PULSE_LAUNCH_CHECK("sample_chunked (choice)");

@@ -667,6 +667,28 @@ def test_temperature_sampling_in_chunks_follows_the_softmax(k):
     assert torch.allclose(counts, want, atol=0.03)
 
 
+@pytest.mark.parametrize("vocab", [1, 64, 2047, 2048, 2049, 6143, 40000])
+def test_draws_at_the_edges_of_a_chunks_steps(k, vocab):
+    """Rows with one, two and three tokens that have a weight, at the first and last place of steps of 64 logits, of a wavefront's share of
+    them and of chunks: u picks the token whose share of the mass it falls in."""
+    places = sorted({p for p in (0, 63, 64, 511, 512, 1535, 1536, 2047, 2048, 4095, vocab - 65, vocab - 1) if 0 <= p < vocab})
+    rows, want, us = [], [], []
+    for a in places:
+        for b in places:
+            kept = sorted({a, b, places[-1]})
+            x = torch.full((vocab,), float("-inf"))
+            x[kept] = 1.5                                   # (equal weights: 1 each)
+            for i, token in enumerate(kept):
+                rows.append(x)
+                want.append(token)
+                us.append((i + 0.5) / len(kept))
+    n = len(rows)
+    out = torch.full((n,), -5, dtype=torch.int32, device=DEV)
+    k.sample_chunked(torch.stack(rows).to(DEV), out, _chunked_scratch(k, n, vocab), temperature=torch.full((n,), 0.7, device=DEV),
+                     uniform=torch.tensor(us, device=DEV))
+    assert out.tolist() == want
+
+
 def test_kernels_refuse_what_they_cannot_do(k):
     from pulse_infer_amd.ops import KernelError
     with pytest.raises(KernelError, match="GPU"):
