@@ -58,9 +58,10 @@ struct TileLoop {
     static constexpr int P = TN * TM, ALL = KK * P;                  // products a depth, and a step
     static constexpr int LDS = X0 + SX * STAGE_X;
     // The next products' operand reads go out between these, over the first READS of them, so that the last is here in time: a
-    // lone wavefront a SIMD issues no product while it issues reads.  Where a step has few products the reads go ahead of them (0):
-    // behind the first they are late (experts of 8 tokens in 64 x 32, a step 1 % slower).
-    static constexpr int READS = P < 24 ? 0 : P * 3 / 4;
+    // lone wavefront a SIMD issues no product while it issues reads.  (Ahead of the products, o of 4,096 x 4,096 in shares in tiles of
+    // 128 x 128: 14.3 -> 15.7 us at 192 rows, 20.4 -> 22.5 at 400; 128 x 64 at 150 rows 18.5 -> 18.9.)  Where a step has four products a
+    // wavefront the reads go ahead of them (0): behind the first they are late (experts of 8 tokens in 64 x 32, a step 1 % slower).
+    static constexpr int READS = P < 8 ? 0 : P * 3 / 4;
     static_assert(WR % (8 * NW) == 0 && XR % (8 * NW) == 0 && TN >= 1 && TM % 2 == 0 && SX >= 2 && S >= SX,
                   "whole chunks and pieces a wavefront");
     static_assert(TILE_BLOCK % WR == 0, "a tile lies inside a block of weight rows");
@@ -199,7 +200,7 @@ struct TileLoop {
         for (int f = 0; f < TN; ++f)
 #pragma unroll
             for (int g = 0; g < TM; ++g) {
-                if constexpr (P >= 24) asm volatile("" : "+a"(acc[f][g]));
+                if constexpr (P >= 12) asm volatile("" : "+a"(acc[f][g]));
                 else asm volatile("" : "+v"(acc[f][g]));
             }
         // the last copies, which nobody reads, must not land in what follows
