@@ -24,6 +24,7 @@
 #include "no_alloc.h"
 
 #include <math.h>
+#include <string.h>
 
 #include <mutex>
 
@@ -1568,6 +1569,54 @@ extern "C" int pulse_sample(const float* logits, int rows, int vocab, int64_t ro
     hipLaunchKernelGGL(sample_kernel, dim3(rows), dim3(SAMPLE_THREADS), 0, stream, logits, vocab, row_stride,
                        temperature, top_k, top_p, uniform, penalty, seen_row, seen_masks, banned, mask_words, out);
     PULSE_LAUNCH_CHECK("sample");
+    return 0;
+}
+
+// A request's options, as its rows bring them to every step.
+struct SampleRow {
+    float temperature;
+    int32_t top_k;
+    float top_p, penalty;
+    uint64_t seed;
+    int32_t seeded, unused;
+};
+static_assert(sizeof(SampleRow) == 32, "the rows lie one after the other");
+
+static uint64_t splitmix64(uint64_t x) {
+    uint64_t z = x + 0x9E3779B97F4A7C15ull;
+    z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
+    z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
+    return z ^ (z >> 31);
+}
+
+// The options of a step's rows as the kernels read them, host memory [6, room]: temperature, top_k, top_p, the uniform number that
+// depends on the row's seed and counter alone, penalty, slot (-1 without a penalty); and their copy to `dev`, queued (null: none).
+// `numbers`: the rows' slots, then their counters; `seeds`: for rows without one of their own (null: none is).  `kinds`: 1 if a row uses top-k, 2
+// top-p, 4 a penalty.  (The host's part of a step of 32 rows up to its last launch, 78 us with this in the interpreter, 43 so.)
+extern "C" int pulse_sample_options(const void* params, const int64_t* numbers, const uint64_t* seeds, int rows, int32_t* host, int64_t room, int32_t* dev,
+                                    int* kinds, hipStream_t stream) {
+    PULSE_REQUIRE(rows >= 0 && room >= rows && host && kinds && (rows == 0 || (params && numbers)), "sample_options: bad arguments");
+    float* const floats = reinterpret_cast<float*>(host);
+    *kinds = 0;
+    for (int r = 0; r < rows; ++r) {
+        SampleRow p;
+        memcpy(&p, static_cast<const char*>(params) + sizeof(SampleRow) * r, sizeof(p));
+        PULSE_REQUIRE(p.seeded || seeds, "sample_options: row %d has no seed", r);
+        const uint64_t z = splitmix64(splitmix64(p.seeded ? p.seed : seeds[r]) ^
+                                      (static_cast<uint64_t>(numbers[static_cast<int64_t>(rows) + r]) * 0xD1342543DE82EF95ull));
+        const bool penalized = p.penalty > 0.f;
+        floats[r] = p.temperature;
+        host[room + r] = p.top_k;
+        floats[2 * room + r] = p.top_p;
+        floats[3 * room + r] = static_cast<float>(z >> 40) / static_cast<float>(1 << 24);
+        floats[4 * room + r] = p.penalty;
+        host[5 * room + r] = penalized ? static_cast<int32_t>(numbers[r]) : -1;
+        *kinds |= (p.top_k > 0 ? 1 : 0) | (p.top_p > 0.f && p.top_p < 1.f ? 2 : 0) | (penalized ? 4 : 0);
+    }
+    if (dev && rows > 0) {
+        const hipError_t e = hipMemcpyAsync(dev, host, static_cast<size_t>(5 * room + rows) * 4, hipMemcpyHostToDevice, stream);
+        PULSE_REQUIRE(e == hipSuccess, "sample_options: the copy failed: %s", hipGetErrorString(e));
+    }
     return 0;
 }
 

@@ -10,7 +10,8 @@ from __future__ import annotations
 
 import ctypes
 import functools
-from typing import Any, Optional
+from array import array
+from typing import Any, Optional, Sequence, Tuple
 
 import torch
 
@@ -1066,6 +1067,34 @@ SAMPLE_REST = 2 * 2048 + 6 + 2 * 128   # as REST_WORDS of sampling.hip
 def sample_chunks(vocab: int) -> int:
     """Chunks of the vocabulary that ``sample_chunked`` cuts a row into."""
     return (vocab + SAMPLE_CHUNK - 1) // SAMPLE_CHUNK
+
+
+SAMPLE_ROW_BYTES = 32    # as SampleRow of sampling.hip
+
+
+def sample_options(host: torch.Tensor, dev: Optional[torch.Tensor], rows: Sequence[bytes], slots: Sequence[int], counters: Sequence[int],
+                   seeds: Sequence[int]) -> Tuple[bool, bool, bool]:
+    """The options of a step's rows (``SamplingParams.packed``) as the sampling kernels read them, into ``host`` int32 [6, room] in host
+    memory: temperature, top_k, top_p, the row's uniform number (its seed's ``counters[r]``-th, ``seeds[r]`` where the request has no seed
+    of its own), penalty, slot (-1 without a penalty), the floats as their bits; from there to ``dev`` (of the same shape; none: no copy),
+    queued.  Whether some row uses top-k, top-p, a penalty."""
+    n, packed = len(rows), b"".join(rows)
+    _need(host.dtype == torch.int32 and host.dim() == 2 and host.shape[0] == 6 and host.shape[1] >= n and host.is_contiguous()
+          and host.device.type == "cpu", "sample_options: host must be int32 [6, rows or more] in host memory")
+    _need(dev is None or (dev.dtype == torch.int32 and dev.shape == host.shape and dev.is_contiguous() and dev.is_cuda),
+          "sample_options: dev must be as host, on a device")
+    own_seeds = 0 not in packed[24::SAMPLE_ROW_BYTES]
+    _need(len(packed) == n * SAMPLE_ROW_BYTES and len(slots) >= n and len(counters) >= n and (own_seeds or len(seeds) >= n),
+          "sample_options: a packed row, a slot, a counter and a seed for every row")
+    numbers = array("q", slots[:n])
+    numbers.extend(counters[:n])
+    others = None if own_seeds else array("Q", [d & 0xFFFFFFFFFFFFFFFF for d in seeds[:n]])
+    kinds = ctypes.c_int(0)
+    call("pulse_sample_options", packed, ctypes.c_void_p(numbers.buffer_info()[0]),
+         ctypes.c_void_p(others.buffer_info()[0] if others is not None else 0), _i32(n), _ptr(host), _i64(host.shape[1]), _ptr(dev),
+         ctypes.byref(kinds), _stream() if dev is not None else None)
+    used = kinds.value
+    return bool(used & 1), bool(used & 2), bool(used & 4)
 
 
 def sample_chunked_scratch(rows: int, vocab: int, device) -> dict:

@@ -10,8 +10,18 @@ with it (the reference seeds one generator from the system, :633-634).
 """
 from __future__ import annotations
 
+import ctypes
+import struct
 from dataclasses import dataclass
 from typing import Optional
+
+
+_MASK = (1 << 64) - 1
+
+
+# A request's options as the native step reads them (SampleRow of csrc/sampling.hip): temperature, top_k, top_p, penalty, seed, whether
+# there is one.
+_ROW = struct.Struct("=fiffQii")
 
 
 @dataclass(frozen=True)
@@ -30,13 +40,16 @@ class SamplingParams:
             raise ValueError(f"top_p must lie in [0, 1], got {self.top_p}")
         if self.presence_penalty < 0.0:
             raise ValueError(f"presence_penalty must not be negative, got {self.presence_penalty}")
+        # (made once a request: a step puts its rows' options together as they are)
+        seed = 0 if self.seed is None else int(self.seed) & _MASK
+        top_k = min(int(self.top_k), 0x7FFFFFFF)
+        single = lambda v: ctypes.c_float(v).value      # (beyond float32's range: infinite)
+        object.__setattr__(self, "packed", _ROW.pack(single(self.temperature), top_k, self.top_p, single(self.presence_penalty), seed,
+                                                     self.seed is not None, 0))
 
     @property
     def greedy(self) -> bool:
         return not self.temperature > 0.0
-
-
-_MASK = (1 << 64) - 1
 
 
 def _splitmix64(x: int) -> int:

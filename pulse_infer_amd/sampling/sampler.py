@@ -9,11 +9,10 @@ from __future__ import annotations
 
 from typing import List, Optional, Sequence
 
-import numpy as np
 import torch
 
 from ..ops import kernels
-from .params import SamplingParams, uniform_for
+from .params import SamplingParams
 
 
 class Sampler:
@@ -33,6 +32,7 @@ class Sampler:
         # before (not for older ones: a pair is used again two calls later)
         self._options_host: List[Optional[torch.Tensor]] = [None, None]
         self._options_dev: List[Optional[torch.Tensor]] = [None, None]
+        self._options_views: List[Optional[tuple]] = [None, None]     # of the device twins: (rows, a view an option)
         self._turn = 0
         if banned_tokens:
             host = torch.zeros(self.words, dtype=torch.int64)
@@ -87,28 +87,23 @@ class Sampler:
             kernels.argmax(logits, out, self._part_val, self._part_idx)
             return out
         # every per-row option in one upload: rows of a [6, R] int32 array, the float ones as their bit patterns
-        use_penalty = self.seen is not None and any(p.presence_penalty > 0.0 for p in params)
         turn = self._turn
         self._turn = 1 - turn
         if self._options_host[turn] is None or self._options_host[turn].shape[1] < rows:
             self._options_host[turn] = torch.empty((6, max(rows, 64)), dtype=torch.int32, pin_memory=True)
             self._options_dev[turn] = torch.empty((6, max(rows, 64)), dtype=torch.int32, device=self.device)
+            self._options_views[turn] = None
         # (the copy out of these pinned rows two calls ago has run: its tokens have been waited for)
-        host = self._options_host[turn].numpy()[:, :rows]
-        as_float = host.view(np.float32)
-        as_float[0] = [p.temperature for p in params]
-        host[1] = [p.top_k for p in params]
-        as_float[2] = [p.top_p for p in params]
-        as_float[3] = [uniform_for(p.seed if p.seed is not None else d, c)
-                       for p, c, d in zip(params, counters, default_seeds)]
-        as_float[4] = [p.presence_penalty for p in params]
-        host[5] = [s if p.presence_penalty > 0.0 else -1 for p, s in zip(params, slots)]
-        self._options_dev[turn].copy_(self._options_host[turn], non_blocking=True)
         dev = self._options_dev[turn]
-        temperature, top_p, uniform = (dev[i, :rows].view(torch.float32) for i in (0, 2, 3))
-        top_k = dev[1, :rows]
-        penalty = dev[4, :rows].view(torch.float32) if use_penalty else None
-        seen_row = dev[5, :rows] if use_penalty else None
+        by_k, by_p, penalized = kernels.sample_options(self._options_host[turn], dev, [p.packed for p in params], slots, counters,
+                                                       default_seeds)
+        views = self._options_views[turn]
+        if views is None or views[0] != rows:
+            floats = tuple(dev[i, :rows].view(torch.float32) for i in (0, 2, 3, 4))
+            views = self._options_views[turn] = (rows, dev[1, :rows], dev[5, :rows], *floats)
+        _, top_k, seen_row, temperature, top_p, uniform, penalty = views
+        if not (penalized and self.seen is not None):
+            penalty = seen_row = None
         seen = self.seen if penalty is not None else None
         # in chunks of the vocabulary; which way a row goes there depends on its own options alone, so a seeded
         # request draws the same tokens whatever else is in the batch.  An option that no row uses is left out
@@ -116,8 +111,7 @@ class Sampler:
         if self._chunked is None or self._chunked["done"].numel() < rows:
             self._chunked = kernels.sample_chunked_scratch(rows, logits.shape[1], self.device)
         kernels.sample_chunked(logits, out, self._chunked, temperature=temperature,
-                               top_k=top_k if any(p.top_k > 0 for p in params) else None,
-                               top_p=top_p if any(0.0 < p.top_p < 1.0 for p in params) else None,
+                               top_k=top_k if by_k else None, top_p=top_p if by_p else None,
                                uniform=uniform, penalty=penalty, seen_row=seen_row, seen_masks=seen,
                                banned=self.banned)
         return out

@@ -20,3 +20,36 @@ def test_options_are_checked():
     for bad in (dict(top_k=-1), dict(top_p=1.5), dict(top_p=-0.1), dict(presence_penalty=-1.0)):
         with pytest.raises(ValueError):
             SamplingParams(**bad)
+
+
+def test_a_steps_options_as_the_kernels_read_them():
+    """Rows with and without seeds of their own, counters and seeds of any sign and size: the same uniform numbers as one by one."""
+    import struct
+
+    import torch
+
+    from pulse_infer_amd.ops import kernels
+    from pulse_infer_amd.ops.library import KernelError
+
+    params = [SamplingParams(), SamplingParams(temperature=0.7, seed=-3), SamplingParams(temperature=1.5, top_k=40, top_p=0.9, seed=2 ** 80 + 5),
+              SamplingParams(temperature=0.8, top_p=1.0), SamplingParams(temperature=1e39, top_k=1, presence_penalty=1.5, seed=0)]
+    slots, counters, seeds = range(3, 8), [0, 7, -2, 2 ** 40, 123456789], [11, 12, 13, -(2 ** 70) - 1, 15]
+    host = torch.full((6, 9), -77, dtype=torch.int32)
+    packed = [p.packed for p in params]
+    assert kernels.sample_options(host, None, packed, slots, counters, seeds) == (True, True, True)
+    single = lambda v: struct.unpack("f", struct.pack("f", v))[0]
+    floats = host.view(torch.float32)
+    assert floats[0, :5].tolist() == [0.0, single(0.7), 1.5, single(0.8), float("inf")]
+    assert host[1, :5].tolist() == [0, 0, 40, 0, 1] and floats[2, :5].tolist() == [0.0, 0.0, single(0.9), 1.0, 0.0]
+    assert floats[3, :5].tolist() == [uniform_for(p.seed if p.seed is not None else d, c) for p, c, d in zip(params, counters, seeds)]
+    assert floats[4, :5].tolist() == [0.0] * 4 + [1.5] and host[5, :5].tolist() == [-1] * 4 + [7]
+    assert (host[:, 5:] == -77).all()                       # nothing beside the rows
+    some = lambda *i: kernels.sample_options(host, None, [packed[j] for j in i], [0] * len(i), [0] * len(i), [0] * len(i))
+    assert some(0, 3) == (False, False, False) and some(1, 4) == (True, False, True)
+    assert kernels.sample_options(host, None, [], [], [], []) == (False, False, False)
+    for bad in (lambda: kernels.sample_options(host[:, :4].contiguous(), None, packed, slots, counters, seeds),
+                lambda: kernels.sample_options(host, None, packed, slots, counters[:4], seeds),
+                lambda: kernels.sample_options(host, None, packed, slots, counters, seeds[:2]),
+                lambda: kernels.sample_options(host.float(), None, packed, slots, counters, seeds)):
+        with pytest.raises(KernelError):
+            bad()
