@@ -1491,10 +1491,8 @@ __global__ __launch_bounds__(PR_THREADS) void attn_prefill_reduce_kernel(const f
 // out[row, head, :] = sum_z w_z o_z / sum_z w_z l_z with w_z = exp2(m_z - max m), over the splits that hold keys of
 // the row.  One workgroup per (row, `hpw` heads): its groups of threads are dealt out over the heads, a head's groups
 // over the splits (with few splits a workgroup would otherwise be mostly idle, and the launch eight times as wide).
-// Everything a thread uses, its head's (m, l) pairs and the partial outputs of its first splits, is asked for before anything
-// waits, so that the kernel is little more than two trips to memory.  The weights stay in registers: a wavefront works on one head
-// and takes a split a lane, or, with several heads a workgroup, a thread has the few pairs of its head to itself.  (Out of LDS, a split
-// after the other in every thread, the 16 splits of one request of 600 keys took 5.0 us, now 4.6: its step 3,247 -> 3,223 us.)
+// The splits' (m, l) pairs go through LDS, and the partial outputs of the first splits are asked for before anything
+// waits, so that the kernel is little more than two trips to memory.
 constexpr int MAX_SPLITS = 1024;
 
 constexpr int REDUCE_THREADS = 256;
@@ -1512,7 +1510,8 @@ __global__ __launch_bounds__(REDUCE_THREADS) void attn_mfma_reduce_kernel(const 
                                                                          const bf16_t* __restrict__ gate, int64_t gate_stride,
                                                                          int gate_width, const float* __restrict__ sink,
                                                                          int chunk) {
-    __shared__ float s_w[MAX_SPLITS];      // (more splits than lanes)
+    __shared__ float s_w[MAX_SPLITS];      // hpw * n_splits <= MAX_SPLITS (hpw > 1 only with few splits)
+    __shared__ float s_l[MAX_SPLITS];
     __shared__ f32x4 s_acc[REDUCE_GROUPS][REDUCE_QUADS];
     // The kernel is a chain of trips to memory and little else, so it is kept to two: the item (and what says how its
     // keys were cut), then everything that needs only the row: its position, the item's last position, the (m, l)
@@ -1529,6 +1528,16 @@ __global__ __launch_bounds__(REDUCE_THREADS) void attn_mfma_reduce_kernel(const 
     const int pos_row = positions[row];
     const int pos_last = positions[row0 + ntok - 1];
     const int from = chunk > 0 ? splits_from(chunk, low_key(0, chunk, positions[row0])) : 0;
+    constexpr int ML_PER = MAX_SPLITS / REDUCE_THREADS;
+    f32x2 ml[ML_PER];
+#pragma unroll
+    for (int j = 0; j < ML_PER; ++j) {
+        const int i = threadIdx.x + j * REDUCE_THREADS;
+        const int hs = i & (hpw - 1), z = i >> hpw_log2;
+        ml[j] = f32x2{0.f, 0.f};
+        if (i < hpw * n_splits && head0 + hs < nq)
+            ml[j] = *reinterpret_cast<const f32x2*>(part_ml + 2 * ((row * nq + head0 + hs) * n_splits + z));
+    }
     // group `grp` of threads takes head grp % hpw and of its splits sg = grp / hpw, sg + gph, ..; a thread four
     // channels of them.
     // The partial outputs are asked for before the weights are known, eight splits of a group at a time.
@@ -1540,17 +1549,8 @@ __global__ __launch_bounds__(REDUCE_THREADS) void attn_mfma_reduce_kernel(const 
     const int head = head0 + hs;
     const bool works = sg < gph && head < nq;
     const int64_t base = (row * nq + (works ? head : head0)) * n_splits;
-    // One head (hpw 1): this lane's splits lane, lane + 64, ..; several: the head's splits, at most half as many as groups
-    constexpr int FEW = REDUCE_GROUPS / 2 > 0 ? REDUCE_GROUPS / 2 : 1;
-    const int lane = threadIdx.x % PULSE_WAVE;
-    const bool one = hpw_log2 == 0;
-    auto pair_of = [&](int z) { return *reinterpret_cast<const f32x2*>(part_ml + 2 * (base + min(z, n_splits - 1))); };
-    const f32x2 own = pair_of(lane);
-    f32x2 few[FEW];
-    if (!one) {
-#pragma unroll
-        for (int z = 0; z < FEW; ++z) few[z] = pair_of(z);
-    }
+    const float* my_w = s_w + (works ? hs : 0) * n_splits;
+    const float* my_l = s_l + (works ? hs : 0) * n_splits;
     constexpr int AHEAD = 8;
     f32x4 first[AHEAD];
 #pragma unroll
@@ -1562,52 +1562,34 @@ __global__ __launch_bounds__(REDUCE_THREADS) void attn_mfma_reduce_kernel(const 
     }
     if (plan && pos_last < split_size) return;   // the item was finished by its only split
     const int valid = min(n_splits, (pos_row - from) / split_size + 1);
-    auto weight = [](float m, float mm) { return m == -INFINITY ? 0.f : exp2f(m - mm); };
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-    float mm = -INFINITY, ll = 0.f;
-    if (one) {
-        mm = lane < valid ? own[0] : -INFINITY;
-        for (int z = lane + PULSE_WAVE; z < valid; z += PULSE_WAVE) mm = fmaxf(mm, pair_of(z)[0]);
-        mm = wave_max(mm);
-        const float w = lane < valid ? weight(own[0], mm) : 0.f;
-        ll = lane < valid ? w * own[1] : 0.f;
-        if (valid > PULSE_WAVE) {       // (the same for the whole workgroup)
-            if (threadIdx.x < PULSE_WAVE) s_w[lane] = w;
-            for (int z = lane + PULSE_WAVE; z < valid; z += PULSE_WAVE) {
-                const f32x2 p = pair_of(z);
-                const float wz = weight(p[0], mm);
-                if (threadIdx.x < PULSE_WAVE) s_w[z] = wz;
-                ll += wz * p[1];
-            }
-            __syncthreads();
+#pragma unroll
+    for (int j = 0; j < ML_PER; ++j) {
+        const int i = threadIdx.x + j * REDUCE_THREADS;
+        const int hs2 = i & (hpw - 1), z = i >> hpw_log2;
+        if (i < hpw * valid && head0 + hs2 < nq) {
+            s_w[hs2 * n_splits + z] = ml[j][0];
+            s_l[hs2 * n_splits + z] = ml[j][1];
         }
-        ll = wave_sum(ll);
+    }
+    __syncthreads();
+    float inv = 0.f;
+    if (works) {
+        float mm = -INFINITY;
+        for (int z = 0; z < valid; ++z) mm = fmaxf(mm, my_w[z]);
+        float ll = 0.f;
+        for (int z = 0; z < valid; ++z) ll += (my_w[z] == -INFINITY ? 0.f : exp2f(my_w[z] - mm)) * my_l[z];
+        ll = with_sink(ll, mm, sink, head);
+        inv = gated(ll > 0.f ? 1.0f / ll : 0.f, gate, gate_stride, row, head, gate_width);
+        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int i = 0; i < AHEAD; ++i) {
             const int z = sg + i * gph;
-            const float wz = valid > PULSE_WAVE ? s_w[min(z, valid - 1)] : __shfl(w, min(z, PULSE_WAVE - 1), PULSE_WAVE);
-            if (z < valid) acc += first[i] * wz;
+            if (z < valid) acc += first[i] * (my_w[z] == -INFINITY ? 0.f : exp2f(my_w[z] - mm));
         }
         for (int z = sg + AHEAD * gph; z < valid; z += gph) {
-            const float wz = valid > PULSE_WAVE ? s_w[z] : weight(pair_of(z)[0], mm);
-            if (works) acc += *reinterpret_cast<const f32x4*>(part_o + (base + z) * D + 4 * quad) * wz;
+            const float wz = my_w[z] == -INFINITY ? 0.f : exp2f(my_w[z] - mm);
+            acc += *reinterpret_cast<const f32x4*>(part_o + (base + z) * D + 4 * quad) * wz;
         }
-    } else {
-#pragma unroll
-        for (int z = 0; z < FEW; ++z) mm = z < valid ? fmaxf(mm, few[z][0]) : mm;
-        float mine = 0.f;      // (a split a group)
-#pragma unroll
-        for (int z = 0; z < FEW; ++z) {
-            const float w = z < valid ? weight(few[z][0], mm) : 0.f;
-            ll += z < valid ? w * few[z][1] : 0.f;
-            mine = z == sg ? w : mine;
-        }
-        if (sg < valid) acc = first[0] * mine;
-    }
-    float inv = 0.f;
-    if (works) {
-        ll = with_sink(ll, mm, sink, head);
-        inv = gated(ll > 0.f ? 1.0f / ll : 0.f, gate, gate_stride, row, head, gate_width);
         s_acc[grp][quad] = acc;
     }
     __syncthreads();
