@@ -4,6 +4,14 @@
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <type_traits>
+#include <utility>
+
+// f(0), f(1) .. f(N - 1) with constants (an unrolled loop whatever its size).
+template <typename F, int... I>
+__device__ __forceinline__ void each(F&& f, std::integer_sequence<int, I...>) { (f(std::integral_constant<int, I>()), ...); }
+template <int N, typename F>
+__device__ __forceinline__ void each(F&& f) { each(f, std::make_integer_sequence<int, N>()); }
 
 // Storage type tags used across the C ABI.
 enum PulseDType : int { PULSE_F32 = 0, PULSE_BF16 = 1 };
@@ -64,6 +72,16 @@ __device__ __forceinline__ void stream_to_lds(const void* p, uint32_t lds_base) 
 }
 __device__ __forceinline__ void load_to_lds(const void* base, uint32_t offset, uint32_t lds_base) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(lds_base), "v"(offset), "s"(base) : "memory", "m0");
+}
+
+// The same in a row: `lds_place` says where, the copies behind it bring 16 bytes a lane from `offset` + BYTES behind the base to BYTES
+// behind that place (-4,096 <= BYTES < 4,096), an instruction each.  (The place is kept in M0, which nothing that the compiler makes of these
+// kernels uses; their assembly was looked at.)
+__device__ __forceinline__ void lds_place(uint32_t lds_base) { asm volatile("s_mov_b32 m0, %0\n\ts_nop 0" : : "s"(lds_base) : "memory", "m0"); }
+template <int BYTES, bool STREAM = false>
+__device__ __forceinline__ void copy_to_place(const void* base, uint32_t offset) {
+    if constexpr (STREAM) asm volatile("global_load_lds_dwordx4 %0, %1 offset:%c2 nt" : : "v"(offset), "s"(base), "n"(BYTES) : "memory");
+    else asm volatile("global_load_lds_dwordx4 %0, %1 offset:%c2" : : "v"(offset), "s"(base), "n"(BYTES) : "memory");
 }
 
 template <typename T> __device__ __forceinline__ float to_f32(T v);

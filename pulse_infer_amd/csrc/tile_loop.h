@@ -21,8 +21,6 @@
 // pointer a lane and M0 set for each, six: 324 -> 306 us at 2,048 rows, 85 -> 81 at 357 in 192 x 256, before the other instruction).
 #pragma once
 #include "common.h"
-#include <type_traits>
-#include <utility>
 
 typedef __attribute__((ext_vector_type(8))) __bf16 tile_bf16x8;
 typedef __attribute__((ext_vector_type(4))) __bf16 tile_bf16x4;
@@ -37,12 +35,6 @@ typedef __attribute__((ext_vector_type(4))) float tile_f32x4;
 // rows 69.9 / 73.6 so, 71.0 / 75.0 in turns; 19,456 x 2,560 26.1 / 31.1 and 26.8 / 31.7.)
 constexpr int TILE_BLOCK = 768;
 __device__ __forceinline__ int tile_first_step(int block, int steps) { return (steps & (steps - 1)) == 0 ? (block * 5) & (steps - 1) : 0; }
-
-// f(0), f(1) .. f(N - 1) with constants (an unrolled loop whatever its size).
-template <typename F, int... I>
-__device__ __forceinline__ void tile_each(F&& f, std::integer_sequence<int, I...>) { (f(std::integral_constant<int, I>()), ...); }
-template <int N, typename F>
-__device__ __forceinline__ void tile_each(F&& f) { tile_each(f, std::make_integer_sequence<int, N>()); }
 
 // FAR: rows further than 4 GB from their base (a pointer a lane, as slow as that is).
 template <int WR, int XR, int WN, int WM, int S, bool NT = false, int SX = S, bool FAR = false>
@@ -113,13 +105,8 @@ struct TileLoop {
                 if constexpr (NT && !is_x) stream_to_lds(at + off, to + i * 1024);
                 else load_to_lds(at + off, to + i * 1024);
             } else {
-                // M0, the place in LDS, holds for the eight chunks behind it (nothing that the compiler makes of this loop uses M0)
-                if constexpr (i % 8 == 0 || j == FIRST)
-                    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0" : : "s"(to + (i / 8 * 8 + 4) * 1024) : "memory", "m0");
-                if constexpr (NT && !is_x)
-                    asm volatile("global_load_lds_dwordx4 %0, %1 offset:%c2 nt" : : "v"(off), "s"(at), "n"(inside(c)) : "memory");
-                else
-                    asm volatile("global_load_lds_dwordx4 %0, %1 offset:%c2" : : "v"(off), "s"(at), "n"(inside(c)) : "memory");
+                if constexpr (i % 8 == 0 || j == FIRST) lds_place(to + (i / 8 * 8 + 4) * 1024);
+                copy_to_place<inside(c), NT && !is_x>(at, off);
             }
         };
         const int h = lane / 16, e = h ^ swz(lane % 16);
@@ -137,13 +124,13 @@ struct TileLoop {
 #pragma unroll
                 for (int i = 0; i < 4; ++i) acc[f][g][i] = 0.f;
 
-        tile_each<S - 1>([&](auto sc) __attribute__((always_inline)) {
+        each<S - 1>([&](auto sc) __attribute__((always_inline)) {
             constexpr int s = sc - S;
-            tile_each<PER>([&](auto j) __attribute__((always_inline)) {
+            each<PER>([&](auto j) __attribute__((always_inline)) {
                 if constexpr (s + SX >= 0 || j >= PER_X) copy(s + S, s + S, s + SX, s + SX, j);
             });
         });
-        tile_each<FIRST>([&](auto j) __attribute__((always_inline)) { copy(S - 1, S - 1, SX - 1, SX - 1, j); });
+        each<FIRST>([&](auto j) __attribute__((always_inline)) { copy(S - 1, S - 1, SX - 1, SX - 1, j); });
         tile_bf16x8 wf[2][TN], xf[2][TM];
         asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" : : "n"(LATER + FIRST) : "memory");
 #pragma unroll
@@ -154,7 +141,7 @@ struct TileLoop {
         for (int s = 0; s < steps; ++s) {
             const int next_w = sw == S - 1 ? 0 : sw + 1, before_w = sw == 0 ? S - 1 : sw - 1;
             const int next_x = sx == SX - 1 ? 0 : sx + 1, before_x = sx == 0 ? SX - 1 : sx - 1;
-            tile_each<KK>([&](auto kc) __attribute__((always_inline)) {
+            each<KK>([&](auto kc) __attribute__((always_inline)) {
                 constexpr int kk = kc, buf = kk & 1, then = kk == KK - 1 ? 0 : kk + 1;
                 const char* const lds_w = lds + (kk == KK - 1 ? next_w : sw) * STAGE_W + w_at[then];
                 const char* const lds_x = lds + (kk == KK - 1 ? next_x : sx) * STAGE_X + x_at[then];
@@ -172,7 +159,7 @@ struct TileLoop {
                     for (int i = 0; i < TN + TM; ++i) read(i);
                 }
                 __builtin_amdgcn_sched_barrier(0);
-                tile_each<P>([&](auto pc) __attribute__((always_inline)) {
+                each<P>([&](auto pc) __attribute__((always_inline)) {
                     // two pieces of X in turns along the pieces of W, and back with the next two
                     constexpr int p = pc, pair = p / (2 * TN), f = p % (2 * TN) / 2, g = 2 * pair + (p % 2 ^ f % 2), n = pair % 2 ? TN - 1 - f : f;
                     acc[n][g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[buf][n], xf[buf][g], acc[n][g], 0, 0, 0);
@@ -185,7 +172,7 @@ struct TileLoop {
                     __builtin_amdgcn_sched_barrier(0);
                     // the copies, spread evenly over the products
                     constexpr int q = (kk == KK - 1 ? 0 : kk + 1) * P + p;
-                    tile_each<(q + 1) * PER / ALL - q * PER / ALL>([&](auto jc) __attribute__((always_inline)) {
+                    each<(q + 1) * PER / ALL - q * PER / ALL>([&](auto jc) __attribute__((always_inline)) {
                         constexpr std::integral_constant<int, q * PER / ALL + jc> j{};
                         if constexpr (kk == KK - 1) copy(s + S, sw, s + SX, sx, j);
                         else copy(s + S - 1, before_w, s + SX - 1, before_x, j);

@@ -1117,19 +1117,22 @@ __device__ __forceinline__ void attn_prefill_wide_workgroup(const MfmaArgs& a, c
     // wavefront's tile changes from block to block.
     const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(
         (void __attribute__((address_space(3)))*)(&s_kv[0])));  // the array's address inside LDS
-    int k_from[Shape::TILE_CHUNKS], v_from[Shape::VALUE_CHUNKS];
+    // (in bytes behind the tile's first, less what the copy's instruction adds: chunk i's place in LDS is its middle chunk's and that)
+    constexpr int K_MID = Shape::TILE_CHUNKS / 2, V_MID = Shape::VALUE_CHUNKS / 2, BACK = 4096;
+    static_assert(Shape::TILE_CHUNKS <= 8 && Shape::VALUE_CHUNKS <= 8, "an instruction's offset reaches four chunks either way");
+    uint32_t k_from[Shape::TILE_CHUNKS], v_from[Shape::VALUE_CHUNKS];
 #pragma unroll
     for (int i = 0; i < Shape::TILE_CHUNKS; ++i) {
         const int slot = 64 * i + lane;         // within the tile's 16 * P slots
         const int key = slot / P, pos = slot % P;
         const int c8 = (pos - piece_rot(key, P) + P) % P;
-        k_from[i] = key * D + c8 * 8;
+        k_from[i] = (key * D + c8 * 8) * 2 + BACK - (i - K_MID) * 1024;
     }
 #pragma unroll
     for (int i = 0; i < Shape::VALUE_CHUNKS; ++i) {
         const int slot = 64 * i + lane;
         const int blk = slot / 32, half = (slot / 16) % 2, chr = slot % 16;
-        v_from[i] = (blk * 16 + chr) * a.page_size + half * 8;
+        v_from[i] = ((blk * 16 + chr) * a.page_size + half * 8) * 2 + BACK - (i - V_MID) * 1024;
     }
     // The page of this wavefront's tile of block b: read from the block table without a branch (an index beyond
     // the table reads its last entry; what it gives is not used) one block ahead of the copy that needs it.
@@ -1166,10 +1169,16 @@ __device__ __forceinline__ void attn_prefill_wide_workgroup(const MfmaArgs& a, c
         const bf16_t* vfrom = a.vc + base + slot0;
         const uint32_t stage0 = lds0 + stage * (Shape::STAGE * 2), to = stage0 + wave * (Shape::TILE_CHUNKS * 1024);
         const uint32_t values_to = stage0 + Shape::STAGE_K * 2 + wave * (Shape::VALUE_CHUNKS * 1024);
-#pragma unroll
-        for (int i = 0; i < Shape::TILE_CHUNKS; ++i) load_to_lds(kfrom + k_from[i], to + i * 1024);
-#pragma unroll
-        for (int i = 0; i < Shape::VALUE_CHUNKS; ++i) load_to_lds(vfrom + v_from[i], values_to + i * 1024);
+        lds_place(to + K_MID * 1024);
+        each<Shape::TILE_CHUNKS>([&](auto i) __attribute__((always_inline)) {
+            const uint32_t from = k_from[i];
+            copy_to_place<(i - K_MID) * 1024>(reinterpret_cast<const char*>(kfrom) - BACK, from);
+        });
+        lds_place(values_to + V_MID * 1024);
+        each<Shape::VALUE_CHUNKS>([&](auto i) __attribute__((always_inline)) {
+            const uint32_t from = v_from[i];
+            copy_to_place<(i - V_MID) * 1024>(reinterpret_cast<const char*>(vfrom) - BACK, from);
+        });
     };
     // Operand reads.  Row r of score tile t is not key 16 t + r but key 32 (t / 2) + 8 (r / 4) + 4 (t % 2) + r % 4 of
     // the block: the four rows that lane group kg gets back of tiles 2 ks and 2 ks + 1 are then the eight
