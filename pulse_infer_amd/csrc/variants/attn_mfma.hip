@@ -986,6 +986,12 @@ __global__ __launch_bounds__(WAVES* PULSE_WAVE) PULSE_ATTN_WAVES_PER_EU void att
 // block's chain, not the matrix cores, bound this kernel, so the copy must stay out of that chain: K and V go from
 // memory straight into LDS (global_load_lds_dwordx4: 16 bytes a lane, lane i to the wavefront's LDS base + 16 i),
 // two stages, the next block on its way while this one is computed, with no register in between.
+// A wavefront takes the scores of the next block while it makes this block's weights, and this block's sums while it looks
+// for the next block's maximum, so that its matrix and its vector instructions alternate; what is rare (masks, caps, stale
+// values, a maximum that grew) stands out of the way, since a taken branch over it cost as much as a product.  Heads of
+// 128, 32 on 8: 2,048 tokens 64.4 -> 57.6 us, 8,192 in two splits 597 -> 575, 4,096 201 -> 187; 509 tokens 18.7 -> 17.5,
+// 97 9.8 -> 10.0 (10.8 -> 11.3 between other kernels, where its code comes cold).  What a step of it waits for now is spread evenly: without the copies it takes 11 % less, without the
+// exponentials 7 %, with half the reads from LDS 4 %; two wavefronts a SIMD keep the matrix cores busy 45 % of the time.
 //
 // LDS holds 16-byte pieces without padding; which piece a lane fetches is chosen so that the matrix-core operand
 // reads are free of bank conflicts:
@@ -1067,7 +1073,7 @@ __device__ __forceinline__ void attn_prefill_wide_workgroup(const MfmaArgs& a, c
     const int tc = r / a.gp;
     const int hc = r % a.gp + chunk * 16;
     bool col_ok[CT];
-    int col_row[CT], pos_c[CT], lo_c[CT];
+    int col_row[CT], pos_c[CT];
     int t_hi[CT], t_pos0[CT], t_lo[CT], t_hi_lo[CT];  // per tile: last and first position, lowest and highest window start
     bool t_any[CT];
     int col_head = g * a.group;
@@ -1079,7 +1085,6 @@ __device__ __forceinline__ void attn_prefill_wide_workgroup(const MfmaArgs& a, c
         col_ok[ct] = tc < wntok && hc < a.group;
         col_row[ct] = row0 + (col_ok[ct] ? wtok0 + tc : 0);
         pos_c[ct] = col_ok[ct] ? a.positions[col_row[ct]] : -1;
-        lo_c[ct] = low_key(a.window, a.chunk, pos_c[ct]);
         t_hi[ct] = uniform(wntok > 0 ? a.positions[row0 + wtok0 + wntok - 1] : -1);
         t_pos0[ct] = uniform(wntok > 0 ? a.positions[row0 + wtok0] : 0);
         t_lo[ct] = low_key(a.window, a.chunk, t_pos0[ct]);
@@ -1120,64 +1125,86 @@ __device__ __forceinline__ void attn_prefill_wide_workgroup(const MfmaArgs& a, c
     // (in bytes behind the tile's first, less what the copy's instruction adds: chunk i's place in LDS is its middle chunk's and that)
     constexpr int K_MID = Shape::TILE_CHUNKS / 2, V_MID = Shape::VALUE_CHUNKS / 2, BACK = 4096;
     static_assert(Shape::TILE_CHUNKS <= 8 && Shape::VALUE_CHUNKS <= 8, "an instruction's offset reaches four chunks either way");
-    uint32_t k_from[Shape::TILE_CHUNKS], v_from[Shape::VALUE_CHUNKS];
+    // Four keys a chunk: the next chunk's lie as far behind in memory as in LDS, and are turned alike in the same eight keys.
+    constexpr int ALIKE = P == 16 ? 2 : 1;
+    uint32_t k_from[Shape::TILE_CHUNKS / ALIKE];
 #pragma unroll
-    for (int i = 0; i < Shape::TILE_CHUNKS; ++i) {
+    for (int i = 0; i < Shape::TILE_CHUNKS; i += ALIKE) {
         const int slot = 64 * i + lane;         // within the tile's 16 * P slots
         const int key = slot / P, pos = slot % P;
         const int c8 = (pos - piece_rot(key, P) + P) % P;
-        k_from[i] = (key * D + c8 * 8) * 2 + BACK - (i - K_MID) * 1024;
+        k_from[i / ALIKE] = (key * D + c8 * 8) * 2 + BACK - (i - K_MID) * 1024;
     }
-#pragma unroll
-    for (int i = 0; i < Shape::VALUE_CHUNKS; ++i) {
-        const int slot = 64 * i + lane;
-        const int blk = slot / 32, half = (slot / 16) % 2, chr = slot % 16;
-        v_from[i] = ((blk * 16 + chr) * a.page_size + half * 8) * 2 + BACK - (i - V_MID) * 1024;
-    }
-    // The page of this wavefront's tile of block b: read from the block table without a branch (an index beyond
-    // the table reads its last entry; what it gives is not used) one block ahead of the copy that needs it.
-    auto page_ahead = [&](int b) {
-        int pi, slot0;
-        page_of(b * BK + 16 * wave, a.page_size, a.page_shift, pi, slot0);
-        // A scalar load written here, so that it stays where it is, a block ahead of its use, and is waited for
+    // (the values' chunks are 32 channels apart, the same for every lane)
+    const uint32_t v_from = ((lane / 32 * 16 + lane % 16) * a.page_size + lane / 16 % 2 * 8) * 2 + V_MID * 1024;
+    const int v_chunk = 32 * 2 * a.page_size - 1024;   // (less what the copy's instruction adds)
+    // Where this wavefront's tile of a block lies: its page comes from the block table, read without a branch (an index beyond
+    // the table reads its last entry; what it gives is not used) two steps ahead of the copy that needs it, and the addresses
+    // are made from it a step ahead, between the products.  From block to block the tile moves on by BK keys.
+    const int first_block = max(lo_item, split_begin) / BK;
+    const int last_block = split_last / BK;
+    const int pages_on = BK / a.page_size, slots_on = BK % a.page_size;
+    int tile_key = first_block * BK + 16 * wave, tile_page, tile_slot;   // of the tile whose page is asked for next
+    page_of(tile_key, a.page_size, a.page_shift, tile_page, tile_slot);
+    struct Tile { int page, slot; bool there; };
+    auto page_ahead = [&]() __attribute__((always_inline)) {
+        // A scalar load written here, so that it stays where it is, ahead of its use, and is waited for
         // with the scalar counter (page_landed) where it is used.  As a vector load it would share the counter of the
         // copies into LDS, and the compiler, which does not see those, would wait for all of them with it: the
         // next block's copy would have to land before this block is computed.
-        const int* entry = bt + min(pi, a.bt_width - 1);
-        int page;
-        asm volatile("s_load_dword %0, %1, 0x0" : "=s"(page) : "s"(entry) : "memory");
-        return page;
+        const int* entry = bt + min(tile_page, a.bt_width - 1);
+        Tile t;
+        asm volatile("s_load_dword %0, %1, 0x0" : "=s"(t.page) : "s"(entry) : "memory");
+        t.slot = tile_slot;
+        t.there = tile_key <= hi && tile_page < a.bt_width;
+        tile_key += BK;
+        tile_page += pages_on;
+        tile_slot += slots_on;
+        if (tile_slot >= a.page_size) {
+            tile_slot -= a.page_size;
+            ++tile_page;
+        }
+        return t;
     };
     // The register a load was asked into holds nothing until the wait: between the two it must not be copied, which
     // the compiler, to whom the load's result looks ready at once, is free to do wherever values meet (the head of a
     // loop, the end of a branch).  So a load and its wait stand in the same straight piece of code, with nothing but
     // the wait touching the variable in between, and only landed values are carried round the loop.
     auto page_landed = [&](int& page) { asm volatile("s_waitcnt lgkmcnt(0)" : "+s"(page) : : "memory"); };
-    auto pages_landed = [&](int& one, int& two) {
-        asm volatile("s_waitcnt lgkmcnt(0)" : "+s"(one), "+s"(two) : : "memory");
+    auto pages_landed = [&](int& one, int& two, int& three) {
+        asm volatile("s_waitcnt lgkmcnt(0)" : "+s"(one), "+s"(two), "+s"(three) : : "memory");
     };
     const int64_t page_elems = static_cast<int64_t>(a.nkv) * a.page_size * D;  // of K and of V alike
     const int head_elems = g * a.page_size * D;
-    auto fetch = [&](int b, int page_read, int stage) {
-        const int jt = b * BK + 16 * wave;
-        int pi, slot0;
-        page_of(jt, a.page_size, a.page_shift, pi, slot0);
-        int page = (jt <= hi && pi < a.bt_width) ? page_read : 0;
-        page = (page >= 0 && page < a.num_pages) ? page : 0;
-        const int64_t base = page * page_elems + head_elems;
-        const bf16_t* kfrom = a.kc + base + slot0 * D;
-        const bf16_t* vfrom = a.vc + base + slot0;
-        const uint32_t stage0 = lds0 + stage * (Shape::STAGE * 2), to = stage0 + wave * (Shape::TILE_CHUNKS * 1024);
-        const uint32_t values_to = stage0 + Shape::STAGE_K * 2 + wave * (Shape::VALUE_CHUNKS * 1024);
-        lds_place(to + K_MID * 1024);
+    // the addresses of a tile's keys and values, in four parts that stand between products (and are kept there)
+    struct Place { int64_t at; const char *keys, *values; };
+    auto find = [&](auto part, Tile& t, Place& to) __attribute__((always_inline)) {
+        if constexpr (part == 0) {
+            t.page = t.there && t.page >= 0 && t.page < a.num_pages ? t.page : 0;
+            asm volatile("" : "+s"(t.page));
+        } else if constexpr (part == 1) {
+            to.at = (t.page * page_elems + (head_elems + t.slot)) * 2;
+            asm volatile("" : "+s"(to.at));
+        } else if constexpr (part == 2) {
+            to.keys = reinterpret_cast<const char*>(a.kc) + to.at + t.slot * ((D - 1) * 2) - BACK;
+            asm volatile("" : "+s"(to.keys));
+        } else {
+            to.values = reinterpret_cast<const char*>(a.vc) + to.at;
+            asm volatile("" : "+s"(to.values));
+        }
+    };
+    auto fetch_keys = [&](const Place& from, int stage) __attribute__((always_inline)) {
+        lds_place(lds0 + stage * (Shape::STAGE * 2) + wave * (Shape::TILE_CHUNKS * 1024) + K_MID * 1024);
         each<Shape::TILE_CHUNKS>([&](auto i) __attribute__((always_inline)) {
-            const uint32_t from = k_from[i];
-            copy_to_place<(i - K_MID) * 1024>(reinterpret_cast<const char*>(kfrom) - BACK, from);
+            const uint32_t at = k_from[i / ALIKE];
+            copy_to_place<(i - K_MID) * 1024>(from.keys, at);
         });
-        lds_place(values_to + V_MID * 1024);
+    };
+    auto fetch_values = [&](const Place& from, int stage) __attribute__((always_inline)) {
+        lds_place(lds0 + (stage * Shape::STAGE + Shape::STAGE_K) * 2 + wave * (Shape::VALUE_CHUNKS * 1024) + V_MID * 1024);
         each<Shape::VALUE_CHUNKS>([&](auto i) __attribute__((always_inline)) {
-            const uint32_t from = v_from[i];
-            copy_to_place<(i - V_MID) * 1024>(reinterpret_cast<const char*>(vfrom) - BACK, from);
+            const uint32_t at = v_from;
+            copy_to_place<(i - V_MID) * 1024>(from.values + i * v_chunk, at);
         });
     };
     // Operand reads.  Row r of score tile t is not key 16 t + r but key 32 (t / 2) + 8 (r / 4) + 4 (t % 2) + r % 4 of
@@ -1185,58 +1212,98 @@ __device__ __forceinline__ void attn_prefill_wide_workgroup(const MfmaArgs& a, c
     // consecutive keys 32 ks + 8 kg .. + 7, whose values for one channel are one 16-byte piece of the value tile,
     // read whole by one lane (eight lanes a cycle read eight neighbouring pieces: no bank is asked twice; as two
     // 8-byte halves of pieces 16 bytes apart every read took two turns).
-    int k_at[2][NCHUNK];
+    // (tiles of odd t read the rows four further on, whose pieces are turned as far: 4 P pieces behind)
+    int k_at[NCHUNK];
+    const int k_row = 8 * (r / 4) + r % 4;
 #pragma unroll
-    for (int par = 0; par < 2; ++par) {
-        const int row = 4 * par + 8 * (r / 4) + r % 4;
-#pragma unroll
-        for (int ch = 0; ch < NCHUNK; ++ch) k_at[par][ch] = (row * P + (4 * ch + kg + piece_rot(row, P)) % P) * 8;
-    }
+    for (int ch = 0; ch < NCHUNK; ++ch) k_at[ch] = (k_row * P + (4 * ch + kg + piece_rot(k_row, P)) % P) * 8;
     const int v_at = (kg >> 1) * VD * 16 + ((kg & 1) * 16 + r) * 8;
 
     const float c2 = a.scale_log2e;
     constexpr float LAZY_BITS = 8.f;
     const float lazy = LAZY_BITS / c2;   // in the raw scores' units
-    auto compute = [&](int b, int stage) {
-        const int j0 = b * BK;
-        const bf16_t* s_k = s_kv + stage * Shape::STAGE;
-        const bf16_t* s_v = s_k + Shape::STAGE_K;
-        // Operand reads run AHEAD steps in front of the products that use them, in an order that is fixed here (the
-        // scheduling fences keep the compiler from regrouping them into bursts that are each waited for in full): a
-        // read's latency is then covered by the products of the steps before it, not added to them.
-        constexpr int AHEAD = 4;
-        f32x4 s[CT][KT];
-        {
-            constexpr int STEPS = KT * NCHUNK;
-            auto k_read = [&](int i) {
-                const int t = i / NCHUNK, ch = i % NCHUNK;
-                return ch * 32 + kg * 8 < D ? *reinterpret_cast<const bf16x8*>(&s_k[32 * (t / 2) * D + k_at[t % 2][ch]]) : zero8();
-            };
-            bf16x8 ak[STEPS];
+    // Operand reads run AHEAD steps in front of the products that use them, in an order that is fixed here (the
+    // scheduling fences keep the compiler from regrouping them into bursts that are each waited for in full): a
+    // read's latency is then covered by the products of the steps before it, not added to them.
+    constexpr int AHEAD = 4;
+    constexpr int STEPS = KT * NCHUNK, V_STEPS = (KT / 2) * NVT, PAIRS = CT * KT * 2;
+    using Scores = f32x4[CT][KT];
+    float alpha[CT], shift[CT];
+    struct Step {   // what lives for one step
+        float mx[CT], psum[CT];
+        bf16x8 pb[CT][KT / 2];
+        u32x4 vw[V_STEPS];
+    };
+    // weights of two scores: p = exp2((s - m) * scale * log2 e), the maximum being tracked on the raw scores (the scale is positive)
+    auto weigh = [&](auto pair, Step& x, Scores& s) __attribute__((always_inline)) {
+        constexpr int t = pair / (2 * CT), ct = pair / 2 % CT, half = pair % 2;
+        if constexpr (t == 0 && half == 0) x.psum[ct] = 0.f;
+#pragma unroll
+        for (int i = 2 * half; i < 2 * half + 2; ++i) {
+            // exp2(-inf) = 0 for masked scores; a dead column keeps -inf + 0 = -inf as well
+            const float e = __builtin_amdgcn_exp2f(fmaf(s[ct][t][i], c2, shift[ct]));
+            x.psum[ct] += e;
+            x.pb[ct][t / 2][4 * (t % 2) + i] = (__bf16)e;
+        }
+    };
+    // the scores of a block (QK) and, between their products, the weights of the block before it (WEIGHTS)
+    auto v_read = [&](int i, const bf16_t* s_v) __attribute__((always_inline)) {
+        const int ks = i / NVT, dt = i % NVT;
+        return *reinterpret_cast<const u32x4*>(&s_v[(2 * ks) * VD * 16 + dt * 256 + v_at]);
+    };
+    auto score = [&](auto QK, auto WEIGHTS, auto aside, Step& x, Scores& s, Scores& before, const bf16_t* s_k, const bf16_t* s_v) __attribute__((always_inline)) {
+        auto k_read = [&](int i) __attribute__((always_inline)) {
+            const int t = i / NCHUNK, ch = i % NCHUNK;
+            return ch * 32 + kg * 8 < D ? *reinterpret_cast<const bf16x8*>(&s_k[(32 * (t / 2) + 4 * (t % 2)) * D + k_at[ch]]) : zero8();
+        };
+        bf16x8 ak[STEPS];
+        if constexpr (QK) {
 #pragma unroll
             for (int i = 0; i < AHEAD && i < STEPS; ++i) ak[i] = k_read(i);
-#pragma unroll
-            for (int i = 0; i < STEPS; ++i) {
-                const int t = i / NCHUNK, ch = i % NCHUNK;
+        }
+        each<STEPS>([&](auto ic) __attribute__((always_inline)) {
+            constexpr int i = ic, t = i / NCHUNK, ch = i % NCHUNK;
+            if constexpr (QK) {
                 if (i + AHEAD < STEPS) ak[i + AHEAD] = k_read(i + AHEAD);
+            }
+            if constexpr (WEIGHTS) {
+                if (i + AHEAD >= STEPS && i + AHEAD - STEPS < V_STEPS) x.vw[i + AHEAD - STEPS] = v_read(i + AHEAD - STEPS, s_v);
+                constexpr int from = i * PAIRS / STEPS, to = (i + 1) * PAIRS / STEPS;
+                each<to - from>([&](auto n) __attribute__((always_inline)) { weigh(std::integral_constant<int, from + n>(), x, before); });
+            }
+            if constexpr (i % (STEPS / 4) == 0) aside(std::integral_constant<int, i / (STEPS / 4)>());
+            if constexpr (QK) {
 #pragma unroll
                 for (int ct = 0; ct < CT; ++ct)
                     s[ct][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ak[i], bq[ct][ch],
                                                                        ch == 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : s[ct][t], 0, 0, 0);
-                __builtin_amdgcn_sched_barrier(0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        });
+        if constexpr (WEIGHTS) {
+#pragma unroll
+            for (int ct = 0; ct < CT; ++ct) {
+                l_part[ct] = l_part[ct] * alpha[ct] + x.psum[ct];
+                asm volatile("" : "+v"(l_part[ct]));   // (here, not where the compiler would sink it to: behind the branches that follow)
+#pragma unroll
+                for (int ks = 0; ks < KT / 2; ++ks) asm volatile("" : "+v"(x.pb[ct][ks]));
             }
         }
-        // the first value operands are asked for before the weights are computed, the rest as the products go
-        constexpr int V_STEPS = (KT / 2) * NVT;
-        auto v_read = [&](int i) {
-            const int ks = i / NVT, dt = i % NVT;
-            return *reinterpret_cast<const u32x4*>(&s_v[(2 * ks) * VD * 16 + dt * 256 + v_at]);
-        };
-        u32x4 vw[V_STEPS];
+    };
+    // Most blocks lie wholly below the tiles' diagonals and inside their windows: every column sees every key, and nothing is masked
+    // (columns that stand for no token or head have q = 0 and are never written).  Only a tile whose first token does not see
+    // the block's last key, or one of whose windows starts inside the block, takes the mask: score i of tile t belongs to key
+    // j0 + 32 (t / 2) + 4 (t % 2) + 8 kg + i, which is seen when 32 (t / 2) + 4 (t % 2) + i lies in [lim_lo, lim_hi] (two compares
+    // and a select a score, on a branch that is the same for the wavefront and lies out of the way of the others).
+    int plain_to = a.cap_out != 0.f ? -1 : 0x7fffffff, plain_from = 0;   // a block all of whose keys lie in [plain_from, plain_to] is left as it is
 #pragma unroll
-        for (int i = 0; i < AHEAD && i < V_STEPS; ++i) vw[i] = v_read(i);
-        __builtin_amdgcn_sched_barrier(0);
-        // the maximum is tracked on the raw scores (the scale is positive); p = exp2((s - m) * scale * log2 e)
+    for (int ct = 0; ct < CT; ++ct) {
+        plain_to = t_any[ct] ? min(plain_to, t_pos0[ct]) : -1;
+        plain_from = max(plain_from, t_hi_lo[ct]);
+    }
+    auto limit = [&](int b, Scores& s) __attribute__((always_inline)) {
+        const int j0 = b * BK;
+        if (__builtin_expect(j0 + BK - 1 <= plain_to && j0 >= plain_from, 1)) return;
         if (a.cap_out != 0.f) {
 #pragma unroll
             for (int ct = 0; ct < CT; ++ct)
@@ -1245,20 +1312,11 @@ __device__ __forceinline__ void attn_prefill_wide_workgroup(const MfmaArgs& a, c
 #pragma unroll
                     for (int i = 0; i < 4; ++i) s[ct][t][i] = capped(s[ct][t][i], a.cap_in, a.cap_out);
         }
-        bf16x8 pb[CT][KT / 2];
-        bool moved = false;
-        float alpha[CT];
 #pragma unroll
         for (int ct = 0; ct < CT; ++ct) {
-            // Most blocks lie wholly below a tile's diagonal and inside its window: every column of the tile sees
-            // every key, and nothing is masked (columns that stand for no token or head have q = 0 and are never
-            // written).  Only a tile whose first token does not see the block's last key, or one of whose windows
-            // starts inside the block, takes the mask: score i of tile t belongs to key j0 + 32 (t / 2) + 4 (t % 2) + 8 kg + i,
-            // which is seen when 32 (t / 2) + 4 (t % 2) + i lies in
-            // [lim_lo, lim_hi] (two compares and a select a score, on a branch that is the same for the wavefront).
             if (j0 + BK - 1 > t_pos0[ct] || j0 < t_hi_lo[ct] || !t_any[ct]) {
                 const int lim_hi = col_ok[ct] ? pos_c[ct] - j0 - 8 * kg : -1;
-                const int lim_lo = lo_c[ct] - j0 - 8 * kg;
+                const int lim_lo = low_key(a.window, a.chunk, pos_c[ct]) - j0 - 8 * kg;
 #pragma unroll
                 for (int t = 0; t < KT; ++t)
 #pragma unroll
@@ -1266,53 +1324,57 @@ __device__ __forceinline__ void attn_prefill_wide_workgroup(const MfmaArgs& a, c
                         s[ct][t][i] = (32 * (t / 2) + 4 * (t % 2) + i <= lim_hi && 32 * (t / 2) + 4 * (t % 2) + i >= lim_lo)
                                           ? s[ct][t][i] : -INFINITY;
             }
-            float mx = -INFINITY;
-#pragma unroll
-            for (int t = 0; t < KT; ++t)
-#pragma unroll
-                for (int i = 0; i < 4; ++i) mx = fmaxf(mx, s[ct][t][i]);
-            mx = across_rows(mx, LaneMax());
-            // The reference point of the exponents follows the maximum only when that has grown by more than
-            // 2^LAZY_BITS in the weights' units: until then weights may exceed 1 (by at most that factor, which float32
-            // sums and bfloat16 weights hold with the same relative precision), and the accumulators, which are most of
-            // a wavefront's registers, are rescaled in few blocks instead of nearly all.  The result is the same
-            // quotient of sums.
-            const float m_new = mx > m[ct] + lazy ? mx : m[ct];
-            const bool dead = m_new == -INFINITY;  // no key of this column so far
-            alpha[ct] = dead ? 1.f : __builtin_amdgcn_exp2f((m[ct] - m_new) * c2);
-            const float shift = dead ? 0.f : -m_new * c2;
-            float psum = 0.f;
-#pragma unroll
-            for (int t = 0; t < KT; ++t)
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    // exp2(-inf) = 0 for masked scores; a dead column keeps -inf + 0 = -inf as well
-                    const float e = __builtin_amdgcn_exp2f(fmaf(s[ct][t][i], c2, shift));
-                    psum += e;
-                    pb[ct][t / 2][4 * (t % 2) + i] = (__bf16)e;
-                }
-            l_part[ct] = l_part[ct] * alpha[ct] + psum;
-            m[ct] = m_new;
-            moved = moved || alpha[ct] != 1.f;
         }
-        // rescale only when some column's maximum moved
-        if (__builtin_amdgcn_ballot_w64(moved) != 0) {
-#pragma unroll
-            for (int ct = 0; ct < CT; ++ct)
-#pragma unroll
-                for (int dt = 0; dt < NVT; ++dt) acc[ct][dt] = acc[ct][dt] * alpha[ct];
-        }
-        // (values under keys outside [lo_item, hi] have been cleared in LDS by clear_stale before this block is computed)
+    };
+    // The values of a block under its weights (PV) and, between their products, the maximum of the next block's scores (MAX)
+    auto sum = [&](auto PV, auto MAX, Step& x, Scores& s, const bf16_t* s_v) __attribute__((always_inline)) {
         __builtin_amdgcn_sched_barrier(0);
+        constexpr int HALF = V_STEPS / 2;   // of the steps take the maximum in the lane, the next one across lanes, the last one the rest
+        each<V_STEPS>([&](auto ic) __attribute__((always_inline)) {
+            constexpr int i = ic, ks = i / NVT, dt = i % NVT;
+            if constexpr (PV) {
+                if (i + AHEAD < V_STEPS) x.vw[i + AHEAD] = v_read(i + AHEAD, s_v);
 #pragma unroll
-        for (int i = 0; i < V_STEPS; ++i) {
-            const int ks = i / NVT, dt = i % NVT;
-            if (i + AHEAD < V_STEPS) vw[i + AHEAD] = v_read(i + AHEAD);
+                for (int ct = 0; ct < CT; ++ct)
+                    acc[ct][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, x.vw[i]), x.pb[ct][ks],
+                                                                          acc[ct][dt], 0, 0, 0);
+            }
+            if constexpr (MAX) {
 #pragma unroll
-            for (int ct = 0; ct < CT; ++ct)
-                acc[ct][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, vw[i]), pb[ct][ks],
-                                                                      acc[ct][dt], 0, 0, 0);
+                for (int ct = 0; ct < CT; ++ct) {
+                    if (i == 0) x.mx[ct] = -INFINITY;
+                    if (i < HALF) {
+#pragma unroll
+                        for (int n = i * KT * 4 / HALF; n < (i + 1) * KT * 4 / HALF; ++n) x.mx[ct] = fmaxf(x.mx[ct], s[ct][n / 4][n % 4]);
+                    }
+                    if (i == HALF) x.mx[ct] = across_rows(x.mx[ct], LaneMax());
+                    if (i == V_STEPS - 1) {
+                        // The reference point of the exponents follows the maximum only when that has grown by more than
+                        // 2^LAZY_BITS in the weights' units: until then weights may exceed 1 (by at most that factor, which float32
+                        // sums and bfloat16 weights hold with the same relative precision), and the accumulators, which are most of
+                        // a wavefront's registers, are rescaled in few blocks instead of nearly all.  The result is the same
+                        // quotient of sums.
+                        const float m_new = x.mx[ct] > m[ct] + lazy ? x.mx[ct] : m[ct];
+                        const bool dead = m_new == -INFINITY;  // no key of this column so far
+                        alpha[ct] = dead ? 1.f : __builtin_amdgcn_exp2f((m[ct] - m_new) * c2);
+                        shift[ct] = dead ? 0.f : -m_new * c2;
+                        m[ct] = m_new;
+                    }
+                }
+            }
             __builtin_amdgcn_sched_barrier(0);
+        });
+        if constexpr (MAX) {
+            // rescale only when some column's maximum moved
+            bool moved = false;
+#pragma unroll
+            for (int ct = 0; ct < CT; ++ct) moved = moved || alpha[ct] != 1.f;
+            if (__builtin_expect(__builtin_amdgcn_ballot_w64(moved) != 0, 0)) {
+#pragma unroll
+                for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+                    for (int dt = 0; dt < NVT; ++dt) acc[ct][dt] = acc[ct][dt] * alpha[ct];
+            }
         }
     };
     // Stale values under keys that no column of the item may see (beyond its last position, below its window) must
@@ -1321,6 +1383,8 @@ __device__ __forceinline__ void attn_prefill_wide_workgroup(const MfmaArgs& a, c
     // in LDS, a 16-byte piece (8 keys of a channel) a thread, before anybody reads them.
     auto clear_stale = [&](int b, int stage) {
         bf16_t* s_v = s_kv + stage * Shape::STAGE + Shape::STAGE_K;
+        int tid = threadIdx.x;
+        asm volatile("" : "+v"(tid));   // what follows from it is not kept in registers from block to block
 #pragma unroll
         for (int t = 0; t < KT; ++t)
             for (int piece = tid; piece < 2 * VD; piece += NW * PULSE_WAVE) {
@@ -1335,36 +1399,98 @@ __device__ __forceinline__ void attn_prefill_wide_workgroup(const MfmaArgs& a, c
             }
     };
 
-    const int first_block = max(lo_item, split_begin) / BK;
-    const int last_block = split_last / BK;
     // (a split that lies below the item's window has no block to walk: nothing is fetched, its columns stay empty)
-    int page_next = 0;   // the page of block b + 1, landed
     if (first_block <= last_block) {
-        int page_first = page_ahead(first_block);
-        int page_second = page_ahead(first_block + 1);
-        pages_landed(page_first, page_second);
-        fetch(first_block, page_first, 0);
-        page_next = page_second;
-    }
-    for (int b = first_block; b <= last_block; ++b) {
-        const int stage = (b - first_block) & 1;
-        // This block's loads were issued a block ago; nothing else is in flight, so the wait does not depend on a
-        // count of loads.
-        asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
-        __syncthreads();  // every wavefront's part of this block has landed
-        if (b < last_block)
-            fetch(b + 1, page_next, stage ^ 1);  // that stage was read a block ago; the barrier that ended that block released it
-        int page_after = page_ahead(b + 2);      // asked for now (past the walk's end it reads an entry nobody uses),
-                                                 // waited for at the end of this block, used in the next
-        // a wavefront skips blocks that none of its columns sees (above its diagonal, below its window)
-        if (b * BK + BK - 1 > hi || b * BK < lo_item) {   // the same for the whole workgroup
-            clear_stale(b, stage);
-            __syncthreads();
+        constexpr std::true_type YES{};
+        constexpr std::false_type NO{};
+        Tile first = page_ahead(), second = page_ahead(), after = page_ahead();   // after: of block b + 3, landed
+        pages_landed(first.page, second.page, after.page);
+        // (the columns' positions and queries land here, as the compiler would wait for them behind the copies, and with them for those)
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct) {
+            asm volatile("" : "+v"(pos_c[ct]));
+#pragma unroll
+            for (int ch = 0; ch < NCHUNK; ++ch) asm volatile("" : "+v"(bq[ct][ch]));
         }
-        if (w_hi >= 0 && b * BK <= w_hi && b * BK + BK - 1 >= w_lo) compute(b, stage);
-        page_landed(page_after);
-        page_next = page_after;
-        __syncthreads();  // everybody has read this block
+        Place next, two;                                                          // of blocks b + 1 and b + 2
+        each<4>([&](auto part) __attribute__((always_inline)) { find(part, first, next); find(part, second, two); });
+        // (the second block's keys are asked for in any case: behind the walk's end they are those of the first page, and not used)
+        fetch_keys(next, 0);
+        fetch_values(next, 0);
+        fetch_keys(two, 1);
+        // A step of the workgroup takes the scores of block b + 1 beside the weights of block b, and the sums of block b beside the
+        // maximum of block b + 1: the matrix cores and the vector units then work at the same time within one wavefront.  What every
+        // step begins with: the keys of block b + 1 and the values of block b were asked for a step ago; nothing else is in flight,
+        // so the wait does not depend on a count of loads.  Behind the barrier every wavefront's part of them has landed, and
+        // everybody has read those of the step before, whose places the next ones take.  The step in front of the first block (EARLY: one
+        // that may be it) finds all that it would ask for under way, and waits for the first keys only.
+        auto step = [&](int b, auto EARLY, auto work) __attribute__((always_inline)) {
+            const int stage = (b - first_block) & 1;
+            if (EARLY && b < first_block) {
+                asm volatile("s_waitcnt vmcnt(%0)" : : "n"(Shape::VALUE_CHUNKS + Shape::TILE_CHUNKS) : "memory");
+                __syncthreads();
+            } else {
+                asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
+                __syncthreads();
+                if (__builtin_expect(b + 2 <= last_block, 1)) fetch_keys(two, stage);
+                if (__builtin_expect(b + 1 <= last_block, 1)) fetch_values(next, stage ^ 1);
+            }
+            Tile then = page_ahead();   // asked for now (past the walk's end it reads an entry nobody uses), landed at the end of this step
+            next = two;
+            const bool stale = (!EARLY || b >= first_block) & ((b * BK + BK - 1 > hi) | (b * BK < lo_item));
+            if (__builtin_expect(stale, 0)) {   // the same for the whole workgroup
+                clear_stale(b, stage);
+                __syncthreads();
+            }
+            Step x;
+            work([&](auto part) __attribute__((always_inline)) { find(part, after, two); }, x,
+                 s_kv + (stage ^ 1) * Shape::STAGE, s_kv + stage * Shape::STAGE + Shape::STAGE_K);
+            page_landed(then.page);
+            after = then;
+        };
+        auto copy_only = [](auto aside, Step&, const bf16_t*, const bf16_t*) __attribute__((always_inline)) { each<4>(aside); };
+        Scores even, odd;   // of the blocks an even and an odd number behind this wavefront's first
+        auto work = [&](int b, Scores& now, Scores& then) __attribute__((always_inline)) {
+            step(b, NO, [&](auto aside, Step& x, const bf16_t* s_k, const bf16_t* s_v) __attribute__((always_inline)) {
+                score(YES, YES, aside, x, then, now, s_k, s_v);
+                limit(b + 1, then);
+                sum(YES, YES, x, then, s_v);
+            });
+        };
+        // This wavefront's blocks: those that one of its columns sees (none for a wavefront without tokens).  It only copies in the
+        // steps that lie before and behind them, so every wavefront goes through the same steps and their barriers.
+        const int own_first = max(first_block, w_lo / BK);
+        const int own_last = w_hi >= 0 ? min(last_block, w_hi / BK) : -1;
+        int b = first_block - 1;
+        if (own_first <= own_last) {
+            for (; b < own_first - 1; ++b) step(b, YES, copy_only);
+            step(b, YES, [&](auto aside, Step& x, const bf16_t* s_k, const bf16_t* s_v) __attribute__((always_inline)) {
+                score(YES, NO, aside, x, even, odd, s_k, s_v);
+                limit(b + 1, even);
+                sum(NO, YES, x, even, s_v);
+            });
+            ++b;
+            for (;;) {
+                if (b == own_last) break;
+                work(b, even, odd);
+                ++b;
+                if (b == own_last) {
+#pragma unroll
+                    for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+                        for (int t = 0; t < KT; ++t) even[ct][t] = odd[ct][t];
+                    break;
+                }
+                work(b, odd, even);
+                ++b;
+            }
+            step(b, NO, [&](auto aside, Step& x, const bf16_t* s_k, const bf16_t* s_v) __attribute__((always_inline)) {
+                score(NO, YES, aside, x, odd, even, s_k, s_v);
+                sum(YES, NO, x, odd, s_v);
+            });
+            ++b;
+        }
+        for (; b <= last_block; ++b) step(b, YES, copy_only);
     }
 
 #pragma unroll
