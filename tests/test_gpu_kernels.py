@@ -993,6 +993,44 @@ def test_attn_mfma_one_far_key_in_a_long_context(k, path):
         kc[page, :, slot, :] = kept
 
 
+@pytest.mark.parametrize("d,nq,nkv,bs,window,chunk,start,count", [
+    (128, 4, 4, 16, 0, 0, 0, 130),       # items of 128 tokens: the wavefronts' walks end in different blocks
+    (128, 4, 4, 48, 70, 0, 37, 131),     # and start in different ones; pages that a block's keys do not fill evenly
+    (128, 8, 2, 80, 0, 0, 63, 17),       # two blocks, a part of an item
+    (64, 4, 4, 64, 33, 0, 5, 260), (32, 4, 4, 48, 0, 96, 50, 200), (192, 4, 4, 16, 100, 0, 0, 129),
+    (128, 24, 3, 16, 0, 0, 0, 1100),     # more items than fill the first turn of three heads
+    (128, 32, 8, 16, 0, 0, 0, 2080)])    # more workgroups than find a place at once
+def test_prompt_portions_walk_their_own_blocks(k, d, nq, nkv, bs, window, chunk, start, count):
+    """Tokens of a portion against the plain formula over just the keys that each sees.  Weights rounded to bfloat16 move a sum of
+    values below 4.5 by 2^-9 of that at most, and so does the result's own rounding: 1.8e-2 together."""
+    from pulse_infer_amd.ops import attention_mfma as M
+    dtype, n = torch.bfloat16, start + count
+    pages = (n + bs - 1) // bs
+    perm = torch.randperm(pages + 2, generator=torch.Generator().manual_seed(11)).tolist()[:pages]
+    kc, vc = _cache(pages + 2, nkv, bs, d, dtype)
+    _stale(kc, vc)
+    ks, kref = as_stored(rnd(n, nkv, d, seed=601), dtype)
+    vs, vref = as_stored(rnd(n, nkv, d, seed=602).clamp(-4.5, 4.5), dtype)
+    _fill_cache(kc, vc, ks, vs, perm, bs)
+    q, qref = as_stored(rnd(count, nq * d, seed=603), dtype)
+    out = torch.zeros(count, nq * d, dtype=dtype, device=DEV)
+
+    class E:
+        first_row = 0
+    E.count, E.start = count, start
+    items = torch.tensor(M.build_items([(0, E)], M.portion_tokens(nq // nkv, d)), dtype=torch.int32, device=DEV)
+    pos = torch.arange(start, n, dtype=torch.int32, device=DEV)
+    M.attn_prefill(q, out, nq, nkv, d, kc, vc, pos, torch.tensor([perm], dtype=torch.int32, device=DEV), items, d ** -0.5, window,
+                   chunk=chunk)
+    got = out.cpu().to(F64).reshape(count, nq, d)
+    assert bool(got.isfinite().all())
+    for i in sorted({*range(0, count, max(1, count // 24)), count - 1, *(t - start for t in (63, 64, 95, 96, 127, 128) if start <= t < n)}):
+        t = start + i
+        low = t - t % chunk if chunk else max(0, t - window + 1) if window else 0
+        want = P.causal_attention(qref[i:i + 1].reshape(1, nq, d), kref[low:t + 1], vref[low:t + 1], d ** -0.5, None, [t - low])
+        assert torch.allclose(got[i], want[0], atol=2e-2, rtol=0), (t, float((got[i] - want[0]).abs().max()))
+
+
 def test_attn_mfma_refuses_other_sizes(k):
     from pulse_infer_amd.ops import KernelError
     from pulse_infer_amd.ops import attention_mfma as M
