@@ -1030,7 +1030,7 @@ struct WideShape {
 #else
 #define PULSE_WIDE_WAVES_PER_EU PULSE_ATTN_WAVES_PER_EU
 #endif
-// s_kv: 2 * Shape::STAGE values of LDS, a stage after the other, the K block first; (bx, by, bz) of (items, heads, splits): the workgroup.
+// s_kv: 2 * Shape::STAGE values of LDS, a stage after the other, the K block first; (bx, by, bz) of (heads, items, splits): the workgroup.
 template <int CT, int KT, int NW, int VD>
 __device__ __forceinline__ void attn_prefill_wide_workgroup(const MfmaArgs& a, const int per, const int bx, const int by, const int bz,
                                                             const int items, const int heads, bf16_t* const s_kv) {
@@ -1048,11 +1048,17 @@ __device__ __forceinline__ void attn_prefill_wide_workgroup(const MfmaArgs& a, c
     // of the list instead, the shortest beside the longest.  One prompt, 32 heads on 8, against items in a row for every head
     // (half of the heads backwards): 2,048 tokens 57.6 -> 55 us (56.7 without the turn), 2,560 91 -> 74, 3,072 125 -> 97,
     // 4,096 187 (in two splits, with their merge) -> 160, 8,192 575 -> 514, 16,384 2,122 -> 1,988.
+    // (Divisions stand behind branches: one takes as long as a trip to LDS, and short prompts are all front.)
     constexpr int UNITS = 256;
-    const int place = bx + items * by, turn = place / heads, first_turns = UNITS / heads;
-    const int item = items * heads <= 2 * UNITS && turn >= first_turns ? turn - first_turns : items - 1 - turn;
-    const int g = place % heads / a.head_chunks;
-    const int chunk = place % heads % a.head_chunks;
+    int item = items - 1 - by, g = bx, chunk = 0;
+    if (items * heads <= 2 * UNITS && (by + 1) * heads > UNITS) {
+        const int first_turns = UNITS / heads;
+        if (by >= first_turns) item = by - first_turns;
+    }
+    if (a.head_chunks > 1) {
+        g = bx / a.head_chunks;
+        chunk = bx % a.head_chunks;
+    }
     const int tid = threadIdx.x;
     const int wave = uniform(tid / PULSE_WAVE);
     const int lane = tid % PULSE_WAVE;
@@ -1076,8 +1082,8 @@ __device__ __forceinline__ void attn_prefill_wide_workgroup(const MfmaArgs& a, c
     const int* bt = a.block_table + static_cast<int64_t>(uniform(a.items[4 * item + 2])) * a.bt_width;
 
     // this wavefront's column tiles and this lane's column in each
-    const int tc = r / a.gp;
-    const int hc = r % a.gp + chunk * 16;
+    const int tc = r >> (31 - __builtin_clz(a.gp));   // (a power of two)
+    const int hc = (r & (a.gp - 1)) + chunk * 16;
     bool col_ok[CT];
     int col_row[CT], pos_c[CT];
     int t_hi[CT], t_pos0[CT], t_lo[CT], t_hi_lo[CT];  // per tile: last and first position, lowest and highest window start
@@ -1149,7 +1155,8 @@ __device__ __forceinline__ void attn_prefill_wide_workgroup(const MfmaArgs& a, c
     // are made from it a step ahead, between the products.  From block to block the tile moves on by BK keys.
     const int first_block = max(lo_item, split_begin) / BK;
     const int last_block = split_last / BK;
-    const int pages_on = BK / a.page_size, slots_on = BK % a.page_size;
+    int pages_on, slots_on;
+    page_of(BK, a.page_size, a.page_shift, pages_on, slots_on);
     int tile_key = first_block * BK + 16 * wave, tile_page, tile_slot;   // of the tile whose page is asked for next
     page_of(tile_key, a.page_size, a.page_shift, tile_page, tile_slot);
     struct Tile { int page, slot; bool there; };
@@ -1535,10 +1542,13 @@ __device__ __forceinline__ void attn_prefill_wide_workgroup(const MfmaArgs& a, c
     }
 }
 
+constexpr int GRID_ITEMS = 65535;   // the heads run along the grid's x, the items along its y, or the other way round where they are more than this
 template <int CT, int KT, int NW>
 __global__ __launch_bounds__(NW* PULSE_WAVE) PULSE_WIDE_WAVES_PER_EU void attn_prefill_wide_kernel(MfmaArgs a, int per) {
     __shared__ __attribute__((aligned(1024))) bf16_t s_kv[2 * WideShape<CT, KT, NW>::STAGE];
-    attn_prefill_wide_workgroup<CT, KT, NW, D>(a, per, blockIdx.x, blockIdx.y, blockIdx.z, gridDim.x, gridDim.y, s_kv);
+    const bool turned = a.n_items > GRID_ITEMS;
+    attn_prefill_wide_workgroup<CT, KT, NW, D>(a, per, turned ? blockIdx.y : blockIdx.x, turned ? blockIdx.x : blockIdx.y, blockIdx.z, a.n_items,
+                                              turned ? gridDim.y : gridDim.x, s_kv);
 }
 
 #define PULSE_NARROW_VALUES (PULSE_HEAD_DIM == 192 && PULSE_WIDE_CT == 2)
@@ -1550,7 +1560,9 @@ constexpr int NARROW_VALUES = 128;
 template <int CT, int KT, int NW>
 __global__ __launch_bounds__(NW* PULSE_WAVE) __attribute__((amdgpu_waves_per_eu(2))) void attn_prefill_values_kernel(MfmaArgs a, int per) {
     __shared__ __attribute__((aligned(1024))) bf16_t s_kv[2 * WideShape<CT, KT, NW, NARROW_VALUES>::STAGE];
-    attn_prefill_wide_workgroup<CT, KT, NW, NARROW_VALUES>(a, per, blockIdx.x, blockIdx.y, blockIdx.z, gridDim.x, gridDim.y, s_kv);
+    const bool turned = a.n_items > GRID_ITEMS;
+    attn_prefill_wide_workgroup<CT, KT, NW, NARROW_VALUES>(a, per, turned ? blockIdx.y : blockIdx.x, turned ? blockIdx.x : blockIdx.y, blockIdx.z, a.n_items,
+                                              turned ? gridDim.y : gridDim.x, s_kv);
 }
 #endif
 
@@ -1572,7 +1584,7 @@ __global__ __launch_bounds__(NW* PULSE_WAVE) PULSE_ATTN_WAVES_PER_EU void attn_b
         attn_mfma_workgroup<false>(tokens, block, *reinterpret_cast<MfmaShared<false>*>(lds));
     } else {
         const int at = block - token_blocks;
-        attn_prefill_wide_workgroup<CT, KT, NW, D>(portions, per, at % items, at / items, 0, items, heads, reinterpret_cast<bf16_t*>(lds));
+        attn_prefill_wide_workgroup<CT, KT, NW, D>(portions, per, at % heads, at / heads, 0, items, heads, reinterpret_cast<bf16_t*>(lds));
     }
 }
 #endif
@@ -2046,14 +2058,18 @@ int attn_prefill(const void* q, int64_t q_stride, void* out, int64_t o_stride, c
                       page_size, num_pages, scale, window, split_size, n_splits, part_o, part_ml, extras)) return 1;
     if (tokens == 0 || n_items == 0) return 0;
     const int gp = a.gp;
+#if PULSE_WIDE
+    const unsigned heads = nkv * a.head_chunks;
+    const dim3 grid = n_items > GRID_ITEMS ? dim3(n_items, heads, n_splits) : dim3(heads, n_items, n_splits);
+#endif
 #if PULSE_WIDE && PULSE_NARROW_VALUES
     if (values <= NARROW_VALUES)
-        hipLaunchKernelGGL((attn_prefill_values_kernel<WIDE_CT, 4, WIDE_NW>), dim3(n_items, nkv * a.head_chunks, n_splits),
+        hipLaunchKernelGGL((attn_prefill_values_kernel<WIDE_CT, 4, WIDE_NW>), grid,
                            dim3(WIDE_NW * PULSE_WAVE), 0, stream, a, 16 / gp);
     else
 #endif
 #if PULSE_WIDE
-    hipLaunchKernelGGL((attn_prefill_wide_kernel<WIDE_CT, 4, WIDE_NW>), dim3(n_items, nkv * a.head_chunks, n_splits),
+    hipLaunchKernelGGL((attn_prefill_wide_kernel<WIDE_CT, 4, WIDE_NW>), grid,
                        dim3(WIDE_NW * PULSE_WAVE), 0, stream, a, 16 / gp);
     if (n_splits > 1) {
         PULSE_LAUNCH_CHECK("attn_prefill");
