@@ -10,14 +10,16 @@
 // pass for SwiGLU behind it) and this package's shared-out product for up to 192 rows; in brackets behind a figure, what it
 // takes inside a step, between other kernels and with the chip warm:
 //                                   97 rows              192                  357                 509
-//   gate + up, 24,576 x 4,096       43 [41]              55                   73 [70]             90 [86]
+//   gate + up, 24,576 x 4,096       38 [39]              53                   66 [68]             84 [88]
 //     library                       54                   64                   84                  96
-//   qkv, 6,144 x 4,096              19 [20]              26                   33 [33]             36 [36]
+//   qkv, 6,144 x 4,096              19 [20]              26                   32 [34]             35 [37]
 //     library                       25                   36                   41                  42
-//   o, 4,096 x 4,096, shares        13 [14]              17                   21 [22]             25 [25]
+//   o, 4,096 x 4,096, shares        12 [14]              14                   21 [24]             24 [26]
 //     library / shared out          25 / 16              37 / 21              29                  32
-//   down, 4,096 x 12,288, shares    25 [27]              31                   43 [46]             53 [52]
+//   down, 4,096 x 12,288, shares    24 [25]              31                   39 [43]             52 [55]
 //     library / shared out          44 / 34              92 / 47              52, shared [46]     59, shared [60]
+// (2,048 rows, inside a step, against the library's: gate + up 284 to 310 for 278 + 30, down in two shares 142 to 155, o 61 to 66, qkv 77 to
+// 84 for its 84; 8,192 rows of gate + up 1,095 to 1,112, 1.49 to 1.51 PFLOP/s.)
 // From some 260 rows on tiles of 192 or 256 rows of X (their weights through three stages, X, which comes from L2, through
 // two where LDS holds no third) take the place of the library's: 357 rows of gate + up ran 96 us in tiles of 192 x 128.
 // Steps of 32 of K in twice the stages, the other way to fit such tiles, bring 64 bytes of a row at a time, which a unit

@@ -504,6 +504,7 @@ void launch_tiles(GroupArgs a, int max_tiles, hipStream_t stream) {
 //   128 rows (weights 256, 3 stages)                       90/130   94/134  95/139   95/144  97/145  163/239  143/246
 //     not past the caches                                  96/138  101/147 102/150  104/154 107/158  164/236  138/241  199/309  276/452  480/786
 //   192 rows (weights 192, down 256; X for down in 2 stages)                                         109/175  156/240  155/241  229/368  450/704
+//     (since the loop's smaller matrix instruction and one-instruction copies, and the faster SwiGLU: 2,048 tokens 197/319)
 //   the kernels above, 32 rows, K shared           78/111 110/167  219/351
 //   the kernels above, 128 rows                   150/231 150/231                                   370/688
 template <bool DOWN>

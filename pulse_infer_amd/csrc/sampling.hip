@@ -1628,7 +1628,8 @@ extern "C" int pulse_sample_options(const void* params, const int64_t* numbers, 
 // these either (many equal values at the edge, a k beyond half of what the segments hold) as pulse_sample does.  What a row's choice
 // is does not depend on the other rows.  Whole steps of rows with
 // mixed options, the host's part among it, us, before the histogram's kernels finished rows: 32,000 values, 3 / 16 / 64 rows
-// 139 / 155 / 191 -> 93 / 119 / 162; 151,936 values 212 / 247 / 331 -> 101 / 130 / 202.
+// 139 / 155 / 191 -> 93 / 119 / 162; 151,936 values 212 / 247 / 331 -> 101 / 130 / 202.  (32 rows of 151,936 since masses and candidates
+// come from one reading and the options are put together in native code: 160 -> 101.)
 // Scratch, with chunks = pulse_sample_chunks(vocab): part_max, part_mass (float32), part_idx, seg_n (int32) of rows * chunks entries; seg_i (int32), seg_x (float32) of rows * chunks * pulse_sample_segment()
 // entries; done (int32) of rows entries; and, optional (null: the rows that are left are gone over by their own workgroups
 // alone, with the same choices, as where it does not start at a multiple of 8 bytes), rest (int32) of rows *
