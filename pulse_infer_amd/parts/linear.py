@@ -102,6 +102,10 @@ class Linear:
                     and out.stride(0) % 8 == 0 and out.data_ptr() % 16 == 0:
                 kernels.gemm_stages(x, w, out)
                 return out
+            if own and out.dtype == torch.float32 and out.is_contiguous() and self.takes_stages_float32(x, w) \
+                    and out.data_ptr() % 16 == 0:
+                kernels.gemm_stages(x, w, out.view(1, *out.shape))
+                return out
             if own and out.dtype == torch.bfloat16 and self.takes_tiles(x, w) and out.stride(1) == 1 \
                     and out.stride(0) % 8 == 0 and out.data_ptr() % 16 == 0:
                 kernels.gemm_tile(x, w, out)
@@ -119,7 +123,7 @@ class Linear:
                     torch.matmul(x, w.t(), out=out)
                 return out
             if out.dtype == torch.float32 and out.is_contiguous():
-                # float32 results of many rows (logits): the library's product with a float32 output
+                # float32 results of many rows: the library's product with a float32 output
                 with timing.region("library matmul (float32 out)"):
                     torch.mm(x, w.t(), out_dtype=torch.float32, out=out)
                 return out
@@ -282,6 +286,18 @@ class Linear:
         if rows >= self.TILE_MIN_ROWS and (OWN_MANY_ROWS == "none" or self.takes_tiles(x, w, swiglu)):
             return False
         return swiglu or self.fills_stages(rows, n, k)
+
+    STAGE_RATE_FLOAT32 = 1000           # with float32 results, which take twice as long to store
+
+    def takes_stages_float32(self, x: torch.Tensor, w: torch.Tensor) -> bool:
+        """Whether a product of more than ``STAGE_ROWS_SHARES`` rows with float32 results runs as this package's product in stages:
+        by its estimate, as plain ones (us, library / this, by estimated flops a picosecond: 5,120 x 5,120 at 1,024 rows (672) 53 /
+        62, 8,192 x 2,048 at 1,024 (922) 33 / 38; 5,120 x 5,120 at 1,536 (1,008) 67.4 / 68.0, 4,096 x 8,192 at 2,048 (1,075) 109 /
+        106, 32,000 x 4,096 at 544 (1,116) 139 / 126, 6,144 x 4,096 at 1,536 (1,210) 67 / 58, 12,288 x 4,096 at 4,096 (1,498) 301 / 278;
+        from 1,000 on 0.94 of the library's time over the 30 sizes measured)."""
+        rows, (n, k) = x.shape[0], w.shape
+        return (rows > self.STAGE_ROWS_SHARES and self.takes_stages(x, w)
+                and kernels.gemm_stages_time(rows, n, k) * 1000 * self.STAGE_RATE_FLOAT32 <= 2 * rows * n * k)
 
     def fills_stages(self, rows: int, n: int, k: int) -> bool:
         """Whether a plain product's tiles keep enough compute units busy: its inner dimension cannot be cut (the result is

@@ -251,3 +251,22 @@ def test_product_in_stages_of_rows_gigabytes_apart(far):
     kernels.gemm_stages(x, w, near)
     kernels.gemm_stages(xf, wf, out)
     assert torch.equal(out, near)
+
+
+@pytest.mark.parametrize("rows,gap,contiguous", [(1030, 0, True), (1030, 8, True), (1030, 4, True), (1030, 0, False), (520, 0, True)])
+def test_float32_results_of_many_rows(rows, gap, contiguous):
+    """16,384 x 1,024 with float32 results: in stages from the estimate's line on, elsewhere as before (fewer rows, rows that are
+    not 16 bytes aligned, results further apart), the same sums within float32 in any order."""
+    from pulse_infer_amd.parts.linear import Linear
+
+    n, k = 16384, 1024
+    lin = Linear((rnd(n, k, seed=2) * k ** -0.5).to(torch.bfloat16).to(DEV), "bfloat16")
+    x = torch.empty(rows, k + gap, dtype=torch.bfloat16, device=DEV)[:, :k]
+    x.copy_(rnd(rows, k, seed=1))
+    assert lin.takes_stages_float32(x, lin.weight) == (rows > 1024 and gap % 8 == 0)
+    out = torch.full((rows, n if contiguous else n + 4), float("nan"), device=DEV)[:, :n]
+    lin.forward(x, out)
+    some = [0, 1, 255, 256, 511, rows - 1]
+    xs, ws = x[some].cpu().to(F64), lin.weight.cpu().to(F64)
+    assert bool(out.isfinite().all())
+    assert ((out[some].cpu().to(F64) - xs @ ws.T).abs() <= (k + 2) * 2.0 ** -24 * (xs.abs() @ ws.abs().T)).all()
