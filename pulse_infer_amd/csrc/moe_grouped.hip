@@ -456,16 +456,15 @@ __global__ __launch_bounds__(WN* WM* PULSE_WAVE) void moe_tile_kernel(GroupArgs 
                     for (int i = 0; i < 4; ++i) {
                         // an expert that is fed weight * x: both products are linear, so the factor goes onto their results
                         float gate = loop.acc[f][g][i] * wgt, up = loop.acc[f + 1][g][i] * wgt;
-                        float slope = 1.0f;
+                        // (expf and a division, whose results are within 8 * 2^-24 of the function: the hardware's exponential and
+                        // reciprocal took 12 us less, 16 experts of 1,536 x 4,096, 8,192 pairs 197 for 209 us, but were up to 30 * 2^-24 off)
                         if (a.act_kind == 1) {   // clamped: min(g, limit) * sigmoid(1.702 g) * (clamp(u) + 1)
                             gate = fminf(gate, a.limit);
-                            up = fminf(fmaxf(up, -a.limit), a.limit) + 1.0f;
-                            slope = 1.702f;
+                            up = fminf(fmaxf(up, -a.limit), a.limit);
+                            v[i] = (__bf16)(gate / (1.0f + expf(-1.702f * gate)) * (up + 1.0f));
+                        } else {
+                            v[i] = (__bf16)(gate / (1.0f + expf(-gate)) * up);
                         }
-                        // (as in the products in stages: the reciprocal of a quarter is a normal number as long as the exponential is
-                        // finite; expf and a division, no nearer to 64 bits behind the rounding, took 12 us more: 16 experts of
-                        // 1,536 x 4,096, 8,192 pairs, 209 -> 197 us.)
-                        v[i] = (__bf16)(0.25f * gate * __builtin_amdgcn_rcpf(fmaf(0.25f, __expf(-slope * gate), 0.25f)) * up);
                     }
                     *reinterpret_cast<tile_bf16x4*>(at + f * 16) = v;
                 }
@@ -504,7 +503,7 @@ void launch_tiles(GroupArgs a, int max_tiles, hipStream_t stream) {
 //   128 rows (weights 256, 3 stages)                       90/130   94/134  95/139   95/144  97/145  163/239  143/246
 //     not past the caches                                  96/138  101/147 102/150  104/154 107/158  164/236  138/241  199/309  276/452  480/786
 //   192 rows (weights 192, down 256; X for down in 2 stages)                                         109/175  156/240  155/241  229/368  450/704
-//     (since the loop's smaller matrix instruction and one-instruction copies, and the faster SwiGLU: 2,048 tokens 197/319)
+//     (since the loop's smaller matrix instruction and one-instruction copies: 2,048 tokens 209/331)
 //   the kernels above, 32 rows, K shared           78/111 110/167  219/351
 //   the kernels above, 128 rows                   150/231 150/231                                   370/688
 template <bool DOWN>

@@ -142,3 +142,30 @@ def test_grouped_experts_do_not_depend_on_the_tiles_of_their_rows(hidden, ff, fo
     assert not torch.isnan(results[0][0]).any() and not torch.isnan(results[0][1]).any()
     for act, y in results[1:]:
         assert torch.equal(act, results[0][0]) and torch.equal(y, results[0][1])
+
+
+@pytest.mark.parametrize("low,high", [(0.1, 8.0), (-22.0, -15.0)])
+def test_activation_of_grouped_experts_is_rounded_once(low, high):
+    """silu(gate) * up is a float32 value within 8 units of 2^-24 of the function (the exponential 2 units, the sum, the quotient and the
+    product one each) and then rounded to bfloat16: what lies further from a tie than that is rounded as the function itself is.  Gates and ups are
+    products of two bfloat16 values, which float32 holds."""
+    from pulse_infer_amd.ops import kernels
+
+    hidden, ff, pairs, rows = 64, 448, 1920, 192
+    x, wg, wu = torch.zeros(pairs, hidden), torch.zeros(1, ff, hidden), torch.zeros(1, ff, hidden)
+    x[:, 0], x[:, 1] = 1.0 + torch.rand(pairs, generator=torch.Generator().manual_seed(1)), 1.0 + torch.arange(pairs) / 128 % 1
+    wg[0, :, 0] = torch.linspace(low, high, ff)              # (gates of up to twice that)
+    wu[0, :, 1] = rnd(ff, seed=2)
+    x, wg, wu = (t.to(torch.bfloat16) for t in (x, wg, wu))
+    g, u = (x.to(F64)[:, i:i + 1] * w.to(F64)[0, :, i] for i, w in ((0, wg), (1, wu)))
+    want = g * torch.sigmoid(g) * u
+    act = torch.full((pairs, ff), float("nan"), dtype=torch.bfloat16, device=DEV)
+    y = torch.full((pairs, hidden), float("nan"), device=DEV)
+    wd = torch.zeros(1, hidden, ff, dtype=torch.bfloat16)
+    idx = torch.zeros(pairs, 1, dtype=torch.int32)
+    ints = torch.full((2 * pairs + 3 * kernels.moe_max_tiles(pairs, 1, rows) + 1,), -5, dtype=torch.int32, device=DEV)
+    kernels.moe_grouped(x.to(DEV), wg.to(DEV), wu.to(DEV), wd.to(DEV), idx.to(DEV), torch.ones(pairs, 1).to(DEV), act, y, None, ints, rows)
+    below, above = (torch.nextafter(act.cpu(), torch.full((), s * float("inf"), dtype=torch.bfloat16)).to(F64) for s in (-1, 1))
+    got = act.cpu().to(F64)
+    bound = 8 * 2.0 ** -24 * want.abs()
+    assert ((want >= (got + below) / 2 - bound) & (want <= (got + above) / 2 + bound)).all()
