@@ -15,6 +15,15 @@ from ..ops import kernels
 from .params import SamplingParams
 
 
+def one_a_row(values: Sequence, rows: int, name: str) -> Sequence:
+    """``values`` for ``rows`` rows: as they are, or the one there is for all of them."""
+    if len(values) == 1 and rows > 1:
+        return [values[0]] * rows
+    if len(values) < rows:
+        raise ValueError(f"sampling: {len(values)} {name} for {rows} rows")
+    return values
+
+
 class Sampler:
     def __init__(self, vocab_size: int, num_slots: int, device: torch.device,
                  banned_tokens: Optional[Sequence[int]] = None):
@@ -86,6 +95,11 @@ class Sampler:
                 self._part_idx = torch.empty(need, dtype=torch.int32, device=self.device)
             kernels.argmax(logits, out, self._part_val, self._part_idx)
             return out
+        params = one_a_row(params, rows, "options")
+        if len(params) != rows:
+            raise ValueError(f"sampling: options of {len(params)} requests for {rows} rows")
+        slots, counters, default_seeds = (one_a_row(v, rows, name) for v, name in (
+            (slots, "slots"), (counters, "counters"), (default_seeds, "seeds")))
         # every per-row option in one upload: rows of a [6, R] int32 array, the float ones as their bit patterns
         turn = self._turn
         self._turn = 1 - turn

@@ -53,3 +53,19 @@ def test_a_steps_options_as_the_kernels_read_them():
                 lambda: kernels.sample_options(host.float(), None, packed, slots, counters, seeds)):
         with pytest.raises(KernelError):
             bad()
+
+
+def test_options_for_other_than_a_steps_rows_are_refused():
+    """What the kernels read of a row is the row's own: fewer or more options than rows are an error, one may stand for all."""
+    import torch
+
+    from pulse_infer_amd.sampling.sampler import Sampler, one_a_row
+
+    sampler, drawn = Sampler(100, 4, torch.device("cpu")), SamplingParams(temperature=0.7, presence_penalty=1.0)
+    for params, slots, counters, seeds in (([drawn] * 3, range(4), [0] * 4, [0] * 4), ([drawn] * 5, range(5), [0] * 5, [0] * 5),
+                                           ([drawn] * 4, range(3), [0] * 4, [0] * 4), ([drawn] * 4, range(4), [0] * 2, [0] * 4),
+                                           ([drawn] * 4, range(4), [0] * 4, [])):
+        with pytest.raises(ValueError, match="sampling"):
+            sampler.launch(torch.zeros(4, 100), params, slots, counters, seeds)
+    assert one_a_row([drawn], 3, "options") == [drawn] * 3 and one_a_row([7], 1, "seeds") == [7]
+    assert list(one_a_row(range(5), 4, "slots")) == [0, 1, 2, 3, 4]      # (those behind the rows are not read)
