@@ -1590,11 +1590,11 @@ static uint64_t splitmix64(uint64_t x) {
 }
 
 // The options of a step's rows as the kernels read them, host memory [6, room]: temperature, top_k, top_p, the uniform number that
-// depends on the row's seed and counter alone, penalty, slot (-1 without a penalty); and their copy to `dev`, queued (null: none).
+// depends on the row's seed and counter alone, penalty, slot (-1 without a penalty).
 // `numbers`: the rows' slots, then their counters; `seeds`: for rows without one of their own (null: none is).  `kinds`: 1 if a row uses top-k, 2
 // top-p, 4 a penalty.  (The host's part of a step of 32 rows up to its last launch, 78 us with this in the interpreter, 43 so.)
-extern "C" int pulse_sample_options(const void* params, const int64_t* numbers, const uint64_t* seeds, int rows, int32_t* host, int64_t room, int32_t* dev,
-                                    int* kinds, hipStream_t stream) {
+extern "C" int pulse_sample_options(const void* params, const int64_t* numbers, const uint64_t* seeds, int rows, int32_t* host, int64_t room,
+                                    int* kinds) {
     PULSE_REQUIRE(rows >= 0 && room >= rows && host && kinds && (rows == 0 || (params && numbers)), "sample_options: bad arguments");
     float* const floats = reinterpret_cast<float*>(host);
     *kinds = 0;
@@ -1612,10 +1612,6 @@ extern "C" int pulse_sample_options(const void* params, const int64_t* numbers, 
         floats[4 * room + r] = p.penalty;
         host[5 * room + r] = penalized ? static_cast<int32_t>(numbers[r]) : -1;
         *kinds |= (p.top_k > 0 ? 1 : 0) | (p.top_p > 0.f && p.top_p < 1.f ? 2 : 0) | (penalized ? 4 : 0);
-    }
-    if (dev && rows > 0) {
-        const hipError_t e = hipMemcpyAsync(dev, host, static_cast<size_t>(5 * room + rows) * 4, hipMemcpyHostToDevice, stream);
-        PULSE_REQUIRE(e == hipSuccess, "sample_options: the copy failed: %s", hipGetErrorString(e));
     }
     return 0;
 }

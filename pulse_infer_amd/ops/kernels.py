@@ -1077,7 +1077,8 @@ def sample_options(host: torch.Tensor, dev: Optional[torch.Tensor], rows: Sequen
     """The options of a step's rows (``SamplingParams.packed``) as the sampling kernels read them, into ``host`` int32 [6, room] in host
     memory: temperature, top_k, top_p, the row's uniform number (its seed's ``counters[r]``-th, ``seeds[r]`` where the request has no seed
     of its own), penalty, slot (-1 without a penalty), the floats as their bits; from there to ``dev`` (of the same shape; none: no copy),
-    queued.  Whether some row uses top-k, top-p, a penalty."""
+    queued.  Whether some row uses top-k, top-p, a penalty.  (torch makes the copy: it keeps pinned memory that is let go of back
+    from others until the copies out of it have run.)"""
     n, packed = len(rows), b"".join(rows)
     _need(host.dtype == torch.int32 and host.dim() == 2 and host.shape[0] == 6 and host.shape[1] >= n and host.is_contiguous()
           and host.device.type == "cpu", "sample_options: host must be int32 [6, rows or more] in host memory")
@@ -1091,8 +1092,9 @@ def sample_options(host: torch.Tensor, dev: Optional[torch.Tensor], rows: Sequen
     others = None if own_seeds else array("Q", [d & 0xFFFFFFFFFFFFFFFF for d in seeds[:n]])
     kinds = ctypes.c_int(0)
     call("pulse_sample_options", packed, ctypes.c_void_p(numbers.buffer_info()[0]),
-         ctypes.c_void_p(others.buffer_info()[0] if others is not None else 0), _i32(n), _ptr(host), _i64(host.shape[1]), _ptr(dev),
-         ctypes.byref(kinds), _stream() if dev is not None else None)
+         ctypes.c_void_p(others.buffer_info()[0] if others is not None else 0), _i32(n), _ptr(host), _i64(host.shape[1]), ctypes.byref(kinds))
+    if dev is not None:
+        dev.copy_(host, non_blocking=True)
     used = kinds.value
     return bool(used & 1), bool(used & 2), bool(used & 4)
 

@@ -689,6 +689,32 @@ def test_draws_at_the_edges_of_a_chunks_steps(k, vocab):
     assert out.tolist() == want
 
 
+def test_a_steps_options_keep_their_memory_until_they_are_up(k):
+    """A sampler that goes while its options' copy is queued behind other work: nobody is given the pinned memory they lie in before
+    the copy has run."""
+    from pulse_infer_amd.sampling import SamplingParams
+    from pulse_infer_amd.sampling.sampler import Sampler
+
+    sampler, x, y = Sampler(1000, 4, torch.device(DEV)), *(torch.zeros(8192, 8192, dtype=torch.bfloat16, device=DEV) for _ in range(2))
+    logits, params = torch.zeros(4, 1000, device=DEV), [SamplingParams(temperature=0.7)] * 4
+    launch = lambda: sampler.launch(logits, params, range(4), [0] * 4, [1] * 4)
+    for _ in range(2):                           # (both pairs of buffers made, the kernels loaded)
+        launch()
+    torch.mm(x, x, out=y)
+    torch.cuda.synchronize()
+    for _ in range(100):                         # some 80 ms of work in front
+        torch.mm(x, x, out=y)
+    launch()
+    behind = torch.cuda.Event()
+    behind.record()
+    used = {t.data_ptr(): t.shape for t in sampler._options_host}
+    del sampler, launch
+    others = [torch.empty(shape, dtype=torch.int32, pin_memory=True) for shape in used.values()]
+    assert not behind.query(), "the work in front was too short to tell"
+    torch.cuda.synchronize()
+    assert sum(t.data_ptr() in used for t in others) < 2
+
+
 def test_kernels_refuse_what_they_cannot_do(k):
     from pulse_infer_amd.ops import KernelError
     with pytest.raises(KernelError, match="GPU"):
