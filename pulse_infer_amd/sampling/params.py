@@ -13,6 +13,7 @@ from __future__ import annotations
 import ctypes
 import struct
 from dataclasses import dataclass
+from functools import cached_property
 from typing import Optional
 
 
@@ -40,12 +41,14 @@ class SamplingParams:
             raise ValueError(f"top_p must lie in [0, 1], got {self.top_p}")
         if self.presence_penalty < 0.0:
             raise ValueError(f"presence_penalty must not be negative, got {self.presence_penalty}")
-        # (made once a request: a step puts its rows' options together as they are)
+
+    @cached_property
+    def packed(self) -> bytes:
+        """The options as a step puts its rows' together, made once a request."""
         seed = 0 if self.seed is None else int(self.seed) & _MASK
         top_k = min(int(self.top_k), 0x7FFFFFFF)
         single = lambda v: ctypes.c_float(v).value      # (beyond float32's range: infinite)
-        object.__setattr__(self, "packed", _ROW.pack(single(self.temperature), top_k, self.top_p, single(self.presence_penalty), seed,
-                                                     self.seed is not None, 0))
+        return _ROW.pack(single(self.temperature), top_k, self.top_p, single(self.presence_penalty), seed, self.seed is not None, 0)
 
     @property
     def greedy(self) -> bool:

@@ -69,3 +69,15 @@ def test_options_for_other_than_a_steps_rows_are_refused():
             sampler.launch(torch.zeros(4, 100), params, slots, counters, seeds)
     assert one_a_row([drawn], 3, "options") == [drawn] * 3 and one_a_row([7], 1, "seeds") == [7]
     assert list(one_a_row(range(5), 4, "slots")) == [0, 1, 2, 3, 4]      # (those behind the rows are not read)
+
+
+def test_options_that_were_stored_field_by_field_can_be_drawn_with():
+    """Objects that were pickled before requests packed their options, or copied: the same row."""
+    import copy
+    import pickle
+
+    made = SamplingParams(temperature=0.7, top_k=5, seed=3)
+    stored = SamplingParams.__new__(SamplingParams)
+    stored.__dict__.update(temperature=0.7, top_k=5, top_p=0.0, presence_penalty=0.0, seed=3, ignore_eos=False)
+    assert stored == made and stored.packed == made.packed == pickle.loads(pickle.dumps(made)).packed == copy.copy(made).packed
+    assert hash(stored) == hash(made)
