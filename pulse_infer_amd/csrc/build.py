@@ -10,7 +10,9 @@ from __future__ import annotations
 
 import hashlib
 import os
+import re
 import shutil
+import struct
 import subprocess
 import sys
 import tempfile
@@ -97,6 +99,53 @@ def _log(msg: str) -> None:
     log.info(msg)
 
 
+# ------------------------------------------------------------------ what holds M0
+# Copies into LDS that follow each other take their place from M0, which one statement sets for several (lds_place and copy_to_place of
+# common.h): the compiler does not know that it lives on between them.  So nothing else in the compiled kernels may touch it.
+_TOUCHES_M0 = re.compile(r"\bm0\b|s_set_gpr_idx|movrel|s_sendmsg|_gws_")
+_SETS_PLACE = re.compile(r"\s*s_mov_b32 m0, s\d+\s*$")
+
+
+def m0_misuses(assembly: str) -> List[str]:
+    """The instructions of a disassembly that set or use M0 in any way but lds_place's."""
+    lines = [line.split("//")[0].rstrip() for line in assembly.splitlines()]
+    return [line.strip() for line, after in zip(lines, lines[1:] + [""]) if _TOUCHES_M0.search(line)
+            and not (_SETS_PLACE.match(line) and after.strip() == "s_nop 0")]
+
+
+def device_code(path: str) -> List[bytes]:
+    """The gfx950 code objects inside an object file or library."""
+    with open(path, "rb") as fh:
+        data = fh.read()
+    magic, found, at = b"__CLANG_OFFLOAD_BUNDLE__", [], 0
+    while (at := data.find(magic, at)) >= 0:
+        place = at + len(magic) + 8
+        for _ in range(struct.unpack_from("<Q", data, place - 8)[0]):
+            offset, size, length = struct.unpack_from("<QQQ", data, place)
+            if size and data[place + 24:place + 24 + length].endswith(ARCH.encode()):
+                found.append(data[at + offset:at + offset + size])
+            place += 24 + length
+        at += len(magic)
+    return found
+
+
+def check_m0(path: str) -> None:
+    """Refuses an object file or library in which something beside lds_place touches M0."""
+    objdump = next((p for p in (shutil.which("llvm-objdump"), "/opt/rocm/llvm/bin/llvm-objdump") if p and os.path.exists(p)), None)
+    if objdump is None:
+        _log(f"no llvm-objdump: {os.path.basename(path)} goes unchecked")
+        return
+    for code in device_code(path):
+        with tempfile.NamedTemporaryFile(suffix=".co") as fh:
+            fh.write(code)
+            fh.flush()
+            proc = subprocess.run([objdump, "-d", "--no-show-raw-insn", f"--mcpu={ARCH}", fh.name], capture_output=True, text=True)
+        if proc.returncode != 0:
+            raise RuntimeError(f"llvm-objdump failed on {path}:\n{proc.stderr[-4000:]}")
+        if wrong := m0_misuses(proc.stdout):
+            raise RuntimeError(f"{path}: M0 is not the copies' own: {wrong[:10]}")
+
+
 def build(force: bool = False, verbose: bool = True) -> str:
     """Compile everything and return the path of the library."""
     if not force:
@@ -131,6 +180,7 @@ def build(force: bool = False, verbose: bool = True) -> str:
         proc = subprocess.run(cmd, capture_output=True, text=True)
         if proc.returncode != 0:
             raise RuntimeError(f"hipcc failed on {name}:\n{proc.stderr[-4000:]}")
+        check_m0(obj)
         if verbose:
             _log(f"compiled {name} ({time.time() - t0:.0f} s)")
         return obj
@@ -216,6 +266,7 @@ def build_variant(source: str, defines: Dict[str, int], force: bool = False, ver
         proc = subprocess.run(cmd, capture_output=True, text=True)
         if proc.returncode != 0:
             raise RuntimeError(f"hipcc failed on {source}.hip {defines}:\n{proc.stderr[-4000:]}")
+        check_m0(tmp)
         os.replace(tmp, lib)
         with open(stamp, "w") as fh:
             fh.write(variant_hash(source, defines))

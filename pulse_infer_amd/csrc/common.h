@@ -75,8 +75,8 @@ __device__ __forceinline__ void load_to_lds(const void* base, uint32_t offset, u
 }
 
 // The same in a row: `lds_place` says where, the copies behind it bring 16 bytes a lane from `offset` + BYTES behind the base to BYTES
-// behind that place (-4,096 <= BYTES < 4,096), an instruction each.  (The place is kept in M0, which nothing that the compiler makes of these
-// kernels uses; their assembly was looked at.)
+// behind that place (-4,096 <= BYTES < 4,096), an instruction each.  (The place is kept in M0 from statement to statement, which the compiler does
+// not know: the build looks through what it made and refuses kernels in which anything else touches M0, check_m0 of build.py.)
 __device__ __forceinline__ void lds_place(uint32_t lds_base) { asm volatile("s_mov_b32 m0, %0\n\ts_nop 0" : : "s"(lds_base) : "memory", "m0"); }
 template <int BYTES, bool STREAM = false>
 __device__ __forceinline__ void copy_to_place(const void* base, uint32_t offset) {

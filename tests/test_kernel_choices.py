@@ -239,3 +239,18 @@ def test_keys_of_four_steps_are_not_cut_over_workgroups(units):
         n, steps = K.attn_wide_splits(items, 2, keys), (keys + 31) // 32
         assert 1 <= n <= 16 and (steps + n - 1) // n >= 3
         assert n == 1 or items * 2 * (n - 1) < 2 * units
+
+
+def test_nothing_but_the_copies_own_statement_touches_m0():
+    """The check of the build: it passes a statement that sets the copies' place, and finds every other use."""
+    from pulse_infer_amd.csrc import build
+
+    place = "\ts_mov_b32 m0, s41                                           // 000000002A00: BEFC0029\n\ts_nop 0   // 0\n"
+    copies = "\tglobal_load_lds_dwordx4 v1, s[2:3] offset:-4096 // 0\n\tv_mfma_f32_16x16x32_bf16 a[0:3], v[0:3], v[4:7], a[0:3] // 0\n"
+    assert build.m0_misuses((place + copies) * 2) == []
+    for wrong in ("\ts_mov_b32 m0, s3 // 0\n", "\ts_mov_b32 m0, -1 // 0\n\ts_nop 0\n", "\ts_set_gpr_idx_on s3, gpr_idx(SRC0) // 0\n",
+                  "\tv_movrels_b32_e32 v1, v2 // 0\n", "\ts_add_u32 s1, m0, s2 // 0\n", "\ts_sendmsg sendmsg(MSG_INTERRUPT) // 0\n",
+                  "\ts_mov_b32 m0, s3 // 0\n\tv_readlane_b32 s3, v1, m0 // 0\n"):
+        assert build.m0_misuses(place + wrong + copies)
+    if (lib := build.existing_library()) is not None:
+        assert len(build.device_code(lib)) > 10 and build.device_code(__file__) == []
