@@ -87,6 +87,7 @@ struct MfmaArgs {
     int chunk;       // > 0: a token sees the keys of its own chunk of this many positions (counted from 0) only; then no window
     int split_size;  // multiple of 32
     int n_splits;
+    int turn;        // prompt portions: the items, from the list's end, that find a compute unit of their own; 0: see attn_prefill_wide_workgroup
     // The longest context of the step as it is now, or null.  The launch (and a recording of it) is made for contexts
     // up to n_splits * split_size; with this the kernel of decoded tokens cuts the keys that are there into n_splits
     // even splits instead (see live_split_size), so that no split stands empty while another walks its full length.
@@ -1025,6 +1026,7 @@ struct WideShape {
     static_assert(KT == NW, "a wavefront copies one key tile and one value tile of every block");
 };
 
+constexpr bool ONE_A_UNIT = PULSE_WIDE_CT > 2 || PULSE_HEAD_DIM > 128;
 #if PULSE_WIDE_CT > 2 || PULSE_HEAD_DIM > 128   // (the accumulators take most of the registers, the stages most of LDS)
 #define PULSE_WIDE_WAVES_PER_EU __attribute__((amdgpu_waves_per_eu(1, 1)))
 #else
@@ -1033,7 +1035,7 @@ struct WideShape {
 // s_kv: 2 * Shape::STAGE values of LDS, a stage after the other, the K block first; (bx, by, bz) of (heads, items, splits): the workgroup.
 template <int CT, int KT, int NW, int VD>
 __device__ __forceinline__ void attn_prefill_wide_workgroup(const MfmaArgs& a, const int per, const int bx, const int by, const int bz,
-                                                            const int items, const int heads, bf16_t* const s_kv) {
+                                                            const int items, bf16_t* const s_kv) {
     using Shape = WideShape<CT, KT, NW, VD>;
     constexpr int NVT = VD / 16;            // tiles of 16 value channels
     constexpr int BK = Shape::BK;
@@ -1042,19 +1044,15 @@ __device__ __forceinline__ void attn_prefill_wide_workgroup(const MfmaArgs& a, c
     constexpr int P = Shape::P;
 
     // The order of the walks: one item of every head after the other, from the last item of the list to the first, so that the
-    // long walks (late portions of a prompt) start first and the short ones fill in behind them, and the eight workgroups that
+    // long walks (the list has them last) start first and the short ones fill in behind them, and the eight workgroups that
     // start together, one a die, take different heads: with 8 of them a die's cache holds one head's keys.  Where every workgroup
-    // finds a place at once, two a compute unit (workgroups w and w + 256), the second of a unit comes from the other end
-    // of the list instead, the shortest beside the longest.  One prompt, 32 heads on 8, against items in a row for every head
-    // (half of the heads backwards): 2,048 tokens 57.6 -> 55 us (56.7 without the turn), 2,560 91 -> 74, 3,072 125 -> 97,
-    // 4,096 187 (in two splits, with their merge) -> 160, 8,192 575 -> 514, 16,384 2,122 -> 1,988.
+    // finds a place at once, two a compute unit (workgroups w and w + units; `turn`, as the host knows whether they do), the second of a
+    // unit comes from the other end of the list instead, the shortest beside the longest.  One prompt, 32 heads on 8, against items
+    // in a row for every head (half of the heads backwards): 2,048 tokens 57.6 -> 55 us (56.7 without the turn), 2,560 91 -> 74, 3,072
+    // 125 -> 97, 4,096 187 (in two splits, with their merge) -> 160, 8,192 575 -> 514, 16,384 2,122 -> 1,988.
     // (Divisions stand behind branches: one takes as long as a trip to LDS, and short prompts are all front.)
-    constexpr int UNITS = 256;
     int item = items - 1 - by, g = bx, chunk = 0;
-    if (items * heads <= 2 * UNITS && (by + 1) * heads > UNITS) {
-        const int first_turns = UNITS / heads;
-        if (by >= first_turns) item = by - first_turns;
-    }
+    if (a.turn > 0 && by >= a.turn) item = by - a.turn;
     if (a.head_chunks > 1) {
         g = bx / a.head_chunks;
         chunk = bx % a.head_chunks;
@@ -1547,22 +1545,20 @@ template <int CT, int KT, int NW>
 __global__ __launch_bounds__(NW* PULSE_WAVE) PULSE_WIDE_WAVES_PER_EU void attn_prefill_wide_kernel(MfmaArgs a, int per) {
     __shared__ __attribute__((aligned(1024))) bf16_t s_kv[2 * WideShape<CT, KT, NW>::STAGE];
     const bool turned = a.n_items > GRID_ITEMS;
-    attn_prefill_wide_workgroup<CT, KT, NW, D>(a, per, turned ? blockIdx.y : blockIdx.x, turned ? blockIdx.x : blockIdx.y, blockIdx.z, a.n_items,
-                                              turned ? gridDim.y : gridDim.x, s_kv);
+    attn_prefill_wide_workgroup<CT, KT, NW, D>(a, per, turned ? blockIdx.y : blockIdx.x, turned ? blockIdx.x : blockIdx.y, blockIdx.z, a.n_items, s_kv);
 }
 
 #define PULSE_NARROW_VALUES (PULSE_HEAD_DIM == 192 && PULSE_WIDE_CT == 2)
+constexpr int NARROW_VALUES = 128;
 #if PULSE_NARROW_VALUES
 // Heads of 192 channels whose values fill 128 of them at most (the latent rows' expanded form): the stages are then 80 KB instead of
 // 96, so that two workgroups share a unit, two wavefronts a SIMD, and a sixth of the products falls away.  32 heads, a prompt of
 // 2,048: 192 -> 79 us, with the same bits.
-constexpr int NARROW_VALUES = 128;
 template <int CT, int KT, int NW>
 __global__ __launch_bounds__(NW* PULSE_WAVE) __attribute__((amdgpu_waves_per_eu(2))) void attn_prefill_values_kernel(MfmaArgs a, int per) {
     __shared__ __attribute__((aligned(1024))) bf16_t s_kv[2 * WideShape<CT, KT, NW, NARROW_VALUES>::STAGE];
     const bool turned = a.n_items > GRID_ITEMS;
-    attn_prefill_wide_workgroup<CT, KT, NW, NARROW_VALUES>(a, per, turned ? blockIdx.y : blockIdx.x, turned ? blockIdx.x : blockIdx.y, blockIdx.z, a.n_items,
-                                              turned ? gridDim.y : gridDim.x, s_kv);
+    attn_prefill_wide_workgroup<CT, KT, NW, NARROW_VALUES>(a, per, turned ? blockIdx.y : blockIdx.x, turned ? blockIdx.x : blockIdx.y, blockIdx.z, a.n_items, s_kv);
 }
 #endif
 
@@ -1584,7 +1580,7 @@ __global__ __launch_bounds__(NW* PULSE_WAVE) PULSE_ATTN_WAVES_PER_EU void attn_b
         attn_mfma_workgroup<false>(tokens, block, *reinterpret_cast<MfmaShared<false>*>(lds));
     } else {
         const int at = block - token_blocks;
-        attn_prefill_wide_workgroup<CT, KT, NW, D>(portions, per, at % heads, at / heads, 0, items, heads, reinterpret_cast<bf16_t*>(lds));
+        attn_prefill_wide_workgroup<CT, KT, NW, D>(portions, per, at % heads, at / heads, 0, items, reinterpret_cast<bf16_t*>(lds));
     }
 }
 #endif
@@ -2042,11 +2038,24 @@ int fill_portions(MfmaArgs& a, const void* q, int64_t q_stride, void* out, int64
     a.scale_log2e = scale * 1.4426950408889634f;
     a.window = window; a.split_size = n_splits > 1 ? split_size : 0; a.n_splits = n_splits;
     a.n_items = n_items;
+    a.turn = 0;
     a.live_context = nullptr;
     a.plan = nullptr;
     a.part_o = n_splits > 1 ? part_o : nullptr; a.part_ml = n_splits > 1 ? part_ml : nullptr;
     if (tokens == 0 || n_items == 0) return 0;
     return take_gate(a, extras, nq, scale);
+}
+
+// MfmaArgs::turn of a launch of its own (in attn_beside_kernel the decoded tokens' workgroups come first): none where a unit holds one
+// workgroup (32 heads of 192 channels, 2,048 tokens: 89 us with a turn, 73 without, two prompts of 1,024 64 and 48), with splits, or where
+// not all find a place at once.
+int first_turn([[maybe_unused]] int64_t n_items, [[maybe_unused]] int64_t heads, [[maybe_unused]] int n_splits, [[maybe_unused]] int values) {
+#if PULSE_WIDE
+    const int64_t units = pulse_compute_units();
+    if (n_splits > 1 || (ONE_A_UNIT && !(PULSE_NARROW_VALUES && values <= NARROW_VALUES))) return 0;
+    if (n_items * heads > units && n_items * heads <= 2 * units) return static_cast<int>(units / heads);
+#endif
+    return 0;
 }
 
 int attn_prefill(const void* q, int64_t q_stride, void* out, int64_t o_stride, const void* kcache, const void* vcache,
@@ -2061,6 +2070,7 @@ int attn_prefill(const void* q, int64_t q_stride, void* out, int64_t o_stride, c
 #if PULSE_WIDE
     const unsigned heads = nkv * a.head_chunks;
     const dim3 grid = n_items > GRID_ITEMS ? dim3(n_items, heads, n_splits) : dim3(heads, n_items, n_splits);
+    a.turn = first_turn(n_items, heads, n_splits, values);
 #endif
 #if PULSE_WIDE && PULSE_NARROW_VALUES
     if (values <= NARROW_VALUES)
@@ -2182,6 +2192,10 @@ extern "C" int pulse_attn_decode(const void* qkv, int64_t qkv_stride, void* out,
                             n_items, tokens, nq, nkv, page_size, num_pages, scale, window, split_size, n_splits,
                             max_context, part_o, part_ml, &prep, live_context, plan, extras, stream);
 }
+
+// The items, from the list's end, that the prompt-portion kernel starts with before it takes the others from the list's beginning; 0:
+// all of them from the end.
+extern "C" int pulse_attn_prefill_turn(int n_items, int heads, int n_splits, int values) { return first_turn(n_items, heads, n_splits, values); }
 
 // Keys a split of the prompt-portion kernel must be a multiple of; 0 when this head size's kernel has no splits.
 extern "C" int pulse_attn_prefill_split_keys() { return SPLIT_KEYS; }

@@ -254,3 +254,16 @@ def test_nothing_but_the_copies_own_statement_touches_m0():
         assert build.m0_misuses(place + wrong + copies)
     if (lib := build.existing_library()) is not None:
         assert len(build.device_code(lib)) > 10 and build.device_code(__file__) == []
+
+
+def test_walks_of_prompts_turn_only_where_two_workgroups_share_a_unit():
+    """Shortest beside longest: where a launch's workgroups find a place at once, two a compute unit, whole walks, none in front."""
+    from pulse_infer_amd.ops.library import load_variant
+
+    turn = lambda d, items, heads, splits=1, values=0: load_variant("attn_mfma", {"PULSE_HEAD_DIM": d}).pulse_attn_prefill_turn(
+        items, heads, splits, values or d)
+    for d in (32, 64, 128):
+        assert [turn(d, n, 8) for n in (1, 32, 33, 64, 65, 4096)] == [0, 0, 32, 32, 0, 0]
+        assert turn(d, 3, 100) == 2 and turn(d, 1, 300) == 0 and turn(d, 40, 8, 2) == 0 and turn(d, 1 << 30, 60000) == 0
+    assert turn(192, 12, 32) == 0 == turn(192, 12, 32, values=160) and turn(192, 12, 32, values=128) == 8 == turn(192, 12, 32, values=64)
+    assert turn(96, 40, 8) == 0      # (a head size whose kernel takes its items in order)
