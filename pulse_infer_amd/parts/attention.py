@@ -259,13 +259,13 @@ class PagedAttention(Part):
         group = self.nq // self.nkv
         per = attention_mfma.tokens_per_item(group)
         portion = attention_mfma.portion_tokens(group, self.d)
-        key = f"static:attention.items:{per}:{portion}"
+        key = f"static:attention.items:{per}:{portion}:{self.d in attention_mfma.WIDE_HEAD_DIMS}"
         if key not in ctx.extras:  # depends only on the step's shape; the same lists serve every layer
             short, long = attention_mfma.split_entries(ctx.entries)
             dev = lambda flat: ctx.to_device(flat) if flat else None
             ctx.extras[key] = (
                 dev(attention_mfma.build_items(short, per)),
-                dev(attention_mfma.build_items(long, portion)),
+                dev(attention_mfma.build_portions(long, portion, self.d)),
                 max((e.start + e.count for _, e in short), default=0))
         short_items, long_items, short_context = ctx.extras[key]
         beside = False

@@ -314,7 +314,7 @@ class LatentAttention(PagedAttention):
         split_size, splits = attention_mfma.choose_prefill_splits(numbered, portion, self.nq, 1, self.expanded, window, tail=False)
         return {"at": at, "n_pages": n_pages, "pages": ctx.to_device(flat), "others": others,
                 "table": ctx.to_device([p for row in rows for p in row]).view(len(rows), width),
-                "items": ctx.to_device(attention_mfma.build_items(numbered, portion)),
+                "items": ctx.to_device(attention_mfma.build_portions(numbered, portion, self.expanded)),
                 "spans": [(e.first_row, e.first_row + e.count) for _, e in numbered], "split_size": split_size, "splits": splits}
 
     def _expanded(self, raw, gate, ctx: StepContext, cache: PagedCacheView, table, tables, out, plan: Dict[str, Any]) -> None:

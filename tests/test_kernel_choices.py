@@ -267,3 +267,24 @@ def test_walks_of_prompts_turn_only_where_two_workgroups_share_a_unit():
         assert turn(d, 3, 100) == 2 and turn(d, 1, 300) == 0 and turn(d, 40, 8, 2) == 0 and turn(d, 1 << 30, 60000) == 0
     assert turn(192, 12, 32) == 0 == turn(192, 12, 32, values=160) and turn(192, 12, 32, values=128) == 8 == turn(192, 12, 32, values=64)
     assert turn(96, 40, 8) == 0      # (a head size whose kernel takes its items in order)
+
+
+def test_items_of_several_prompts_stand_in_the_order_of_their_walks():
+    """The same items, the longest walks last; a single prompt's, and those of kernels that take them in order, as they were."""
+    from pulse_infer_amd.ops import attention_mfma as M
+
+    lists = [[(0, 2048)], [(0, 4096), (0, 512)], [(0, 512), (0, 4096)], [(3000, 70), (0, 513), (7000, 512), (100, 31)], [(0, 300)] * 5]
+    for spans in lists:
+        entries, row = [], 7
+        for index, (start, count) in enumerate(spans):
+            entries.append((index + 2, E(start, count)))
+            entries[-1][1].first_row = row
+            row += count
+        for d, per in ((128, 32), (64, 8), (192, 128)):
+            plain, made = M.build_items(entries, per), M.build_portions(entries, per, d)
+            fours = lambda flat: [tuple(flat[i:i + 4]) for i in range(0, len(flat), 4)]
+            assert sorted(fours(plain)) == sorted(fours(made)) and (len(spans) > 1 or plain == made)
+            of = dict(entries)
+            walks = [of[i].start + row0 - of[i].first_row + n for row0, n, i, _ in fours(made)]
+            assert walks == sorted(walks)
+            assert M.build_portions(entries, per, 96) == plain
