@@ -280,7 +280,6 @@ PREFILL_SPLIT_KEYS = 64        # a split of the prompt-portion kernel is a whole
 PREFILL_SPLIT_HEAD_DIMS = WIDE_HEAD_DIMS
 PREFILL_MAX_SPLITS = 64
 PREFILL_SCRATCH_BYTES = 1 << 30
-TAIL_SPLIT_MIN_BLOCKS = 64     # with `tail`, walks from here on (4,096 keys) are cut at three quarters on a full chip
 
 
 CHUNK_SLACK = 48     # keys that the splits of an item cover beside its chunk: a block's rounding, its other tokens'
@@ -293,42 +292,32 @@ def split_span(max_context: int, chunk: int) -> int:
 
 
 def choose_prefill_splits(entries: Sequence, portion: int, nkv: int, group: int, d: int, window: int,
-                          target_groups: Optional[int] = None, min_blocks: int = 8, tail: bool = True) -> Tuple[int, int]:
+                          target_groups: Optional[int] = None, min_blocks: int = 8) -> Tuple[int, int]:
     """(split_size, n_splits) for the prompt-portion kernel over these (index, entry) pairs.
 
     A workgroup walks its item's keys block by block, so the longest item sets the kernel's time while the chip
     waits.  Cutting the keys into splits with workgroups of their own pays when there are fewer workgroups than the
     chip runs at a time (``target_groups``, two a compute unit unless given; a short portion over a long context):
-    they get as many splits as fill it.  Splits never hold fewer than ``min_blocks`` blocks, and nothing is cut
-    otherwise, but for the tail of a long whole prompt (``tail``, below): the partial results cost a trip through memory
-    and a second launch."""
+    they get as many splits as fill it.  Splits never hold fewer than ``min_blocks`` blocks, and a full chip's walks are never
+    cut: the kernel starts the longest first, so that the short ones fill in behind them, and the partial results cost a trip
+    through memory and a second launch (one prompt whole and cut at three quarters of its longest walk: 4,096 tokens 160 and 171
+    us, 8,192 515 and 552, 16,384 1,989 and 2,045)."""
     if d not in PREFILL_SPLIT_HEAD_DIMS or window > 0:   # (a window keeps every walk short)
         return 0, 1
     if target_groups is None:
         target_groups = 2 * compute_units()
     longest = tokens = items = 0
-    walks = []
     for _, e in entries:
         tokens += e.count
-        for b in range(0, e.count, portion):
-            blocks = (e.start + min(b + portion, e.count) - 1) // PREFILL_SPLIT_KEYS + 1
-            longest = max(longest, blocks)
-            walks.append(blocks)
-            items += 1
+        items += (e.count + portion - 1) // portion
+        if e.count > 0:
+            longest = max(longest, (e.start + e.count - 1) // PREFILL_SPLIT_KEYS + 1)
     if items == 0:
         return 0, 1
     per_item = nkv * ((group + 15) // 16)
     groups = items * per_item
     budget = PREFILL_SCRATCH_BYTES // max(1, tokens * nkv * group * d * 4)
     if groups >= target_groups:
-        # A full chip.  The kernel starts the longest walks first, so that the short ones fill in behind them, and cutting
-        # gains nothing any more (``tail=False``, the engine's choice; one prompt whole and cut at three quarters of
-        # its longest walk: 4,096 tokens 160 and 171 us, 8,192 515 and 552, 16,384 1,989 and 2,045).  With ``tail`` the
-        # walks of a long whole prompt are cut there all the same, where no more than its last items run on.
-        cut = 3 * longest // 4
-        late = sum(1 for w in walks if w > cut)
-        if tail and longest >= TAIL_SPLIT_MIN_BLOCKS and budget >= 2 and 10 * late <= 3 * items:
-            return cut * PREFILL_SPLIT_KEYS, 2
         return 0, 1
     size = max(min_blocks, (longest * groups + target_groups - 1) // target_groups)
     n_splits = (longest + size - 1) // size

@@ -274,7 +274,7 @@ class PagedAttention(Part):
             if skey not in ctx.extras:
                 ctx.extras[skey] = attention_mfma.choose_prefill_splits(
                     attention_mfma.split_entries(ctx.entries)[1], portion, self.nkv, group, self.d,
-                    window or self.chunk, tail=False)
+                    window or self.chunk)
             split_size, n_splits = ctx.extras[skey]
             part_o = part_ml = None
             # (portions whose walks are whole go in the launch of the single tokens and short portions, if there are any)

@@ -311,7 +311,7 @@ class LatentAttention(PagedAttention):
             else:
                 others.append((e.first_row, e.first_row + e.count))
         portion = attention_mfma.portion_tokens(1, self.expanded)
-        split_size, splits = attention_mfma.choose_prefill_splits(numbered, portion, self.nq, 1, self.expanded, window, tail=False)
+        split_size, splits = attention_mfma.choose_prefill_splits(numbered, portion, self.nq, 1, self.expanded, window)
         return {"at": at, "n_pages": n_pages, "pages": ctx.to_device(flat), "others": others,
                 "table": ctx.to_device([p for row in rows for p in row]).view(len(rows), width),
                 "items": ctx.to_device(attention_mfma.build_portions(numbered, portion, self.expanded)),

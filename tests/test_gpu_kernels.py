@@ -915,8 +915,8 @@ def test_attn_prefill_with_its_keys_in_splits(k, case, size):
     _mfma_case(k, split=None, portion_split=size, **case)
 
 
-@pytest.mark.parametrize("n", [2048, 8192])
-def test_attn_prefill_at_the_benchmark_shape(k, n):
+@pytest.mark.parametrize("n,cut", [(2048, 0), (8192, 0), (8192, 6144)])
+def test_attn_prefill_at_the_benchmark_shape(k, n, cut):
     """A whole prompt of 2,048 (and 8,192) tokens at 32 query heads over 8 kv heads of 128 (every workgroup of the chip busy, items
     of every length, one diagonal block each): rows at the edges of items, of key blocks and of pages against the
     plain formula.  (The profile of this kernel is taken from this test.)"""
@@ -940,9 +940,9 @@ def test_attn_prefill_at_the_benchmark_shape(k, n):
     entries = [(0, E(0, n))]
     portion = M.portion_tokens(nq // nkv, d)
     items = torch.tensor(M.build_items(entries, portion), dtype=torch.int32, device=DEV)
-    # a full chip is not cut, but for the last quarter of the walks of a long prompt, which get a second split
-    split_size, n_splits = M.choose_prefill_splits(entries, portion, nkv, nq // nkv, d, 0)
-    assert (split_size, n_splits) == ((0, 1) if n < 4096 else (3 * n // 4, 2))
+    # a full chip's walks are whole; cut all the same, the last quarter of them gets a second split
+    assert M.choose_prefill_splits(entries, portion, nkv, nq // nkv, d, 0) == (0, 1)
+    split_size, n_splits = (cut, 2) if cut else (0, 1)
     part_o = torch.full((n * nq * n_splits, d), float("nan"), device=DEV) if n_splits > 1 else None
     part_ml = torch.full((n * nq * n_splits, 2), float("nan"), device=DEV) if n_splits > 1 else None
     pos = torch.arange(n, dtype=torch.int32, device=DEV)
