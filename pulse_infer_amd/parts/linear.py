@@ -272,31 +272,34 @@ class Linear:
     STAGE_ROWS_SWIGLU = (256, 1 << 30)
     STAGE_ROWS_SHARES = 512             # beyond, only where ``library_shares_for`` says so
     STAGE_CUT_ROWS = 128                # the rows that updates of up to 192 rows are cut into shares for
-    STAGE_RATE = 875                    # plain products of more rows: estimated flops a picosecond
+    STAGE_RATE = 925                    # plain products of more rows: estimated flops a picosecond
+    STAGE_LONG_K = (12288, 16384)       # and inner dimensions, see ``fills_stages``
     STAGE_MIN_WEIGHT = 1 << 22
 
     def takes_stages(self, x: torch.Tensor, w: Optional[torch.Tensor] = None, swiglu: bool = False) -> bool:
         """Whether a bfloat16 product of this many rows (with SwiGLU inside, or as it is) runs as this package's product
         in stages."""
         w = self.weight if w is None else w
+        return self.may_stage(x, w, swiglu) and (swiglu or self.fills_stages(x.shape[0], *w.shape))
+
+    def may_stage(self, x: torch.Tensor, w: torch.Tensor, swiglu: bool = False) -> bool:
+        """Whether the product in stages takes these operands, ``OWN_MANY_ROWS`` allowing."""
         rows, (n, k) = x.shape[0], w.shape
         if not (self.library and x.dtype == torch.bfloat16 and self.STAGE_ROWS[0] <= rows <= self.STAGE_ROWS_SWIGLU[1]
                 and n * k >= self.STAGE_MIN_WEIGHT and self.operands_ok(x) and kernels.gemm_stages_takes(rows, n, k, swiglu)):
             return False
-        if rows >= self.TILE_MIN_ROWS and (OWN_MANY_ROWS == "none" or self.takes_tiles(x, w, swiglu)):
-            return False
-        return swiglu or self.fills_stages(rows, n, k)
+        return rows < self.TILE_MIN_ROWS or (OWN_MANY_ROWS != "none" and not self.takes_tiles(x, w, swiglu))
 
     STAGE_RATE_FLOAT32 = 1000           # with float32 results, which take twice as long to store
 
     def takes_stages_float32(self, x: torch.Tensor, w: torch.Tensor) -> bool:
         """Whether a product of more than ``STAGE_ROWS_SHARES`` rows with float32 results runs as this package's product in stages:
-        by its estimate, as plain ones (us, library / this, by estimated flops a picosecond: 5,120 x 5,120 at 1,024 rows (672) 53 /
-        62, 8,192 x 2,048 at 1,024 (922) 33 / 38; 5,120 x 5,120 at 1,536 (1,008) 67.4 / 68.0, 4,096 x 8,192 at 2,048 (1,075) 109 /
-        106, 32,000 x 4,096 at 544 (1,116) 139 / 126, 6,144 x 4,096 at 1,536 (1,210) 67 / 58, 12,288 x 4,096 at 4,096 (1,498) 301 / 278;
-        from 1,000 on 0.94 of the library's time over the 30 sizes measured)."""
+        by its estimate (us, library / this, by estimated flops a picosecond: 5,120 x 5,120 at 1,024 rows (672) 53 /
+        62, 8,192 x 2,048 at 1,024 (922) 33 / 38; 5,120 x 5,120 at 1,536 (1,008) 75 / 71, 4,096 x 8,192 at 2,048 (1,075) 112 /
+        110, 32,000 x 4,096 at 544 (1,116) 142 / 128, 12,288 x 4,096 at 800 (1,080) 70 / 75 and 4,096 (1,498) 306 / 283, 8,192 x 2,048 at
+        4,096 (1,498) 118 / 113; from 1,000 on 0.93 of the library's time over the 51 sizes measured, one of them more than 3 % slower)."""
         rows, (n, k) = x.shape[0], w.shape
-        return (rows > self.STAGE_ROWS_SHARES and self.takes_stages(x, w)
+        return (rows > self.STAGE_ROWS_SHARES and self.may_stage(x, w)
                 and kernels.gemm_stages_time(rows, n, k) * 1000 * self.STAGE_RATE_FLOAT32 <= 2 * rows * n * k)
 
     def fills_stages(self, rows: int, n: int, k: int) -> bool:
@@ -312,19 +315,28 @@ class Linear:
         of 96 x 128) 36 / 32, 8,192 x 2,048 at 300 (0.75) 24 / 21, 6,144 x 4,096 at 512 (1.0) 37 / 34.
 
         Beyond 512 rows its estimate decides, that is how far its tiles fill their rounds and how large they are (estimated flops a
-        picosecond: us, library / this): 4,096 x 8,192 at 1,536 (807) 92 / 102, 2,048 x 2,048 at 1,536 (449) 19 / 23, 5,120 x 5,120 at 800
-        (525) 57 / 59, 10,240 x 5,120 at 544 (714) 64 / 69; 6,144 x 4,096 at 1,200 (945) 57 / 57, 1,536 (1,210) 70 / 59, 2,048 (1,383) 81 / 74
-        and 8,192 (1,498) 267 / 276, 5,120 x 5,120 at 1,536 (1,008) 76 / 70 and 8,192 (1,337) 454 / 309, 10,240 x 5,120 at 1,200 (1,097) 128 /
-        107, 4,096 x 4,096 at 2,048 (1,075) 59 / 57.  Over the sizes measured beyond 512 rows the rule comes to 0.967 of the library's
-        time.  (The library's times jump with the rows,
+        picosecond: us, library / this): 1,024 x 4,096 at 8,192 (922) 57 / 66, 8,192 x 4,096 at 1,024 (922) 59 / 66, 10,240 x 5,120 at 544
+        (714) 64 / 69; 6,144 x 4,096 at 1,200 (945) 57 / 57, 1,536 (1,210) 70 / 59 and 2,048 (1,383) 81 / 74, 5,120 x 5,120 at 1,536 (1,008)
+        76 / 70 and 8,192 (1,337) 454 / 309, 10,240 x 5,120 at 1,200 (1,097) 128 / 107, 4,096 x 4,096 at 2,048 (1,075) 59 / 57.  Two kinds
+        of products stay with the library all the same.  Those whose tiles of 256 x 256 fill every round, as its own do: 6,144 x 4,096 at
+        8,192 rows 267 / 276, 4,096 x 4,096 at 4,096 88 / 93, 4,096 x 8,192 at 8,192 342 / 364, 16,384 x 2,048 at 4,096 190 / 205, 8,192 x 4,096
+        at 1,800 90 / 95 (1.04 of its time over 81 sizes, a tile's front and its way out beside a walk of few steps; but 4,096 x 12,288 at 4,096
+        269 / 257 and 8,192 527 / 510).  And inner dimensions of 16,384 and more in tiles of 192 x 256: 5,120 x 25,600 at 1,800 371 /
+        444 and 4,096 801 / 914, 5,120 x 17,408 at 4,096 532 / 583 (in those of 256 x 256 at 2,560 562 / 311, of 192 x 192 at 1,536 351 / 214).
+        Over 391 sizes of 23 weights beyond 512 rows the rule comes to 0.96 of the library's time, 27 of them by 3 to 6 % on the wrong
+        side.  (The library's times jump with the rows,
         28 us at 255 and 42 at 256 for 6,144 x 4,096, so a rule of sizes leaves some on the wrong side: 5 to 15 % at a twentieth of the 375
-        sizes measured, 6,144 x 2,560 at 255 20 / 23, 4,608 x 3,072 at 444 25 / 29.)"""
+        sizes measured up to 512 rows, 6,144 x 2,560 at 255 20 / 23, 4,608 x 3,072 at 444 25 / 29.)"""
         tile_n, tile_m = kernels.gemm_stages_tile(rows, n, k)
         tiles, units = ((n + tile_n - 1) // tile_n) * ((rows + tile_m - 1) // tile_m), compute_units()
         fill = tiles / (((tiles + units - 1) // units) * units)
         if rows <= self.STAGE_ROWS[1]:
             return fill >= 0.7 or (k <= 2048 and fill >= 0.33)
         if rows > self.STAGE_ROWS_SHARES:
+            side = self.LIBRARY_TILE
+            theirs = ((n + side - 1) // side) * ((rows + side - 1) // side)
+            if (theirs % units == 0 and k < self.STAGE_LONG_K[0]) or (k >= self.STAGE_LONG_K[1] and (tile_n, tile_m) == (192, 256)):
+                return False
             return kernels.gemm_stages_time(rows, n, k) * 1000 * self.STAGE_RATE <= 2 * rows * n * k
         return n <= 32 * units and (fill >= 0.95 or (fill >= 0.7 and (k <= 2048 or (k <= 4096 and tile_n * tile_m >= 96 * 128))))
 

@@ -204,7 +204,7 @@ def test_updates_in_shares_of_many_rows_are_this_packages(units, monkeypatch):
 
 def test_plain_products_in_stages_keep_the_compute_units_busy(monkeypatch):
     """Narrow weights whose tiles leave most units idle stay with the library, whose product can cut their inner dimension;
-    what fills the chip goes in stages, up to 255 rows and, while the weight is narrow, to 1,024."""
+    what fills the chip goes in stages, beyond 512 rows where the library's own tiles do not fill it better."""
     import torch
     from pulse_infer_amd.ops import device, kernels
     from pulse_infer_amd.parts import linear
@@ -220,6 +220,12 @@ def test_plain_products_in_stages_keep_the_compute_units_busy(monkeypatch):
         assert all(takes(m, n, k) for m in (65, 97, 128, 192, 255))
     assert takes(357, 6144, 4096) and takes(512, 6144, 4096) and not takes(700, 4096, 4096) and not takes(1100, 6144, 4096)
     assert not takes(64, 6144, 4096) and not takes(300, 12288, 4096)
+    # beyond 512 rows by the estimate (1,152 and 840, 941 and 922 flops a picosecond), but for tiles of 256 x 256 that fill every round ...
+    assert takes(1300, 6144, 4096) and not takes(1280, 5120, 17408) and takes(1024, 7168, 5120) and not takes(1024, 8192, 4096)
+    assert takes(2048, 6144, 4096) and not takes(8192, 6144, 4096) and not takes(4096, 4096, 4096) and not takes(1800, 8192, 4096)
+    assert takes(4096, 4096, 12288) and takes(8192, 5120, 5120)
+    # ... and long inner dimensions in tiles of 192 x 256
+    assert takes(1536, 5120, 17408) and not takes(1800, 5120, 17408) and not takes(4096, 5120, 25600) and takes(2560, 5120, 17408)
     for m in (65, 255, 256, 1024):
         for n, k in ((2112, 7168), (5120, 8192), (3072, 2048), (24576, 1536)):
             tile = kernels.gemm_stages_tile(m, n, k)
