@@ -264,12 +264,12 @@ class Linear:
     # Where the product in stages is the fastest (more figures are beside its kernel).  With SwiGLU inside: wherever it takes the
     # shape (us against the library's product and the pass behind it: 24,576 x 4,096 at 357 / 512 / 800 / 2,048 / 8,192 rows 62 / 80 /
     # 147 / 284 / 1,116 against 91 / 104 / 165 / 337 / 1,305; 34,816 x 5,120 at 544 / 2,048 183 / 549 against 218 / 664; 51,200 x 5,120 at
-    # 300 / 640 / 4,096 185 / 318 / 1,472 against 203 / 359 / 1,880; 19,456 x 2,560 at 257 / 3,000 40 / 231 against 54 / 290).  Plain products:
-    # see ``fills_stages``.  Updates in shares: up to 512 rows all that are not small (4,096 x 4,096 at 512 rows 25 us against
+    # 300 / 640 / 4,096 185 / 318 / 1,472 against 203 / 359 / 1,880; 19,456 x 2,560 at 257 / 3,000 40 / 231 against 54 / 290; over 240 sizes of
+    # 16 weights from 2,048 x 2,048 and 4,096 x 1,024 on 0.72 of their time, the worst 9,728 x 2,560 and 16,384 x 3,072 at 257 rows 1.06 and
+    # 1.09, 2,048 x 8,192 at 1,536 and 3,000 1.14 and 1.07).  Plain products: see ``fills_stages``.  Updates in shares: up to 512 rows all that are not small (4,096 x 4,096 at 512 rows 25 us against
     # the library's 28, 2,560 x 9,728 at 357 28 against 40), beyond those of a wide inner dimension and few tiles
     # (``library_shares_for``).  Small products stay where they are.
-    STAGE_ROWS = (65, 256)              # with SwiGLU and in shares any of these (the last one if ``OWN_MANY_ROWS`` leaves it to it)
-    STAGE_ROWS_SWIGLU = (256, 1 << 30)
+    STAGE_ROWS = (65, 256)              # in shares any of these (the last one if ``OWN_MANY_ROWS`` leaves it to it); with SwiGLU from the first on
     STAGE_ROWS_SHARES = 512             # beyond, only where ``library_shares_for`` says so
     STAGE_CUT_ROWS = 128                # the rows that updates of up to 192 rows are cut into shares for
     STAGE_RATE = 925                    # plain products of more rows: estimated flops a picosecond
@@ -285,7 +285,7 @@ class Linear:
     def may_stage(self, x: torch.Tensor, w: torch.Tensor, swiglu: bool = False) -> bool:
         """Whether the product in stages takes these operands, ``OWN_MANY_ROWS`` allowing."""
         rows, (n, k) = x.shape[0], w.shape
-        if not (self.library and x.dtype == torch.bfloat16 and self.STAGE_ROWS[0] <= rows <= self.STAGE_ROWS_SWIGLU[1]
+        if not (self.library and x.dtype == torch.bfloat16 and self.STAGE_ROWS[0] <= rows
                 and n * k >= self.STAGE_MIN_WEIGHT and self.operands_ok(x) and kernels.gemm_stages_takes(rows, n, k, swiglu)):
             return False
         return rows < self.TILE_MIN_ROWS or (OWN_MANY_ROWS != "none" and not self.takes_tiles(x, w, swiglu))

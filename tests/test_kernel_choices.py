@@ -157,11 +157,26 @@ def test_which_products_of_many_rows_the_option_decides(units, monkeypatch):
                 assert not o.takes_stages(rows(m)) and not o.stage_shares_for(rows(m))
             if m > Linear.STAGE_ROWS_SHARES:
                 assert not o.stage_shares_for(rows(m))
-            if m > Linear.STAGE_ROWS_SWIGLU[1]:
-                assert not gate_up.takes_stages(rows(m), swiglu=True)
     monkeypatch.setattr(linear, "OWN_MANY_ROWS", "stages")
-    for m in (256, 257, 512, 768):
-        assert gate_up.takes_stages(rows(m), swiglu=True) or (24576 > 192 * units and m > 256)
+    small = Linear(torch.empty(4096, 1024, dtype=torch.bfloat16, device="meta"), "bfloat16")
+    for m in (256, 257, 512, 513, 768, 769, 1536, 1537, 2048, 8192, 100000):
+        assert gate_up.takes_stages(rows(m), swiglu=True)
+        assert small.takes_stages(torch.empty(m, 1024, dtype=torch.bfloat16, device="meta"), swiglu=True)
+
+
+def test_updates_of_many_rows_go_in_two_shares_while_these_fill_the_chip_once(monkeypatch):
+    """As many tiles of 256 x 256 as half the compute units; with the library's products up to a hundred."""
+    import torch
+    from pulse_infer_amd.ops import device
+    from pulse_infer_amd.parts import linear
+    from pulse_infer_amd.parts.linear import Linear
+
+    monkeypatch.setattr(device, "_units", 256)
+    down = Linear(torch.empty(4096, 12288, dtype=torch.bfloat16, device="meta"), "bfloat16")      # (16 tiles a tile of rows)
+    for policy, last in (("stages", 2048), ("swiglu", 2048), ("none", 1536)):
+        monkeypatch.setattr(linear, "OWN_MANY_ROWS", policy)
+        shares = [down.library_shares_for(torch.empty(m, 12288, dtype=torch.bfloat16, device="meta")) for m in (768, 769, last, last + 1, 8192)]
+        assert shares == [4, 2, 2, 0, 0]
 
 
 def test_shares_of_an_update_depend_on_the_weight_alone_up_to_192_rows(units):
