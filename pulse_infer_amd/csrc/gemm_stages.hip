@@ -145,13 +145,15 @@ void launch(StageArgs a, hipStream_t stream) {
 // weight rows and rows of X a tile (the kernels below, in this order)
 constexpr int SHAPES[][2] = {{64, 64}, {64, 128}, {96, 128}, {128, 64}, {128, 128}, {192, 128}, {256, 128},
                                {192, 192}, {192, 256}, {256, 192}, {256, 256}};
-constexpr int64_t FAR_ROWS = 1 << 22;   // values between rows: 256 of them come to 2 GB
+constexpr int64_t FAR_ROWS = 1 << 22;   // values between rows that pulse_gemm_tile refuses
+// Whether a tile's last row lies as near its first as a lane's 32-bit offset reaches (with the pieces and BACK and `inside` of TileLoop).
+bool reaches(int rows, int64_t ld) { return (rows - 1) * ld * 2 + 8192 < (int64_t{1} << 32); }
 constexpr int NUM_SHAPES = sizeof(SHAPES) / sizeof(SHAPES[0]);
 
 template <int MODE>
 void launch_shape(int shape, const StageArgs& a, hipStream_t s) {
-    // (a tile's last row must lie less than 4 GB behind its first; what does not goes by pointers, in the smallest tiles)
-    if (a.ldx >= FAR_ROWS || a.ldw >= FAR_ROWS) return launch<MODE, 64, 64, 2, 2, 6, 6, true, true>(a, s);
+    // (what does not goes by pointers, in the smallest tiles: rows from 16 MB apart on in the largest ones, 68 MB in these)
+    if (!reaches(SHAPES[shape][0], a.ldw) || !reaches(SHAPES[shape][1], a.ldx)) return launch<MODE, 64, 64, 2, 2, 6, 6, true, true>(a, s);
     switch (shape) {
         case 0: return launch<MODE, 64, 64, 2, 2, 6>(a, s);
         case 1: return launch<MODE, 64, 128, 2, 2, 6>(a, s);

@@ -275,6 +275,7 @@ class Linear:
     STAGE_RATE = 925                    # plain products of more rows: estimated flops a picosecond
     STAGE_LONG_K = (12288, 16384)       # and inner dimensions, see ``fills_stages``
     STAGE_MIN_WEIGHT = 1 << 22
+    STAGE_FAR = 1 << 23                 # values between rows: what lies further apart goes in small tiles, which the estimate does not know of
 
     def takes_stages(self, x: torch.Tensor, w: Optional[torch.Tensor] = None, swiglu: bool = False) -> bool:
         """Whether a bfloat16 product of this many rows (with SwiGLU inside, or as it is) runs as this package's product
@@ -287,6 +288,8 @@ class Linear:
         rows, (n, k) = x.shape[0], w.shape
         if not (self.library and x.dtype == torch.bfloat16 and self.STAGE_ROWS[0] <= rows
                 and n * k >= self.STAGE_MIN_WEIGHT and self.operands_ok(x) and kernels.gemm_stages_takes(rows, n, k, swiglu)):
+            return False
+        if rows > self.STAGE_ROWS_SHARES and max(x.stride(0), w.stride(0)) >= self.STAGE_FAR:
             return False
         return rows < self.TILE_MIN_ROWS or (OWN_MANY_ROWS != "none" and not self.takes_tiles(x, w, swiglu))
 

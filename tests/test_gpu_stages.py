@@ -233,15 +233,20 @@ def test_blocks_of_weight_rows_start_together_where_their_rows_are_no_power_of_t
 
 
 @pytest.mark.parametrize("far", ["x", "w", "both"])
-def test_product_in_stages_of_rows_gigabytes_apart(far):
-    """A tile's rows more than 4 GB behind its first: by pointers, the same bits as of rows that lie together."""
+@pytest.mark.parametrize("apart", [(1 << 22) + 8, 17000008, 34000000, 34100008])
+def test_product_in_stages_of_rows_gigabytes_apart(far, apart):
+    """A tile's last row (64 a tile) 0.5, 2.1, 4.28 and 4.3 GB behind its first, which is more than offsets of 32 bits reach: the same
+    bits as of rows that lie together.  (4 GB in front of the operands, so that an offset taken for a negative one finds other values.)"""
     from pulse_infer_amd.ops import kernels
 
-    m, n, k = 70, 160, 192
+    m, n, k = 130, 160, 192
     x, w, _, _ = product(m, n, k)
-    apart = (1 << 22) + 8
-    xf, wf = (torch.empty_strided(t.shape, (apart, 1), dtype=t.dtype, device=DEV).copy_(t) if far in (name, "both") else t
-              for name, t in (("x", x), ("w", w)))
+    front = 1 << 31
+
+    def spread(t):
+        room = torch.empty(front + t.shape[0] * apart, dtype=t.dtype, device=DEV)
+        return room.as_strided(t.shape, (apart, 1), front).copy_(t)
+    xf, wf = (spread(t) if far in (name, "both") else t for name, t in (("x", x), ("w", w)))
     for swiglu, width in ((False, n), (True, n // 2)):
         near, out = (torch.full((m, width), float("nan"), dtype=torch.bfloat16, device=DEV) for _ in range(2))
         kernels.gemm_stages(x, w, near, swiglu=swiglu)
