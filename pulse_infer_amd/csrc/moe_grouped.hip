@@ -23,6 +23,8 @@
 
 #include <math.h>
 
+#include <algorithm>
+
 namespace {
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
@@ -534,8 +536,9 @@ extern "C" int pulse_moe_group(const int* idx, int pairs, int experts, int tile_
 
 static bool aligned16(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
 
-// Whether `rows` rows of K values, and a tile's rows of a weight, lie less than 4 GB behind the first (moe_tile_kernel's offsets).
-static bool near_rows(int64_t rows, int K) { return K < (1 << 22) && rows * K < (1ll << 30); }
+// Whether `rows` rows of K values, and a tile's rows of a weight (256 at most), lie as near the first as moe_tile_kernel's 32-bit offsets
+// reach (with the pieces and BACK and `inside` of TileLoop).
+static bool near_rows(int64_t rows, int64_t K) { return std::max<int64_t>(rows, 256) * K * 2 + 8192 < (int64_t{1} << 32); }
 
 extern "C" int pulse_moe_gate_up_grouped(const void* x, const void* wg, const void* wu, const int* order,
                                          const int* tile_expert, const int* tile_row0, const int* tile_rows,

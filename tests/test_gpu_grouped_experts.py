@@ -95,7 +95,7 @@ def test_grouped_experts_with_room_for_more_pairs_than_offsets_reach():
     wd = (rnd(experts, hidden, ff, seed=5) * ff ** -0.5).to(torch.bfloat16).to(DEV)
     idx = (torch.arange(pairs, dtype=torch.int32) % experts).to(DEV)
     few = kernels.moe_max_tiles(pairs, experts, rows)
-    many = (1 << 24) // rows + few
+    many = (1 << 25) // rows + few
     rank, order = (torch.empty(pairs, dtype=torch.int32, device=DEV) for _ in range(2))
     tile_expert, tile_row0, tile_rows = (torch.empty(many, dtype=torch.int32, device=DEV) for _ in range(3))
     num = torch.empty(1, dtype=torch.int32, device=DEV)
@@ -116,6 +116,33 @@ def test_grouped_experts_with_room_for_more_pairs_than_offsets_reach():
         kernels.call("pulse_moe_down_grouped", p(act), p(wd), *lists, i32(tiles), i32(rows), p(y), i32(hidden), i32(ff), kernels._stream())
         out, size = (torch.einsum("tf,thf->th", a, b) for a, b in ((got, wd.cpu().to(F64)[e]), (got.abs(), wd.cpu().to(F64)[e].abs())))
         assert ((y.cpu().to(F64) - out).abs() <= (ff + 4) * 2.0 ** -24 * size).all(), tiles
+
+
+def test_grouped_experts_of_tokens_four_gigabytes_apart():
+    """A list's tokens up to 4.29 GB behind the first, as far as an offset of 32 bits reaches.  (4 GB in front of them, so that an offset
+    taken for a negative one finds other values.)"""
+    from pulse_infer_amd.ops import kernels
+
+    hidden, ff, experts, rows = 4096, 64, 2, 192
+    pairs = ((1 << 31) - 4096) // hidden - (experts + 1) * rows        # (lists have room for a last tile an expert)
+    pairs -= pairs % rows
+    few = kernels.moe_max_tiles(pairs, experts, rows)
+    assert 2 ** 32 - 2 ** 23 < 2 * pairs * hidden < 2 * (few * rows + 1) * hidden + 8192 < 2 ** 32
+    x = torch.empty((1 << 31) + pairs * hidden, dtype=torch.bfloat16, device=DEV)[1 << 31:].view(pairs, hidden).normal_()
+    wg, wu = ((rnd(experts, ff, hidden, seed=3 + i) * hidden ** -0.5).to(torch.bfloat16).to(DEV) for i in range(2))
+    idx = (torch.arange(pairs, dtype=torch.int32) % experts).to(DEV)
+    ints = [torch.empty(n, dtype=torch.int32, device=DEV) for n in (pairs, pairs, few, few, few, 1)]
+    act = torch.full((pairs, ff), float("nan"), dtype=torch.bfloat16, device=DEV)
+    p, i32 = kernels._ptr, kernels._i32
+    kernels.call("pulse_moe_group", p(idx), i32(pairs), i32(experts), i32(rows), i32(few), *(p(t) for t in ints), kernels._stream())
+    kernels.call("pulse_moe_gate_up_grouped", p(x), p(wg), p(wu), *(p(t) for t in ints[1:]), i32(few), i32(rows), p(act), i32(hidden),
+                 i32(ff), i32(1), p(None), i32(0), kernels._f32(0.0), kernels._stream())
+    assert not torch.isnan(act).any()
+    some = torch.tensor([0, 1, 191, 192, pairs // 2, pairs // 2 + 1, pairs - 2, pairs - 1])
+    xs, e = x[some.to(DEV)].cpu().to(F64), some % experts
+    g, u = (torch.einsum("th,tfh->tf", xs, w.cpu().to(F64)[e]) for w in (wg, wu))
+    want = g * torch.sigmoid(g) * u
+    assert ((act[some.to(DEV)].cpu().to(F64) - want).abs() <= 2.0 ** -8 * want.abs() + 1e-5 * (1.0 + want.abs().max())).all()
 
 
 @pytest.mark.parametrize("hidden,ff", [(64, 64), (1024, 448)])
