@@ -64,6 +64,7 @@ def _splitmix64(x: int) -> int:
 
 
 def uniform_for(seed: int, counter: int) -> float:
-    """A number in [0, 1) that depends only on (seed, counter): the counter-th draw of a request."""
+    """A number in [0, 1) that depends only on (seed, counter): the counter-th draw of a request.  (The plain form of what the native
+    step makes for its rows, for programs that want to know a request's draws, and to test that by.)"""
     z = _splitmix64(_splitmix64(seed & _MASK) ^ ((counter * 0xD1342543DE82EF95) & _MASK))
     return (z >> 40) / float(1 << 24)
