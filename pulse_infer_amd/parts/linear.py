@@ -274,6 +274,7 @@ class Linear:
     STAGE_CUT_ROWS = 128                # the rows that updates of up to 192 rows are cut into shares for
     STAGE_RATE = 925                    # plain products of more rows: estimated flops a picosecond
     STAGE_LONG_K = (12288, 16384)       # and inner dimensions, see ``fills_stages``
+    STAGE_SHORT_K = 512
     STAGE_MIN_WEIGHT = 1 << 22
     STAGE_FAR = 1 << 23                 # values between rows: what lies further apart goes in small tiles, which the estimate does not know of
 
@@ -324,7 +325,8 @@ class Linear:
         of products stay with the library all the same.  Those whose tiles of 256 x 256 fill every round, as its own do: 6,144 x 4,096 at
         8,192 rows 267 / 276, 4,096 x 4,096 at 4,096 88 / 93, 4,096 x 8,192 at 8,192 342 / 364, 16,384 x 2,048 at 4,096 190 / 205, 8,192 x 4,096
         at 1,800 90 / 95 (1.04 of its time over 81 sizes, a tile's front and its way out beside a walk of few steps; but 4,096 x 12,288 at 4,096
-        269 / 257 and 8,192 527 / 510).  And inner dimensions of 16,384 and more in tiles of 192 x 256: 5,120 x 25,600 at 1,800 371 /
+        269 / 257 and 8,192 527 / 510, and one or two rounds of at most eight steps, 8,192 x 512 at 2,048 23.8 / 21.3 and 4,096 41.5 / 40.7, 8,192
+        77 / 82).  And inner dimensions of 16,384 and more in tiles of 192 x 256: 5,120 x 25,600 at 1,800 371 /
         444 and 4,096 801 / 914, 5,120 x 17,408 at 4,096 532 / 583 (in those of 256 x 256 at 2,560 562 / 311, of 192 x 192 at 1,536 351 / 214).
         Over 391 sizes of 23 weights beyond 512 rows the rule comes to 0.96 of the library's time, 27 of them by 3 to 6 % on the wrong
         side.  (The library's times jump with the rows,
@@ -338,7 +340,9 @@ class Linear:
         if rows > self.STAGE_ROWS_SHARES:
             side = self.LIBRARY_TILE
             theirs = ((n + side - 1) // side) * ((rows + side - 1) // side)
-            if (theirs % units == 0 and k < self.STAGE_LONG_K[0]) or (k >= self.STAGE_LONG_K[1] and (tile_n, tile_m) == (192, 256)):
+            few = k <= self.STAGE_SHORT_K and theirs <= 2 * units
+            if (theirs % units == 0 and k < self.STAGE_LONG_K[0] and not few) \
+                    or (k >= self.STAGE_LONG_K[1] and (tile_n, tile_m) == (192, 256)):
                 return False
             return kernels.gemm_stages_time(rows, n, k) * 1000 * self.STAGE_RATE <= 2 * rows * n * k
         return n <= 32 * units and (fill >= 0.95 or (fill >= 0.7 and (k <= 2048 or (k <= 4096 and tile_n * tile_m >= 96 * 128))))

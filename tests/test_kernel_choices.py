@@ -239,6 +239,7 @@ def test_plain_products_in_stages_keep_the_compute_units_busy(monkeypatch):
     assert takes(1300, 6144, 4096) and not takes(1280, 5120, 17408) and takes(1024, 7168, 5120) and not takes(1024, 8192, 4096)
     assert takes(2048, 6144, 4096) and not takes(8192, 6144, 4096) and not takes(4096, 4096, 4096) and not takes(1800, 8192, 4096)
     assert takes(4096, 4096, 12288) and takes(8192, 5120, 5120)
+    assert takes(2048, 8192, 512) and takes(4096, 8192, 512) and not takes(8192, 8192, 512) and not takes(2048, 8192, 576)
     # ... and long inner dimensions in tiles of 192 x 256
     assert takes(1536, 5120, 17408) and not takes(1800, 5120, 17408) and not takes(4096, 5120, 25600) and takes(2560, 5120, 17408)
     for m in (65, 255, 256, 1024):
