@@ -2,24 +2,24 @@
 // bfloat16 operands, float32 sums on the matrix cores, on the loop of tile_loop.h.
 // (reference: cuBLAS for every product, src/ops/kernels/cuda/matmul_kernel.cu:132-154)
 //
-// What bounds it: the bytes that the fullest compute unit copies into LDS.  A unit takes in 28 to 54 bytes a nanosecond over a
-// launch, least where they are weights that come from memory, and the matrix cores are busy for 13 to 46 % of it, LDS waits
-// make 1 to 6 % (counters at 97, 357 and 509 rows; from 300 rows on the power limit comes near: 357 rows of gate + up take 58 us with
+// What bounds it: the bytes that the fullest compute unit copies into LDS.  A unit takes in 29 to 55 bytes a nanosecond over a
+// launch, least where they are weights that come from memory, and the matrix cores are busy for 13 to 50 % of it, LDS waits
+// make 3 to 7 % (counters at 97, 357 and 509 rows; from 300 rows on the power limit comes near: 357 rows of gate + up take 58 us with
 // operands of zeros, 62 to 65 with others, 2,048 rows 224 and 284), so the shape and the shares of K are chosen for the least bytes
 // (`plan_for`).  Measured alone with weights from memory, us, against the vendor library's product (gate and up: with its
 // pass for SwiGLU behind it) and this package's shared-out product for up to 192 rows; in brackets behind a figure, what it
 // takes inside a step, between other kernels and with the chip warm:
 //                                   97 rows              192                  357                 509
-//   gate + up, 24,576 x 4,096       38 [39]              53                   66 [68]             84 [88]
+//   gate + up, 24,576 x 4,096       38 [38]              53                   66 [68]             84 [88]
 //     library                       54                   64                   84                  96
-//   qkv, 6,144 x 4,096              19 [20]              26                   32 [34]             35 [37]
+//   qkv, 6,144 x 4,096              19 [20]              26                   32 [33]             35 [35]
 //     library                       25                   36                   41                  42
 //   o, 4,096 x 4,096, shares        12 [14]              14                   21 [24]             24 [26]
 //     library / shared out          25 / 16              37 / 21              29                  32
 //   down, 4,096 x 12,288, shares    24 [25]              31                   39 [43]             52 [55]
 //     library / shared out          44 / 34              92 / 47              52, shared [46]     59, shared [60]
-// (2,048 rows, inside a step, against the library's: gate + up 284 to 310 for 278 + 30, down in two shares 142 to 155, o 61 to 66, qkv 77 to
-// 84 for its 84; 8,192 rows of gate + up 1,095 to 1,112, 1.49 to 1.51 PFLOP/s.)
+// (2,048 rows, inside a step, against the library's: gate + up 284 to 316 for 278 + 30, down in two shares 142 to 158, o 61 to 66, qkv 77 to
+// 84 for its 84; 8,192 rows of gate + up 1,095 to 1,130, 1.46 to 1.51 PFLOP/s.  Cards differ by a tenth.)
 // From some 260 rows on tiles of 192 or 256 rows of X (their weights through three stages, X, which comes from L2, through
 // two where LDS holds no third) take the place of the library's: 357 rows of gate + up ran 96 us in tiles of 192 x 128.
 // Steps of 32 of K in twice the stages, the other way to fit such tiles, bring 64 bytes of a row at a time, which a unit
