@@ -332,9 +332,10 @@ __device__ __forceinline__ mass_t mass_through(mass_t v) {
 }
 
 // What the kernels in front of left_kernel leave of a row that the chunks could not choose for, in 32-bit words: the histogram
-// over [lowest, best] (rows with top-k: counts; top-p alone: masses; 64 bits each), the row's smallest number (and a word of nothing,
-// for the 64-bit ones behind it), the mass of the bins above the one with top-p's edge, that of the row, and every chunk's of the former.
-constexpr int REST_LOWEST = 2 * HIST_BINS, REST_BASE = REST_LOWEST + 2, REST_WHOLE = REST_LOWEST + 4;
+// over [lowest, best] (rows with top-k: counts; top-p alone: masses; 64 bits each), the row's smallest number, whether its token was
+// chosen from what they left (the tests ask; no kernel does), the mass of the bins above the one with top-p's edge, that of the row, and
+// every chunk's of the former.
+constexpr int REST_LOWEST = 2 * HIST_BINS, REST_CHOSEN = REST_LOWEST + 1, REST_BASE = REST_LOWEST + 2, REST_WHOLE = REST_LOWEST + 4;
 constexpr int REST_CHUNKS = REST_LOWEST + 6, REST_MOST_CHUNKS = 2 * PULSE_WAVE;
 constexpr int REST_WORDS = REST_CHUNKS + 2 * REST_MOST_CHUNKS;
 static_assert(REST_WORDS % 2 == 0 && REST_CHUNKS % 2 == 0, "64-bit words");
@@ -1066,9 +1067,9 @@ __device__ __forceinline__ void string_segments(const int* seg_i, const float* s
 // passes over a short row cost no more than that, without it.
 enum { LEFT = 0, CHOSEN = 1, LEFT_COUNTED = 2, LEFT_ALONE = 3 };
 
-// What rest_kernel adds a row's histogram to.
+// What rest_kernel adds a row's histogram to, and that the row's token is not chosen.
 __device__ __forceinline__ void clear_rest(int* rest) {
-    for (int b = threadIdx.x; b <= REST_LOWEST; b += blockDim.x) rest[b] = 0;
+    for (int b = threadIdx.x; b <= REST_CHOSEN; b += blockDim.x) rest[b] = 0;
 }
 
 // The choice of every row from what the kernels before left, a workgroup a row: the largest logit for greedy rows;
@@ -1167,7 +1168,7 @@ __global__ __launch_bounds__(CHOOSE_THREADS) void chunked_choose_kernel(
             done[r] = enough ? 1 : 0;
         }
         if (left && !enough)      // (by this wavefront alone)
-            for (int b = lane; b <= REST_LOWEST; b += PULSE_WAVE) left[static_cast<int64_t>(r) * REST_WORDS + b] = 0;
+            for (int b = lane; b <= REST_CHOSEN; b += PULSE_WAVE) left[static_cast<int64_t>(r) * REST_WORDS + b] = 0;
         return;
     }
     // a draw from the whole vocabulary: the chunk in which it falls, chunk masses in chunk order
@@ -1407,7 +1408,7 @@ __device__ __forceinline__ bool left_choose(
         int token;            // (with top-k every list is enough)
         if (n <= 8 * PULSE_WAVE) finish_on_list<8>(list_i, list_x, n, true, left.k, use_p, left.p, 0.f, left.best, left.inv_t, uniform[r], best_i, token);
         else finish_on_list<LIST_PER_LANE>(list_i, list_x, n, true, left.k, use_p, left.p, 0.f, left.best, left.inv_t, uniform[r], best_i, token);
-        if (lane == 0) out[r] = token;
+        if (lane == 0) { out[r] = token; rest[REST_CHOSEN] = 1; }
         return true;
     }
     const Weigh weigh(left.best, left.inv_t, vocab);
@@ -1459,6 +1460,7 @@ __device__ __forceinline__ bool left_choose(
         int j = 0;
         while (target >= before + ms[j]) before += ms[j++];
         out[r] = begin + j;
+        rest[REST_CHOSEN] = 1;
     }
     return true;
 }
