@@ -991,7 +991,7 @@ __global__ __launch_bounds__(WAVES* PULSE_WAVE) PULSE_ATTN_WAVES_PER_EU void att
 // for the next block's maximum, so that its matrix and its vector instructions alternate; what is rare (masks, caps, stale
 // values, a maximum that grew) stands out of the way, since a taken branch over it cost as much as a product.  Heads of
 // 128, 32 on 8: 2,048 tokens 64.4 -> 57.6 us, 8,192 in two splits 597 -> 575, 4,096 201 -> 187; 509 tokens 18.7 -> 17.5,
-// 97 9.8 -> 10.0 (10.8 -> 11.3 between other kernels, where its code comes cold).  What a step of it waits for now is spread evenly: without the copies it takes 11 % less, without the
+// 97 9.8 -> 10.0 (10.6 -> 11.2 between other kernels, where its code, 51 KB for 30, comes cold).  What a step of it waits for now is spread evenly: without the copies it takes 11 % less, without the
 // exponentials 7 %, with half the reads from LDS 4 %; two wavefronts a SIMD keep the matrix cores busy 45 % of the time.
 //
 // LDS holds 16-byte pieces without padding; which piece a lane fetches is chosen so that the matrix-core operand
@@ -1425,7 +1425,8 @@ __device__ __forceinline__ void attn_prefill_wide_workgroup(const MfmaArgs& a, c
         }
         Place next, two;                                                          // of blocks b + 1 and b + 2
         each<4>([&](auto part) __attribute__((always_inline)) { find(part, first, next); find(part, second, two); });
-        // (the second block's keys are asked for in any case: behind the walk's end they are those of the first page, and not used)
+        // (the second block's keys are asked for in any case: behind the walk's end they are those of the first page, and not used; a branch
+        // around them took longer than they do, 97 tokens between other kernels 11.2 -> 11.5 us)
         fetch_keys(next, 0);
         fetch_values(next, 0);
         fetch_keys(two, 1);
