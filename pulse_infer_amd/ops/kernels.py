@@ -758,6 +758,78 @@ def attn_wide_splits(n_items: int, chunks: int, keys: int) -> int:
     return max(1, min(want, 16, 1 if steps <= 4 else (steps + 2) // 3))
 
 
+LATENT_ROWS = 32            # of an item of ``attn_latent``
+LATENT_KEYS = 64            # of a block of keys there
+LATENT_MAX_WIDTH = 576      # channels of a stored row that it takes, and of them as values
+LATENT_MAX_VALUES = 512
+
+
+def attn_latent_takes(q: torch.Tensor, kcache: torch.Tensor, d: int, wv: int) -> bool:
+    """Whether ``attn_latent`` takes these operands: what ``attn_wide`` takes with one kv head, up to its widths."""
+    return (attn_wide_takes(q, kcache, d) and kcache.shape[1] == 1 and d <= LATENT_MAX_WIDTH and 0 < wv <= min(d, LATENT_MAX_VALUES)
+            and wv % 16 == 0)
+
+
+def attn_latent_items(entries, nq: int):
+    """The work list of ``attn_latent`` for entries (anything with ``first_row`` and ``count``): items of 32 rows, ``hp`` heads of
+    32 // hp consecutive tokens of one entry.  Returns (flat list of quadruples first token, tokens, first head, heads; hp)."""
+    hp = min(nq, LATENT_ROWS)
+    tp = LATENT_ROWS // hp
+    flat = []
+    for e in entries:
+        for t in range(0, e.count, tp):
+            for hb in range(0, nq, hp):
+                flat.extend((e.first_row + t, min(tp, e.count - t), hb, min(hp, nq - hb)))
+    return flat, hp
+
+
+def attn_latent_splits(n_items: int, keys: int) -> int:
+    """Over how many workgroups ``attn_latent`` shares an item's keys out: as many as give every compute unit one (a workgroup
+    fills it), in equal numbers of whole blocks, at most the 64 that the merge takes.  us in 1 / 2 / .. splits: 8 requests of
+    1,500 tokens 4 / 12 / 24 35 / 19.1 / 17.7, of 4,000 16 / 32 / 48 31 / 27 / 32; 64 of 500 2 / 4 / 8 33 / 27 / 37; one of 5,000
+    20 / 40 / 64 27 / 24 / 22."""
+    from .device import compute_units
+    blocks = (keys + LATENT_KEYS - 1) // LATENT_KEYS
+    want = min(64, max(1, compute_units() // max(1, n_items)))
+    each = max(1, (blocks + want - 1) // want)
+    return max(1, (blocks + each - 1) // each)
+
+
+def attn_latent(q: torch.Tensor, out: torch.Tensor, nq: int, d: int, wv: int, kcache: torch.Tensor, vcache: torch.Tensor,
+                positions: torch.Tensor, token_entry: torch.Tensor, block_table: torch.Tensor, items: torch.Tensor, hp: int,
+                scale: float, window: int = 0, sink: Optional[torch.Tensor] = None, softcap: float = 0.0, n_splits: int = 1,
+                part: Optional[torch.Tensor] = None, part_ml: Optional[torch.Tensor] = None) -> None:
+    """Paged attention on the matrix cores over latent rows that all query heads share: out float32 [T, nq * d], of a head's
+    channels the first ``wv``, of the rows that the items hold.  Window, sinks and score cap as for ``attn_generic``; scratch
+    for splits, a row an item's row and split: ``part`` float32 [items * 32 * n_splits, wv], ``part_ml`` [.., 2]."""
+    _gpu("attn_latent", q, out, kcache, vcache, positions, token_entry, block_table, items, sink)
+    tokens = q.shape[0]
+    _need(attn_latent_takes(q, kcache, d, wv), "attn_latent: bfloat16 operands, one kv head, pages of a multiple of 16 keys, rows of up to "
+          f"{LATENT_MAX_WIDTH} channels in sixteens")
+    if n_splits > 1:
+        _gpu("attn_latent", part, part_ml)
+        for t, width in ((part, wv), (part_ml, 2)):
+            _need(t is not None and t.dtype == torch.float32 and t.is_contiguous()
+                  and t.numel() >= items.numel() // 4 * LATENT_ROWS * n_splits * width, "attn_latent: the splits' scratch is too small")
+    _need(q.dim() == 2 and q.stride(1) == 1 and q.shape[1] >= nq * d, "attn_latent: q too narrow")
+    _need(out.dtype == torch.float32 and out.dim() == 2 and out.stride(1) == 1 and out.shape[0] == tokens
+          and out.shape[1] >= nq * d, f"attn_latent: out must be float32 [{tokens}, {nq * d}]")
+    pages, page_size = _check_cache("attn_latent", kcache, vcache, 1, d)
+    _int_vec("attn_latent: positions", positions, tokens)
+    _int_vec("attn_latent: token_entry", token_entry, tokens)
+    _need(block_table.dim() == 2 and block_table.dtype == torch.int32 and block_table.is_contiguous(),
+          "attn_latent: block_table must be contiguous int32 [entries, width]")
+    _need(items.dtype == torch.int32 and items.is_contiguous() and items.numel() % 4 == 0, "attn_latent: items are int32 quadruples")
+    if sink is not None:
+        _need(sink.dtype == torch.float32 and sink.is_contiguous() and sink.numel() == nq, f"attn_latent: the sinks must be float32 [{nq}]")
+    call("pulse_attn_latent", _ptr(q), _i64(q.stride(0) if tokens > 1 else q.shape[1]), _ptr(out),
+         _i64(out.stride(0) if tokens > 1 else out.shape[1]), _ptr(kcache), _ptr(vcache), _ptr(positions), _ptr(token_entry),
+         _ptr(block_table), _i32(block_table.shape[1]), _ptr(items), _i32(items.numel() // 4), _i32(hp), _i32(nq), _i32(d), _i32(wv),
+         _i32(page_size), _i32(pages), _f32(scale), _i32(window), _ptr(sink), _f32(softcap), _i32(n_splits),
+         _ptr(part if n_splits > 1 else None), _ptr(part_ml if n_splits > 1 else None), _stream(),
+         label=f"d={d} values={wv} splits={n_splits}")
+
+
 def head_mix(x: torch.Tensor, mix: torch.Tensor, out: torch.Tensor, heads: int, kv_heads: int, d: int, dv: int,
              out_d: int, scale: float = 1.0) -> None:
     """out[t, h, e] = scale * sum_g mix[h, g] * x[t, g, h // (heads // kv_heads), e] for e < dv, zero for dv <= e <

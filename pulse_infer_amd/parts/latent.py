@@ -7,8 +7,8 @@ value W_uv,h c; scores are (q . key) * scale over all earlier tokens, softmax wi
 heads' results, side by side, are multiplied element by element by sigmoid(Wg x) (optional) and projected by Wo.
 
 Scores and weighted sums are linear in c, so the part works in the latent space and paged attention kernels serve it
-as they are (those of ``attention`` where they are compiled for rows this wide, else ``pulse_attn_wide``, else the
-generic one): one kv head whose stored key is [c | k_rot] and whose stored value is c, query head
+as they are (those of ``attention`` where they are compiled for rows this wide, else ``pulse_attn_latent``, for still wider
+rows ``pulse_attn_wide``, else the generic one): one kv head whose stored key is [c | k_rot] and whose stored value is c, query head
 h = [W_uk,h^T q_plain,h | q_rot,h], and W_uv,h applied to the weighted sum of latent rows afterwards.  Keys and values
 are stored ``stored`` = latent_dim + rotary_dim (rounded up to 16) channels wide, the rest zeros.
 
@@ -236,25 +236,34 @@ class LatentAttention(PagedAttention):
             self.attend(q, o, ctx, cache, table)
         elif self._wide(q, cache):
             o = ws.buffer("latent.rows", tokens, self.nq * self.d, torch.float32)
-            key = f"static:latent.wide_items:{self.nq}:{'some' if plan else 'all'}"
+            wv = (self.rank + 15) // 16 * 16
+            shared = kernels.attn_latent_takes(q, cache.keys, self.d, wv)      # (else wider rows than that kernel has room for)
+            key = f"static:latent.items:{self.nq}:{shared}:{'some' if plan else 'all'}"
             if key not in ctx.extras:
-                row_tiles = kernels.attn_wide_row_tiles(ctx.num_tokens)
                 entries = [e for i, e in enumerate(ctx.entries) if plan is None or i not in plan["at"]]
-                flat, hp = kernels.attn_wide_items(entries, self.nq, 1, row_tiles)
+                row_tiles = kernels.attn_wide_row_tiles(ctx.num_tokens)
+                flat, hp = kernels.attn_latent_items(entries, self.nq) if shared else kernels.attn_wide_items(entries, self.nq, 1, row_tiles)
                 ctx.extras[key] = (ctx.to_device(flat), hp, row_tiles)
             items, hp, row_tiles = ctx.extras[key]
-            wv = (self.rank + 15) // 16 * 16
             seen = min(ctx.max_context, window + 32) if window else ctx.max_context
-            splits = kernels.attn_wide_splits(items.numel() // 4, (wv + 255) // 256, seen) if row_tiles == 1 else 1
-            if plan is not None:
+            if shared:
+                splits = kernels.attn_latent_splits(items.numel() // 4, seen)
+            elif plan is not None:
                 splits = 1     # (the merge of splits covers every row of the step)
+            else:
+                splits = kernels.attn_wide_splits(items.numel() // 4, (wv + 255) // 256, seen) if row_tiles == 1 else 1
             part = part_ml = None
             if splits > 1:
-                part = ws.buffer("attn_wide.part", tokens * self.nq * splits, self.d, torch.float32)
-                part_ml = ws.buffer("attn_wide.part_ml", tokens * self.nq * splits, 2, torch.float32)
-            kernels.attn_wide(q, o, self.nq, 1, self.d, wv, False, cache.keys, cache.values, ctx.positions,
-                              ctx.token_entry, table, items, hp, self.scale, window, 0, self.sink, self.score_cap, row_tiles,
-                              splits, part, part_ml)
+                rows = items.numel() // 4 * kernels.LATENT_ROWS if shared else tokens * self.nq
+                part = ws.buffer("attn_wide.part", rows * splits, wv if shared else self.d, torch.float32)
+                part_ml = ws.buffer("attn_wide.part_ml", rows * splits, 2, torch.float32)
+            if shared:
+                kernels.attn_latent(q, o, self.nq, self.d, wv, cache.keys, cache.values, ctx.positions, ctx.token_entry, table, items,
+                                    hp, self.scale, window, self.sink, self.score_cap, splits, part, part_ml)
+            else:
+                kernels.attn_wide(q, o, self.nq, 1, self.d, wv, False, cache.keys, cache.values, ctx.positions,
+                                  ctx.token_entry, table, items, hp, self.scale, window, 0, self.sink, self.score_cap, row_tiles,
+                                  splits, part, part_ml)
         else:
             o = ws.buffer("latent.rows", tokens, self.nq * self.d, torch.float32)
             kernels.attn_generic(q, o, self.nq, 1, self.d, cache.keys, cache.values, ctx.positions, ctx.token_entry,

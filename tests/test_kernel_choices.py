@@ -1,6 +1,7 @@
 """Decisions the host takes for the kernels (no GPU needed): what must hold of every choice, whatever the
 numbers the cost rules currently prefer, and for another count of compute units than the MI355X's."""
 import itertools
+import types
 
 import pytest
 
@@ -259,6 +260,24 @@ def test_keys_of_four_steps_are_not_cut_over_workgroups(units):
         n, steps = K.attn_wide_splits(items, 2, keys), (keys + 31) // 32
         assert 1 <= n <= 16 and (steps + n - 1) // n >= 3
         assert n == 1 or items * 2 * (n - 1) < 2 * units
+
+
+def test_latent_rows_are_shared_out_in_whole_blocks(units):
+    """attn_latent's splits: no more workgroups than units where an item is cut, none without a block, at most 64; its items hold
+    every (token, head) of the entries once."""
+    from pulse_infer_amd.ops import kernels as K
+
+    for items, keys in itertools.product((1, 3, 8, 32, 200, 256, 1000), (1, 64, 65, 128, 600, 4097, 40000)):
+        n, blocks = K.attn_latent_splits(items, keys), (keys + 63) // 64
+        assert 1 <= n <= 64 and (n == 1 or items * n <= units)
+        each = -(-blocks // n)
+        assert (n - 1) * each < blocks <= n * each
+    entries = [types.SimpleNamespace(first_row=a, count=n) for a, n in ((0, 1), (1, 7), (8, 64))]
+    for nq in (1, 4, 12, 16, 20, 32, 40, 64):
+        flat, hp = K.attn_latent_items(entries, nq)
+        held = [(t, h) for t0, nt, h0, nh in zip(*[iter(flat)] * 4) for t in range(t0, t0 + nt) for h in range(h0, h0 + nh)]
+        assert sorted(held) == [(t, h) for t in range(72) for h in range(nq)]
+        assert all(nt * hp <= 32 and nh <= hp for nt, nh in zip(flat[1::4], flat[3::4]))
 
 
 def test_nothing_but_the_copies_own_statement_touches_m0():
