@@ -17,6 +17,7 @@ from ..parts.base import (BLOCKS, EMBEDDINGS, HEADS, NORMS, POSITIONS, BuildCont
                           StepContext, Workspace, joined, says)
 from ..parts.rejoin import OriginRejoin
 from ..weights.store import TensorSpec, WeightLoader
+from .alike import AlikeRuns
 from .spec import ModelSpec
 
 ACT_DTYPES = {"bfloat16": torch.bfloat16, "float32": torch.float32}
@@ -109,7 +110,9 @@ class CausalLM:
         if self.rejoins:
             OriginRejoin.keep_origin(h, ctx, self.act_dtype)
         order = self.spec.order
-        for index, run in enumerate(order):
+
+        def forward(index: int) -> None:
+            run = order[index]
             # who reads the residual once this block is through: the block behind it (the final norm after the last
             # one gathers the wanted rows and stays a kernel of its own)
             follower = self.blocks[order[index + 1].layer] if index + 1 < len(order) else None
@@ -123,6 +126,15 @@ class CausalLM:
                 kernels.residual_add_row(stream.h, self.offsets[run.offset[0]][run.offset[1]])
                 stream.stats = stream.copy = None
             self.blocks[run.layer].forward(stream, ctx, cache_views[index])
+
+        alike = AlikeRuns.of(self, cache_views)
+        index = 0
+        while index < len(order):
+            if alike is not None:
+                index = alike.go(index, stream, forward)
+            else:
+                forward(index)
+                index += 1
         logits = torch.empty((ctx.num_wanted, self.vocab_size), dtype=torch.float32, device=self.device)
         if ctx.num_wanted == 0:
             return logits

@@ -8,6 +8,7 @@ from __future__ import annotations
 
 import ctypes
 import threading
+from contextlib import contextmanager
 from typing import Optional
 
 from ..csrc import build as _build
@@ -73,12 +74,39 @@ def load_variant(source: str, defines: dict) -> ctypes.CDLL:
         return lib
 
 
+def refused(lib: ctypes.CDLL, name: str) -> None:
+    raise KernelError(f"{name}: {lib.pulse_last_error().decode(errors='replace')}")
+
+
+# Calls that hand over scratch of torch's pool, which is the pool's again when they return.
+_BORROWING = ("pulse_gemm_f32_scratched",)
+_heard = threading.local()      # .calls: a list while this thread's calls are listened to
+
+
+def listening() -> bool:
+    return getattr(_heard, "calls", None) is not None
+
+
+@contextmanager
+def listen():
+    """The calls that this thread makes inside, as (library, name, entry point, arguments, whether they may be made again)."""
+    calls: list = []
+    _heard.calls = calls
+    try:
+        yield calls
+    finally:
+        _heard.calls = None
+
+
 def _invoke(lib: ctypes.CDLL, name: str, args) -> None:
     fn = getattr(lib, name)
     fn.restype = ctypes.c_int
+    calls = getattr(_heard, "calls", None)
+    if calls is not None:
+        calls.append((lib, name, fn, args, name not in _BORROWING))
     code = fn(*args)
     if code != 0:
-        raise KernelError(f"{name}: {lib.pulse_last_error().decode(errors='replace')}")
+        refused(lib, name)
 
 
 def call_in(lib: ctypes.CDLL, name: str, *args, label: str = "") -> None:
