@@ -233,6 +233,10 @@ constexpr int WAVE_CAP = 128;                           // candidates a wavefron
 constexpr int LIST_CAP = SAMPLE_WAVES * WAVE_CAP;       // candidates of a row
 constexpr int LIST_PER_LANE = LIST_CAP / PULSE_WAVE;
 
+// The first bit (from the top) in which two keys differ, -1 for none; what of a key lies above a bit.
+__device__ __forceinline__ int first_bit(uint32_t a, uint32_t b) { return a == b ? -1 : 31 - __builtin_clz(a ^ b); }
+__device__ __forceinline__ uint32_t above_bit(uint32_t key, int bit) { return bit >= 31 ? 0u : key & ~((2u << bit) - 1u); }
+
 // The end of the choice on a short list in LDS, by one wavefront: `n` candidates in vocabulary order (`list_i`, their
 // values `list_x`, which are overwritten), among them every token that top-k keeps.  The k-th largest value by a
 // search bit by bit, then top-p on what that kept (relative to its mass; without top-k relative to `whole`, the mass
@@ -250,15 +254,28 @@ __device__ bool finish_on_list(const int* list_i, float* list_x, int n, bool by_
         keys[j] = e < n ? order_key(list_x[e]) : 0u;
         wts[j] = e < n ? expf((list_x[e] - best) * inv_t) : 0.f;
     }
-    // the k-th largest key, bit by bit
+    // The searches go bit by bit, from the first bit on in which the list's largest and smallest key (then the largest and the k-th
+    // largest) differ: what is above is in all of them.  (32 rows of 151,936 with top-k 50, the list's choice alone on its wavefront: 10.3 us from
+    // the top bit and by lanes' counts, 9.1 so; left_kernel's top-k of mixed rows 16.8 and 14.0.)
+    uint32_t most = 0u, least = 0xffffffffu;
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+        most = max(most, keys[j]);
+        least = min(least, lane + j * PULSE_WAVE < n ? keys[j] : 0xffffffffu);
+    }
+    most = wave_reduce(most, [](uint32_t a, uint32_t b) { return max(a, b); });
+    least = wave_reduce(least, [](uint32_t a, uint32_t b) { return min(a, b); });
+    // the k-th largest key
     uint32_t keep = 0u;
     if (by_k) {
-        for (int bit = 31; bit >= 0; --bit) {
+        const int from = first_bit(most, least);
+        keep = from < 0 ? most : above_bit(most, from);
+        for (int bit = from; bit >= 0; --bit) {
             const uint32_t cand = keep | (1u << bit);
-            int c = 0;
+            int c = 0;      // (a key past the list is below every candidate)
 #pragma unroll
-            for (int j = 0; j < PER; ++j) c += (lane + j * PULSE_WAVE < n && keys[j] >= cand) ? 1 : 0;
-            if (wave_sum(c) >= k) keep = cand;
+            for (int j = 0; j < PER; ++j) c += __builtin_popcountll(__ballot(keys[j] >= cand));
+            if (c >= k) keep = cand;
         }
     }
     if (use_p) {
@@ -268,8 +285,10 @@ __device__ bool finish_on_list(const int* list_i, float* list_x, int n, bool by_
         mass = wave_sum(mass);
         const float want = p * (by_k ? mass : whole);
         if (!by_k && !(mass >= want)) return false;   // without top-k the list must hold all of the top_p set
-        uint32_t thr = 0u;
-        for (int bit = 31; bit >= 0; --bit) {
+        const uint32_t lowest = by_k ? keep : least;
+        const int from = first_bit(most, lowest);
+        uint32_t thr = from < 0 ? most : above_bit(most, from);
+        for (int bit = from; bit >= 0; --bit) {
             const uint32_t cand = thr | (1u << bit);
             const uint32_t lim = cand > keep ? cand : keep;
             float part_mass = 0.f;
@@ -316,9 +335,12 @@ struct Weigh {
     }
 };
 
-__device__ __forceinline__ mass_t mass_sum(mass_t v) {
-#pragma unroll
-    for (int off = PULSE_WAVE / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, PULSE_WAVE);
+__device__ __forceinline__ mass_t mass_sum(mass_t v) {      // (by lane moves: shuffles are trips through LDS)
+    auto step = [&](auto apart) __attribute__((always_inline)) {
+        const WaveTwo low = wave_two<decltype(apart)::value>(static_cast<uint32_t>(v)), high = wave_two<decltype(apart)::value>(static_cast<uint32_t>(v >> 32));
+        v = ((static_cast<mass_t>(high.a) << 32) | low.a) + ((static_cast<mass_t>(high.b) << 32) | low.b);
+    };
+    step(Int<32>()); step(Int<16>()); step(Int<8>()); step(Int<4>()); step(Int<2>()); step(Int<1>());
     return v;
 }
 // The sum over the lanes up to this one.
@@ -379,15 +401,22 @@ __device__ int edge_bin(const mass_t* hist, float p, int k, mass_t* waves, int* 
 }
 
 // The largest of the keys at or above which the mass is at least p of the whole: `n` tokens of the edge's bin, `base` the mass
-// above it (the masses through the bin reach that share, so there is one).  Every token's own sum, no order: called by a whole workgroup,
-// `best` (LDS) cleared before and read behind a barrier.
+// above it (the masses through the bin reach that share, so there is one).  Every token's own sum, no order, by as many neighbouring lanes
+// as there are for each (32 flat rows of 151,936, some 250 tokens in the bin, a lane each: 24 us of left_kernel, so 17.6).  Called by
+// a whole workgroup, `best` (LDS) cleared before and read behind a barrier.
 __device__ void edge_key(const uint32_t* keys, const mass_t* masses, int n, int threads, mass_t base, mass_t whole, float p, uint32_t* best) {
     const double want = static_cast<double>(p) * static_cast<double>(whole);
-    for (int e = threadIdx.x; e < n; e += threads) {
-        const uint32_t key = keys[e];
-        mass_t through = base;
-        for (int j = 0; j < n; ++j) through += keys[j] >= key ? masses[j] : 0;
-        if (static_cast<double>(through) >= want) atomicMax(best, key);
+    int each = 1;
+    while (each < PULSE_WAVE && 2 * each * n <= threads) each *= 2;
+    const int sub = threadIdx.x & (each - 1);
+    for (int e0 = 0; e0 < n; e0 += threads / each) {
+        const int e = e0 + static_cast<int>(threadIdx.x) / each;
+        const uint32_t key = keys[min(e, n - 1)];
+        mass_t through = 0;
+#pragma unroll 8
+        for (int j = sub; j < n; j += each) through += keys[j] >= key ? masses[j] : 0;
+        for (int off = 1; off < each; off *= 2) through += __shfl_xor(through, off, PULSE_WAVE);
+        if (sub == 0 && e < n && static_cast<double>(base + through) >= want) atomicMax(best, key);
     }
 }
 
@@ -1233,9 +1262,12 @@ __global__ __launch_bounds__(CHOOSE_THREADS) void chunked_choose_kernel(
 // leaves the row); with it a row is finished in chunks as well (left_collect_kernel, left_choose), unless a chunk has more
 // tokens at the edge than its segment holds: those rows a workgroup goes over alone (sample_row), in the launch that chooses.
 // (left_choose by a kernel of its own: every call waits for one launch more, top-p or top-k in 33 to 37 us, 37 to 41.)
-// 32 rows of 151,936, six of them flat under top-p alone and six with a k above the number of chunks: these three kernels 41 us,
+// 32 rows of 151,936, six of them flat under top-p alone and six with a k above the number of chunks: these three kernels 35 us,
 // where the histogram with float32 masses and sample_kernel's passes took 31 and 128.
-constexpr int REST_GROUPS = 32;                                             // workgroups for a row's histogram
+// Workgroups for a row's histogram: each adds its bins to the row's, which is what bounds them (32 rows of 151,936 under top-p alone:
+// 8 groups 15.1 us, 16 13.4, 32 15.9, 64 24.6; of 32,000: 7.2, 9.0, 12.6, 18.8), unless the rows are few (a whole step of one: 32 groups
+// 70.2 us, 16 72.6; of three of 32,000 72.3, 8 groups 74.4).
+constexpr int REST_GROUPS = 16, REST_GROUPS_FEW = 32, REST_SPAN = 4096, REST_FEW_ROWS = 8;
 
 // Whether a row is left, and what is known of it.
 struct LeftRow {
@@ -1278,11 +1310,11 @@ __global__ __launch_bounds__(SIMPLE_THREADS) void rest_kernel(
     const Weigh weigh(left.best, left.inv_t, vocab);
     const int first = blockIdx.x * SIMPLE_THREADS + threadIdx.x;
     if (left.k > 0)
-        sweep(row, first, vocab, REST_GROUPS * SIMPLE_THREADS, [&](int, float x) {
+        sweep(row, first, vocab, static_cast<int>(gridDim.x) * SIMPLE_THREADS, [&](int, float x) {
             if (x != -INFINITY) atomicAdd(&hist[bin_at(x, left.best, left.scale)], static_cast<mass_t>(1));
         });
     else
-        sweep(row, first, vocab, REST_GROUPS * SIMPLE_THREADS, [&](int, float x) {
+        sweep(row, first, vocab, static_cast<int>(gridDim.x) * SIMPLE_THREADS, [&](int, float x) {
             if (x != -INFINITY) atomicAdd(&hist[bin_at(x, left.best, left.scale)], weigh(x));
         });
     __syncthreads();
@@ -1668,7 +1700,8 @@ extern "C" int pulse_sample_chunked_rest(const float* logits, int rows, int voca
                        part_idx, part_mass, seg_i, seg_x, seg_n, chunks, out, done, rest);
     PULSE_LAUNCH_CHECK("sample_chunked (choice)");
     if (prepare) {
-        hipLaunchKernelGGL(rest_kernel, dim3(REST_GROUPS, rows), dim3(SIMPLE_THREADS), 0, stream, logits, vocab, row_stride, temperature,
+        const int groups = rows <= REST_FEW_ROWS ? REST_GROUPS_FEW : min(REST_GROUPS, (vocab + REST_SPAN - 1) / REST_SPAN);
+        hipLaunchKernelGGL(rest_kernel, dim3(groups, rows), dim3(SIMPLE_THREADS), 0, stream, logits, vocab, row_stride, temperature,
                            top_k, top_p, penalty, seen_row, seen_masks, banned, mask_words, part_max, part_min, chunks,
                            static_cast<const int*>(done), rest);
         if (chunks <= REST_MOST_CHUNKS) {

@@ -1674,6 +1674,36 @@ def test_rows_left_by_the_chunks_are_chosen_the_same_with_and_without_many_workg
         assert left.sum() >= 8 and (chosen[left] == 1).sum() >= 6        # most of them did not need the workgroup a row
 
 
+@pytest.mark.parametrize("n", [1, 2, 15, 16, 17, 64, 65, 255, 256, 257, 513, 1024])
+def test_edge_of_top_p_among_many_close_tokens(k, n):
+    """Top-p alone with its edge among n tokens of one bin of the histogram, a row that the chunks' short lists cannot hold: the tokens
+    that the definition in 64 bits names, u being the middle of a kept token's share (half of it, 4e-4 of the kept mass at
+    least, is the margin; p lies in the middle of a token's share too)."""
+    vocab, rows = 32768, 10
+    gen = torch.Generator().manual_seed(n)
+    x = torch.full((vocab,), -float("inf"))
+    x[torch.arange(0, vocab, 16)] = -10.0                     # more in every chunk than a segment holds
+    at = torch.arange(n)                                       # (in eight of the sixteen chunks)
+    close = at % 8 * 4096 + torch.randperm(1000, generator=gen)[at // 8] * 2 + 9
+    x[close] = -3.0 - 0.004 * torch.randperm(n, generator=gen) / n
+    x[5], x[7] = 0.0, -20.0
+    weight = x.double().exp()
+    order = torch.cat([torch.tensor([5]), close[x[close].argsort(descending=True)]])
+    kept = order[: 2 + int(0.6 * (n - 1))]
+    p = (weight[kept].sum() - weight[kept[-1]] / 2) / weight.sum()
+    want = torch.cat([kept[:1], kept[-1:], kept[torch.randint(0, kept.numel(), (rows - 2,), generator=gen)]])
+    u = []
+    for token in want.tolist():
+        u.append((weight[kept[kept < token]].sum() + weight[token] / 2) / weight[kept].sum())
+    out = torch.full((rows,), -9, dtype=torch.int32, device=DEV)
+    scratch = _chunked_scratch(k, rows, vocab)
+    k.sample_chunked(x.repeat(rows, 1).to(DEV), out, scratch, temperature=torch.ones(rows, device=DEV),
+                     top_k=torch.zeros(rows, dtype=torch.int32, device=DEV), top_p=torch.full((rows,), float(p), device=DEV),
+                     uniform=torch.tensor(u, dtype=torch.float32, device=DEV))
+    assert out.tolist() == want.tolist()
+    assert (scratch["done"][:rows] == 0).all()
+
+
 @pytest.mark.parametrize("vocab", [5, 40, 2049, 32000, 151936])
 @pytest.mark.parametrize("p", [0.0, 0.9])
 @pytest.mark.parametrize("more", [2, 60])
