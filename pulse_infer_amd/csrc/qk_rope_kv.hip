@@ -17,6 +17,8 @@
 // which they start), e.g. from the raw key columns for a design whose values are its keys as projected.
 #include "common.h"
 
+#include <algorithm>
+
 namespace {
 
 constexpr int MAX_PAIRS_PER_LANE = 4;  // head_dim <= 512
@@ -33,6 +35,9 @@ struct QkRopeArgs {
     int v_head0;     // the values of kv head g are columns (v_head0 + g) * d .. of the row
     float temp_coef; // query temperature: q *= 1 + temp_coef * ln(floor((pos + 1) / temp_every) + 1); temp_every 0: none
     int temp_every;
+    const float* parts;      // the rows as float32 shares of the projection, added up here in their order; null: qkv's
+    int shares;
+    int64_t part_stride, part_row;
 };
 
 // The factor of the query temperature at a position (1 when there is none).
@@ -217,12 +222,28 @@ __device__ __forceinline__ void load4<float>(const float* p, float* out) {
     for (int i = 0; i < 4; ++i) out[i] = v[i];
 }
 
+// Four neighbouring values of a row's shares, added up in their order (four shares are asked for together; past the last: the last
+// again, for nobody).
+__device__ __forceinline__ vf4 sum4(const float* p, int shares, int64_t part_stride) {
+    constexpr int AHEAD = 4;
+    vf4 sum = {0.f, 0.f, 0.f, 0.f};
+    for (int s0 = 0; s0 < shares; s0 += AHEAD) {
+        vf4 v[AHEAD];
+#pragma unroll
+        for (int u = 0; u < AHEAD; ++u) v[u] = *reinterpret_cast<const vf4*>(p + min(s0 + u, shares - 1) * part_stride);
+#pragma unroll
+        for (int u = 0; u < AHEAD; ++u)
+            if (s0 + u < shares) sum += v[u];
+    }
+    return sum;
+}
+
 __device__ __forceinline__ uint32_t pack2(float lo, float hi) {
     return static_cast<uint32_t>(f32_to_bf16(lo)) | (static_cast<uint32_t>(f32_to_bf16(hi)) << 16);
 }
 
 // One wavefront of it: the heads from number `y` * 64 / LPH on of token t.
-template <typename TW, int PAIRING, int LPH>
+template <typename TW, int PAIRING, int LPH, bool PARTS>
 __device__ __forceinline__ void qk_rope_rows(int t, int y, int lane, bf16_t* __restrict__ qkv, const TW* __restrict__ q_w,
                                              const TW* __restrict__ k_w, const float* __restrict__ cos_t,
                                              const float* __restrict__ sin_t, bf16_t* __restrict__ kcache,
@@ -252,7 +273,12 @@ __device__ __forceinline__ void qk_rope_rows(int t, int y, int lane, bf16_t* __r
 
     // every load before anything waits for one
     float e[8], wv[8], cs[4], sn[4];
-    if (PAIRING == 0) {
+    if constexpr (PARTS) {
+        const float* part = a.parts + static_cast<int64_t>(t) * a.part_row + static_cast<int64_t>(on ? hh : 0) * d;
+        const vf4 lo = sum4(part + oa, a.shares, a.part_stride), hi = sum4(part + ob, a.shares, a.part_stride);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) e[i] = lo[i], e[4 + i] = hi[i];
+    } else if (PAIRING == 0) {
         load8<bf16_t>(x + oa, e);
     } else {
         load4<bf16_t>(x + oa, e);
@@ -346,6 +372,7 @@ __device__ __forceinline__ void qk_rope_rows(int t, int y, int lane, bf16_t* __r
 constexpr int VW_TOKENS = 16;
 constexpr int VEC_THREADS = 256;
 
+template <bool PARTS>
 __device__ __forceinline__ void v_page_rows(int tile, int g, const bf16_t* __restrict__ qkv, bf16_t* __restrict__ vcache,
                                             const int* __restrict__ positions, const int* __restrict__ token_entry,
                                             const int* __restrict__ block_table, const QkRopeArgs& a, int tokens) {
@@ -356,9 +383,17 @@ __device__ __forceinline__ void v_page_rows(int tile, int g, const bf16_t* __res
     const int page = block_table[static_cast<int64_t>(token_entry[t]) * a.bt_width + pos / a.page_size];
     if (page < 0 || page >= a.num_pages) return;
     const int slot = pos % a.page_size;
-    const bf16_t* src = qkv + static_cast<int64_t>(t) * a.row_stride + static_cast<int64_t>(a.v_head0 + g) * a.d;
+    const int64_t column = static_cast<int64_t>(a.v_head0 + g) * a.d;
+    const bf16_t* src = qkv + static_cast<int64_t>(t) * a.row_stride + column;
     bf16_t* dst = vcache + (static_cast<int64_t>(page) * a.nkv + g) * a.d * a.page_size + slot;
     for (int c0 = cg * 8; c0 < a.d; c0 += 8 * (VEC_THREADS / VW_TOKENS)) {
+        if constexpr (PARTS) {
+            const float* part = a.parts + static_cast<int64_t>(t) * a.part_row + column + c0;
+            const vf4 lo = sum4(part, a.shares, a.part_stride), hi = sum4(part + 4, a.shares, a.part_stride);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) dst[static_cast<int64_t>(c0 + i) * a.page_size] = f32_to_bf16(i < 4 ? lo[i % 4] : hi[i % 4]);
+            continue;
+        }
         const uint4 raw = *reinterpret_cast<const uint4*>(src + c0);
         const uint32_t words[4] = {raw.x, raw.y, raw.z, raw.w};
 #pragma unroll
@@ -367,11 +402,15 @@ __device__ __forceinline__ void v_page_rows(int tile, int g, const bf16_t* __res
     }
 }
 
+// With PARTS the rows come as float32 shares of the projection (4 bytes a value and share): the lanes ask for four
+// shares' pieces of 16 bytes together.  40 heads of 128 at 97 / 160 / 357 tokens: 3.6 / 4.2 / 4.4 us from rounded rows, 4.5 / 5.0 / 8.5
+// from four shares, whose product takes 17.9 / 22.4 / 23.6 us where the whole one takes 20.3 / 27.4 / 32.3.
+//
 // Both in one launch: the first `rope_groups` workgroups are four wavefronts of rows each, the others 16 tokens' values of a
 // kv head.  (Neither reads what the other writes: q's columns are the only ones written in place, and the values are never
 // among them.)  Two launches took 4.0 + 2.9 us at 97 tokens, 5.6 + 4.8 at 509, 12.3 + 5.3 at 2,048 (32 + 8 heads of 128);
 // one 4.0, 5.7, 15.6.
-template <typename TW, int PAIRING, int LPH>
+template <typename TW, int PAIRING, int LPH, bool PARTS>
 __global__ __launch_bounds__(VEC_THREADS) void qk_rope_kv_vec_kernel(bf16_t* __restrict__ qkv, const TW* __restrict__ q_w,
                                                                      const TW* __restrict__ k_w,
                                                                      const float* __restrict__ cos_t,
@@ -387,15 +426,15 @@ __global__ __launch_bounds__(VEC_THREADS) void qk_rope_kv_vec_kernel(bf16_t* __r
         const unsigned row = __builtin_amdgcn_readfirstlane(b * (VEC_THREADS / PULSE_WAVE) + threadIdx.x / PULSE_WAVE);
         const unsigned t = row / static_cast<unsigned>(per_token);
         if (t >= static_cast<unsigned>(tokens)) return;
-        qk_rope_rows<TW, PAIRING, LPH>(static_cast<int>(t), static_cast<int>(row - t * per_token), threadIdx.x % PULSE_WAVE, qkv, q_w,
+        qk_rope_rows<TW, PAIRING, LPH, PARTS>(static_cast<int>(t), static_cast<int>(row - t * per_token), threadIdx.x % PULSE_WAVE, qkv, q_w,
                                        k_w, cos_t, sin_t, kcache, positions, token_entry, block_table, a);
     } else {
-        v_page_rows((b - rope_groups) / a.nkv, (b - rope_groups) % a.nkv, qkv, vcache, positions, token_entry, block_table, a,
+        v_page_rows<PARTS>((b - rope_groups) / a.nkv, (b - rope_groups) % a.nkv, qkv, vcache, positions, token_entry, block_table, a,
                     tokens);
     }
 }
 
-template <typename TW, int PAIRING>
+template <typename TW, int PAIRING, bool PARTS>
 void launch_vec(int lph, hipStream_t stream, int tokens, int heads, bf16_t* qkv, const TW* q_w, const TW* k_w,
                 const float* cos_t, const float* sin_t, bf16_t* kcache, bf16_t* vcache, const int* positions,
                 const int* token_entry, const int* block_table, const QkRopeArgs& a) {
@@ -404,7 +443,7 @@ void launch_vec(int lph, hipStream_t stream, int tokens, int heads, bf16_t* qkv,
     do {                                                                                                                \
         const int per_token = (heads + 64 / L - 1) / (64 / L);                                                          \
         const int rope_groups = static_cast<int>((static_cast<int64_t>(tokens) * per_token + 3) / 4);                   \
-        hipLaunchKernelGGL((qk_rope_kv_vec_kernel<TW, PAIRING, L>), dim3(rope_groups + value_groups), dim3(VEC_THREADS), 0, \
+        hipLaunchKernelGGL((qk_rope_kv_vec_kernel<TW, PAIRING, L, PARTS>), dim3(rope_groups + value_groups), dim3(VEC_THREADS), 0, \
                            stream, qkv, q_w, k_w, cos_t, sin_t, kcache, vcache, positions, token_entry, block_table, a,  \
                            tokens, per_token, rope_groups);                                                             \
     } while (0)
@@ -419,7 +458,7 @@ void launch_vec(int lph, hipStream_t stream, int tokens, int heads, bf16_t* qkv,
 
 }  // namespace
 
-extern "C" int pulse_qk_rope_kv(void* qkv, int x_dtype, int64_t row_stride, const void* q_w, const void* k_w,
+static int qk_rope_kv(const float* parts, int shares, int64_t part_stride, int64_t part_row, void* qkv, int x_dtype, int64_t row_stride, const void* q_w, const void* k_w,
                                 int w_dtype, float eps, const float* cos_t, const float* sin_t, int rotary_dim,
                                 int pairing, void* kcache, void* vcache, int c_dtype, const int* positions,
                                 const int* token_entry, const int* block_table, int bt_width, int tokens, int nq,
@@ -445,8 +484,16 @@ extern "C" int pulse_qk_rope_kv(void* qkv, int x_dtype, int64_t row_stride, cons
     } else {
         PULSE_REQUIRE(row_stride >= static_cast<int64_t>(nq) * d, "qk_rope_kv: row stride too small");
     }
+    if (parts) {
+        const int columns = write_kv ? std::max(nq + nkv, v_head0 + nkv) : nq;
+        PULSE_REQUIRE(shares > 0 && part_row >= static_cast<int64_t>(columns) * d && part_row % 4 == 0 && part_stride % 4 == 0 &&
+                      (shares == 1 || part_stride >= static_cast<int64_t>(tokens - 1) * part_row + static_cast<int64_t>(columns) * d) &&
+                      reinterpret_cast<uintptr_t>(parts) % 16 == 0, "qk_rope_kv: %d shares of rows %lld apart overlap or are not aligned",
+                      shares, static_cast<long long>(part_row));
+    }
     if (tokens == 0) return 0;
     QkRopeArgs a;
+    a.parts = parts; a.shares = shares; a.part_stride = part_stride; a.part_row = part_row;
     a.nq = nq; a.nkv = nkv; a.d = d; a.row_stride = row_stride; a.eps = eps;
     a.rotary_dim = (cos_t ? rotary_dim : 0); a.pairing = pairing;
     a.page_size = page_size; a.num_pages = num_pages; a.bt_width = bt_width; a.write_kv = write_kv;
@@ -460,18 +507,18 @@ extern "C" int pulse_qk_rope_kv(void* qkv, int x_dtype, int64_t row_stride, cons
                      (cos_t == nullptr || ((reinterpret_cast<uintptr_t>(cos_t) % 16) == 0 && (reinterpret_cast<uintptr_t>(sin_t) % 16) == 0));
     if (vec) {
         const int lph = d / 8;
+#define PULSE_ROPE(P, S)                                                                                                  \
+    launch_vec<TW, P, S>(lph, stream, tokens, heads, static_cast<bf16_t*>(qkv), static_cast<const TW*>(q_w),              \
+                         static_cast<const TW*>(k_w), cos_t, sin_t, static_cast<bf16_t*>(kcache),                         \
+                         static_cast<bf16_t*>(vcache), positions, token_entry, block_table, a)
         PULSE_DISPATCH_DTYPE(w_dtype, TW,
-            if (pairing == 0)
-                launch_vec<TW, 0>(lph, stream, tokens, heads, static_cast<bf16_t*>(qkv), static_cast<const TW*>(q_w),
-                                  static_cast<const TW*>(k_w), cos_t, sin_t, static_cast<bf16_t*>(kcache),
-                                  static_cast<bf16_t*>(vcache), positions, token_entry, block_table, a);
-            else
-                launch_vec<TW, 1>(lph, stream, tokens, heads, static_cast<bf16_t*>(qkv), static_cast<const TW*>(q_w),
-                                  static_cast<const TW*>(k_w), cos_t, sin_t, static_cast<bf16_t*>(kcache),
-                                  static_cast<bf16_t*>(vcache), positions, token_entry, block_table, a));
+            if (pairing == 0) { if (parts) PULSE_ROPE(0, true); else PULSE_ROPE(0, false); }
+            else { if (parts) PULSE_ROPE(1, true); else PULSE_ROPE(1, false); });
+#undef PULSE_ROPE
         PULSE_LAUNCH_CHECK("qk_rope_kv");
         return 0;
     }
+    PULSE_REQUIRE(!parts, "qk_rope_kv: shares need bfloat16 rows and pages, aligned and in chunks of eight values");
     const dim3 grid(tokens, heads);
     PULSE_DISPATCH_DTYPE(x_dtype, TX, PULSE_DISPATCH_DTYPE(w_dtype, TW, PULSE_DISPATCH_DTYPE(c_dtype, TC,
         hipLaunchKernelGGL((qk_rope_kv_kernel<TX, TW, TC>), grid, dim3(64), 0, stream, static_cast<TX*>(qkv),
@@ -480,4 +527,29 @@ extern "C" int pulse_qk_rope_kv(void* qkv, int x_dtype, int64_t row_stride, cons
                            block_table, a))));
     PULSE_LAUNCH_CHECK("qk_rope_kv");
     return 0;
+}
+
+extern "C" int pulse_qk_rope_kv(void* qkv, int x_dtype, int64_t row_stride, const void* q_w, const void* k_w,
+                                int w_dtype, float eps, const float* cos_t, const float* sin_t, int rotary_dim,
+                                int pairing, void* kcache, void* vcache, int c_dtype, const int* positions,
+                                const int* token_entry, const int* block_table, int bt_width, int tokens, int nq,
+                                int nkv, int d, int page_size, int num_pages, int write_kv, int plain_norm,
+                                int v_head0, float temp_coef, int temp_every, hipStream_t stream) {
+    return qk_rope_kv(nullptr, 0, 0, 0, qkv, x_dtype, row_stride, q_w, k_w, w_dtype, eps, cos_t, sin_t, rotary_dim, pairing, kcache, vcache, c_dtype, positions,
+                      token_entry, block_table, bt_width, tokens, nq, nkv, d, page_size, num_pages, write_kv, plain_norm, v_head0, temp_coef,
+                      temp_every, stream);
+}
+
+// The same with the projection's rows as `shares` float32 results [tokens, part_row], `part_stride` values apart, that are added up
+// in their order (a product whose inner dimension was shared out over workgroups); qkv only receives q.
+extern "C" int pulse_qk_rope_kv_parts(const float* parts, int shares, int64_t part_stride, int64_t part_row, void* qkv, int x_dtype, int64_t row_stride, const void* q_w, const void* k_w,
+                                int w_dtype, float eps, const float* cos_t, const float* sin_t, int rotary_dim,
+                                int pairing, void* kcache, void* vcache, int c_dtype, const int* positions,
+                                const int* token_entry, const int* block_table, int bt_width, int tokens, int nq,
+                                int nkv, int d, int page_size, int num_pages, int write_kv, int plain_norm,
+                                int v_head0, float temp_coef, int temp_every, hipStream_t stream) {
+    PULSE_REQUIRE(parts, "qk_rope_kv: null pointer");
+    return qk_rope_kv(parts, shares, part_stride, part_row, qkv, x_dtype, row_stride, q_w, k_w, w_dtype, eps, cos_t, sin_t, rotary_dim, pairing, kcache, vcache, c_dtype, positions,
+                      token_entry, block_table, bt_width, tokens, nq, nkv, d, page_size, num_pages, write_kv, plain_norm, v_head0, temp_coef,
+                      temp_every, stream);
 }

@@ -568,8 +568,9 @@ def qk_rope_kv(qkv: torch.Tensor, nq: int, nkv: int, d: int, q_weight: Optional[
                rotary_dim: int, pairing: int, kcache: Optional[torch.Tensor], vcache: Optional[torch.Tensor],
                positions: torch.Tensor, token_entry: torch.Tensor, block_table: Optional[torch.Tensor],
                write_kv: bool = True, plain_norm: bool = False, v_head0: Optional[int] = None,
-               q_temperature: Optional[tuple] = None) -> None:
-    """Per-head norm and rotation of q (in place) and k, and the page write of k and v.  ``plain_norm``: q and k are
+               q_temperature: Optional[tuple] = None, parts: Optional[torch.Tensor] = None) -> None:
+    """Per-head norm and rotation of q (in place) and k, and the page write of k and v.  ``parts`` float32 [shares, T, columns]:
+    the projection's rows are the sum of these shares, in their order, and ``qkv`` only receives q (see ``qk_rope_takes_parts``).  ``plain_norm``: q and k are
     divided by their root mean square without weights; ``v_head0``: the head number at which the values start in a
     row (default nq + nkv: behind the keys; nq: the values are the raw keys); ``q_temperature`` = (coef, every):
     q *= 1 + coef * ln(floor((position + 1) / every) + 1) after the norm."""
@@ -604,12 +605,24 @@ def qk_rope_kv(qkv: torch.Tensor, nq: int, nkv: int, d: int, q_weight: Optional[
               "qk_rope_kv: block_table must be contiguous int32 [entries, width]")
         width = block_table.shape[1]
         c_tag = _tag(kcache, "qk_rope_kv")
-    call("pulse_qk_rope_kv", _ptr(qkv), _i32(_tag(qkv, "qk_rope_kv")), _i64(qkv.stride(0)), _ptr(q_weight),
+    front = ()
+    if parts is not None:
+        _gpu("qk_rope_kv", parts)
+        _need(parts.dtype == torch.float32 and parts.dim() == 3 and parts.shape[1] == tokens and parts.shape[2] >= cols
+              and parts.is_contiguous(), f"qk_rope_kv: the shares must be contiguous float32 [shares, {tokens}, {cols}]")
+        front = (_ptr(parts), _i32(parts.shape[0]), _i64(parts.stride(0)), _i64(parts.stride(1)))
+    call("pulse_qk_rope_kv_parts" if front else "pulse_qk_rope_kv", *front, _ptr(qkv), _i32(_tag(qkv, "qk_rope_kv")), _i64(qkv.stride(0)), _ptr(q_weight),
          _ptr(k_weight), _i32(w_tag), _f32(eps), _ptr(cos), _ptr(sin), _i32(rotary_dim if cos is not None else 0),
          _i32(pairing), _ptr(kcache if write_kv else None), _ptr(vcache if write_kv else None), _i32(c_tag),
          _ptr(positions), _ptr(token_entry), _ptr(block_table if write_kv else None), _i32(width), _i32(tokens),
          _i32(nq), _i32(nkv), _i32(d), _i32(page_size), _i32(pages), _i32(1 if write_kv else 0),
          _i32(1 if plain_norm else 0), _i32(v_head0), _f32(temp_coef), _i32(temp_every), _stream())
+
+
+def qk_rope_takes_parts(qkv: torch.Tensor, d: int, rotary_dim: int, kcache: torch.Tensor, *weights: Optional[torch.Tensor]) -> bool:
+    """Whether ``qk_rope_kv`` takes these rows as float32 shares: in 16-byte pieces that neither heads nor rotation cut."""
+    return (qkv.dtype == torch.bfloat16 and kcache.dtype == torch.bfloat16 and d % 8 == 0 and rotary_dim % 8 == 0
+            and qkv.stride(0) % 8 == 0 and all(t is None or t.data_ptr() % 16 == 0 for t in (qkv, kcache, *weights)))
 
 
 def attn_generic(q: torch.Tensor, out: torch.Tensor, nq: int, nkv: int, d: int, kcache: torch.Tensor,

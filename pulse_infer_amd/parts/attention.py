@@ -199,12 +199,19 @@ class PagedAttention(Part):
         qkv = ws.buffer("attention.qkv", tokens, cols, self.act_dtype)
         if isinstance(x, LazyNorm) and not self.qkv.takes_lazy(x, rows=rows):
             x = x.materialize(ws.buffer("attention.normed", tokens, self.hidden, self.act_dtype))
-        self.qkv.forward(x, qkv, rows=rows)
         gate = qkv[:, self.kv_cols:self.kv_cols + self.nq] if self.output_gate else None
         tables = ctx.position_product(self.position, self.encodings) if self.position is not None else None
         table = ctx.block_tables[cache.group]
         attn = ws.buffer("attention.out", tokens, q_cols, self.act_dtype)
-        if self.decodes_from_raw(ctx, cache, qkv, tables):
+        from_raw = self.decodes_from_raw(ctx, cache, qkv, tables)
+        # (of the projection only q, k and v are read behind the rotation, which may take them as shares; a gate lies beside them)
+        parts = None
+        if not from_raw and rows is None and not self.output_gate and not isinstance(x, LazyNorm) and kernels.qk_rope_takes_parts(
+                qkv, self.d, tables.rotary_dim if tables is not None else 0, cache.keys, self.q_w, self.k_w):
+            parts = self.qkv.forward_parts(x, ws)
+        if parts is None:
+            self.qkv.forward(x, qkv, rows=rows)
+        if from_raw:
             # decoded tokens only: the attention kernel prepares q and each token's own key itself
             self.attend(qkv, attn, ctx, cache, table, raw=(tables, write), gate=gate)
         else:
@@ -213,7 +220,7 @@ class PagedAttention(Part):
                 tables.cos if tables is not None else None, tables.sin if tables is not None else None,
                 tables.rotary_dim if tables is not None else 0, tables.pairing if tables is not None else 0,
                 cache.keys, cache.values, ctx.positions, ctx.token_entry, table, write_kv=write,
-                plain_norm=self.plain_norm, v_head0=self.v_head0, q_temperature=self.q_temperature)
+                plain_norm=self.plain_norm, v_head0=self.v_head0, q_temperature=self.q_temperature, parts=parts)
             self.attend(qkv, attn, ctx, cache, table, gate=gate)
         out = ws.buffer("attention.proj", tokens, self.hidden, self.act_dtype)
         if residual is not None:

@@ -362,6 +362,32 @@ class Linear:
             return 0
         return kernels.gemm_stages_shares(self.STAGE_CUT_ROWS if rows <= self.SHARES_ROWS[1] else rows, n, k)
 
+    PARTS_MIN_K = 4096           # a plain product's inner dimension from which on its consumer had better add shares up
+
+    def forward_parts(self, x: torch.Tensor, workspace: Workspace) -> Optional[torch.Tensor]:
+        """The product as float32 shares [shares, rows, out] in a buffer of the workspace, for a caller whose next kernel adds
+        them up on the way (the rotation of q and k), or None: it is the faster one as it is (``forward``).
+
+        The whole product has few tiles at some hundreds of rows, and a tile's walk takes as long as K is long; shares fill the chip
+        and cost the consumer their way from memory.  Measured, qkv and the rotation behind it, us, as they are / in shares: 6,144 x
+        4,096 at 65 / 97 / 160 / 256 / 357 / 512 rows 25.0 / 22.4 / 30.8 / 33.3 / 37.7 / 39.7 and 19.6 / 22.4 / 27.7 / 30.1 / 34.6 / 38.6,
+        7,168 x 5,120 35.8 / 33.9 / 47.7 / 44.4 / 52.7 / 59.0 and 25.2 / 28.1 / 37.5 / 41.9 / 42.4 / 54.2, 10,240 x 8,192 81 / 60 / 65 / 74 / 90 / 101
+        and 46 / 48 / 52 / 60 / 75 / 86; of shorter inner dimensions it depends on the rows: 6,144 x 2,560 at 65 / 97 / 160 / 357 rows 21.4 / 19.3 / 27.4 /
+        30.7 and 17.0 / 19.7 / 24.9 / 32.6, 4,096 x 2,048 13.7 / 13.7 / 14.1 / 19.7 and 12.4 / 12.3 / 15.6 / 22.1.  Where a product's
+        smallest tiles fill the chip once, it stays whole: 5,120 x 4,096 at 160 rows 22.5 and 26.0.  (Over 66 sizes of six weights of 4,096
+        columns and more 0.88 of the time, two of them 1 to 2 % slower.)"""
+        rows, (n, k) = x.shape[0], self.weight.shape
+        if not (k >= self.PARTS_MIN_K and rows <= self.STAGE_ROWS_SHARES and self.may_stage(x, self.weight)) or n % 4:
+            return None
+        shares = kernels.gemm_stages_shares(max(rows, self.STAGE_CUT_ROWS), n, k)
+        tile_n, tile_m = kernels.gemm_stages_tile(rows, n, k)
+        tiles, units = ((n + tile_n - 1) // tile_n) * ((rows + tile_m - 1) // tile_m), compute_units()
+        if shares < 2 or (tile_n * tile_m <= 64 * 64 and 0.9 * units <= tiles <= units):
+            return None
+        parts = workspace.buffer(f"linear.shares.{n}.{k}", shares * rows, n, torch.float32).view(shares, rows, n)
+        kernels.gemm_stages(x, self.weight, parts)
+        return parts
+
     TILE_MIN_ROWS = 256          # from here on the tiled product for many rows is a candidate, and ``OWN_MANY_ROWS`` decides
 
     def takes_tiles(self, x: torch.Tensor, w: Optional[torch.Tensor] = None, swiglu: bool = False) -> bool:

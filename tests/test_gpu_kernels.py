@@ -227,6 +227,59 @@ def test_qk_rope_kv(k, dtype, case):
     assert torch.all(kcpu[~touched.unsqueeze(1).expand(-1, nkv, -1)] == 0)  # nothing else was written
 
 
+@pytest.mark.parametrize("shares", [1, 2, 8, 9, 17])
+@pytest.mark.parametrize("case", [
+    dict(nq=4, nkv=2, d=128, rot=128, pairing="half", norm=True, bs=16),
+    dict(nq=7, nkv=7, d=64, rot=32, pairing="half", norm=True, bs=16),
+    dict(nq=5, nkv=1, d=80, rot=80, pairing="interleaved", norm=False, bs=16),
+    dict(nq=3, nkv=1, d=256, rot=0, pairing="half", norm=False, bs=32, v_head0=3),
+])
+def test_qk_rope_kv_adds_shares(k, case, shares):
+    """The projection's rows as float32 shares: q, k and the pages as of their sum in 64 bits, the values the shares' sum in
+    32 bits and their order, rounded once; nothing of the projection's buffer but q is written."""
+    nq, nkv, d, rot, bs = case["nq"], case["nkv"], case["d"], case["rot"], case["bs"]
+    v_head0 = case.get("v_head0", nq + nkv)
+    eps, theta, tokens = 2e-5, 7e4, 35
+    heads = max(nq + nkv, v_head0 + nkv)
+    positions = list(range(6, 6 + tokens - 1)) + [0]
+    entry = [0] * (tokens - 1) + [1]
+    width = positions[-2] // bs + 1
+    table = torch.full((2, width), -1, dtype=torch.int32)
+    table[0] = torch.arange(3, 3 + width, dtype=torch.int32)
+    table[1, 0] = 1
+    kc, vc = _cache(3 + width + 1, nkv, bs, d, torch.bfloat16)
+    parts = (rnd(shares * tokens, heads * d + 4, seed=shares) * shares ** -0.5).to(torch.float32).view(shares, tokens, -1)
+    qkv = torch.full((tokens, heads * d + 8), 3.0, dtype=torch.bfloat16, device=DEV)
+    qw, qwref = as_stored(1 + 0.1 * rnd(d, seed=10), torch.bfloat16)
+    kw, kwref = as_stored(1 + 0.1 * rnd(d, seed=11), torch.bfloat16)
+    cos, sin = _tables(k, positions, theta, rot) if rot else (None, None)
+    weights = (qw, kw) if case["norm"] else (None, None)
+    assert k.qk_rope_takes_parts(qkv, d, rot, kc, *weights)
+    k.qk_rope_kv(qkv, nq, nkv, d, *weights, eps, cos, sin, rot, 0 if case["pairing"] == "interleaved" else 1, kc, vc,
+                 torch.tensor(positions, dtype=torch.int32, device=DEV), torch.tensor(entry, dtype=torch.int32, device=DEV),
+                 table.to(DEV), v_head0=v_head0, parts=parts.to(DEV))
+    ref = parts.to(F64).sum(0)
+    q = ref[:, :nq * d].reshape(tokens, nq, d)
+    kk = ref[:, nq * d:(nq + nkv) * d].reshape(tokens, nkv, d)
+    inorder = parts[0].clone()
+    for part in parts[1:]:
+        inorder += part
+    vv = inorder[:, v_head0 * d:(v_head0 + nkv) * d].to(torch.bfloat16).to(F64).reshape(tokens, nkv, d)
+    if case["norm"]:
+        q, kk = P.rms_norm(q, qwref, eps), P.rms_norm(kk, kwref, eps)
+    if rot:
+        q = P.rope(q, positions, theta, rot, case["pairing"])
+        kk = P.rope(kk, positions, theta, rot, case["pairing"])
+    got = qkv.cpu().to(F64)
+    assert torch.allclose(got[:, :nq * d].reshape(tokens, nq, d), q, **tol(torch.bfloat16))
+    assert (got[:, nq * d:] == 3.0).all()
+    kcpu, vcpu = kc.cpu().to(F64), vc.cpu().to(F64)
+    for t, (p, e) in enumerate(zip(positions, entry)):
+        page, slot = int(table[e, p // bs]), p % bs
+        assert torch.allclose(kcpu[page, :, slot, :], kk[t], **tol(torch.bfloat16))
+        assert torch.equal(vcpu[page, :, :, slot], vv[t])
+
+
 def _fill_cache(kc, vc, keys, vals, table_row, bs):
     """Put keys/vals [S, nkv, d] of one request into its pages."""
     for j in range(keys.shape[0]):
