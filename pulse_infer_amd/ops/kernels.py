@@ -1853,14 +1853,61 @@ def moe_max_tiles(pairs: int, experts: int, tile_rows: int) -> int:
     return (pairs + tile_rows - 1) // tile_rows + experts
 
 
+def _moe_places(scratch: torch.Tensor, pairs: int, tiles: int) -> tuple:
+    """Where the groups' parts lie in their scratch: rank, order, the tiles' experts, first places and rows, their number."""
+    base = scratch.data_ptr()
+    return tuple(ctypes.c_void_p(base + 4 * n)
+                 for n in (0, pairs, 2 * pairs, 2 * pairs + tiles, 2 * pairs + 2 * tiles, 2 * pairs + 3 * tiles))
+
+
+ROUTER_GROUPS_TOKENS = 16       # as TILE_TOKENS of moe.hip
+ROUTER_GROUPS_OUTPUTS = 256     # as GROUP_OUTPUTS of moe.hip
+
+
+def moe_router_groups(x: torch.Tensor, w_router: torch.Tensor, correction: Optional[torch.Tensor]) -> bool:
+    """Whether ``moe_router_grouped`` takes these rows: one workgroup's tokens, all in bfloat16."""
+    return (0 < x.shape[0] <= ROUTER_GROUPS_TOKENS and w_router.shape[0] <= ROUTER_GROUPS_OUTPUTS and x.shape[1] % 32 == 0
+            and all(t is None or t.dtype == torch.bfloat16 for t in (x, w_router, correction))
+            and x.data_ptr() % 16 == 0 and w_router.data_ptr() % 16 == 0)
+
+
+def moe_router_grouped(x: torch.Tensor, w_router: torch.Tensor, correction: Optional[torch.Tensor], top: int, idx: torch.Tensor,
+                       weight: torch.Tensor, experts: int, tile_rows: int, scratch: torch.Tensor, score: str = "softmax",
+                       renormalize: bool = True, groups: tuple = (0, 0), weight_scale: float = 1.0) -> None:
+    """``moe_router`` and the groups of its choices by expert in one launch, for what ``moe_router_groups`` takes.  ``scratch`` as for
+    ``moe_grouped``, which is then told ``grouped``."""
+    _need(score in ROUTER_SCORES, f"moe_router_grouped: unknown score function '{score}'")
+    _gpu("moe_router_grouped", x, w_router, correction, idx, weight, scratch)
+    tokens, hidden = x.shape
+    n = w_router.shape[0]
+    _need(moe_router_groups(x, w_router, correction) and x.is_contiguous() and w_router.is_contiguous() and w_router.shape[1] == hidden,
+          f"moe_router_grouped: x [T, {hidden}] and the router's weight [outputs, {hidden}] must be contiguous bfloat16, for "
+          f"{ROUTER_GROUPS_TOKENS} tokens and {ROUTER_GROUPS_OUTPUTS} outputs at most")
+    _need(correction is None or (correction.numel() == n and correction.is_contiguous()),
+          f"moe_router_grouped: the correction must hold {n} values")
+    _need(idx.dtype == torch.int32 and idx.is_contiguous() and tuple(idx.shape) == (tokens, top)
+          and weight.dtype == torch.float32 and weight.is_contiguous() and tuple(weight.shape) == (tokens, top),
+          f"moe_router_grouped: idx int32 and weight float32 must be [{tokens}, {top}]")
+    pairs, tiles = tokens * top, moe_max_tiles(tokens * top, experts, tile_rows)
+    _need(tile_rows in MOE_TILE_ROWS and 0 < experts <= n, f"moe_router_grouped: tiles of {MOE_TILE_ROWS} rows, experts among the outputs")
+    _need(scratch.dtype == torch.int32 and scratch.is_contiguous() and scratch.numel() >= 2 * pairs + 3 * tiles + 1,
+          "moe_router_grouped: the integer scratch is too small")
+    _, order, t_expert, t_row0, t_rows, count = _moe_places(scratch, pairs, tiles)
+    call("pulse_moe_router_grouped", _ptr(x), _ptr(w_router), _ptr(correction), _ptr(idx), _ptr(weight), _i32(tokens), _i32(hidden),
+         _i32(n), _i32(top), _i32(ROUTER_SCORES[score]), _i32(1 if renormalize else 0), _i32(groups[0]), _i32(groups[1]),
+         _f32(weight_scale), _i32(experts), _i32(tile_rows), _i32(tiles), order, t_expert, t_row0, t_rows, count, _stream())
+
+
 def moe_grouped(x: torch.Tensor, w_gate: torch.Tensor, w_up: torch.Tensor, w_down: torch.Tensor, idx: torch.Tensor,
                 weight: torch.Tensor, act: torch.Tensor, y: torch.Tensor, out: Optional[torch.Tensor], scratch: torch.Tensor,
-                tile_rows: int, weight_on_input: bool = False, activation: str = "silu", limit: float = 0.0) -> None:
+                tile_rows: int, weight_on_input: bool = False, activation: str = "silu", limit: float = 0.0,
+                grouped: bool = False) -> None:
     """out[t] = sum_k weight[t, k] * (expert idx[t, k] of x[t], or x[t] itself for an identity expert), the experts'
     products grouped by expert on the matrix cores.  ``act`` bfloat16 [T * top, ff] and ``y`` float32 [T * top, hidden]
     are scratch; ``scratch`` int32 holds 2 * T * top + 3 * moe_max_tiles + 1 entries.  ``weight_on_input``: an expert is
     fed weight * x and the results are added as they are; ``activation`` / ``limit`` as for ``moe_gate_up``.  ``out`` None:
-    the sum is left to the caller, ``y`` [T * top, hidden] holds what the experts gave."""
+    the sum is left to the caller, ``y`` [T * top, hidden] holds what the experts gave.  ``grouped``: ``scratch`` holds the groups
+    already (``moe_router_grouped`` with the same sizes)."""
     _need(activation in EXPERT_ACTIVATIONS, f"moe_grouped: unknown activation '{activation}'")
     _gpu("moe_grouped", x, w_gate, w_up, w_down, idx, weight, act, y, out, scratch)
     tokens, hidden = x.shape
@@ -1882,12 +1929,10 @@ def moe_grouped(x: torch.Tensor, w_gate: torch.Tensor, w_up: torch.Tensor, w_dow
     tiles = moe_max_tiles(pairs, experts, tile_rows)
     _need(scratch.dtype == torch.int32 and scratch.is_contiguous() and scratch.numel() >= 2 * pairs + 3 * tiles + 1,
           "moe_grouped: the integer scratch is too small")
-    base = scratch.data_ptr()
-    at = lambda n: ctypes.c_void_p(base + 4 * n)
-    rank, order = at(0), at(pairs)
-    t_expert, t_row0, t_rows, count = at(2 * pairs), at(2 * pairs + tiles), at(2 * pairs + 2 * tiles), at(2 * pairs + 3 * tiles)
-    call("pulse_moe_group", _ptr(idx), _i32(pairs), _i32(experts), _i32(tile_rows), _i32(tiles), rank, order, t_expert,
-         t_row0, t_rows, count, _stream())
+    rank, order, t_expert, t_row0, t_rows, count = _moe_places(scratch, pairs, tiles)
+    if not grouped:
+        call("pulse_moe_group", _ptr(idx), _i32(pairs), _i32(experts), _i32(tile_rows), _i32(tiles), rank, order, t_expert,
+             t_row0, t_rows, count, _stream())
     call("pulse_moe_gate_up_grouped", _ptr(x), _ptr(w_gate), _ptr(w_up), order, t_expert, t_row0, t_rows, count, _i32(tiles),
          _i32(tile_rows), _ptr(act), _i32(hidden), _i32(ff), _i32(top), _ptr(weight if weight_on_input else None),
          _i32(EXPERT_ACTIVATIONS[activation]), _f32(limit), _stream())

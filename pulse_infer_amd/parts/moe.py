@@ -153,24 +153,31 @@ class RoutedExperts(Part):
         ws = ctx.workspace
         idx = ws.buffer("moe.idx", tokens, self.top, torch.int32)
         weight = ws.buffer("moe.weight", tokens, self.top, torch.float32)
-        kernels.moe_router(x, self.router, self.correction, self.top, idx, weight, score=self.score,
-                           renormalize=self.renormalize, groups=self.groups,
-                           weight_scale=self.weight_scale)   # logits in float32 inside
+        how = dict(score=self.score, renormalize=self.renormalize, groups=self.groups, weight_scale=self.weight_scale)
+        grouped = kernels.moe_grouped_takes(x, self.w_gate, self.w_down)
+        ints = None
+        if grouped:
+            pairs = tokens * self.top
+            rows = kernels.moe_tile_rows(pairs, self.experts)
+            ints = ws.buffer("moe.ints", 2 * pairs + 3 * kernels.moe_max_tiles(pairs, self.experts, rows) + 1, 1, torch.int32).view(-1)
+        # (logits in float32 inside)
+        together = grouped and kernels.moe_router_groups(x, self.router, self.correction)
+        if together:
+            kernels.moe_router_grouped(x, self.router, self.correction, self.top, idx, weight, self.experts, rows, ints, **how)
+        else:
+            kernels.moe_router(x, self.router, self.correction, self.top, idx, weight, **how)
         act = ws.buffer("moe.act", tokens * self.top, self.ff, self.act_dtype)
         routed = ws.buffer("moe.out", tokens, self.hidden, torch.float32)
         later = None
-        if kernels.moe_grouped_takes(x, self.w_gate, self.w_down):
+        if grouped:
             # bfloat16: the pairs grouped by expert on the device, every expert's rows on the matrix cores
-            pairs = tokens * self.top
-            rows = kernels.moe_tile_rows(pairs, self.experts)
             y = ws.buffer("moe.y", pairs, self.hidden, torch.float32)
-            ints = ws.buffer("moe.ints", 2 * pairs + 3 * kernels.moe_max_tiles(pairs, self.experts, rows) + 1, 1, torch.int32)
             if defer and not self.identity and self.shared_gate is None:
                 later = ExpertSum(y, idx, None if self.weight_on_input else weight, self.experts)
             kernels.moe_grouped(x, self.w_gate, self.w_up, self.w_down, idx, weight, act, y,
-                                routed if later is None else None, ints.view(-1), rows,
+                                routed if later is None else None, ints, rows,
                                 weight_on_input=self.weight_on_input, activation=self.expert_activation,
-                                limit=self.limit)
+                                limit=self.limit, grouped=together)
         else:
             kernels.moe_gate_up(x, self.w_gate, self.w_up, idx, act, in_weight=weight if self.weight_on_input else None,
                                 activation=self.expert_activation, limit=self.limit)

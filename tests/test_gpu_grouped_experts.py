@@ -85,6 +85,40 @@ def test_router_logits_at_the_edges_of_its_blocks(n, hidden, tokens):
             break
 
 
+@pytest.mark.parametrize("tokens", [1, 7, 16])
+@pytest.mark.parametrize("n, experts, top, groups", [(2, 2, 1, (0, 0)), (16, 16, 4, (4, 2)), (64, 61, 8, (0, 0)), (65, 65, 6, (5, 3)),
+                                                     (256, 256, 64, (0, 0)), (250, 200, 33, (0, 0))])
+def test_router_and_groups_in_one_launch(tokens, n, experts, top, groups):
+    """The choices and weights of the router alone, bit by bit; every pair of an expert in one of its places, and tiles that hold an
+    expert's places one after the other."""
+    from pulse_infer_amd.ops import kernels
+
+    hidden, rows = 288, 32
+    x, w = rnd(tokens, hidden, seed=1).to(torch.bfloat16), (rnd(n, hidden, seed=2) * hidden ** -0.5).to(torch.bfloat16)
+    correction = (rnd(n, seed=3) * 0.1).to(torch.bfloat16).to(DEV)
+    x, w = x.to(DEV), w.to(DEV)
+    how = dict(score="sigmoid", renormalize=True, groups=groups, weight_scale=1.5)
+    idx, idx1 = (torch.full((tokens, top), -5, dtype=torch.int32, device=DEV) for _ in range(2))
+    weight, weight1 = (torch.full((tokens, top), float("nan"), device=DEV) for _ in range(2))
+    kernels.moe_router(x, w, correction, top, idx, weight, **how)
+    pairs = tokens * top
+    tiles = kernels.moe_max_tiles(pairs, experts, rows)
+    ints = torch.full((2 * pairs + 3 * tiles + 1,), -9, dtype=torch.int32, device=DEV)
+    assert kernels.moe_router_groups(x, w, correction)
+    kernels.moe_router_grouped(x, w, correction, top, idx1, weight1, experts, rows, ints, **how)
+    assert torch.equal(idx, idx1) and torch.equal(weight, weight1)
+    chosen, got = idx.cpu().flatten().tolist(), ints.cpu().tolist()
+    order, count = got[pairs:2 * pairs], got[-1]
+    t_expert, t_row0, t_rows = (got[2 * pairs + i * tiles:2 * pairs + (i + 1) * tiles][:count] for i in range(3))
+    want = {e: sorted(a for a, c in enumerate(chosen) if c == e) for e in set(chosen) if e < experts}
+    assert sum(t_rows) == sum(len(v) for v in want.values()) and all(0 < r <= rows for r in t_rows)
+    held = {}
+    for e, row0, r in zip(t_expert, t_row0, t_rows):
+        held.setdefault(e, []).extend(order[row0:row0 + r])
+    assert {e: sorted(v) for e, v in held.items()} == want
+    assert t_row0 == [sum(t_rows[:i]) for i in range(count)] and t_expert == sorted(t_expert)
+
+
 def test_grouped_experts_with_room_for_more_pairs_than_offsets_reach():
     """Lists with room for so many pairs that their rows may lie more than 4 GB apart take the kernels that go by pointers."""
     from pulse_infer_amd.ops import kernels
