@@ -619,10 +619,11 @@ def qk_rope_kv(qkv: torch.Tensor, nq: int, nkv: int, d: int, q_weight: Optional[
          _i32(1 if plain_norm else 0), _i32(v_head0), _f32(temp_coef), _i32(temp_every), _stream())
 
 
-def qk_rope_takes_parts(qkv: torch.Tensor, d: int, rotary_dim: int, kcache: torch.Tensor, *weights: Optional[torch.Tensor]) -> bool:
-    """Whether ``qk_rope_kv`` takes these rows as float32 shares: in 16-byte pieces that neither heads nor rotation cut."""
+def qk_rope_takes_parts(qkv: torch.Tensor, d: int, rotary_dim: int, kcache: torch.Tensor, *others: Optional[torch.Tensor]) -> bool:
+    """Whether ``qk_rope_kv`` takes these rows as float32 shares: in 16-byte pieces that neither heads nor rotation cut (``others``: the
+    norms' weights and the rotation's tables)."""
     return (qkv.dtype == torch.bfloat16 and kcache.dtype == torch.bfloat16 and d % 8 == 0 and rotary_dim % 8 == 0
-            and qkv.stride(0) % 8 == 0 and all(t is None or t.data_ptr() % 16 == 0 for t in (qkv, kcache, *weights)))
+            and qkv.stride(0) % 8 == 0 and all(t is None or t.data_ptr() % 16 == 0 for t in (qkv, kcache, *others)))
 
 
 def attn_generic(q: torch.Tensor, out: torch.Tensor, nq: int, nkv: int, d: int, kcache: torch.Tensor,
