@@ -10,7 +10,8 @@ are alike are launched from that record, their own tensors put in.
 Alike are runs of a pre-norm block of paged attention and a gated feed-forward whose attributes, their parts' attributes and
 their cache views are equal and whose tensors have equal types, shapes, strides and alignment.  That is looked at in every step,
 of the objects as they are then, and a record does not outlive its step.  Whatever else happens in the two runs (a product of the
-vendor library, an update added with statistics for the next norm, memory asked for) leaves everything to the parts.
+vendor library, an update added with statistics for the next norm, memory asked for, a tensor that both have or that a call names
+in any other way than by its first byte) leaves everything to the parts.
 """
 from __future__ import annotations
 
@@ -48,6 +49,11 @@ def _same_tensors(a: Tuple, b: Tuple) -> bool:
     return len(a) == len(b) and all(
         isinstance(y, torch.Tensor) and x.dtype == y.dtype and x.shape == y.shape and x.stride() == y.stride()
         and x.device == y.device and (x.data_ptr() ^ y.data_ptr()) % 16 == 0 for x, y in zip(a, b))
+
+
+def _reach(tensor: torch.Tensor) -> int:
+    """Bytes from a tensor's first value to the end of its last."""
+    return (sum((n - 1) * s for n, s in zip(tensor.shape, tensor.stride())) + 1) * tensor.element_size() if tensor.numel() else 0
 
 
 class AlikeRuns:
@@ -115,7 +121,8 @@ class AlikeRuns:
         if linear.library_calls != before or left[0] is None or left[0] != left[1]:
             self.tries = 0
             return index + 2
-        places = self._places(records, self._table(index), self._table(index + 1))
+        extents = [_reach(t) for t in (*first[1], self.blocks[self.order[index + 1].layer].mixer_norm.weight)]
+        places = self._places(records, self._table(index), self._table(index + 1), extents)
         if places is None:
             self.tries = 0
             return index + 2
@@ -139,11 +146,16 @@ class AlikeRuns:
         return update.data_ptr(), update.dtype, update.shape, update.stride(), stream.pending_scale
 
     @staticmethod
-    def _places(records: List[List[Tuple]], first: List[int], second: List[int]) -> Optional[List[Tuple]]:
-        """The second run's calls with the arguments that name tensors of its own, or None where they are not the first's."""
+    def _places(records: List[List[Tuple]], first: List[int], second: List[int], extents: List[int]) -> Optional[List[Tuple]]:
+        """The second run's calls with the arguments that name tensors of its own, or None where they are not the first's.  The
+        tensors lie from ``first`` and ``second`` on, ``extents`` bytes each.  Arguments that are equal in both calls stay as they are
+        for every run, so none of them may lie in a tensor of the two (a tensor that both have: another run may have one of its own)."""
         if len(records[0]) != len(records[1]) or len(set(first)) != len(first) or len(set(second)) != len(second):
             return None
+        if any(a == b for a, b in zip(first, second)):
+            return None
         at = {pointer: i for i, pointer in enumerate(first)}
+        inside = lambda value: any(p <= value < p + n for pointers in (first, second) for p, n in zip(pointers, extents))
         out = []
         for (lib, name, fn, a_args, clean), (lib_b, name_b, fn_b, b_args, clean_b) in zip(*records):
             if lib is not lib_b or name != name_b or len(a_args) != len(b_args) or not (clean and clean_b):
@@ -159,11 +171,14 @@ class AlikeRuns:
                         if b.value != second[at[a.value]]:
                             return None
                         own.append((b, at[a.value]))
-                    elif a.value != b.value:
+                    elif a.value != b.value or (isinstance(a, ctypes.c_void_p) and inside(a.value or 0)):
                         return None
                     continue
                 struct = getattr(a, "_obj", None), getattr(b, "_obj", None)
-                if None in struct or bytes(struct[0]) != bytes(struct[1]):     # (a structure by reference: no tensor of a run in it)
+                if None in struct or bytes(struct[0]) != bytes(struct[1]):     # (a structure by reference)
+                    return None
+                held = bytes(struct[0])
+                if any(inside(int.from_bytes(held[i:i + 8], "little")) for i in range(0, len(held) - 7, 8)):   # (a pointer's place)
                     return None
             out.append((fn_b, name, lib, b_args, own))
         return out
