@@ -93,9 +93,9 @@ class AlikeRuns:
         return other[0] == first[0] and _same_tensors(first[1], other[1])
 
     def _table(self, index: int) -> List[int]:
-        """Where the tensors lie that a run's calls may name: its own, its cache's, and the norm's that reads its result."""
-        follower = self.blocks[self.order[index + 1].layer].mixer_norm.weight
-        return [t.data_ptr() for t in self._describe(index)[1]] + [follower.data_ptr()]
+        """Where the tensors lie that a run's calls may name: its own and its cache's.  (Of the norm that reads its result only an
+        update with statistics wants to know; ``_left`` refuses it.)"""
+        return [t.data_ptr() for t in self._describe(index)[1]]
 
     def go(self, index: int, stream: Any, forward) -> int:
         """Run ``index`` (through ``forward(index)``) and as many behind it as are alike; the index behind them.  The last run of the
@@ -121,8 +121,7 @@ class AlikeRuns:
         if linear.library_calls != before or left[0] is None or left[0] != left[1]:
             self.tries = 0
             return index + 2
-        extents = [_reach(t) for t in (*first[1], self.blocks[self.order[index + 1].layer].mixer_norm.weight)]
-        places = self._places(records, self._table(index), self._table(index + 1), extents)
+        places = self._places(records, self._table(index), self._table(index + 1), [_reach(t) for t in first[1]])
         if places is None:
             self.tries = 0
             return index + 2

@@ -145,3 +145,16 @@ def test_layers_without_sinks_are_launched_from_the_record():
     launches = Launches(blocks, [RunSpec(layer) for layer in range(9)])
     launches.calls_of = lambda index: Launches.calls_of(launches, index)[1:]
     assert launches.step() == [0, 1, 2, 8]      # (the last run is left to its parts)
+
+
+@pytest.mark.parametrize("kinds", [[2], [3], [5, 8]])
+def test_a_block_of_another_kind_behind_alike_runs(kinds):
+    """Its norms have other names, and nobody asks it for theirs."""
+    blocks = [block() if layer not in kinds else made(ParallelBlock, norm=made(RMSNorm, weight=torch.zeros(4))) for layer in range(10)]
+    for b in blocks:
+        if type(b) is PreNormBlock:
+            del b.mixer.sink
+    launches = Launches(blocks, [RunSpec(layer) for layer in range(10)])
+    launches.calls_of = lambda index: [(P(7), P(blocks[index].mixer.qkv.weight.data_ptr()))]
+    through = launches.step()
+    assert through == {2: [0, 1, 2, 3, 4, 9], 3: list(range(10)), 5: [0, 1, 2, *range(4, 10)]}[kinds[0]]
