@@ -29,6 +29,7 @@ typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 typedef __attribute__((ext_vector_type(4))) unsigned int u32x4;
+typedef __attribute__((ext_vector_type(2))) unsigned short u16x2;
 
 constexpr int ROWS = 32;             // of an item, two tiles of 16
 constexpr int KEYS = 64;             // of a block
@@ -49,6 +50,14 @@ struct LatentArgs {
     float* part_ml;       // [items, ROWS, n_splits, 2] maximum and sum of weights
 };
 
+// Integers that are only read.  AGAIN: by scalar loads also behind stores (where there are none the compiler sees that by itself, and
+// asks for the queries first).
+template <bool AGAIN>
+__device__ __forceinline__ auto scalars(const int* p) {
+    if constexpr (AGAIN) return (const __attribute__((address_space(4))) int*)reinterpret_cast<uintptr_t>(p);
+    else return p;
+}
+
 // A row's result is its sums times this: 1 / sum of weights; a sink is one more term of that sum, exp(sink), with no key and no value.
 __device__ __forceinline__ float whole_share(float m, float l, const float* sink, int head) {
     float scale_out = 1.f;
@@ -62,7 +71,13 @@ __device__ __forceinline__ float whole_share(float m, float l, const float* sink
 }
 
 // CHUNKS: of 192 channels, as many as hold the head's; USUAL: exactly as many, every wavefront's value channels, and pages of 16 keys.
-template <int CHUNKS, bool USUAL>
+//
+// SEVERAL: items may hold several tokens.  A value that is not finite and that not all of them see would reach the others too (zero
+// times it).  So the blocks that not all see in full are looked through; where one is found, nothing is stored and the tokens come one
+// at a time, with every value that the token does not see cleared.  (A kernel of its own: short portions wait for it, us without /
+// with: 8 x 16 tokens on 1,000 keys at 16 heads 37.2 / 38.1, 3 x 51 10.1 / 11.2; a decoded token, which needs none of it, would take
+// 11.9 / 12.4 on 600 keys.)
+template <int CHUNKS, bool USUAL, bool SEVERAL>
 __global__ __launch_bounds__(WAVES* PULSE_WAVE, 2) void attn_latent_kernel(const bf16_t* __restrict__ q, float* __restrict__ out,
                                                                            const bf16_t* __restrict__ kcache,
                                                                            const bf16_t* __restrict__ vcache,
@@ -81,230 +96,259 @@ __global__ __launch_bounds__(WAVES* PULSE_WAVE, 2) void attn_latent_kernel(const
     __shared__ float max_s[PAGES][ROWS], sum_s[PAGES][ROWS];
     const int* it = items + 4 * blockIdx.x;
     const int t0 = it[0], nt = it[1], head0 = it[2], nh = it[3];
-    const int lane = threadIdx.x % PULSE_WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / PULSE_WAVE);
-    const int kt = wave % PAGES, half = wave / PAGES;
-    const int r = lane % 16, g = lane / 16;
-    const int d = USUAL ? WIDTH : a.d, page_size = USUAL ? 16 : a.page_size;
+    for (int from = 0, to = nt;;) {      // (all tokens at once, or one after the other)
+        int thread = threadIdx.x;
+        if constexpr (SEVERAL) asm volatile("" : "+v"(thread));      // (nothing made of it is kept in registers for another pass)
+        const int lane = thread % PULSE_WAVE, wave = __builtin_amdgcn_readfirstlane(thread / PULSE_WAVE);
+        const int kt = wave % PAGES, half = wave / PAGES;
+        const int r = lane % 16, g = lane / 16;
+        const int d = USUAL ? WIDTH : a.d, page_size = USUAL ? 16 : a.page_size;
 
-    // the rows' queries (rows that nobody has repeat the first token's first head; channels behind the head's are zeros)
-    constexpr int Q_PIECES = ROWS * WIDTH / 8, Q_EACH = (Q_PIECES + THREADS - 1) / THREADS;     // of 16 bytes; those of a thread
-    u32x4 qv[Q_EACH];
+        // the rows' queries (rows that nobody has repeat the first token's first head; channels behind the head's are zeros)
+        constexpr int Q_PIECES = ROWS * WIDTH / 8, Q_EACH = (Q_PIECES + THREADS - 1) / THREADS;     // of 16 bytes; those of a thread
+        u32x4 qv[Q_EACH];
 #pragma unroll
-    for (int i = 0; i < Q_EACH; ++i) {
-        const int at = min(static_cast<int>(threadIdx.x) + i * THREADS, Q_PIECES - 1), row = at / (WIDTH / 8), e = at % (WIDTH / 8) * 8;
-        const int ti = row / a.hp, hi = row % a.hp;
-        const bool there = ti < nt && hi < nh;
-        qv[i] = *reinterpret_cast<const u32x4*>(q + static_cast<int64_t>(t0 + (there ? ti : 0)) * a.q_stride +
-                                                static_cast<int64_t>(head0 + (there ? hi : 0)) * d + min(e, d - 8));
-    }
-    const int* bt = block_table + static_cast<int64_t>(token_entry[t0]) * a.bt_width;
-    const int pos_first = positions[t0], pos_last = positions[t0 + nt - 1];
-    const int lo = (a.window > 0 && pos_first - a.window + 1 > 0) ? pos_first - a.window + 1 : 0;
-    const int lo16 = lo & ~15;
-    const int blocks = (pos_last + 1 - lo16 + KEYS - 1) / KEYS;
-    const int per = (blocks + a.n_splits - 1) / a.n_splits;
-    const int block0 = static_cast<int>(blockIdx.y) * per, block1 = min(blocks, block0 + per);
-
-    // the page of a block's tile of 16 keys, -1 where there is none
-    pulse_i32x4 page, found;      // (vectors: of arrays that a lane or a wavefront chooses from, the compiler makes memory)
-    auto look_up = [&](int block) __attribute__((always_inline)) {      // (a block ahead, so that the table's trip lies behind another)
-#pragma unroll
-        for (int t = 0; t < PAGES; ++t) found[t] = bt[min((lo16 + block * KEYS + 16 * t) / page_size, a.bt_width - 1)];
-    };
-    auto take_pages = [&](int block) __attribute__((always_inline)) {
-#pragma unroll
-        for (int t = 0; t < PAGES; ++t) {
-            const int j = lo16 + block * KEYS + 16 * t, pi = j / page_size;
-            const int p = __builtin_amdgcn_readfirstlane(found[t]);
-            page[t] = (j <= pos_last) & (pi < a.bt_width) & (p >= 0) & (p < a.num_pages) ? p : -1;
+        for (int i = 0; i < Q_EACH; ++i) {
+            const int at = min(thread + i * THREADS, Q_PIECES - 1), row = at / (WIDTH / 8), e = at % (WIDTH / 8) * 8;
+            const int ti = row / a.hp, hi = row % a.hp;
+            const bool there = ti < nt && hi < nh;
+            qv[i] = *reinterpret_cast<const u32x4*>(q + static_cast<int64_t>(t0 + (there ? ti : 0)) * a.q_stride +
+                                                    static_cast<int64_t>(head0 + (there ? hi : 0)) * d + min(e, d - 8));
         }
-    };
-    auto own_page = [&]() __attribute__((always_inline)) {
-        int mine = page[0];
-#pragma unroll
-        for (int t = 1; t < PAGES; ++t) mine = kt == t ? page[t] : mine;
-        return mine;
-    };
-    bf16x8 ka[PIECES];
-    auto ask_keys = [&](int block) __attribute__((always_inline)) {      // (addresses that always hold keys; masked behind)
-        const int off = (lo16 + block * KEYS + 16 * kt) % page_size;
-        const int e0 = 32 * PIECES * half + 8 * g;
-        const bf16_t* krow = kcache + (static_cast<int64_t>(max(own_page(), 0)) * page_size + off + r) * d + (USUAL ? e0 : 0);
-#pragma unroll
-        for (int u = 0; u < PIECES; ++u) ka[u] = *reinterpret_cast<const bf16x8*>(krow + (USUAL ? 32 * u : min(e0 + 32 * u, d - 8)));
-    };
-    const int tiles = USUAL ? CT : max(0, min(CT, a.wv / 16 - CT * wave));   // of value channels, this wavefront's
-    u32x4 values[2][CT][2];                                              // of this block and the next, in turn
-    auto ask_values = [&](int block, u32x4 (&va)[CT][2]) __attribute__((always_inline)) {
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            const int p = g / 2 ? page[2 * u + 1] : page[2 * u];
-            const int off = (lo16 + block * KEYS + 32 * u + 16 * (g / 2)) % page_size + 8 * (g % 2);
-            const bf16_t* base = vcache + (static_cast<int64_t>(max(p, 0)) * d + (tiles > 0 ? 16 * CT * wave : 0) + r) * page_size + off;
-#pragma unroll
-            for (int c = 0; c < CT; ++c) va[c][u] = *reinterpret_cast<const u32x4*>(base + (USUAL ? c : max(0, min(c, tiles - 1))) * (16 * page_size));
-        }
-    };
+        __builtin_amdgcn_sched_barrier(0);      // (the queries are asked for before the trips to the lists)
+        const auto bt = scalars<SEVERAL>(block_table) + static_cast<int64_t>(scalars<SEVERAL>(token_entry)[t0]) * a.bt_width;
+        const int pos_first = scalars<SEVERAL>(positions)[t0], pos_last = scalars<SEVERAL>(positions)[t0 + nt - 1];
+        const int lo = (a.window > 0 && pos_first - a.window + 1 > 0) ? pos_first - a.window + 1 : 0;
+        const int lo16 = lo & ~15;
+        const int blocks = (pos_last + 1 - lo16 + KEYS - 1) / KEYS;
+        const int per = (blocks + a.n_splits - 1) / a.n_splits;
+        const int block0 = static_cast<int>(blockIdx.y) * per, block1 = min(blocks, block0 + per);
 
-    int pos[2], token[2], head[2];
-    bool valid[2];
+        // the page of a block's tile of 16 keys, -1 where there is none
+        pulse_i32x4 page, found;      // (vectors: of arrays that a lane or a wavefront chooses from, the compiler makes memory)
+        auto look_up = [&](int block) __attribute__((always_inline)) {      // (a block ahead, so that the table's trip lies behind another)
 #pragma unroll
-    for (int rr = 0; rr < 2; ++rr) {
-        const int row = 16 * rr + r, ti = row / a.hp, hi = row % a.hp;
-        valid[rr] = ti < nt && hi < nh;
-        token[rr] = t0 + (valid[rr] ? ti : 0);
-        head[rr] = head0 + (valid[rr] ? hi : 0);
-        pos[rr] = positions[token[rr]];
-    }
-    const bool own_valid = half ? valid[1] : valid[0];
-    const int own_pos = half ? pos[1] : pos[0];
-    float m_run[2] = {-INFINITY, -INFINITY}, l_run = 0.f;
-    f32x4 acc[2][CT];
-#pragma unroll
-    for (int rr = 0; rr < 2; ++rr)
-#pragma unroll
-        for (int c = 0; c < CT; ++c) acc[rr][c] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-    look_up(block0);
-    take_pages(block0);
-    look_up(block0 + 1);
-    ask_keys(block0);          // (a workgroup without blocks asks for the first page's, for nobody)
-    ask_values(block0, values[0]);
-#pragma unroll
-    for (int i = 0; i < Q_EACH; ++i) {
-        const int at = min(static_cast<int>(threadIdx.x) + i * THREADS, Q_PIECES - 1), e = at % (WIDTH / 8) * 8;   // (the last piece several times)
-        *reinterpret_cast<u32x4*>(&q_s[at / (WIDTH / 8) * Q_STRIDE + e]) = e < d ? qv[i] : u32x4{0u, 0u, 0u, 0u};
-    }
-    __syncthreads();
-
-    auto step = [&](int block, u32x4 (&va)[CT][2], u32x4 (&va_next)[CT][2]) __attribute__((always_inline)) {
-        const int j0 = lo16 + block * KEYS;
-        if constexpr (!USUAL) {
-#pragma unroll
-            for (int u = 0; u < PIECES; ++u)
-                if (32 * (PIECES * half + u) + 8 * g >= d) ka[u] = __builtin_bit_cast(bf16x8, u32x4{0u, 0u, 0u, 0u});
-        }
-        f32x4 s[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
-        // (a piece's queries ahead of its products, no more: the keys and values in flight take the registers)
-        bf16x8 qb[2][2];
-        const bf16_t* q_at = &q_s[r * Q_STRIDE + 32 * PIECES * half + 8 * g];
-        auto read_queries = [&](int u) __attribute__((always_inline)) {
-#pragma unroll
-            for (int rr = 0; rr < 2; ++rr) qb[u % 2][rr] = *reinterpret_cast<const bf16x8*>(q_at + 16 * rr * Q_STRIDE + 32 * u);
+            for (int t = 0; t < PAGES; ++t) found[t] = bt[min((lo16 + block * KEYS + 16 * t) / page_size, a.bt_width - 1)];
         };
-        read_queries(0);
+        auto take_pages = [&](int block) __attribute__((always_inline)) {
 #pragma unroll
-        for (int u = 0; u < PIECES; ++u) {
-            if (u + 1 < PIECES) read_queries(u + 1);
-            __builtin_amdgcn_sched_barrier(0);
+            for (int t = 0; t < PAGES; ++t) {
+                const int j = lo16 + block * KEYS + 16 * t, pi = j / page_size;
+                const int p = __builtin_amdgcn_readfirstlane(found[t]);
+                page[t] = (j <= pos_last) & (pi < a.bt_width) & (p >= 0) & (p < a.num_pages) ? p : -1;
+            }
+        };
+        auto own_page = [&]() __attribute__((always_inline)) {
+            int mine = page[0];
 #pragma unroll
-            for (int rr = 0; rr < 2; ++rr) s[rr] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka[u], qb[u % 2][rr], s[rr], 0, 0, 0);
-        }
-        const f32x4 s0 = s[0], s1 = s[1];
-        half_s[wave][lane] = half ? s0 : s1;
-        __syncthreads();
-        f32x4 own = half ? s1 : s0;
-        own += half_s[(wave + PAGES) % WAVES][lane];
-        // what of this block's values has never been stored is cleared (a weight of zero times whatever lies there must stay zero)
-        const bool there = own_page() >= 0;
-        const bool whole = j0 + KEYS - 1 <= pos_last && page[0] >= 0 && page[1] >= 0 && page[2] >= 0 && page[3] >= 0;
-        if (!whole) {
+            for (int t = 1; t < PAGES; ++t) mine = kt == t ? page[t] : mine;
+            return mine;
+        };
+        bf16x8 ka[PIECES];
+        auto ask_keys = [&](int block) __attribute__((always_inline)) {      // (addresses that always hold keys; masked behind)
+            const int off = (lo16 + block * KEYS + 16 * kt) % page_size;
+            const int e0 = 32 * PIECES * half + 8 * g;
+            const bf16_t* krow = kcache + (static_cast<int64_t>(max(own_page(), 0)) * page_size + off + r) * d + (USUAL ? e0 : 0);
+#pragma unroll
+            for (int u = 0; u < PIECES; ++u) ka[u] = *reinterpret_cast<const bf16x8*>(krow + (USUAL ? 32 * u : min(e0 + 32 * u, d - 8)));
+        };
+        const int tiles = USUAL ? CT : max(0, min(CT, a.wv / 16 - CT * wave));   // of value channels, this wavefront's
+        u32x4 values[2][CT][2];                                              // of this block and the next, in turn
+        auto ask_values = [&](int block, u32x4 (&va)[CT][2]) __attribute__((always_inline)) {
 #pragma unroll
             for (int u = 0; u < 2; ++u) {
                 const int p = g / 2 ? page[2 * u + 1] : page[2 * u];
-                const int stored = p >= 0 ? pos_last + 1 - (j0 + 32 * u + 8 * g) : 0;
+                const int off = (lo16 + block * KEYS + 32 * u + 16 * (g / 2)) % page_size + 8 * (g % 2);
+                const bf16_t* base = vcache + (static_cast<int64_t>(max(p, 0)) * d + (tiles > 0 ? 16 * CT * wave : 0) + r) * page_size + off;
 #pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                    const uint32_t keep = (2 * k < stored ? 0x0000FFFFu : 0u) | (2 * k + 1 < stored ? 0xFFFF0000u : 0u);
-#pragma unroll
-                    for (int c = 0; c < CT; ++c) va[c][u][k] &= keep;
-                }
+                for (int c = 0; c < CT; ++c) va[c][u] = *reinterpret_cast<const u32x4*>(base + (USUAL ? c : max(0, min(c, tiles - 1))) * (16 * page_size));
             }
-        }
-        if (block + 1 < block1) {
-            take_pages(block + 1);
-            look_up(block + 2);
-            ask_keys(block + 1);
-            ask_values(block + 1, va_next);
-        }
-        float mx = -INFINITY;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int j = j0 + 16 * kt + 4 * g + i;
-            float x = own[i] * a.scale;
-            if (a.cap > 0.f) x = a.cap * tanhf(x / a.cap);
-            own[i] = own_valid && there && j <= own_pos && (a.window == 0 || own_pos - j < a.window) ? x : -INFINITY;
-            mx = fmaxf(mx, own[i]);
-        }
-        mx = across_rows(mx, LaneMax());
-        if (g == 0) max_s[kt][16 * half + r] = mx;
-        __syncthreads();
-        float alpha[2];
+        };
+
+        int pos[2], token[2], head[2];
+        bool valid[2];
 #pragma unroll
         for (int rr = 0; rr < 2; ++rr) {
-            float m_new = m_run[rr];
-#pragma unroll
-            for (int w = 0; w < PAGES; ++w) m_new = fmaxf(m_new, max_s[w][16 * rr + r]);
-            alpha[rr] = m_new == -INFINITY ? 1.f : expf(m_run[rr] - m_new);
-            m_run[rr] = m_new;
+            const int row = 16 * rr + r, ti = row / a.hp, hi = row % a.hp;
+            valid[rr] = ti >= from && ti < to && hi < nh;
+            token[rr] = t0 + (valid[rr] ? ti : 0);
+            head[rr] = head0 + (valid[rr] ? hi : 0);
+            pos[rr] = positions[token[rr]];
         }
-        const float m_own = half ? m_run[1] : m_run[0];
-        float sum = 0.f;
-        bf16x4 p4;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const float p = own[i] == -INFINITY ? 0.f : expf(own[i] - m_own);
-            sum += p;
-            p4[i] = static_cast<__bf16>(p);
-        }
-        *reinterpret_cast<bf16x4*>(&p_s[(16 * half + r) * P_STRIDE + 16 * kt + 4 * g]) = p4;
-        l_run = l_run * (half ? alpha[1] : alpha[0]) + sum;
-        __syncthreads();
+        const int seen_last = SEVERAL ? scalars<SEVERAL>(positions)[t0 + to - 1] : pos_last;       // the keys that any of the pass's tokens sees
+        const int seen_first = from == 0 ? lo : a.window > 0 ? max(0, seen_last - a.window + 1) : 0;
+        u16x2 odd = {0, 0};      // the largest of the values that not all of them see, without their signs
+        const bool own_valid = half ? valid[1] : valid[0];
+        const int own_pos = half ? pos[1] : pos[0];
+        float m_run[2] = {-INFINITY, -INFINITY}, l_run = 0.f;
+        f32x4 acc[2][CT];
 #pragma unroll
         for (int rr = 0; rr < 2; ++rr)
 #pragma unroll
-            for (int c = 0; c < CT; ++c) acc[rr][c] *= alpha[rr];
+            for (int c = 0; c < CT; ++c) acc[rr][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+        look_up(block0);
+        take_pages(block0);
+        look_up(block0 + 1);
+        ask_keys(block0);          // (a workgroup without blocks asks for the first page's, for nobody)
+        ask_values(block0, values[0]);
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            bf16x8 pb[2];
-#pragma unroll
-            for (int rr = 0; rr < 2; ++rr) pb[rr] = *reinterpret_cast<const bf16x8*>(&p_s[(16 * rr + r) * P_STRIDE + 32 * u + 8 * g]);
-#pragma unroll
-            for (int c = 0; c < CT; ++c)
-#pragma unroll
-                for (int rr = 0; rr < 2; ++rr)
-                    acc[rr][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, va[c][u]), pb[rr], acc[rr][c], 0, 0, 0);
+        for (int i = 0; i < Q_EACH; ++i) {
+            const int at = min(thread + i * THREADS, Q_PIECES - 1), e = at % (WIDTH / 8) * 8;   // (the last piece several times)
+            *reinterpret_cast<u32x4*>(&q_s[at / (WIDTH / 8) * Q_STRIDE + e]) = e < d ? qv[i] : u32x4{0u, 0u, 0u, 0u};
         }
-        // (the next block's weights are written behind two more barriers, its halves and maxima behind one, after all have been read)
-    };
-    for (int block = block0; block < block1; block += 2) {
-        step(block, values[0], values[1]);
-        if (block + 1 < block1) step(block + 1, values[1], values[0]);
-    }
-    // a row's sum over the lanes and the wavefronts that share it
-    l_run = across_rows(l_run, LaneSum());
-    if (g == 0) sum_s[kt][16 * half + r] = l_run;
-    __syncthreads();
+        __syncthreads();
+
+        auto step = [&](int block, u32x4 (&va)[CT][2], u32x4 (&va_next)[CT][2]) __attribute__((always_inline)) {
+            const int j0 = lo16 + block * KEYS;
+            if constexpr (!USUAL) {
 #pragma unroll
-    for (int rr = 0; rr < 2; ++rr) {
-        float l = 0.f;
+                for (int u = 0; u < PIECES; ++u)
+                    if (32 * (PIECES * half + u) + 8 * g >= d) ka[u] = __builtin_bit_cast(bf16x8, u32x4{0u, 0u, 0u, 0u});
+            }
+            f32x4 s[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+            // (a piece's queries ahead of its products, no more: the keys and values in flight take the registers)
+            bf16x8 qb[2][2];
+            const bf16_t* q_at = &q_s[r * Q_STRIDE + 32 * PIECES * half + 8 * g];
+            auto read_queries = [&](int u) __attribute__((always_inline)) {
 #pragma unroll
-        for (int w = 0; w < PAGES; ++w) l += sum_s[w][16 * rr + r];
-        float* row;
-        float share = 1.f;
-        if (a.n_splits > 1) {       // one of several workgroups over these keys: the sums as they are, for the merge
-            const int64_t at = (static_cast<int64_t>(blockIdx.x) * ROWS + 16 * rr + r) * a.n_splits + blockIdx.y;
-            if (valid[rr] && wave == 0 && g == 0) { a.part_ml[2 * at] = m_run[rr]; a.part_ml[2 * at + 1] = l; }
-            row = a.part + at * a.wv;
-        } else {
-            share = whole_share(m_run[rr], l, sink, head[rr]);
-            row = out + static_cast<int64_t>(token[rr]) * a.o_stride + static_cast<int64_t>(head[rr]) * d;
+                for (int rr = 0; rr < 2; ++rr) qb[u % 2][rr] = *reinterpret_cast<const bf16x8*>(q_at + 16 * rr * Q_STRIDE + 32 * u);
+            };
+            read_queries(0);
+#pragma unroll
+            for (int u = 0; u < PIECES; ++u) {
+                if (u + 1 < PIECES) read_queries(u + 1);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int rr = 0; rr < 2; ++rr) s[rr] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka[u], qb[u % 2][rr], s[rr], 0, 0, 0);
+            }
+            const f32x4 s0 = s[0], s1 = s[1];
+            half_s[wave][lane] = half ? s0 : s1;
+            __syncthreads();
+            f32x4 own = half ? s1 : s0;
+            own += half_s[(wave + PAGES) % WAVES][lane];
+            // what of this block's values nobody sees, or has never been stored, is cleared (a weight of zero times whatever lies there
+            // must stay zero)
+            const bool there = own_page() >= 0;
+            const bool whole = j0 >= seen_first && j0 + KEYS - 1 <= seen_last && page[0] >= 0 && page[1] >= 0 && page[2] >= 0 && page[3] >= 0;
+            if (!whole) {
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+                    const int p = g / 2 ? page[2 * u + 1] : page[2 * u];
+                    const int gone = seen_first - (j0 + 32 * u + 8 * g);
+                    const uint32_t seen = p >= 0 ? seen_last + 1 - seen_first : 0;
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        const uint32_t keep = (static_cast<uint32_t>(2 * k - gone) < seen ? 0x0000FFFFu : 0u) |
+                                              (static_cast<uint32_t>(2 * k + 1 - gone) < seen ? 0xFFFF0000u : 0u);
+#pragma unroll
+                        for (int c = 0; c < CT; ++c) va[c][u][k] &= keep;
+                    }
+                }
+            }
+            if (SEVERAL && to - from > 1 && (j0 + KEYS - 1 > pos_first || (a.window > 0 && j0 <= pos_last - a.window))) {
+#pragma unroll
+                for (int u = 0; u < 2; ++u)
+#pragma unroll
+                    for (int c = 0; c < CT; ++c)
+#pragma unroll
+                        for (int k = 0; k < 4; ++k)
+                            odd = __builtin_elementwise_max(odd, __builtin_bit_cast(u16x2, va[c][u][k] & 0x7FFF7FFFu));
+            }
+            if (block + 1 < block1) {
+                take_pages(block + 1);
+                look_up(block + 2);
+                ask_keys(block + 1);
+                ask_values(block + 1, va_next);
+            }
+            float mx = -INFINITY;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int j = j0 + 16 * kt + 4 * g + i;
+                float x = own[i] * a.scale;
+                if (a.cap > 0.f) x = a.cap * tanhf(x / a.cap);
+                own[i] = own_valid && there && j <= own_pos && (a.window == 0 || own_pos - j < a.window) ? x : -INFINITY;
+                mx = fmaxf(mx, own[i]);
+            }
+            mx = across_rows(mx, LaneMax());
+            if (g == 0) max_s[kt][16 * half + r] = mx;
+            __syncthreads();
+            float alpha[2];
+#pragma unroll
+            for (int rr = 0; rr < 2; ++rr) {
+                float m_new = m_run[rr];
+#pragma unroll
+                for (int w = 0; w < PAGES; ++w) m_new = fmaxf(m_new, max_s[w][16 * rr + r]);
+                alpha[rr] = m_new == -INFINITY ? 1.f : expf(m_run[rr] - m_new);
+                m_run[rr] = m_new;
+            }
+            const float m_own = half ? m_run[1] : m_run[0];
+            float sum = 0.f;
+            bf16x4 p4;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float p = own[i] == -INFINITY ? 0.f : expf(own[i] - m_own);
+                sum += p;
+                p4[i] = static_cast<__bf16>(p);
+            }
+            *reinterpret_cast<bf16x4*>(&p_s[(16 * half + r) * P_STRIDE + 16 * kt + 4 * g]) = p4;
+            l_run = l_run * (half ? alpha[1] : alpha[0]) + sum;
+            __syncthreads();
+#pragma unroll
+            for (int rr = 0; rr < 2; ++rr)
+#pragma unroll
+                for (int c = 0; c < CT; ++c) acc[rr][c] *= alpha[rr];
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                bf16x8 pb[2];
+#pragma unroll
+                for (int rr = 0; rr < 2; ++rr) pb[rr] = *reinterpret_cast<const bf16x8*>(&p_s[(16 * rr + r) * P_STRIDE + 32 * u + 8 * g]);
+#pragma unroll
+                for (int c = 0; c < CT; ++c)
+#pragma unroll
+                    for (int rr = 0; rr < 2; ++rr)
+                        acc[rr][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, va[c][u]), pb[rr], acc[rr][c], 0, 0, 0);
+            }
+            // (the next block's weights are written behind two more barriers, its halves and maxima behind one, after all have been read)
+        };
+        for (int block = block0; block < block1; block += 2) {
+            step(block, values[0], values[1]);
+            if (block + 1 < block1) step(block + 1, values[1], values[0]);
         }
-        if (valid[rr]) {
-#pragma unroll
-            for (int c = 0; c < CT; ++c)
-                if (c < tiles) *reinterpret_cast<f32x4*>(row + 16 * (CT * wave + c) + 4 * g) = acc[rr][c] * share;
+        if constexpr (SEVERAL) {
+            if (to - from > 1 && __syncthreads_or(max(odd[0], odd[1]) >= 0x7F80)) {
+                to = 1;
+                continue;
+            }
         }
+        // a row's sum over the lanes and the wavefronts that share it
+        l_run = across_rows(l_run, LaneSum());
+        if (g == 0) sum_s[kt][16 * half + r] = l_run;
+        __syncthreads();
+#pragma unroll
+        for (int rr = 0; rr < 2; ++rr) {
+            float l = 0.f;
+#pragma unroll
+            for (int w = 0; w < PAGES; ++w) l += sum_s[w][16 * rr + r];
+            float* row;
+            float share = 1.f;
+            if (a.n_splits > 1) {       // one of several workgroups over these keys: the sums as they are, for the merge
+                const int64_t at = (static_cast<int64_t>(blockIdx.x) * ROWS + 16 * rr + r) * a.n_splits + blockIdx.y;
+                if (valid[rr] && wave == 0 && g == 0) { a.part_ml[2 * at] = m_run[rr]; a.part_ml[2 * at + 1] = l; }
+                row = a.part + at * a.wv;
+            } else {
+                share = whole_share(m_run[rr], l, sink, head[rr]);
+                row = out + static_cast<int64_t>(token[rr]) * a.o_stride + static_cast<int64_t>(head[rr]) * d;
+            }
+            if (valid[rr]) {
+#pragma unroll
+                for (int c = 0; c < CT; ++c)
+                    if (c < tiles) *reinterpret_cast<f32x4*>(row + 16 * (CT * wave + c) + 4 * g) = acc[rr][c] * share;
+            }
+        }
+        if (!SEVERAL || to == nt) break;
+        from = to++;
+        __syncthreads();
     }
 }
 
@@ -355,13 +399,13 @@ __global__ __launch_bounds__(256) void attn_latent_merge_kernel(const float* __r
 
 // q [tokens, q_stride] bfloat16: head h's query at h * d.  out float32 [tokens, o_stride]: of head h's d channels at h * d the first
 // wv are written.  items int32 [n_items, 4]: first token, tokens, first head, heads; row r (of 32) of an item is token r / hp, head
-// r % hp; rows that no item holds are left as they are.  n_splits > 1: the keys of every item are shared out over that many
+// r % hp; rows that no item holds are left as they are.  several: whether an item may hold several tokens.  n_splits > 1: the keys of every item are shared out over that many
 // workgroups, whose sums (part float32 [n_items, 32, n_splits, wv], part_ml [n_items, 32, n_splits, 2]) a second kernel brings
 // together.  kcache [pages, 1, page, d], vcache [pages, 1, d, page] bfloat16.
 extern "C" int pulse_attn_latent(const void* q, int64_t q_stride, float* out, int64_t o_stride, const void* kcache,
                                  const void* vcache, const int* positions, const int* token_entry, const int* block_table,
-                                 int bt_width, const int* items, int n_items, int hp, int nq, int d, int wv, int page_size,
-                                 int num_pages, float scale, int window, const float* sink, float softcap, int n_splits,
+                                 int bt_width, const int* items, int n_items, int hp, int several, int nq, int d, int wv,
+                                 int page_size, int num_pages, float scale, int window, const float* sink, float softcap, int n_splits,
                                  float* part, float* part_ml, hipStream_t stream) {
     PULSE_REQUIRE(nq > 0 && d >= 16 && d % 16 == 0 && d <= 576, "attn_latent: %d heads of %d channels", nq, d);
     PULSE_REQUIRE(wv > 0 && wv % 16 == 0 && wv <= d && wv <= 16 * CT * WAVES, "attn_latent: %d of %d value channels", wv, d);
@@ -382,9 +426,14 @@ extern "C" int pulse_attn_latent(const void* q, int64_t q_stride, float* out, in
     a.scale = scale; a.cap = softcap; a.window = window;
     a.n_splits = n_splits; a.part = part; a.part_ml = part_ml;
     auto launch = [&](auto chunks, auto usual) {
-        hipLaunchKernelGGL((attn_latent_kernel<decltype(chunks)::value, decltype(usual)::value>), dim3(n_items, n_splits), dim3(WAVES * PULSE_WAVE), 0, stream,
-                           static_cast<const bf16_t*>(q), out, static_cast<const bf16_t*>(kcache), static_cast<const bf16_t*>(vcache),
-                           positions, token_entry, block_table, items, sink, a);
+        auto run = [&](auto several_v) {
+            hipLaunchKernelGGL((attn_latent_kernel<decltype(chunks)::value, decltype(usual)::value, decltype(several_v)::value>),
+                               dim3(n_items, n_splits), dim3(WAVES * PULSE_WAVE), 0, stream, static_cast<const bf16_t*>(q), out,
+                               static_cast<const bf16_t*>(kcache), static_cast<const bf16_t*>(vcache), positions, token_entry,
+                               block_table, items, sink, a);
+        };
+        if (several && hp <= ROWS / 2) run(std::true_type());      // (with more heads an item holds one token)
+        else run(std::false_type());
     };
     if (d == 576 && wv == 16 * CT * WAVES && page_size == 16) launch(std::integral_constant<int, 3>(), std::true_type());
     else if (d > 384) launch(std::integral_constant<int, 3>(), std::false_type());

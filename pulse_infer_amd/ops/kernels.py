@@ -812,9 +812,10 @@ def attn_latent_splits(n_items: int, keys: int) -> int:
 def attn_latent(q: torch.Tensor, out: torch.Tensor, nq: int, d: int, wv: int, kcache: torch.Tensor, vcache: torch.Tensor,
                 positions: torch.Tensor, token_entry: torch.Tensor, block_table: torch.Tensor, items: torch.Tensor, hp: int,
                 scale: float, window: int = 0, sink: Optional[torch.Tensor] = None, softcap: float = 0.0, n_splits: int = 1,
-                part: Optional[torch.Tensor] = None, part_ml: Optional[torch.Tensor] = None) -> None:
+                part: Optional[torch.Tensor] = None, part_ml: Optional[torch.Tensor] = None, several: bool = True) -> None:
     """Paged attention on the matrix cores over latent rows that all query heads share: out float32 [T, nq * d], of a head's
-    channels the first ``wv``, of the rows that the items hold.  Window, sinks and score cap as for ``attn_generic``; scratch
+    channels the first ``wv``, of the rows that the items hold.  ``several`` False: every item holds one token.  Window, sinks and
+    score cap as for ``attn_generic``; scratch
     for splits, a row an item's row and split: ``part`` float32 [items * 32 * n_splits, wv], ``part_ml`` [.., 2]."""
     _gpu("attn_latent", q, out, kcache, vcache, positions, token_entry, block_table, items, sink)
     tokens = q.shape[0]
@@ -838,8 +839,8 @@ def attn_latent(q: torch.Tensor, out: torch.Tensor, nq: int, d: int, wv: int, kc
         _need(sink.dtype == torch.float32 and sink.is_contiguous() and sink.numel() == nq, f"attn_latent: the sinks must be float32 [{nq}]")
     call("pulse_attn_latent", _ptr(q), _i64(q.stride(0) if tokens > 1 else q.shape[1]), _ptr(out),
          _i64(out.stride(0) if tokens > 1 else out.shape[1]), _ptr(kcache), _ptr(vcache), _ptr(positions), _ptr(token_entry),
-         _ptr(block_table), _i32(block_table.shape[1]), _ptr(items), _i32(items.numel() // 4), _i32(hp), _i32(nq), _i32(d), _i32(wv),
-         _i32(page_size), _i32(pages), _f32(scale), _i32(window), _ptr(sink), _f32(softcap), _i32(n_splits),
+         _ptr(block_table), _i32(block_table.shape[1]), _ptr(items), _i32(items.numel() // 4), _i32(hp), _i32(1 if several else 0), _i32(nq), _i32(d),
+         _i32(wv), _i32(page_size), _i32(pages), _f32(scale), _i32(window), _ptr(sink), _f32(softcap), _i32(n_splits),
          _ptr(part if n_splits > 1 else None), _ptr(part_ml if n_splits > 1 else None), _stream(),
          label=f"d={d} values={wv} splits={n_splits}")
 

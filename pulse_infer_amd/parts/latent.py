@@ -243,8 +243,8 @@ class LatentAttention(PagedAttention):
                 entries = [e for i, e in enumerate(ctx.entries) if plan is None or i not in plan["at"]]
                 row_tiles = kernels.attn_wide_row_tiles(ctx.num_tokens)
                 flat, hp = kernels.attn_latent_items(entries, self.nq) if shared else kernels.attn_wide_items(entries, self.nq, 1, row_tiles)
-                ctx.extras[key] = (ctx.to_device(flat), hp, row_tiles)
-            items, hp, row_tiles = ctx.extras[key]
+                ctx.extras[key] = (ctx.to_device(flat), hp, row_tiles, any(e.count > 1 for e in entries))
+            items, hp, row_tiles, several = ctx.extras[key]
             seen = min(ctx.max_context, window + 32) if window else ctx.max_context
             if shared:
                 splits = kernels.attn_latent_splits(items.numel() // 4, seen)
@@ -259,7 +259,7 @@ class LatentAttention(PagedAttention):
                 part_ml = ws.buffer("attn_wide.part_ml", rows * splits, 2, torch.float32)
             if shared:
                 kernels.attn_latent(q, o, self.nq, self.d, wv, cache.keys, cache.values, ctx.positions, ctx.token_entry, table, items,
-                                    hp, self.scale, window, self.sink, self.score_cap, splits, part, part_ml)
+                                    hp, self.scale, window, self.sink, self.score_cap, splits, part, part_ml, several)
             else:
                 kernels.attn_wide(q, o, self.nq, 1, self.d, wv, False, cache.keys, cache.values, ctx.positions,
                                   ctx.token_entry, table, items, hp, self.scale, window, 0, self.sink, self.score_cap, row_tiles,

@@ -43,7 +43,7 @@ def attend(q, rows, spans, nq, d, wv, page=16, splits=1, window=0, sink=None, ca
     ml = torch.full((part.shape[0], 2), float("nan"), device=DEV)
     kernels.attn_latent(q.to(DEV), out, nq, d, wv, kc.to(DEV), vc.to(DEV), ints(positions), ints(entry),
                         order.to(torch.int32).to(DEV).contiguous(), ints(flat), hp, scale, window,
-                        None if sink is None else sink.to(DEV), cap, splits, part, ml)
+                        None if sink is None else sink.to(DEV), cap, splits, part, ml, several=max(flat[1::4]) > 1)
     return out.cpu().view(tokens, nq, d)
 
 
@@ -116,3 +116,24 @@ def test_a_value_that_is_not_a_number_is_not_hidden():
     for splits in (1, 4):
         got = attend(q, rows, [1, 1], nq, d, wv, splits=splits)
         assert not torch.isnan(got[0, :, :wv]).any() and torch.isnan(got[1, :, :wv]).all()
+
+
+@pytest.mark.parametrize("odd", [float("nan"), float("inf")])
+@pytest.mark.parametrize("nq,d,wv,span,splits,window", [(16, 576, 512, 2, 1, 0), (16, 576, 512, 7, 3, 20), (4, 320, 256, 11, 1, 20),
+                                                        (4, 576, 512, 16, 2, 0), (1, 288, 256, 40, 1, 0), (32, 576, 512, 3, 1, 20)])
+def test_a_value_that_is_not_finite_stays_with_the_tokens_that_see_it(nq, d, wv, span, splits, window, odd):
+    """Tokens that share a workgroup with one that sees it and do not see it themselves: of its own position, of one before them
+    that their window has left behind, of one that nobody's window holds any more."""
+    n = 131
+    for place in (n - 1, n - span + 1, n - span // 2, *((n - span - window + 2, n - span - window) if window else ())):
+        rows = [rnd(n, d, seed=1), rnd(n - 3, d, seed=2)]
+        rows[0][place, 5] = odd
+        q = rnd(2 * span, nq * d, seed=3)
+        scale = 2.0 * d ** -0.5
+        got = attend(q, rows, [span, span], nq, d, wv, splits=splits, window=window, scale=scale)[..., :wv].to(F64)
+        want, size = expected(q, rows, [span, span], nq, d, wv, window=window, scale=scale)
+        hit = [place <= p and not (window and p - place >= window) for p in range(n - span, n)] + [False] * span
+        assert torch.isfinite(want).all((1, 2)).tolist() == [not h for h in hit]
+        assert torch.equal(torch.isfinite(got), torch.isfinite(want)), place     # (a score of minus infinity spoils its channel alone)
+        rest = torch.isfinite(want)
+        assert ((got - want).abs() <= 2.0 ** -8 * size + 1e-4)[rest].all(), place
