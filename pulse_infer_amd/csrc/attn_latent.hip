@@ -154,14 +154,16 @@ __global__ __launch_bounds__(WAVES* PULSE_WAVE, 2) void attn_latent_kernel(const
         };
         const int tiles = USUAL ? CT : max(0, min(CT, a.wv / 16 - CT * wave));   // of value channels, this wavefront's
         u32x4 values[2][CT][2];                                              // of this block and the next, in turn
+        const bool idle = !USUAL && tiles == 0;      // no value channels: nothing to bring in and nothing to add up
         auto ask_values = [&](int block, u32x4 (&va)[CT][2]) __attribute__((always_inline)) {
+            if (idle) return;
 #pragma unroll
             for (int u = 0; u < 2; ++u) {
                 const int p = g / 2 ? page[2 * u + 1] : page[2 * u];
                 const int off = (lo16 + block * KEYS + 32 * u + 16 * (g / 2)) % page_size + 8 * (g % 2);
-                const bf16_t* base = vcache + (static_cast<int64_t>(max(p, 0)) * d + (tiles > 0 ? 16 * CT * wave : 0) + r) * page_size + off;
+                const bf16_t* base = vcache + (static_cast<int64_t>(max(p, 0)) * d + 16 * CT * wave + r) * page_size + off;
 #pragma unroll
-                for (int c = 0; c < CT; ++c) va[c][u] = *reinterpret_cast<const u32x4*>(base + (USUAL ? c : max(0, min(c, tiles - 1))) * (16 * page_size));
+                for (int c = 0; c < CT; ++c) va[c][u] = *reinterpret_cast<const u32x4*>(base + (USUAL ? c : min(c, tiles - 1)) * (16 * page_size));
             }
         };
 
@@ -231,7 +233,7 @@ __global__ __launch_bounds__(WAVES* PULSE_WAVE, 2) void attn_latent_kernel(const
             // must stay zero)
             const bool there = own_page() >= 0;
             const bool whole = j0 >= seen_first && j0 + KEYS - 1 <= seen_last && page[0] >= 0 && page[1] >= 0 && page[2] >= 0 && page[3] >= 0;
-            if (!whole) {
+            if (!whole && !idle) {
 #pragma unroll
                 for (int u = 0; u < 2; ++u) {
                     const int p = g / 2 ? page[2 * u + 1] : page[2 * u];
@@ -246,7 +248,7 @@ __global__ __launch_bounds__(WAVES* PULSE_WAVE, 2) void attn_latent_kernel(const
                     }
                 }
             }
-            if (SEVERAL && to - from > 1 && (j0 + KEYS - 1 > pos_first || (a.window > 0 && j0 <= pos_last - a.window))) {
+            if (SEVERAL && !idle && to - from > 1 && (j0 + KEYS - 1 > pos_first || (a.window > 0 && j0 <= pos_last - a.window))) {
 #pragma unroll
                 for (int u = 0; u < 2; ++u)
 #pragma unroll
@@ -294,6 +296,7 @@ __global__ __launch_bounds__(WAVES* PULSE_WAVE, 2) void attn_latent_kernel(const
             *reinterpret_cast<bf16x4*>(&p_s[(16 * half + r) * P_STRIDE + 16 * kt + 4 * g]) = p4;
             l_run = l_run * (half ? alpha[1] : alpha[0]) + sum;
             __syncthreads();
+            if (idle) return;
 #pragma unroll
             for (int rr = 0; rr < 2; ++rr)
 #pragma unroll

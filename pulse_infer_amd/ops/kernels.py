@@ -779,7 +779,13 @@ LATENT_MAX_VALUES = 512
 
 
 def attn_latent_takes(q: torch.Tensor, kcache: torch.Tensor, d: int, wv: int) -> bool:
-    """Whether ``attn_latent`` takes these operands: what ``attn_wide`` takes with one kv head, up to its widths."""
+    """Whether ``attn_latent`` takes these operands: what ``attn_wide`` takes with one kv head, up to its widths.  It is the faster one
+    whatever the heads and widths (us, ``attn_wide`` / it; stored / value channels, heads): 8 requests of 1,500 tokens 576 / 512, 1 head
+    19 / 13, 16 21 / 15, 32 28 / 18, 128 62 / 31; 288 / 256, 8 13.7 / 11.5, 32 17.6 / 13.0, 128 29.5 / 22.6; 8 x 16 tokens on 1,000 keys
+    576 / 512, 8 47 / 27, 16 75 / 38, 32 145 / 51; 288 / 256, 8 24.2 / 19.8, 16 27.8 / 26.9; 3 x 51 tokens 288 / 256, 8 10.9 / 8.8, 32
+    12.0 / 7.9, 64 14.9 / 14.5; prompts of 2,048 and 4,096 tokens 576 / 512, 16 1,022 / 344 and 288 / 256, 16 998 / 834.  (Of 240 sizes
+    from 272 / 256 to 576 / 512, one to 128 heads, one is 1 % slower, and of 192 value channels 64 heads of some 40 tokens, whose
+    second round of workgroups is a short one: 13.1 / 13.8.)"""
     return (attn_wide_takes(q, kcache, d) and kcache.shape[1] == 1 and d <= LATENT_MAX_WIDTH and 0 < wv <= min(d, LATENT_MAX_VALUES)
             and wv % 16 == 0)
 
