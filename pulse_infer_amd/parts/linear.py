@@ -364,26 +364,55 @@ class Linear:
 
     PARTS_MIN_K = 4096           # a plain product's inner dimension from which on its consumer had better add shares up
 
-    def forward_parts(self, x: torch.Tensor, workspace: Workspace) -> Optional[torch.Tensor]:
-        """The product as float32 shares [shares, rows, out] in a buffer of the workspace, for a caller whose next kernel adds
-        them up on the way (the rotation of q and k), or None: it is the faster one as it is (``forward``).
+    def parts_shares_for(self, x: torch.Tensor) -> int:
+        """Into how many shares of the inner dimension a plain product is cut for a consumer that adds them up on the way (the rotation
+        of q and k, ``forward_parts``); 0: it is the faster one as it is.
 
         The whole product has few tiles at some hundreds of rows, and a tile's walk takes as long as K is long; shares fill the chip
-        and cost the consumer their way from memory.  Measured, qkv and the rotation behind it, us, as they are / in shares: 6,144 x
-        4,096 at 65 / 97 / 160 / 256 / 357 / 512 rows 25.0 / 22.4 / 30.8 / 33.3 / 37.7 / 39.7 and 19.6 / 22.4 / 27.7 / 30.1 / 34.6 / 38.6,
-        7,168 x 5,120 35.8 / 33.9 / 47.7 / 44.4 / 52.7 / 59.0 and 25.2 / 28.1 / 37.5 / 41.9 / 42.4 / 54.2, 10,240 x 8,192 81 / 60 / 65 / 74 / 90 / 101
-        and 46 / 48 / 52 / 60 / 75 / 86; of shorter inner dimensions it depends on the rows: 6,144 x 2,560 at 65 / 97 / 160 / 357 rows 21.4 / 19.3 / 27.4 /
-        30.7 and 17.0 / 19.7 / 24.9 / 32.6, 4,096 x 2,048 13.7 / 13.7 / 14.1 / 19.7 and 12.4 / 12.3 / 15.6 / 22.1.  Where a product's
-        smallest tiles fill the chip once, it stays whole: 5,120 x 4,096 at 160 rows 22.5 and 26.0.  (Over 66 sizes of six weights of 4,096
-        columns and more 0.88 of the time, two of them 1 to 2 % slower.)"""
+        and cost the consumer their way from memory.  Product and rotation, us, whole (own / the library's) / in shares: 6,144 x 4,096 at
+        65 / 97 / 128 / 129 / 192 / 193 / 256 / 257 / 357 / 384 rows 23.9 / 22.0 / 25.0 / 30.0 / 29.4 / 29.3 / 32.8 / 35.7 / 37.3 / 38.6 and
+        19.5 / 21.8 / 23.2 / 26.7 / 28.2 / 28.5 / 29.6 / 30.5 / 33.4 / 33.4; 7,168 x 5,120 at 65 / 129 / 256 / 387 36 / 46 / 43 / 53 and 28 / 31 /
+        38 / 47; 10,240 x 8,192 at 65 / 192 / 512 78 / 67 / 101 and 49 / 54 / 89.  Of shorter inner dimensions it depends on the rows: 6,144 x 2,560
+        at 65 / 97 / 160 / 357 21.4 / 19.3 / 27.4 / 30.7 and 17.0 / 19.7 / 24.9 / 32.6.
+
+        Up to 256 rows the cut depends on the weight's shape alone, and where the whole product would be the one in stages at
+        each of these rows, so does the question whether to cut: a row's sums do not depend on how many rows are beside it.  Of other
+        shapes a product whose smallest tiles fill the chip once stays whole (5,120 x 4,096 at 160 rows 22.3 / 25.5).  Beyond, one whose own
+        tiles fill their rounds (6,144 x 4,096 at 388 / 448 / 512 rows 38.5 / 35.6 / 39.3 and 37.1 / 36.4 / 38.5 in two shares, for
+        which a row's results take twice the room), and one of so many tiles that the library's fill the chip half (18,432 x 7,168 at 300 rows
+        111 / 118).  Over 425 sizes of 17 weights 0.80 of the time, five of them 3 to 7 % and one 12 % slower (most where the
+        library's time jumps at 257 rows)."""
         rows, (n, k) = x.shape[0], self.weight.shape
         if not (k >= self.PARTS_MIN_K and rows <= self.STAGE_ROWS_SHARES and self.may_stage(x, self.weight)) or n % 4:
-            return None
-        shares = kernels.gemm_stages_shares(max(rows, self.STAGE_CUT_ROWS), n, k)
+            return 0
         tile_n, tile_m = kernels.gemm_stages_tile(rows, n, k)
         tiles, units = ((n + tile_n - 1) // tile_n) * ((rows + tile_m - 1) // tile_m), compute_units()
-        if shares < 2 or (tile_n * tile_m <= 64 * 64 and 0.9 * units <= tiles <= units):
+        if rows <= self.STAGE_ROWS[1]:
+            shares = kernels.gemm_stages_shares(self.SHARES_ROWS[1], n, k)
+            whole = tile_n * tile_m <= 64 * 64 and 0.9 * units <= tiles <= units and not self.always_stages(n, k, units)
+        else:
+            shares = kernels.gemm_stages_shares(rows, n, k)
+            side = self.LIBRARY_TILE
+            theirs = ((n + side - 1) // side) * ((rows + side - 1) // side)
+            whole = theirs > units // 2 or (self.takes_stages(x) and tiles >= 0.9 * units * ((tiles + units - 1) // units))
+        return 0 if whole or shares < 2 else shares
+
+    def always_stages(self, n: int, k: int, units: int) -> bool:
+        """Whether a plain product of this shape goes in stages at every number of rows up to 255."""
+        key = (n, k, units)
+        if key not in Linear._always:
+            Linear._always[key] = all(self.fills_stages(rows, n, k) for rows in range(self.STAGE_ROWS[0], self.TILE_MIN_ROWS))
+        return Linear._always[key]
+
+    _always: dict = {}           # (of shapes; a function of the sizes alone)
+
+    def forward_parts(self, x: torch.Tensor, workspace: Workspace) -> Optional[torch.Tensor]:
+        """The product as float32 shares [shares, rows, out] in a buffer of the workspace, for a caller whose next kernel adds
+        them up on the way, or None: it is the faster one as it is (``parts_shares_for``)."""
+        shares = self.parts_shares_for(x)
+        if not shares:
             return None
+        rows, (n, k) = x.shape[0], self.weight.shape
         parts = workspace.buffer(f"linear.shares.{n}.{k}", shares * rows, n, torch.float32).view(shares, rows, n)
         kernels.gemm_stages(x, self.weight, parts)
         return parts

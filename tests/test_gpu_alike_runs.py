@@ -20,14 +20,18 @@ def built(**changes):
     return build_model(cfg, RandomSource(expected_tensors(cfg.model_spec()), seed=3), mode="bfloat16")
 
 
-def steps(model):
+FEW_ROWS = ([("a", 40)], [("a", 1), ("b", 33)], [("a", 1), ("b", 1), ("c", 17)], [("d", 60)], [("a", 5), ("b", 20), ("d", 1)])
+MORE_ROWS = ([("a", 97)], [("a", 1), ("b", 128)], [("c", 192)], [("a", 20), ("c", 45)])      # 97, 129, 192 and 65
+
+
+def steps(model, plan=FEW_ROWS):
     """Logits of a prompt, of portions beside decoded tokens and of another prompt, at 17 to 64 rows; pages dealt out anew."""
     from pulse_infer_amd.engine.runner import ModelRunner, StepEntry
 
     runner = ModelRunner(model, page_size=16, num_pages=40, max_requests=4)
     token = lambda i, n: [(7 * i + 13 * k) % 300 for k in range(n)]
     out, fed = [], {}
-    for entries in ([("a", 40)], [("a", 1), ("b", 33)], [("a", 1), ("b", 1), ("c", 17)], [("d", 60)], [("a", 5), ("b", 20), ("d", 1)]):
+    for entries in plan:
         made = []
         for name, n in entries:
             if name not in fed:
@@ -40,7 +44,7 @@ def steps(model):
     return out
 
 
-def counted(monkeypatch, model, on):
+def counted(monkeypatch, model, on, plan=FEW_ROWS):
     from pulse_infer_amd.models import alike
     from pulse_infer_amd.ops import library
 
@@ -50,7 +54,7 @@ def counted(monkeypatch, model, on):
         patch.setattr(library, "_invoke", lambda lib, name, args: (calls.append(name), was(lib, name, args)))
         if not on:
             patch.setattr(alike, "MIN_RUNS", 10 ** 6)
-        return steps(model), len(calls)
+        return steps(model, plan), len(calls)
 
 
 def test_alike_runs_give_the_bits_of_their_parts(monkeypatch):
@@ -96,3 +100,37 @@ def test_weights_replaced_between_steps_are_the_ones_that_are_used(monkeypatch):
     recorded, _ = counted(monkeypatch, model, True)
     through, _ = counted(monkeypatch, model, False)
     assert all(torch.equal(a, b) for a, b in zip(recorded, through)) and not torch.equal(first[0], recorded[0])
+
+
+def test_projections_in_shares_are_launched_from_a_record(monkeypatch):
+    """Layers 4,096 wide at 65 to 192 rows: q, k and v leave their product as shares that the rotation adds up.  The bits of the same
+    step through its parts, and the results of the whole product within the rounding of bfloat16."""
+    from pulse_infer_amd.parts.linear import Linear
+
+    model = built(hidden_size=4096, num_hidden_layers=9, num_attention_heads=16, num_key_value_heads=8)
+    recorded, few = counted(monkeypatch, model, True, MORE_ROWS)
+    through, many = counted(monkeypatch, model, False, MORE_ROWS)
+    assert few < 0.7 * many          # runs 3 .. 7 of nine
+    for a, b in zip(recorded, through):
+        assert torch.equal(a, b)
+    made = []
+    real = Linear.forward_parts
+    monkeypatch.setattr(Linear, "forward_parts", lambda self, x, ws: made.append(real(self, x, ws)) or made[-1])
+    assert all(torch.equal(a, b) for a, b in zip(steps(model, MORE_ROWS), through))
+    assert made and all(parts is not None for parts in made)
+    monkeypatch.setattr(Linear, "forward_parts", lambda self, x, ws: None)
+    for a, b in zip(through, steps(model, MORE_ROWS)):
+        assert not torch.equal(a, b) and float((a - b).abs().max()) <= 4e-2 * float(b.abs().max())
+
+
+def test_a_rows_projection_does_not_depend_on_the_rows_beside_it():
+    from pulse_infer_amd.parts.base import Workspace
+    from pulse_infer_amd.parts.linear import Linear
+
+    gen = torch.Generator().manual_seed(11)
+    x = torch.randn(256, 4096, generator=gen).to(torch.bfloat16).to("cuda:0")
+    linear = Linear((torch.randn(6144, 4096, generator=gen) / 64).to(torch.bfloat16).to("cuda:0"), "bfloat16")
+    ws = Workspace(torch.device("cuda:0"))
+    want = linear.forward_parts(x[:65], ws).clone()
+    for rows in (66, 96, 128, 129, 130, 192, 193, 255, 256):
+        assert torch.equal(linear.forward_parts(x[:rows], ws)[:, :65], want), rows

@@ -196,6 +196,34 @@ def test_shares_of_an_update_depend_on_the_weight_alone_up_to_192_rows(units):
             assert 0 <= shares <= 16 and (shares == 0 or k % (64 * shares) == 0)
 
 
+def test_a_projections_shares_depend_on_the_weight_alone_up_to_256_rows(monkeypatch):
+    """One cut of q, k and v from 65 rows on, none to be had on one row and not on the next, wherever the whole product had one
+    order of its sums; beyond 256 rows whole again where shares are no gain."""
+    import torch
+    from pulse_infer_amd.ops import device
+    from pulse_infer_amd.parts import linear
+    from pulse_infer_amd.parts.linear import Linear
+
+    monkeypatch.setattr(device, "_units", 256)
+    monkeypatch.setattr(linear, "OWN_MANY_ROWS", "stages")
+    meta = lambda *shape: torch.empty(*shape, dtype=torch.bfloat16, device="meta")
+    shares = lambda rows, n, k: Linear(meta(n, k), "bfloat16").parts_shares_for(meta(rows, k))
+    for n, k in ((6144, 4096), (7168, 5120), (8192, 4096), (12288, 4096), (8192, 8192)):
+        cuts = {shares(m, n, k) for m in range(65, 257)}
+        assert len(cuts) == 1 and cuts != {0}, (n, k, cuts)
+        cut = cuts.pop()
+        assert k % (64 * cut) == 0
+    for n, k in ((5120, 4096), (10240, 8192), (3072, 4096)):      # (some rows of these are the library's when whole)
+        assert len({shares(m, n, k) for m in range(65, 257)} - {0}) == 1
+    assert shares(128, 5120, 4096) and not shares(129, 5120, 4096) and not shares(192, 5120, 4096) and shares(193, 5120, 4096)
+    assert not shares(64, 6144, 4096) and not shares(513, 6144, 4096)
+    assert shares(357, 6144, 4096) == 4 and shares(384, 6144, 4096) == 4 and not any(shares(m, 6144, 4096) for m in (385, 448, 509, 512))
+    assert shares(512, 7168, 5120) and shares(256, 18432, 7168) and not any(shares(m, 18432, 7168) for m in (257, 300, 512))
+    assert not shares(97, 6144, 2560) and not shares(97, 6142, 4096) and not shares(97, 1000, 4096)
+    monkeypatch.setattr(linear, "OWN_MANY_ROWS", "none")
+    assert shares(255, 6144, 4096) == 4 and not shares(256, 6144, 4096) and not shares(357, 6144, 4096)
+
+
 def test_updates_in_shares_of_many_rows_are_this_packages(units, monkeypatch):
     """Wherever an update beyond 192 rows is worth making in shares, the product in stages makes them, also of small
     weights, unless the option gives it to the tiled product or to the library."""
