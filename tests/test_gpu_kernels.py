@@ -233,6 +233,8 @@ def test_qk_rope_kv(k, dtype, case):
     dict(nq=7, nkv=7, d=64, rot=32, pairing="half", norm=True, bs=16),
     dict(nq=5, nkv=1, d=80, rot=80, pairing="interleaved", norm=False, bs=16),
     dict(nq=3, nkv=1, d=256, rot=0, pairing="half", norm=False, bs=32, v_head0=3),
+    dict(nq=6, nkv=2, d=64, rot=64, pairing="interleaved", norm=False, plain=True, temperature=(0.35, 8), bs=16, v_head0=6),
+    dict(nq=4, nkv=4, d=96, rot=32, pairing="half", norm=True, temperature=(0.2, 3), bs=16),
 ])
 def test_qk_rope_kv_adds_shares(k, case, shares):
     """The projection's rows as float32 shares: q, k and the pages as of their sum in 64 bits, the values the shares' sum in
@@ -257,7 +259,8 @@ def test_qk_rope_kv_adds_shares(k, case, shares):
     assert k.qk_rope_takes_parts(qkv, d, rot, kc, *weights)
     k.qk_rope_kv(qkv, nq, nkv, d, *weights, eps, cos, sin, rot, 0 if case["pairing"] == "interleaved" else 1, kc, vc,
                  torch.tensor(positions, dtype=torch.int32, device=DEV), torch.tensor(entry, dtype=torch.int32, device=DEV),
-                 table.to(DEV), v_head0=v_head0, parts=parts.to(DEV))
+                 table.to(DEV), plain_norm=case.get("plain", False), v_head0=v_head0,
+                 q_temperature=case.get("temperature"), parts=parts.to(DEV))
     ref = parts.to(F64).sum(0)
     q = ref[:, :nq * d].reshape(tokens, nq, d)
     kk = ref[:, nq * d:(nq + nkv) * d].reshape(tokens, nkv, d)
@@ -267,6 +270,12 @@ def test_qk_rope_kv_adds_shares(k, case, shares):
     vv = inorder[:, v_head0 * d:(v_head0 + nkv) * d].to(torch.bfloat16).to(F64).reshape(tokens, nkv, d)
     if case["norm"]:
         q, kk = P.rms_norm(q, qwref, eps), P.rms_norm(kk, kwref, eps)
+    if case.get("plain"):
+        q, kk = (P.rms_norm(x, torch.ones(d, dtype=F64), eps) for x in (q, kk))
+    if "temperature" in case:
+        coef, every = case["temperature"]
+        at = torch.tensor(positions, dtype=F64)
+        q = q * (1 + coef * torch.log(torch.floor((at + 1) / every) + 1)).view(-1, 1, 1)
     if rot:
         q = P.rope(q, positions, theta, rot, case["pairing"])
         kk = P.rope(kk, positions, theta, rot, case["pairing"])
