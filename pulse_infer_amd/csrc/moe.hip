@@ -78,6 +78,11 @@ struct Corrections {
     }
 };
 
+// Outputs a choice up to which ranking them all is faster than a search a choice (us for many tokens, search / ranks: 4 outputs a
+// choice, 16 and 4 -0.8, 32 and 8 -1.6; 6, 24 and 4 -0.2, 48 and 8 -0.6; 8, 32 and 4 +0.4, 64 and 8 +0.3; 16, 64 and 4 +2.2; 64, 64 and one
+// 20.9 / 24.6 in all).
+constexpr int RANK_OUTPUTS = 6;
+
 // One wavefront routes one token: `row` holds its n router logits (in global memory or in LDS).  `chosen` (LDS, or null): the token's
 // choices once more.
 template <typename TW, int PER = ROUTE_PER_LANE>
@@ -121,7 +126,7 @@ __device__ __forceinline__ void route_row(const float* row, const Corrections<TW
     float total = 0.f;
     float mine = 0.f;   // lane k keeps the score of choice k (top <= 64)
     int mine_idx = 0;
-    if constexpr (PER == 1) {
+    if (PER == 1 && n <= RANK_OUTPUTS * top) {
         // An output a lane: its place among the choices is the number of outputs before it (a larger score, or the same and a lower
         // number); the lane of that place receives its number and score.  (A search for the largest a choice, 16 outputs and 4 choices:
         // the launch 12.4 us, so 11.7.)

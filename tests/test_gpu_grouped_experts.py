@@ -85,6 +85,27 @@ def test_router_logits_at_the_edges_of_its_blocks(n, hidden, tokens):
             break
 
 
+@pytest.mark.parametrize("tokens", [3, 40])
+@pytest.mark.parametrize("n, top", [(1, 1), (6, 1), (7, 1), (24, 4), (25, 4), (48, 8), (49, 8), (64, 10), (64, 11), (64, 64)])
+def test_equal_outputs_are_chosen_in_their_order(n, top, tokens):
+    """Ranked (up to six outputs a choice) and searched for: several outputs of the same weights, the lower number first."""
+    from pulse_infer_amd.ops import kernels
+
+    hidden = 256
+    x = rnd(tokens, hidden, seed=1).to(torch.bfloat16)
+    kinds = (rnd(5, hidden, seed=2) * hidden ** -0.5).to(torch.bfloat16)
+    of = torch.randint(0, 5, (n,), generator=torch.Generator().manual_seed(n))
+    idx = torch.full((tokens, top), -5, dtype=torch.int32, device=DEV)
+    weight = torch.full((tokens, top), float("nan"), device=DEV)
+    kernels.moe_router(x.to(DEV), kinds[of].to(DEV), None, top, idx, weight)
+    z = (x.to(F64) @ kinds.to(F64).T)[:, of]
+    order = z.sort(dim=1, descending=True, stable=True).indices[:, :top]
+    assert torch.equal(idx.cpu().long(), order)      # (five values a token, further apart than sums in 32 bits err)
+    want = torch.softmax(z, 1).gather(1, order)
+    want = want / want.sum(1, keepdim=True)
+    assert ((weight.cpu().to(F64) - want).abs() <= 1e-5 * want).all()
+
+
 @pytest.mark.parametrize("tokens", [1, 7, 16])
 @pytest.mark.parametrize("n, experts, top, groups", [(2, 2, 1, (0, 0)), (16, 16, 4, (4, 2)), (64, 61, 8, (0, 0)), (65, 65, 6, (5, 3)),
                                                      (256, 256, 64, (0, 0)), (250, 200, 33, (0, 0))])
