@@ -104,24 +104,32 @@ class AlikeRuns:
             forward(index)
             return index + 1
         self.tries -= 1
+        before = linear.library_calls
+
+        def heard(run: int) -> Optional[List[Tuple]]:
+            """The run's calls, or None where it leaves more than they do."""
+            with library.listen() as calls:
+                forward(run)
+            left.append(self._left(stream))
+            return calls if linear.library_calls == before and left[-1] is not None and left[-1] == left[0] else None
+
+        # (the first run by itself: where a model's steps are none to record, that is all they wait for)
+        left: List[Tuple] = []
+        records = [heard(index)]
+        if records[0] is None:
+            self.tries = 0
+            return index + 1
         names = _attributes(self.blocks[self.order[index].layer])
         self._plain_of = attrgetter(*[n for n, is_tensor in names if not is_tensor])
         self._tensors_of = attrgetter(*[n for n, is_tensor in names if is_tensor])
         self._parts_of = attrgetter("mixer", "mixer.qkv", "mixer.o", "ffn", "ffn.gate_up", "ffn.down", "mixer_norm", "ffn_norm")
         first = self._describe(index)
         if not self._alike(first, index + 1):
-            forward(index)
             return index + 1
-        before, records, left = linear.library_calls, [], []
-        for i in (index, index + 1):
-            with library.listen() as calls:
-                forward(i)
-            records.append(calls)
-            left.append(self._left(stream))
-        if linear.library_calls != before or left[0] is None or left[0] != left[1]:
-            self.tries = 0
-            return index + 2
-        places = self._places(records, self._table(index), self._table(index + 1), [_reach(t) for t in first[1]])
+        records.append(heard(index + 1))
+        places = None
+        if records[1] is not None:
+            places = self._places(records, self._table(index), self._table(index + 1), [_reach(t) for t in first[1]])
         if places is None:
             self.tries = 0
             return index + 2

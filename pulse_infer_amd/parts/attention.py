@@ -206,9 +206,9 @@ class PagedAttention(Part):
         from_raw = self.decodes_from_raw(ctx, cache, qkv, tables)
         # (of the projection only q, k and v are read behind the rotation, which may take them as shares; a gate lies beside them)
         parts = None
-        if not from_raw and rows is None and not self.output_gate and not isinstance(x, LazyNorm) and kernels.qk_rope_takes_parts(
-                qkv, self.d, tables.rotary_dim if tables is not None else 0, cache.keys, self.q_w, self.k_w,
-                *((tables.cos, tables.sin) if tables is not None else ())):
+        if self.qkv.may_part(tokens) and not from_raw and rows is None and not self.output_gate and not isinstance(x, LazyNorm) \
+                and kernels.qk_rope_takes_parts(qkv, self.d, tables.rotary_dim if tables is not None else 0, cache.keys, self.q_w, self.k_w,
+                                                *((tables.cos, tables.sin) if tables is not None else ())):
             parts = self.qkv.forward_parts(x, ws)
         if parts is None:
             self.qkv.forward(x, qkv, rows=rows)

@@ -364,6 +364,10 @@ class Linear:
 
     PARTS_MIN_K = 4096           # a plain product's inner dimension from which on its consumer had better add shares up
 
+    def may_part(self, rows: int) -> bool:
+        """Whether a plain product of that many rows can be one in shares at all (a question for every layer of every step)."""
+        return self.in_features >= self.PARTS_MIN_K and self.STAGE_ROWS[0] <= rows <= self.STAGE_ROWS_SHARES
+
     def parts_shares_for(self, x: torch.Tensor) -> int:
         """Into how many shares of the inner dimension a plain product is cut for a consumer that adds them up on the way (the rotation
         of q and k, ``forward_parts``); 0: it is the faster one as it is.
@@ -383,7 +387,7 @@ class Linear:
         111 / 118).  Over 425 sizes of 17 weights 0.80 of the time, five of them 3 to 7 % and one 12 % slower (most where the
         library's time jumps at 257 rows)."""
         rows, (n, k) = x.shape[0], self.weight.shape
-        if not (k >= self.PARTS_MIN_K and rows <= self.STAGE_ROWS_SHARES and self.may_stage(x, self.weight)) or n % 4:
+        if not (self.may_part(rows) and self.may_stage(x, self.weight)) or n % 4:
             return 0
         tile_n, tile_m = kernels.gemm_stages_tile(rows, n, k)
         tiles, units = ((n + tile_n - 1) // tile_n) * ((rows + tile_m - 1) // tile_m), compute_units()
