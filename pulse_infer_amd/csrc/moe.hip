@@ -457,6 +457,10 @@ extern "C" int pulse_moe_route(const float* z, const void* correction, int c_dty
     return 0;
 }
 
+// Bytes that a row and its logits take in LDS (of every form of router: what one refuses, the others do too), and the most there are.
+constexpr size_t ROUTER_MEMORY = 60 * 1024;
+static size_t router_memory(int hidden, int n) { return sizeof(float) * (static_cast<size_t>(hidden) + 2 * n); }
+
 extern "C" int pulse_moe_router(const void* x, int x_dtype, const void* w, const void* correction, int w_dtype, int* idx,
                                 float* weight, int tokens, int hidden, int n, int top, int score_fn, int renorm,
                                 int groups, int keep, float wscale, hipStream_t stream) {
@@ -467,8 +471,8 @@ extern "C" int pulse_moe_router(const void* x, int x_dtype, const void* w, const
     PULSE_REQUIRE(n <= PULSE_WAVE * ROUTE_PER_LANE && top <= PULSE_WAVE,
                   "moe_router: at most %d router outputs and %d choices", PULSE_WAVE * ROUTE_PER_LANE, PULSE_WAVE);
     PULSE_REQUIRE(pulse_dtype_ok(x_dtype) && pulse_dtype_ok(w_dtype), "moe_router: bad dtype tag");
-    const size_t lds = sizeof(float) * (static_cast<size_t>(hidden) + 2 * n);
-    PULSE_REQUIRE(lds <= 60 * 1024, "moe_router: rows of %d values do not fit the workgroup's memory", hidden);
+    const size_t lds = router_memory(hidden, n);
+    PULSE_REQUIRE(lds <= ROUTER_MEMORY, "moe_router: rows of %d values do not fit the workgroup's memory", hidden);
     if (tokens == 0) return 0;
     if (x_dtype == PULSE_BF16 && w_dtype == PULSE_BF16 && hidden % 32 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0 &&
         reinterpret_cast<uintptr_t>(w) % 16 == 0) {
@@ -568,8 +572,8 @@ extern "C" int pulse_token_gate_add(const void* x, const void* w, int w_dtype, c
     return 0;
 }
 
-// The same for bfloat16 rows and weights of at most 16 tokens and 256 outputs (16-byte aligned, rows of a multiple of 32 values), with
-// what pulse_moe_group makes of the choices (but for `rank`).
+// pulse_moe_router for bfloat16 rows and weights of at most 16 tokens and 256 outputs (16-byte aligned, rows of a multiple of 32
+// values), with what pulse_moe_group makes of the choices (but for `rank`).
 extern "C" int pulse_moe_router_grouped(const void* x, const void* w, const void* correction, int* idx, float* weight, int tokens,
                                         int hidden, int n, int top, int score_fn, int renorm, int groups, int keep, float wscale,
                                         int experts, int tile_rows_max, int max_tiles, int* order, int* tile_expert, int* tile_row0,
@@ -581,6 +585,7 @@ extern "C" int pulse_moe_router_grouped(const void* x, const void* w, const void
                   "moe_router_grouped: at most %d tokens, %d outputs and %d choices", TILE_TOKENS, GROUP_OUTPUTS, PULSE_WAVE);
     PULSE_REQUIRE(hidden % 32 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0 && reinterpret_cast<uintptr_t>(w) % 16 == 0,
                   "moe_router_grouped: rows must be multiples of 32 values and 16-byte aligned");
+    PULSE_REQUIRE(router_memory(hidden, n) <= ROUTER_MEMORY, "moe_router_grouped: rows of %d values do not fit the workgroup's memory", hidden);
     PULSE_REQUIRE(tile_rows_max > 0 && tile_rows_max % 16 == 0, "moe_router_grouped: tiles hold a multiple of 16 rows");
     PULSE_REQUIRE(max_tiles >= (tokens * top + tile_rows_max - 1) / tile_rows_max + experts,
                   "moe_router_grouped: %d tiles cannot hold %d pairs of %d experts in every case", max_tiles, tokens * top, experts);

@@ -355,3 +355,20 @@ def test_items_of_several_prompts_stand_in_the_order_of_their_walks():
             walks = [of[i].start + row0 - of[i].first_row + n for row0, n, i, _ in fours(made)]
             assert walks == sorted(walks)
             assert M.build_portions(entries, per, 96) == plain
+
+
+def test_both_routers_refuse_rows_that_are_too_wide():
+    """What the router alone refuses is refused also where few tokens' choices are grouped in its launch."""
+    import ctypes
+    from pulse_infer_amd.ops import library
+
+    lib = library.load()
+    room = ctypes.create_string_buffer(64)
+    here = ctypes.c_void_p(ctypes.addressof(room) + 15 & ~15)
+    i, f = ctypes.c_int, ctypes.c_float
+    for hidden in (15360, 1 << 20):
+        assert lib.pulse_moe_router(here, i(1), here, None, i(1), here, here, i(8), i(hidden), i(16), i(4), i(0), i(1), i(0), i(0), f(1.0), None)
+        assert b"do not fit" in lib.pulse_last_error()
+        assert lib.pulse_moe_router_grouped(here, here, None, here, here, i(8), i(hidden), i(16), i(4), i(0), i(1), i(0), i(0), f(1.0), i(16),
+                                            i(32), i(17), here, here, here, here, here, None)
+        assert b"moe_router_grouped" in lib.pulse_last_error() and b"do not fit" in lib.pulse_last_error()
