@@ -240,7 +240,8 @@ template <int V>
 struct Steps { static constexpr int value = V; };
 
 // With GROUP all tokens are one workgroup's, which also groups their choices by expert, as moe_group_kernel does (see there): a launch
-// less, and choices that need not come back from memory.  8 tokens, 16 outputs of 4,096: 10.8 + 3.4 us in two launches, 11.7 in one.
+// less, and choices that need not come back from memory.  8 tokens of 4,096 values, 16 outputs and 4 choices / 32 and 4 / 64 and 8 / 128 and
+// 8 / 256 and 8: 12.6 / 18.2 / 30.9 / 55.7 / 100.5 us in two launches of a graph, 10.2 / 16.5 / 29.1 / 53.6 / 98.3 in one.
 constexpr int GROUP_OUTPUTS = 256;
 struct TileGroups {
     int experts, tile_rows, max_tiles;
@@ -334,7 +335,7 @@ __global__ __launch_bounds__(1024) void moe_router_tile_kernel(const bf16_t* __r
             meet[wave][lane] = acc;
             __syncthreads();
             if (share == 0) {
-                if (shares == TILE_WAVES) {          // (all asked for together)
+                if (shares == TILE_WAVES) {          // (up to 16 outputs, the most shares: all asked for together)
 #pragma unroll
                     for (int i = 1; i < TILE_WAVES; ++i) acc += meet[wave + i < TILE_WAVES ? wave + i : 0][lane];
                 } else {

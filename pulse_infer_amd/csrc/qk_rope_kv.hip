@@ -404,7 +404,7 @@ __device__ __forceinline__ void v_page_rows(int tile, int g, const bf16_t* __res
 
 // With PARTS the rows come as float32 shares of the projection (4 bytes a value and share): the lanes ask for four
 // shares' pieces of 16 bytes together.  40 heads of 128 at 97 / 160 / 357 tokens: 3.6 / 4.2 / 4.4 us from rounded rows, 4.5 / 5.0 / 8.5
-// from four shares, whose product takes 17.9 / 22.4 / 23.6 us where the whole one takes 20.3 / 27.4 / 32.3.
+// from four shares (figures of the product and the rotation together, by which it is decided, are at Linear.parts_shares_for).
 //
 // Both in one launch: the first `rope_groups` workgroups are four wavefronts of rows each, the others 16 tokens' values of a
 // kv head.  (Neither reads what the other writes: q's columns are the only ones written in place, and the values are never
