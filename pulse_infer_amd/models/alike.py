@@ -88,9 +88,9 @@ class AlikeRuns:
     def _alike(self, first: Tuple, index: int) -> bool:
         try:
             other = self._describe(index)
-        except AttributeError:
+            return bool(other[0] == first[0]) and _same_tensors(first[1], other[1])
+        except (AttributeError, TypeError, ValueError, RuntimeError):      # (one that it has not; a comparison without an answer)
             return False
-        return other[0] == first[0] and _same_tensors(first[1], other[1])
 
     def _table(self, index: int) -> List[int]:
         """Where the tensors lie that a run's calls may name: its own and its cache's.  (Of the norm that reads its result only an

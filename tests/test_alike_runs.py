@@ -3,6 +3,7 @@ import ctypes
 
 import types
 
+import numpy as np
 import pytest
 import torch
 
@@ -158,3 +159,22 @@ def test_a_block_of_another_kind_behind_alike_runs(kinds):
     launches.calls_of = lambda index: [(P(7), P(blocks[index].mixer.qkv.weight.data_ptr()))]
     through = launches.step()
     assert through == {2: [0, 1, 2, 3, 4, 9], 3: list(range(10)), 5: [0, 1, 2, *range(4, 10)]}[kinds[0]]
+
+
+def without_sinks():
+    blocks = [block() for _ in range(9)]
+    for b in blocks:
+        del b.mixer.sink
+    launches = Launches(blocks, [RunSpec(layer) for layer in range(9)])
+    launches.calls_of = lambda index: [(P(7), P(blocks[index].mixer.qkv.weight.data_ptr()))]
+    return blocks, launches
+
+
+@pytest.mark.parametrize("kind", ["arrays", "tensors", "array and none"])
+def test_attributes_that_cannot_be_compared_leave_the_runs_to_their_parts(kind):
+    """Whatever somebody keeps at a block: a comparison that has no answer is no error of the step."""
+    blocks, launches = without_sinks()
+    for layer, b in enumerate(blocks):
+        b.mixer.note = {"arrays": lambda: np.arange(3), "tensors": lambda: [torch.arange(3)],
+                        "array and none": lambda: np.arange(3) if layer != 4 else None}[kind]()
+    assert launches.step() == list(range(9))
