@@ -178,3 +178,14 @@ def test_attributes_that_cannot_be_compared_leave_the_runs_to_their_parts(kind):
         b.mixer.note = {"arrays": lambda: np.arange(3), "tensors": lambda: [torch.arange(3)],
                         "array and none": lambda: np.arange(3) if layer != 4 else None}[kind]()
     assert launches.step() == list(range(9))
+
+
+@pytest.mark.parametrize("place", ["block", "mixer", "norm"])
+def test_a_method_replaced_at_every_block_is_called_for_every_block(place):
+    """The same function put in a method's place at all of them: nothing else tells them apart."""
+    blocks, launches = without_sinks()
+    of = {"block": (lambda b: b, "forward"), "mixer": (lambda b: b.mixer, "attend"), "norm": (lambda b: b.mixer_norm, "apply")}[place]
+    watched = lambda *args, **kw: None
+    for b in blocks:
+        setattr(of[0](b), of[1], watched)
+    assert launches.step() == list(range(9))
