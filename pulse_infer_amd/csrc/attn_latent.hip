@@ -402,9 +402,9 @@ __global__ __launch_bounds__(256) void attn_latent_merge_kernel(const float* __r
 
 // q [tokens, q_stride] bfloat16: head h's query at h * d.  out float32 [tokens, o_stride]: of head h's d channels at h * d the first
 // wv are written.  items int32 [n_items, 4]: first token, tokens, first head, heads; row r (of 32) of an item is token r / hp, head
-// r % hp; rows that no item holds are left as they are.  several: whether an item may hold several tokens.  n_splits > 1: the keys of every item are shared out over that many
-// workgroups, whose sums (part float32 [n_items, 32, n_splits, wv], part_ml [n_items, 32, n_splits, 2]) a second kernel brings
-// together.  kcache [pages, 1, page, d], vcache [pages, 1, d, page] bfloat16.
+// r % hp; rows that no item holds are left as they are.  several: whether an item may hold several tokens.  n_splits > 1: the keys
+// of every item are shared out over that many workgroups, whose sums (part float32 [n_items, 32, n_splits, wv], part_ml [n_items, 32,
+// n_splits, 2]) a second kernel brings together.  kcache [pages, 1, page, d], vcache [pages, 1, d, page] bfloat16.
 extern "C" int pulse_attn_latent(const void* q, int64_t q_stride, float* out, int64_t o_stride, const void* kcache,
                                  const void* vcache, const int* positions, const int* token_entry, const int* block_table,
                                  int bt_width, const int* items, int n_items, int hp, int several, int nq, int d, int wv,
